@@ -69,10 +69,13 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  *        columns walked once, each X row segment loaded once and multiplied into every row
  *        of the block that has a nonzero there.  The fastest so_matmul for large matrices;
  *        so_matmul uses it whenever it is present and the launch covers most of the chip.
+ *        The layout also holds a second copy for smaller launches: quads of four rows with the
+ *        union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip);
+ *        so_matmul takes whichever of the two, or the kernels of the other layouts, is fastest.
  *        Sums are taken column by column, not in a row's slot order: results agree with
  *        the reference to fp32 round-off (max |y - ref| <= 1e-5 * max |ref|), are not
  *        bit-identical to it, and are the same bits on every launch.  Rows may be in any
- *        order.  Costs about 1.4x the ROW arrays in HBM; with it so_matmul keeps a
+ *        order.  Costs about 3x the ROW arrays in HBM; with it so_matmul keeps a
  *        workspace in the context that grows on first use of a larger output.
  * IDX16: a second copy of the columns in 16 bits (needs n <= 65536; costs 2 bytes per slot,
  *        and as much again for the SLOT copy when that is asked for too).  so_matvec then

@@ -13,6 +13,8 @@
 // its own tiles' slice of X.
 #include "so_internal.h"
 
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 namespace {
@@ -279,12 +281,52 @@ so_status launch_shared_gather(so_ctx *ctx, const so_ellpack *E, const float *dX
 
 } // namespace
 
+namespace {
+
+enum class RbmKernel { None, Merged, Quad };
+
+// Which of the RBM layout's two kernels a launch takes, or None for the kernels below, by estimated time (us).
+// Both sides of each line were measured on the shapes the quad kernel's model was fitted to (csrc/matmul_quad.hip),
+// us with the weights out of L2:
+//   quad against the row kernel: 2048 x 2048 x 64 at 95 / 90 / 80 / 50 % sparse 8.6 / 9.4 / 10.5 / 13.0 against
+//   6.7 / 14.2 / 17.4 / 63.4; 1024 x 1024 x 64 at 90 / 70 / 50 % 7.1 / 7.6 / 7.8 against 5.3 / 9.5 / 13.4 -- the row
+//   kernel moves 256 bytes per nonzero and 64 columns at about 11 TB/s, and a row takes 18 ns per nonzero on its own;
+//   quad against row-block-merged: 4096 x 4096 x 256 at 90 / 80 / 70 / 50 % 45 / 60 / 72 / 91 against 29 / 48 / 65 / 97
+//   -- 2.85 us per million (nonzero, 64 columns) on top of 9.5, and no faster on fewer workgroups than compute units.
+RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    const bool merged = so_matmul_rbm_applies(ctx, E, C), quad = so_matmul_quad_applies(ctx, E, C);
+    if (merged && ctx->tune.matmul_rbm == 1) return RbmKernel::Merged;
+    if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
+    if (quad && ctx->tune.matmul_quad == 1) return RbmKernel::Quad;
+    const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
+    const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
+    double best = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
+    RbmKernel k = RbmKernel::None;
+    if (merged) {
+        // one workgroup per (128 rows, 64 columns, share of the columns): pays when that grid covers most of the chip
+        const double wgs = (double)E->rbmm.nb * slabs * E->rbmm.ksplit;
+        const double us = 9.5 + 2.85e-6 * work * std::ceil(wgs / cus) * cus / wgs;
+        if (4.0 * wgs >= 3.0 * cus && (us < best || !quad)) { best = us; k = RbmKernel::Merged; }
+    }
+    if (quad && ctx->tune.matmul_quad != 0 && so_matmul_quad_estimate(ctx, E, C) < 0.95 * best) k = RbmKernel::Quad;
+    return k;
+}
+
+} // namespace
+
 extern "C" so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     SO_REQUIRE(ctx && E, "so_matmul_reserve: null argument");
-    if (E->m == 0 || C == 0 || !so_matmul_rbm_applies(ctx, E, C)) return SO_OK;
-    const so_status st = so_matmul_rbm_reserve(ctx, E, C);
-    return st != SO_OK ? st : so_matmul_rbm_set_pitch(ctx, E, C);
+    if (E->m == 0 || C == 0) return SO_OK;
+    // Both kernels of the layout: which one runs is settled at launch, where the tuning overrides may have changed.
+    so_status st = SO_OK;
+    if (so_matmul_quad_applies(ctx, E, C)) st = so_matmul_quad_reserve(ctx, E, C);
+    if (st == SO_OK && so_matmul_rbm_applies(ctx, E, C)) {
+        st = so_matmul_rbm_reserve(ctx, E, C);
+        if (st == SO_OK) st = so_matmul_rbm_set_pitch(ctx, E, C);
+    }
+    return st;
 }
 
 extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
@@ -298,16 +340,14 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     // one workgroup per (4 rows, 64 columns) at most: the grid must fit 31 bits
     SO_REQUIRE(((uint64_t)E->m / 4 + 8) * ((uint64_t)C / 64 + 1) < (1ull << 31), "so_matmul: %u x %u output is too large for one launch", E->m, C);
 
-    // The row-block-merged kernel, on handles uploaded with its layout (accurate to fp32 round-off, not
-    // bit-identical to the row order: the caller asked for it by asking for the layout).  It takes one
-    // workgroup per (128 rows, 64 columns, share of the columns), so like the LDS-staged kernel it pays
-    // when that grid covers most of the chip (SPARSEOPS_MATMUL_RBM=1 forces it, =0 forbids it).
-    if (so_matmul_rbm_applies(ctx, E, C) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
-        const uint64_t groups = (uint64_t)E->rbmm.nb * so_ceil_div(C, 64) * E->rbmm.ksplit;
-        bool rbm = 4 * groups >= 3 * (uint64_t)ctx->compute_units;
-        if (ctx->tune.matmul_rbm >= 0) rbm = ctx->tune.matmul_rbm == 1;
-        if (rbm) {
-            const so_status st = so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
+    // The kernels of the RBM layout, on handles uploaded with it (accurate to fp32 round-off, not bit-identical to
+    // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids both, =1
+    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one).
+    if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
+        const RbmKernel k = rbm_kernel(ctx, E, C);
+        if (k != RbmKernel::None) {
+            const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, dX, C, dBias, dY, act)
+                                                      : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
             return SO_OK;

@@ -218,15 +218,18 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
     if (ctx->tune.matmul_rbm_split == 1 || ctx->tune.matmul_rbm_split == 2 || ctx->tune.matmul_rbm_split == 4) ks = (uint32_t)ctx->tune.matmul_rbm_split;
     R.ksplit = ks;
     const uint32_t NS = NW * ks, per = NS * SLOTS, hdr_dw = 8 + NS * 2;
-    std::vector<uint32_t> hdr((size_t)R.nb * hdr_dw, 0), rec, xrows;
-    std::vector<float> w;
-    rec.reserve((size_t)(E->total_nnz / 40 + (size_t)R.nb * NS * (TAILRECS + 8)) * RECDW);
-    w.reserve(rec.capacity());
+    std::vector<uint32_t> hdr((size_t)R.nb * hdr_dw, 0);
+    // The blocks are independent of one another: built in parallel, each with records numbered from 0, then laid end to end.
+    struct Block { std::vector<uint32_t> rec, xrows; std::vector<float> w; uint64_t slots = 0, parts = 0; bool too_large = false; };
+    std::vector<Block> blocks(R.nb);
+    const auto pad_pair = std::make_pair(TRASH, -0.0f);
+    so_parallel(R.nb, E->total_nnz * 4, [&](uint32_t b0, uint32_t b1) {
     std::vector<std::vector<std::pair<uint32_t, float>>> cols(n);
     std::vector<uint32_t> used;
-    uint64_t slots_total = 0, parts_total = 0;
-    const auto pad_pair = std::make_pair(TRASH, -0.0f);
-    for (uint32_t b = 0; b < R.nb; ++b) {
+    for (uint32_t b = b0; b < b1; ++b) {
+        std::vector<uint32_t> &rec = blocks[b].rec, &xrows = blocks[b].xrows;
+        std::vector<float> &w = blocks[b].w;
+        uint64_t &slots_total = blocks[b].slots, &parts_total = blocks[b].parts;
         for (uint32_t j : used) cols[j].clear();
         used.clear();
         for (uint32_t i = b * RB; i < std::min(m, (b + 1) * RB); ++i)
@@ -264,7 +267,7 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
             } else {
                 while (L.size() % per) { Part d; d.j = 0; d.pr.assign(s, pad_pair); L.push_back(std::move(d)); }
             }
-            if (L.size() / per > 0xffffu) { so_set_error("so_ellpack_upload: too many columns for the RBM layout"); return SO_ERR_INVALID; }
+            if (L.size() / per > 0xffffu) { blocks[b].too_large = true; return; }
             q[s] = (uint32_t)(L.size() / per);
             cls[s] = std::move(L);
         }
@@ -272,7 +275,6 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
         for (uint32_t s = CMIN; s <= MAXP; ++s) h[(s - CMIN) / 2] |= q[s] << (16 * ((s - CMIN) % 2));
         for (uint32_t st = 0; st < NS; ++st) {
             const uint32_t entry = CMIN + st % NCLASS;
-            if (rec.size() / RECDW > 0xfffffff0ull) { so_set_error("so_ellpack_upload: matrix too large for the RBM layout"); return SO_ERR_INVALID; }
             h[8 + st * 2] = (uint32_t)(rec.size() / RECDW);
             h[8 + st * 2 + 1] = entry;
             for (uint32_t v = 0; v < NCLASS; ++v) {
@@ -305,32 +307,47 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
             }
         }
     }
-    R.nrec = rec.size() / RECDW;
+    });
+    std::vector<size_t> first(R.nb + 1, 0);                       // each block's first record
+    uint64_t slots_total = 0, parts_total = 0;
+    for (uint32_t b = 0; b < R.nb; ++b) {
+        if (blocks[b].too_large) { so_set_error("so_ellpack_upload: too many columns for the RBM layout"); return SO_ERR_INVALID; }
+        first[b + 1] = first[b] + blocks[b].rec.size() / RECDW;
+        slots_total += blocks[b].slots;
+        parts_total += blocks[b].parts;
+    }
+    if (first[R.nb] > 0xfffffff0ull) { so_set_error("so_ellpack_upload: matrix too large for the RBM layout"); return SO_ERR_INVALID; }
+    // records, weights, headers and X rows in one allocation and one copy
+    const size_t nrec = first[R.nb], rec_words = nrec * RECDW;
+    std::vector<uint32_t> blob(2 * rec_words + hdr.size() + nrec * SLOTS);
+    uint32_t *rec = blob.data(), *whdr = rec + 2 * rec_words, *xrows = whdr + hdr.size();
+    float *w = reinterpret_cast<float *>(rec + rec_words);
+    so_parallel(R.nb, rec_words / 8, [&](uint32_t b0, uint32_t b1) {
+        for (uint32_t b = b0; b < b1; ++b) {
+            std::copy(blocks[b].rec.begin(), blocks[b].rec.end(), rec + first[b] * RECDW);
+            std::copy(blocks[b].xrows.begin(), blocks[b].xrows.end(), xrows + first[b] * SLOTS);
+            std::copy(blocks[b].w.begin(), blocks[b].w.end(), w + first[b] * RECDW);
+            for (uint32_t st = 0; st < NS; ++st) hdr[(size_t)b * hdr_dw + 8 + st * 2] += (uint32_t)first[b];
+        }
+    });
+    std::copy(hdr.begin(), hdr.end(), whdr);
+    R.nrec = nrec;
     R.slots = slots_total;
     R.xloads = parts_total;
     void *p = nullptr;
-    so_status s = so_malloc(ctx, hdr.size() * 4, &p);
+    const so_status s = so_malloc(ctx, blob.size() * 4, &p);
     if (s != SO_OK) return s;
-    R.d_hdr = (uint32_t *)p;
-    if ((s = so_malloc(ctx, rec.size() * 4, &p)) != SO_OK) return s;
     R.d_rec = (uint32_t *)p;
-    if ((s = so_malloc(ctx, w.size() * 4, &p)) != SO_OK) return s;
-    R.d_w = (float *)p;
-    if ((s = so_malloc(ctx, xrows.size() * 4, &p)) != SO_OK) return s;
-    R.d_xrows = (uint32_t *)p;
-    if ((s = so_h2d(ctx, R.d_xrows, xrows.data(), xrows.size() * 4)) != SO_OK) return s;
-    if ((s = so_h2d(ctx, R.d_hdr, hdr.data(), hdr.size() * 4)) != SO_OK) return s;
-    if ((s = so_h2d(ctx, R.d_rec, rec.data(), rec.size() * 4)) != SO_OK) return s;
-    return so_h2d(ctx, R.d_w, w.data(), w.size() * 4);
+    R.d_w = (float *)(R.d_rec + rec_words);
+    R.d_hdr = R.d_rec + 2 * rec_words;
+    R.d_xrows = R.d_hdr + hdr.size();
+    return so_h2d(ctx, p, blob.data(), blob.size() * 4);
 }
 
 void so_rbmm_free(so_ellpack *E)
 {
     so_rbmm &R = E->rbmm;
-    if (R.d_hdr) (void)hipFree(R.d_hdr);
     if (R.d_rec) (void)hipFree(R.d_rec);
-    if (R.d_w) (void)hipFree(R.d_w);
-    if (R.d_xrows) (void)hipFree(R.d_xrows);
     R = so_rbmm();
 }
 
@@ -350,8 +367,13 @@ so_status so_matmul_rbm_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C)
     SO_REQUIRE(tiles * R.ksplit < (1ull << 28), "so_matmul: %u x %u output is too large for one launch", E->m, C);
     if (R.ksplit == 1) return SO_OK;
     const size_t need_part = (size_t)tiles * R.ksplit * RB * 64 * sizeof(float), need_cnt = (size_t)tiles * sizeof(uint32_t);
+    return so_matmul_workspace(ctx, need_part, need_cnt);
+}
+
+so_status so_matmul_workspace(so_ctx *ctx, size_t need_part, size_t need_cnt)
+{
     if (need_part <= ctx->mm_part_bytes && need_cnt <= ctx->mm_counter_bytes) return SO_OK;
-    SO_REQUIRE(!ctx->capturing, "so_matmul: the row-block-merged kernel's workspace must grow, which cannot be done while a graph is "
+    SO_REQUIRE(!ctx->capturing, "so_matmul: the kernel's workspace must grow, which cannot be done while a graph is "
                                 "being recorded (call so_matmul_reserve, or launch this shape once, before recording)");
     SO_HIP(hipStreamSynchronize(ctx->stream));
     if (ctx->mm_part) { (void)hipFree(ctx->mm_part); ctx->mm_part = nullptr; ctx->mm_part_bytes = 0; }

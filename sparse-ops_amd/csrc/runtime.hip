@@ -66,6 +66,9 @@ static void read_tuning(so_tuning &t)
     t.matmul_share = env_int("SPARSEOPS_MATMUL_SHARE", -1);
     t.matmul_rbm = env_int("SPARSEOPS_MATMUL_RBM", -1);
     t.matmul_rbm_split = env_int("SPARSEOPS_MATMUL_RBM_SPLIT", 0);
+    t.matmul_quad = env_int("SPARSEOPS_MATMUL_QUAD", -1);
+    t.matmul_quad_rows = env_int("SPARSEOPS_MATMUL_QUAD_ROWS", -1);
+    t.matmul_quad_split = env_int("SPARSEOPS_MATMUL_QUAD_SPLIT", 0);
     const int lanes = env_int("SPARSEOPS_MATVEC_LANES", 0);
     t.matvec_lanes = (lanes == 8 || lanes == 16 || lanes == 32 || lanes == 64) ? lanes : 0;
     t.matvec_idx16 = env_int("SPARSEOPS_MATVEC_IDX16", -1);
@@ -341,6 +344,7 @@ static void free_ellpack_arrays(so_ellpack *E)
     if (E->tiled.d_info) (void)hipFree(E->tiled.d_info);
     if (E->tiled.d_rows) (void)hipFree(E->tiled.d_rows);
     so_rbmm_free(E);
+    so_quads_free(E);
 }
 
 // Device copy of a host array with 16 zeroed bytes after the last element, so a
@@ -381,8 +385,10 @@ static so_status build_tiled(so_ctx *ctx, so_ellpack *E, const float *Wd, const 
         std::stable_sort(blockwise.begin() + b0, blockwise.begin() + std::min(m, b0 + 64), longer_first);
     if ((uint64_t)m * T.ntiles <= (1ull << 28)) {                     // the comparison needs 2 bytes per (row, tile)
         std::vector<uint16_t> per_tile((size_t)m * T.ntiles, 0);      // a tile has at most 256 columns
-        for (uint32_t i = 0; i < m; ++i)
-            for (uint32_t k = 0; k < nnz[i]; ++k) ++per_tile[(size_t)i * T.ntiles + idx[(size_t)i * r + k] / KT];
+        so_parallel(m, E->total_nnz, [&](uint32_t i0, uint32_t i1) {
+            for (uint32_t i = i0; i < i1; ++i)
+                for (uint32_t k = 0; k < nnz[i]; ++k) ++per_tile[(size_t)i * T.ntiles + idx[(size_t)i * r + k] / KT];
+        });
         const auto steps_of = [&](const std::vector<uint32_t> &ord) {
             uint64_t total = 0;
             for (uint32_t q0 = 0; q0 < m; q0 += 4)
@@ -398,15 +404,13 @@ static so_status build_tiled(so_ctx *ctx, so_ellpack *E, const float *Wd, const 
     std::vector<uint32_t> qrows((size_t)T.nquads * 4, 0xffffffffu);
     for (uint32_t i = 0; i < m; ++i) qrows[i] = order[i];
 
+    // Steps per (quad, tile) first, then every quad fills in its own chunks.
     std::vector<so_tile_info> info((size_t)T.nquads * T.ntiles);
-    std::vector<so_tile_entry> entries;
-    entries.reserve((size_t)E->total_nnz + (size_t)E->total_nnz / 3 + 256);
-    uint64_t total_steps = 0;
-    for (uint32_t q = 0; q < T.nquads; ++q) {
+    const auto walk = [&](uint32_t q, const auto &tile) {             // tile(t, first slot of each row in tile t, slots)
         uint32_t pos[4] = {0, 0, 0, 0};
         for (uint32_t t = 0; t < T.ntiles; ++t) {
             const uint64_t col_end = (uint64_t)(t + 1) * KT;
-            uint32_t cnt[4] = {0, 0, 0, 0}, steps = 0;
+            uint32_t cnt[4] = {0, 0, 0, 0};
             for (int g = 0; g < 4; ++g) {
                 const uint32_t row = qrows[(size_t)q * 4 + g];
                 if (row == 0xffffffffu) continue;
@@ -414,33 +418,47 @@ static so_status build_tiled(so_ctx *ctx, so_ellpack *E, const float *Wd, const 
                 uint32_t p = pos[g];
                 while (p < nnz[row] && c[p] < col_end) ++p;
                 cnt[g] = p - pos[g];
-                steps = std::max(steps, cnt[g]);
             }
-            steps = (steps + 3u) & ~3u;
-            if (entries.size() / 64 > 0xfffffff0ull) { so_set_error("so_ellpack_upload: matrix too large for the tiled layout"); return SO_ERR_INVALID; }
-            info[(size_t)q * T.ntiles + t] = so_tile_info{(uint32_t)(entries.size() / 64), steps};
-            total_steps += steps;
-            // The zero row sits after both tile buffers; offsets are relative to the buffer the tile uses.
-            // A padding step is fma(-0, +0, acc): adding -0 leaves every accumulator, -0 included, as it is.
-            const uint32_t zero_off = so_tiled::kZeroRowOff - (t & 1u) * so_tiled::kTileBytes;
-            const uint32_t nch = (steps + 15) / 16;
-            for (uint32_t ch = 0; ch < nch; ++ch)
-                for (int g = 0; g < 4; ++g) {
-                    const uint32_t row = qrows[(size_t)q * 4 + g];
-                    for (uint32_t k = 0; k < 16; ++k) {
-                        const uint32_t sidx = ch * 16 + k;
-                        so_tile_entry e{-0.0f, zero_off};
-                        if (sidx < cnt[g]) {
-                            const size_t slot = (size_t)row * r + pos[g] + sidx;
-                            e.w = Wd[slot];
-                            e.off = (idx[slot] - t * KT) * ROWB;
-                        }
-                        entries.push_back(e);
-                    }
-                }
+            tile(t, pos, cnt);
             for (int g = 0; g < 4; ++g) pos[g] += cnt[g];
         }
+    };
+    so_parallel(T.nquads, E->total_nnz, [&](uint32_t q0, uint32_t q1) {
+        for (uint32_t q = q0; q < q1; ++q)
+            walk(q, [&](uint32_t t, const uint32_t *, const uint32_t *cnt) {
+                info[(size_t)q * T.ntiles + t].steps = (std::max(std::max(cnt[0], cnt[1]), std::max(cnt[2], cnt[3])) + 3u) & ~3u;
+            });
+    });
+    uint64_t total_steps = 0, chunks = 0;
+    for (so_tile_info &i : info) {
+        if (chunks > 0xfffffff0ull) { so_set_error("so_ellpack_upload: matrix too large for the tiled layout"); return SO_ERR_INVALID; }
+        i.chunk0 = (uint32_t)chunks;
+        chunks += (i.steps + 15) / 16;
+        total_steps += i.steps;
     }
+    std::vector<so_tile_entry> entries((size_t)chunks * 64);
+    so_parallel(T.nquads, E->total_nnz, [&](uint32_t q0, uint32_t q1) {
+        for (uint32_t q = q0; q < q1; ++q)
+            walk(q, [&](uint32_t t, const uint32_t *pos, const uint32_t *cnt) {
+                // The zero row sits after both tile buffers; offsets are relative to the buffer the tile uses.
+                // A padding step is fma(-0, +0, acc): adding -0 leaves every accumulator, -0 included, as it is.
+                const uint32_t zero_off = so_tiled::kZeroRowOff - (t & 1u) * so_tiled::kTileBytes;
+                const so_tile_info &in = info[(size_t)q * T.ntiles + t];
+                so_tile_entry *out = entries.data() + (size_t)in.chunk0 * 64;
+                for (uint32_t ch = 0; ch < (in.steps + 15) / 16; ++ch)
+                    for (int g = 0; g < 4; ++g)
+                        for (uint32_t k = 0; k < 16; ++k) {
+                            const uint32_t sidx = ch * 16 + k;
+                            so_tile_entry e{-0.0f, zero_off};
+                            if (sidx < cnt[g]) {
+                                const size_t slot = (size_t)qrows[(size_t)q * 4 + g] * r + pos[g] + sidx;
+                                e.w = Wd[slot];
+                                e.off = (idx[slot] - t * KT) * ROWB;
+                            }
+                            *out++ = e;
+                        }
+            });
+    });
     // Three zero chunks of slack: the kernel always fetches three chunks per tile.
     entries.resize(entries.size() + 3 * 64, so_tile_entry{-0.0f, so_tiled::kZeroRowOff});
     T.total_steps = total_steps;
@@ -558,6 +576,7 @@ extern "C" so_status so_ellpack_upload(so_ctx *ctx, const float *Wd, const uint3
 
     if (s == SO_OK && (layouts & SO_LAYOUT_TILED) && m > 0) s = build_tiled(ctx, E, Wd, idx, nnz);
     if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_rbmm_build(ctx, E, Wd, idx, nnz);
+    if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_quads_build(ctx, E, Wd, idx, nnz);
 
     if (s != SO_OK) {
         free_ellpack_arrays(E);

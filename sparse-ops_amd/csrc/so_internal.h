@@ -1,9 +1,11 @@
 // Internal definitions shared by the HIP translation units of libsparseops_hip.so.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sparseops_hip.h"
@@ -16,6 +18,9 @@ struct so_tuning {
     int matmul_share = -1;   // SPARSEOPS_MATMUL_SHARE: 0 forbids the shared-gather kernel for few-row launches
     int matmul_rbm = -1;     // SPARSEOPS_MATMUL_RBM: 0 forbids the row-block-merged kernel on handles that carry its layout, 1 forces it
     int matmul_rbm_split = 0;   // SPARSEOPS_MATMUL_RBM_SPLIT: 1, 2 or 4 workgroups per tile for RBM layouts built from now on
+    int matmul_quad = -1;    // SPARSEOPS_MATMUL_QUAD: 0 forbids the quad-union kernel on handles with the RBM layout, 1 forces it
+    int matmul_quad_rows = -1;  // SPARSEOPS_MATMUL_QUAD_ROWS: log2 of the quads per workgroup (0..4)
+    int matmul_quad_split = 0;  // SPARSEOPS_MATMUL_QUAD_SPLIT: workgroups per output tile
     int matvec_lanes = 0;    // SPARSEOPS_MATVEC_LANES: 8, 16, 32 or 64 lanes per row
     int matvec_idx16 = -1;   // SPARSEOPS_MATVEC_IDX16: 0 keeps so_matvec on the 32-bit columns of a handle that has both
     int conv_min_cg = 0;     // SPARSEOPS_CONV_MIN_CG: fewest channel groups per workgroup a small grid may shrink to (16: never shrink)
@@ -99,6 +104,18 @@ struct so_rbmm {
     uint32_t pitch = 0;                           // row pitch of X (bytes) the records' offsets are written for; 0: none yet
 };
 
+// Quad-union copy of the matrix for so_matmul on the matrix cores (csrc/matmul_quad.hip): four consecutive rows
+// share a list of columns, cut by tiles of 256 columns and stored in chunks of 16 steps.
+struct so_quads {
+    static constexpr uint32_t kTileRows = 256;    // X rows per LDS tile
+    static constexpr uint32_t kMaxSplit = 64;     // most workgroups per output tile
+    uint32_t nquads = 0, ntiles = 0;
+    uint64_t total_units = 0;                     // units of four steps over all (quad, tile) runs
+    float *d_w = nullptr;                         // [chunks + slack][64]
+    uint32_t *d_off = nullptr;                    // [chunks + slack][4] words: X row inside the tile, a byte per step
+    uint2 *d_info = nullptr;                      // [nquads][ntiles] {first chunk, units}
+};
+
 struct so_ellpack {
     uint32_t m = 0, n = 0, r = 0;
     uint64_t total_nnz = 0;
@@ -114,7 +131,8 @@ struct so_ellpack {
     uint16_t *d_idxT16 = nullptr;// [r*m] the same for d_idxT (SO_LAYOUT_SLOT with SO_LAYOUT_IDX16)
     so_bin bins[4];              // SO_LAYOUT_BINS
     so_tiled tiled;              // SO_LAYOUT_TILED
-    so_rbmm rbmm;                // SO_LAYOUT_RBM
+    so_rbmm rbmm;                // SO_LAYOUT_RBM, where that kernel may be the faster one
+    so_quads quads;              // SO_LAYOUT_RBM
 };
 
 // Row-block-merged re-encoding of a matrix (include/rbm_conv.hpp:8-27 of the reference), flattened:
@@ -148,6 +166,18 @@ so_status so_matmul_rbm_set_pitch(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_rbm_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_rbm_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
                                const float *dBias, float *dY, int act);
+
+// Grows the context's matmul workspace (partial tiles, a zeroed counter per tile).  Never while a graph is being recorded.
+so_status so_matmul_workspace(so_ctx *ctx, size_t part_bytes, size_t counter_bytes);
+
+// csrc/matmul_quad.hip: the quad-union layout and its kernel.
+so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz);
+void so_quads_free(so_ellpack *E);
+bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);   // us
+so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
+so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
+                                const float *dBias, float *dY, int act);
 
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
 // since the last look (their results are invalid).  Every entry point that waits for the stream ends with this.
@@ -185,6 +215,20 @@ hipError_t so_allow_big_lds(so_ctx *ctx, const void *kernel);
             return SO_ERR_HIP;                                                    \
         }                                                                         \
     } while (0)
+
+// f(first, last) over ranges of 0 .. count on up to 16 threads: the layout builders' loops.  `work` = elements that
+// the whole loop touches: a thread costs some 30 us to start, which 100 000 elements repay.
+template <class F>
+void so_parallel(uint32_t count, uint64_t work, F &&f)
+{
+    const uint64_t most = std::min<uint64_t>({std::max(1u, std::thread::hardware_concurrency()), 16u, count, work / 100000u + 1u});
+    const uint32_t nt = (uint32_t)std::max<uint64_t>(1u, most);
+    std::vector<std::thread> threads;
+    for (uint32_t t = 1; t < nt; ++t)
+        threads.emplace_back([&, t] { f((uint32_t)((uint64_t)count * t / nt), (uint32_t)((uint64_t)count * (t + 1) / nt)); });
+    f(0u, (uint32_t)((uint64_t)count / nt));
+    for (auto &t : threads) t.join();
+}
 
 static inline uint32_t so_ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 

@@ -30,9 +30,9 @@ int matmul_layouts(const Ellpack &E, uint32_t C, bool fast)
     for (uint32_t c : E.nnz) total += c;
     const bool big = E.m >= 512 && E.n >= 512 && total >= 32ull * E.m;
     if (!big || C < 64) return SO_LAYOUT_ROW;
-    // The row-block-merged kernel pays its fixed costs (sums over 12 or 24 streams) only with enough columns per
-    // stream: below ~1500 columns the K-tiled kernel is ahead (4096 x 784 x 256: 11.2 us against 13.8).
-    if (fast && E.n >= 1536) return SO_LAYOUT_ROW | SO_LAYOUT_RBM;
+    // The layout's quad-union kernel is ahead of the K-tiled one below the row-block-merged kernel's sizes as well
+    // (4096 x 784 x 256 at 90 %: 12.0 us against 15.2).
+    if (fast) return SO_LAYOUT_ROW | SO_LAYOUT_RBM;
     return C % 4 == 0 ? (SO_LAYOUT_ROW | SO_LAYOUT_TILED) : SO_LAYOUT_ROW;
 }
 } // namespace sparseops

@@ -1,0 +1,112 @@
+"""The quad-union kernel of SO_LAYOUT_RBM (csrc/matmul_quad.hip), forced, at the edges of its tiles: rows in quads of
+4 and blocks of up to 64, tiles of 256 X rows, slabs of 64 dense columns in groups of 4, chunks of 16 steps in units of
+4, every rows-per-workgroup and K-split choice.
+
+Bound: max|y - ref| <= 1e-5 * max|ref| against the in-order oracle and the fp64 product, as for the layout's other
+kernel (tests/test_gpu_matmul_rbm.py): the same products, summed in another order in fp32."""
+
+import numpy as np
+import pytest
+
+from conftest import as_oracle, rel_err, sparse_matrix
+
+import datagen
+import hipabi
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+RBM = hipabi.LAYOUT_ROW | hipabi.LAYOUT_RBM
+
+
+def quad_matmul(ctx, E, X, bias, act="none", rows=None, split=None):
+    m, C = E.m, X.shape[1]
+    with ctx.tuning(SPARSEOPS_MATMUL_QUAD="1", SPARSEOPS_MATMUL_QUAD_ROWS=rows, SPARSEOPS_MATMUL_QUAD_SPLIT=split):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+        dX, dY, dB = ctx.array(X), ctx.empty((m, C)), ctx.array(bias) if bias is not None else None
+        outs = []
+        for _ in range(2):
+            dY.upload(np.full((m, C), np.nan, np.float32))
+            ctx.matmul(dE, dX, C, dB, dY, act)
+            outs.append(dY.download())
+        for a in (dX, dY, dB):
+            if a is not None:
+                a.free()
+        dE.free()
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)
+    return outs[0]
+
+
+@pytest.mark.parametrize("m,n,C,sp", [
+    (1, 1, 4, .0), (3, 2, 5, .0), (4, 255, 7, .5), (5, 256, 63, .5), (63, 257, 64, .9), (64, 300, 65, .7), (65, 511, 66, .3),
+    (130, 513, 67, .95), (129, 1025, 130, .8), (300, 700, 256, .5), (257, 2100, 101, .6), (17, 4096, 12, .99), (1000, 512, 32, .0)])
+@pytest.mark.parametrize("rows,split", [(None, None), (4, 1), (2, 3), (0, 2)])
+def test_quad_shapes(ctx, oracle, m, n, C, sp, rows, split):
+    rng = np.random.default_rng(m * 31 + n * 7 + C)
+    W = sparse_matrix(rng, m, n, sp)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    E = datagen.encode_dense(W)
+    Y = quad_matmul(ctx, E, X, b, "relu" if split == 3 else "none", rows, split)
+    ref = W.astype(np.float64) @ X + b[:, None]
+    assert rel_err(Y, np.maximum(ref, 0) if split == 3 else ref) <= TOL
+    assert rel_err(Y, oracle.matmul(as_oracle(E), X, b, "relu" if split == 3 else "none")) <= TOL
+
+
+def test_quad_unordered_repeated_and_special_values(ctx, oracle):
+    """Reversed rows, a column that a row names twice, empty rows, a dense row; and an infinity in X reaches exactly
+    the rows that use it, although a quad's other rows meet it with a zero weight."""
+    rng = np.random.default_rng(11)
+    m, n, C = 140, 600, 70
+    W = sparse_matrix(rng, m, n, .8)
+    W[7], W[9] = 0, rng.standard_normal(n)
+    E = datagen.encode_dense(W)
+    for i in range(0, m, 2):
+        c = int(E.nnz[i])
+        E.Wd[i, :c], E.idx[i, :c] = E.Wd[i, :c][::-1].copy(), E.idx[i, :c][::-1].copy()
+    c = int(E.nnz[20])
+    E.idx[20, 1] = E.idx[20, 0]
+    Wd = np.zeros((m, n))
+    for i in range(m):
+        np.add.at(Wd[i], E.idx[i, :E.nnz[i]], E.Wd[i, :E.nnz[i]].astype(np.float64))
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    assert rel_err(quad_matmul(ctx, E, X, None), Wd @ X) <= TOL
+    X[0, :], X[17, 3], X[300, 5] = np.inf, -np.inf, np.nan
+    E = datagen.encode_dense(W)
+    for split in (1, 3):
+        Y = quad_matmul(ctx, E, X, None, split=split)
+        Yo = oracle.matmul(as_oracle(E), X, None)
+        assert np.array_equal(np.isnan(Y), np.isnan(Yo)) and np.array_equal(np.isinf(Y), np.isinf(Yo))
+        fin = np.isfinite(Yo)
+        assert np.array_equal(Y[np.isinf(Yo)], Yo[np.isinf(Yo)])
+        assert np.abs(Y[fin] - Yo[fin]).max() <= TOL * np.abs(Yo[fin]).max()
+
+
+def test_quad_in_a_launch_graph(ctx, oracle):
+    """so_matmul_reserve sizes the workspace of a K split ahead of a recording; replays give the eager launch's bits."""
+    rng = np.random.default_rng(3)
+    W = sparse_matrix(rng, 300, 1100, .7)
+    E = datagen.encode_dense(W)
+    C = 40
+    with ctx.tuning(SPARSEOPS_MATMUL_QUAD="1", SPARSEOPS_MATMUL_QUAD_SPLIT="4"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+        dX, dY = ctx.empty((1100, C)), ctx.empty((300, C))
+        ctx.matmul_reserve(dE, C)
+        ctx.graph_begin()
+        ctx.matmul(dE, dX, C, None, dY, "tanh")
+        g = ctx.graph_end()
+        for _ in range(3):
+            X = rng.standard_normal((1100, C)).astype(np.float32) * 0.1
+            dX.upload(X)
+            ctx.matmul(dE, dX, C, None, dY, "tanh")
+            eager = dY.download()
+            ctx.fill_zero(dY)
+            ctx.sync()
+            ctx.graph_launch(g)
+            assert np.array_equal(dY.download(), eager)
+            # tanh's slope is at most 1: the sums' bound carries over, plus the device tanhf's 1e-6
+            pre = np.abs(oracle.matmul(as_oracle(E), X, None)).max()
+            assert np.abs(eager - np.tanh(W.astype(np.float64) @ X)).max() <= TOL * pre + 1e-6
+        ctx.graph_free(g)
+        for a in (dX, dY):
+            a.free()
+        dE.free()
