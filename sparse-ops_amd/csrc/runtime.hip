@@ -131,6 +131,7 @@ extern "C" so_status so_init(int device, so_ctx **out)
         return e == hipErrorOutOfMemory ? SO_ERR_OOM : SO_ERR_HIP;
     }
     *ctx->h_wait_gave_up = 0;
+    ctx->h_encode_header = ctx->h_wait_gave_up + 8;      // the same 64 bytes
     *out = ctx;
     return SO_OK;
 }
@@ -610,19 +611,101 @@ extern "C" so_status so_ellpack_dims(const so_ellpack *E, uint32_t *m, uint32_t 
 
 namespace {
 
-// One wave per row: its stored nonzeros go to their columns (ascending, distinct, so no two
-// lanes write the same element).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of a dense matrix start anywhere
+
+// Decoding: a workgroup builds kDecodeSpan consecutive elements of W in LDS -- whole rows, or a part of one longer
+// row -- and writes them out once, 16 bytes per lane, past the caches (nontemporal: a plain store of W takes twice as
+// long and pushes the matrix out of the Infinity Cache).  The span starts as zeros and is put back to zeros after each
+// use by clearing what was scattered.  Slots are requested eight per thread at a time, those of the next span while
+// this one is written out.
+// Bound by the write of W: 8192 x 8192, 90 % sparse, 50 us (6.4 TB/s of its 322 MB), 80 on buffers not used before;
+// 143 and 114 as a fill of W followed by a scatter of single words into it.  Without the requests ahead the chain
+// length -> slots -> span -> write made it 67 and 140.
+constexpr uint32_t kDecodeSpan = 8192;       // 32 KB: five workgroups per compute unit
+constexpr uint32_t kDecodeSlots = 8;         // slots a thread has in registers
+
 __global__ __launch_bounds__(256)
 void ellpack_decode_kernel(const float *__restrict__ Wd, const uint32_t *__restrict__ idx,
                            const uint32_t *__restrict__ nnz, uint32_t m, uint32_t n, uint32_t r,
-                           float *__restrict__ W)
+                           float *__restrict__ W, uint32_t rows_per_span, uint32_t spans)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t nwaves = gridDim.x * 4u;
-    for (uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6); row < m; row += nwaves) {
-        const uint32_t cnt = nnz[row];
-        for (uint32_t k = lane; k < cnt; k += 64u)
-            W[(size_t)row * n + idx[(size_t)row * r + k]] = Wd[(size_t)row * r + k];
+    __shared__ __attribute__((aligned(16))) float span[kDecodeSpan];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    f32x4u *span4 = reinterpret_cast<f32x4u *>(span);
+    for (uint32_t k = tid; k < kDecodeSpan / 4u; k += 256u) *reinterpret_cast<float4 *>(span + 4u * k) = make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint32_t per_row = (n + kDecodeSpan - 1u) / kDecodeSpan;       // spans of a row (1 when a span holds whole rows)
+    // one row per span: all four waves share it; several: a wave takes every fourth
+    const bool one = rows_per_span == 1u;
+    const uint32_t k0 = one ? tid : lane, kstep = one ? 256u : 64u, first = one ? 0u : wave;
+
+    // Slots k0 + k * kstep .. of one row: columns relative to the span (0xffffffff: no such slot) and values.
+    auto request = [&](uint32_t row, uint32_t from, uint32_t cnt, uint32_t (&at)[kDecodeSlots], float (&v)[kDecodeSlots]) {
+        const uint32_t *ix = idx + (size_t)row * r;
+        const float *wd = Wd + (size_t)row * r;
+#pragma unroll
+        for (uint32_t u = 0; u < kDecodeSlots; ++u) {
+            const uint32_t k = from + k0 + u * kstep;
+            at[u] = 0xffffffffu;
+            if (k < cnt) { at[u] = ix[k]; v[u] = wd[k]; }
+        }
+    };
+    auto rows_of = [&](uint32_t sp, uint32_t &row0, uint32_t &col0) {
+        row0 = per_row == 1u ? sp * rows_per_span : sp / per_row;
+        col0 = per_row == 1u ? 0u : (sp - row0 * per_row) * kDecodeSpan;
+    };
+    uint32_t at[kDecodeSlots], at_next[kDecodeSlots], row0, col0, cnt = 0, cnt_next = 0;
+    float v[kDecodeSlots], v_next[kDecodeSlots];
+    if (one && blockIdx.x < spans) {
+        rows_of(blockIdx.x, row0, col0);
+        cnt = nnz[row0];
+        request(row0, 0, cnt, at, v);
+        if (blockIdx.x + gridDim.x < spans) { rows_of(blockIdx.x + gridDim.x, row0, col0); cnt_next = nnz[row0]; }
+    }
+    for (uint32_t sp = blockIdx.x; sp < spans; sp += gridDim.x) {
+        rows_of(sp, row0, col0);
+        const uint32_t rows = min(rows_per_span, m - row0);
+        const uint32_t count = per_row == 1u ? rows * n : min(kDecodeSpan, n - col0);
+        float *out = W + (size_t)row0 * n + col0;
+        // value = false: the same places back to zero
+        auto scatter = [&](uint32_t i, const uint32_t (&a)[kDecodeSlots], const float (&x)[kDecodeSlots], bool value) {
+#pragma unroll
+            for (uint32_t u = 0; u < kDecodeSlots; ++u) {
+                const uint32_t c = a[u] - col0;
+                if (a[u] != 0xffffffffu && c < count) span[i * n + c] = value ? x[u] : 0.0f;
+            }
+        };
+        auto scatter_rest = [&](bool value) {          // what the registers do not hold
+            uint32_t a[kDecodeSlots];
+            float x[kDecodeSlots];
+            for (uint32_t i = first; i < rows; i += one ? 1u : 4u) {
+                const uint32_t c = one ? cnt : nnz[row0 + i];
+                for (uint32_t from = one ? kDecodeSlots * kstep : 0u; from < c; from += kDecodeSlots * kstep) {
+                    request(row0 + i, from, c, a, x);
+                    scatter(i, a, x, value);
+                }
+            }
+        };
+        __syncthreads();                               // the span is all zeros
+        if (one) scatter(0, at, v, true);
+        scatter_rest(true);
+        __syncthreads();
+        const uint32_t next = sp + gridDim.x;
+        uint32_t cnt_after = 0;
+        if (one && next < spans) {
+            uint32_t r1, c1;
+            rows_of(next, r1, c1);
+            request(r1, 0, cnt_next, at_next, v_next);
+            if (next + gridDim.x < spans) { rows_of(next + gridDim.x, r1, c1); cnt_after = nnz[r1]; }
+        }
+        for (uint32_t k = tid; k < count / 4u; k += 256u) __builtin_nontemporal_store(span4[k], reinterpret_cast<f32x4u *>(out) + k);
+        if (tid < (count & 3u)) out[(count & ~3u) + tid] = span[(count & ~3u) + tid];
+        __syncthreads();
+        if (one) scatter(0, at, v, false);
+        scatter_rest(false);
+        cnt = cnt_next;
+        cnt_next = cnt_after;
+#pragma unroll
+        for (uint32_t u = 0; u < kDecodeSlots; ++u) { at[u] = at_next[u]; v[u] = v_next[u]; }
     }
 }
 
@@ -631,53 +714,87 @@ void ellpack_decode_kernel(const float *__restrict__ Wd, const uint32_t *__restr
 namespace {
 
 // The encoder's counting pass leaves one partial result per workgroup -- the longest row and the
-// number of nonzeros among the workgroup's kEncodeRowsPerBlock rows -- in a scratch buffer; a
-// one-workgroup pass folds them into the buffer's header {r, total nnz (low, high), 0}, which the
-// packing pass reads on the device, so the row pitch of the output never travels through the host.
-// Layout of the scratch buffer: header (kEncodeHeaderBytes), then one uint2 {max, sum} per workgroup.
-constexpr uint32_t kEncodeRowsPerBlock = 16;      // 4 waves x 4 rows
+// number of nonzeros among the workgroup's rows -- in a scratch buffer; the packing pass folds them
+// (each workgroup for itself up to kEncodeFoldBlocks of them; beyond, a one-workgroup pass does it once)
+// into {r, total nnz}, so the row pitch of the output never travels through the host.
+// Layout of the scratch buffer: header {r, total nnz (low, high), 0} (kEncodeHeaderBytes), then one uint2
+// {max, sum} per workgroup.
+constexpr uint32_t kEncodeRowsPerBlock = 16;      // most rows of a counting workgroup: 4 waves x 4 rows
+constexpr uint32_t kEncodeFoldBlocks = 1024;      // partials a packing workgroup folds itself: 8 KB, four loads per thread
 constexpr uint32_t kEncodeMaxBlocks = 65536;      // workgroups whose partials the static scratch array holds
 constexpr uint32_t kEncodeHeaderBytes = 256;
 constexpr uint32_t kEncodeMaxCols = (1u << 28) - 1;     // the 16 rows of a workgroup, all dense, still count in 32 bits
 constexpr size_t kEncodeScratchBytes = kEncodeHeaderBytes + (size_t)kEncodeMaxBlocks * sizeof(uint2);
 static_assert(kEncodeScratchBytes <= kStaticScratchBytes, "the static scratch array holds the encoder's partials");
 
+// Rows per counting workgroup: with few rows the four waves of a workgroup share one, so that the chip is covered;
+// never more partials than kEncodeFoldBlocks up to 16 384 rows.
+static uint32_t encode_rows_per_block(uint32_t m) { return m <= 1024u ? 1u : m <= 4096u ? 4u : kEncodeRowsPerBlock; }
+
 static size_t encode_scratch_bytes(uint32_t m)
 {
-    return kEncodeHeaderBytes + (size_t)so_ceil_div(m, kEncodeRowsPerBlock) * sizeof(uint2);
+    return kEncodeHeaderBytes + (size_t)so_ceil_div(m, encode_rows_per_block(m)) * sizeof(uint2);
 }
 
-// Pass 1: one wave per row counts the entries with v != 0.0f; the workgroup's maximum and sum go
-// to partial[blockIdx.x].
+// Four consecutive elements of a row from column j on (zeros past its end).
+__device__ __forceinline__ f32x4u row_group(const float *wr, uint32_t j, uint32_t n)
+{
+    if (j + 4u <= n) return *reinterpret_cast<const f32x4u *>(wr + j);
+    f32x4u v = {0.f, 0.f, 0.f, 0.f};
+    if (j < n) v[0] = wr[j];
+    if (j + 1u < n) v[1] = wr[j + 1u];
+    if (j + 2u < n) v[2] = wr[j + 2u];
+    return v;
+}
+
+// Pass 1: counts the entries with v != 0.0f of every row, 16 bytes per lane and eight loads in flight; the
+// workgroup's maximum and sum go to partial[blockIdx.x].  Bound by the read of W: 8192 x 8192 in 43 us (6.2 TB/s;
+// one word per lane and load: 188).  `sharers` = 1: a wave per row; 4: the workgroup's waves share one row.
 __global__ __launch_bounds__(256)
 void ellpack_count_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, uint32_t *__restrict__ nnz,
-                          uint2 *__restrict__ partial)
+                          uint2 *__restrict__ partial, uint32_t rows_per_block, uint32_t sharers)
 {
     __shared__ uint32_t wmax[4], wsum[4];
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t part = sharers == 1u ? 0u : wave;
     uint32_t vmax = 0, vsum = 0;
-    for (uint32_t k = 0; k < kEncodeRowsPerBlock / 4u; ++k) {
-        const uint32_t row = blockIdx.x * kEncodeRowsPerBlock + k * 4u + wave;
-        if (row >= m) break;
+    for (uint32_t row = blockIdx.x * rows_per_block + (sharers == 1u ? wave : 0u); row < min(m, (blockIdx.x + 1u) * rows_per_block); row += 4u) {
         const float *wr = W + (size_t)row * n;
-        uint32_t c = 0;
-        for (uint32_t j = lane; j < n; j += 64u) c += wr[j] != 0.0f ? 1u : 0u;
+        uint32_t c = 0, j = part * 256u + lane * 4u;
+        const uint32_t step = sharers * 256u;
+        for (; j + 7u * step + 4u <= n; j += 8u * step) {
+            f32x4u v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const f32x4u *>(wr + j + u * step);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) c += v[u][e] != 0.0f ? 1u : 0u;
+        }
+        for (; j < n; j += step) {
+            const f32x4u v = row_group(wr, j, n);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c += v[e] != 0.0f ? 1u : 0u;
+        }
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
-        if (lane == 0) nnz[row] = c;
+        if (sharers == 1u && lane == 0) nnz[row] = c;
         vmax = max(vmax, c);
         vsum += c;
     }
     if (lane == 0) { wmax[wave] = vmax; wsum[wave] = vsum; }
     __syncthreads();
-    if (threadIdx.x == 0)
-        partial[blockIdx.x] = make_uint2(max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])),
-                                         wsum[0] + wsum[1] + wsum[2] + wsum[3]);
+    if (threadIdx.x == 0) {
+        const uint32_t sum = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+        if (sharers != 1u) nnz[blockIdx.x] = sum;
+        partial[blockIdx.x] = make_uint2(sharers != 1u ? sum : max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3])), sum);
+    }
 }
 
 // Folds the partials into header = {r, total nnz low word, high word, 0}.  One workgroup.
 __global__ __launch_bounds__(1024)
-void ellpack_count_fold_kernel(const uint2 *__restrict__ partial, uint32_t nblocks, uint32_t *__restrict__ header)
+void ellpack_count_fold_kernel(const uint2 *__restrict__ partial, uint32_t nblocks, uint32_t *__restrict__ header,
+                               uint32_t *__restrict__ host_header)
 {
     __shared__ uint32_t smax[16];
     __shared__ unsigned long long ssum[16];
@@ -701,65 +818,136 @@ void ellpack_count_fold_kernel(const uint2 *__restrict__ partial, uint32_t nbloc
         header[1] = (uint32_t)vsum;
         header[2] = (uint32_t)(vsum >> 32);
         header[3] = 0u;
+        if (host_header) { host_header[0] = vmax; host_header[1] = (uint32_t)vsum; host_header[2] = (uint32_t)(vsum >> 32); }
     }
 }
 
-// Pass 2: one wave per row packs (value, column) in ascending column order with row pitch
-// r = header[0], then zero-fills the row's remaining slots.  For each group of 64 columns the lanes
-// that hold a nonzero get consecutive slots (a prefix count over the wave's ballot), so the order
-// inside the row is the column order.  Writes nothing when r exceeds r_cap (the caller's arrays
-// hold m * r_cap slots); the wave that owns the last row also clears `tail_words` words after the
-// arrays' last slot.
+// Pass 2: packs (value, column) of every row in ascending column order with row pitch r, then zero-fills the
+// row's remaining slots.  A lane holds four consecutive elements of each group of 256; the place of an element is
+// the number of nonzeros in lower lanes (a prefix count over the wave's four ballots) plus those before it in its own
+// lane.  `sharers` = 4: the workgroup's waves take a quarter each of 8192 columns at a time and tell one another their
+// counts through LDS; 1: a wave per row.  Writes nothing when r exceeds r_cap (the caller's arrays hold m * r_cap
+// slots); the last row's owner also clears `tail_words` words after the arrays' last slot.  Rows are taken from the
+// last one back: the counting pass has left the end of W in the Infinity Cache.  `fold` != 0: r and the total come
+// from that many partials (the first workgroup leaves them in the header), else from the header.
+// Bound by the second read of W: 8192 x 8192, 90 % sparse, 90 -> 58 us (the whole encode, read-back included, 326 -> 127).
+template <int SHARERS>
 __global__ __launch_bounds__(256)
-void ellpack_pack_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, const uint32_t *__restrict__ header,
-                         uint32_t r_cap, const uint32_t *__restrict__ nnz, float *__restrict__ Wd,
-                         uint32_t *__restrict__ idx, uint32_t tail_words)
+void ellpack_pack_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, uint32_t *__restrict__ header, uint32_t fold,
+                         uint32_t *__restrict__ host_header, uint32_t r_cap, const uint32_t *__restrict__ nnz,
+                         float *__restrict__ Wd, uint32_t *__restrict__ idx, uint32_t tail_words)
 {
-    const uint32_t r = header[0];
+    constexpr uint32_t G = 8;                                // groups of 256 elements a wave holds at a time
+    __shared__ uint32_t smax[4], count[2][4];
+    __shared__ unsigned long long ssum[4];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    uint32_t r = 0;
+    if (fold == 0u) {
+        r = header[0];
+    } else {
+        const uint2 *partial = reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(header) + kEncodeHeaderBytes);
+        unsigned long long sum = 0;
+        for (uint32_t i = tid; i < fold; i += 256u) { const uint2 p = partial[i]; r = max(r, p.x); sum += p.y; }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) { r = max(r, (uint32_t)__shfl_xor(r, off, 64)); sum += __shfl_xor(sum, off, 64); }
+        if (lane == 0) { smax[wave] = r; ssum[wave] = sum; }
+        __syncthreads();
+        r = max(max(smax[0], smax[1]), max(smax[2], smax[3]));
+        if (blockIdx.x == 0 && tid == 0) {
+            sum = ssum[0] + ssum[1] + ssum[2] + ssum[3];
+            header[0] = r; header[1] = (uint32_t)sum; header[2] = (uint32_t)(sum >> 32); header[3] = 0u;
+            if (host_header) { host_header[0] = r; host_header[1] = (uint32_t)sum; host_header[2] = (uint32_t)(sum >> 32); }
+        }
+    }
     if (r > r_cap) return;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t nwaves = gridDim.x * 4u;
-    for (uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6); row < m; row += nwaves) {
+    const uint32_t part = SHARERS == 1 ? 0u : wave;
+    const uint32_t stride = SHARERS == 1 ? gridDim.x * 4u : gridDim.x;
+    uint32_t turn = 0;
+    for (uint32_t i = SHARERS == 1 ? blockIdx.x * 4u + wave : blockIdx.x; i < m; i += stride) {
+        const uint32_t row = m - 1u - i;
         const float *wr = W + (size_t)row * n;
         float *wd = Wd + (size_t)row * r;
         uint32_t *ix = idx + (size_t)row * r;
         uint32_t base = 0;
-        for (uint32_t j0 = 0; j0 < n; j0 += 64u) {
-            const uint32_t j = j0 + lane;
-            const float v = j < n ? wr[j] : 0.0f;
-            const bool keep = v != 0.0f;
-            const uint64_t mask = __ballot(keep);
-            if (keep) {
-                const uint32_t pos = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-                wd[pos] = v;
-                ix[pos] = j;
+        for (uint32_t j0 = 0; j0 < n; j0 += SHARERS * G * 256u) {
+            const uint32_t jw = j0 + part * (G * 256u) + lane * 4u;
+            f32x4u v[G];
+            if (j0 + (part + 1u) * (G * 256u) <= n) {
+#pragma unroll
+                for (uint32_t u = 0; u < G; ++u) v[u] = *reinterpret_cast<const f32x4u *>(wr + jw + u * 256u);
+            } else {
+#pragma unroll
+                for (uint32_t u = 0; u < G; ++u) v[u] = row_group(wr, jw + u * 256u, n);
             }
-            base += (uint32_t)__popcll(mask);
+            if constexpr (SHARERS != 1) {
+                uint32_t c = 0;
+#pragma unroll
+                for (uint32_t u = 0; u < G; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) c += (uint32_t)__popcll(__ballot(v[u][e] != 0.0f));
+                if (lane == 0) count[turn & 1u][wave] = c;
+                __syncthreads();
+            }
+            uint32_t at = base;
+            if constexpr (SHARERS != 1) {
+                const uint32_t *c = count[turn & 1u];
+                const uint32_t c0 = c[0], c1 = c[1], c2 = c[2], c3 = c[3];
+                at += wave == 0 ? 0u : wave == 1 ? c0 : wave == 2 ? c0 + c1 : c0 + c1 + c2;
+                base += c0 + c1 + c2 + c3;
+                ++turn;                                      // the other half of `count` next time: one barrier is enough
+            }
+            at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+            for (uint32_t u = 0; u < G; ++u) {
+                uint64_t mask[4];
+                uint32_t pos = at;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    mask[e] = __ballot(v[u][e] != 0.0f);
+                    pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask[e] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask[e], pos));
+                    at += (uint32_t)__popcll(mask[e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (v[u][e] != 0.0f) {
+                        wd[pos] = v[u][e];
+                        ix[pos] = jw + u * 256u + (uint32_t)e;
+                        ++pos;
+                    }
+            }
+            if constexpr (SHARERS == 1) base = at;
         }
-        const uint32_t end = row + 1 == m ? r + tail_words : r;
-        for (uint32_t k = nnz[row] + lane; k < end; k += 64u) { wd[k] = 0.0f; ix[k] = 0u; }
+        const uint32_t end = row + 1u == m ? r + tail_words : r;
+        for (uint32_t k = nnz[row] + (SHARERS == 1 ? lane : tid); k < end; k += SHARERS * 64u) { wd[k] = 0.0f; ix[k] = 0u; }
     }
 }
 
-// The three passes on the context's stream.  `scratch` holds encode_scratch_bytes(m) bytes; dWd and
-// dIdx hold m * r_cap slots (+ tail_words).
+// The passes on the context's stream.  `scratch` holds encode_scratch_bytes(m) bytes; dWd and dIdx hold
+// m * r_cap slots (+ tail_words).  `host_header` (pinned, may be null) receives r and the total once the stream has got there.
 so_status encode_launch(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, void *scratch, uint32_t r_cap,
-                        uint32_t *dNnz, float *dWd, uint32_t *dIdx, uint32_t tail_words, bool count, bool pack)
+                        uint32_t *dNnz, float *dWd, uint32_t *dIdx, uint32_t tail_words, bool count, bool pack, uint32_t *host_header)
 {
     uint32_t *header = (uint32_t *)scratch;
     uint2 *partial = (uint2 *)((char *)scratch + kEncodeHeaderBytes);
-    const uint32_t nblocks = so_ceil_div(m, kEncodeRowsPerBlock);
+    const uint32_t rpb = encode_rows_per_block(m), nblocks = so_ceil_div(m, rpb);
+    const bool fold_apart = !pack || m == 0 || nblocks > kEncodeFoldBlocks;
     if (count) {
         if (nblocks) {
-            ellpack_count_kernel<<<nblocks, 256, 0, ctx->stream>>>(dDense, m, n, dNnz, partial);
+            ellpack_count_kernel<<<nblocks, 256, 0, ctx->stream>>>(dDense, m, n, dNnz, partial, rpb, rpb == 1u ? 4u : 1u);
             SO_LAUNCH_CHECK();
         }
-        ellpack_count_fold_kernel<<<1, 1024, 0, ctx->stream>>>(partial, nblocks, header);
-        SO_LAUNCH_CHECK();
+        if (fold_apart) {
+            ellpack_count_fold_kernel<<<1, 1024, 0, ctx->stream>>>(partial, nblocks, header, host_header);
+            SO_LAUNCH_CHECK();
+        }
     }
     if (pack && m) {
-        const uint32_t blocks = std::max(1u, std::min(so_ceil_div(m, 4u), 16u * (uint32_t)ctx->compute_units));
-        ellpack_pack_kernel<<<blocks, 256, 0, ctx->stream>>>(dDense, m, n, header, r_cap, dNnz, dWd, dIdx, tail_words);
+        // A row of 1024 columns or more is shared by a workgroup's four waves.
+        const uint32_t fold = count && !fold_apart ? nblocks : 0u;
+        const bool shared = n >= 1024u;
+        const uint32_t blocks = std::max(1u, std::min(shared ? m : so_ceil_div(m, 4u), 16u * (uint32_t)ctx->compute_units));
+        if (shared) ellpack_pack_kernel<4><<<blocks, 256, 0, ctx->stream>>>(dDense, m, n, header, fold, host_header, r_cap, dNnz, dWd, dIdx, tail_words);
+        else ellpack_pack_kernel<1><<<blocks, 256, 0, ctx->stream>>>(dDense, m, n, header, fold, host_header, r_cap, dNnz, dWd, dIdx, tail_words);
         SO_LAUNCH_CHECK();
     }
     return SO_OK;
@@ -778,13 +966,13 @@ extern "C" so_status so_ellpack_encode(so_ctx *ctx, const float *dDense, uint32_
     E->m = m; E->n = n;
     E->layouts = SO_LAYOUT_ROW;
     void *p = nullptr, *scratch = nullptr;
-    uint32_t header[4] = {0, 0, 0, 0};
     so_status s = so_malloc(ctx, (size_t)m * sizeof(uint32_t) + 16, &p);
     if (s == SO_OK) { E->d_nnz = (uint32_t *)p; s = so_fill_zero(ctx, (char *)p + (size_t)m * sizeof(uint32_t), 16); }
     if (s == SO_OK) s = so_malloc(ctx, encode_scratch_bytes(m), &scratch);
-    if (s == SO_OK) s = encode_launch(ctx, dDense, m, n, scratch, 0, E->d_nnz, nullptr, nullptr, 0, true, false);
-    if (s == SO_OK) s = so_d2h(ctx, header, scratch, sizeof header);
+    if (s == SO_OK) s = encode_launch(ctx, dDense, m, n, scratch, 0, E->d_nnz, nullptr, nullptr, 0, true, false, ctx->h_encode_header);
+    if (s == SO_OK) s = so_stream_wait(ctx, "so_ellpack_encode");
     if (s == SO_OK) {
+        const uint32_t *header = ctx->h_encode_header;
         E->r = E->max_nnz = header[0];                   // r = longest row (src/ellpack_encoder.cpp:10-17)
         E->total_nnz = (uint64_t)header[1] | ((uint64_t)header[2] << 32);
         const size_t bytes = (size_t)m * E->r * sizeof(float) + 16;
@@ -797,7 +985,7 @@ extern "C" so_status so_ellpack_encode(so_ctx *ctx, const float *dDense, uint32_
         }
     }
     if (s == SO_OK && (size_t)m * E->r != 0)
-        s = encode_launch(ctx, dDense, m, n, scratch, E->r, E->d_nnz, E->d_Wd, E->d_idx, 4, false, true);
+        s = encode_launch(ctx, dDense, m, n, scratch, E->r, E->d_nnz, E->d_Wd, E->d_idx, 4, false, true, nullptr);
     if (scratch) {
         (void)hipStreamSynchronize(ctx->stream);
         (void)hipFree(scratch);
@@ -823,14 +1011,15 @@ extern "C" so_status so_ellpack_encode_noalloc(so_ctx *ctx, const float *dDense,
     SO_REQUIRE(m == 0 || dNnz != nullptr, "so_ellpack_encode_noalloc: dNnz is null");
     SO_REQUIRE((uint64_t)m * r_cap == 0 || (dWd != nullptr && dIdx != nullptr), "so_ellpack_encode_noalloc: dWd/dIdx is null");
     SO_REQUIRE(ctx->static_scratch != nullptr, "so_ellpack_encode_noalloc: the context has no scratch address");
+    const bool counts = r_out || total_nnz_out;
+    SO_REQUIRE(!counts || !ctx->capturing, "so_ellpack_encode_noalloc: r_out/total_nnz_out need a wait, which a graph recording forbids");
+    // The kernels leave the counts in pinned host memory themselves: no copy to queue behind them.
     const so_status s = encode_launch(ctx, dDense, m, n, ctx->static_scratch, r_cap, dNnz, dWd, dIdx, 0, true,
-                                      (uint64_t)m * r_cap != 0);
-    if (s != SO_OK || (!r_out && !total_nnz_out)) return s;
-    SO_REQUIRE(!ctx->capturing, "so_ellpack_encode_noalloc: r_out/total_nnz_out need a wait, which a graph recording forbids");
-    uint32_t header[4] = {0, 0, 0, 0};
-    SO_HIP(hipMemcpyAsync(header, ctx->static_scratch, sizeof header, hipMemcpyDeviceToHost, ctx->stream));
+                                      (uint64_t)m * r_cap != 0, counts ? ctx->h_encode_header : nullptr);
+    if (s != SO_OK || !counts) return s;
     const so_status waited = so_stream_wait(ctx, "so_ellpack_encode_noalloc");
     if (waited != SO_OK) return waited;
+    const uint32_t *header = ctx->h_encode_header;
     if (r_out) *r_out = header[0];
     if (total_nnz_out) *total_nnz_out = (uint64_t)header[1] | ((uint64_t)header[2] << 32);
     SO_REQUIRE(header[0] <= r_cap, "so_ellpack_encode_noalloc: the longest row has %u nonzeros, dWd/dIdx hold %u per row (nothing was packed)",
@@ -844,11 +1033,14 @@ extern "C" so_status so_ellpack_decode(so_ctx *ctx, const so_ellpack *E, float *
     const size_t total = (size_t)E->m * E->n;
     if (total == 0) return SO_OK;
     SO_REQUIRE(dDense != nullptr, "so_ellpack_decode: null output");
-    so_status s = so_fill_zero(ctx, dDense, total * sizeof(float));
-    if (s != SO_OK) return s;
-    if (E->r == 0) return SO_OK;
-    const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, 4u), 16u * (uint32_t)ctx->compute_units));
-    ellpack_decode_kernel<<<blocks, 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->m, E->n, E->r, dDense);
+    if (E->r == 0) return so_fill_zero(ctx, dDense, total * sizeof(float));
+    // Whole rows per span while they fit, but at least two spans per compute unit where the matrix has them.
+    const uint32_t per_row = so_ceil_div(E->n, kDecodeSpan);
+    const uint32_t rows = per_row > 1 ? 1u : std::max(1u, std::min(kDecodeSpan / E->n, so_ceil_div(E->m, 2u * (uint32_t)ctx->compute_units)));
+    const uint64_t spans = per_row > 1 ? (uint64_t)E->m * per_row : so_ceil_div(E->m, rows);
+    SO_REQUIRE(spans < (1ull << 32), "so_ellpack_decode: %u x %u is too large for one launch", E->m, E->n);
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(spans, 5ull * (uint64_t)ctx->compute_units);
+    ellpack_decode_kernel<<<blocks, 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->m, E->n, E->r, dDense, rows, (uint32_t)spans);
     SO_LAUNCH_CHECK();
     return SO_OK;
 }

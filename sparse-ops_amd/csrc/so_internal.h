@@ -46,6 +46,7 @@ struct so_ctx {
     uint32_t *d_wait_gave_up = nullptr;
     uint32_t *h_wait_gave_up = nullptr;
     bool waits_pending = false;
+    uint32_t *h_encode_header = nullptr;   // pinned: {r, total nnz (low, high)} of the last encode that asked for them
     float *mm_part = nullptr;
     size_t mm_part_bytes = 0;
     uint32_t *mm_counters = nullptr;
