@@ -913,6 +913,7 @@ extern "C" so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan)
     if (plan->d_taps) (void)hipFree(plan->d_taps);
     free_window(plan);
     so_conv_rbm_release(plan);
+    so_conv_columns_free(plan);
     delete plan;
     return SO_OK;
 }
@@ -920,31 +921,34 @@ extern "C" so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan)
 extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t B)
 {
     SO_REQUIRE(ctx && plan, "so_conv_plan_tune: null argument");
-    // The layout depends on the batch only through the number of batch tiles.
+    // The windowed layout depends on the batch only through the number of batch tiles: rebuilt only if the batch
+    // changes the batch tile the chunks are sized for or the choice of channels per wave.  A plan without the layout
+    // (the geometry did not suit the batch tile tried last) is tried again when the batch tile changes: a smaller tile
+    // holds more channels per chunk.  The column kernel's streams are for one batch.
     const uint32_t batch = std::max(4u, B / 4u * 4u);
-    if (batch == plan->tuned_batch) return SO_OK;
     const so_ellpack *E = plan->E;
     const uint32_t lpp = window_lpp(batch) ? window_lpp(batch) : kWinLPP;
-    // Rebuild only if the batch changes the batch tile the chunks are sized for or the choice of
-    // channels per wave.  A plan without the layout (the geometry did not suit the batch tile tried
-    // last) is tried again when the batch tile changes: a smaller tile holds more channels per chunk.
-    if (plan->win.cc == 0) {
-        if (lpp == plan->tried_lpp) { plan->tuned_batch = batch; return SO_OK; }
-    } else {
+    bool window = batch != plan->tuned_batch;
+    if (window && plan->win.cc == 0) window = lpp != plan->tried_lpp;
+    else if (window) {
         const double run = (double)E->total_nnz / (double)plan->g.Cout / plan->win.nch;
-        if (lpp == plan->win.lpp && choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) == plan->win.cpw) {
-            plan->tuned_batch = batch;
-            return SO_OK;
-        }
+        window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw;
     }
+    const bool columns = B <= kColMaxBatch && plan->col.batch != B;
+    plan->tuned_batch = batch;
+    if (!window && !columns) return SO_OK;
     const size_t slots = (size_t)E->m * E->r;
     std::vector<uint32_t> idx(slots), nnz(E->m);
     std::vector<float> Wd(slots);
     so_status s = so_ellpack_download(ctx, E, SO_LAYOUT_ROW, Wd.data(), idx.data(), nnz.data());
     if (s != SO_OK) return s;
     SO_HIP(hipStreamSynchronize(ctx->stream));      // no launch may still be reading the old arrays
+    if (columns) {
+        so_conv_columns_free(plan);
+        s = so_conv_columns_build(ctx, plan, idx, nnz, Wd, B);
+        if (s != SO_OK || !window) return s;
+    }
     free_window(plan);
-    plan->tuned_batch = batch;
     s = build_window(ctx, plan, idx, nnz, Wd, batch);
     if (s != SO_OK) return s;
     return so_conv_rbm_rebuild(ctx, plan);          // the record streams follow the window's chunks
@@ -969,6 +973,25 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     if (g.Cout == 0 || ncols == 0) return SO_OK;
     SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
     SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
+    // The column kernel where the plan has its streams for this batch: below four entries always (the windowed kernel
+    // does not take them), at four where its shorter chains on more waves win -- the windowed kernel's time there is
+    // about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (7x7x512 27.6 against 22.8 us, 14x14x256
+    // 17.5 against 24.4).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
+    if (plan->col.batch == B && B != 0 && ctx->tune.conv_columns != 0) {
+        bool use = B < 4 || plan->win.cc == 0 || ctx->tune.conv_columns == 1;
+        if (!use && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
+            const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw, B), (uint64_t)ctx->compute_units);
+            use = so_conv_columns_estimate(ctx, plan) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
+        }
+        if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for
+        bool done = false;
+        const so_status s = use ? so_conv_columns_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done) : SO_OK;
+        if (s != SO_OK) return s;
+        if (done) {
+            SO_LAUNCH_CHECK();
+            return SO_OK;
+        }
+    }
     // Batch entries per lane: as many as divide B and keep 16/8-byte alignment.
     const uintptr_t align = (uintptr_t)dX | (uintptr_t)dY | (uintptr_t)dResid;
     int maxvec = 4;

@@ -1,0 +1,328 @@
+// so_conv2d for small batches: a wave owns one output channel and 64 output columns, a column being one
+// (pixel, batch entry) pair.
+//
+// The LDS-windowed kernel (csrc/conv.hip) gives a lane four batch entries of a pixel, so a batch of one is carried as
+// four and a 7 x 7 layer of 512 channels keeps half of the chip's 1024 SIMDs busy with a quarter of their lanes.  Here
+// a lane is a column, whatever the batch: TH x TW output pixels x B entries on 64 lanes, one 4-byte LDS read and one
+// multiply-add per stored nonzero.  An output's multiply-adds form one chain in slot order (bias first), as everywhere
+// in this library's convolutions: same bits.
+//
+// Decomposition.  A workgroup of G (16, 8 or 4) waves takes G channels on one tile.  The tile's input window -- all
+// input channels if 150 KB of LDS hold them, else a chunk at a time -- is copied to LDS with zeros outside the image; a
+// channel's entries {weight, LDS offset of its tap} come 16 at a time in lanes (the same 16 in every row of 16), four
+// such groups ahead, and are handed round by DPP: per entry one address add, one read, one multiply-add.  The reads run
+// two quads of entries ahead of the multiply-adds.  Workgroups shrink to 8 or 4 waves where that spreads the launch
+// over more compute units.
+//
+// What bounds it: a wave's own chain.  An entry takes a wave on a SIMD of its own 28 clocks (add, read and multiply-add
+// each wait for the one before; four at a time, the adds between the multiply-adds), so the chains of 922 of a
+// ResNet-18-shaped 7 x 7 x 512 layer at 80 % are 11 of its 16 us; the rest is launch, first loads and the window's copy.
+#include "so_internal.h"
+#include "conv_internal.h"
+#include "dpp_steps.h"
+
+#include <cmath>
+#include <cstring>
+
+namespace {
+
+struct ColArgs {
+    uint32_t TH, TW, tiles_x;
+    uint32_t PE;                 // pixels of a window plane in LDS order (rows of IP pixels)
+    uint32_t IP, PL;             // row pitch in pixels; floats per plane (PE * B)
+    uint32_t cc, nch, G, waves;  // channels per chunk, chunks; computing waves (= channels) and waves of a workgroup
+    uint32_t sth, stw, sbh, sbw; // window pixels per output pixel, input pixels per window pixel
+    uint32_t mB, mIP, mPL, mTW, mTilesX;
+};
+
+// The four multiply-adds of one quad of entries (weights in lanes N1 .. N1 + 3 of w, operands in xf) between the four
+// address adds of another (offsets in lanes N0 .. of off), then that one's LDS reads (to xr): a multiply-add of the
+// chain may follow the one before it after 9 clocks, and the adds fill that time.
+template <int N0, int N1>
+__device__ __forceinline__ void step4(uint32_t base, uint32_t off, float (&xr)[4], float w, const float (&xf)[4], float &acc)
+{
+    uint32_t p0, p1, p2, p3;
+    asm("v_add_u32_dpp %[p0], %[off], %[base] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x0] row_newbcast:%[m0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p1], %[off], %[base] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x1] row_newbcast:%[m1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p2], %[off], %[base] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x2] row_newbcast:%[m2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p3], %[off], %[base] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x3] row_newbcast:%[m3] row_mask:0xf bank_mask:0xf"
+        : [p0] "=&v"(p0), [p1] "=&v"(p1), [p2] "=&v"(p2), [p3] "=&v"(p3), [acc] "+v"(acc)
+        : [off] "v"(off), [base] "v"(base), [w] "v"(w), [x0] "v"(xf[0]), [x1] "v"(xf[1]), [x2] "v"(xf[2]), [x3] "v"(xf[3]),
+          [n0] "n"(N0), [n1] "n"(N0 + 1), [n2] "n"(N0 + 2), [n3] "n"(N0 + 3), [m0] "n"(N1), [m1] "n"(N1 + 1), [m2] "n"(N1 + 2), [m3] "n"(N1 + 3));
+    typedef const float __attribute__((address_space(3))) *lds_float;
+    xr[0] = *(lds_float)p0;
+    xr[1] = *(lds_float)p1;
+    xr[2] = *(lds_float)p2;
+    xr[3] = *(lds_float)p3;
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int N1>
+__device__ __forceinline__ void fma4(float w, const float (&x)[4], float &acc)
+{
+    so_dpp::fmac_bcast<N1>(acc, w, x[0]);
+    so_dpp::fmac_bcast<N1 + 1>(acc, w, x[1]);
+    so_dpp::fmac_bcast<N1 + 2>(acc, w, x[2]);
+    so_dpp::fmac_bcast<N1 + 3>(acc, w, x[3]);
+}
+
+template <int ACT>
+__global__ __launch_bounds__(1024)
+void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__restrict__ first_group, ColArgs a, so_conv_geom g,
+                          const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
+                          const float *__restrict__ resid, float *__restrict__ Y)
+{
+    extern __shared__ __attribute__((aligned(16))) float window[];     // [cc + 1][PL]: the last plane all zeros (padding entries point there)
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, threads = a.waves * 64u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t co = blockIdx.y * a.G + wave;
+    const bool computes = wave < a.G && co < g.Cout;                   // the other waves only help copying
+    const uint32_t tile_y = window_div(blockIdx.x, a.tiles_x, a.mTilesX);
+    const uint32_t th0 = tile_y * a.TH, tw0 = (blockIdx.x - tile_y * a.tiles_x) * a.TW;
+
+    // the wave's entries, groups of 16 (the stream ends with eight padding groups)
+    const uint32_t *__restrict__ first = first_group + (size_t)(computes ? co : 0u) * a.nch;
+    const int2 *__restrict__ ep = entries + (lane & 15u);
+    int2 cur[4], nxt[4];
+
+    // this lane's output column
+    const uint32_t pix = window_div(lane, B, a.mB), b = lane - pix * B;
+    const uint32_t ty = window_div(pix, a.TW, a.mTW), tx = pix - ty * a.TW;
+    const bool live = computes && pix < a.TH * a.TW && th0 + ty < g.H_out && tw0 + tx < g.W_out;
+    const uint32_t lane_off = live ? ((ty * a.sth * a.IP + tx * a.stw) * B + b) * 4u : 0u;
+    float acc = bias && computes ? bias[co] : 0.0f;
+
+    for (uint32_t k = tid; k < a.PL; k += threads) window[a.cc * a.PL + k] = 0.0f;
+    // Input channels [t * cc, t * cc + cc) of the window, straight from memory into LDS: consecutive threads take
+    // consecutive places -- of several planes at once where a plane is shorter than the workgroup -- and step over
+    // channels; places outside the image are written with zeros instead.
+    const bool several = a.PL < threads;
+    const uint32_t per_pass = several ? window_div(threads, a.PL, a.mPL) : 1u;
+    const uint32_t plane = several ? window_div(tid, a.PL, a.mPL) : 0u;
+    const uint32_t image = g.H_in * g.W_in * B;
+    const uint32_t lds0 = so_lds::lds_address(window) + wave * 256u;
+    auto copy_window = [&](uint32_t t) {
+        const uint32_t c0 = t * a.cc, cn = min(a.cc, g.Cin - c0);
+        if (plane >= per_pass) return;
+        uint32_t to = lds0;
+        for (uint32_t e = tid - plane * a.PL; e < a.PL; e += threads, to += threads * 4u) {
+            const uint32_t pe = window_div(e, B, a.mB), be = e - pe * B;
+            const uint32_t ih = window_div(pe, a.IP, a.mIP), iw = pe - ih * a.IP;
+            const int32_t gh = (int32_t)(th0 * g.stride_h + ih * a.sbh) - (int32_t)g.pad_h;
+            const int32_t gw = (int32_t)(tw0 * g.stride_w + iw * a.sbw) - (int32_t)g.pad_w;
+            if ((uint32_t)gh < g.H_in && (uint32_t)gw < g.W_in) {
+                const uint32_t from = (plane * image + ((uint32_t)gh * g.W_in + (uint32_t)gw) * B + be) * 4u;
+                const float *src = X + (size_t)c0 * image;
+                // the last pass may hold fewer planes than this thread's
+                const uint32_t whole = cn / per_pass * per_pass;
+                uint32_t m0 = to;
+                for (uint32_t c = 0; c < whole; c += per_pass) {
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(m0), "v"(from), "s"(src) : "memory", "m0");
+                    src += (size_t)per_pass * image;
+                    m0 += per_pass * a.PL * 4u;
+                }
+                if (whole + plane < cn)
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(m0), "v"(from), "s"(src) : "memory", "m0");
+            } else {
+                for (uint32_t c = plane; c < cn; c += per_pass) window[c * a.PL + e] = 0.0f;
+            }
+        }
+    };
+    const uint32_t base = so_lds::lds_address(window) + lane_off;
+    // Quads 2 and 3 of the group before this one still owe their multiply-adds: operands in xA, xB, weights in owed.
+    float xA[4] = {0.f, 0.f, 0.f, 0.f}, xB[4] = {0.f, 0.f, 0.f, 0.f}, xC[4], xD[4], owed = -0.0f;
+    auto group = [&](const int2 &e) {
+        float w = __int_as_float(e.x);
+        uint32_t off = (uint32_t)e.y;
+        asm volatile("s_nop 4" : "+v"(w), "+v"(off), "+v"(owed));      // DPP operands: not within two cycles of a vector write
+        step4<0, 8>(base, off, xC, owed, xA, acc);
+        step4<4, 12>(base, off, xD, owed, xB, acc);
+        step4<8, 0>(base, off, xA, w, xC, acc);
+        step4<12, 4>(base, off, xB, w, xD, acc);
+        owed = w;
+    };
+    for (uint32_t t = 0; t < a.nch; ++t) {
+        if (t) __syncthreads();                                        // every wave has read what it needs of the last chunk
+        copy_window(t);
+        const uint32_t g0 = __builtin_amdgcn_readfirstlane(first[t]), g1 = computes ? __builtin_amdgcn_readfirstlane(first[t + 1u]) : 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) cur[i] = ep[(size_t)(g0 + i) * 16u];
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");             // this thread's part of the window is in LDS
+        __syncthreads();
+        for (uint32_t gi = g0; gi < g1; gi += 4u) {
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) nxt[i] = ep[(size_t)(gi + 4u + i) * 16u];
+            group(cur[0]);
+            if (gi + 1u < g1) group(cur[1]);
+            if (gi + 2u < g1) group(cur[2]);
+            if (gi + 3u < g1) group(cur[3]);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) cur[i] = nxt[i];
+        }
+    }
+    asm volatile("s_nop 4" : "+v"(owed));
+    fma4<8>(owed, xA, acc);
+    fma4<12>(owed, xB, acc);
+
+    if (live) {
+        const size_t at = (((size_t)co * g.H_out + th0 + ty) * g.W_out + tw0 + tx) * B + b;
+        if (resid) acc += resid[at];
+        Y[at] = so_epilogue<ACT>(acc);
+    }
+}
+
+template <int ACT>
+void launch_columns(so_ctx *ctx, const so_conv_plan *plan, const ColArgs &a, dim3 grid, size_t lds, const float *dX, uint32_t B,
+                    const float *dBias, const float *dResid, float *dY)
+{
+    conv2d_column_kernel<ACT><<<grid, a.waves * 64u, lds, ctx->stream>>>(plan->col.d_entries, plan->col.d_first, a, plan->g, dX, B, dBias, dResid, dY);
+}
+
+constexpr uint64_t kColLds = 150 * 1024;
+
+} // namespace
+
+void so_conv_columns_free(so_conv_plan *plan)
+{
+    if (plan->col.d_entries) (void)hipFree(plan->col.d_entries);
+    if (plan->col.d_first) (void)hipFree(plan->col.d_first);
+    plan->col = so_conv_columns();
+}
+
+// Sizes the tile for batch B and uploads the entry streams; leaves the plan without them where the kernel does not apply.
+so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
+                                const std::vector<float> &Wd, uint32_t B)
+{
+    const so_conv_geom &g = plan->g;
+    const so_ellpack *E = plan->E;
+    if (B == 0 || B > kColMaxBatch || E->r == 0 || E->total_nnz == 0 || !E->ascending || (size_t)ctx->max_lds_bytes < kColLds) return SO_OK;
+    so_conv_columns c;
+    const uint32_t px = 64u / B, sth = window_step(g.kH, g.stride_h), stw = window_step(g.kW, g.stride_w);
+    uint64_t best_tiles = ~0ull, best_win = ~0ull;
+    for (uint32_t th = 1; th <= px && th <= g.H_out; ++th)
+        for (uint32_t tw = 1; th * tw <= px && tw <= g.W_out; ++tw) {
+            const uint64_t tiles = (uint64_t)so_ceil_div(g.H_out, th) * so_ceil_div(g.W_out, tw);
+            const uint64_t win = (uint64_t)((th - 1) * sth + (g.kH - 1) * g.dil_h + 1) * ((tw - 1) * stw + (g.kW - 1) * g.dil_w + 1);
+            if (tiles < best_tiles || (tiles == best_tiles && win < best_win)) { best_tiles = tiles; best_win = win; c.TH = th; c.TW = tw; }
+        }
+    if (c.TH == 0) return SO_OK;
+    c.tiles_x = so_ceil_div(g.W_out, c.TW);
+    c.tiles_y = so_ceil_div(g.H_out, c.TH);
+    const uint32_t IH = (c.TH - 1) * sth + (g.kH - 1) * g.dil_h + 1, IW = (c.TW - 1) * stw + (g.kW - 1) * g.dil_w + 1;
+    // A tile as wide as the image whose first and last window columns both lie outside it: the last column of a row and
+    // the first of the next, zeros both, share their place (7 x 7 x 512: 147 KB instead of 166, one chunk instead of two).
+    const bool share = c.tiles_x == 1 && IW > 1 && g.pad_w >= 1 && g.kW > 1 && (uint64_t)IW - 1 >= (uint64_t)g.W_in + g.pad_w;
+    c.IP = share ? IW - 1 : IW;
+    c.PE = (IH - 1) * c.IP + IW;
+    const uint64_t plane = (uint64_t)c.PE * B;
+    if (plane * 4 * 2 > kColLds) return SO_OK;
+    c.cc = (uint32_t)std::min<uint64_t>(g.Cin, kColLds / (plane * 4) - 1);
+    c.nch = so_ceil_div(g.Cin, c.cc);
+    c.cc = so_ceil_div(g.Cin, c.nch);
+    // window_div: operand * divisor below 2^32
+    if ((uint64_t)c.tiles_x * c.tiles_x * c.tiles_y >= (1ull << 32) || plane * plane >= (1ull << 32) || plane * 1024 >= (1ull << 32)) return SO_OK;
+    if ((uint64_t)c.tiles_x * c.tiles_y >= (1ull << 31) || ((uint64_t)c.cc + 1024) * g.H_in * g.W_in * B >= (1ull << 30)) return SO_OK;
+    const uint32_t kHW = g.kH * g.kW;
+    std::vector<uint32_t> first((size_t)E->m * c.nch + 1);
+    std::vector<int2> entries;
+    entries.reserve((size_t)E->total_nnz + (size_t)E->m * c.nch * 8 + 128);
+    uint32_t pad_bits;
+    const float neg_zero = -0.0f;
+    std::memcpy(&pad_bits, &neg_zero, 4);
+    const int2 pad = make_int2((int)pad_bits, (int)(c.cc * plane * 4));
+    for (uint32_t co = 0; co < E->m; ++co) {
+        uint32_t j = 0;
+        for (uint32_t t = 0; t < c.nch; ++t) {
+            first[(size_t)co * c.nch + t] = (uint32_t)(entries.size() / 16);
+            for (; j < nnz[co]; ++j) {
+                const size_t slot = (size_t)co * E->r + j;
+                const uint32_t k = idx[slot], cin = k / kHW, kh = (k / g.kW) % g.kH, kw = k % g.kW;
+                if (cin >= (t + 1) * c.cc) break;
+                uint32_t wb;
+                std::memcpy(&wb, &Wd[slot], 4);
+                entries.push_back(make_int2((int)wb, (int)(((uint64_t)(cin - t * c.cc) * plane + (uint64_t)(kh * g.dil_h * c.IP + kw * g.dil_w) * B) * 4)));
+            }
+            while (entries.size() % 16) entries.push_back(pad);
+        }
+    }
+    first.back() = (uint32_t)(entries.size() / 16);
+    if (entries.size() / 16 > 0xfffffff0ull) return SO_OK;
+    entries.resize(entries.size() + 128, pad);
+    for (const void *k : {(const void *)conv2d_column_kernel<SO_ACT_NONE>, (const void *)conv2d_column_kernel<SO_ACT_RELU>,
+                          (const void *)conv2d_column_kernel<SO_ACT_SIGMOID>, (const void *)conv2d_column_kernel<SO_ACT_TANH>})
+        SO_HIP(so_allow_big_lds(ctx, k));
+    void *p = nullptr;
+    so_status s = so_malloc(ctx, entries.size() * sizeof(int2), &p);
+    if (s != SO_OK) return s;
+    c.d_entries = (int2 *)p;
+    if ((s = so_malloc(ctx, first.size() * 4, &p)) == SO_OK) {
+        c.d_first = (uint32_t *)p;
+        s = so_h2d(ctx, c.d_entries, entries.data(), entries.size() * sizeof(int2));
+        if (s == SO_OK) s = so_h2d(ctx, c.d_first, first.data(), first.size() * 4);
+    }
+    c.batch = B;
+    plan->col = c;
+    if (s != SO_OK) so_conv_columns_free(plan);
+    return s;
+}
+
+namespace {
+
+struct ColShape { uint32_t G, waves; size_t lds; double us; };
+
+// Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
+// longest chain at 12 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
+// more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 9.0 us, 28x28x128 10.2, 14x14x256
+// 10.4, 7x7x512 16; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
+ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan)
+{
+    const so_conv_columns &c = plan->col;
+    const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
+    ColShape best{16, 16, 0, 1e30};
+    for (uint32_t G = 16; G >= 4; G /= 2) {
+        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0};
+        s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
+        const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
+        const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
+        const double rounds = std::ceil(wgs / (cus * fit)), resident = std::min(fit, std::ceil(wgs / cus));
+        s.us = 3.0 + rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.012, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        if (s.us < best.us) best = s;
+    }
+    return best;
+}
+
+} // namespace
+
+double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan) { return column_shape(ctx, plan).us; }
+
+so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
+                                 const float *dResid, float *dY, int act, bool *done)
+{
+    const so_conv_columns &c = plan->col;
+    const so_conv_geom &g = plan->g;
+    *done = false;
+    if (c.batch != B) return SO_OK;
+    ColArgs a;
+    a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch;
+    a.sth = window_step(g.kH, g.stride_h); a.stw = window_step(g.kW, g.stride_w);
+    a.sbh = window_subsample(g.kH, g.stride_h); a.sbw = window_subsample(g.kW, g.stride_w);
+    a.mB = window_magic(B); a.mIP = window_magic(a.IP); a.mPL = window_magic(a.PL); a.mTW = window_magic(a.TW); a.mTilesX = window_magic(a.tiles_x);
+    const uint64_t tiles = (uint64_t)c.tiles_x * c.tiles_y;
+    const ColShape shape = column_shape(ctx, plan);
+    a.G = shape.G;
+    a.waves = shape.waves;
+    const size_t lds = shape.lds;
+    const dim3 grid((uint32_t)tiles, so_ceil_div(g.Cout, a.G));
+    if (grid.y > 65535u) return SO_OK;
+    switch (act) {
+    case SO_ACT_RELU:    launch_columns<SO_ACT_RELU>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
+    case SO_ACT_SIGMOID: launch_columns<SO_ACT_SIGMOID>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
+    case SO_ACT_TANH:    launch_columns<SO_ACT_TANH>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
+    default:             launch_columns<SO_ACT_NONE>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
+    }
+    *done = true;
+    return SO_OK;
+}

@@ -22,12 +22,13 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
     M.has_conv = false;
     for (const LayerPlan &L : M.layers) M.has_conv |= L.conv != nullptr;
     // The convolutions work on batch tiles of 16, 8 or 4 entries, and the larger the tile the less a
-    // batch entry costs: a batch is carried in rows of 4 (up to 4 entries), 8 (up to 8) or the next
+    // batch entry costs: a batch is carried in rows of 4 (2 to 4 entries), 8 (up to 8) or the next
     // multiple of 16 (the extra columns are zeros on input and are never copied out; batch entries
     // do not interact).  Measured on a ResNet-18-shaped stack: 12 entries as 12 0.86 ms, as 16
-    // 0.76 ms; 24 as 24 1.31 ms, as 32 1.24 ms.
+    // 0.76 ms; 24 as 24 1.31 ms, as 32 1.24 ms.  A single entry has a kernel of its own: 0.35 ms as 4, 0.25 as 1
+    // (two entries as 2: 0.34).
     uint32_t pbatch = batch;
-    if (M.has_conv) pbatch = batch <= 4 ? 4u : batch <= 8 ? 8u : (batch + 15u) / 16u * 16u;
+    if (M.has_conv && batch > 1) pbatch = batch <= 4 ? 4u : batch <= 8 ? 8u : (batch + 15u) / 16u * 16u;
     // Slot offsets for this batch, 256-byte aligned.
     std::size_t total = 0;
     std::size_t widest = std::max(M.in_features, M.out_features);
@@ -137,6 +138,7 @@ void SparseOnnxModel::run_batch_major(const float *input, uint32_t B, float *out
 {
     Impl &M = *impl_;
     if (B != M.batch) const_cast<SparseOnnxModel *>(this)->resize_buffers(B);
+    if (B == 1) { run(input, B, output); return; }      // one sample is the same in either order
     so_ctx *ctx = context();
     std::lock_guard<std::mutex> lock(context_mutex());
     check(so_h2d(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float)), "so_h2d(input)");

@@ -1,0 +1,55 @@
+"""The column kernel for small batches (csrc/conv_columns.hip) on plans tuned for the batch, bit for bit against the
+oracle: tiles and planes that are no multiple of anything, a window larger than the workgroup, several channel chunks,
+rows whose padding columns share a place, strides on 1-wide axes, dilation, empty and dense channels, the residual form,
+padding entries that must not turn an infinity in the input into a NaN."""
+
+import numpy as np
+import pytest
+
+from conftest import as_oracle, sparse_matrix
+
+import datagen
+import hipabi
+
+pytestmark = pytest.mark.gpu
+
+CASES = [  # Cin, Cout, H, W, kernel, stride, pad, dilation, sparsity
+    (3, 5, 7, 9, (3, 3), (1, 1), (1, 1), (1, 1), .5), (1, 1, 1, 1, (1, 1), (1, 1), (0, 0), (1, 1), .0), (20, 33, 7, 7, (3, 3), (1, 1), (1, 1), (1, 1), .8),
+    (3, 16, 33, 31, (7, 7), (2, 2), (3, 3), (1, 1), .8), (40, 24, 13, 14, (3, 3), (2, 2), (1, 1), (1, 1), .7), (64, 48, 14, 14, (1, 1), (2, 2), (0, 0), (1, 1), .8),
+    (7, 6, 12, 20, (3, 2), (1, 3), (2, 0), (2, 1), .3), (5, 9, 17, 5, (1, 5), (3, 1), (0, 2), (1, 1), .5), (600, 20, 7, 7, (3, 3), (1, 1), (1, 1), (1, 1), .9),
+    (900, 12, 8, 9, (3, 3), (1, 1), (1, 1), (1, 1), .95), (6, 8, 30, 30, (9, 9), (3, 3), (4, 4), (2, 2), .6)]
+
+
+@pytest.mark.parametrize("Cin,Cout,H,Wi,k,s,p,d,sp", CASES)
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+def test_columns_match_oracle(ctx, oracle, Cin, Cout, H, Wi, k, s, p, d, sp, B):
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin * 31 + Cout + H * 7 + B)
+    Wc = sparse_matrix(rng, Cout, Cin * k[0] * k[1], sp)
+    if Cout > 4:
+        Wc[2] = 0
+        Wc[4] = rng.standard_normal(Wc.shape[1])
+    E = datagen.encode_dense(Wc)
+    g, og = hipabi.conv_geom(Cin, Cout, k[0], k[1], H, Wi, s, p, d), ocg(Cin, Cout, k[0], k[1], H, Wi, s, p, d)
+    X = rng.standard_normal((Cin, H, Wi, B)).astype(np.float32)
+    R = rng.standard_normal((Cout, g.H_out, g.W_out, B)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    with ctx.tuning(SPARSEOPS_CONV_COLUMNS="1"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+        plan = ctx.conv_plan(dE, g)
+        ctx.conv_plan_tune(plan, B)
+        dX, dY, dB, dR = ctx.array(X), ctx.empty(R.shape), ctx.array(b), ctx.array(R)
+        for residual in (None, dR):
+            dY.upload(np.full(R.shape, np.nan, np.float32))
+            ctx.conv2d(plan, dX, B, dB, dY, "relu", residual=residual)
+            want = oracle.conv2d_pf(as_oracle(E), og, X, B, b, "none")
+            want = np.maximum(want if residual is None else want + R, 0)
+            assert np.array_equal(dY.download(), want)
+        X[0, 0, 0, 0] = np.inf
+        dX.upload(X)
+        ctx.conv2d(plan, dX, B, dB, dY, "none")
+        want = oracle.conv2d_pf(as_oracle(E), og, X, B, b, "none")
+        assert np.array_equal(dY.download(), want, equal_nan=True)
+        ctx.conv_plan_free(plan)
+        for a in (dX, dY, dB, dR, dE):
+            a.free()
