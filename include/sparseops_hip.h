@@ -122,6 +122,12 @@ so_status so_malloc(so_ctx *ctx, size_t bytes, void **dptr);
 so_status so_free(so_ctx *ctx, void *dptr);
 so_status so_h2d(so_ctx *ctx, void *dst, const void *src, size_t bytes); /* waits */
 so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t bytes); /* waits */
+/* The same for calls that keep their operands in host memory, without a wait per array: so_stage_in copies up to
+ * two host arrays (the second may be null, with 0 bytes) to pinned memory and queues the rest of the way on the
+ * context's stream; it returns with the host arrays free for reuse and the device arrays valid for later work on that
+ * stream.  so_stage_out queues a device array's way back, waits for it and reports as so_d2h does. */
+so_status so_stage_in(so_ctx *ctx, void *dst, const void *src, size_t bytes, void *dst2, const void *src2, size_t bytes2);
+so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes);
 so_status so_d2d(so_ctx *ctx, void *dst, const void *src, size_t bytes);
 so_status so_fill_zero(so_ctx *ctx, void *dptr, size_t bytes); /* fill kernel, graph-safe */
 /* Waits for the context's stream.  The LDS-staged kernels synchronise their waves through counters

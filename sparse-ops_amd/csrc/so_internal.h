@@ -48,6 +48,11 @@ struct so_ctx {
     uint32_t *h_wait_gave_up = nullptr;
     bool waits_pending = false;
     uint32_t *h_encode_header = nullptr;   // pinned: {r, total nnz (low, high)} of the last encode that asked for them
+    // Staging of host arrays (so_stage_in, so_stage_out): pinned memory, the flag of the last way out in it, its bytes in use
+    char *h_stage = nullptr;
+    uint32_t *d_stage_done = nullptr;      // workgroups of a way out that have finished
+    size_t stage_used = 0;
+    uint32_t stage_turn = 0;
     float *mm_part = nullptr;
     size_t mm_part_bytes = 0;
     uint32_t *mm_counters = nullptr;

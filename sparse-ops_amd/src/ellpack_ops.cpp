@@ -17,6 +17,16 @@ Staging &staging()
     return *s;
 }
 
+// X (its device buffer is reserved) and the bias, if there is one, on their way to the device; the bias there.
+const float *stage_operands(so_ctx *ctx, const float *X, std::size_t xbytes, const float *bias, uint32_t m)
+{
+    Staging &st = staging();
+    const std::size_t bias_bytes = bias ? std::size_t(m) * sizeof(float) : 0;
+    if (bias) st.bias.reserve(bias_bytes);
+    sparseops::check(so_stage_in(ctx, st.x.get(), X, xbytes, bias ? st.bias.get() : nullptr, bias, bias_bytes), "so_stage_in(X, bias)");
+    return bias ? st.bias.f32() : nullptr;
+}
+
 } // namespace
 
 namespace sparseops {
@@ -52,15 +62,9 @@ void matmul_host(const Ellpack &E, const float *X, uint32_t C, const float *bias
     const std::size_t ybytes = std::size_t(E.m) * C * sizeof(float);
     st.x.reserve(xbytes);
     st.y.reserve(ybytes);
-    check(so_h2d(ctx, st.x.get(), X, xbytes), "so_h2d(X)");
-    const float *dBias = nullptr;
-    if (bias) {
-        st.bias.reserve(std::size_t(E.m) * sizeof(float));
-        check(so_h2d(ctx, st.bias.get(), bias, std::size_t(E.m) * sizeof(float)), "so_h2d(bias)");
-        dBias = st.bias.f32();
-    }
+    const float *dBias = stage_operands(ctx, X, xbytes, bias, E.m);
     check(so_matmul(ctx, dE, st.x.f32(), C, dBias, st.y.f32(), act), "so_matmul");
-    check(so_d2h(ctx, Y, st.y.get(), ybytes), "so_d2h(Y)");
+    check(so_stage_out(ctx, Y, st.y.get(), ybytes), "so_stage_out(Y)");
 }
 
 } // namespace
@@ -95,13 +99,7 @@ void ellpack_matvec(const Ellpack &E, const float *x, const float *bias, float *
     Staging &st = staging();
     st.x.reserve(std::size_t(E.n) * sizeof(float));
     st.y.reserve(std::size_t(E.m) * sizeof(float));
-    check(so_h2d(ctx, st.x.get(), x, std::size_t(E.n) * sizeof(float)), "so_h2d(x)");
-    const float *dBias = nullptr;
-    if (bias) {
-        st.bias.reserve(std::size_t(E.m) * sizeof(float));
-        check(so_h2d(ctx, st.bias.get(), bias, std::size_t(E.m) * sizeof(float)), "so_h2d(bias)");
-        dBias = st.bias.f32();
-    }
+    const float *dBias = stage_operands(ctx, x, std::size_t(E.n) * sizeof(float), bias, E.m);
     check(so_matvec(ctx, dE, st.x.f32(), dBias, st.y.f32(), 0), "so_matvec");
-    check(so_d2h(ctx, y, st.y.get(), std::size_t(E.m) * sizeof(float)), "so_d2h(y)");
+    check(so_stage_out(ctx, y, st.y.get(), std::size_t(E.m) * sizeof(float)), "so_stage_out(y)");
 }

@@ -20,9 +20,9 @@ void act_inplace(int act, float *data, std::size_t len)
     if (len == 0) return;
     static DeviceBuffer &buf = *new DeviceBuffer();      // grow-only, lives as long as the context (never destroyed)
     buf.reserve(len * sizeof(float));
-    check(so_h2d(ctx, buf.get(), data, len * sizeof(float)), "so_h2d");
+    check(so_stage_in(ctx, buf.get(), data, len * sizeof(float), nullptr, nullptr, 0), "so_stage_in");
     check(so_act(ctx, act, buf.f32(), len, buf.f32()), "so_act");
-    check(so_d2h(ctx, data, buf.get(), len * sizeof(float)), "so_d2h");
+    check(so_stage_out(ctx, data, buf.get(), len * sizeof(float)), "so_stage_out");
 }
 
 bool rows_ascend(const Ellpack &E)
@@ -81,29 +81,26 @@ void conv_any(const ConvAttr &c, const float *src, uint32_t B, float *dst, Layou
     M.in.reserve(in * sizeof(float));
     M.out.reserve(out * sizeof(float));
     if (layout != Layout::PatchMajor) M.staged.reserve(std::max(in, out) * sizeof(float));
-    if (layout == Layout::PatchMajor) {
-        check(so_h2d(ctx, M.in.get(), src, in * sizeof(float)), "so_h2d(src)");
-    } else {
-        check(so_h2d(ctx, M.staged.get(), src, in * sizeof(float)), "so_h2d(src)");
+    const std::size_t bias_bytes = c.bias_ptr ? std::size_t(c.Cout) * sizeof(float) : 0;
+    if (bias_bytes) M.bias.reserve(bias_bytes);
+    check(so_stage_in(ctx, layout == Layout::PatchMajor ? M.in.get() : M.staged.get(), src, in * sizeof(float), bias_bytes ? M.bias.get() : nullptr,
+                      c.bias_ptr, bias_bytes), "so_stage_in(src, bias)");
+    if (layout != Layout::PatchMajor) {
         if (layout == Layout::COrder)        // (B, C*H*W) row-major -> [C*H*W][B]
             check(so_transpose(ctx, M.staged.f32(), B, uint32_t(in / B), M.in.f32()), "so_transpose");
         else                                 // Fortran (B,C,H,W) is [W][H][C][B] in memory
             check(so_reverse_axes3(ctx, M.staged.f32(), c.W_in, c.H_in, c.Cin, B, M.in.f32()), "so_reverse_axes3");
     }
-    if (c.bias_ptr) {
-        M.bias.reserve(std::size_t(c.Cout) * sizeof(float));
-        check(so_h2d(ctx, M.bias.get(), c.bias_ptr, std::size_t(c.Cout) * sizeof(float)), "so_h2d(bias)");
-    }
     check(so_conv2d(ctx, M.plan, M.in.f32(), B, c.bias_ptr ? M.bias.f32() : nullptr, M.out.f32(),
                     c.fuse_relu ? SO_ACT_RELU : SO_ACT_NONE), "so_conv2d");
     if (layout == Layout::PatchMajor) {
-        check(so_d2h(ctx, dst, M.out.get(), out * sizeof(float)), "so_d2h(dst)");
+        check(so_stage_out(ctx, dst, M.out.get(), out * sizeof(float)), "so_stage_out(dst)");
     } else {
         if (layout == Layout::COrder)
             check(so_transpose(ctx, M.out.f32(), uint32_t(out / B), B, M.staged.f32()), "so_transpose");
         else
             check(so_reverse_axes3(ctx, M.out.f32(), c.Cout, c.H_out, c.W_out, B, M.staged.f32()), "so_reverse_axes3");
-        check(so_d2h(ctx, dst, M.staged.get(), out * sizeof(float)), "so_d2h(dst)");
+        check(so_stage_out(ctx, dst, M.staged.get(), out * sizeof(float)), "so_stage_out(dst)");
     }
 }
 

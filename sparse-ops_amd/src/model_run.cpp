@@ -122,16 +122,16 @@ void SparseOnnxModel::run(const float *input, uint32_t B, float *output) const
     so_ctx *ctx = context();
     std::lock_guard<std::mutex> lock(context_mutex());
     if (!M.padded()) {
-        check(so_h2d(ctx, M.slot_ptr(M.input_slot), input, M.in_features * B * sizeof(float)), "so_h2d(input)");
+        check(so_stage_in(ctx, M.slot_ptr(M.input_slot), input, M.in_features * B * sizeof(float), nullptr, nullptr, 0), "so_stage_in(input)");
         M.launch_chain();
-        check(so_d2h(ctx, output, M.slot_ptr(M.output_slot), M.out_features * B * sizeof(float)), "so_d2h(output)");
+        check(so_stage_out(ctx, output, M.slot_ptr(M.output_slot), M.out_features * B * sizeof(float)), "so_stage_out(output)");
         return;
     }
-    check(so_h2d(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float)), "so_h2d(input)");
+    check(so_stage_in(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float), nullptr, nullptr, 0), "so_stage_in(input)");
     M.rows_in(M.stage_in.f32());
     M.launch_chain();
     M.rows_out(M.stage_out.f32());
-    check(so_d2h(ctx, output, M.stage_out.get(), M.out_features * B * sizeof(float)), "so_d2h(output)");
+    check(so_stage_out(ctx, output, M.stage_out.get(), M.out_features * B * sizeof(float)), "so_stage_out(output)");
 }
 
 void SparseOnnxModel::run_batch_major(const float *input, uint32_t B, float *output) const
@@ -141,7 +141,7 @@ void SparseOnnxModel::run_batch_major(const float *input, uint32_t B, float *out
     if (B == 1) { run(input, B, output); return; }      // one sample is the same in either order
     so_ctx *ctx = context();
     std::lock_guard<std::mutex> lock(context_mutex());
-    check(so_h2d(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float)), "so_h2d(input)");
+    check(so_stage_in(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float), nullptr, nullptr, 0), "so_stage_in(input)");
     if (!M.padded()) {
         check(so_transpose(ctx, M.stage_in.f32(), B, uint32_t(M.in_features), M.slot_ptr(M.input_slot)), "so_transpose(input)");
         M.launch_chain();
@@ -153,7 +153,7 @@ void SparseOnnxModel::run_batch_major(const float *input, uint32_t B, float *out
         M.rows_out(M.stage_mid.f32());
         check(so_transpose(ctx, M.stage_mid.f32(), uint32_t(M.out_features), B, M.stage_out.f32()), "so_transpose(output)");
     }
-    check(so_d2h(ctx, output, M.stage_out.get(), M.out_features * B * sizeof(float)), "so_d2h(output)");
+    check(so_stage_out(ctx, output, M.stage_out.get(), M.out_features * B * sizeof(float)), "so_stage_out(output)");
 }
 
 void SparseOnnxModel::run_device(const float *dInput, uint32_t B, float *dOutput) const
