@@ -275,7 +275,8 @@ static bool stage_ready(so_ctx *ctx)
     if (ctx->h_stage) return true;
     void *p = nullptr, *d = nullptr;
     if (hipHostMalloc(&p, kStageFlag + 64, hipHostMallocCoherent) != hipSuccess) { (void)hipGetLastError(); return false; }
-    if (hipMalloc(&d, 64) != hipSuccess || hipMemset(d, 0, 64) != hipSuccess) {
+    // cleared on the context's stream, which does not wait for the null stream
+    if (hipMalloc(&d, 64) != hipSuccess || so_fill_zero(ctx, d, 64) != SO_OK) {
         (void)hipGetLastError();
         if (d) (void)hipFree(d);
         (void)hipHostFree(p);
