@@ -149,12 +149,13 @@ __device__ __forceinline__ float group_row_dot(const float *__restrict__ Wd, con
 
 // G lanes per row: a wave works on 64/G rows at a time (whole waves for rows longer than 512
 // slots, a half, a quarter or an eighth of a wave for shorter ones, so that short rows do not leave lanes idle).
-template <bool XLDS, int G, bool I16>
+// ACT: with an activation (so_matmul's products with a single column).
+template <bool XLDS, int G, bool I16, bool ACT>
 __global__ __launch_bounds__(kBlock)
 void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ idx,
                         const uint32_t *__restrict__ nnz, uint32_t count, uint32_t r,
                         const float *__restrict__ x, uint32_t n,
-                        const float *__restrict__ bias, float *__restrict__ y)
+                        const float *__restrict__ bias, float *__restrict__ y, int act)
 {
     extern __shared__ float lds_x[];
     constexpr uint32_t RPW = 64 / G;                                     // rows per wave
@@ -191,7 +192,12 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
             }
         }
         const float s = group_sum<G>((a0 + a1) + (a2 + a3));
-        if (sub == 0 && row < count) y[row] = (bias ? bias[row] : 0.0f) + s;
+        if (sub == 0 && row < count) {
+            float v = (bias ? bias[row] : 0.0f) + s;
+            if (ACT) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
+                       : act == SO_ACT_TANH ? so_epilogue<SO_ACT_TANH>(v) : v;
+            y[row] = v;
+        }
         cur = nxt;
         beg = nbeg;
         end = nend;
@@ -372,7 +378,53 @@ bool use_lds(so_ctx *ctx, K kernel, uint32_t n, uint64_t nnz_total, uint32_t blo
     return true;
 }
 
+// The row kernel on the row-major arrays, on the 16-bit columns when the handle has them.
+template <bool ACT>
+void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, int act)
+{
+    const uint32_t cus = (uint32_t)ctx->compute_units;
+    const size_t lds = (size_t)E->n * sizeof(float);
+    const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
+    const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
+    // Lanes per row by the longest row (one pass of 16 G slots should cover it), but never so
+    // few that compute units are left without rows.
+    uint32_t G = E->max_nnz <= 128 ? 8u : E->max_nnz <= 256 ? 16u : E->max_nnz <= 512 ? 32u : 64u;
+    if (ctx->tune.matvec_lanes) G = (uint32_t)ctx->tune.matvec_lanes;
+    else
+        while (G < 64 && so_ceil_div(E->m, kWavesPerBlock * (64u / G)) < cus) G *= 2;
+    // One resident workgroup per compute unit (the pipelined rows need the registers); each of
+    // its 16 waves keeps two passes' loads in flight.
+    const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
+#define SO_MV_ROWS(G, I16)                                                                                         \
+    do {                                                                                                       \
+        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, ACT>, E->n, E->total_nnz, blocks))                        \
+            matvec_rows_kernel<true, G, I16, ACT><<<blocks, kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
+                                                                                   dx, E->n, dBias, dy, act);       \
+        else                                                                                                   \
+            matvec_rows_kernel<false, G, I16, ACT><<<blocks, kBlock, 0, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
+                                                                                  dx, E->n, dBias, dy, act);        \
+    } while (0)
+#define SO_MV_ROWS_G(I16)                                                                                          \
+    do {                                                                                                       \
+        if (G == 8) SO_MV_ROWS(8, I16);                                                                        \
+        else if (G == 16) SO_MV_ROWS(16, I16);                                                                 \
+        else if (G == 32) SO_MV_ROWS(32, I16);                                                                 \
+        else SO_MV_ROWS(64, I16);                                                                              \
+    } while (0)
+    if (i16) SO_MV_ROWS_G(true);
+    else SO_MV_ROWS_G(false);
+#undef SO_MV_ROWS_G
+#undef SO_MV_ROWS
+}
+
 } // namespace
+
+so_status so_matvec_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, int act)
+{
+    if (act == SO_ACT_NONE) launch_rows<false>(ctx, E, dx, dBias, dy, act);
+    else launch_rows<true>(ctx, E, dx, dBias, dy, act);
+    return SO_OK;
+}
 
 extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx,
                                const float *dBias, float *dy, int layout)
@@ -404,35 +456,7 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
     const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
     const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
     if (layout == SO_LAYOUT_ROW) {
-        // Lanes per row by the longest row (one pass of 16 G slots should cover it), but never so
-        // few that compute units are left without rows.
-        uint32_t G = E->max_nnz <= 128 ? 8u : E->max_nnz <= 256 ? 16u : E->max_nnz <= 512 ? 32u : 64u;
-        if (ctx->tune.matvec_lanes) G = (uint32_t)ctx->tune.matvec_lanes;
-        else
-            while (G < 64 && so_ceil_div(E->m, kWavesPerBlock * (64u / G)) < cus) G *= 2;
-        // One resident workgroup per compute unit (the pipelined rows need the registers); each of
-        // its 16 waves keeps two passes' loads in flight.
-        const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
-#define SO_MV_ROWS(G, I16)                                                                                         \
-        do {                                                                                                       \
-            if (use_lds(ctx, matvec_rows_kernel<true, G, I16>, E->n, E->total_nnz, blocks))                        \
-                matvec_rows_kernel<true, G, I16><<<blocks, kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
-                                                                                       dx, E->n, dBias, dy);       \
-            else                                                                                                   \
-                matvec_rows_kernel<false, G, I16><<<blocks, kBlock, 0, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
-                                                                                      dx, E->n, dBias, dy);        \
-        } while (0)
-#define SO_MV_ROWS_G(I16)                                                                                          \
-        do {                                                                                                       \
-            if (G == 8) SO_MV_ROWS(8, I16);                                                                        \
-            else if (G == 16) SO_MV_ROWS(16, I16);                                                                 \
-            else if (G == 32) SO_MV_ROWS(32, I16);                                                                 \
-            else SO_MV_ROWS(64, I16);                                                                              \
-        } while (0)
-        if (i16) SO_MV_ROWS_G(true);
-        else SO_MV_ROWS_G(false);
-#undef SO_MV_ROWS_G
-#undef SO_MV_ROWS
+        launch_rows<false>(ctx, E, dx, dBias, dy, SO_ACT_NONE);
     } else if (layout == SO_LAYOUT_SLOT) {
         const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kBlock), 2u * cus));
 #define SO_MV_SLOT(T, COLS)                                                                                        \

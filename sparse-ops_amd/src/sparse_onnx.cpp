@@ -459,7 +459,11 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     // Large fully connected layers run on the row-block-merged kernel (fp32 round-off accuracy, the fastest);
     // SPARSEOPS_MATMUL_RBM=0 at load time keeps every layer on the kernels that give the reference's bits.
     const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM");
-    const bool fast_fc = !(rbm_env && rbm_env[0] == '0');
+    // So does a batch below 64 in a model with convolutions: there every sample has the same bits whatever batch it
+    // travels in, and its classifier is a few microseconds of the pass.
+    bool convs = false;
+    for (const auto &p : pend) convs = convs || p.plan.op == Op::Conv;
+    const bool fast_fc = !(rbm_env && rbm_env[0] == '0') && !(convs && B0 < 64);
     for (auto &p : pend) {
         if (p.plan.op != Op::MatMul && p.plan.op != Op::Conv) continue;
         p.plan.dE = mirror(*p.plan.E, p.plan.op == Op::MatMul ? matmul_layouts(*p.plan.E, uint32_t(B0), fast_fc) : SO_LAYOUT_ROW);

@@ -104,6 +104,23 @@ def test_mlp_config4(backend, oracle, tmp_path):
     assert np.array_equal(model.run(X), Y)               # deterministic across replays
 
 
+@pytest.mark.parametrize("B,dims", [(3, (700, 1030, 600, 9)), (4, (700, 1030, 600, 9)), (5, (515, 512, 513)), (33, (1100, 700, 520)), (63, (700, 1030, 600))])
+def test_mlp_wide_layers_at_small_batches(backend, ctx, oracle, tmp_path, B, dims):
+    """Large layers take the quad-union kernel from 4 columns on and so_matvec's row kernel at one, whatever batch the
+    model was loaded at.
+    Bound: the sums are those of the layout's kernels, 1e-5 of the largest value (tests/test_gpu_matmul_quad.py) per layer;
+    the activations' slopes are at most 1 and a layer's gain here about 1, so the layers' errors add up at most."""
+    rng = np.random.default_rng(B)
+    Ws = [datagen.magnitude_prune((rng.standard_normal((o, i)) / np.sqrt(.4 * i)).astype(np.float32), .6) for i, o in zip(dims[:-1], dims[1:])]
+    acts = (["Relu", "Tanh", None] if len(Ws) == 3 else ["Relu", None])
+    model = backend.SparseOnnxModel(ow.save(str(tmp_path / "mlp.onnx"), ow.mlp_model(Ws, acts, B)))
+    for b in (B, 1, B, 70):
+        X = rng.standard_normal((b, dims[0])).astype(np.float32)
+        Y, Yo = model.run(X), oracle_mlp(oracle, Ws, acts, X)
+        assert rel_err(Y, Yo) <= 1e-5 * len(Ws), b
+        assert np.array_equal(_run_device(model, ctx, X), Y)
+
+
 def cnn_model(rng, B, H=16):
     """The reference's full_test.py topology (tests/full_test.py:21-41):
     Conv3x3 -> ReLU -> MaxPool -> {Conv3x3 -> ReLU, Conv1x1} -> Add -> GAP -> Flatten -> FC -> ReLU,
