@@ -293,16 +293,18 @@ enum class RbmKernel { None, Merged, Quad, Vector };
 //   kernel moves 256 bytes per nonzero and 64 columns at about 11 TB/s, and a row takes 18 ns per nonzero on its own;
 //   quad against row-block-merged: 4096 x 4096 x 256 at 90 / 80 / 70 / 50 % 45 / 60 / 72 / 91 against 29 / 48 / 65 / 97
 //   -- 2.85 us per million (nonzero, 64 columns) on top of 9.5, and no faster on fewer workgroups than compute units.
-//   One column: so_matvec's row kernel, which spreads a row over the lanes, from rows of 64 nonzeros.  The row kernel has
-//   one lane at work and fetches a line of X per nonzero.  Longest row, us row kernel / that one: 4096 x 4096 1756 101.8 / 9.1,
-//   479 19.7 / 4.8, 159 7.9 / 4.1, 69 4.6 / 4.0; 1024 x 4096 62 3.7 / 3.7; 4096 x 512 23 3.5 / 3.9; 10 x 512 63 4.0 / 3.2, 16 3.2 / 3.4.
+//   One to three columns: so_matvec's row kernel on each, which spreads a row over the lanes, from rows of 64 nonzeros
+//   per column.  The row kernel has C lanes at work and fetches a line of X per nonzero.  Longest row, us row kernel /
+//   that one: one column, 4096 x 4096 1756 101.8 / 9.1, 479 19.7 / 4.8, 159 7.9 / 4.1, 69 4.6 / 4.0; 1024 x 4096
+//   62 3.7 / 3.7; 4096 x 512 23 3.5 / 3.9; 10 x 512 63 4.0 / 3.2, 16 3.2 / 3.4; two, 4096 x 4096 487 19.6 / 8.4, 162
+//   7.8 / 7.4; 10 x 512 262 6.0 / 3.4; three, 4096 x 4096 1759 114 / 27, 487 19.7 / 13.1; 4096 x 1024 244 11.0 / 10.4.
 RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const bool merged = so_matmul_rbm_applies(ctx, E, C), quad = so_matmul_quad_applies(ctx, E, C);
     if (merged && ctx->tune.matmul_rbm == 1) return RbmKernel::Merged;
     if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
     if (quad && ctx->tune.matmul_quad == 1) return RbmKernel::Quad;
-    if (C == 1 && E->max_nnz >= 64) return RbmKernel::Vector;
+    if (C <= 3 && E->max_nnz >= 64u * C) return RbmKernel::Vector;
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
     double best = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
@@ -351,7 +353,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
         const RbmKernel k = rbm_kernel(ctx, E, C);
         if (k != RbmKernel::None) {
             const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, dX, C, dBias, dY, act)
-                               : k == RbmKernel::Vector ? so_matvec_rows(ctx, E, dX, dBias, dY, act)
+                               : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();

@@ -61,11 +61,16 @@ __device__ __forceinline__ float group_sum(float v)
     return v;
 }
 
-// Stage x in LDS (XLDS) or read it through the cache hierarchy.
+// Stage x in LDS (XLDS) or read it through the cache hierarchy.  `pitch`: floats from one element of x to the next.
 template <bool XLDS>
-__device__ __forceinline__ const float *stage_x(const float *__restrict__ x, uint32_t n, float *lds)
+__device__ __forceinline__ const float *stage_x(const float *__restrict__ x, uint32_t n, float *lds, uint32_t pitch = 1u)
 {
     if (!XLDS) return x;
+    if (pitch != 1u) {
+        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) lds[i] = x[(size_t)i * pitch];
+        __syncthreads();
+        return lds;
+    }
     const uint32_t n4 = ((reinterpret_cast<uintptr_t>(x) & 15u) == 0) ? n / 4 : 0;     // 16-byte copies when x is aligned
     for (uint32_t i = threadIdx.x; i < n4; i += blockDim.x)
         reinterpret_cast<float4 *>(lds)[i] = reinterpret_cast<const float4 *>(x)[i];
@@ -101,7 +106,7 @@ __device__ __forceinline__ void row_issue(const f32x4 *__restrict__ Wd4, const t
 
 template <int G, bool I16>
 __device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg, uint64_t end, uint64_t q0, const float *xs,
-                                            float &a0, float &a1, float &a2, float &a3)
+                                            float &a0, float &a1, float &a2, float &a3, size_t pitch = 1)
 {
     // slot k of group u is live iff its distance from the row's start is in [0, end - beg): one
     // unsigned 32-bit comparison (a slot before the row gives a huge distance)
@@ -113,8 +118,8 @@ __device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg
         const bool v0 = (uint32_t)rel < len, v1 = (uint32_t)(rel + 1) < len;
         const bool v2 = (uint32_t)(rel + 2) < len, v3 = (uint32_t)(rel + 3) < len;
         const u32x4 c = ColGroup<I16>::cols(L.c[u]);
-        const float x0 = xs[v0 ? c.x : 0u], x1 = xs[v1 ? c.y : 0u];
-        const float x2 = xs[v2 ? c.z : 0u], x3 = xs[v3 ? c.w : 0u];
+        const float x0 = xs[(v0 ? c.x : 0u) * pitch], x1 = xs[(v1 ? c.y : 0u) * pitch];
+        const float x2 = xs[(v2 ? c.z : 0u) * pitch], x3 = xs[(v3 ? c.w : 0u) * pitch];
         a0 = __builtin_fmaf(v0 ? L.w[u].x : 0.0f, v0 ? x0 : 0.0f, a0);
         a1 = __builtin_fmaf(v1 ? L.w[u].y : 0.0f, v1 ? x1 : 0.0f, a1);
         a2 = __builtin_fmaf(v2 ? L.w[u].z : 0.0f, v2 ? x2 : 0.0f, a2);
@@ -149,13 +154,14 @@ __device__ __forceinline__ float group_row_dot(const float *__restrict__ Wd, con
 
 // G lanes per row: a wave works on 64/G rows at a time (whole waves for rows longer than 512
 // slots, a half, a quarter or an eighth of a wave for shorter ones, so that short rows do not leave lanes idle).
-// ACT: with an activation (so_matmul's products with a single column).
-template <bool XLDS, int G, bool I16, bool ACT>
+// MM: so_matmul's products with few columns, one of the row-major X and Y per blockIdx.y (their rows `C` floats apart),
+// with an activation.
+template <bool XLDS, int G, bool I16, bool MM>
 __global__ __launch_bounds__(kBlock)
 void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ idx,
                         const uint32_t *__restrict__ nnz, uint32_t count, uint32_t r,
                         const float *__restrict__ x, uint32_t n,
-                        const float *__restrict__ bias, float *__restrict__ y, int act)
+                        const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act)
 {
     extern __shared__ float lds_x[];
     constexpr uint32_t RPW = 64 / G;                                     // rows per wave
@@ -173,7 +179,9 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
     uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
     RowLoads<I16> cur, nxt;
     if (row < count) row_issue<G, I16>(Wd4, idx4, beg, end, (beg >> 2) + sub, cur);
-    const float *xs = stage_x<XLDS>(x, n, lds_x);
+    const uint32_t pitch = MM ? C : 1u;
+    const float *xs = stage_x<XLDS>(MM ? x + blockIdx.y : x, n, lds_x, pitch);
+    const size_t xpitch = MM && !XLDS ? C : 1u;
     // all groups of a wave make the same number of trips (the reductions need every lane)
     for (uint32_t base = wave * RPW; base < count; base += stride, row += stride) {
         const uint64_t nrow = (uint64_t)row + stride;
@@ -184,19 +192,19 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
         if (row < count && end > beg) {
             const uint64_t qlast = (end - 1) >> 2;
             uint64_t q0 = (beg >> 2) + sub;
-            row_consume<G, I16>(cur, beg, end, q0, xs, a0, a1, a2, a3);
+            row_consume<G, I16>(cur, beg, end, q0, xs, a0, a1, a2, a3, xpitch);
             for (q0 += 4 * G; q0 <= qlast; q0 += 4 * G) {        // rows longer than one pass
                 RowLoads<I16> more;
                 row_issue<G, I16>(Wd4, idx4, beg, end, q0, more);
-                row_consume<G, I16>(more, beg, end, q0, xs, a0, a1, a2, a3);
+                row_consume<G, I16>(more, beg, end, q0, xs, a0, a1, a2, a3, xpitch);
             }
         }
         const float s = group_sum<G>((a0 + a1) + (a2 + a3));
         if (sub == 0 && row < count) {
             float v = (bias ? bias[row] : 0.0f) + s;
-            if (ACT) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
+            if (MM) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
                        : act == SO_ACT_TANH ? so_epilogue<SO_ACT_TANH>(v) : v;
-            y[row] = v;
+            y[MM ? (size_t)row * C + blockIdx.y : row] = v;
         }
         cur = nxt;
         beg = nbeg;
@@ -379,8 +387,8 @@ bool use_lds(so_ctx *ctx, K kernel, uint32_t n, uint64_t nnz_total, uint32_t blo
 }
 
 // The row kernel on the row-major arrays, on the 16-bit columns when the handle has them.
-template <bool ACT>
-void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, int act)
+template <bool MM>
+void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, const float *dBias, float *dy, int act)
 {
     const uint32_t cus = (uint32_t)ctx->compute_units;
     const size_t lds = (size_t)E->n * sizeof(float);
@@ -397,12 +405,12 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float 
     const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
 #define SO_MV_ROWS(G, I16)                                                                                         \
     do {                                                                                                       \
-        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, ACT>, E->n, E->total_nnz, blocks))                        \
-            matvec_rows_kernel<true, G, I16, ACT><<<blocks, kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
-                                                                                   dx, E->n, dBias, dy, act);       \
+        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, MM>, E->n, E->total_nnz, blocks))                        \
+            matvec_rows_kernel<true, G, I16, MM><<<dim3(blocks, C), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
+                                                                                   dx, E->n, dBias, dy, C, act);       \
         else                                                                                                   \
-            matvec_rows_kernel<false, G, I16, ACT><<<blocks, kBlock, 0, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
-                                                                                  dx, E->n, dBias, dy, act);        \
+            matvec_rows_kernel<false, G, I16, MM><<<dim3(blocks, C), kBlock, 0, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
+                                                                                  dx, E->n, dBias, dy, C, act);        \
     } while (0)
 #define SO_MV_ROWS_G(I16)                                                                                          \
     do {                                                                                                       \
@@ -419,10 +427,9 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float 
 
 } // namespace
 
-so_status so_matvec_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, int act)
+so_status so_matvec_columns(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
-    if (act == SO_ACT_NONE) launch_rows<false>(ctx, E, dx, dBias, dy, act);
-    else launch_rows<true>(ctx, E, dx, dBias, dy, act);
+    launch_rows<true>(ctx, E, dX, C, dBias, dY, act);
     return SO_OK;
 }
 
@@ -456,7 +463,7 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
     const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
     const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
     if (layout == SO_LAYOUT_ROW) {
-        launch_rows<false>(ctx, E, dx, dBias, dy, SO_ACT_NONE);
+        launch_rows<false>(ctx, E, dx, 1, dBias, dy, SO_ACT_NONE);
     } else if (layout == SO_LAYOUT_SLOT) {
         const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kBlock), 2u * cus));
 #define SO_MV_SLOT(T, COLS)                                                                                        \

@@ -177,8 +177,8 @@ so_status so_matmul_rbm_launch(so_ctx *ctx, const so_ellpack *E, const float *dX
 // Grows the context's matmul workspace (partial tiles, a zeroed counter per tile).  Never while a graph is being recorded.
 so_status so_matmul_workspace(so_ctx *ctx, size_t part_bytes, size_t counter_bytes);
 
-// csrc/matvec.hip: the row kernel of so_matvec with an activation.
-so_status so_matvec_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, int act);
+// csrc/matvec.hip: the row kernel of so_matvec on each of C columns, with an activation.
+so_status so_matvec_columns(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
 
 // csrc/matmul_quad.hip: the quad-union layout and its kernel.
 so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz);

@@ -42,9 +42,9 @@ int matmul_layouts(const Ellpack &E, uint32_t C, bool fast)
     if (!big) return SO_LAYOUT_ROW;
     // The layout's quad-union kernel is ahead of the K-tiled one below the row-block-merged kernel's sizes as well
     // (4096 x 784 x 256 at 90 %: 12.0 us against 15.2) and, from the 4 columns it needs, of the row kernel, which
-    // fetches a line of X per nonzero however few of its columns there are; a single column goes to so_matvec's kernel.
-    // At any C: the batch may grow after the load.  MLP 784-4096-4096-4096-10 host to host, batch 1 / 4 / 16 / 48: 117 / 116 /
-    // 118 / 125 us with ROW alone, 39 / 67 / 69 / 75 now.
+    // fetches a line of X per nonzero however few of its columns there are; up to three columns go to so_matvec's kernel.
+    // At any C: the batch may grow after the load.  MLP 784-4096-4096-4096-10 host to host, batch 1 / 2 / 3 / 4 / 16 / 48:
+    // 117 / 117 / 118 / 116 / 118 / 125 us with ROW alone, 39 / 57 / 66 / 67 / 69 / 75 now.
     if (fast) return SO_LAYOUT_ROW | SO_LAYOUT_RBM;
     if (C < 64) return SO_LAYOUT_ROW;
     return C % 4 == 0 ? (SO_LAYOUT_ROW | SO_LAYOUT_TILED) : SO_LAYOUT_ROW;

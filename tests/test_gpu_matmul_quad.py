@@ -110,3 +110,36 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         for a in (dX, dY):
             a.free()
         dE.free()
+
+
+@pytest.mark.parametrize("m,n,C,sp", [(1, 64, 1, .0), (5, 4097, 3, .5), (16, 70, 1, .0), (130, 513, 2, .5), (257, 700, 3, .7), (1000, 1025, 1, .8),
+                                      (65, 50000, 2, .99), (4100, 300, 3, .3)])
+@pytest.mark.parametrize("act", ["none", "relu", "sigmoid", "tanh"])
+@pytest.mark.parametrize("idx16", [False, True])
+def test_few_columns_on_the_matvec_kernel(ctx, oracle, m, n, C, sp, act, idx16):
+    """One to three columns: a row over the lanes of a wave or a part of one, x in LDS or not, an infinity in X in the rows
+    that use it only.  The activations' slopes are at most 1: the sums' bound carries over, plus the device functions' 1e-6."""
+    rng = np.random.default_rng(m + n)
+    W = sparse_matrix(rng, m, n, sp)
+    if m > 4:
+        W[m // 2] = 0
+    W[0, 0] = 1.0
+    E = datagen.encode_dense(W)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM | (hipabi.LAYOUT_IDX16 if idx16 else 0))
+    dX, dY, dB = ctx.array(X), ctx.empty((m, C)), ctx.array(b)
+    pre = np.abs(W.astype(np.float64) @ X + b[:, None]).max()
+    for special in (False, True):
+        if special:
+            X[0, C - 1] = np.inf
+            dX.upload(X)
+        dY.upload(np.full((m, C), np.nan, np.float32))
+        ctx.matmul(dE, dX, C, dB, dY, act)
+        Y, Yo = dY.download(), oracle.matmul(as_oracle(E), X, b, act)
+        fin = np.isfinite(Yo)
+        assert np.array_equal(Y[~fin], Yo[~fin], equal_nan=True)
+        assert np.abs(Y[fin] - Yo[fin]).max(initial=0.0) <= TOL * pre + 1e-6
+    for a in (dX, dY, dB):
+        a.free()
+    dE.free()

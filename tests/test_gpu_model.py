@@ -106,7 +106,7 @@ def test_mlp_config4(backend, oracle, tmp_path):
 
 @pytest.mark.parametrize("B,dims", [(3, (700, 1030, 600, 9)), (4, (700, 1030, 600, 9)), (5, (515, 512, 513)), (33, (1100, 700, 520)), (63, (700, 1030, 600))])
 def test_mlp_wide_layers_at_small_batches(backend, ctx, oracle, tmp_path, B, dims):
-    """Large layers take the quad-union kernel from 4 columns on and so_matvec's row kernel at one, whatever batch the
+    """Large layers take the quad-union kernel from 4 columns on and so_matvec's row kernel below, whatever batch the
     model was loaded at.
     Bound: the sums are those of the layout's kernels, 1e-5 of the largest value (tests/test_gpu_matmul_quad.py) per layer;
     the activations' slopes are at most 1 and a layer's gain here about 1, so the layers' errors add up at most."""
