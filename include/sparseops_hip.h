@@ -315,7 +315,9 @@ so_status so_copy_rows(so_ctx *ctx, const float *dSrc, size_t src_stride, uint32
  * Record every launch made on the context between begin and end into one
  * hipGraph, then replay it with a single submission (SparseOnnxModel::run uses
  * this for layer chains of eight layers or more, src/model_run.cpp:28-127).  No allocation, copy to
- * or from the host, or timer call may happen while recording. */
+ * or from the host, or timer call may happen while recording.  A graph keeps so_matmul's workspace of
+ * the time of its recording, so later launches may grow the context's; the handles, plans and arrays
+ * that were recorded must outlive it. */
 typedef struct so_graph so_graph;
 so_status so_graph_begin(so_ctx *ctx);
 so_status so_graph_end(so_ctx *ctx, so_graph **out);

@@ -491,7 +491,8 @@ so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *d
     const so_quads &Q = E->quads;
     const uint32_t per_xcd = so_ceil_div((uint64_t)p.rbs * p.nslab * p.ks, 8);
     const QuadArgs a{Q.d_w, Q.d_off, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, p.qw_log2, p.ks, p.tiles_per, p.nslab, p.rbs, per_xcd,
-                     dX, dBias, dY, ctx->mm_part, ctx->mm_counters, E->d_Wd, E->d_idx, E->d_nnz, E->r};
+                     dX, dBias, dY, ctx->mm_part ? (float *)ctx->mm_part->p : nullptr,
+                     ctx->mm_counters ? (uint32_t *)ctx->mm_counters->p : nullptr, E->d_Wd, E->d_idx, E->d_nnz, E->r};
     const uint32_t blocks = 8u * per_xcd;
     switch (act) {
     case SO_ACT_RELU:    return launch_quad<SO_ACT_RELU>(ctx, a, blocks);

@@ -198,7 +198,8 @@ so_status launch_rbm(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t
     const uint32_t nslabs = so_ceil_div(C, 64);
     const uint32_t blocks = so_ceil_div(R.nb, 8 / R.ksplit) * 8 * nslabs;      // ksplit is 1, 2 or 4
     ellpack_matmul_rbm_kernel<ACT><<<blocks, NW * 64, LDS_BYTES, ctx->stream>>>(
-        R.d_hdr, R.d_rec, R.d_w, R.nrec, E->m, E->n, R.nb, R.ksplit, dX, C, dBias, dY, nslabs, ctx->mm_part, ctx->mm_counters);
+        R.d_hdr, R.d_rec, R.d_w, R.nrec, E->m, E->n, R.nb, R.ksplit, dX, C, dBias, dY, nslabs,
+        ctx->mm_part ? (float *)ctx->mm_part->p : nullptr, ctx->mm_counters ? (uint32_t *)ctx->mm_counters->p : nullptr);
     return SO_OK;
 }
 
@@ -372,19 +373,25 @@ so_status so_matmul_rbm_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C)
 
 so_status so_matmul_workspace(so_ctx *ctx, size_t need_part, size_t need_cnt)
 {
-    if (need_part <= ctx->mm_part_bytes && need_cnt <= ctx->mm_counter_bytes) return SO_OK;
+    const size_t part = ctx->mm_part ? ctx->mm_part->bytes : 0, cnt = ctx->mm_counters ? ctx->mm_counters->bytes : 0;
+    if (need_part <= part && need_cnt <= cnt) {
+        const so_status s = so_keep_recorded(ctx, ctx->mm_part);
+        return s != SO_OK ? s : so_keep_recorded(ctx, ctx->mm_counters);
+    }
     SO_REQUIRE(!ctx->capturing, "so_matmul: the kernel's workspace must grow, which cannot be done while a graph is "
                                 "being recorded (call so_matmul_reserve, or launch this shape once, before recording)");
     SO_HIP(hipStreamSynchronize(ctx->stream));
-    if (ctx->mm_part) { (void)hipFree(ctx->mm_part); ctx->mm_part = nullptr; ctx->mm_part_bytes = 0; }
-    if (ctx->mm_counters) { (void)hipFree(ctx->mm_counters); ctx->mm_counters = nullptr; ctx->mm_counter_bytes = 0; }
-    const size_t pb = need_part + need_part / 4, cb = std::max<size_t>(need_cnt * 2, 4096);
-    SO_HIP(hipMalloc((void **)&ctx->mm_part, pb));
-    ctx->mm_part_bytes = pb;
-    SO_HIP(hipMalloc((void **)&ctx->mm_counters, cb));
-    ctx->mm_counter_bytes = cb;
-    SO_HIP(hipMemsetAsync(ctx->mm_counters, 0, cb, ctx->stream));
+    // Given up here; a graph recorded with them keeps them.  Their counters are zero between launches, so it may go on.
+    ctx->mm_part.reset();
+    ctx->mm_counters.reset();
+    so_block_ref new_part, new_cnt;
+    so_status s = so_block_make(ctx, need_part + need_part / 4, &new_part);
+    if (s == SO_OK) s = so_block_make(ctx, std::max<size_t>(need_cnt * 2, 4096), &new_cnt);
+    if (s != SO_OK) return s;
+    SO_HIP(hipMemsetAsync(new_cnt->p, 0, new_cnt->bytes, ctx->stream));
     SO_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->mm_part = std::move(new_part);
+    ctx->mm_counters = std::move(new_cnt);
     return SO_OK;
 }
 

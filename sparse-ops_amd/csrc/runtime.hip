@@ -168,9 +168,35 @@ extern "C" so_status so_destroy(so_ctx *ctx)
     if (ctx->h_wait_gave_up) (void)hipHostFree(ctx->h_wait_gave_up);
     if (ctx->h_stage) (void)hipHostFree(ctx->h_stage);
     if (ctx->d_stage_done) (void)hipFree(ctx->d_stage_done);
-    if (ctx->mm_part) (void)hipFree(ctx->mm_part);
-    if (ctx->mm_counters) (void)hipFree(ctx->mm_counters);
     delete ctx;
+    return SO_OK;
+}
+
+so_status so_block_make(so_ctx *ctx, size_t bytes, so_block_ref *out)
+{
+    try {
+        so_block_ref b = std::make_shared<so_block>();
+        SO_HIP(hipSetDevice(ctx->device));
+        SO_HIP(hipMalloc(&b->p, std::max<size_t>(bytes, 4)));
+        b->bytes = bytes;
+        *out = std::move(b);
+    } catch (const std::bad_alloc &) {
+        so_set_error("host allocation failed");
+        return SO_ERR_OOM;
+    }
+    return SO_OK;
+}
+
+so_status so_keep_recorded(so_ctx *ctx, const so_block_ref &block)
+{
+    if (!ctx->capturing || !block) return SO_OK;
+    if (std::find(ctx->recorded.begin(), ctx->recorded.end(), block) != ctx->recorded.end()) return SO_OK;
+    try {
+        ctx->recorded.push_back(block);
+    } catch (const std::bad_alloc &) {
+        so_set_error("host allocation failed");
+        return SO_ERR_OOM;
+    }
     return SO_OK;
 }
 
@@ -426,11 +452,14 @@ extern "C" so_status so_graph_end(so_ctx *ctx, so_graph **out)
     SO_REQUIRE(ctx->capturing, "so_graph_end: not recording");
     *out = nullptr;
     ctx->capturing = false;
+    std::vector<so_block_ref> uses = std::move(ctx->recorded);
+    ctx->recorded.clear();
     hipGraph_t graph = nullptr;
     SO_HIP(hipStreamEndCapture(ctx->stream, &graph));
     so_graph *g = new (std::nothrow) so_graph();
     if (!g) { (void)hipGraphDestroy(graph); so_set_error("so_graph_end: host allocation failed"); return SO_ERR_OOM; }
     g->graph = graph;
+    g->uses = std::move(uses);
     hipError_t e = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
     if (e != hipSuccess) {
         so_set_error("hipGraphInstantiate failed: %s", hipGetErrorString(e));

@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
+#include <memory>
 #include <string>
 #include <thread>
 #include <vector>
@@ -33,6 +34,19 @@ struct so_tuning {
     int conv_rbm = -1;       // SPARSEOPS_CONV_RBM: 0 forbids the row-block-merged kernel on plans that carry its streams
 };
 
+// Device memory that the library may replace by itself (a workspace that grows, a layout that is rewritten): its kernels
+// get the address as an argument, so a recorded graph replays with it.  Owned together by whoever uses it now and by
+// every graph recorded with it, and freed with the last of them.
+struct so_block {
+    void *p = nullptr;
+    size_t bytes = 0;
+    so_block() = default;
+    so_block(const so_block &) = delete;
+    so_block &operator=(const so_block &) = delete;
+    ~so_block() { if (p) (void)hipFree(p); }
+};
+using so_block_ref = std::shared_ptr<so_block>;
+
 struct so_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -41,7 +55,6 @@ struct so_ctx {
     int max_lds_bytes = 0;   // largest LDS allocation one workgroup may ask for
     bool capturing = false;
     void *static_scratch = nullptr;   // this device's address of the library's static scratch array (so_ellpack_encode_noalloc)
-    // workspace of the row-block-merged matmul (csrc/matmul_rbm.hip): partial tiles of the workgroups that share a tile, a counter per tile
     // Bounded waits (csrc/lds_sync.h): a device word in which waves that gave up count themselves, its pinned
     // host copy, and whether a kernel that waits that way has been launched since the word was last looked at.
     uint32_t *d_wait_gave_up = nullptr;
@@ -53,10 +66,9 @@ struct so_ctx {
     uint32_t *d_stage_done = nullptr;      // workgroups of a way out that have finished
     size_t stage_used = 0;
     uint32_t stage_turn = 0;
-    float *mm_part = nullptr;
-    size_t mm_part_bytes = 0;
-    uint32_t *mm_counters = nullptr;
-    size_t mm_counter_bytes = 0;
+    // Workspace of so_matmul's kernels that split a tile over workgroups: partial tiles, a zeroed counter per tile
+    so_block_ref mm_part, mm_counters;
+    std::vector<so_block_ref> recorded;          // what the launches of the recording under way use (so_keep_recorded)
     std::string name;
     so_tuning tune;
     std::vector<const void *> big_lds_kernels;   // kernels already allowed max_lds_bytes of dynamic LDS on this device
@@ -157,6 +169,7 @@ struct so_rbm {
 struct so_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    std::vector<so_block_ref> uses;              // kept alive for the replays
 };
 
 void so_set_error(const char *fmt, ...);
@@ -173,6 +186,11 @@ so_status so_matmul_rbm_set_pitch(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_rbm_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_rbm_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
                                const float *dBias, float *dY, int act);
+
+// A block of `bytes` on the context's device (at least one).
+so_status so_block_make(so_ctx *ctx, size_t bytes, so_block_ref *out);
+// To be called for every block that a launch uses: while a graph is being recorded, the graph keeps it.
+so_status so_keep_recorded(so_ctx *ctx, const so_block_ref &block);
 
 // Grows the context's matmul workspace (partial tiles, a zeroed counter per tile).  Never while a graph is being recorded.
 so_status so_matmul_workspace(so_ctx *ctx, size_t part_bytes, size_t counter_bytes);

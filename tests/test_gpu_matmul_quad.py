@@ -112,6 +112,41 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         dE.free()
 
 
+@pytest.mark.parametrize("kernel", ["SPARSEOPS_MATMUL_QUAD", "SPARSEOPS_MATMUL_RBM"])
+def test_recorded_graph_outlives_its_workspace(ctx, kernel):
+    """A larger launch makes the context's workspace grow; a graph recorded before keeps the one it was recorded with, so
+    its replays still give the eager launch's bits, and leave alone what was allocated since."""
+    rng = np.random.default_rng(5)
+    C = 40
+    small, large = (datagen.encode_dense(sparse_matrix(rng, m, n, .7)) for m, n in ((300, 1100), (900, 3000)))
+    with ctx.tuning(**{kernel: "1", "SPARSEOPS_MATMUL_QUAD_SPLIT": "4", "SPARSEOPS_MATMUL_RBM_SPLIT": "4"}):
+        dS, dL = (ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM) for E in (small, large))
+        dX, dY = ctx.array(rng.standard_normal((1100, C)).astype(np.float32)), ctx.empty((300, C))
+        ctx.matmul(dS, dX, C, None, dY, "relu")
+        eager = dY.download()
+        ctx.graph_begin()
+        ctx.matmul(dS, dX, C, None, dY, "relu")
+        g = ctx.graph_end()
+        arrays = [dX, dY]
+        for Cl in (64, 700, 5000):
+            Xl = ctx.array(rng.standard_normal((3000, Cl)).astype(np.float32))
+            Yl = ctx.empty((900, Cl))
+            ctx.matmul(dL, Xl, Cl, None, Yl, "none")
+            Y0 = Yl.download()
+            filler = [ctx.array(np.full(1 << k, 3, np.float32)) for k in range(10, 22)]
+            for _ in range(3):
+                ctx.fill_zero(dY)
+                ctx.graph_launch(g)
+                assert np.array_equal(dY.download(), eager)
+            assert all((f.download() == 3).all() for f in filler)
+            ctx.matmul(dL, Xl, Cl, None, Yl, "none")
+            assert np.array_equal(Yl.download(), Y0)
+            arrays += [Xl, Yl] + filler
+        ctx.graph_free(g)
+        for a in arrays + [dS, dL]:
+            a.free()
+
+
 @pytest.mark.parametrize("m,n,C,sp", [(1, 64, 1, .0), (5, 4097, 3, .5), (16, 70, 1, .0), (130, 513, 2, .5), (257, 700, 3, .7), (1000, 1025, 1, .8),
                                       (65, 50000, 2, .99), (4100, 300, 3, .3)])
 @pytest.mark.parametrize("act", ["none", "relu", "sigmoid", "tanh"])
