@@ -385,8 +385,9 @@ so_status so_matmul_workspace(so_ctx *ctx, size_t need_part, size_t need_cnt)
     ctx->mm_part.reset();
     ctx->mm_counters.reset();
     so_block_ref new_part, new_cnt;
-    so_status s = so_block_make(ctx, need_part + need_part / 4, &new_part);
-    if (s == SO_OK) s = so_block_make(ctx, std::max<size_t>(need_cnt * 2, 4096), &new_cnt);
+    // neither shrinks: what was reserved for another matrix stays reserved
+    so_status s = so_block_make(ctx, need_part > part ? need_part + need_part / 4 : part, &new_part);
+    if (s == SO_OK) s = so_block_make(ctx, need_cnt > cnt ? std::max<size_t>(need_cnt * 2, 4096) : cnt, &new_cnt);
     if (s != SO_OK) return s;
     SO_HIP(hipMemsetAsync(new_cnt->p, 0, new_cnt->bytes, ctx->stream));
     SO_HIP(hipStreamSynchronize(ctx->stream));

@@ -112,6 +112,38 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         dE.free()
 
 
+def test_reserved_workspace_stays_reserved():
+    """A matrix that needs more counters and smaller partial tiles than the one reserved before it: both can be recorded."""
+    rng = np.random.default_rng(6)
+    C = 64
+    c = hipabi.Context()
+    cases = [(3840, 2100, "4", "8"), (4400, 600, "0", "2")]        # 60 tiles of 8 x 16 KB; 1100 of 2 x 1 KB
+    handles = []
+    for m, n, rows, split in cases:
+        E = datagen.encode_dense(sparse_matrix(rng, m, n, .97))
+        handles.append((c.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM), c.array(rng.standard_normal((n, C)).astype(np.float32)), c.empty((m, C))))
+    for (m, n, rows, split), (dE, _, _) in zip(cases, handles):
+        with c.tuning(SPARSEOPS_MATMUL_QUAD="1", SPARSEOPS_MATMUL_QUAD_ROWS=rows, SPARSEOPS_MATMUL_QUAD_SPLIT=split):
+            c.matmul_reserve(dE, C)
+    for (m, n, rows, split), (dE, dX, dY) in zip(cases, handles):
+        with c.tuning(SPARSEOPS_MATMUL_QUAD="1", SPARSEOPS_MATMUL_QUAD_ROWS=rows, SPARSEOPS_MATMUL_QUAD_SPLIT=split):
+            c.graph_begin()
+            try:
+                c.matmul(dE, dX, C, None, dY)
+            finally:
+                g = c.graph_end()
+            c.matmul(dE, dX, C, None, dY)
+            eager = dY.download()
+            c.fill_zero(dY)
+            c.graph_launch(g)
+            assert np.array_equal(dY.download(), eager)
+            c.graph_free(g)
+    for h in handles:
+        for a in h:
+            a.free()
+    c.close()
+
+
 @pytest.mark.parametrize("kernel", ["SPARSEOPS_MATMUL_QUAD", "SPARSEOPS_MATMUL_RBM"])
 def test_recorded_graph_outlives_its_workspace(ctx, kernel):
     """A larger launch makes the context's workspace grow; a graph recorded before keeps the one it was recorded with, so
