@@ -338,6 +338,8 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
     void *p = nullptr;
     const so_status s = so_malloc(ctx, blob.size() * 4, &p);
     if (s != SO_OK) return s;
+    R.d_blob = p;
+    R.recs = std::make_shared<so_block>();
     R.d_rec = (uint32_t *)p;
     R.d_w = (float *)(R.d_rec + rec_words);
     R.d_hdr = R.d_rec + 2 * rec_words;
@@ -348,7 +350,7 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
 void so_rbmm_free(so_ellpack *E)
 {
     so_rbmm &R = E->rbmm;
-    if (R.d_rec) (void)hipFree(R.d_rec);
+    if (R.d_blob) (void)hipFree(R.d_blob);
     R = so_rbmm();
 }
 
@@ -398,15 +400,24 @@ so_status so_matmul_workspace(so_ctx *ctx, size_t need_part, size_t need_cnt)
 
 // The records address X rows by byte offset (row * pitch): rewritten for dense width C when the handle was
 // last used with another (stream-ordered; launches of one handle with different C must not overlap on
-// different streams).  Never inside a recording: the rewrite would become a node of the graph, run again
+// different streams).  Records that a recorded graph replays with stay as they are: the new width's go to a block
+// of their own.  Never inside a recording: the rewrite would become a node of the graph, run again
 // on every replay, and leave launches outside the graph with records that were never written.
 so_status so_matmul_rbm_set_pitch(so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_rbmm &R = E->rbmm;
-    if (R.pitch == C * 4u) return SO_OK;
+    if (R.pitch == C * 4u) return so_keep_recorded(ctx, R.recs);
     SO_REQUIRE(!ctx->capturing, "so_matmul: the row-block-merged records must be rewritten for %u dense columns, which cannot be done "
                                 "while a graph is being recorded (call so_matmul_reserve, or launch this shape once, before recording)", C);
     so_rbmm &Rw = const_cast<so_ellpack *>(E)->rbmm;
+    if (R.recs.use_count() > 1) {
+        so_block_ref fresh;
+        const so_status s = so_block_make(ctx, R.nrec * RECBYTES, &fresh);
+        if (s != SO_OK) return s;
+        SO_HIP(hipMemcpyAsync(fresh->p, R.d_rec, R.nrec * RECBYTES, hipMemcpyDeviceToDevice, ctx->stream));
+        Rw.recs = std::move(fresh);
+        Rw.d_rec = (uint32_t *)Rw.recs->p;
+    }
     const uint64_t words = R.nrec * 4;
     rbmm_offsets_kernel<<<so_ceil_div(words, 256), 256, 0, ctx->stream>>>(Rw.d_rec, Rw.d_xrows, R.nrec, C * 4u);
     Rw.pitch = C * 4u;

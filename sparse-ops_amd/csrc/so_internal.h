@@ -116,10 +116,12 @@ struct so_rbmm {
     uint32_t nb = 0, ksplit = 1;
     uint64_t nrec = 0;                            // records (= weight blocks), tails included
     uint64_t slots = 0, xloads = 0;               // multiply-adds a 64-column slab costs (padding included), X row segments it loads
+    void *d_blob = nullptr;                       // one allocation for the arrays below
     uint32_t *d_hdr = nullptr;                    // per block: iterations per class (6 dwords + 2 spare), then per stream {first record, first class}
     uint32_t *d_rec = nullptr;
     float *d_w = nullptr;
     uint32_t *d_xrows = nullptr;                  // [nrec][4]: the X rows of every record; the records hold row * pitch
+    so_block_ref recs;                            // owner of d_rec where set_pitch moved it; else empty, held by graphs recorded with d_rec all the same
     uint32_t pitch = 0;                           // row pitch of X (bytes) the records' offsets are written for; 0: none yet
 };
 

@@ -211,6 +211,36 @@ def test_rbm_in_a_launch_graph(ctx, oracle):
         dE.free()
 
 
+def test_rbm_graphs_of_several_widths(ctx):
+    """The handle's records hold X row offsets for one width: a graph recorded at one keeps giving its eager launch's bits
+    after launches, reservations and recordings of the same handle at others."""
+    rng = np.random.default_rng(18)
+    E = datagen.encode_dense(sparse_matrix(rng, 400, 1500, .8))
+    with ctx.tuning(SPARSEOPS_MATMUL_RBM="1", SPARSEOPS_MATMUL_RBM_SPLIT="2"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+        runs = []
+        for C in (40, 72, 40, 129):
+            dX, dY = ctx.array(rng.standard_normal((1500, C)).astype(np.float32)), ctx.empty((400, C))
+            ctx.matmul(dE, dX, C, None, dY, "relu")
+            eager = dY.download()
+            ctx.matmul_reserve(dE, C)
+            ctx.graph_begin()
+            ctx.matmul(dE, dX, C, None, dY, "relu")
+            runs.append((C, dX, dY, eager, ctx.graph_end()))
+            ctx.matmul_reserve(dE, C + 4)
+            for C0, X0, Y0, eager0, g in runs:
+                ctx.fill_zero(Y0)
+                ctx.graph_launch(g)
+                assert np.array_equal(Y0.download(), eager0), (C, C0)
+        for C, dX, dY, eager, g in runs:
+            ctx.graph_free(g)
+            ctx.matmul(dE, dX, C, None, dY, "relu")
+            assert np.array_equal(dY.download(), eager), C
+            dX.free()
+            dY.free()
+        dE.free()
+
+
 @pytest.mark.parametrize("seed", range(16))
 def test_rbm_random_sweep(ctx, oracle, seed):
     """Seeded random shapes, densities, K splits and sparsity patterns (uniform, a few dense columns, a few dense
