@@ -231,8 +231,11 @@ so_status so_conv_plan_create(so_ctx *ctx, const so_ellpack *E, const so_conv_ge
 so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan);
 /* Re-sizes the plan's internal layouts for launches with batch B (how many output channels
  * a wave takes depends on how many workgroups the batch yields).  Optional: results never
- * depend on it; plans are created for batch 32.  Not to be called while a launch that uses
- * the plan may be in flight on another stream, nor during graph capture (it allocates).
+ * depend on it; plans are created for batch 32.  For a batch of at most four it also makes the
+ * column kernel's streams for exactly that batch, once; they stay until the plan is freed.
+ * Not to be called while a launch that uses the plan may be in flight on another stream, nor during
+ * graph capture (it allocates).  A graph recorded with the plan before is recorded again afterwards
+ * (SparseOnnxModel::resize_buffers does), unless the new batch falls into the same four-entry step.
  * No counterpart in the reference. */
 so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t B);
 /* The LDS-windowed kernel's parameters for this plan (no counterpart in the reference:

@@ -924,7 +924,7 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
     // The windowed layout depends on the batch only through the number of batch tiles: rebuilt only if the batch
     // changes the batch tile the chunks are sized for or the choice of channels per wave.  A plan without the layout
     // (the geometry did not suit the batch tile tried last) is tried again when the batch tile changes: a smaller tile
-    // holds more channels per chunk.  The column kernel's streams are for one batch.
+    // holds more channels per chunk.  The column kernel's streams are for one batch each, built once.
     const uint32_t batch = std::max(4u, B / 4u * 4u);
     const so_ellpack *E = plan->E;
     const uint32_t lpp = window_lpp(batch) ? window_lpp(batch) : kWinLPP;
@@ -934,20 +934,21 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
         const double run = (double)E->total_nnz / (double)plan->g.Cout / plan->win.nch;
         window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw;
     }
-    const bool columns = B <= kColMaxBatch && plan->col.batch != B;
-    plan->tuned_batch = batch;
-    if (!window && !columns) return SO_OK;
+    const bool columns = B >= 1 && B <= kColMaxBatch && !plan->col_tried[B - 1];
+    if (!window && !columns) { plan->tuned_batch = batch; return SO_OK; }
     const size_t slots = (size_t)E->m * E->r;
     std::vector<uint32_t> idx(slots), nnz(E->m);
     std::vector<float> Wd(slots);
     so_status s = so_ellpack_download(ctx, E, SO_LAYOUT_ROW, Wd.data(), idx.data(), nnz.data());
     if (s != SO_OK) return s;
-    SO_HIP(hipStreamSynchronize(ctx->stream));      // no launch may still be reading the old arrays
     if (columns) {
-        so_conv_columns_free(plan);
         s = so_conv_columns_build(ctx, plan, idx, nnz, Wd, B);
-        if (s != SO_OK || !window) return s;
+        if (s != SO_OK) return s;
+        plan->col_tried[B - 1] = true;
     }
+    plan->tuned_batch = batch;
+    if (!window) return SO_OK;
+    SO_HIP(hipStreamSynchronize(ctx->stream));      // no launch may still be reading the old arrays
     free_window(plan);
     s = build_window(ctx, plan, idx, nnz, Wd, batch);
     if (s != SO_OK) return s;
@@ -977,11 +978,11 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     // does not take them), at four where its shorter chains on more waves win -- the windowed kernel's time there is
     // about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (7x7x512 27.6 against 22.8 us, 14x14x256
     // 17.5 against 24.4).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
-    if (plan->col.batch == B && B != 0 && ctx->tune.conv_columns != 0) {
+    if (so_conv_columns_for(plan, B) && ctx->tune.conv_columns != 0) {
         bool use = B < 4 || plan->win.cc == 0 || ctx->tune.conv_columns == 1;
         if (!use && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
             const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw, B), (uint64_t)ctx->compute_units);
-            use = so_conv_columns_estimate(ctx, plan) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
+            use = so_conv_columns_estimate(ctx, plan, B) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
         }
         if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for
         bool done = false;

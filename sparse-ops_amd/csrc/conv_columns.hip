@@ -178,7 +178,8 @@ template <int ACT>
 void launch_columns(so_ctx *ctx, const so_conv_plan *plan, const ColArgs &a, dim3 grid, size_t lds, const float *dX, uint32_t B,
                     const float *dBias, const float *dResid, float *dY)
 {
-    conv2d_column_kernel<ACT><<<grid, a.waves * 64u, lds, ctx->stream>>>(plan->col.d_entries, plan->col.d_first, a, plan->g, dX, B, dBias, dResid, dY);
+    const so_conv_columns &c = plan->col[B - 1];
+    conv2d_column_kernel<ACT><<<grid, a.waves * 64u, lds, ctx->stream>>>(c.d_entries, c.d_first, a, plan->g, dX, B, dBias, dResid, dY);
 }
 
 constexpr uint64_t kColLds = 150 * 1024;
@@ -187,9 +188,16 @@ constexpr uint64_t kColLds = 150 * 1024;
 
 void so_conv_columns_free(so_conv_plan *plan)
 {
-    if (plan->col.d_entries) (void)hipFree(plan->col.d_entries);
-    if (plan->col.d_first) (void)hipFree(plan->col.d_first);
-    plan->col = so_conv_columns();
+    for (so_conv_columns &c : plan->col) {
+        if (c.d_entries) (void)hipFree(c.d_entries);
+        if (c.d_first) (void)hipFree(c.d_first);
+        c = so_conv_columns();
+    }
+}
+
+const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B)
+{
+    return B >= 1 && B <= kColMaxBatch && plan->col[B - 1].batch == B ? &plan->col[B - 1] : nullptr;
 }
 
 // Sizes the tile for batch B and uploads the entry streams; leaves the plan without them where the kernel does not apply.
@@ -263,10 +271,14 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
         s = so_h2d(ctx, c.d_entries, entries.data(), entries.size() * sizeof(int2));
         if (s == SO_OK) s = so_h2d(ctx, c.d_first, first.data(), first.size() * 4);
     }
+    if (s != SO_OK) {
+        (void)hipFree(c.d_entries);
+        if (c.d_first) (void)hipFree(c.d_first);
+        return s;
+    }
     c.batch = B;
-    plan->col = c;
-    if (s != SO_OK) so_conv_columns_free(plan);
-    return s;
+    plan->col[B - 1] = c;
+    return SO_OK;
 }
 
 namespace {
@@ -277,9 +289,8 @@ struct ColShape { uint32_t G, waves; size_t lds; double us; };
 // longest chain at 12 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
 // more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 9.0 us, 28x28x128 10.2, 14x14x256
 // 10.4, 7x7x512 16; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
-ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan)
+ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
 {
-    const so_conv_columns &c = plan->col;
     const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
     ColShape best{16, 16, 0, 1e30};
     for (uint32_t G = 16; G >= 4; G /= 2) {
@@ -296,22 +307,22 @@ ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan)
 
 } // namespace
 
-double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan) { return column_shape(ctx, plan).us; }
+double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, plan->col[B - 1]).us; }
 
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done)
 {
-    const so_conv_columns &c = plan->col;
-    const so_conv_geom &g = plan->g;
     *done = false;
-    if (c.batch != B) return SO_OK;
+    if (!so_conv_columns_for(plan, B)) return SO_OK;
+    const so_conv_columns &c = plan->col[B - 1];
+    const so_conv_geom &g = plan->g;
     ColArgs a;
     a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch;
     a.sth = window_step(g.kH, g.stride_h); a.stw = window_step(g.kW, g.stride_w);
     a.sbh = window_subsample(g.kH, g.stride_h); a.sbw = window_subsample(g.kW, g.stride_w);
     a.mB = window_magic(B); a.mIP = window_magic(a.IP); a.mPL = window_magic(a.PL); a.mTW = window_magic(a.TW); a.mTilesX = window_magic(a.tiles_x);
     const uint64_t tiles = (uint64_t)c.tiles_x * c.tiles_y;
-    const ColShape shape = column_shape(ctx, plan);
+    const ColShape shape = column_shape(ctx, plan, c);
     a.G = shape.G;
     a.waves = shape.waves;
     const size_t lds = shape.lds;

@@ -39,7 +39,7 @@ struct so_conv_rbm {
 // Entry streams of the column kernel for small batches (conv_columns.hip).
 constexpr uint32_t kColMaxBatch = 4;
 struct so_conv_columns {
-    uint32_t batch = 0;              // the batch the tile and the offsets are for; 0: not built
+    uint32_t batch = 0;              // the batch the tile and the offsets are for; 0: not built, or the kernel does not apply
     uint32_t TH = 0, TW = 0, tiles_x = 0, tiles_y = 0, IP = 0, PE = 0, cc = 0, nch = 0;
     int2 *d_entries = nullptr;       // groups of 16 {weight bits, LDS byte offset}, channel by channel, chunk by chunk
     uint32_t *d_first = nullptr;     // [Cout * nch + 1]: first group of (channel, chunk)
@@ -53,14 +53,16 @@ struct so_conv_plan {
     int2 *d_taps = nullptr;  // per slot: x = (cin*H + dh)*W + dw (elements of B floats), y = dh<<16 | (dw & 0xffff)
     so_conv_window win;      // win.cc == 0: not built
     so_conv_rbm rbm;         // rbm.d_sets == nullptr: no streams
-    so_conv_columns col;     // col.batch == 0: no streams
+    so_conv_columns col[kColMaxBatch];   // streams for batch 1 + index, made by the first tuning for it and kept: graphs may replay with them
+    bool col_tried[kColMaxBatch] = {};   // that tuning has happened, whether the kernel applies or not
 };
 
 // conv_columns.hip
 void so_conv_columns_free(so_conv_plan *plan);
 so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
                                 const std::vector<float> &Wd, uint32_t B);
-double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan);      // us
+const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B);  // null: the plan has no streams for the batch
+double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);      // us
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done);
 

@@ -53,3 +53,48 @@ def test_columns_match_oracle(ctx, oracle, Cin, Cout, H, Wi, k, s, p, d, sp, B):
         ctx.conv_plan_free(plan)
         for a in (dX, dY, dB, dR, dE):
             a.free()
+
+
+@pytest.mark.parametrize("ordered", [True, False])
+def test_streams_are_made_once_per_batch_and_kept(ctx, oracle, ordered):
+    """Tuning for one small batch after another neither takes away the streams that a recorded graph replays with nor makes
+    any again -- also where the kernel does not apply (rows that do not ascend): a second tuning for a batch copies nothing,
+    so it is even possible while a graph is being recorded, where a download is refused."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(21)
+    args = (12, 20, 3, 3, 9, 11, (1, 1), (1, 1), (1, 1))
+    g, og = hipabi.conv_geom(*args), ocg(*args)
+    E = datagen.encode_dense(sparse_matrix(rng, 20, 12 * 9, .6))
+    if not ordered:
+        c = int(E.nnz[3])
+        E.Wd[3, :c], E.idx[3, :c] = E.Wd[3, :c][::-1].copy(), E.idx[3, :c][::-1].copy()
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan = ctx.conv_plan(dE, g)
+    runs = []
+    for B in (1, 2, 3, 4):
+        X = rng.standard_normal((12, 9, 11, B)).astype(np.float32)
+        dX, dY = ctx.array(X), ctx.empty((20, g.H_out, g.W_out, B))
+        ctx.conv_plan_tune(plan, B)
+        ctx.graph_begin()
+        try:
+            ctx.conv_plan_tune(plan, B)
+            ctx.conv2d(plan, dX, B, None, dY, "none")
+        finally:
+            graph = ctx.graph_end()
+        runs.append((graph, dX, dY, oracle.conv2d_pf(as_oracle(E), og, X, B, None, "none")))
+        for graph, _, dY, want in runs:
+            ctx.fill_zero(dY)
+            ctx.graph_launch(graph)
+            assert np.array_equal(dY.download(), want)
+    ctx.graph_begin()
+    try:
+        for B in (1, 4, 2, 3, 1):
+            ctx.conv_plan_tune(plan, B)
+    finally:
+        ctx.graph_free(ctx.graph_end())
+    for graph, dX, dY, _ in runs:
+        ctx.graph_free(graph)
+        dX.free()
+        dY.free()
+    ctx.conv_plan_free(plan)
+    dE.free()
