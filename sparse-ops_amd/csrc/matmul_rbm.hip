@@ -308,7 +308,7 @@ so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint3
             }
         }
     }
-    });
+    }, (uint64_t)n * 64);                                         // a range's table of columns: the vectors and what they hold
     std::vector<size_t> first(R.nb + 1, 0);                       // each block's first record
     uint64_t slots_total = 0, parts_total = 0;
     for (uint32_t b = 0; b < R.nb; ++b) {

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdarg>
 #include <cstring>
+#include <exception>
 #include <new>
 
 static thread_local std::string g_last_error;
@@ -680,66 +681,72 @@ extern "C" so_status so_ellpack_upload(so_ctx *ctx, const float *Wd, const uint3
     if (!ascending) layouts &= ~SO_LAYOUT_TILED;
     E->layouts = layouts | SO_LAYOUT_ROW;
 
-    so_status s = upload_array(ctx, Wd, slots, &E->d_Wd);
-    if (s == SO_OK) s = upload_array(ctx, idx, slots, &E->d_idx);
-    if (s == SO_OK) s = upload_array(ctx, nnz, (size_t)m, &E->d_nnz);
+    so_status s = SO_OK;
+    try {
+        s = upload_array(ctx, Wd, slots, &E->d_Wd);
+        if (s == SO_OK) s = upload_array(ctx, idx, slots, &E->d_idx);
+        if (s == SO_OK) s = upload_array(ctx, nnz, (size_t)m, &E->d_nnz);
 
-    if (s == SO_OK && (layouts & SO_LAYOUT_SLOT)) {
-        std::vector<float> WdT(slots);
-        std::vector<uint32_t> idxT(slots);
-        for (uint32_t i = 0; i < m; ++i)
-            for (uint32_t k = 0; k < r; ++k) {
-                WdT[(size_t)k * m + i] = Wd[(size_t)i * r + k];
-                idxT[(size_t)k * m + i] = idx[(size_t)i * r + k];
+        if (s == SO_OK && (layouts & SO_LAYOUT_SLOT)) {
+            std::vector<float> WdT(slots);
+            std::vector<uint32_t> idxT(slots);
+            for (uint32_t i = 0; i < m; ++i)
+                for (uint32_t k = 0; k < r; ++k) {
+                    WdT[(size_t)k * m + i] = Wd[(size_t)i * r + k];
+                    idxT[(size_t)k * m + i] = idx[(size_t)i * r + k];
+                }
+            s = upload_array(ctx, WdT.data(), slots, &E->d_WdT);
+            if (s == SO_OK) s = upload_array(ctx, idxT.data(), slots, &E->d_idxT);
+            if (s == SO_OK && (layouts & SO_LAYOUT_IDX16)) {
+                std::vector<uint16_t> idxT16(slots);
+                for (size_t k = 0; k < slots; ++k) idxT16[k] = (uint16_t)idxT[k];
+                s = upload_array(ctx, idxT16.data(), slots, &E->d_idxT16);
             }
-        s = upload_array(ctx, WdT.data(), slots, &E->d_WdT);
-        if (s == SO_OK) s = upload_array(ctx, idxT.data(), slots, &E->d_idxT);
+        }
+
         if (s == SO_OK && (layouts & SO_LAYOUT_IDX16)) {
-            std::vector<uint16_t> idxT16(slots);
-            for (size_t k = 0; k < slots; ++k) idxT16[k] = (uint16_t)idxT[k];
-            s = upload_array(ctx, idxT16.data(), slots, &E->d_idxT16);
+            // The same slots as d_idx, two bytes each: so_matvec streams 6 bytes per nonzero instead of 8.
+            // Padding slots keep the low half of whatever they hold; no kernel uses them.
+            std::vector<uint16_t> idx16(slots);
+            for (size_t k = 0; k < slots; ++k) idx16[k] = (uint16_t)idx[k];
+            s = upload_array(ctx, idx16.data(), slots, &E->d_idx16);
         }
-    }
 
-    if (s == SO_OK && (layouts & SO_LAYOUT_IDX16)) {
-        // The same slots as d_idx, two bytes each: so_matvec streams 6 bytes per nonzero instead of 8.
-        // Padding slots keep the low half of whatever they hold; no kernel uses them.
-        std::vector<uint16_t> idx16(slots);
-        for (size_t k = 0; k < slots; ++k) idx16[k] = (uint16_t)idx[k];
-        s = upload_array(ctx, idx16.data(), slots, &E->d_idx16);
-    }
-
-    if (s == SO_OK && (layouts & SO_LAYOUT_BINS)) {
-        // Length classes: <= 16 nonzeros -> 4 lanes per row, <= 128 -> 16 lanes, <= 4096 -> a whole
-        // wave, longer -> a whole workgroup (a single wave would walk such a row long after every
-        // other row is done).  Long rows first inside a class, so the last waves to start are the
-        // short ones.
-        static const uint32_t group[4] = {4, 16, 64, 1024};
-        static const uint32_t limit[4] = {16, 128, 4096, 0xffffffffu};
-        std::vector<uint32_t> rows[4];
-        for (uint32_t i = 0; i < m; ++i) {
-            int b = 0;
-            while (nnz[i] > limit[b]) ++b;
-            rows[b].push_back(i);
-        }
-        for (int b = 0; b < 4 && s == SO_OK; ++b) {
-            std::stable_sort(rows[b].begin(), rows[b].end(),
-                             [&](uint32_t a, uint32_t c) { return nnz[a] > nnz[c]; });
-            E->bins[b].group = group[b];
-            E->bins[b].count = (uint32_t)rows[b].size();
-            // (row, its length) pairs: a wave learns where its row is and how long in one load
-            std::vector<uint32_t> pairs(2 * rows[b].size());
-            for (size_t k = 0; k < rows[b].size(); ++k) {
-                pairs[2 * k] = rows[b][k];
-                pairs[2 * k + 1] = nnz[rows[b][k]];
+        if (s == SO_OK && (layouts & SO_LAYOUT_BINS)) {
+            // Length classes: <= 16 nonzeros -> 4 lanes per row, <= 128 -> 16 lanes, <= 4096 -> a whole
+            // wave, longer -> a whole workgroup (a single wave would walk such a row long after every
+            // other row is done).  Long rows first inside a class, so the last waves to start are the
+            // short ones.
+            static const uint32_t group[4] = {4, 16, 64, 1024};
+            static const uint32_t limit[4] = {16, 128, 4096, 0xffffffffu};
+            std::vector<uint32_t> rows[4];
+            for (uint32_t i = 0; i < m; ++i) {
+                int b = 0;
+                while (nnz[i] > limit[b]) ++b;
+                rows[b].push_back(i);
             }
-            if (!pairs.empty()) s = upload_array(ctx, pairs.data(), pairs.size(), &E->bins[b].d_rows);
+            for (int b = 0; b < 4 && s == SO_OK; ++b) {
+                std::stable_sort(rows[b].begin(), rows[b].end(),
+                                 [&](uint32_t a, uint32_t c) { return nnz[a] > nnz[c]; });
+                E->bins[b].group = group[b];
+                E->bins[b].count = (uint32_t)rows[b].size();
+                // (row, its length) pairs: a wave learns where its row is and how long in one load
+                std::vector<uint32_t> pairs(2 * rows[b].size());
+                for (size_t k = 0; k < rows[b].size(); ++k) {
+                    pairs[2 * k] = rows[b][k];
+                    pairs[2 * k + 1] = nnz[rows[b][k]];
+                }
+                if (!pairs.empty()) s = upload_array(ctx, pairs.data(), pairs.size(), &E->bins[b].d_rows);
+            }
         }
-    }
 
-    if (s == SO_OK && (layouts & SO_LAYOUT_TILED) && m > 0) s = build_tiled(ctx, E, Wd, idx, nnz);
-    if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_rbmm_build(ctx, E, Wd, idx, nnz);
-    if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_quads_build(ctx, E, Wd, idx, nnz);
+        if (s == SO_OK && (layouts & SO_LAYOUT_TILED) && m > 0) s = build_tiled(ctx, E, Wd, idx, nnz);
+        if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_rbmm_build(ctx, E, Wd, idx, nnz);
+        if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_quads_build(ctx, E, Wd, idx, nnz);
+    } catch (const std::exception &e) {                  // a builder ran out of host memory, on whichever thread
+        so_set_error("so_ellpack_upload: building the layouts failed: %s", e.what());
+        s = SO_ERR_OOM;
+    }
 
     if (s != SO_OK) {
         free_ellpack_arrays(E);

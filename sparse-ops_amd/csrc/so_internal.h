@@ -6,9 +6,9 @@
 #include <cstdio>
 #include <memory>
 #include <string>
-#include <thread>
 #include <vector>
 
+#include "parallel.h"
 #include "sparseops_hip.h"
 
 // Tuning overrides, read from the environment when the context is created (and again by
@@ -245,20 +245,6 @@ hipError_t so_allow_big_lds(so_ctx *ctx, const void *kernel);
             return SO_ERR_HIP;                                                    \
         }                                                                         \
     } while (0)
-
-// f(first, last) over ranges of 0 .. count on up to 16 threads: the layout builders' loops.  `work` = elements that
-// the whole loop touches: a thread costs some 30 us to start, which 100 000 elements repay.
-template <class F>
-void so_parallel(uint32_t count, uint64_t work, F &&f)
-{
-    const uint64_t most = std::min<uint64_t>({std::max(1u, std::thread::hardware_concurrency()), 16u, count, work / 100000u + 1u});
-    const uint32_t nt = (uint32_t)std::max<uint64_t>(1u, most);
-    std::vector<std::thread> threads;
-    for (uint32_t t = 1; t < nt; ++t)
-        threads.emplace_back([&, t] { f((uint32_t)((uint64_t)count * t / nt), (uint32_t)((uint64_t)count * (t + 1) / nt)); });
-    f(0u, (uint32_t)((uint64_t)count / nt));
-    for (auto &t : threads) t.join();
-}
 
 static inline uint32_t so_ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
