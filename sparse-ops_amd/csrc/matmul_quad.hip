@@ -476,7 +476,7 @@ void so_quads_free(so_ellpack *E)
 
 bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    return E->quads.d_w != nullptr && C >= 4 && C < (1u << 21) && (size_t)ctx->max_lds_bytes >= LDS_BYTES;
+    return E->quads.d_w != nullptr && E->n != 0 && C >= 4 && C < (1u << 21) && (size_t)ctx->max_lds_bytes >= LDS_BYTES;
 }
 
 double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C) { return choose(ctx, E, C).us; }

@@ -356,7 +356,7 @@ void so_rbmm_free(so_ellpack *E)
 
 bool so_matmul_rbm_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    if (!(E->layouts & SO_LAYOUT_RBM) || E->rbmm.d_rec == nullptr) return false;
+    if (!(E->layouts & SO_LAYOUT_RBM) || E->rbmm.d_rec == nullptr || E->n == 0) return false;
     if ((uint64_t)E->n * C * 4u > 0xffffffffull) return false;          // X row offsets are 32-bit byte offsets
     return (size_t)ctx->max_lds_bytes >= LDS_BYTES;
 }

@@ -112,6 +112,24 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         dE.free()
 
 
+@pytest.mark.parametrize("forced", [None, "SPARSEOPS_MATMUL_QUAD", "SPARSEOPS_MATMUL_RBM"])
+def test_no_columns(ctx, forced):
+    """A matrix without columns has no row of X to read: the layout's kernels, which read ahead, are not for it."""
+    b = np.linspace(-1, 1, 300).astype(np.float32)
+    E = datagen.encode_dense(np.zeros((300, 0), np.float32))
+    with ctx.tuning(**({forced: "1"} if forced else {})):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, 300, 0, E.r, RBM)
+        dX, dB = ctx.empty((4,)), ctx.array(b)
+        for C in (1, 64, 130):
+            dY = ctx.array(np.full((300, C), np.nan, np.float32))
+            ctx.matmul_reserve(dE, C)
+            ctx.matmul(dE, dX, C, dB, dY, "relu")
+            assert np.array_equal(dY.download(), np.repeat(np.maximum(b, 0)[:, None], C, axis=1))
+            dY.free()
+        for a in (dX, dB, dE):
+            a.free()
+
+
 def test_reserved_workspace_stays_reserved():
     """A matrix that needs more counters and smaller partial tiles than the one reserved before it: both can be recorded."""
     rng = np.random.default_rng(6)
