@@ -203,8 +203,9 @@ so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t 
 /* Makes sure a later so_matmul(ctx, E, ..., C, ...) allocates and prepares nothing: on a handle with the RBM
  * layout the context's workspace is grown to what C dense columns need and the handle's records are written
  * for that width (a no-op for every other layout).  so_matmul does both itself on first use of a larger output
- * or another width, but refuses to while a graph is being recorded: a caller that
- * records so_matmul into a graph calls this first (SparseOnnxModel::resize_buffers does, for every fully
+ * or another width, but not while a graph is being recorded: a launch that would need it is then recorded on
+ * a slower kernel without a workspace, or refused where the row-block-merged kernel is the one for it.  A caller
+ * that records so_matmul into a graph calls this first (SparseOnnxModel::resize_buffers does, for every fully
  * connected layer -- the reference's documented way to get its allocation-free run(), README.md:146).
  * No counterpart in the reference. */
 so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);

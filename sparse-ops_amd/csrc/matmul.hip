@@ -301,9 +301,12 @@ enum class RbmKernel { None, Merged, Quad, Vector };
 RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const bool merged = so_matmul_rbm_applies(ctx, E, C), quad = so_matmul_quad_applies(ctx, E, C);
+    // A recording cannot grow the workspace: the quad kernel is for what has been reserved (the others but the
+    // row-block-merged one, which refuses, need none).
+    const bool reserved = !ctx->capturing || !quad || so_matmul_quad_ready(ctx, E, C);
     if (merged && ctx->tune.matmul_rbm == 1) return RbmKernel::Merged;
     if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
-    if (quad && ctx->tune.matmul_quad == 1) return RbmKernel::Quad;
+    if (quad && ctx->tune.matmul_quad == 1 && reserved) return RbmKernel::Quad;
     if (C <= 3 && E->max_nnz >= 64u * C) return RbmKernel::Vector;
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
@@ -315,7 +318,7 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
         const double us = 9.5 + 2.85e-6 * work * std::ceil(wgs / cus) * cus / wgs;
         if (4.0 * wgs >= 3.0 * cus && (us < best || !quad)) { best = us; k = RbmKernel::Merged; }
     }
-    if (quad && ctx->tune.matmul_quad != 0 && so_matmul_quad_estimate(ctx, E, C) < 0.95 * best) k = RbmKernel::Quad;
+    if (quad && reserved && ctx->tune.matmul_quad != 0 && so_matmul_quad_estimate(ctx, E, C) < 0.95 * best) k = RbmKernel::Quad;
     return k;
 }
 

@@ -372,12 +372,14 @@ so_status launch_quad(so_ctx *ctx, const QuadArgs &a, uint32_t blocks)
     return SO_OK;
 }
 
+size_t part_bytes(const QuadPlan &p) { return (size_t)p.rbs * p.nslab * p.ks * (1u << p.qw_log2) * 64 * 16; }
+size_t counter_bytes(const QuadPlan &p) { return (size_t)p.rbs * p.nslab * sizeof(uint32_t); }
+
 so_status workspace(so_ctx *ctx, const so_ellpack *E, uint32_t C, const QuadPlan &p)
 {
     if (p.ks == 1) return SO_OK;
-    const uint64_t tiles = (uint64_t)p.rbs * p.nslab;
-    SO_REQUIRE(tiles * p.ks < (1ull << 28), "so_matmul: %u x %u output is too large for one launch", E->m, C);
-    return so_matmul_workspace(ctx, (size_t)tiles * p.ks * (1u << p.qw_log2) * 64 * 16, (size_t)tiles * sizeof(uint32_t));
+    SO_REQUIRE((uint64_t)p.rbs * p.nslab * p.ks < (1ull << 28), "so_matmul: %u x %u output is too large for one launch", E->m, C);
+    return so_matmul_workspace(ctx, part_bytes(p), counter_bytes(p));
 }
 
 // ------------------------------------------------------------------ the builder
@@ -482,6 +484,12 @@ bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C) { return choose(ctx, E, C).us; }
 
 so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C) { return workspace(ctx, E, C, choose(ctx, E, C)); }
+
+bool so_matmul_quad_ready(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    const QuadPlan p = choose(ctx, E, C);
+    return p.ks == 1 || (ctx->mm_part && ctx->mm_counters && part_bytes(p) <= ctx->mm_part->bytes && counter_bytes(p) <= ctx->mm_counters->bytes);
+}
 
 so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {

@@ -205,6 +205,7 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
 void so_quads_free(so_ellpack *E);
 bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
 double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);   // us
+bool so_matmul_quad_ready(const so_ctx *ctx, const so_ellpack *E, uint32_t C);        // the workspace need not grow for this launch
 so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
                                 const float *dBias, float *dY, int act);

@@ -130,6 +130,38 @@ def test_no_columns(ctx, forced):
             a.free()
 
 
+def test_recording_without_a_reservation(oracle):
+    """A launch that is too small for the row-block-merged kernel can be recorded on a context that has no workspace yet;
+    with the reservation it is recorded on the kernel that an eager launch takes."""
+    rng = np.random.default_rng(9)
+    E = datagen.encode_dense(sparse_matrix(rng, 512, 4000, .6))
+    C = 16
+    X = rng.standard_normal((4000, C)).astype(np.float32)
+    c = hipabi.Context()
+    dE = c.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+    dX, dY = c.array(X), c.empty((512, C))
+    want = oracle.matmul(as_oracle(E), X, None)
+    for reserved in (False, True):
+        if reserved:
+            c.matmul_reserve(dE, C)
+        c.graph_begin()
+        try:
+            c.matmul(dE, dX, C, None, dY)
+        finally:
+            g = c.graph_end()
+        for _ in range(2):
+            c.fill_zero(dY)
+            c.graph_launch(g)
+            Y = dY.download()
+            assert rel_err(Y, want) <= TOL
+        c.graph_free(g)
+    c.matmul(dE, dX, C, None, dY)
+    assert np.array_equal(dY.download(), Y) and not np.array_equal(Y, want)      # another order of summation than the oracle's
+    for a in (dX, dY, dE):
+        a.free()
+    c.close()
+
+
 def test_reserved_workspace_stays_reserved():
     """A matrix that needs more counters and smaller partial tiles than the one reserved before it: both can be recorded."""
     rng = np.random.default_rng(6)
