@@ -298,15 +298,20 @@ enum class RbmKernel { None, Merged, Quad, Vector };
 //   that one: one column, 4096 x 4096 1756 101.8 / 9.1, 479 19.7 / 4.8, 159 7.9 / 4.1, 69 4.6 / 4.0; 1024 x 4096
 //   62 3.7 / 3.7; 4096 x 512 23 3.5 / 3.9; 10 x 512 63 4.0 / 3.2, 16 3.2 / 3.4; two, 4096 x 4096 487 19.6 / 8.4, 162
 //   7.8 / 7.4; 10 x 512 262 6.0 / 3.4; three, 4096 x 4096 1759 114 / 27, 487 19.7 / 13.1; 4096 x 1024 244 11.0 / 10.4.
-RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+// `plan` is set where it is Quad: the search for it is the larger part of this function's 0.2 (two K tiles) to 0.6 us (16).
+RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan)
 {
     const bool merged = so_matmul_rbm_applies(ctx, E, C), quad = so_matmul_quad_applies(ctx, E, C);
-    // A recording cannot grow the workspace: the quad kernel is for what has been reserved (the others but the
-    // row-block-merged one, which refuses, need none).
-    const bool reserved = !ctx->capturing || !quad || so_matmul_quad_ready(ctx, E, C);
     if (merged && ctx->tune.matmul_rbm == 1) return RbmKernel::Merged;
     if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
-    if (quad && ctx->tune.matmul_quad == 1 && reserved) return RbmKernel::Quad;
+    // Below `us`?  A recording cannot grow the workspace: the quad kernel is then for what has been reserved (the others
+    // but the row-block-merged one, which refuses, need none).
+    const auto quad_below = [&](double us) {
+        if (!quad || ctx->tune.matmul_quad == 0 || us <= kQuadLeastUs) return false;
+        *plan = so_matmul_quad_choose(ctx, E, C);
+        return plan->us < us && (!ctx->capturing || so_matmul_quad_ready(ctx, *plan));
+    };
+    if (ctx->tune.matmul_quad == 1 && quad_below(1e30)) return RbmKernel::Quad;
     if (C <= 3 && E->max_nnz >= 64u * C) return RbmKernel::Vector;
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
@@ -318,8 +323,7 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
         const double us = 9.5 + 2.85e-6 * work * std::ceil(wgs / cus) * cus / wgs;
         if (4.0 * wgs >= 3.0 * cus && (us < best || !quad)) { best = us; k = RbmKernel::Merged; }
     }
-    if (quad && reserved && ctx->tune.matmul_quad != 0 && so_matmul_quad_estimate(ctx, E, C) < 0.95 * best) k = RbmKernel::Quad;
-    return k;
+    return quad_below(0.95 * best) ? RbmKernel::Quad : k;
 }
 
 } // namespace
@@ -353,9 +357,10 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids both, =1
     // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one).
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
-        const RbmKernel k = rbm_kernel(ctx, E, C);
+        so_quad_plan plan;
+        const RbmKernel k = rbm_kernel(ctx, E, C, &plan);
         if (k != RbmKernel::None) {
-            const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, dX, C, dBias, dY, act)
+            const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, plan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;

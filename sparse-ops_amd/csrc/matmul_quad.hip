@@ -327,17 +327,17 @@ void ellpack_matmul_quad_kernel(QuadArgs a)
     }
 }
 
-struct QuadPlan { uint32_t qw_log2, ks, tiles_per, nslab, rbs; double us; };
+} // namespace
 
 // Rows per workgroup and K split by estimated time (us).  The model -- rounds of one workgroup per compute unit,
 // each with its start-up and, per tile, the larger of the multiply-adds and of what a tile's X values take to
 // arrive; for a split the exchange of partial tiles -- was fitted to 900 launches over 44 shapes (10..4096 rows,
 // 512..4096 columns, 4..256 dense columns, 50-95 % sparse): 5.8 % r.m.s., and its choice takes 2 % longer than
 // the best one on average.
-QuadPlan choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+so_quad_plan so_matmul_quad_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
-    QuadPlan best{};
+    so_quad_plan best{};
     best.us = 1e30;
     const uint32_t nslab = so_ceil_div(C, 64);
     const double units = (double)Q.total_units / ((double)Q.nquads * Q.ntiles), cus = ctx->compute_units;
@@ -349,8 +349,9 @@ QuadPlan choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
             const double full = std::min(1.0, wgs / cus), sustained = std::min(1.0, tiles_per / 8.0);   // long launches on the whole chip run at lower clocks
             const double multiply = 0.68 + (0.0635 + 0.01 * full * sustained) / WAVES * units * (1u << ql);
             const double tile = std::max(multiply, 0.42 * (0.4 + 0.6 * full));
+            // (kQuadLeastUs: one round, one tile)
             const double us = std::ceil(wgs / cus) * (3.8 + tiles_per * tile) + (parts > 1 ? 1.75 + 0.007 * (1u << ql) * parts : 0.0);
-            if (us < best.us) best = QuadPlan{ql, parts, tiles_per, nslab, rbs, us};
+            if (us < best.us) best = so_quad_plan{ql, parts, tiles_per, nslab, rbs, us};
         }
     }
     if (ctx->tune.matmul_quad_rows >= 0 && ctx->tune.matmul_quad_rows <= (int)LOG_WAVES) {
@@ -364,6 +365,8 @@ QuadPlan choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
     return best;
 }
 
+namespace {
+
 template <int ACT>
 so_status launch_quad(so_ctx *ctx, const QuadArgs &a, uint32_t blocks)
 {
@@ -372,10 +375,10 @@ so_status launch_quad(so_ctx *ctx, const QuadArgs &a, uint32_t blocks)
     return SO_OK;
 }
 
-size_t part_bytes(const QuadPlan &p) { return (size_t)p.rbs * p.nslab * p.ks * (1u << p.qw_log2) * 64 * 16; }
-size_t counter_bytes(const QuadPlan &p) { return (size_t)p.rbs * p.nslab * sizeof(uint32_t); }
+size_t part_bytes(const so_quad_plan &p) { return (size_t)p.rbs * p.nslab * p.ks * (1u << p.qw_log2) * 64 * 16; }
+size_t counter_bytes(const so_quad_plan &p) { return (size_t)p.rbs * p.nslab * sizeof(uint32_t); }
 
-so_status workspace(so_ctx *ctx, const so_ellpack *E, uint32_t C, const QuadPlan &p)
+so_status workspace(so_ctx *ctx, const so_ellpack *E, uint32_t C, const so_quad_plan &p)
 {
     if (p.ks == 1) return SO_OK;
     SO_REQUIRE((uint64_t)p.rbs * p.nslab * p.ks < (1ull << 28), "so_matmul: %u x %u output is too large for one launch", E->m, C);
@@ -481,19 +484,15 @@ bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
     return E->quads.d_w != nullptr && E->n != 0 && C >= 4 && C < (1u << 21) && (size_t)ctx->max_lds_bytes >= LDS_BYTES;
 }
 
-double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C) { return choose(ctx, E, C).us; }
+so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C) { return workspace(ctx, E, C, so_matmul_quad_choose(ctx, E, C)); }
 
-so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C) { return workspace(ctx, E, C, choose(ctx, E, C)); }
-
-bool so_matmul_quad_ready(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+bool so_matmul_quad_ready(const so_ctx *ctx, const so_quad_plan &p)
 {
-    const QuadPlan p = choose(ctx, E, C);
     return p.ks == 1 || (ctx->mm_part && ctx->mm_counters && part_bytes(p) <= ctx->mm_part->bytes && counter_bytes(p) <= ctx->mm_counters->bytes);
 }
 
-so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
+so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_plan &p, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
-    const QuadPlan p = choose(ctx, E, C);
     const so_status s = workspace(ctx, E, C, p);
     if (s != SO_OK) return s;
     const so_quads &Q = E->quads;

@@ -203,11 +203,14 @@ so_status so_matvec_columns(so_ctx *ctx, const so_ellpack *E, const float *dX, u
 // csrc/matmul_quad.hip: the quad-union layout and its kernel.
 so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz);
 void so_quads_free(so_ellpack *E);
+// How a launch is split: quads per workgroup (log2), workgroups per output tile and the K tiles of each, slabs of 64 columns, row blocks.
+struct so_quad_plan { uint32_t qw_log2, ks, tiles_per, nslab, rbs; double us; };
+constexpr double kQuadLeastUs = 4.4;                                                  // no plan takes less (estimated)
 bool so_matmul_quad_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
-double so_matmul_quad_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);   // us
-bool so_matmul_quad_ready(const so_ctx *ctx, const so_ellpack *E, uint32_t C);        // the workspace need not grow for this launch
+so_quad_plan so_matmul_quad_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+bool so_matmul_quad_ready(const so_ctx *ctx, const so_quad_plan &p);                  // the workspace need not grow for this launch
 so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
-so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
+so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_plan &p, const float *dX, uint32_t C,
                                 const float *dBias, float *dY, int act);
 
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
