@@ -782,17 +782,17 @@ namespace {
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));   // rows of a dense matrix start anywhere
 
-// Decoding: a workgroup builds kDecodeSpan consecutive elements of W in LDS -- whole rows, or a part of one longer
+// Decoding: a workgroup builds up to kDecodeSpan consecutive elements of W in LDS -- whole rows, or a part of one longer
 // row -- and writes them out once, 16 bytes per lane, past the caches (nontemporal: a plain store of W takes twice as
-// long and pushes the matrix out of the Infinity Cache).  The span starts as zeros and is put back to zeros after each
-// use by clearing what was scattered.  Slots are requested eight per thread at a time, those of the next span while
-// this one is written out.
+// long and pushes the matrix out of the Infinity Cache).
 // Bound by the write of W: 8192 x 8192, 90 % sparse, 50 us (6.4 TB/s of its 322 MB), 80 on buffers not used before;
 // 143 and 114 as a fill of W followed by a scatter of single words into it.  Without the requests ahead the chain
 // length -> slots -> span -> write made it 67 and 140.
 constexpr uint32_t kDecodeSpan = 8192;       // 32 KB: five workgroups per compute unit
 constexpr uint32_t kDecodeSlots = 8;         // slots a thread has in registers
 
+// Several rows per span, a wave takes every fourth.  The span starts as zeros and is put back to zeros after each use by
+// clearing what was scattered.
 __global__ __launch_bounds__(256)
 void ellpack_decode_kernel(const float *__restrict__ Wd, const uint32_t *__restrict__ idx,
                            const uint32_t *__restrict__ nnz, uint32_t m, uint32_t n, uint32_t r,
@@ -802,79 +802,143 @@ void ellpack_decode_kernel(const float *__restrict__ Wd, const uint32_t *__restr
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     f32x4u *span4 = reinterpret_cast<f32x4u *>(span);
     for (uint32_t k = tid; k < kDecodeSpan / 4u; k += 256u) *reinterpret_cast<float4 *>(span + 4u * k) = make_float4(0.f, 0.f, 0.f, 0.f);
-    const uint32_t per_row = (n + kDecodeSpan - 1u) / kDecodeSpan;       // spans of a row (1 when a span holds whole rows)
-    // one row per span: all four waves share it; several: a wave takes every fourth
-    const bool one = rows_per_span == 1u;
-    const uint32_t k0 = one ? tid : lane, kstep = one ? 256u : 64u, first = one ? 0u : wave;
-
-    // Slots k0 + k * kstep .. of one row: columns relative to the span (0xffffffff: no such slot) and values.
-    auto request = [&](uint32_t row, uint32_t from, uint32_t cnt, uint32_t (&at)[kDecodeSlots], float (&v)[kDecodeSlots]) {
-        const uint32_t *ix = idx + (size_t)row * r;
-        const float *wd = Wd + (size_t)row * r;
-#pragma unroll
-        for (uint32_t u = 0; u < kDecodeSlots; ++u) {
-            const uint32_t k = from + k0 + u * kstep;
-            at[u] = 0xffffffffu;
-            if (k < cnt) { at[u] = ix[k]; v[u] = wd[k]; }
-        }
-    };
-    auto rows_of = [&](uint32_t sp, uint32_t &row0, uint32_t &col0) {
-        row0 = per_row == 1u ? sp * rows_per_span : sp / per_row;
-        col0 = per_row == 1u ? 0u : (sp - row0 * per_row) * kDecodeSpan;
-    };
-    uint32_t at[kDecodeSlots], at_next[kDecodeSlots], row0, col0, cnt = 0, cnt_next = 0;
-    float v[kDecodeSlots], v_next[kDecodeSlots];
-    if (one && blockIdx.x < spans) {
-        rows_of(blockIdx.x, row0, col0);
-        cnt = nnz[row0];
-        request(row0, 0, cnt, at, v);
-        if (blockIdx.x + gridDim.x < spans) { rows_of(blockIdx.x + gridDim.x, row0, col0); cnt_next = nnz[row0]; }
-    }
     for (uint32_t sp = blockIdx.x; sp < spans; sp += gridDim.x) {
-        rows_of(sp, row0, col0);
-        const uint32_t rows = min(rows_per_span, m - row0);
-        const uint32_t count = per_row == 1u ? rows * n : min(kDecodeSpan, n - col0);
-        float *out = W + (size_t)row0 * n + col0;
-        // value = false: the same places back to zero
-        auto scatter = [&](uint32_t i, const uint32_t (&a)[kDecodeSlots], const float (&x)[kDecodeSlots], bool value) {
+        const uint32_t row0 = sp * rows_per_span, rows = min(rows_per_span, m - row0), count = rows * n;
+        float *out = W + (size_t)row0 * n;
+        auto scatter = [&](bool value) {               // false: the same places back to zero
+            for (uint32_t i = wave; i < rows; i += 4u) {
+                const uint32_t c = nnz[row0 + i];
+                const uint32_t *ix = idx + (size_t)(row0 + i) * r;
+                const float *wd = Wd + (size_t)(row0 + i) * r;
+                for (uint32_t from = lane; from < c; from += kDecodeSlots * 64u) {
+                    uint32_t at[kDecodeSlots];
+                    float v[kDecodeSlots];
 #pragma unroll
-            for (uint32_t u = 0; u < kDecodeSlots; ++u) {
-                const uint32_t c = a[u] - col0;
-                if (a[u] != 0xffffffffu && c < count) span[i * n + c] = value ? x[u] : 0.0f;
-            }
-        };
-        auto scatter_rest = [&](bool value) {          // what the registers do not hold
-            uint32_t a[kDecodeSlots];
-            float x[kDecodeSlots];
-            for (uint32_t i = first; i < rows; i += one ? 1u : 4u) {
-                const uint32_t c = one ? cnt : nnz[row0 + i];
-                for (uint32_t from = one ? kDecodeSlots * kstep : 0u; from < c; from += kDecodeSlots * kstep) {
-                    request(row0 + i, from, c, a, x);
-                    scatter(i, a, x, value);
+                    for (uint32_t u = 0; u < kDecodeSlots; ++u)
+                        if (from + u * 64u < c) { at[u] = ix[from + u * 64u]; v[u] = wd[from + u * 64u]; }
+#pragma unroll
+                    for (uint32_t u = 0; u < kDecodeSlots; ++u)
+                        if (from + u * 64u < c) span[i * n + at[u]] = value ? v[u] : 0.0f;
                 }
             }
         };
         __syncthreads();                               // the span is all zeros
-        if (one) scatter(0, at, v, true);
-        scatter_rest(true);
+        scatter(true);
         __syncthreads();
-        const uint32_t next = sp + gridDim.x;
-        uint32_t cnt_after = 0;
-        if (one && next < spans) {
-            uint32_t r1, c1;
-            rows_of(next, r1, c1);
-            request(r1, 0, cnt_next, at_next, v_next);
-            if (next + gridDim.x < spans) { rows_of(next + gridDim.x, r1, c1); cnt_after = nnz[r1]; }
-        }
         for (uint32_t k = tid; k < count / 4u; k += 256u) __builtin_nontemporal_store(span4[k], reinterpret_cast<f32x4u *>(out) + k);
         if (tid < (count & 3u)) out[(count & ~3u) + tid] = span[(count & ~3u) + tid];
         __syncthreads();
-        if (one) scatter(0, at, v, false);
-        scatter_rest(false);
-        cnt = cnt_next;
-        cnt_next = cnt_after;
+        scatter(false);
+    }
+}
+
+// A span is (part of) one row; a work item is one of the row's `segs` shares of `per_seg` spans of `width` columns.  The
+// row's slots come in batches of 2048 (eight per thread), the next batch -- of this row, else the next item's first -- on
+// its way while this one is scattered and the span is written out.  Where the columns ascend (SORTED) a batch that reaches
+// past the span is kept for the next one, so every slot is read once however many spans the row has; else each span
+// goes through the whole row.  1024 x 65536, half full: 537 us with the whole row for each span, 360 as a fill and a
+// scatter, 104 so; 10 % full 132, 145 and 53; 64 x 262144, 10 % full 61, 155 and 19.
+template <bool SORTED>
+__global__ __launch_bounds__(256)
+void ellpack_decode_wide_kernel(const float *__restrict__ Wd, const uint32_t *__restrict__ idx, const uint32_t *__restrict__ nnz,
+                                uint32_t n, uint32_t r, float *__restrict__ W, uint32_t width, uint32_t per_seg, uint32_t segs, uint32_t items)
+{
+    constexpr uint32_t kBatch = kDecodeSlots * 256u;
+    __shared__ __attribute__((aligned(16))) float span[kDecodeSpan];
+    const uint32_t tid = threadIdx.x;
+    f32x4u *span4 = reinterpret_cast<f32x4u *>(span);
+    for (uint32_t k = tid; k < kDecodeSpan / 4u; k += 256u) *reinterpret_cast<float4 *>(span + 4u * k) = make_float4(0.f, 0.f, 0.f, 0.f);
+
+    struct Batch { uint32_t at[kDecodeSlots], last; float v[kDecodeSlots]; };      // columns (0xffffffff: no such slot), the last slot's among them, values
+    auto request = [&](uint32_t row, uint32_t from, uint32_t cnt, Batch &b) {
+        const uint32_t *ix = idx + (size_t)row * r;
+        const float *wd = Wd + (size_t)row * r;
 #pragma unroll
-        for (uint32_t u = 0; u < kDecodeSlots; ++u) { at[u] = at_next[u]; v[u] = v_next[u]; }
+        for (uint32_t u = 0; u < kDecodeSlots; ++u) {
+            const uint32_t k = from + tid + u * 256u;
+            b.at[u] = 0xffffffffu;
+            if (k < cnt) { b.at[u] = ix[k]; b.v[u] = wd[k]; }
+        }
+        if (SORTED && from + kBatch < cnt) b.last = ix[from + kBatch - 1u];        // only looked at when the row goes on
+    };
+    // SORTED: the row's first slot with a column of `col` or more
+    auto first_slot = [&](uint32_t row, uint32_t col, uint32_t cnt) {
+        const uint32_t *ix = idx + (size_t)row * r;
+        uint32_t lo = 0, hi = cnt;
+        while (lo < hi) {
+            const uint32_t step = (hi - lo + 255u) / 256u, k = lo + tid * step;
+            const uint32_t below = (uint32_t)__syncthreads_count(k < hi && ix[k] < col);
+            hi = min(hi, lo + below * step);
+            lo = below == 0u ? lo : lo + (below - 1u) * step + 1u;
+        }
+        return lo;
+    };
+    Batch cur, nxt;
+    uint32_t item = blockIdx.x, row, col, col_end, cnt, from, cnt_next = 0, cnt_after = 0;      // cnt_next, cnt_after: rows of the two items to come (segs = 1)
+    const uint32_t stride = gridDim.x;
+    auto place = [&] {
+        row = item / segs;
+        col = (item - row * segs) * per_seg * width;
+        col_end = (uint32_t)min((uint64_t)n, (uint64_t)col + (uint64_t)per_seg * width);
+    };
+    auto look_ahead = [&] {              // what follows the batch in `cur`
+        if (from + kBatch < cnt) request(row, from + kBatch, cnt, nxt);
+        else if (segs == 1u && item + stride < items) request(item + stride, 0, cnt_next, nxt);
+    };
+    place();
+    cnt = nnz[row];
+    from = SORTED && segs > 1u ? first_slot(row, col, cnt) : 0u;
+    request(row, from, cnt, cur);
+    if (segs == 1u && item + stride < items) cnt_next = nnz[item + stride];
+    look_ahead();
+    if (segs == 1u && item + 2u * stride < items) cnt_after = nnz[item + 2u * stride];
+    for (;;) {
+        for (;; col += width) {
+            const uint32_t count = min(width, n - col);
+            __syncthreads();                               // the span is all zeros
+            for (;;) {
+#pragma unroll
+                for (uint32_t u = 0; u < kDecodeSlots; ++u) {
+                    const uint32_t c = cur.at[u] - col;
+                    if (cur.at[u] != 0xffffffffu && c < count) span[c] = cur.v[u];
+                }
+                if (from + kBatch >= cnt || (SORTED && cur.last >= col + count)) break;
+                cur = nxt;
+                from += kBatch;
+                look_ahead();
+            }
+            __syncthreads();
+            float *out = W + (size_t)row * n + col;
+            for (uint32_t k = tid; k < count / 4u; k += 256u) {
+                __builtin_nontemporal_store(span4[k], reinterpret_cast<f32x4u *>(out) + k);
+                span4[k] = f32x4u{0.f, 0.f, 0.f, 0.f};
+            }
+            if (tid < (count & 3u)) {
+                out[(count & ~3u) + tid] = span[(count & ~3u) + tid];
+                span[(count & ~3u) + tid] = 0.0f;
+            }
+            if (col_end - col <= width) break;
+            if (!SORTED && from != 0u) {                   // from the row's start again
+                from = 0;
+                request(row, 0, cnt, cur);
+                look_ahead();
+            }
+        }
+        item += stride;
+        if (item >= items) break;
+        place();
+        if (segs == 1u) {
+            cur = nxt;
+            cnt = cnt_next;
+            cnt_next = cnt_after;
+            from = 0;
+        } else {
+            cnt = nnz[row];
+            from = SORTED ? first_slot(row, col, cnt) : 0u;
+            request(row, from, cnt, cur);
+        }
+        look_ahead();
+        if (segs == 1u && item + 2u * stride < items) cnt_after = nnz[item + 2u * stride];
     }
 }
 
@@ -1203,13 +1267,23 @@ extern "C" so_status so_ellpack_decode(so_ctx *ctx, const so_ellpack *E, float *
     if (total == 0) return SO_OK;
     SO_REQUIRE(dDense != nullptr, "so_ellpack_decode: null output");
     if (E->r == 0) return so_fill_zero(ctx, dDense, total * sizeof(float));
+    const uint32_t cus = (uint32_t)ctx->compute_units;
     // Whole rows per span while they fit, but at least two spans per compute unit where the matrix has them.
     const uint32_t per_row = so_ceil_div(E->n, kDecodeSpan);
-    const uint32_t rows = per_row > 1 ? 1u : std::max(1u, std::min(kDecodeSpan / E->n, so_ceil_div(E->m, 2u * (uint32_t)ctx->compute_units)));
-    const uint64_t spans = per_row > 1 ? (uint64_t)E->m * per_row : so_ceil_div(E->m, rows);
-    SO_REQUIRE(spans < (1ull << 32), "so_ellpack_decode: %u x %u is too large for one launch", E->m, E->n);
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(spans, 5ull * (uint64_t)ctx->compute_units);
-    ellpack_decode_kernel<<<blocks, 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->m, E->n, E->r, dDense, rows, (uint32_t)spans);
+    const uint32_t rows = per_row > 1 ? 1u : std::max(1u, std::min(kDecodeSpan / E->n, so_ceil_div(E->m, 2u * cus)));
+    if (rows > 1) {
+        const uint32_t spans = so_ceil_div(E->m, rows);
+        ellpack_decode_kernel<<<std::min(spans, 5u * cus), 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->m, E->n, E->r, dDense, rows, spans);
+    } else {
+        // spans of equal width (whole cache lines), a row shared by several workgroups where there are few rows
+        const uint32_t width = per_row > 1 ? so_ceil_div(so_ceil_div(E->n, per_row), 64u) * 64u : E->n, spans = so_ceil_div(E->n, width);
+        const uint32_t per_seg = E->m >= 2u * cus ? spans : so_ceil_div(spans, std::min(spans, so_ceil_div(5u * cus, E->m)));
+        const uint32_t segs = so_ceil_div(spans, per_seg);
+        SO_REQUIRE((uint64_t)E->m * segs < (1ull << 31), "so_ellpack_decode: %u x %u is too large for one launch", E->m, E->n);
+        const uint32_t items = E->m * segs, blocks = std::min(items, 5u * cus);
+        if (E->ascending) ellpack_decode_wide_kernel<true><<<blocks, 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->n, E->r, dDense, width, per_seg, segs, items);
+        else ellpack_decode_wide_kernel<false><<<blocks, 256, 0, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->n, E->r, dDense, width, per_seg, segs, items);
+    }
     SO_LAUNCH_CHECK();
     return SO_OK;
 }

@@ -41,3 +41,26 @@ def test_encode_decode_edges(ctx, m, n, keep):
     assert np.array_equal(dR.decode(), dense, equal_nan=True)
     for a in (dW, dWd, dIdx, dNnz, dE, dR):
         a.free()
+
+
+@pytest.mark.parametrize("m,n,keep", [
+    (3, 8193, 1.0), (5, 20000, .4), (2, 30011, .5), (1300, 8200, .02), (600, 9001, .3), (1, 150000, .9), (9, 65536, .25), (1290, 8192, .3)])
+def test_decode_rows_of_several_spans(ctx, m, n, keep):
+    """Rows of several decode spans and of more slots than a workgroup holds at a time (2048), ascending and not, shared by
+    several workgroups (below two rows per compute unit) and not, empty, full, crowded into one span; more rows than workgroups."""
+    rng = np.random.default_rng(m + n)
+    W = datagen.bernoulli_dense(rng, m, n, keep) if keep < 1 else rng.standard_normal((m, n)).astype(np.float32)
+    W[m // 2, : n // 2] = 0
+    W[m // 3, n // 3:] = 0
+    W[(m - 1) // 4] = 0 if m > 4 else 1
+    W[m - 1] = np.arange(n) + 1 if m > 1 else W[m - 1]
+    E = datagen.encode_dense(W)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, m, n, E.r, hipabi.LAYOUT_ROW)
+    assert np.array_equal(dE.decode(), W)
+    for i in range(0, m, max(1, m // 7)):
+        p = rng.permutation(int(E.nnz[i]))
+        E.Wd[i, :len(p)], E.idx[i, :len(p)] = E.Wd[i, p], E.idx[i, p]
+    dR = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, m, n, E.r, hipabi.LAYOUT_ROW)
+    assert np.array_equal(dR.decode(), W)
+    dE.free()
+    dR.free()
