@@ -81,6 +81,30 @@ def test_quad_unordered_repeated_and_special_values(ctx, oracle):
         assert np.abs(Y[fin] - Yo[fin]).max() <= TOL * np.abs(Yo[fin]).max()
 
 
+@pytest.mark.parametrize("C", [4, 5, 66, 131])
+@pytest.mark.parametrize("n,sp", [(40, .5), (700, .8), (2100, .4)])
+def test_quad_outputs_that_meet_a_foreign_infinity(ctx, C, n, sp):
+    """Every column of X has an infinity in a row that half of the matrix's rows do not use: those outputs, NaN as computed
+    with the quad's other rows, are computed again from the row's own nonzeros (up to 1260 of them, 16 lanes a row, groups
+    of four columns, the last group past the end of X's rows), to the same bound."""
+    rng = np.random.default_rng(n + C)
+    m = 90
+    W = sparse_matrix(rng, m, n, sp)
+    j = n // 2
+    W[:, j] = np.where(np.arange(m) % 3 == 1, 0, 2)
+    W[17] = 0
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    E = datagen.encode_dense(W)
+    X[j] = 0
+    ref = W.astype(np.float64) @ X + b[:, None]
+    X[j] = np.where(np.arange(C) % 2, np.inf, -np.inf)
+    Y = quad_matmul(ctx, E, X, b)
+    uses = W[:, j] != 0
+    assert np.array_equal(Y[uses], np.repeat(X[j][None], uses.sum(), axis=0))
+    assert rel_err(Y[~uses], ref[~uses]) <= TOL
+
+
 def test_quad_in_a_launch_graph(ctx, oracle):
     """so_matmul_reserve sizes the workspace of a K split ahead of a recording; replays give the eager launch's bits."""
     rng = np.random.default_rng(3)
