@@ -109,6 +109,9 @@ __device__ __forceinline__ f32x4 exact_outputs(const QuadArgs &a, uint32_t row, 
 // weights and X row bytes of a chunk are requested DEPTH chunks ahead (they come from memory once, so
 // memory's latency has to be covered, not L2's) into a ring of registers, across tile boundaries, and the
 // compiler's own waits would assume the worst over all ways into a ring slot, which is to wait for everything.
+// The ring (v84 .. v95) is also in flight between the blocks, where the compiler believes its registers hold values: it
+// must neither move nor spill them there, nor issue vector memory instructions of its own, which the waits would count.
+// csrc/check_quad_ring.py looks for both in the assembly of every build.
 //
 //   ENTER_S  the run starts at ring slot S: LDS reads of its chunk
 //   CHUNK_S  `n` chunks left, this one's LDS reads under way.  Slot S+1's requests have at least
@@ -240,7 +243,7 @@ void ellpack_matmul_quad_kernel(QuadArgs a)
     const uint32_t wstep = 256u * kw, ostep = 16u * kw, lane4 = lane * 4u, quarter4 = quarter * 4u;
     float w0, w1, w2, w3, w4, w5;
     uint32_t o0, o1, o2, o3, o4, o5;
-    asm volatile(SO_ASK("v84", "v90") SO_ASK("v85", "v91") SO_ASK("v86", "v92") SO_ASK("v87", "v93") SO_ASK("v88", "v94") SO_ASK("v89", "v95")
+    asm volatile("; ring: first requests\n\t" SO_ASK("v84", "v90") SO_ASK("v85", "v91") SO_ASK("v86", "v92") SO_ASK("v87", "v93") SO_ASK("v88", "v94") SO_ASK("v89", "v95")
                  : "={v84}"(w0), "={v85}"(w1), "={v86}"(w2), "={v87}"(w3), "={v88}"(w4), "={v89}"(w5), "={v90}"(o0), "={v91}"(o1), "={v92}"(o2),
                    "={v93}"(o3), "={v94}"(o4), "={v95}"(o5), "+{s[40:41]}"(wp), "+{s[42:43]}"(op)
                  : [lane4] "v"(lane4), [quarter4] "v"(quarter4), [wstep] "s"(wstep), [ostep] "s"(ostep) : "memory", "scc");
@@ -276,7 +279,7 @@ void ellpack_matmul_quad_kernel(QuadArgs a)
         if (t + 1u < t1) fetch(t + 1u);
     }
     // the ring's last requests (and a tail fetch, none): nothing is outstanding from here on
-    asm volatile("s_waitcnt vmcnt(0)" : "+{v84}"(w0), "+{v85}"(w1), "+{v86}"(w2), "+{v87}"(w3), "+{v88}"(w4), "+{v89}"(w5), "+{v90}"(o0), "+{v91}"(o1),
+    asm volatile("; ring: drained\n\ts_waitcnt vmcnt(0)" : "+{v84}"(w0), "+{v85}"(w1), "+{v86}"(w2), "+{v87}"(w3), "+{v88}"(w4), "+{v89}"(w5), "+{v90}"(o0), "+{v91}"(o1),
                  "+{v92}"(o2), "+{v93}"(o3), "+{v94}"(o4), "+{v95}"(o5) : : "memory");
 
     // Sum over the quarters: after the two exchanges quarter q of the wave holds row q, four columns per lane.
