@@ -990,6 +990,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
         if (s != SO_OK) return s;
         if (done) {
             SO_LAUNCH_CHECK();
+            ctx->last_kernel = "columns";
             return SO_OK;
         }
     }
@@ -1009,6 +1010,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
             if (s != SO_OK) return s;
             if (done) {
                 SO_LAUNCH_CHECK();
+                ctx->last_kernel = "merged-window";
                 return SO_OK;
             }
         }
@@ -1021,6 +1023,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
             if (s != SO_OK) return s;
             if (done) {
                 SO_LAUNCH_CHECK();
+                ctx->last_kernel = "window";
                 return SO_OK;
             }
         }
@@ -1029,6 +1032,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     else if (maxvec >= 2 && B % 2 == 0 && (align & 7) == 0) conv_launch<2>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
     else conv_launch<1>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
     SO_LAUNCH_CHECK();
+    ctx->last_kernel = "gather";
     return SO_OK;
 }
 

@@ -365,6 +365,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
+            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Vector ? "vector" : "merged";
             return SO_OK;
         }
     }
@@ -385,6 +386,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
         const so_status st = so_matmul_tiled_launch(ctx, E, dX, C, dBias, dY, act);
         if (st != SO_OK) return st;
         SO_LAUNCH_CHECK();
+        ctx->last_kernel = "tiled";
         return SO_OK;
     }
 
@@ -410,6 +412,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
         }
         if (st != SO_OK) return st;
         SO_LAUNCH_CHECK();
+        ctx->last_kernel = "shared";
         return SO_OK;
     }
     if (row_tiles <= 4ull * (uint64_t)ctx->compute_units && E->max_nnz >= 64)
@@ -418,5 +421,6 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     else if (vec == 2) launch_act<2>(ctx, E, dX, C, dBias, dY, act);
     else launch_act<1>(ctx, E, dX, C, dBias, dY, act);
     SO_LAUNCH_CHECK();
+    ctx->last_kernel = "row";
     return SO_OK;
 }

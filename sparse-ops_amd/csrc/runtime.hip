@@ -201,6 +201,8 @@ so_status so_keep_recorded(so_ctx *ctx, const so_block_ref &block)
     return SO_OK;
 }
 
+extern "C" const char *so_last_kernel(const so_ctx *ctx) { return ctx ? ctx->last_kernel : ""; }
+
 extern "C" so_status so_device_info(so_ctx *ctx, char *name, size_t name_len, int *compute_units)
 {
     SO_REQUIRE(ctx != nullptr, "so_device_info: ctx is null");

@@ -71,6 +71,7 @@ struct so_ctx {
     std::vector<so_block_ref> recorded;          // what the launches of the recording under way use (so_keep_recorded)
     std::string name;
     so_tuning tune;
+    const char *last_kernel = "";                // so_last_kernel
     std::vector<const void *> big_lds_kernels;   // kernels already allowed max_lds_bytes of dynamic LDS on this device
 };
 

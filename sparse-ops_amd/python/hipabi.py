@@ -20,7 +20,7 @@ LAYOUT_ROW, LAYOUT_SLOT, LAYOUT_BINS, LAYOUT_TILED, LAYOUT_RBM, LAYOUT_IDX16 = 1
 SYMBOLS = (
     "so_device_count so_init so_destroy so_last_error so_device_info so_tuning_reload so_malloc so_free so_h2d so_d2h "
     "so_stage_in so_stage_out so_d2d so_fill_zero so_sync so_timer_begin so_timer_end so_ellpack_upload so_ellpack_free "
-    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_matvec so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
+    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
     "so_conv2d so_maxpool so_gap so_add so_act so_transpose so_reverse_axes3 so_copy_rows so_graph_begin so_graph_end "
     "so_graph_launch so_graph_free so_rbm_upload so_rbm_free so_rbm_dims so_conv_plan_set_rbm so_conv_plan_rbm_info").split()
 
@@ -113,6 +113,7 @@ def load_library(path=None):
         fn = getattr(lib, name)
         fn.argtypes = argtypes
         fn.restype = ct.c_int
+    lib.so_last_kernel.argtypes, lib.so_last_kernel.restype = [_vp], ct.c_char_p
     return lib
 
 
@@ -289,6 +290,10 @@ class Context:
 
     def matmul_reserve(self, E, C):
         self._ck(self.lib.so_matmul_reserve(self.h, E.h, C))
+
+    def last_kernel(self):
+        """The kernel that the last matmul or conv2d launched (so_last_kernel)."""
+        return self.lib.so_last_kernel(self.h).decode()
 
     def matvec(self, E, dx, dBias, dy, layout=0):
         self._ck(self.lib.so_matvec(self.h, E.h, dx.ptr, dBias.ptr if dBias else None, dy.ptr, layout))

@@ -42,12 +42,14 @@ def test_columns_match_oracle(ctx, oracle, Cin, Cout, H, Wi, k, s, p, d, sp, B):
         for residual in (None, dR):
             dY.upload(np.full(R.shape, np.nan, np.float32))
             ctx.conv2d(plan, dX, B, dB, dY, "relu", residual=residual)
+            assert ctx.last_kernel() == "columns"
             want = oracle.conv2d_pf(as_oracle(E), og, X, B, b, "none")
             want = np.maximum(want if residual is None else want + R, 0)
             assert np.array_equal(dY.download(), want)
         X[0, 0, 0, 0] = np.inf
         dX.upload(X)
         ctx.conv2d(plan, dX, B, dB, dY, "none")
+        assert ctx.last_kernel() == "columns"
         want = oracle.conv2d_pf(as_oracle(E), og, X, B, b, "none")
         assert np.array_equal(dY.download(), want, equal_nan=True)
         ctx.conv_plan_free(plan)
@@ -79,6 +81,8 @@ def test_streams_are_made_once_per_batch_and_kept(ctx, oracle, ordered):
         try:
             ctx.conv_plan_tune(plan, B)
             ctx.conv2d(plan, dX, B, None, dY, "none")
+            if B < 4:
+                assert ctx.last_kernel() == ("columns" if ordered else "gather")
         finally:
             graph = ctx.graph_end()
         runs.append((graph, dX, dY, oracle.conv2d_pf(as_oracle(E), og, X, B, None, "none")))

@@ -27,6 +27,7 @@ def quad_matmul(ctx, E, X, bias, act="none", rows=None, split=None):
         for _ in range(2):
             dY.upload(np.full((m, C), np.nan, np.float32))
             ctx.matmul(dE, dX, C, dB, dY, act)
+            assert ctx.last_kernel() == "quad"
             outs.append(dY.download())
         for a in (dX, dY, dB):
             if a is not None:
@@ -117,6 +118,7 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         ctx.matmul_reserve(dE, C)
         ctx.graph_begin()
         ctx.matmul(dE, dX, C, None, dY, "tanh")
+        assert ctx.last_kernel() == "quad"
         g = ctx.graph_end()
         for _ in range(3):
             X = rng.standard_normal((1100, C)).astype(np.float32) * 0.1
@@ -148,6 +150,7 @@ def test_no_columns(ctx, forced):
             dY = ctx.array(np.full((300, C), np.nan, np.float32))
             ctx.matmul_reserve(dE, C)
             ctx.matmul(dE, dX, C, dB, dY, "relu")
+            assert ctx.last_kernel() in ("row", "shared")
             assert np.array_equal(dY.download(), np.repeat(np.maximum(b, 0)[:, None], C, axis=1))
             dY.free()
         for a in (dX, dB, dE):
@@ -171,6 +174,7 @@ def test_recording_without_a_reservation(oracle):
         c.graph_begin()
         try:
             c.matmul(dE, dX, C, None, dY)
+            assert c.last_kernel() == ("quad" if reserved else "row")
         finally:
             g = c.graph_end()
         for _ in range(2):
@@ -229,6 +233,7 @@ def test_recorded_graph_outlives_its_workspace(ctx, kernel):
         dS, dL = (ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM) for E in (small, large))
         dX, dY = ctx.array(rng.standard_normal((1100, C)).astype(np.float32)), ctx.empty((300, C))
         ctx.matmul(dS, dX, C, None, dY, "relu")
+        assert ctx.last_kernel() == ("quad" if "QUAD" in kernel else "merged")
         eager = dY.download()
         ctx.graph_begin()
         ctx.matmul(dS, dX, C, None, dY, "relu")
@@ -277,6 +282,7 @@ def test_few_columns_on_the_matvec_kernel(ctx, oracle, m, n, C, sp, act, idx16):
             dX.upload(X)
         dY.upload(np.full((m, C), np.nan, np.float32))
         ctx.matmul(dE, dX, C, dB, dY, act)
+        assert ctx.last_kernel() == "vector"
         Y, Yo = dY.download(), oracle.matmul(as_oracle(E), X, b, act)
         fin = np.isfinite(Yo)
         assert np.array_equal(Y[~fin], Yo[~fin], equal_nan=True)

@@ -32,6 +32,7 @@ def rbm_matmul(ctx, E, X, bias, act="none", split=None, repeat=1):
         for _ in range(repeat):
             dY.upload(np.full((E.m, X.shape[1]), np.nan, np.float32))
             ctx.matmul(dE, dX, X.shape[1], dB, dY, act)
+            assert ctx.last_kernel() == "merged" or dY.nbytes == 0
             outs.append(dY.download())
         for a in (dX, dY, dB):
             if a is not None:
