@@ -75,7 +75,9 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  *        Sums are taken column by column, not in a row's slot order: results agree with
  *        the reference to fp32 round-off (max |y - ref| <= 1e-5 * max |ref|), are not
  *        bit-identical to it, and are the same bits on every launch.  Rows may be in any
- *        order.  Costs about 3x the ROW arrays in HBM; with it so_matmul keeps a
+ *        order.  Costs about 3x the ROW arrays in HBM -- 1.4x for the first copy, more where rows hold few
+ *        nonzeros, and at most 4x for the second, which a matrix that would need more (about 99 % sparse) or that
+ *        finds no room for it is kept without; with the layout so_matmul keeps a
  *        workspace in the context that grows on first use of a larger output.
  * IDX16: a second copy of the columns in 16 bits (needs n <= 65536; costs 2 bytes per slot,
  *        and as much again for the SLOT copy when that is asked for too).  so_matvec then

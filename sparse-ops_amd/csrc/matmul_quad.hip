@@ -460,6 +460,12 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
     so_quads &Q = E->quads;
     Q.nquads = so_ceil_div(E->m, 4);
     Q.ntiles = std::max(1u, so_ceil_div(E->n, KT));
+    // The tables have an entry per (quad, tile) and a run of columns there is at least one chunk of 272 bytes, so the copy
+    // of a very sparse matrix is many times the matrix (65536 x 65536, 10 nonzeros a row: 270 MB beside 5), while the
+    // kernel would multiply padding: such a handle does without.  Four times the nonzeros' values and columns is
+    // reached at about 8 nonzeros per run (99.2 % sparse); a mebibyte is no matter.
+    const uint64_t most = std::max<uint64_t>(1u << 20, 32 * E->total_nnz);
+    if ((uint64_t)Q.nquads * Q.ntiles * sizeof(uint2) > most) { Q = so_quads(); return SO_OK; }
     std::vector<uint32_t> steps((size_t)Q.nquads * Q.ntiles, 0);
     so_parallel(Q.nquads, E->total_nnz, [&](uint32_t q0, uint32_t q1) {
         std::vector<Entry> tmp;
@@ -473,8 +479,8 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
         info[k] = make_uint2((uint32_t)chunks, units);
         chunks += (units + 3) / 4;
         Q.total_units += units;
-        if (chunks > 0xfffff000ull) { so_set_error("so_ellpack_upload: matrix too large for the RBM layout"); return SO_ERR_INVALID; }
     }
+    if (chunks > 0xfffff000ull || chunks * 272 + info.size() * sizeof(uint2) > most) { Q = so_quads(); return SO_OK; }
     // padding steps: zero weights on the tile's first row
     // (the three arrays in one allocation and one copy: each of either costs a small matrix a tenth of a millisecond)
     const size_t w_bytes = (size_t)(chunks + SLACK) * 256, off_bytes = (size_t)(chunks + SLACK) * 16;
@@ -498,7 +504,7 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
     });
     void *p = nullptr;
     const so_status s = so_malloc(ctx, blob.size(), &p);
-    if (s != SO_OK) return s;
+    if (s != SO_OK) { Q = so_quads(); return s; }
     Q.d_w = (float *)p;
     Q.d_off = (uint32_t *)((char *)p + w_bytes);
     Q.d_info = (uint2 *)((char *)p + w_bytes + off_bytes);

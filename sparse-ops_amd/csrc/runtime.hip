@@ -744,7 +744,15 @@ extern "C" so_status so_ellpack_upload(so_ctx *ctx, const float *Wd, const uint3
 
         if (s == SO_OK && (layouts & SO_LAYOUT_TILED) && m > 0) s = build_tiled(ctx, E, Wd, idx, nnz);
         if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_rbmm_build(ctx, E, Wd, idx, nnz);
-        if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) s = so_quads_build(ctx, E, Wd, idx, nnz);
+        if (s == SO_OK && (layouts & SO_LAYOUT_RBM) && m > 0) {
+            // the layout's second copy: where there is no memory for it the handle does without
+            try {
+                s = so_quads_build(ctx, E, Wd, idx, nnz);
+            } catch (const std::bad_alloc &) {
+                s = SO_ERR_OOM;
+            }
+            if (s == SO_ERR_OOM) { (void)hipGetLastError(); so_quads_free(E); s = SO_OK; }
+        }
     } catch (const std::exception &e) {                  // a builder ran out of host memory, on whichever thread
         so_set_error("so_ellpack_upload: building the layouts failed: %s", e.what());
         s = SO_ERR_OOM;

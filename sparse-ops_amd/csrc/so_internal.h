@@ -153,8 +153,8 @@ struct so_ellpack {
     uint16_t *d_idxT16 = nullptr;// [r*m] the same for d_idxT (SO_LAYOUT_SLOT with SO_LAYOUT_IDX16)
     so_bin bins[4];              // SO_LAYOUT_BINS
     so_tiled tiled;              // SO_LAYOUT_TILED
-    so_rbmm rbmm;                // SO_LAYOUT_RBM, where that kernel may be the faster one
-    so_quads quads;              // SO_LAYOUT_RBM
+    so_rbmm rbmm;                // SO_LAYOUT_RBM
+    so_quads quads;              // SO_LAYOUT_RBM, unless the matrix is too sparse for it (d_w is null)
 };
 
 // Row-block-merged re-encoding of a matrix (include/rbm_conv.hpp:8-27 of the reference), flattened:

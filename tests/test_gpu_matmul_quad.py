@@ -138,6 +138,28 @@ def test_quad_in_a_launch_graph(ctx, oracle):
         dE.free()
 
 
+@pytest.mark.parametrize("m,n,per_row,quads", [(65536, 65536, 10, False), (2048, 16384, 16, False), (2048, 16384, 60, False),
+                                               (2048, 16384, 400, True), (300, 9000, 3, True)])
+def test_very_sparse_matrices_do_without_the_quads(ctx, oracle, m, n, per_row, quads):
+    """Few nonzeros per (quad, 256 columns): the copy would be many times the matrix.  By the table's size alone, by the
+    chunks counted, and not: dense enough, too small to matter.  The handle works either way, forced or not."""
+    rng = np.random.default_rng(per_row)
+    idx = np.sort(rng.choice(n // per_row, (m, per_row)).astype(np.uint32) + np.arange(per_row, dtype=np.uint32) * (n // per_row), axis=1)
+    Wd, nnz = rng.standard_normal((m, per_row)).astype(np.float32), np.full(m, per_row, np.uint32)
+    X = rng.standard_normal((n, 8)).astype(np.float32)
+    dE = ctx.upload_ellpack(Wd, idx, nnz, m, n, per_row, RBM)
+    dX, dY = ctx.array(X), ctx.empty((m, 8))
+    ref = (Wd[:, :, None].astype(np.float64) * X[idx]).sum(axis=1)
+    for forced in (None, "1"):
+        with ctx.tuning(SPARSEOPS_MATMUL_QUAD=forced):
+            ctx.matmul_reserve(dE, 8)
+            ctx.matmul(dE, dX, 8, None, dY)
+            assert forced is None or (ctx.last_kernel() == "quad") == quads
+            assert rel_err(dY.download(), ref) <= TOL
+    for a in (dX, dY, dE):
+        a.free()
+
+
 @pytest.mark.parametrize("forced", [None, "SPARSEOPS_MATMUL_QUAD", "SPARSEOPS_MATMUL_RBM"])
 def test_no_columns(ctx, forced):
     """A matrix without columns has no row of X to read: the layout's kernels, which read ahead, are not for it."""
