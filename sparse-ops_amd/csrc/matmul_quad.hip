@@ -422,24 +422,38 @@ so_status workspace(so_ctx *ctx, const so_ellpack *E, uint32_t C, const so_quad_
 
 struct Entry { uint32_t col, row; float w; };
 
-// The union columns of quad q, ascending, with up to four weights each (a column that a row names twice
-// gets two steps): calls step(col, weights) for every step.
+// Rows with ascending columns: tile(t, mask, weights) for every tile of quad q, with a bit per union column and, where
+// WEIGHTS, the four weights of each (weights[4 * column ..], zeros elsewhere: tile puts back zeros where it takes them).
+template <bool WEIGHTS, class F>
+void walk_tiles(const so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz, uint32_t q, float *weights, F &&tile)
+{
+    static_assert(KT == 256, "four words of columns per tile");
+    const uint32_t r0 = q * 4, rows = std::min(4u, E->m - r0);
+    uint32_t pos[4] = {0, 0, 0, 0};
+    for (uint32_t t = 0; t < E->quads.ntiles; ++t) {
+        const uint32_t base = t * KT;
+        uint64_t mask[4] = {0, 0, 0, 0};
+        for (uint32_t i = 0; i < rows; ++i) {
+            const uint32_t *ix = idx + (size_t)(r0 + i) * E->r;
+            const float *wd = Wd + (size_t)(r0 + i) * E->r;
+            uint32_t k = pos[i];
+            for (; k < nnz[r0 + i] && ix[k] - base < KT; ++k) {
+                const uint32_t c = ix[k] - base;
+                mask[c >> 6] |= 1ull << (c & 63);
+                if (WEIGHTS) weights[4 * c + i] = wd[k];
+            }
+            pos[i] = k;
+        }
+        tile(t, mask, weights);
+    }
+}
+
+// Rows in any order: the union columns of quad q, ascending, with up to four weights each (a column that a row names
+// twice gets two steps): calls step(col, weights) for every step.
 template <class F>
 void walk_quad(const so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz, uint32_t q, std::vector<Entry> &tmp, F &&step)
 {
     const uint32_t r0 = q * 4, rows = std::min(4u, E->m - r0);
-    if (E->ascending) {
-        const uint32_t *ip[4]; const float *wp[4]; uint32_t left[4] = {0, 0, 0, 0};
-        for (uint32_t i = 0; i < rows; ++i) { ip[i] = idx + (size_t)(r0 + i) * E->r; wp[i] = Wd + (size_t)(r0 + i) * E->r; left[i] = nnz[r0 + i]; }
-        for (;;) {
-            uint32_t col = 0xffffffffu;
-            for (uint32_t i = 0; i < rows; ++i) if (left[i]) col = std::min(col, *ip[i]);
-            if (col == 0xffffffffu) return;
-            float w[4] = {0.f, 0.f, 0.f, 0.f};
-            for (uint32_t i = 0; i < rows; ++i) if (left[i] && *ip[i] == col) { w[i] = *wp[i]; ++ip[i]; ++wp[i]; --left[i]; }
-            step(col, w);
-        }
-    }
     tmp.clear();
     for (uint32_t i = 0; i < rows; ++i)
         for (uint32_t k = 0; k < nnz[r0 + i]; ++k) tmp.push_back({idx[(size_t)(r0 + i) * E->r + k], i, Wd[(size_t)(r0 + i) * E->r + k]});
@@ -469,7 +483,14 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
     std::vector<uint32_t> steps((size_t)Q.nquads * Q.ntiles, 0);
     so_parallel(Q.nquads, E->total_nnz, [&](uint32_t q0, uint32_t q1) {
         std::vector<Entry> tmp;
-        for (uint32_t q = q0; q < q1; ++q) walk_quad(E, Wd, idx, nnz, q, tmp, [&](uint32_t col, const float *) { ++steps[(size_t)q * Q.ntiles + col / KT]; });
+        for (uint32_t q = q0; q < q1; ++q) {
+            uint32_t *const count = steps.data() + (size_t)q * Q.ntiles;
+            if (E->ascending)
+                walk_tiles<false>(E, Wd, idx, nnz, q, nullptr, [&](uint32_t t, const uint64_t *mask, float *) {
+                    for (int k = 0; k < 4; ++k) count[t] += (uint32_t)__builtin_popcountll(mask[k]);
+                });
+            else walk_quad(E, Wd, idx, nnz, q, tmp, [&](uint32_t col, const float *) { ++count[col / KT]; });
+        }
     });
     std::vector<uint2> info(steps.size());
     uint64_t chunks = 0;
@@ -490,16 +511,31 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
     std::memcpy(off + off_bytes, info.data(), info.size() * sizeof(uint2));
     so_parallel(Q.nquads, E->total_nnz, [&](uint32_t q0, uint32_t q1) {
         std::vector<Entry> tmp;
+        std::vector<float> weights(4 * KT, 0.0f);
+        const auto put = [&](size_t s, uint32_t c, const float *wt) {       // step s: column c of its tile
+            const size_t chunk = s >> 4, unit = (s >> 2) & 3, quarter = s & 3;
+            std::memcpy(w + chunk * 64 + quarter * 16 + unit * 4, wt, 16);
+            off[chunk * 16 + quarter * 4 + unit] = (uint8_t)c;
+        };
         for (uint32_t q = q0; q < q1; ++q) {
+            const uint2 *const runs = info.data() + (size_t)q * Q.ntiles;
             uint32_t tile = 0xffffffffu;
             size_t s = 0;
-            walk_quad(E, Wd, idx, nnz, q, tmp, [&](uint32_t col, const float *wt) {
-                if (col / KT != tile) { tile = col / KT; s = (size_t)info[(size_t)q * Q.ntiles + tile].x * 16; }
-                const size_t c = s >> 4, unit = (s >> 2) & 3, quarter = s & 3;
-                for (int i = 0; i < 4; ++i) w[c * 64 + quarter * 16 + unit * 4 + i] = wt[i];
-                off[c * 16 + quarter * 4 + unit] = (uint8_t)(col - tile * KT);
-                ++s;
-            });
+            if (E->ascending)
+                walk_tiles<true>(E, Wd, idx, nnz, q, weights.data(), [&](uint32_t t, const uint64_t *mask, float *wt) {
+                    s = (size_t)runs[t].x * 16;
+                    for (uint32_t k = 0; k < 4; ++k)
+                        for (uint64_t left = mask[k]; left != 0; left &= left - 1) {
+                            const uint32_t c = k * 64 + (uint32_t)__builtin_ctzll(left);
+                            put(s++, c, wt + 4 * c);
+                            std::memset(wt + 4 * c, 0, 16);
+                        }
+                });
+            else
+                walk_quad(E, Wd, idx, nnz, q, tmp, [&](uint32_t col, const float *wt) {
+                    if (col / KT != tile) { tile = col / KT; s = (size_t)runs[tile].x * 16; }
+                    put(s++, col - tile * KT, wt);
+                });
         }
     });
     void *p = nullptr;
