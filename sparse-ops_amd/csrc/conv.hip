@@ -974,13 +974,14 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     if (g.Cout == 0 || ncols == 0) return SO_OK;
     SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
     SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
-    // The column kernel where the plan has its streams for this batch: below four entries always (the windowed kernel
-    // does not take them), at four where its shorter chains on more waves win -- the windowed kernel's time there is
-    // about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (7x7x512 27.6 against 22.8 us, 14x14x256
-    // 17.5 against 24.4).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
+    // The column kernel where the plan has its streams for this batch: below four entries, which the windowed kernel does
+    // not take, where it pays against the gather kernel (so_conv_columns_pays), at four where its shorter chains on more
+    // waves win -- the windowed kernel's time there is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the
+    // chip (7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
     if (so_conv_columns_for(plan, B) && ctx->tune.conv_columns != 0) {
-        bool use = B < 4 || plan->win.cc == 0 || ctx->tune.conv_columns == 1;
-        if (!use && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
+        const bool alone = B < 4 || plan->win.cc == 0;           // no windowed kernel: else the gather kernel
+        bool use = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
+        if (!use && !alone && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
             const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw, B), (uint64_t)ctx->compute_units);
             use = so_conv_columns_estimate(ctx, plan, B) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
         }

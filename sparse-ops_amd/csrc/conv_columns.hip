@@ -283,7 +283,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
 
 namespace {
 
-struct ColShape { uint32_t G, waves; size_t lds; double us; };
+struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 
 // Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
 // longest chain at 12 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
@@ -292,20 +292,42 @@ struct ColShape { uint32_t G, waves; size_t lds; double us; };
 ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
 {
     const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
-    ColShape best{16, 16, 0, 1e30};
+    ColShape best{16, 16, 0, 1e30, 1.0};
     for (uint32_t G = 16; G >= 4; G /= 2) {
-        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0};
+        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0, 0.0};
         s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
         const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
         const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
-        const double rounds = std::ceil(wgs / (cus * fit)), resident = std::min(fit, std::ceil(wgs / cus));
-        s.us = 3.0 + rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.012, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        const double resident = std::min(fit, std::ceil(wgs / cus));
+        s.rounds = std::ceil(wgs / (cus * fit));
+        s.us = 3.0 + s.rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.012, 0.0075 * std::max(1.0, resident * G / 4.0)));
         if (s.us < best.us) best = s;
     }
     return best;
 }
 
 } // namespace
+
+// Whether the kernel is taken before the gather kernel: both walk a channel's entries for every output, this one after a
+// copy of the window, which entries enough repay -- more of them where the gather kernel has two or four batch entries to
+// fetch at once, or no taps that share cache lines to fetch them from.  us, gather kernel / this one, at batch 1 and 2:
+//   one round of workgroups: 64 x 56 x 56 -> 64, 3x3, 116 entries a channel 21.2 / 8.5 and 22.7 / 13.3; 7 -> 8 at 31 x 30, 3x3/2, 31 entries
+//   6.7 / 3.7 and 6.8 / 4.1; 5 -> 47 at 14 x 10, 3x3/2, 9 entries 4.1 / 3.4 and 4.1 / 3.5; 4 -> 314 at 34 x 38, 1x1/2, 4 entries
+//   3.3 / 3.5 and 3.4 / 4.8; a large window for few entries: 587 -> 359 at 19 x 17, 1x1/2, 30 entries 6.8 / 8.8 and 5.5 / 13.4,
+//   106 -> 41 at 123 x 150, 3x3/2, 48 entries 13.1 / 14.9 and 17.8 / 42;
+//   more rounds, 3x3 to 7x7: 3 -> 16 at 512 x 512, 13 entries 39.7 / 45.7 and 42 / 86; 3 -> 32 at 1000 x 1000, 19 entries 243 / 325 and
+//   309 / 638; 7 -> 220 at 450 x 451, /2, 32 entries 185 / 158 and 197 / 285; 17 -> 5 at 651 x 456, /2, 75 entries 24.6 / 17.6 and 25.1 / 26.2;
+//   34 -> 116 at 160 x 207, 168 entries 224 / 91 and 327 / 228; 1x1: 33 -> 197 at 509 x 526, /2, 10 entries 97 / 695 and 131 / 1121; 63 -> 74
+//   at 92 x 74, 63 entries 13.4 / 14.8 and 20 / 27; 214 -> 12 at 77 x 77, 214 entries 21.8 / 10.2 and 29.6 / 9.4.  At batch 4 (plans without
+//   the windowed layout): 72 entries 133 / 170, 75 29.5 / 28.0, 118 54.5 / 46.6, 147 79 / 72.
+bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B)
+{
+    const so_conv_columns &c = plan->col[B - 1];
+    const double entries = (double)plan->E->total_nnz / plan->g.Cout, window = (double)c.cc * c.nch * c.PE * B;
+    if (entries < 8.0 || window > 480.0 * entries) return false;
+    const double least = B == 4 ? 100.0 : B == 2 || plan->g.kH * plan->g.kW == 1 ? 64.0 : 20.0;
+    return entries >= least || column_shape(ctx, plan, c).rounds <= 1.0;
+}
 
 double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, plan->col[B - 1]).us; }
 

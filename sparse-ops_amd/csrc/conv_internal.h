@@ -62,6 +62,7 @@ void so_conv_columns_free(so_conv_plan *plan);
 so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
                                 const std::vector<float> &Wd, uint32_t B);
 const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B);  // null: the plan has no streams for the batch
+bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);            // against the gather kernel
 double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);      // us
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done);

@@ -102,3 +102,39 @@ def test_streams_are_made_once_per_batch_and_kept(ctx, oracle, ordered):
         dY.free()
     ctx.conv_plan_free(plan)
     dE.free()
+
+
+@pytest.mark.parametrize("Cin,Cout,H,Wi,k,s,per_row,kernels", [        # kernels at batch 1, 2 and 3
+    (16, 96, 200, 190, 1, 1, 6, "gather gather gather"),               # short rows, many workgroups
+    (24, 200, 150, 180, 1, 2, 12, "gather gather gather"), (3, 96, 200, 190, 3, 1, 12, "gather gather gather"),
+    (8, 128, 120, 130, 3, 1, 36, "columns gather columns"),            # enough for one entry of the batch, not for a pair
+    (16, 64, 120, 130, 3, 1, 90, "columns columns columns"),
+    (5, 40, 14, 10, 3, 2, 9, "columns columns columns"), (5, 40, 14, 10, 3, 2, 5, "gather gather gather"),   # one round
+    (580, 40, 19, 17, 1, 2, 30, "gather gather gather")])              # one round, a large window for few entries
+def test_small_batches_take_the_faster_kernel(ctx, oracle, Cin, Cout, H, Wi, k, s, per_row, kernels):
+    """A plan tuned for a small batch keeps to the gather kernel where rows are too short for the column kernel's copy of the
+    window, and the two give the same bits."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(per_row)
+    Wc = np.zeros((Cout, Cin * k * k), np.float32)
+    for row in Wc:
+        row[rng.permutation(Wc.shape[1])[:per_row]] = rng.standard_normal(per_row)
+    E = datagen.encode_dense(Wc)
+    g, og = (f(Cin, Cout, k, k, H, Wi, (s, s), (k // 2, k // 2), (1, 1)) for f in (hipabi.conv_geom, ocg))
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    for B, kernel in zip((1, 2, 3), kernels.split()):
+        plan = ctx.conv_plan(dE, g)
+        ctx.conv_plan_tune(plan, B)
+        X = rng.standard_normal((Cin, H, Wi, B)).astype(np.float32)
+        dX, dY = ctx.array(X), ctx.empty((Cout, g.H_out, g.W_out, B))
+        want = oracle.conv2d_pf(as_oracle(E), og, X, B, None, "none")
+        for forced in (None, "0", "1"):
+            with ctx.tuning(**({"SPARSEOPS_CONV_COLUMNS": forced} if forced else {})):
+                dY.upload(np.full(want.shape, np.nan, np.float32))
+                ctx.conv2d(plan, dX, B, None, dY, "none")
+                assert ctx.last_kernel() == (kernel if forced is None else "gather" if forced == "0" else "columns")
+                assert np.array_equal(dY.download(), want)
+        ctx.conv_plan_free(plan)
+        dX.free()
+        dY.free()
+    dE.free()
