@@ -53,6 +53,31 @@ def test_quad_shapes(ctx, oracle, m, n, C, sp, rows, split):
     assert rel_err(Y, oracle.matmul(as_oracle(E), X, b, "relu" if split == 3 else "none")) <= TOL
 
 
+def test_quad_multiply_adds_are_fused_and_keep_subnormals(ctx, oracle):
+    """Rows i of a quad with nonzeros in columns i and i + 4: union steps of one quarter of one chunk, so an output is
+    one chain of two multiply-adds, and its bits are the in-order oracle's (fmaf) -- with weights, X and results below
+    the normal range, and with second products that nearly cancel the first."""
+    rng = np.random.default_rng(5)
+    m, n, C = 512, 8, 64
+    rows = np.arange(m)
+    W = np.zeros((m, n), np.float32)
+    for k in (0, 4):
+        W[rows, rows % 4 + k] = np.ldexp(rng.uniform(1, 2, m), rng.integers(-148, 10, m))
+    X = np.ldexp(rng.uniform(-2, 2, (n, C)), rng.integers(-148, 10, (n, C))).astype(np.float32)
+    W[::2, :] = np.where(W[::2] != 0, rng.uniform(1, 2, (m // 2, n)), 0)
+    X[4:, ::2] = -X[:4, ::2]
+    W[::8, 4] = W[::8, 0] * np.float32(1 + 2.0 ** -22)
+    E = datagen.encode_dense(W)
+    want = oracle.matmul(as_oracle(E), X, None, "none")
+    tiny = np.float32(np.finfo(np.float32).tiny)
+    for a in (E.Wd, X, want):
+        assert ((a != 0) & (np.abs(a) < tiny)).sum() > 10
+    fused = W.astype(np.float64) @ X                       # products are exact here: what separate roundings would change
+    assert (want != (W[rows, rows % 4, None] * X[rows % 4] + W[rows, rows % 4 + 4, None] * X[rows % 4 + 4])).sum() > 100
+    assert np.abs(want - fused).max() <= 2.0 ** -23 * np.abs(fused).max()
+    assert np.array_equal(quad_matmul(ctx, E, X, None), want)
+
+
 def test_quad_unordered_repeated_and_special_values(ctx, oracle):
     """Reversed rows, a column that a row names twice, empty rows, a dense row; and an infinity in X reaches exactly
     the rows that use it, although a quad's other rows meet it with a zero weight."""
