@@ -67,12 +67,12 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  * RBM  : row-block-merged, the reference's blocked-CSC idea (include/rbm_conv.hpp:8-27,
  *        src/layers/rbm_conv.cpp:7-73) for so_matmul: rows in blocks of 128, a block's used
  *        columns walked once, each X row segment loaded once and multiplied into every row
- *        of the block that has a nonzero there.  The fastest so_matmul for large matrices;
- *        so_matmul uses it whenever it is present and the launch covers most of the chip.
- *        The layout also holds a second copy for smaller launches: quads of four rows with the
- *        union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip);
- *        so_matmul takes whichever of the two, or the kernels of the other layouts, is fastest.
- *        Sums are taken column by column, not in a row's slot order: results agree with
+ *        of the block that has a nonzero there.  The fastest so_matmul for large, very sparse matrices.
+ *        The layout also holds a second copy for smaller launches and fuller matrices: quads of four rows
+ *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip).
+ *        so_matmul takes whichever of the two, so_matvec's row kernel (one to three columns) or the kernels
+ *        of the other layouts it estimates to be the fastest.
+ *        Sums are not taken in a row's slot order: results agree with
  *        the reference to fp32 round-off (max |y - ref| <= 1e-5 * max |ref|), are not
  *        bit-identical to it, and are the same bits on every launch.  Rows may be in any
  *        order.  Costs about 3x the ROW arrays in HBM -- 1.4x for the first copy, more where rows hold few

@@ -285,12 +285,13 @@ namespace {
 
 enum class RbmKernel { None, Merged, Quad, Vector };
 
-// Which of the RBM layout's two kernels a launch takes, or None for the kernels below, by estimated time (us).
-// Both sides of each line were measured on the shapes the quad kernel's model was fitted to (csrc/matmul_quad.hip),
-// us with the weights out of L2:
-//   quad against the row kernel: 2048 x 2048 x 64 at 95 / 90 / 80 / 50 % sparse 8.6 / 9.4 / 10.5 / 13.0 against
-//   6.7 / 14.2 / 17.4 / 63.4; 1024 x 1024 x 64 at 90 / 70 / 50 % 7.1 / 7.6 / 7.8 against 5.3 / 9.5 / 13.4 -- the row
-//   kernel moves 256 bytes per nonzero and 64 columns at about 11 TB/s, and a row takes 18 ns per nonzero on its own;
+// Which of the three kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
+// time.  Both sides of each line were measured, us with one handle launched again and again, in brackets with 48 handles
+// and X in turn, whose weights come from memory:
+//   quad against the row kernel: 2048 x 2048 x 64 at 95 / 90 / 80 / 50 % sparse 8.1 / 8.8 / 10.1 / 11.7 [8.6 / 9.8 / 11.3 / 13.5]
+//   against 6.6 / 9.9 / 16.9 / 35.6 [9.2 / 15.5 / 39.9 / 85.4]; 1024 x 1024 x 64 at 90 / 70 / 50 % 7.0 / 7.5 / 7.8 [7.3 / 7.8 / 8.1]
+//   against 5.1 / 9.1 / 13.0 [7.1 / 14.2 / 25.7] -- the row kernel moves 256 bytes per nonzero and 64 columns at about
+//   11 TB/s (half of that with the weights from memory), and a row takes 18 ns per nonzero on its own;
 //   quad against row-block-merged: 4096 x 4096 x 256 at 90 / 80 / 70 / 50 % 45 / 60 / 72 / 91 against 29 / 48 / 65 / 97
 //   -- 2.85 us per million (nonzero, 64 columns) on top of 9.5, and no faster on fewer workgroups than compute units.
 //   One to three columns: so_matvec's row kernel on each, which spreads a row over the lanes, from rows of 64 nonzeros
@@ -354,7 +355,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     SO_REQUIRE(((uint64_t)E->m / 4 + 8) * ((uint64_t)C / 64 + 1) < (1ull << 31), "so_matmul: %u x %u output is too large for one launch", E->m, C);
 
     // The kernels of the RBM layout, on handles uploaded with it (accurate to fp32 round-off, not bit-identical to
-    // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids both, =1
+    // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids all three, =1
     // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one).
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
         so_quad_plan plan;

@@ -3,7 +3,7 @@
 // Four consecutive rows (a quad) share one list of columns: the union of their nonzero columns, each
 // with the four rows' weights (zero where a row has none).  v_mfma_f32_4x4x1_16b_f32 multiplies four
 // weights by 64 values of an X row in 8 clocks of a SIMD, in plain fp32 with one rounding per
-// multiply-add (checked bit for bit against fmaf, subnormals included), so one union column costs 8
+// multiply-add, subnormals kept (tests/test_gpu_matmul_quad.py compares with fmaf bit for bit), so one union column costs 8
 // clocks per 64 dense columns whatever it holds: 2 rows' worth of useful multiply-adds at 50 % density,
 // 1.58 at 30 %, 1.36 at 20 %, 1.16 at 10 %.  There is nothing to issue per nonzero -- no M0 write, no
 // DPP multiply-add -- which is what bounds the row-block-merged kernel (csrc/matmul_rbm.hip).
@@ -22,17 +22,18 @@
 // weights, one word of four X row bytes per quarter, four v_perm that turn them into LDS addresses.
 // The quarters hold partial sums over a quarter of the steps each and are added at the end.
 //
-// What bounds it.  Large launches: the matrix pipe, 69 % busy at 4096 x 4096 x 256, 50 % dense (91 us; the
-// counters' other 31 %: a vector instruction takes 4-5 clocks from the MFMAs, they do not overlap on a SIMD --
+// What bounds it.  Large launches: the matrix pipe, 69 % busy at 4096 x 4096 x 256, 50 % dense (86 us;
+// profiles/ellpack_matmul_quad__4096sq_c256_50pct__pmc.txt; the other 31 %: a vector instruction takes 4-5 clocks from the MFMAs, they do not overlap on a SIMD --
 // 9.95 clocks per MFMA with one address add per 4 of them, 8.7 without, 8.2 with nothing but MFMAs -- and
 // 0.7 us per tile of barrier, first LDS reads and the slowest wave; without the stream or the X loads the
 // launch takes 87).  Small ones: latencies in a row -- launch 2.5 us, first loads 1.5, exchange of partial tiles 3.
 // Two workgroups of 8 waves per compute unit with 128-row tiles instead of one of 16 measured the same or up to 5 %
 // slower; the compiler's waits (it waits for all outstanding loads at every chunk) nearly twice the time.
 //
-// Measured, weights out of L2, 64 dense columns, before (row kernel) and now: 2048 x 2048 at 90 / 80 / 50 %
-// sparse 14.2 / 17.4 / 63.4 us and 9.1 / 10.4 / 12.3 (0.84 GFLOP of nonzeros at 80 %: 21 TFLOP/s); 1024 x 1024 at
-// 50 % 13.4 and 7.9; 4096 x 784 x 256 at 90 % (K-tiled kernel) 15.2 and 11.9; 10 x 4096 x 256 (shared gather) 8.6 and 7.5.
+// Measured, one handle launched again and again, 64 dense columns, before (row kernel) and now: 2048 x 2048 at 90 / 80 / 50 %
+// sparse 9.9 / 16.9 / 35.6 us and 8.8 / 10.1 / 11.7 (0.107 GFLOP of nonzeros at 80 %: 10.7 TFLOP/s); 1024 x 1024 at 50 %
+// 13.0 and 7.8; with the weights from memory 15.5 / 39.9 / 85.4 and 9.8 / 11.3 / 13.5; 25.7 and 8.1.  4096 x 784 x 256 at 90 %
+// (K-tiled kernel) 15.2 and 11.9; 10 x 4096 x 256 (shared gather) 8.6 and 7.5.
 //
 // The order of summation differs from the reference's slot order: results agree with it to fp32
 // round-off and are the same bits on every launch.  A zero weight times a non-finite X value would leave
@@ -364,9 +365,9 @@ void ellpack_matmul_quad_kernel(QuadArgs a)
 
 // Rows per workgroup and K split by estimated time (us).  The model -- rounds of one workgroup per compute unit,
 // each with its start-up and, per tile, the larger of the multiply-adds and of what a tile's X values take to
-// arrive; for a split the exchange of partial tiles -- was fitted to 900 launches over 44 shapes (10..4096 rows,
-// 512..4096 columns, 4..256 dense columns, 50-95 % sparse): 5.8 % r.m.s., and its choice takes 2 % longer than
-// the best one on average.
+// arrive; for a split the exchange of partial tiles -- was fitted to launches of 10..4096 rows, 512..4096 columns, 4..256
+// dense columns, 50-95 % sparse.  Over the 18 shapes of profiles/matmul_quad__plans.txt its choice takes 1.4 % longer than the
+// best of all plans on average, 6 % at most.
 so_quad_plan so_matmul_quad_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;

@@ -17,7 +17,7 @@ struct so_tuning {
     int matmul_tiled = -1;   // SPARSEOPS_MATMUL_TILED: 1 forces the LDS-staged kernel, 0 forbids it
     int matmul_vec = 0;      // SPARSEOPS_MATMUL_VEC: 1 or 2 columns per lane at most
     int matmul_share = -1;   // SPARSEOPS_MATMUL_SHARE: 0 forbids the shared-gather kernel for few-row launches
-    int matmul_rbm = -1;     // SPARSEOPS_MATMUL_RBM: 0 forbids the row-block-merged kernel on handles that carry its layout, 1 forces it
+    int matmul_rbm = -1;     // SPARSEOPS_MATMUL_RBM: 0 forbids every kernel that is only for handles with the RBM layout, 1 forces the row-block-merged one
     int matmul_rbm_split = 0;   // SPARSEOPS_MATMUL_RBM_SPLIT: 1, 2 or 4 workgroups per tile for RBM layouts built from now on
     int matmul_quad = -1;    // SPARSEOPS_MATMUL_QUAD: 0 forbids the quad-union kernel on handles with the RBM layout, 1 forces it
     int matmul_quad_rows = -1;  // SPARSEOPS_MATMUL_QUAD_ROWS: log2 of the quads per workgroup (0..4)

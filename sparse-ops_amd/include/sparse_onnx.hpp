@@ -17,6 +17,12 @@
 // An activation that directly follows a MatMul/Gemm/Conv whose result has no other
 // consumer is fused into that kernel's epilogue (the reference fuses Relu only,
 // src/sparse_onnx.cpp:573-620; a fused Sigmoid/Tanh equals the separate layer).
+//
+// Rounding: convolutions, and fully connected layers below 512 rows, 512 columns or 32 nonzeros a row, have the reference's
+// bits.  Larger fully connected layers add a row's products in another order (within 1e-5 of the largest output,
+// measured 1e-6), which also depends on the batch, so a sample's bits do -- in every model without convolutions, and in
+// one with convolutions that is loaded at a batch of 64 or more.  SPARSEOPS_MATMUL_RBM=0 in the environment at load
+// time keeps the reference's bits everywhere.
 #pragma once
 
 #include <cstddef>

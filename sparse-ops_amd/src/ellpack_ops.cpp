@@ -32,7 +32,7 @@ const float *stage_operands(so_ctx *ctx, const float *X, std::size_t xbytes, con
 namespace sparseops {
 // Device layouts worth keeping for Y = E * X with C dense columns.  Large, reasonably filled
 // matrices and wide X pay for a second copy: the K-tiled one (LDS-staged kernel, the reference's
-// bits) or, with `fast`, the row-block-merged one (the fastest kernel; sums in another order,
+// bits) or, with `fast`, the RBM layout's two (the fastest kernels; sums in another order,
 // accurate to fp32 round-off).
 int matmul_layouts(const Ellpack &E, uint32_t C, bool fast)
 {

@@ -456,11 +456,13 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     // Weights, conv plans and biases into HBM.
     so_ctx *ctx = context();
     std::size_t bias_total = 0;
-    // Large fully connected layers run on the row-block-merged kernel (fp32 round-off accuracy, the fastest);
+    // Large fully connected layers run on the RBM layout's kernels (fp32 round-off accuracy, the fastest);
     // SPARSEOPS_MATMUL_RBM=0 at load time keeps every layer on the kernels that give the reference's bits.
     const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM");
-    // So does a batch below 64 in a model with convolutions: there every sample has the same bits whatever batch it
-    // travels in, and its classifier is a few microseconds of the pass.
+    // So does a model with convolutions that is loaded at a batch below 64, whatever batch it is resized to later: its
+    // samples have the same bits in every batch, and its classifier is a few microseconds of the pass.  Loaded at 64 or
+    // more it keeps the fast layers at every batch, and a sample's bits then depend on the batch (the kernel is chosen
+    // by launch), as they do in a model without convolutions.
     bool convs = false;
     for (const auto &p : pend) convs = convs || p.plan.op == Op::Conv;
     const bool fast_fc = !(rbm_env && rbm_env[0] == '0') && !(convs && B0 < 64);
