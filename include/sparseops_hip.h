@@ -69,15 +69,18 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  *        columns walked once, each X row segment loaded once and multiplied into every row
  *        of the block that has a nonzero there.  The fastest so_matmul for large, very sparse matrices.
  *        The layout also holds a second copy for smaller launches and fuller matrices: quads of four rows
- *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip).
- *        so_matmul takes whichever of the two, so_matvec's row kernel (one to three columns) or the kernels
+ *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip); and, for matrices
+ *        full enough that a launch at some width is estimated to gain by it (half full to about 75 % sparse, from a
+ *        few million entries on), a third: the dense matrix as three bf16 planes whose sum is the fp32 matrix, multiplied
+ *        on the bf16 matrix cores in fp32 precision (csrc/matmul_planes.hip).
+ *        so_matmul takes whichever of them, so_matvec's row kernel (one to three columns) or the kernels
  *        of the other layouts it estimates to be the fastest.
  *        Sums are not taken in a row's slot order: results agree with
  *        the reference to fp32 round-off (max |y - ref| <= 1e-5 * max |ref|), are not
  *        bit-identical to it, and are the same bits on every launch.  Rows may be in any
  *        order.  Costs about 3x the ROW arrays in HBM -- 1.4x for the first copy, more where rows hold few
  *        nonzeros, and at most 4x for the second, which a matrix that would need more (about 99 % sparse) or that
- *        finds no room for it is kept without; with the layout so_matmul keeps a
+ *        finds no room for it is kept without; the third is 6 bytes per entry of the dense matrix; with the layout so_matmul keeps a
  *        workspace in the context that grows on first use of a larger output.
  * IDX16: a second copy of the columns in 16 bits (needs n <= 65536; costs 2 bytes per slot,
  *        and as much again for the SLOT copy when that is asked for too).  so_matvec then

@@ -283,9 +283,9 @@ so_status launch_shared_gather(so_ctx *ctx, const so_ellpack *E, const float *dX
 
 namespace {
 
-enum class RbmKernel { None, Merged, Quad, Vector };
+enum class RbmKernel { None, Merged, Quad, Vector, Planes };
 
-// Which of the three kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
+// Which of the kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
 // time.  Both sides of each line were measured, us with one handle launched again and again, in brackets with 48 handles
 // and X in turn, whose weights come from memory:
 //   quad against the row kernel: 2048 x 2048 x 64 at 95 / 90 / 80 / 50 % sparse 8.1 / 8.8 / 10.1 / 11.7 [8.6 / 9.8 / 11.3 / 13.5]
@@ -300,42 +300,76 @@ enum class RbmKernel { None, Merged, Quad, Vector };
 //   62 3.7 / 3.7; 4096 x 512 23 3.5 / 3.9; 10 x 512 63 4.0 / 3.2, 16 3.2 / 3.4; two, 4096 x 4096 487 19.6 / 8.4, 162
 //   7.8 / 7.4; 10 x 512 262 6.0 / 3.4; three, 4096 x 4096 1759 114 / 27, 487 19.7 / 13.1; 4096 x 1024 244 11.0 / 10.4.
 // `plan` is set where it is Quad: the search for it is the larger part of this function's 0.2 (two K tiles) to 0.6 us (16).
-RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan)
+// `us`: the estimate.
+RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, double *us)
 {
     const bool merged = so_matmul_rbm_applies(ctx, E, C), quad = so_matmul_quad_applies(ctx, E, C);
-    if (merged && ctx->tune.matmul_rbm == 1) return RbmKernel::Merged;
-    if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
-    // Below `us`?  A recording cannot grow the workspace: the quad kernel is then for what has been reserved (the others
+    // Below `limit`?  A recording cannot grow the workspace: the quad kernel is then for what has been reserved (the others
     // but the row-block-merged one, which refuses, need none).
-    const auto quad_below = [&](double us) {
-        if (!quad || ctx->tune.matmul_quad == 0 || us <= kQuadLeastUs) return false;
+    const auto quad_below = [&](double limit) {
+        if (!quad || ctx->tune.matmul_quad == 0 || limit <= kQuadLeastUs) return false;
         *plan = so_matmul_quad_choose(ctx, E, C);
-        return plan->us < us && (!ctx->capturing || so_matmul_quad_ready(ctx, *plan));
+        return plan->us < limit && (!ctx->capturing || so_matmul_quad_ready(ctx, *plan));
     };
-    if (ctx->tune.matmul_quad == 1 && quad_below(1e30)) return RbmKernel::Quad;
-    if (C <= 3 && E->max_nnz >= 64u * C) return RbmKernel::Vector;
+    if (ctx->tune.matmul_quad == 1 && quad_below(1e30)) { *us = 0.0; return RbmKernel::Quad; }
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
-    double best = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
+    *us = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
     RbmKernel k = RbmKernel::None;
     if (merged) {
         // one workgroup per (128 rows, 64 columns, share of the columns): pays when that grid covers most of the chip
         const double wgs = (double)E->rbmm.nb * slabs * E->rbmm.ksplit;
-        const double us = 9.5 + 2.85e-6 * work * std::ceil(wgs / cus) * cus / wgs;
-        if (4.0 * wgs >= 3.0 * cus && (us < best || !quad)) { best = us; k = RbmKernel::Merged; }
+        const double t = 9.5 + 2.85e-6 * work * std::ceil(wgs / cus) * cus / wgs;
+        if (4.0 * wgs >= 3.0 * cus && (t < *us || !quad)) { *us = t; k = RbmKernel::Merged; }
     }
-    return quad_below(0.95 * best) ? RbmKernel::Quad : k;
+    if (!quad_below(0.95 * *us)) return k;
+    *us = plan->us;
+    return RbmKernel::Quad;
+}
+
+// The bf16-planes kernel where it is estimated a tenth below the others: us, planes against the fastest of them, one handle launched
+// again and again: 4096 x 4096 x 256 at 50 / 70 / 80 % sparse 45 / 44 / 43 against 84 (quad) / 61 / 43 (merged); 3001 x 2777 x 101 at
+// 70 % 18.5 against 27.1 (merged); 2048 x 2048 x 256 at 60 / 80 % 17.0 / 16.9 against 23.4 / 18.1 (quad); 4096 x 1024 x 200 at 70 %
+// 15.8 against 19.6; 1024 x 4096 x 200 at 70 % 18.4 against 22.2; 2048 x 2048 x 128 at 70 % 14.8 against 14.1; 4096 x 784 x 256 at 90 % 15.0 against 10.8.
+constexpr double kPlanesBelow = 0.9;
+
+RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, so_planes_plan *planes)
+{
+    if (ctx->tune.matmul_rbm == 1 && so_matmul_rbm_applies(ctx, E, C)) return RbmKernel::Merged;
+    if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
+    const bool have = ctx->tune.matmul_planes != 0 && so_matmul_planes_applies(ctx, E, C);
+    const bool vector = C <= 3 && E->max_nnz >= 64u * C;
+    double us = 0.0;
+    RbmKernel k = RbmKernel::Vector;
+    if (!vector || (have && ctx->tune.matmul_planes == 1)) k = rbm_kernel_but_planes(ctx, E, C, plan, &us);
+    if (!have || (vector && ctx->tune.matmul_planes != 1)) return k;
+    *planes = so_matmul_planes_choose(ctx, E->m, E->n, C);
+    return (ctx->tune.matmul_planes == 1 || planes->us < kPlanesBelow * us) && (!ctx->capturing || so_matmul_planes_ready(ctx, *planes)) ? RbmKernel::Planes : k;
 }
 
 } // namespace
+
+// Widths from one slab to the widest of the fully connected layers this was measured on.
+bool so_planes_pays(const so_ctx *ctx, const so_ellpack *E)
+{
+    if (ctx->tune.matmul_planes >= 0) return ctx->tune.matmul_planes == 1;
+    for (uint32_t C : {64u, 128u, 256u}) {
+        so_quad_plan plan;
+        double us;
+        (void)rbm_kernel_but_planes(ctx, E, C, &plan, &us);
+        if (so_matmul_planes_choose(ctx, E->m, E->n, C).us < kPlanesBelow * us) return true;
+    }
+    return false;
+}
 
 extern "C" so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     SO_REQUIRE(ctx && E, "so_matmul_reserve: null argument");
     if (E->m == 0 || C == 0) return SO_OK;
-    // Both kernels of the layout: which one runs is settled at launch, where the tuning overrides may have changed.
+    // All kernels of the layout: which one runs is settled at launch, where the tuning overrides may have changed.
     so_status st = SO_OK;
     if (so_matmul_quad_applies(ctx, E, C)) st = so_matmul_quad_reserve(ctx, E, C);
+    if (st == SO_OK && so_matmul_planes_applies(ctx, E, C)) st = so_matmul_planes_reserve(ctx, E, C);
     if (st == SO_OK && so_matmul_rbm_applies(ctx, E, C)) {
         st = so_matmul_rbm_reserve(ctx, E, C);
         if (st == SO_OK) st = so_matmul_rbm_set_pitch(ctx, E, C);
@@ -355,18 +389,20 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     SO_REQUIRE(((uint64_t)E->m / 4 + 8) * ((uint64_t)C / 64 + 1) < (1ull << 31), "so_matmul: %u x %u output is too large for one launch", E->m, C);
 
     // The kernels of the RBM layout, on handles uploaded with it (accurate to fp32 round-off, not bit-identical to
-    // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids all three, =1
-    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one).
+    // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids all of them, =1
+    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one, SPARSEOPS_MATMUL_PLANES the bf16-planes one).
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
         so_quad_plan plan;
-        const RbmKernel k = rbm_kernel(ctx, E, C, &plan);
+        so_planes_plan pplan;
+        const RbmKernel k = rbm_kernel(ctx, E, C, &plan, &pplan);
         if (k != RbmKernel::None) {
             const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, plan, dX, C, dBias, dY, act)
+                               : k == RbmKernel::Planes ? so_matmul_planes_launch(ctx, E, pplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
-            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Vector ? "vector" : "merged";
+            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
             return SO_OK;
         }
     }

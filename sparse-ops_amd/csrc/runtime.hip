@@ -71,6 +71,8 @@ static void read_tuning(so_tuning &t)
     t.matmul_quad = env_int("SPARSEOPS_MATMUL_QUAD", -1);
     t.matmul_quad_rows = env_int("SPARSEOPS_MATMUL_QUAD_ROWS", -1);
     t.matmul_quad_split = env_int("SPARSEOPS_MATMUL_QUAD_SPLIT", 0);
+    t.matmul_planes = env_int("SPARSEOPS_MATMUL_PLANES", -1);
+    t.matmul_planes_split = env_int("SPARSEOPS_MATMUL_PLANES_SPLIT", 0);
     const int lanes = env_int("SPARSEOPS_MATVEC_LANES", 0);
     t.matvec_lanes = (lanes == 8 || lanes == 16 || lanes == 32 || lanes == 64) ? lanes : 0;
     t.matvec_idx16 = env_int("SPARSEOPS_MATVEC_IDX16", -1);
@@ -510,6 +512,7 @@ static void free_ellpack_arrays(so_ellpack *E)
     if (E->tiled.d_info) (void)hipFree(E->tiled.d_info);
     if (E->tiled.d_rows) (void)hipFree(E->tiled.d_rows);
     so_rbmm_free(E);
+    so_planes_free(E);
     so_quads_free(E);
 }
 
@@ -752,6 +755,9 @@ extern "C" so_status so_ellpack_upload(so_ctx *ctx, const float *Wd, const uint3
                 s = SO_ERR_OOM;
             }
             if (s == SO_ERR_OOM) { (void)hipGetLastError(); so_quads_free(E); s = SO_OK; }
+            // and a third where the matrix is full enough
+            if (s == SO_OK && so_planes_pays(ctx, E)) s = so_planes_build(ctx, E, Wd, nnz);
+            if (s == SO_ERR_OOM) { (void)hipGetLastError(); so_planes_free(E); s = SO_OK; }
         }
     } catch (const std::exception &e) {                  // a builder ran out of host memory, on whichever thread
         so_set_error("so_ellpack_upload: building the layouts failed: %s", e.what());

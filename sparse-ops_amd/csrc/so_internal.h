@@ -22,6 +22,8 @@ struct so_tuning {
     int matmul_quad = -1;    // SPARSEOPS_MATMUL_QUAD: 0 forbids the quad-union kernel on handles with the RBM layout, 1 forces it
     int matmul_quad_rows = -1;  // SPARSEOPS_MATMUL_QUAD_ROWS: log2 of the quads per workgroup (0..4)
     int matmul_quad_split = 0;  // SPARSEOPS_MATMUL_QUAD_SPLIT: workgroups per output tile
+    int matmul_planes = -1;  // SPARSEOPS_MATMUL_PLANES: 0 forbids the bf16-planes kernel on handles with the RBM layout, 1 forces it where the handle has the planes
+    int matmul_planes_split = 0;   // SPARSEOPS_MATMUL_PLANES_SPLIT: workgroups per output tile
     int matvec_lanes = 0;    // SPARSEOPS_MATVEC_LANES: 8, 16, 32 or 64 lanes per row
     int matvec_idx16 = -1;   // SPARSEOPS_MATVEC_IDX16: 0 keeps so_matvec on the 32-bit columns of a handle that has both
     int conv_min_cg = 0;     // SPARSEOPS_CONV_MIN_CG: fewest channel groups per workgroup a small grid may shrink to (16: never shrink)
@@ -138,6 +140,13 @@ struct so_quads {
     uint2 *d_info = nullptr;                      // [nquads][ntiles] {first chunk, units}
 };
 
+// The matrix, dense, as three bf16 planes for so_matmul on the bf16 matrix cores (csrc/matmul_planes.hip).
+struct so_planes {
+    static constexpr uint32_t kMaxSplit = 16;     // most workgroups per output tile
+    uint32_t k16 = 0;                             // runs of 16 columns kept per row tile
+    void *d_a = nullptr;                          // [row tile of 32][k16][plane][64 lanes][8] bf16
+};
+
 struct so_ellpack {
     uint32_t m = 0, n = 0, r = 0;
     uint64_t total_nnz = 0;
@@ -155,6 +164,7 @@ struct so_ellpack {
     so_tiled tiled;              // SO_LAYOUT_TILED
     so_rbmm rbmm;                // SO_LAYOUT_RBM
     so_quads quads;              // SO_LAYOUT_RBM, unless the matrix is too sparse for it (d_w is null)
+    so_planes planes;            // SO_LAYOUT_RBM, where so_planes_pays says so (else d_a is null)
 };
 
 // Row-block-merged re-encoding of a matrix (include/rbm_conv.hpp:8-27 of the reference), flattened:
@@ -213,6 +223,18 @@ bool so_matmul_quad_ready(const so_ctx *ctx, const so_quad_plan &p);            
 so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_plan &p, const float *dX, uint32_t C,
                                 const float *dBias, float *dY, int act);
+
+// csrc/matmul_planes.hip: the bf16 planes and their kernel.
+struct so_planes_plan { uint32_t ks, iters, iters_per, nslab, mbs; double us; };   // workgroups per tile, iterations in all and of each, slabs, row blocks
+bool so_planes_pays(const so_ctx *ctx, const so_ellpack *E);                              // csrc/matmul.hip: by estimate, some launch of the handle would take the kernel
+so_status so_planes_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *nnz);
+void so_planes_free(so_ellpack *E);
+bool so_matmul_planes_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+so_planes_plan so_matmul_planes_choose(const so_ctx *ctx, uint32_t m, uint32_t n, uint32_t C);
+bool so_matmul_planes_ready(const so_ctx *ctx, const so_planes_plan &p);                  // the workspace need not grow for this launch
+so_status so_matmul_planes_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
+so_status so_matmul_planes_launch(so_ctx *ctx, const so_ellpack *E, const so_planes_plan &p, const float *dX, uint32_t C,
+                                  const float *dBias, float *dY, int act);
 
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
 // since the last look (their results are invalid).  Every entry point that waits for the stream ends with this.

@@ -1,0 +1,194 @@
+"""The bf16-planes kernel of SO_LAYOUT_RBM (csrc/matmul_planes.hip), forced, at the edges of its tiles: blocks of 128 rows,
+slabs of 64 dense columns, iterations of 64 columns of the matrix, totals that leave the registers every 8 iterations,
+every number of workgroups per tile.
+
+Bound: max|y - ref| <= 1e-5 * max|ref| against the in-order oracle and the fp64 product, as for the layout's other kernels
+(tests/test_gpu_matmul_rbm.py).  Beside it the error in the 2-norm: with x = hi + mid + lo exactly, the products left out
+are below 2^-26 of |w x|, and a sum that is rounded once per 16 terms over at most 32 roundings, five times that often for
+parts 2^-9 as large, once per 512 terms and once per workgroup, each time by at most 2^-24 of a partial sum, is off by less than
+(sqrt(32 + n / 512 + 16) + 1) * 2^-24 of the 2-norm when roundings are independent: 2.5 times that is asked."""
+
+import numpy as np
+import pytest
+
+from conftest import as_oracle, rel_err, sparse_matrix
+
+import datagen
+import hipabi
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+RBM = hipabi.LAYOUT_ROW | hipabi.LAYOUT_RBM
+
+
+def planes_matmul(ctx, E, X, bias, act="none", split=None):
+    m, C = E.m, X.shape[1]
+    with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1", SPARSEOPS_MATMUL_PLANES_SPLIT=split):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+        dX, dY, dB = ctx.array(X), ctx.empty((m, C)), ctx.array(bias) if bias is not None else None
+        outs = []
+        for _ in range(2):
+            dY.upload(np.full((m, C), np.nan, np.float32))
+            ctx.matmul(dE, dX, C, dB, dY, act)
+            assert ctx.last_kernel() == "planes"
+            outs.append(dY.download())
+        for a in (dX, dY, dB):
+            if a is not None:
+                a.free()
+        dE.free()
+    assert np.array_equal(outs[0], outs[1], equal_nan=True)
+    return outs[0]
+
+
+@pytest.mark.parametrize("m,n,C,sp", [
+    (1, 1, 1, .0), (3, 15, 5, .0), (31, 16, 31, .5), (32, 17, 32, .5), (33, 63, 33, .9), (127, 64, 63, .3), (128, 65, 64, .7),
+    (129, 511, 65, .5), (300, 512, 130, .8), (257, 513, 200, .6), (64, 1100, 256, .5), (500, 2777, 101, .7)])
+@pytest.mark.parametrize("split,act", [(None, "none"), (1, "relu"), (2, "none"), (3, "relu"), (16, "none")])
+def test_planes_shapes(ctx, oracle, m, n, C, sp, split, act):
+    rng = np.random.default_rng(m * 31 + n * 7 + C)
+    W = sparse_matrix(rng, m, n, sp)
+    W[rng.integers(m), rng.integers(n)] = 1.5
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    E = datagen.encode_dense(W)
+    Y = planes_matmul(ctx, E, X, b, act, split)
+    ref = W.astype(np.float64) @ X + b[:, None]
+    if act == "relu":
+        ref = np.maximum(ref, 0)
+    assert rel_err(Y, ref) <= TOL
+    assert rel_err(Y, oracle.matmul(as_oracle(E), X, b, act)) <= TOL
+    assert np.linalg.norm(Y - ref) <= 2.5 * (np.sqrt(48 + n / 512) + 1) * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("act", ["sigmoid", "tanh"])
+def test_planes_epilogues(ctx, oracle, act):
+    rng = np.random.default_rng(1)
+    W = sparse_matrix(rng, 200, 700, .6)
+    X = rng.standard_normal((700, 70)).astype(np.float32) * 0.1
+    E = datagen.encode_dense(W)
+    Y, Yo = planes_matmul(ctx, E, X, None, act), oracle.matmul(as_oracle(E), X, None, act)
+    pre = np.abs(oracle.matmul(as_oracle(E), X, None, "none")).max()
+    # the bound of the sums times the slope, and what the device's expf / tanhf differ by (tests/test_gpu_matmul_rbm.py)
+    assert np.abs(Y.astype(np.float64) - Yo).max() <= TOL * pre * (0.25 if act == "sigmoid" else 1.0) + 1e-6
+
+
+@pytest.mark.parametrize("split", [1, 3])
+def test_planes_values_that_are_not_finite(ctx, oracle, split):
+    """An infinity or a NaN in X reaches exactly the rows that use it, although the others meet it with a zero; sums that
+    come near the largest float (where a plane, rounded up, is beyond it) stay finite."""
+    rng = np.random.default_rng(11)
+    m, n, C = 200, 600, 70
+    W = sparse_matrix(rng, m, n, .6)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    X[0, :9], X[17, 3], X[300, 5], X[599, 69] = np.inf, -np.inf, np.nan, np.inf
+    W[:, 40] = np.where(np.arange(m) % 2 == 0, 1, 0)
+    X[:, 20] = 0
+    X[40, 20] = 3.4e38                               # to bf16: infinity
+    X[:, 21] = 0
+    X[40, 21] = 1.7e38                               # to bf16: 2^127
+    W[2, 40] = 2
+    E = datagen.encode_dense(W)
+    Y, Yo = planes_matmul(ctx, E, X, None, split=split), oracle.matmul(as_oracle(E), X, None)
+    assert np.isfinite(Yo[:, 20:22]).sum() >= 2 * m - 1 and Yo[2, 21] == np.float32(3.4e38)
+    assert np.array_equal(np.isnan(Y), np.isnan(Yo)) and np.array_equal(np.isinf(Y), np.isinf(Yo))
+    assert np.array_equal(Y[np.isinf(Yo)], Yo[np.isinf(Yo)])
+    for c in range(C):
+        fin = np.isfinite(Yo[:, c])
+        assert np.abs(Y[fin, c] - Yo[fin, c]).max(initial=0.0) <= TOL * np.abs(Yo[fin, c]).max(initial=0.0)
+
+
+@pytest.mark.parametrize("exponent", [-60, -109, -112, -126, -140])
+def test_planes_values_too_small_for_three_planes(ctx, oracle, exponent):
+    """Columns of X with values whose lowest plane would fall below the smallest bf16 are as exact as the others."""
+    rng = np.random.default_rng(7)
+    m, n, C = 150, 700, 66
+    W = sparse_matrix(rng, m, n, .7)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    small = np.ldexp(rng.uniform(1, 2, (n, 30)), exponent + rng.integers(0, 3, (n, 30))).astype(np.float32)
+    X[:, 10:40] = small
+    X[::3, 12] = 0
+    X[5, 0] = small[0, 0]                             # one among ordinary values
+    E = datagen.encode_dense(W)
+    Y = planes_matmul(ctx, E, X, None, split=2)
+    Yo = oracle.matmul(as_oracle(E), X, None)
+    ref = W.astype(np.float64) @ X.astype(np.float64)
+    for c in range(C):
+        # a sum of subnormal products is rounded to 2^-149 per term, whatever its size
+        assert np.abs(Y[:, c] - ref[:, c]).max() <= TOL * np.abs(ref[:, c]).max() + n * 2.0 ** -149, c
+        assert np.abs(Y[:, c] - Yo[:, c]).max() <= TOL * np.abs(Yo[:, c]).max() + n * 2.0 ** -149, c
+
+
+def test_planes_left_out(ctx):
+    """Weights without room for three planes, rows whose columns do not ascend: the handle does without, whatever is asked."""
+    rng = np.random.default_rng(3)
+    W = sparse_matrix(rng, 100, 200, .5)
+    X = rng.standard_normal((200, 8)).astype(np.float32)
+    cases = []
+    for value in (1e-35, 1e37, np.inf, np.nan):
+        V = W.copy()
+        V[3, 5] = value
+        cases.append(datagen.encode_dense(V))
+    E = datagen.encode_dense(W)
+    c = int(E.nnz[9])
+    E.Wd[9, :c], E.idx[9, :c] = E.Wd[9, :c][::-1].copy(), E.idx[9, :c][::-1].copy()
+    cases.append(E)
+    for E in cases:
+        with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1"):
+            dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM)
+            dX, dY = ctx.array(X), ctx.empty((100, 8))
+            ctx.matmul(dE, dX, 8, None, dY)
+            assert ctx.last_kernel() != "planes"
+            dE.free()
+
+
+def test_planes_by_default(ctx, oracle):
+    """The dispatch's own choice: a half-full matrix on a wide batch takes the kernel, a batch of ones or a very sparse matrix does not;
+    a column's bits do not depend on its neighbours."""
+    rng = np.random.default_rng(2)
+    m = n = 2048
+    X = rng.standard_normal((n, 200)).astype(np.float32)
+    for sp, C, want in ((.5, 200, True), (.5, 1, False), (.95, 200, False)):
+        W = sparse_matrix(rng, m, n, sp)
+        E = datagen.encode_dense(W)
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, m, n, E.r, RBM)
+        x = np.ascontiguousarray(X[:, :C])
+        dX, dY = ctx.array(x), ctx.empty((m, C))
+        ctx.matmul(dE, dX, C, None, dY)
+        assert (ctx.last_kernel() == "planes") == want
+        Y = dY.download()
+        assert rel_err(Y, W.astype(np.float64) @ x) <= TOL
+        if want:
+            perm = rng.permutation(C)
+            dX.upload(np.ascontiguousarray(x[:, perm]))
+            ctx.matmul(dE, dX, C, None, dY)
+            assert np.array_equal(dY.download(), Y[:, perm])
+        dE.free()
+
+
+def test_planes_in_a_recorded_graph(ctx):
+    """Reserved, recorded and replayed with new inputs; eager launches of another width between the replays."""
+    rng = np.random.default_rng(4)
+    m, n, C = 400, 1300, 100
+    W = sparse_matrix(rng, m, n, .6)
+    E = datagen.encode_dense(W)
+    with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, m, n, E.r, RBM)
+        dX, dY, dZ = ctx.empty((n, C)), ctx.empty((m, C)), ctx.empty((m, 7))
+        ctx.matmul_reserve(dE, C)
+        ctx.graph_begin()
+        ctx.matmul(dE, dX, C, None, dY)
+        assert ctx.last_kernel() == "planes"
+        g = ctx.graph_end()
+        dx = ctx.array(rng.standard_normal((n, 7)).astype(np.float32))
+        for _ in range(3):
+            X = rng.standard_normal((n, C)).astype(np.float32)
+            dX.upload(X)
+            ctx.graph_launch(g)
+            ctx.sync()
+            Y = dY.download()
+            ctx.matmul(dE, dX, C, None, dY)
+            assert np.array_equal(dY.download(), Y)
+            assert rel_err(Y, W.astype(np.float64) @ X) <= TOL
+            ctx.matmul(dE, dx, 7, None, dZ)
+        ctx.graph_free(g)
+        dE.free()
