@@ -69,7 +69,7 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  *        columns walked once, each X row segment loaded once and multiplied into every row
  *        of the block that has a nonzero there.  The fastest so_matmul for large, very sparse matrices.
  *        The layout also holds a second copy for smaller launches and fuller matrices: quads of four rows
- *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip); and, for matrices
+ *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip, up to 32 dense columns csrc/matmul_narrow.hip); and, for matrices
  *        full enough that a launch at some width is estimated to gain by it (half full to about 75 % sparse, from a
  *        few million entries on), a third: the dense matrix as three bf16 planes whose sum is the fp32 matrix, multiplied
  *        on the bf16 matrix cores in fp32 precision (csrc/matmul_planes.hip).
@@ -214,7 +214,7 @@ so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t 
  * connected layer -- the reference's documented way to get its allocation-free run(), README.md:146).
  * No counterpart in the reference. */
 so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
-/* Which kernel the context's last so_matmul or so_conv2d launched, for tests and tuning: "merged", "quad" and "vector" (on
+/* Which kernel the context's last so_matmul or so_conv2d launched, for tests and tuning: "merged", "quad", "narrow" and "vector" (on
  * handles with the RBM layout), "tiled", "shared", "row"; "columns", "merged-window", "window", "gather"; "" before the
  * first.  A static string.  No counterpart in the reference. */
 const char *so_last_kernel(const so_ctx *ctx);

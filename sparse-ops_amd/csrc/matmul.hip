@@ -283,7 +283,7 @@ so_status launch_shared_gather(so_ctx *ctx, const so_ellpack *E, const float *dX
 
 namespace {
 
-enum class RbmKernel { None, Merged, Quad, Vector, Planes };
+enum class RbmKernel { None, Merged, Quad, Vector, Planes, Narrow };
 
 // Which of the kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
 // time.  Both sides of each line were measured, us with one handle launched again and again, in brackets with 48 handles
@@ -333,18 +333,35 @@ RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t
 // 15.8 against 19.6; 1024 x 4096 x 200 at 70 % 18.4 against 22.2; 2048 x 2048 x 128 at 70 % 14.8 against 14.1; 4096 x 784 x 256 at 90 % 15.0 against 10.8.
 constexpr double kPlanesBelow = 0.9;
 
+// The narrow kernel where it is estimated an eighth below the others (whose estimates are up to a tenth too high here): us, the others and
+// the narrow one, one handle launched again and again: quad 2847 x 1952 x 8 at 61 % sparse 14.7 / 7.8, 4096 x 2048 x 16 at 90 / 50 %
+// 10.9 / 7.8 and 17.6 / 11.5, 1152 x 546 x 18 at 54 % 7.2 / 5.4, 317 x 930 x 11 at 74 % 6.8 / 4.8, 2745 x 1203 x 30 at 56 % 11.7 / 11.0;
+// shared-gather 1145 columns, 21 rows, 5 dense 6.6 / 4.1, 627, 41, 28 4.8 / 5.5; row 1595, 981, 10 7.2 / 5.4, 1067, 3000, 28 5.1 / 6.7.  In place
+// of so_matvec's row kernel at two and three columns from a million nonzeros on: 1.16 million, three columns, 10.6 / 5.5; 2.7 million, two, 11.4 / 9.1;
+// 0.91 million, two, 4.5 / 5.3; with one column not: 1.4 million 6.7 / 7.1.
+constexpr double kNarrowBelow = 0.88;
+constexpr uint64_t kNarrowVectorNnz = 1000000;
+
 RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, so_planes_plan *planes)
 {
     if (ctx->tune.matmul_rbm == 1 && so_matmul_rbm_applies(ctx, E, C)) return RbmKernel::Merged;
     if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
+    if (ctx->tune.matmul_narrow == 1 && so_matmul_narrow_applies(ctx, E, C)) return RbmKernel::Narrow;
     const bool have = ctx->tune.matmul_planes != 0 && so_matmul_planes_applies(ctx, E, C);
     const bool vector = C <= 3 && E->max_nnz >= 64u * C;
     double us = 0.0;
     RbmKernel k = RbmKernel::Vector;
     if (!vector || (have && ctx->tune.matmul_planes == 1)) k = rbm_kernel_but_planes(ctx, E, C, plan, &us);
-    if (!have || (vector && ctx->tune.matmul_planes != 1)) return k;
-    *planes = so_matmul_planes_choose(ctx, E->m, E->n, C);
-    return (ctx->tune.matmul_planes == 1 || planes->us < kPlanesBelow * us) && (!ctx->capturing || so_matmul_planes_ready(ctx, *planes)) ? RbmKernel::Planes : k;
+    if (have && (!vector || ctx->tune.matmul_planes == 1)) {
+        *planes = so_matmul_planes_choose(ctx, E->m, E->n, C);
+        if ((ctx->tune.matmul_planes == 1 || planes->us < kPlanesBelow * us) && (!ctx->capturing || so_matmul_planes_ready(ctx, *planes))) {
+            k = RbmKernel::Planes;
+            us = planes->us;
+        }
+    }
+    // (an override that forces another kernel, or forbids the quad-union copy's, stands)
+    if (ctx->tune.matmul_narrow == 0 || ctx->tune.matmul_quad >= 0 || ctx->tune.matmul_planes == 1 || !so_matmul_narrow_applies(ctx, E, C)) return k;
+    return (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : so_matmul_narrow_estimate(ctx, E, C) < kNarrowBelow * us) ? RbmKernel::Narrow : k;
 }
 
 } // namespace
@@ -390,19 +407,20 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
 
     // The kernels of the RBM layout, on handles uploaded with it (accurate to fp32 round-off, not bit-identical to
     // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids all of them, =1
-    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one, SPARSEOPS_MATMUL_PLANES the bf16-planes one).
+    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one, SPARSEOPS_MATMUL_PLANES the bf16-planes one, SPARSEOPS_MATMUL_NARROW the narrow one).
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
         so_quad_plan plan;
         so_planes_plan pplan;
         const RbmKernel k = rbm_kernel(ctx, E, C, &plan, &pplan);
         if (k != RbmKernel::None) {
             const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, plan, dX, C, dBias, dY, act)
+                               : k == RbmKernel::Narrow ? so_matmul_narrow_launch(ctx, E, dX, C, dBias, dY, act)
                                : k == RbmKernel::Planes ? so_matmul_planes_launch(ctx, E, pplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
-            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
+            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Narrow ? "narrow" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
             return SO_OK;
         }
     }

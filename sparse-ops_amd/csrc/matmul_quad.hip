@@ -502,6 +502,7 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
         chunks += (units + 3) / 4;
         Q.total_units += units;
     }
+    Q.total_chunks = chunks;
     if (chunks > 0xfffff000ull || chunks * 272 + info.size() * sizeof(uint2) > most) { Q = so_quads(); return SO_OK; }
     // padding steps: zero weights on the tile's first row
     // (the three arrays in one allocation and one copy: each of either costs a small matrix a tenth of a millisecond)

@@ -22,6 +22,7 @@ struct so_tuning {
     int matmul_quad = -1;    // SPARSEOPS_MATMUL_QUAD: 0 forbids the quad-union kernel on handles with the RBM layout, 1 forces it
     int matmul_quad_rows = -1;  // SPARSEOPS_MATMUL_QUAD_ROWS: log2 of the quads per workgroup (0..4)
     int matmul_quad_split = 0;  // SPARSEOPS_MATMUL_QUAD_SPLIT: workgroups per output tile
+    int matmul_narrow = -1;  // SPARSEOPS_MATMUL_NARROW: 0 forbids the narrow kernel on handles with the RBM layout, 1 forces it where it applies
     int matmul_planes = -1;  // SPARSEOPS_MATMUL_PLANES: 0 forbids the bf16-planes kernel on handles with the RBM layout, 1 forces it where the handle has the planes
     int matmul_planes_split = 0;   // SPARSEOPS_MATMUL_PLANES_SPLIT: workgroups per output tile
     int matvec_lanes = 0;    // SPARSEOPS_MATVEC_LANES: 8, 16, 32 or 64 lanes per row
@@ -134,7 +135,7 @@ struct so_quads {
     static constexpr uint32_t kTileRows = 256;    // X rows per LDS tile
     static constexpr uint32_t kMaxSplit = 64;     // most workgroups per output tile
     uint32_t nquads = 0, ntiles = 0;
-    uint64_t total_units = 0;                     // units of four steps over all (quad, tile) runs
+    uint64_t total_units = 0, total_chunks = 0;   // units of four steps and chunks over all (quad, tile) runs
     float *d_w = nullptr;                         // [chunks + slack][64]
     uint32_t *d_off = nullptr;                    // [chunks + slack][4] words: X row inside the tile, a byte per step
     uint2 *d_info = nullptr;                      // [nquads][ntiles] {first chunk, units}
@@ -223,6 +224,11 @@ bool so_matmul_quad_ready(const so_ctx *ctx, const so_quad_plan &p);            
 so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_plan &p, const float *dX, uint32_t C,
                                 const float *dBias, float *dY, int act);
+
+// csrc/matmul_narrow.hip: up to 32 dense columns on the quad-union copy.
+bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+double so_matmul_narrow_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);     // us
+so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
 
 // csrc/matmul_planes.hip: the bf16 planes and their kernel.
 struct so_planes_plan { uint32_t ks, iters, iters_per, nslab, mbs; double us; };   // workgroups per tile, iterations in all and of each, slabs, row blocks
