@@ -133,6 +133,11 @@ so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t bytes); /* wait
  * stream.  so_stage_out queues a device array's way back, waits for it and reports as so_d2h does. */
 so_status so_stage_in(so_ctx *ctx, void *dst, const void *src, size_t bytes, void *dst2, const void *src2, size_t bytes2);
 so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes);
+/* The same with a transpose on the way: dDst[cols][stride] from the host's src[rows][cols], zeros in the places from `rows` to
+ * `stride` of its rows; the host's dst[cols][rows] from dSrc[rows][stride].  *done = 0, with nothing queued, for arrays that
+ * the staging memory does not hold (about 4 MB in, 1 MB out).  No counterpart in the reference. */
+so_status so_stage_in_transposed(so_ctx *ctx, float *dDst, uint32_t stride, const float *src, uint32_t rows, uint32_t cols, int *done);
+so_status so_stage_out_transposed(so_ctx *ctx, float *dst, const float *dSrc, uint32_t stride, uint32_t rows, uint32_t cols, int *done);
 so_status so_d2d(so_ctx *ctx, void *dst, const void *src, size_t bytes);
 so_status so_fill_zero(so_ctx *ctx, void *dptr, size_t bytes); /* fill kernel, graph-safe */
 /* Waits for the context's stream.  The LDS-staged kernels synchronise their waves through counters

@@ -265,7 +265,13 @@ extern "C" so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t byte
 // piece reads that over the link while the next piece is copied; the way out is a kernel that writes pinned memory and
 // then a word that the host polls.  Host to host, before and now: a 1500 x 1000 ellpack_matvec with bias 49 and 19 us,
 // the MLP 784-4096-4096-4096-10 at batch 256 150 and 141, one image through the ResNet-18-shaped stack 312 and 284.
-constexpr size_t kStageIn = 4u << 20, kStageOut = 1u << 20, kStagePiece = 256u << 10;
+//
+// Bound by latencies in a row: per kernel the launch, the link's 2 to 3 us and 256 KB at about 50 GB/s.  A model's input and output
+// are [batch][features] on the host and [features][batch] in memory, so their kernels transpose (and pad) on the way, in
+// pieces of columns that double from 128 KB on, instead of a transpose and a padding kernel each behind the copies: the same MLP
+// 141 -> 123 us (at batch 2 / 4 / 16 54 / 67 / 69 -> 44 / 45 / 60, its narrow kernel included), 100-300-20 at batch 7 27 -> 20, the ResNet-18-shaped
+// stack on 12 images of 96 x 96 246 -> 222.
+constexpr size_t kStageIn = 4u << 20, kStageOut = 1u << 20, kStagePiece = 256u << 10, kStagePieceFirst = 128u << 10, kStagePieceMost = 1u << 20;
 constexpr size_t kStageFlag = kStageIn + kStageOut;      // {turn, waits given up} behind the two areas
 
 // Words of up to two arrays, 16 bytes per thread and load (ends by the word).
@@ -282,13 +288,48 @@ void so_stage_in_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint
     if (threadIdx.x < words2 % 4u) dst2[quads2 * 4u + threadIdx.x] = src2[quads2 * 4u + threadIdx.x];
 }
 
-// The last workgroup to finish tells the host: `turn`, and beside it the word of the bounded waits.
+// dst[c * stride + r] = src[r * pitch + c] for the `rows` rows of a piece of `cols` columns, zeros for the rows up to `stride`: 64 columns
+// by 32 rows per workgroup, 16 bytes per lane over the link (pitch is a multiple of four), 128 bytes at a time to memory.
 __global__ __launch_bounds__(256)
-void so_stage_out_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
+void so_stage_in_transposed_kernel(float *dst, uint32_t stride, const float *src, uint32_t pitch, uint32_t rows, uint32_t cols)
+{
+    __shared__ float tile[64][33];
+    const uint32_t r0 = blockIdx.y * 32u, c0 = blockIdx.x * 64u;
+    const uint32_t c4 = (threadIdx.x & 15u) * 4u;
+    float4 v[2];
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        const uint32_t r = r0 + k * 16u + (threadIdx.x >> 4);
+        v[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r < rows && c0 + c4 < cols) v[k] = *reinterpret_cast<const float4 *>(src + (size_t)r * pitch + c0 + c4);
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 2; ++k) {
+        const uint32_t r = k * 16u + (threadIdx.x >> 4);
+        tile[c4][r] = v[k].x; tile[c4 + 1u][r] = v[k].y; tile[c4 + 2u][r] = v[k].z; tile[c4 + 3u][r] = v[k].w;
+    }
+    __syncthreads();
+    const uint32_t r = threadIdx.x & 31u;
+    for (uint32_t c = threadIdx.x >> 5; c < 64u; c += 8u)
+        if (c0 + c < cols && r0 + r < stride) dst[(size_t)(c0 + c) * stride + r0 + r] = tile[c][r];
+}
+
+// The last workgroup to finish tells the host: `turn`, and beside it the word of the bounded waits.  `cols` != 0: dst is the transpose
+// of src, whose rows of `cols` words lie `pitch` apart.
+__global__ __launch_bounds__(256)
+void so_stage_out_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t cols, uint32_t pitch, uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
 {
     const uint32_t quads = words / 4u, stride = gridDim.x * 256u;
-    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
-    if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = src[quads * 4u + threadIdx.x];
+    if (cols != 0u) {
+        const uint32_t rows = words / cols;
+        auto word = [&](uint32_t e) { const uint32_t c = e / rows; return src[(size_t)(e - c * rows) * pitch + c]; };
+        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride)
+            reinterpret_cast<uint4 *>(dst)[i] = make_uint4(word(4u * i), word(4u * i + 1u), word(4u * i + 2u), word(4u * i + 3u));
+        if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = word(quads * 4u + threadIdx.x);
+    } else {
+        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+        if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = src[quads * 4u + threadIdx.x];
+    }
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x != 0) return;
@@ -355,17 +396,14 @@ extern "C" so_status so_stage_in(so_ctx *ctx, void *dst, const void *src, size_t
     return SO_OK;
 }
 
-extern "C" so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes)
+// A copy of `bytes` (a transpose where cols != 0) to the staging memory, the wait for it, and from there to dst.  *told: false where the
+// stream ended without the word.
+static so_status stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes, uint32_t cols, uint32_t pitch, const char *who, bool *told)
 {
-    SO_REQUIRE(ctx != nullptr, "so_stage_out: ctx is null");
-    if (bytes == 0) return SO_OK;
-    SO_REQUIRE(dst && src, "so_stage_out: null pointer");
-    SO_REQUIRE(!ctx->capturing, "so_stage_out: not allowed while a graph is being recorded");
-    if (bytes > kStageOut || bytes % 4 != 0 || ((uintptr_t)src & 15) != 0 || !stage_ready(ctx)) return so_d2h(ctx, dst, src, bytes);
     volatile uint32_t *const flag = (volatile uint32_t *)(ctx->h_stage + kStageFlag);
     const uint32_t turn = ++ctx->stage_turn;
     const uint32_t blocks = (uint32_t)std::min<size_t>((bytes + 8191) / 8192, 128);
-    so_stage_out_kernel<<<blocks, 256, 0, ctx->stream>>>((uint32_t *)(ctx->h_stage + kStageIn), (const uint32_t *)src, (uint32_t)(bytes / 4),
+    so_stage_out_kernel<<<blocks, 256, 0, ctx->stream>>>((uint32_t *)(ctx->h_stage + kStageIn), (const uint32_t *)src, (uint32_t)(bytes / 4), cols, pitch,
                                                          ctx->d_stage_done, ctx->d_wait_gave_up, (uint32_t *)flag, turn);
     SO_LAUNCH_CHECK();
     // The word comes when the stream's work is done; a stream that has ended without it, or failed, ends the wait as well.
@@ -374,16 +412,69 @@ extern "C" so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_
             const hipError_t e = hipStreamQuery(ctx->stream);
             if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
             SO_HIP(e);
-            if (*flag != turn) return so_d2h(ctx, dst, src, bytes);
+            if (*flag != turn) { *told = false; return SO_OK; }
         }
         __builtin_ia32_pause();
     }
     std::atomic_thread_fence(std::memory_order_acquire);
+    *told = true;
     ctx->stage_used = 0;                       // the stream's earlier work, and with it every way in, is done
-    if (ctx->waits_pending && flag[1] != 0) return so_stream_wait(ctx, "so_stage_out");
+    if (ctx->waits_pending && flag[1] != 0) return so_stream_wait(ctx, who);
     ctx->waits_pending = false;
     std::memcpy(dst, ctx->h_stage + kStageIn, bytes);
     return SO_OK;
+}
+
+extern "C" so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes)
+{
+    SO_REQUIRE(ctx != nullptr, "so_stage_out: ctx is null");
+    if (bytes == 0) return SO_OK;
+    SO_REQUIRE(dst && src, "so_stage_out: null pointer");
+    SO_REQUIRE(!ctx->capturing, "so_stage_out: not allowed while a graph is being recorded");
+    if (bytes > kStageOut || bytes % 4 != 0 || ((uintptr_t)src & 15) != 0 || !stage_ready(ctx)) return so_d2h(ctx, dst, src, bytes);
+    bool told = false;
+    const so_status s = stage_out(ctx, dst, src, bytes, 0u, 0u, "so_stage_out", &told);
+    return s != SO_OK || told ? s : so_d2h(ctx, dst, src, bytes);
+}
+
+extern "C" so_status so_stage_in_transposed(so_ctx *ctx, float *dDst, uint32_t stride, const float *src, uint32_t rows, uint32_t cols, int *done)
+{
+    SO_REQUIRE(ctx && done, "so_stage_in_transposed: null argument");
+    *done = 1;
+    if (rows == 0 || cols == 0) return SO_OK;
+    SO_REQUIRE(dDst && src, "so_stage_in_transposed: null pointer");
+    SO_REQUIRE(stride >= rows, "so_stage_in_transposed: %u values a row, %u rows", stride, rows);
+    SO_REQUIRE(!ctx->capturing, "so_stage_in_transposed: not allowed while a graph is being recorded");
+    const size_t row_bytes = ((size_t)cols + 3) / 4 * 16, want = (row_bytes + 16 * 64) * rows;      // (every piece's rows end on four values)
+    if (want > kStageIn || ctx->stage_used + want > kStageIn || so_ceil_div(stride, 32) > 65535u || !stage_ready(ctx)) { *done = 0; return SO_OK; }
+    // pieces of columns: the first small, so that the link starts early, each of the others twice the one before it
+    size_t piece = kStagePieceFirst;
+    for (uint32_t at = 0; at < cols; piece = std::min(2 * piece, kStagePieceMost)) {
+        const uint32_t n = (uint32_t)std::min<size_t>(cols - at, std::max<size_t>(64, piece / (4 * (size_t)rows) / 64 * 64)), pitch = (n + 3u) / 4u * 4u;
+        float *const h = (float *)(ctx->h_stage + ctx->stage_used);
+        for (uint32_t r = 0; r < rows; ++r) std::memcpy(h + (size_t)r * pitch, src + (size_t)r * cols + at, (size_t)n * 4);
+        so_stage_in_transposed_kernel<<<dim3(so_ceil_div(n, 64), so_ceil_div(stride, 32)), 256, 0, ctx->stream>>>(dDst + (size_t)at * stride, stride, h, pitch, rows, n);
+        SO_LAUNCH_CHECK();
+        ctx->stage_used += ((size_t)rows * pitch * 4 + 255) / 256 * 256;
+        at += n;
+    }
+    return SO_OK;
+}
+
+extern "C" so_status so_stage_out_transposed(so_ctx *ctx, float *dst, const float *dSrc, uint32_t stride, uint32_t rows, uint32_t cols, int *done)
+{
+    SO_REQUIRE(ctx && done, "so_stage_out_transposed: null argument");
+    *done = 1;
+    if (rows == 0 || cols == 0) return SO_OK;
+    SO_REQUIRE(dst && dSrc, "so_stage_out_transposed: null pointer");
+    SO_REQUIRE(stride >= cols, "so_stage_out_transposed: %u values a row, %u columns", stride, cols);
+    SO_REQUIRE(!ctx->capturing, "so_stage_out_transposed: not allowed while a graph is being recorded");
+    *done = 0;
+    if ((uint64_t)rows * cols * 4 > kStageOut || !stage_ready(ctx)) return SO_OK;
+    bool told = false;
+    const so_status s = stage_out(ctx, dst, dSrc, (size_t)rows * cols * 4, cols, stride, "so_stage_out_transposed", &told);
+    *done = told;
+    return s;
 }
 
 extern "C" so_status so_d2d(so_ctx *ctx, void *dst, const void *src, size_t bytes)

@@ -19,7 +19,7 @@ LAYOUT_ROW, LAYOUT_SLOT, LAYOUT_BINS, LAYOUT_TILED, LAYOUT_RBM, LAYOUT_IDX16 = 1
 # Every symbol include/sparseops_hip.h declares.
 SYMBOLS = (
     "so_device_count so_init so_destroy so_last_error so_device_info so_tuning_reload so_malloc so_free so_h2d so_d2h "
-    "so_stage_in so_stage_out so_d2d so_fill_zero so_sync so_timer_begin so_timer_end so_ellpack_upload so_ellpack_free "
+    "so_stage_in so_stage_out so_stage_in_transposed so_stage_out_transposed so_d2d so_fill_zero so_sync so_timer_begin so_timer_end so_ellpack_upload so_ellpack_free "
     "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
     "so_conv2d so_maxpool so_gap so_add so_act so_transpose so_reverse_axes3 so_copy_rows so_graph_begin so_graph_end "
     "so_graph_launch so_graph_free so_rbm_upload so_rbm_free so_rbm_dims so_conv_plan_set_rbm so_conv_plan_rbm_info").split()
@@ -79,6 +79,8 @@ def load_library(path=None):
         "so_ellpack_download": [_vp, _vp, ct.c_int, _vp, _vp, _vp],
         "so_stage_in": [_vp, _vp, _vp, ct.c_size_t, _vp, _vp, ct.c_size_t],
         "so_stage_out": [_vp, _vp, _vp, ct.c_size_t],
+        "so_stage_in_transposed": [_vp, _vp, ct.c_uint32, _vp, ct.c_uint32, ct.c_uint32, ct.POINTER(ct.c_int)],
+        "so_stage_out_transposed": [_vp, _vp, _vp, ct.c_uint32, ct.c_uint32, ct.c_uint32, ct.POINTER(ct.c_int)],
         "so_ellpack_decode": [_vp, _vp, _vp],
         "so_ellpack_encode": [_vp, _vp, _u32, _u32, ct.POINTER(_vp)],
         "so_ellpack_encode_noalloc": [_vp, _vp, _u32, _u32, _u32, _vp, _vp, _vp, ct.POINTER(_u32), ct.POINTER(ct.c_uint64)],

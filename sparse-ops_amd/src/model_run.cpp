@@ -141,18 +141,20 @@ void SparseOnnxModel::run_batch_major(const float *input, uint32_t B, float *out
     if (B == 1) { run(input, B, output); return; }      // one sample is the same in either order
     so_ctx *ctx = context();
     std::lock_guard<std::mutex> lock(context_mutex());
-    check(so_stage_in(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float), nullptr, nullptr, 0), "so_stage_in(input)");
-    if (!M.padded()) {
-        check(so_transpose(ctx, M.stage_in.f32(), B, uint32_t(M.in_features), M.slot_ptr(M.input_slot)), "so_transpose(input)");
-        M.launch_chain();
-        check(so_transpose(ctx, M.slot_ptr(M.output_slot), uint32_t(M.out_features), B, M.stage_out.f32()), "so_transpose(output)");
-    } else {
-        check(so_transpose(ctx, M.stage_in.f32(), B, uint32_t(M.in_features), M.stage_mid.f32()), "so_transpose(input)");
-        M.rows_in(M.stage_mid.f32());
-        M.launch_chain();
-        M.rows_out(M.stage_mid.f32());
-        check(so_transpose(ctx, M.stage_mid.f32(), uint32_t(M.out_features), B, M.stage_out.f32()), "so_transpose(output)");
+    // Both ways through the staging memory as one pass each where it holds the arrays: transposed, and padded to the arena's rows,
+    // as they cross the link.
+    int done = 0;
+    check(so_stage_in_transposed(ctx, M.slot_ptr(M.input_slot), M.pbatch, input, B, uint32_t(M.in_features), &done), "so_stage_in_transposed(input)");
+    if (!done) {
+        check(so_stage_in(ctx, M.stage_in.get(), input, M.in_features * B * sizeof(float), nullptr, nullptr, 0), "so_stage_in(input)");
+        check(so_transpose(ctx, M.stage_in.f32(), B, uint32_t(M.in_features), M.padded() ? M.stage_mid.f32() : M.slot_ptr(M.input_slot)), "so_transpose(input)");
+        if (M.padded()) M.rows_in(M.stage_mid.f32());
     }
+    M.launch_chain();
+    check(so_stage_out_transposed(ctx, output, M.slot_ptr(M.output_slot), M.pbatch, uint32_t(M.out_features), B, &done), "so_stage_out_transposed(output)");
+    if (done) return;
+    if (M.padded()) M.rows_out(M.stage_mid.f32());
+    check(so_transpose(ctx, M.padded() ? M.stage_mid.f32() : M.slot_ptr(M.output_slot), uint32_t(M.out_features), B, M.stage_out.f32()), "so_transpose(output)");
     check(so_stage_out(ctx, output, M.stage_out.get(), M.out_features * B * sizeof(float)), "so_stage_out(output)");
 }
 

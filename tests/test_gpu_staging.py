@@ -82,3 +82,31 @@ def test_reports_waits_that_gave_up(ctx):
         assert np.array_equal(out, dY.download().view(np.uint32).ravel())
     for a in (dX, dY, dE):
         a.free()
+
+
+@pytest.mark.parametrize("rows,cols,stride", [(1, 1, 1), (2, 3, 4), (4, 63, 4), (5, 65, 8), (31, 64, 31), (33, 130, 48), (256, 784, 256), (100, 1000, 112),
+                                              (3, 90000, 4), (7, 149000, 8), (16, 65000, 16), (3, 349000, 4)])
+def test_transposed_there_and_back(ctx, rows, cols, stride):
+    """Pieces of 64 columns and more, tiles of 64 x 32, rows of no multiple of four, padding, sizes around what the staging
+    memory holds: the bytes, the zeros behind them and nothing beyond."""
+    rng = np.random.default_rng(rows + cols)
+    fits_in = ((cols + 3) // 4 * 16 + 1024) * rows <= IN
+    d = ctx.array(np.full(cols * stride + 8, 7.0, np.float32))
+    done = ct.c_int(-1)
+    for turn in range(3):
+        a = rng.integers(0, 1 << 32, (rows, cols), dtype=np.uint32)
+        ctx._ck(ctx.lib.so_stage_in_transposed(ctx.h, d.ptr, stride, a.ctypes.data_as(ct.c_void_p), rows, cols, ct.byref(done)))
+        assert done.value == int(fits_in)
+        if not fits_in:
+            break
+        got = d.download().view(np.uint32)
+        assert np.array_equal(got[:cols * stride].reshape(cols, stride)[:, :rows], a.T) and not got[:cols * stride].reshape(cols, stride)[:, rows:].any()
+        assert (d.download()[cols * stride:] == 7.0).all()
+        out = np.zeros((rows, cols), np.uint32)
+        ctx._ck(ctx.lib.so_stage_out_transposed(ctx.h, out.ctypes.data_as(ct.c_void_p), d.ptr, stride, cols, rows, ct.byref(done)))
+        assert done.value == int(rows * cols * 4 <= OUT)
+        if done.value:
+            assert np.array_equal(out, a)
+    assert ctx.lib.so_stage_in_transposed(ctx.h, d.ptr, rows - 1, None, rows, cols, ct.byref(done)) == hipabi.SO_ERR_INVALID
+    assert ctx.lib.so_stage_out_transposed(ctx.h, None, d.ptr, stride, cols, rows, ct.byref(done)) == hipabi.SO_ERR_INVALID
+    d.free()
