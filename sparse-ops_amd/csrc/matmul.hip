@@ -342,11 +342,14 @@ constexpr double kPlanesBelow = 0.9;
 constexpr double kNarrowBelow = 0.88;
 constexpr uint64_t kNarrowVectorNnz = 1000000;
 
-RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, so_planes_plan *planes)
+RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, so_planes_plan *planes, so_narrow_plan *narrow)
 {
     if (ctx->tune.matmul_rbm == 1 && so_matmul_rbm_applies(ctx, E, C)) return RbmKernel::Merged;
     if (ctx->tune.matmul_rbm == 0) return RbmKernel::None;
-    if (ctx->tune.matmul_narrow == 1 && so_matmul_narrow_applies(ctx, E, C)) return RbmKernel::Narrow;
+    if (ctx->tune.matmul_narrow == 1 && so_matmul_narrow_applies(ctx, E, C)) {
+        *narrow = so_matmul_narrow_choose(ctx, E, C);
+        return RbmKernel::Narrow;
+    }
     const bool have = ctx->tune.matmul_planes != 0 && so_matmul_planes_applies(ctx, E, C);
     const bool vector = C <= 3 && E->max_nnz >= 64u * C;
     double us = 0.0;
@@ -361,7 +364,8 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad
     }
     // (an override that forces another kernel, or forbids the quad-union copy's, stands)
     if (ctx->tune.matmul_narrow == 0 || ctx->tune.matmul_quad >= 0 || ctx->tune.matmul_planes == 1 || !so_matmul_narrow_applies(ctx, E, C)) return k;
-    return (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : so_matmul_narrow_estimate(ctx, E, C) < kNarrowBelow * us) ? RbmKernel::Narrow : k;
+    *narrow = so_matmul_narrow_choose(ctx, E, C);
+    return (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : narrow->us < kNarrowBelow * us) ? RbmKernel::Narrow : k;
 }
 
 } // namespace
@@ -411,10 +415,11 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
         so_quad_plan plan;
         so_planes_plan pplan;
-        const RbmKernel k = rbm_kernel(ctx, E, C, &plan, &pplan);
+        so_narrow_plan nplan;
+        const RbmKernel k = rbm_kernel(ctx, E, C, &plan, &pplan, &nplan);
         if (k != RbmKernel::None) {
             const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, plan, dX, C, dBias, dY, act)
-                               : k == RbmKernel::Narrow ? so_matmul_narrow_launch(ctx, E, dX, C, dBias, dY, act)
+                               : k == RbmKernel::Narrow ? so_matmul_narrow_launch(ctx, E, nplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Planes ? so_matmul_planes_launch(ctx, E, pplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);

@@ -1,4 +1,4 @@
-// Narrow matmul: Y = act(E X + bias) for up to 32 dense columns on the quad-union copy of the matrix (matmul_quad.hip,
+// Narrow matmul: Y = act(E X + bias) for up to 32 dense columns, or for few rows, on the quad-union copy of the matrix (matmul_quad.hip,
 // layout SO_LAYOUT_RBM).
 //
 // The quad-union kernel gives 64 lanes 64 columns, four union columns (steps) at a time; with 8 columns seven eighths of its LDS
@@ -19,6 +19,10 @@
 // Measured, one handle launched again and again, the quad-union kernel and this one: 2847 x 1952 x 8, 61 % sparse, 14.7 and 7.7 us
 // (17.5 MB of copy); 4096 x 2048 x 16, 50 %, 17.6 and 11.5; 317 x 930 x 11, 74 %, 6.8 and 4.8; 10 x 512 x 4, 80 %, 4.5 (row
 // kernel) and 3.8.  Error against 64 bits: 0.67 of the replaced kernels' on average over 120 launches.
+//
+// More columns, in slabs of 16 or 32: pays where a matrix is so small that the quad-union kernel's exchange of partial tiles and its
+// tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 6.8 and 4.6 us; 256 x 1136 x 36, 69 %, 7.5 and 5.4; 45 x 757 x 224, 75 %
+// (shared gather) 5.4 and 4.6.  Every slab reads the copy of the matrix again, so large ones stay there.
 //
 // Sums, zero weights and values that are not finite: as there.
 #include "so_internal.h"
@@ -62,6 +66,7 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t qw = 1u << a.qw_log2, kw = WAVES >> a.qw_log2;
     const uint32_t wq = wave & (qw - 1u), wk = wave >> a.qw_log2, quad = (blockIdx.x << a.qw_log2) + wq;
+    const uint32_t c0 = blockIdx.y * (4u * GROUPS), cols = min(a.C - c0, 4u * GROUPS);       // the slab's columns
 
     // the wave's chunks: every kw-th of the quad's.  Lane t holds the first chunk of tile t, so the tile of a chunk is a count of lanes.
     uint32_t first = 0xffffffffu, begin = 0, end = 0;
@@ -110,7 +115,26 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
             }
         }
     };
-    if (total < 4u) {
+    // Slabs: C is a multiple of four.  Places past the last column get values of others, which reach no output.
+    auto stage_slab = [&](auto loads) {
+        constexpr uint32_t N = decltype(loads)::value;
+        const float *const X = a.X + c0;
+        f32x4 v[N];
+#pragma unroll
+        for (uint32_t u = 0; u < N; ++u) {
+            const uint32_t g = min(tid + u * THREADS, a.n * GROUPS - 1u);
+            v[u] = *reinterpret_cast<const f32x4u *>(X + ((size_t)(g / GROUPS) * a.C + min(g % GROUPS * 4u, cols - 4u)));
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < N; ++u)
+            if (tid + u * THREADS < a.n * GROUPS) reinterpret_cast<f32x4 *>(lds)[tid + u * THREADS] = v[u];
+    };
+    if (gridDim.y > 1u) {
+        if constexpr (GROUPS >= 4u) {
+            if (a.n * GROUPS <= 4u * THREADS) stage_slab(std::integral_constant<uint32_t, 4>());
+            else stage_slab(std::integral_constant<uint32_t, MOST_GROUPS / THREADS>());
+        }
+    } else if (total < 4u) {
         if (tid < total) *reinterpret_cast<float *>(lds + tid / a.C * (GROUPS * 16u) + tid % a.C * 4u) = a.X[tid];
     } else if (groups <= 4u * THREADS) stage(std::integral_constant<uint32_t, 4>());
     else stage(std::integral_constant<uint32_t, MOST_GROUPS / THREADS>());
@@ -214,11 +238,11 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     const uint32_t row = quad * 4u + (lane >> 4);
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-        const bool live = row < a.m && col + k < a.C;
+        const bool live = row < a.m && col + k < cols;
         // A zero weight times a value of X that is not finite: an output that came out as NaN is computed again from the
         // row's own nonzeros, by the whole wave.
         for (uint64_t left = __ballot(live && __builtin_isnan(out[k])); left != 0u; left &= left - 1u) {
-            const uint32_t l = (uint32_t)__builtin_ctzll(left), rr = __builtin_amdgcn_readlane(row, l), cc = __builtin_amdgcn_readlane(col, l) + k;
+            const uint32_t l = (uint32_t)__builtin_ctzll(left), rr = __builtin_amdgcn_readlane(row, l), cc = c0 + __builtin_amdgcn_readlane(col, l) + k;
             const uint32_t cnt = a.nnz[rr];
             float sum = 0.0f;
             for (uint32_t e = lane; e < cnt; e += 64u) sum = __builtin_fmaf(a.Wd[(size_t)rr * a.r + e], a.X[(size_t)a.idx[(size_t)rr * a.r + e] * a.C + cc], sum);
@@ -226,15 +250,15 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
             for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
             if (lane == l) out[k] = sum;
         }
-        if (live) a.Y[(size_t)row * a.C + col + k] = so_epilogue<ACT>(out[k] + (a.bias ? a.bias[row] : 0.0f));
+        if (live) a.Y[(size_t)row * a.C + c0 + col + k] = so_epilogue<ACT>(out[k] + (a.bias ? a.bias[row] : 0.0f));
     }
 }
 
-// 16-byte groups of a row of X in LDS.
+// 16-byte groups of a row of X in LDS for C <= 32 columns.
 uint32_t groups_for(uint32_t C) { return C <= 4 ? 1u : C <= 8 ? 2u : C <= 16 ? 4u : 8u; }
 
 template <int V, int R>
-so_status launch(so_ctx *ctx, const NarrowArgs &a, uint32_t blocks, size_t lds, int act)
+so_status launch(so_ctx *ctx, const NarrowArgs &a, dim3 blocks, size_t lds, int act)
 {
 #define SO_NARROW(A)                                                                              \
     SO_HIP(so_allow_big_lds(ctx, (const void *)ellpack_matmul_narrow_kernel<V, R, A>));           \
@@ -250,41 +274,50 @@ so_status launch(so_ctx *ctx, const NarrowArgs &a, uint32_t blocks, size_t lds, 
     return SO_OK;
 }
 
-size_t lds_bytes(uint32_t n, uint32_t C) { return std::max<size_t>((size_t)n * groups_for(C) * 16u, RED_BYTES); }
+size_t lds_bytes(uint32_t n, uint32_t groups) { return std::max<size_t>((size_t)n * groups * 16u, RED_BYTES); }
 
-uint32_t quads_log2(const so_ctx *ctx, const so_ellpack *E)
+bool fits(const so_ctx *ctx, const so_ellpack *E, uint32_t groups)
 {
-    uint32_t ql = 0;
-    while (ql < LOG_WAVES && so_ceil_div(E->quads.nquads, 1u << ql) > (uint32_t)ctx->compute_units) ++ql;
-    return ql;
+    return (uint64_t)E->n * groups <= MOST_GROUPS && lds_bytes(E->n, groups) <= (size_t)ctx->max_lds_bytes;
 }
 
 } // namespace
 
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    return E->quads.d_w != nullptr && E->n != 0 && C >= 1 && C <= 32 && (uint64_t)E->n * groups_for(C) <= MOST_GROUPS && lds_bytes(E->n, C) <= (size_t)ctx->max_lds_bytes;
+    return E->quads.d_w != nullptr && E->n != 0 && C >= 1 && C <= (1u << 20) && (C <= 32 || C % 4 == 0) && E->quads.ntiles <= 64 && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
 }
 
-// Fitted to 260 launches of 10..4096 rows, 512..4096 columns, 1..32 dense columns, 50-95 % sparse, one handle again and again: 3 %
-// off on average, 11 % at most.  A workgroup's start and its copy of X, the chunks of a wave, the copy's bytes.
-double so_matmul_narrow_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+// Up to 32 columns the narrowest slab that holds them, beyond (whole groups of four only: the others' copies take up to twice as
+// long) slabs of 16 or 32 columns (blockIdx.y), whichever is estimated faster; as few quads per workgroup as give no more workgroups than compute units.  The estimate -- a workgroup's start and its
+// copy of X, the chunks of a wave, the bytes that slabs share -- was fitted to 260 launches of 10..4096 rows, 512..4096 columns, 1..32 dense columns, 50-95 %
+// sparse, one handle again and again: 3 % off on average, 11 % at most.
+so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
-    const uint32_t ql = quads_log2(ctx, E), groups = groups_for(C);
-    const double rounds = so_ceil_div(so_ceil_div(Q.nquads, 1u << ql), (uint64_t)ctx->compute_units);
-    const double copy = 1e-4 * E->n * C * (C % 4u ? 0.77 : 0.65), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
-    return 2.5 + rounds * (1.0 + (groups == 8u ? 0.3 : 0.0) + copy + chunks * (0.079 + 0.0185 * groups)) + 1.1e-5 * Q.total_chunks;
+    so_narrow_plan best{};
+    best.us = 1e30;
+    for (uint32_t groups : {1u, 2u, 4u, 8u}) {
+        if (C <= 32 ? groups != groups_for(C) : groups < 4u || !fits(ctx, E, groups)) continue;
+        const uint32_t slabs = so_ceil_div(C, 4u * groups);
+        uint32_t ql = 0;
+        while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
+        const double rounds = so_ceil_div((uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs, (uint64_t)ctx->compute_units);
+        const double copy = 1e-4 * E->n * (slabs > 1 ? 4.6 * groups : C) * (C % 4u ? 0.77 : 0.65), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
+        const double us = 2.5 + rounds * (1.0 + (groups == 8u ? 0.3 : 0.0) + copy + chunks * (0.079 + 0.0185 * groups)) + 1.1e-5 * Q.total_chunks;
+        if (us < best.us) best = so_narrow_plan{ql, groups, slabs, us};
+    }
+    return best;
 }
 
-so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
+so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const so_narrow_plan &p, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
     const so_quads &Q = E->quads;
-    const uint32_t ql = quads_log2(ctx, E);
-    const NarrowArgs a{Q.d_w, (const uint8_t *)Q.d_off, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, ql, (uint32_t)(((1ull << 32) + C - 1u) / C), dX, dBias, dY, E->d_Wd, E->d_idx, E->d_nnz, E->r};
-    const uint32_t blocks = so_ceil_div(Q.nquads, 1u << ql);
-    const size_t lds = lds_bytes(E->n, C);
-    switch (groups_for(C)) {
+    const NarrowArgs a{Q.d_w, (const uint8_t *)Q.d_off, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, p.qw_log2, (uint32_t)(((1ull << 32) + C - 1u) / C),
+                       dX, dBias, dY, E->d_Wd, E->d_idx, E->d_nnz, E->r};
+    const dim3 blocks(so_ceil_div(Q.nquads, 1u << p.qw_log2), p.slabs);
+    const size_t lds = lds_bytes(E->n, p.groups);
+    switch (p.groups) {
     case 1:  return launch<1, 1>(ctx, a, blocks, lds, act);
     case 2:  return launch<2, 1>(ctx, a, blocks, lds, act);
     case 4:  return launch<4, 1>(ctx, a, blocks, lds, act);

@@ -225,10 +225,11 @@ so_status so_matmul_quad_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_plan &p, const float *dX, uint32_t C,
                                 const float *dBias, float *dY, int act);
 
-// csrc/matmul_narrow.hip: up to 32 dense columns on the quad-union copy.
+// csrc/matmul_narrow.hip: few dense columns, or few rows, on the quad-union copy.
+struct so_narrow_plan { uint32_t qw_log2, groups, slabs; double us; };   // log2 of the quads per workgroup, 16-byte groups of a slab's row of X, slabs
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
-double so_matmul_narrow_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);     // us
-so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
+so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const so_narrow_plan &p, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
 
 // csrc/matmul_planes.hip: the bf16 planes and their kernel.
 struct so_planes_plan { uint32_t ks, iters, iters_per, nslab, mbs; double us; };   // workgroups per tile, iterations in all and of each, slabs, row blocks

@@ -1,4 +1,4 @@
-"""The narrow kernel of SO_LAYOUT_RBM (csrc/matmul_narrow.hip): up to 32 dense columns, forced, at the edges of its column
+"""The narrow kernel of SO_LAYOUT_RBM (csrc/matmul_narrow.hip): up to 32 dense columns, or slabs of 16 and 32, forced, at the edges of its column
 groups (4, 8, 16, 32), its copy of X (4096 and 10 240 groups of four values; rows of no multiple of four), its chunks of 16
 steps and batches of 4 chunks, its tiles of 256 columns and 4 rows and its quads per workgroup (more than 1024 rows: two); and
 which calls it takes by itself.
@@ -38,7 +38,7 @@ def narrow_matmul(ctx, E, X, bias, act="none", at=0):
 @pytest.mark.parametrize("m,n,C,sp", [
     (1, 1, 1, .0), (1, 1, 3, .0), (3, 2, 4, .0), (4, 255, 5, .5), (5, 256, 8, .5), (63, 257, 9, .5), (64, 300, 16, .7), (65, 511, 17, .3), (130, 513, 31, .95),
     (129, 1025, 32, .8), (300, 10240, 4, .9), (20, 10240, 3, .5), (17, 5120, 8, .99), (40, 2560, 13, .2), (1000, 1280, 30, .6), (1025, 700, 2, .5),
-    (2049, 600, 7, .9), (4097, 512, 12, .7), (16400, 300, 6, .9), (33000, 260, 4, .97)])
+    (2049, 600, 7, .9), (10, 2560, 36, .5), (77, 1280, 64, .6), (130, 900, 100, .7), (500, 513, 132, .9), (4097, 512, 12, .7), (16400, 300, 6, .9), (33000, 260, 4, .97)])
 @pytest.mark.parametrize("at", [0, 1])
 def test_narrow_shapes(ctx, oracle, m, n, C, sp, at):
     rng = np.random.default_rng(m * 31 + n * 7 + C)
@@ -89,7 +89,7 @@ def test_rows_in_any_order(ctx, oracle):
         a.free()
 
 
-@pytest.mark.parametrize("m,n,C,sp,want", [(2000, 1500, 8, .6, True), (2000, 1500, 33, .6, False), (2000, 2600, 16, .6, False), (2000, 600, 30, .97, False),
+@pytest.mark.parametrize("m,n,C,sp,want", [(2000, 1500, 8, .6, True), (2000, 1500, 33, .6, False), (2000, 1500, 64, .6, False), (84, 692, 148, .5, True), (84, 692, 149, .5, False), (2000, 2600, 16, .6, False), (2000, 600, 30, .97, False),
                                            (2000, 1500, 3, .5, True), (300, 1500, 3, .5, False), (2000, 1500, 1, .5, False)])
 def test_which_calls_take_it(ctx, m, n, C, sp, want):
     """Also while a graph is recorded (no workspace is needed), whose replays give the same bits."""
