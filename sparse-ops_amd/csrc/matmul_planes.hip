@@ -43,6 +43,8 @@ constexpr uint32_t BUF = STEPS * NT * 3 * FRAG;         // LDS of one iteration'
 constexpr uint32_t SPILL = 8;                           // iterations after which the large sums leave their registers
 constexpr uint32_t SUMS_AT = 2 * BUF, FLAGS_AT = SUMS_AT + BM * BN * 4, LDS_BYTES = FLAGS_AT + BN * 4 + 16;
 static_assert(SPLITTERS == KI / 8 * BN, "a splitting thread takes one column's group of 8 rows");
+constexpr uint32_t kMostColumns = (1u << 24) - 1u;      // a row tile's planes, 192 bytes per column, are addressed with 32 bits
+static_assert(((uint64_t)kMostColumns + KI) / 16 * 3 * FRAG <= 0xffffffffull, "offsets into a row tile's planes");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -373,7 +375,7 @@ so_planes_plan so_matmul_planes_choose(const so_ctx *ctx, uint32_t m, uint32_t n
 so_status so_planes_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *nnz)
 {
     so_planes &P = E->planes;
-    if (!E->ascending || E->total_nnz == 0) return SO_OK;            // (a column named twice by a row has one place)
+    if (!E->ascending || E->total_nnz == 0 || E->n > kMostColumns) return SO_OK;       // (a column named twice by a row has one place)
     // values that have room for three planes, and no overflow on the way
     std::atomic<bool> room{true};
     so_parallel(E->m, E->total_nnz, [&](uint32_t i0, uint32_t i1) {

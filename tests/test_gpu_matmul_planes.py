@@ -141,6 +141,27 @@ def test_planes_left_out(ctx):
             dE.free()
 
 
+@pytest.mark.parametrize("n,want", [(2 ** 24 - 1, True), (2 ** 24, False), (22369664, False)])
+def test_planes_very_many_columns(ctx, n, want):
+    """192 bytes of planes per column and row tile: beyond 2^32 of them (22 369 600 columns) an offset no longer fits 32 bits, and
+    handles do without from 2^24 columns on.  The last columns count."""
+    m, r, C = 3, 40, 2
+    rng = np.random.default_rng(5)
+    idx = np.sort(rng.choice(n - 1, (m, r), replace=False), axis=1).astype(np.uint32)
+    idx[:, -1] = n - 1
+    Wd = rng.standard_normal((m, r)).astype(np.float32)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    ref = (Wd[:, :, None].astype(np.float64) * X[idx]).sum(axis=1)
+    with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1"):
+        dE = ctx.upload_ellpack(Wd, idx, np.full(m, r, np.uint32), m, n, r, RBM)
+        dX, dY = ctx.array(X), ctx.empty((m, C))
+        ctx.matmul(dE, dX, C, None, dY)
+        assert (ctx.last_kernel() == "planes") == want
+        assert rel_err(dY.download(), ref) <= TOL
+    for a in (dX, dY, dE):
+        a.free()
+
+
 def test_planes_by_default(ctx, oracle):
     """The dispatch's own choice: a half-full matrix on a wide batch takes the kernel, a batch of ones or a very sparse matrix does not;
     a column's bits do not depend on its neighbours."""
