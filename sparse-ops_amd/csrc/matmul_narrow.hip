@@ -36,6 +36,7 @@ namespace {
 constexpr uint32_t KT = so_quads::kTileRows, WAVES = 16, LOG_WAVES = 4, THREADS = WAVES * 64, AHEAD = 4;
 constexpr uint32_t MOST_GROUPS = 10 * THREADS;   // 16-byte groups of X in LDS: 160 KB
 constexpr uint32_t RED_BYTES = THREADS * 8;       // the waves' sums, in the place of X
+constexpr uint32_t MOST_COLUMNS = 65535u * 16u;   // slabs of 16 are counted by blockIdx.y
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -285,7 +286,7 @@ bool fits(const so_ctx *ctx, const so_ellpack *E, uint32_t groups)
 
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    return E->quads.d_w != nullptr && E->n != 0 && C >= 1 && C <= (1u << 20) && (C <= 32 || C % 4 == 0) && E->quads.ntiles <= 64 && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
+    return E->quads.d_w != nullptr && E->n != 0 && C >= 1 && C <= MOST_COLUMNS && (C <= 32 || C % 4 == 0) && E->quads.ntiles <= 64 && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
 }
 
 // Up to 32 columns the narrowest slab that holds them, beyond (whole groups of four only: the others' copies take up to twice as

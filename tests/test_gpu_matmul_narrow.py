@@ -71,6 +71,24 @@ def test_values_that_are_not_finite(ctx, oracle, C):
     assert np.abs(Y[fin] - want[fin]).max() <= TOL * np.abs(want[fin]).max()
 
 
+@pytest.mark.parametrize("C,want", [(65535 * 16, "narrow"), (65535 * 16 + 4, None), (2 ** 20, None)])
+def test_very_wide(ctx, C, want):
+    """A grid has at most 65 535 workgroups in y: slabs of 16 columns, all that fit beside more than 1280 rows of X, end at 1 048 560."""
+    n, cols = 1281, np.array([0, 700, 1280], np.uint32)
+    Wd = np.array([[1.5, -2.0, 0.75]], np.float32)
+    rows = np.random.default_rng(C).standard_normal((3, C)).astype(np.float32)
+    dE, dX, dY = ctx.upload_ellpack(Wd, cols[None], np.array([3], np.uint32), 1, n, 3, RBM), ctx.empty((n, C)), ctx.empty((1, C))
+    ctx.fill_zero(dX)
+    for k, x in zip(cols, rows):
+        ctx._ck(ctx.lib.so_h2d(ctx.h, dX.ptr + 4 * int(k) * C, hipabi._ptr(x), x.nbytes))
+    with ctx.tuning(SPARSEOPS_MATMUL_NARROW="1"):
+        ctx.matmul(dE, dX, C, None, dY)
+        assert (ctx.last_kernel() == "narrow") == (want == "narrow")
+    assert rel_err(dY.download(), Wd.astype(np.float64) @ rows) <= TOL
+    for a in (dX, dY, dE):
+        a.free()
+
+
 def test_rows_in_any_order(ctx, oracle):
     """Columns of a row unordered and named twice: two steps of the union."""
     rng = np.random.default_rng(2)
