@@ -71,8 +71,8 @@ enum { SO_ACT_NONE = 0, SO_ACT_RELU = 1, SO_ACT_SIGMOID = 2, SO_ACT_TANH = 3 };
  *        The layout also holds a second copy for smaller launches and fuller matrices: quads of four rows
  *        with the union of their columns, multiplied on the matrix cores in fp32 (csrc/matmul_quad.hip, up to 32 dense columns csrc/matmul_narrow.hip); and, for matrices
  *        full enough that a launch at some width is estimated to gain by it (half full to about 75 % sparse, from a
- *        few million entries on), a third: the dense matrix as three bf16 planes whose sum is the fp32 matrix, multiplied
- *        on the bf16 matrix cores in fp32 precision (csrc/matmul_planes.hip).
+ *        few million entries on; stored weights of 2^-76 to 2^39 in size), a third: the dense matrix as three bf16 planes whose sum is
+ *        the fp32 matrix, multiplied on the bf16 matrix cores in fp32 precision (csrc/matmul_planes.hip).
  *        so_matmul takes whichever of them, so_matvec's row kernel (one to three columns) or the kernels
  *        of the other layouts it estimates to be the fastest.
  *        Sums are not taken in a row's slot order: results agree with

@@ -41,10 +41,26 @@ constexpr uint32_t STEPS = 4, KI = 16 * STEPS;          // an iteration: runs of
 constexpr uint32_t BM = 128, BN = 64, NT = BN / 32;     // a workgroup's rows and dense columns
 constexpr uint32_t BUF = STEPS * NT * 3 * FRAG;         // LDS of one iteration's X
 constexpr uint32_t SPILL = 8;                           // iterations after which the large sums leave their registers
-constexpr uint32_t SUMS_AT = 2 * BUF, FLAGS_AT = SUMS_AT + BM * BN * 4, LDS_BYTES = FLAGS_AT + BN * 4 + 16;
+constexpr uint32_t SUMS_AT = 2 * BUF, KEPT_AT = SUMS_AT + BM * BN * 4, FLAGS_AT = KEPT_AT + BM * BN * 4, LDS_BYTES = FLAGS_AT + 16;
 static_assert(SPLITTERS == KI / 8 * BN, "a splitting thread takes one column's group of 8 rows");
 constexpr uint32_t kMostColumns = (1u << 24) - 1u;      // a row tile's planes, 192 bytes per column, are addressed with 32 bits
 static_assert(((uint64_t)kMostColumns + KI) / 16 * 3 * FRAG <= 0xffffffffull, "offsets into a row tile's planes");
+
+// The planes hold X times 2^24 and the matrix times 2^-24: then the last bit of any float of X, 2^-149, is a bf16 of normal size, and so
+// is that of any weight from kLeastWeight on.  A pass for large values takes X times 2^-64.  With weights of at most kMostWeight and fewer than
+// 2^24 columns no sum of values below kLarge, nor of large ones scaled down, leaves the range: 24 + 39 + 40 bits, 24 + 39 - 24 + 128 - 64.
+constexpr float kUp = 0x1p24f, kLarge = 0x1p40f, kLargeDown = 0x1p-88f, kMostWeight = 0x1p39f, kLeastWeight = 0x1p-76f;
+
+// The passes of a workgroup over its range of K: ordinarily the first alone.
+enum Pass : uint32_t { ALL, SMALL, LARGE, NOT_FINITE };
+// flags[ALL] asks for the others, flags[LARGE] and flags[NOT_FINITE] say whether there is anything to do in them.
+__device__ __forceinline__ uint32_t next_pass(uint32_t pass, const uint32_t *flags)
+{
+    const auto set = [&](uint32_t p) { return __builtin_amdgcn_readfirstlane(flags[p]) != 0u; };
+    if (pass == ALL) return set(ALL) ? SMALL : ALL;
+    if (pass == SMALL && set(LARGE)) return LARGE;
+    return pass != NOT_FINITE && set(NOT_FINITE) ? NOT_FINITE : ALL;
+}
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -60,9 +76,6 @@ struct PlanesArgs {
     const float *X, *bias;
     float *Y, *part;
     uint32_t *counters;
-    const float *Wd;            // the ROW arrays, for outputs that are computed again
-    const uint32_t *idx, *nnz;
-    uint32_t r;
 };
 
 // Two floats to bf16 (nearest even), the first in the low half; `v` keeps what is left of them.
@@ -78,41 +91,32 @@ __device__ __forceinline__ uint32_t last_plane(float v0, float v1)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{v0, v1}, bf16x2));
 }
 
-// Sum over row `row`'s own nonzeros of one column of X, added up by the 16 lanes that share the row.
-__device__ __forceinline__ float exact_output(const PlanesArgs &a, uint32_t row, uint32_t col, uint32_t sub)
+// Of two bf16 numbers their signs, as +-1 or 0.
+__device__ __forceinline__ uint32_t signs_of(uint32_t pair)
 {
-    constexpr uint32_t AHEAD = 8;
-    const uint32_t cnt = row < a.m ? a.nnz[row] : 0u;
-    const float *w = a.Wd + (size_t)row * a.r;
-    const uint32_t *ix = a.idx + (size_t)row * a.r;
-    float sum = 0.0f;
-    for (uint32_t k = sub; k < cnt; k += 16u * AHEAD) {
-        float wk[AHEAD], x[AHEAD];
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u) {
-            const uint32_t at = min(k + 16u * u, cnt - 1u);
-            wk[u] = w[at];
-            x[u] = a.X[(size_t)ix[at] * a.C + col];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u)
-            if (k + 16u * u < cnt) sum = __builtin_fmaf(wk[u], x[u], sum);
-    }
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    return sum;
+    const uint32_t some = (((pair & 0x7fff7fffu) + 0x7fff7fffu) & 0x80008000u) >> 15;      // a bit per number that is not 0
+    return some * 0x3f80u | (pair & (some << 15));
 }
 
 // A workgroup owns 128 rows x 64 columns and a range of K.  Twelve waves: four multiply, 32 rows x 64 columns each; eight
 // fetch X, split it and store the planes in LDS, an iteration of 64 rows of X ahead (two buffers, a barrier per iteration).
 // A SIMD has one of the former and two of the latter, so that the splitting's vector instructions run in the shadow of
 // the MFMAs.
+//
+// Values that the scaled planes cannot hold -- infinities, NaNs and finite ones from 2^104 on -- come out of the splitting as NaN, and sums
+// that overflow do not come out finite.  The workgroup then goes over its range of K again: with the values below 2^40
+// alone, with the finite ones above it alone (scaled down), and for infinities and NaNs with the signs of the matrix, counting in whole
+// numbers what an output receives: as many of one sign as in all is an infinity, otherwise a NaN.  A zero of the matrix meets none of them.
+// Us with ordinary values, with an infinity in one column, an infinity or a NaN in each, 1e32 in each: 3001 x 2777 x 101 at 70 % 21, 43, 44, 46 (the
+// row-block-merged kernel 29 with any); 4096 x 4096 x 256 at 50 % 49, 106, 122, 129 (the quad-union kernel 97, 197, 2380, 92).  Tiny
+// values cost nothing.  (Giving up every column with one of these, or with a nonzero value below 2^-110, and summing its outputs
+// over the nonzeros took 98 with one such column, 4660 with one such value in each; 240 and 14 400.)
 template <int ACT>
 __global__ __launch_bounds__(THREADS)
 void ellpack_matmul_planes_kernel(PlanesArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    uint32_t *flags = reinterpret_cast<uint32_t *>(lds + FLAGS_AT);  // [BN] columns with values too small to be split, then the arrival word
+    uint32_t *flags = reinterpret_cast<uint32_t *>(lds + FLAGS_AT);  // by pass; [SMALL]: the arrival word
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // Workgroup ids go round the 8 XCDs; an XCD takes a contiguous share of the (K part, row block, slab) triples, so that
@@ -121,7 +125,7 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
     if ((blockIdx.x >> 3) >= a.per_xcd || id >= tiles * a.ks) return;
     const uint32_t kp = id / tiles, tile = id - kp * tiles, mb = tile / a.nslab, slab = tile - mb * a.nslab;
     const uint32_t it0 = kp * a.iters_per, count = min(a.iters, it0 + a.iters_per) - it0;
-    if (tid < BN + 1u) flags[tid] = 0u;
+    if (tid < 4u) flags[tid] = 0u;
 
     if (wave >= MULTIPLIERS / 64u) {
         // A thread takes 8 rows of one column, a wave the same rows.  Rows past the last one come as zeros: out of the buffer's range.
@@ -131,7 +135,7 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
         for (uint32_t j = 0; j < 8; ++j) at[j] = (g * 8u + j) * pitch + min(slab * BN + xc, a.C - 1u) * 4u;
         u32x4 *const to = reinterpret_cast<u32x4 *>(lds + ((g >> 1) * NT + (xc >> 5)) * 3u * FRAG) + (g & 1u) * 32u + (xc & 31u);
         float x[2][8];
-        uint32_t least = 0xffffffffu;
+        float odd = 0.0f;                                            // becomes NaN with a value that the planes do not hold
         auto request = [&](int set, uint32_t it) {
             const uint64_t from = (uint64_t)it * step, end = (uint64_t)a.n * pitch;
             const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.X) + from / 4u, 0, from < end ? (int)(uint32_t)(end - from) : 0, 0x00020000);
@@ -143,42 +147,69 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
             u32x4 p0, p1, p2;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                float v0 = x[set][2 * e], v1 = x[set][2 * e + 1];
-                // the smallest nonzero value (times two, minus one, as an integer: a zero becomes the largest)
-                least = min(least, min((__float_as_uint(v0) << 1) - 1u, (__float_as_uint(v1) << 1) - 1u));
+                float v0 = x[set][2 * e] * kUp, v1 = x[set][2 * e + 1] * kUp;
                 p0[e] = take_plane(v0, v1);
                 p1[e] = take_plane(v0, v1);
                 p2[e] = last_plane(v0, v1);
+                odd = __builtin_elementwise_maximum(odd, __builtin_elementwise_maximum(v0, v1));   // (inf - inf)
             }
             u32x4 *p = to + set * (BUF / 16u);
             p[0] = p0; p[64] = p1; p[128] = p2;
             __builtin_amdgcn_sched_barrier(0);
         };
-        request(0, it0);
-        request(1, it0 + 1u);
-        split(0);
-        __syncthreads();
-        // (nothing in the loops is conditional, so that the compiler's waits leave the younger requests in flight; what they
-        // fetch past the end is not used)
-        for (uint32_t i = 0; i + 1u < count; i += 2u) {
-            request(0, it0 + i + 2u);
-            split(1);
+        auto fill = [&](auto &&put) {
+            request(0, it0);
+            request(1, it0 + 1u);
+            put(0);
             __syncthreads();
-            request(1, it0 + i + 3u);
-            split(0);
+            // (nothing in the loops is conditional, so that the compiler's waits leave the younger requests in flight; what they
+            // fetch past the end is not used)
+            for (uint32_t i = 0; i + 1u < count; i += 2u) {
+                request(0, it0 + i + 2u);
+                put(1);
+                __syncthreads();
+                request(1, it0 + i + 3u);
+                put(0);
+                __syncthreads();
+            }
+            if (count & 1u) __syncthreads();
+        };
+        fill(split);
+        if (__builtin_isnan(odd)) flags[ALL] = 1u;
+        __syncthreads();
+#pragma unroll 1
+        for (uint32_t pass = next_pass(ALL, flags); __builtin_expect(pass != ALL, 0); pass = next_pass(pass, flags)) {
+            bool large = false, not_finite = false;
+            fill([&](int set) {
+                uint32_t sign[8], any[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float v = x[set][j], size = __builtin_fabsf(v);
+                    const bool below = size < kLarge, finite = size <= 3.40282347e38f;
+                    large |= !below && finite;
+                    not_finite |= !finite;
+                    any[j] = finite ? 0u : 0x3f80u;
+                    sign[j] = finite || __builtin_isnan(v) ? 0u : __float_as_uint(v) >> 31 << 15 | 0x3f80u;
+                    x[set][j] = pass == SMALL ? (below ? v : 0.0f) : !below && finite ? v * kLargeDown : 0.0f;
+                }
+                if (pass != NOT_FINITE) { split(set); return; }
+                u32x4 *p = to + set * (BUF / 16u);
+                p[0] = u32x4{sign[0] | sign[1] << 16, sign[2] | sign[3] << 16, sign[4] | sign[5] << 16, sign[6] | sign[7] << 16};
+                p[64] = u32x4{any[0] | any[1] << 16, any[2] | any[3] << 16, any[4] | any[5] << 16, any[6] | any[7] << 16};
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if (pass == SMALL && large) flags[LARGE] = 1u;
+            if (pass == SMALL && not_finite) flags[NOT_FINITE] = 1u;
             __syncthreads();
         }
-        if (count & 1u) __syncthreads();
-        // A value below 2^-110 has no room for three planes: its column is computed again from the nonzeros, by way of NaN.
-        if (least < ((17u << 23) << 1) - 1u) flags[xc] = 1u;
-        __syncthreads();
         if (a.ks > 1u) { __syncthreads(); __syncthreads(); }
         return;
     }
 
-    f32x16 big[2], small[2];
-    f32x4 *const sums = reinterpret_cast<f32x4 *>(lds + SUMS_AT) + tid;
+    f32x4 s[8];                                                      // element i = 4 j + e of tile t: s[4 t + j][e]
     {
+        f32x16 big[2], small[2];
+        f32x4 *const sums = reinterpret_cast<f32x4 *>(lds + SUMS_AT) + tid, *const kept = reinterpret_cast<f32x4 *>(lds + KEPT_AT) + tid;
         const uint32_t rt = min(mb * 4u + wave, (a.m + 31u) / 32u - 1u);   // row tiles past the last repeat it
         const uint32_t bytes = a.k16 * 3u * FRAG, lane16 = lane * 16u;
         const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(a.A) + (size_t)rt * bytes, 0, (int)bytes, 0x00020000);
@@ -198,55 +229,104 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, p), __builtin_bit_cast(bf16x8, q), acc, 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         };
+        auto clear = [&] {
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+            for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int k = 0; k < 16; ++k) big[t][k] = small[t][k] = 0.0f;
+                for (int k = 0; k < 16; ++k) big[t][k] = small[t][k] = 0.0f;
+        };
+        auto multiply = [&] {
+            clear();
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sums[j * MULTIPLIERS] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // A run's six products of one tile while the other tile's operands come from LDS; the matrix's are requested an
-        // iteration ahead, into the registers of the run that is done with.
+            for (int j = 0; j < 8; ++j) sums[j * MULTIPLIERS] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // A run's six products of one tile while the other tile's operands come from LDS; the matrix's are requested an
+            // iteration ahead, into the registers of the run that is done with.
 #pragma unroll
-        for (int s = 0; s < (int)STEPS; ++s) request(s, 0u);
-        __syncthreads();
-        for (uint32_t i = 0; i < count; ++i) {
-            const uint32_t buf = i & 1u;
-            read(buf, 0, 0);
-#pragma unroll
-            for (int s = 0; s < (int)STEPS; ++s) {
-                const u32x4 *v = w[s];
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    if (t == 0) read(buf, s, 1);
-                    else if (s + 1 < (int)STEPS) read(buf, s + 1, 0);
-                    mfma(v[2], x[t][0], small[t]); mfma(v[0], x[t][0], big[t]); mfma(v[0], x[t][2], small[t]);
-                    mfma(v[1], x[t][1], small[t]); mfma(v[1], x[t][0], small[t]); mfma(v[0], x[t][1], small[t]);
-                }
-                request(s, i + 1u);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            // long sums are rounded more often: each lane keeps its totals in LDS
-            if (i % SPILL == SPILL - 1u) {
-                f32x4 v[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = sums[j * MULTIPLIERS];
-#pragma unroll
-                for (int k = 0; k < 32; ++k) { v[k / 4][k % 4] += big[k / 16][k % 16]; big[k / 16][k % 16] = 0.0f; }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) sums[j * MULTIPLIERS] = v[j];
-            }
+            for (int s = 0; s < (int)STEPS; ++s) request(s, 0u);
             __syncthreads();
+            for (uint32_t i = 0; i < count; ++i) {
+                const uint32_t buf = i & 1u;
+                read(buf, 0, 0);
+#pragma unroll
+                for (int s = 0; s < (int)STEPS; ++s) {
+                    const u32x4 *v = w[s];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        if (t == 0) read(buf, s, 1);
+                        else if (s + 1 < (int)STEPS) read(buf, s + 1, 0);
+                        mfma(v[2], x[t][0], small[t]); mfma(v[0], x[t][0], big[t]); mfma(v[0], x[t][2], small[t]);
+                        mfma(v[1], x[t][1], small[t]); mfma(v[1], x[t][0], small[t]); mfma(v[0], x[t][1], small[t]);
+                    }
+                    request(s, i + 1u);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // long sums are rounded more often: each lane keeps its totals in LDS
+                if (i % SPILL == SPILL - 1u) {
+                    f32x4 v[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[j] = sums[j * MULTIPLIERS];
+#pragma unroll
+                    for (int k = 0; k < 32; ++k) { v[k / 4][k % 4] += big[k / 16][k % 16]; big[k / 16][k % 16] = 0.0f; }
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) sums[j * MULTIPLIERS] = v[j];
+                }
+                __syncthreads();
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                s[j] = sums[j * MULTIPLIERS];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[j][e] += big[j / 4][j % 4 * 4 + e] + small[j / 4][j % 4 * 4 + e];
+            }
+        };
+        multiply();
+        float most = 0.0f;                                           // infinite or NaN where a sum is not finite
+#pragma unroll
+        for (int k = 0; k < 32; k += 2)
+            most = __builtin_elementwise_maximum(most, __builtin_elementwise_maximum(__builtin_fabsf(s[k / 4][k % 4]), __builtin_fabsf(s[k / 4][k % 4 + 1])));
+        if (!(most <= 3.40282347e38f)) flags[ALL] = 1u;
+        __syncthreads();                                             // the flags
+        uint32_t pass = next_pass(ALL, flags);
+        if (__builtin_expect(pass != ALL, 0)) {
+#pragma unroll 1
+            do {
+                multiply();
+#pragma unroll
+                for (int j = 0; j < 8; ++j) kept[j * MULTIPLIERS] = pass == SMALL ? s[j] : kept[j * MULTIPLIERS] + s[j] * (1.0f / kLargeDown);
+                __syncthreads();
+                pass = next_pass(pass, flags);
+            } while (pass == LARGE);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) s[j] = kept[j * MULTIPLIERS];
+            if (pass == NOT_FINITE) {
+                clear();
+                __syncthreads();
+#pragma unroll 1
+                for (uint32_t i = 0; i < count; ++i) {
+#pragma unroll
+                    for (int s = 0; s < (int)STEPS; ++s) request(s, i);
+#pragma unroll
+                    for (int s = 0; s < (int)STEPS; ++s) {
+                        u32x4 sign, any;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) { sign[k] = signs_of(w[s][0][k]); any[k] = sign[k] & 0x7fff7fffu; }
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            read(i & 1u, s, t);
+                            mfma(sign, x[t][0], big[t]);
+                            mfma(any, x[t][1], small[t]);
+                        }
+                    }
+                    __syncthreads();
+                }
+                __syncthreads();
+#pragma unroll
+                for (int k = 0; k < 32; ++k) {
+                    const float signs = big[k / 16][k % 16], all = small[k / 16][k % 16];
+                    if (all != 0.0f) s[k / 4][k % 4] = __builtin_fabsf(signs) == all ? __builtin_copysignf(INFINITY, signs) : NAN;
+                }
+            }
         }
-    }
-    __syncthreads();                                                 // the flags
-    f32x4 s[8];                                                      // element i = 4 j + e of tile t: s[4 t + j][e]
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const bool lost = flags[t * 32u + (lane & 31u)] != 0u;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[4 * t + i / 4][i % 4] = lost ? NAN : big[t][i] + small[t][i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[4 * t + j] += sums[(t * 4 + j) * MULTIPLIERS];
     }
     if (a.ks > 1u) {
         // sc1: written through to memory, whichever XCD the tile's other workgroups run on
@@ -256,9 +336,9 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
         for (int j = 0; j < 8; ++j) __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, s[j]), pr, (int)((kp * 8u + j) * 4096u + tid * 16u), 0, SC1);
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
         __syncthreads();
-        if (tid == 0) flags[BN] = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 0) flags[SMALL] = __hip_atomic_fetch_add(&a.counters[tile], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        if (flags[BN] != a.ks - 1u) return;                          // the last workgroup of the tile to arrive finishes it
+        if (flags[SMALL] != a.ks - 1u) return;                          // the last workgroup of the tile to arrive finishes it
         if (tid == 0) __hip_atomic_store(&a.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // ready for the next launch
 #pragma unroll
         for (int j = 0; j < 8; ++j) s[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -286,32 +366,13 @@ void ellpack_matmul_planes_kernel(PlanesArgs a)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const uint32_t c = slab * BN + t * 32u + (lane & 31u);
-        uint32_t lost = 0;                                           // a bit per row of the tile that is not finite
-        if (c < a.C) {
-            const uint32_t at = (row0 + 4u * half) * pitch + c * 4u;
+        if (c >= a.C) continue;
+        const uint32_t at = (row0 + 4u * half) * pitch + c * 4u;
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = s[4 * t + j][e];
-                    lost |= !(__builtin_fabsf(v) <= 3.40282347e38f) ? 1u << (8 * j + e) : 0u;      // the planes of a finite sum may overflow
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(so_epilogue<ACT>(v + bias[j][e])), yr, (int)(at + (8u * j + e) * pitch), 0, 0);
-                }
-            lost <<= 4u * half;
-        }
-        lost |= __shfl_xor(lost, 32, 64);
-        // those again, from the row's own nonzeros: four rows of a column at a time
-#pragma unroll 1
-        for (uint64_t left = __ballot(lost != 0u && half == 0u); left != 0u; left &= left - 1u) {
-            const uint32_t l = (uint32_t)__builtin_ctzll(left), rows = __builtin_amdgcn_readlane(lost, l), cc = __builtin_amdgcn_readlane(c, l);
-#pragma unroll 1
-            for (uint32_t q = 0; q < 32u; q += 4u) {
-                if (((rows >> q) & 15u) == 0u) continue;
-                const uint32_t in = q + (lane >> 4), row = row0 + in;
-                const float v = exact_output(a, row, cc, lane & 15u);
-                if ((lane & 15u) == 0u && row < a.m && ((rows >> in) & 1u)) a.Y[(size_t)row * a.C + cc] = so_epilogue<ACT>(v + (a.bias ? a.bias[row] : 0.0f));
-            }
-        }
+            for (int e = 0; e < 4; ++e)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(so_epilogue<ACT>(s[4 * t + j][e] + bias[j][e])), yr, (int)(at + (8u * j + e) * pitch), 0, 0);
     }
 }
 
@@ -323,7 +384,7 @@ void planes_scatter_kernel(const float *__restrict__ Wd, const uint32_t *__restr
     const uint32_t row = blockIdx.x;
     for (uint32_t s = threadIdx.x; s < nnz[row]; s += 256u) {
         const uint32_t k = idx[(size_t)row * r + s];
-        float v = Wd[(size_t)row * r + s], zero = 0.0f;
+        float v = Wd[(size_t)row * r + s] * (1.0f / kUp), zero = 0.0f;
         const uint32_t p0 = take_plane(v, zero), p1 = take_plane(v, zero), p2 = last_plane(v, zero);
         uint16_t *to = A + ((size_t)(row >> 5) * k16 + (k >> 4)) * (3 * FRAG / 2) + ((row & 31u) + ((k >> 3) & 1u) * 32u) * 8u + (k & 7u);
         to[0] = (uint16_t)p0; to[FRAG / 2] = (uint16_t)p1; to[FRAG] = (uint16_t)p2;
@@ -376,14 +437,14 @@ so_status so_planes_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uin
 {
     so_planes &P = E->planes;
     if (!E->ascending || E->total_nnz == 0 || E->n > kMostColumns) return SO_OK;       // (a column named twice by a row has one place)
-    // values that have room for three planes, and no overflow on the way
+    // values that have room for three planes and overflow nothing, and no stored zeros (which make NaNs of infinities in X)
     std::atomic<bool> room{true};
     so_parallel(E->m, E->total_nnz, [&](uint32_t i0, uint32_t i1) {
         bool ok = true;
         for (uint32_t i = i0; i < i1 && ok; ++i)
             for (uint32_t k = 0; k < nnz[i]; ++k) {
                 const float v = std::fabs(Wd[(size_t)i * E->r + k]);
-                ok = ok && v <= 0x1p120f && (v == 0.0f || v >= 0x1p-100f);
+                ok = ok && v <= kMostWeight && v >= kLeastWeight;
             }
         if (!ok) room = false;
     });
@@ -425,8 +486,7 @@ so_status so_matmul_planes_launch(so_ctx *ctx, const so_ellpack *E, const so_pla
     if (s != SO_OK) return s;
     const uint32_t per_xcd = so_ceil_div((uint64_t)p.mbs * p.nslab * p.ks, 8);
     const PlanesArgs a{(const char *)E->planes.d_a, E->m, E->n, C, E->planes.k16, p.ks, p.iters, p.iters_per, p.nslab, p.mbs, per_xcd, dX, dBias, dY,
-                       ctx->mm_part ? (float *)ctx->mm_part->p : nullptr, ctx->mm_counters ? (uint32_t *)ctx->mm_counters->p : nullptr,
-                       E->d_Wd, E->d_idx, E->d_nnz, E->r};
+                       ctx->mm_part ? (float *)ctx->mm_part->p : nullptr, ctx->mm_counters ? (uint32_t *)ctx->mm_counters->p : nullptr};
     const uint32_t blocks = 8u * per_xcd;
     switch (act) {
     case SO_ACT_RELU:    return launch<SO_ACT_RELU>(ctx, a, blocks);

@@ -118,19 +118,81 @@ def test_planes_values_too_small_for_three_planes(ctx, oracle, exponent):
         assert np.abs(Y[:, c] - Yo[:, c]).max() <= TOL * np.abs(Yo[:, c]).max() + n * 2.0 ** -149, c
 
 
+@pytest.mark.parametrize("split", [1, 2, 3])
+@pytest.mark.parametrize("m,n,C", [(130, 640, 66), (200, 705, 130)])
+def test_planes_values_of_any_size(ctx, oracle, split, m, n, C):
+    """Values around 2^40, 2^104 and the largest float beside ordinary and tiny ones, alone and many in a column, and infinities and NaNs among
+    them: the passes that a workgroup takes for them, one, two, three and four; a slab without any beside one with."""
+    rng = np.random.default_rng(m + split)
+    W = sparse_matrix(rng, m, n, .6)
+    W[:, 5] = np.where(np.arange(m) % 2, 0, 2.0 ** -30)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    for c, e in ((1, 39), (2, 40), (3, 41), (4, 70), (5, 103), (6, 104), (7, 105), (8, 115), (C - 1, 60)):
+        X[rng.integers(n), c] = np.ldexp(np.float32(1.37), e)
+        X[0, c] = np.ldexp(np.float32(-1.21), e)
+    X[:, 9] = np.ldexp(X[:, 9], 112)                 # sums near 2^117
+    X[:, 10] = np.ldexp(X[:, 10], 90)                # values that fit, sums that do not
+    X[::2, 11] = np.ldexp(X[::2, 11], -140)          # both ends of the range
+    X[1::2, 11] = np.ldexp(X[1::2, 11], 100)
+    X[5, 12] = -3.4028235e38                         # the lowest value, times 2^-30 or nothing
+    X[n - 1, 13], X[3, 13], X[n // 2, 14], X[9, 14] = np.inf, 1e30, np.nan, 1e-42
+    X[:, 15] = np.inf
+    X[2, 16], X[n - 2, 16] = np.inf, -np.inf
+    E = datagen.encode_dense(W)
+    Y, Yo = planes_matmul(ctx, E, X, None, split=split), oracle.matmul(as_oracle(E), X, None)
+    assert np.array_equal(np.isnan(Y), np.isnan(Yo)) and np.array_equal(Y[np.isinf(Yo)], Yo[np.isinf(Yo)])
+    for c in range(C):
+        fin = np.isfinite(Yo[:, c])
+        ref = W[fin].astype(np.float64) @ np.where(np.isfinite(X[:, c]), X[:, c], 0).astype(np.float64)
+        assert np.abs(Y[fin, c] - ref).max(initial=0.0) <= TOL * np.abs(ref).max(initial=0.0), c
+
+
+@pytest.mark.parametrize("value,most", [(1e-38, 1.5), (1e25, 1.5), (1e35, 10.0), (np.inf, 10.0), (np.nan, 10.0)])
+def test_planes_time_with_such_values(ctx, value, most):
+    """One value in every column: tiny and large ones cost nothing, those that the planes do not hold two or three passes more (not a sum
+    over the nonzeros per output, a hundred times as long)."""
+    rng = np.random.default_rng(6)
+    m, n, C = 2048, 2048, 128
+    W = sparse_matrix(rng, m, n, .6)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    E = datagen.encode_dense(W)
+    with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, m, n, E.r, RBM)
+        dX, dY = ctx.array(X), ctx.empty((m, C))
+
+        def shortest():
+            ms = []
+            for _ in range(5):
+                ctx.timer_begin()
+                for _ in range(10):
+                    ctx.matmul(dE, dX, C, None, dY)
+                ms.append(ctx.timer_end())
+            return min(ms)
+        shortest()
+        before = shortest()
+        X[rng.integers(0, n, C), np.arange(C)] = value
+        dX.upload(X)
+        assert shortest() <= most * before
+    for a in (dX, dY, dE):
+        a.free()
+
+
 def test_planes_left_out(ctx):
-    """Weights without room for three planes, rows whose columns do not ascend: the handle does without, whatever is asked."""
+    """Weights without room for three planes, stored zeros, rows whose columns do not ascend: the handle does without, whatever is asked."""
     rng = np.random.default_rng(3)
     W = sparse_matrix(rng, 100, 200, .5)
     X = rng.standard_normal((200, 8)).astype(np.float32)
     cases = []
-    for value in (1e-35, 1e37, np.inf, np.nan):
+    for value in (1e-35, 1e12, 1e37, np.inf, np.nan):
         V = W.copy()
         V[3, 5] = value
         cases.append(datagen.encode_dense(V))
     E = datagen.encode_dense(W)
     c = int(E.nnz[9])
     E.Wd[9, :c], E.idx[9, :c] = E.Wd[9, :c][::-1].copy(), E.idx[9, :c][::-1].copy()
+    cases.append(E)
+    E = datagen.encode_dense(W)
+    E.Wd[7, 1] = 0                                   # times an infinity in X: NaN
     cases.append(E)
     for E in cases:
         with ctx.tuning(SPARSEOPS_MATMUL_PLANES="1"):
