@@ -24,8 +24,11 @@
 // tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 6.8 and 4.6 us; 256 x 1136 x 36, 69 %, 7.5 and 5.4; 45 x 757 x 224, 75 %
 // (shared gather) 5.4 and 4.6.  Every slab reads the copy of the matrix again, so large ones stay there.
 //
-// Sums, zero weights and values that are not finite: as there.
+// Sums, zero weights and values that are not finite: as there.  With an infinity in one column of X / in each, us: 2847 x 1952 x 8 16 / 21 (the quad-union
+// kernel 35 / 52), 1067 x 900 x 28, 60 %, 11 / 27 (12 / 36), 256 x 1136 x 36 8 / 15 (10 / 28), 2000 x 1500 x 3, 50 %, 13 / 13 (row kernel 12); output
+// by output, a whole wave for each, it took 24 / 90, 13 / 116, 10 / 80 and 18 / 42.
 #include "so_internal.h"
+#include "exact_outputs.h"
 
 #include <algorithm>
 #include <cmath>
@@ -237,22 +240,29 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     }
     if (wk != 0 || quad >= a.nquads) return;
     const uint32_t row = quad * 4u + (lane >> 4);
+    const auto live = [&](int k) { return row < a.m && col + k < cols; };
+    // A zero weight times a value of X that is not finite: outputs that came out as NaN are computed again from the
+    // rows' own nonzeros, a group of four columns of all four rows at a time.
+    uint32_t lost = 0;                                               // a bit per group
 #pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const bool live = row < a.m && col + k < cols;
-        // A zero weight times a value of X that is not finite: an output that came out as NaN is computed again from the
-        // row's own nonzeros, by the whole wave.
-        for (uint64_t left = __ballot(live && __builtin_isnan(out[k])); left != 0u; left &= left - 1u) {
-            const uint32_t l = (uint32_t)__builtin_ctzll(left), rr = __builtin_amdgcn_readlane(row, l), cc = c0 + __builtin_amdgcn_readlane(col, l) + k;
-            const uint32_t cnt = a.nnz[rr];
-            float sum = 0.0f;
-            for (uint32_t e = lane; e < cnt; e += 64u) sum = __builtin_fmaf(a.Wd[(size_t)rr * a.r + e], a.X[(size_t)a.idx[(size_t)rr * a.r + e] * a.C + cc], sum);
+    for (int k = 0; k < R; ++k) lost |= live(k) && __builtin_isnan(out[k]) ? 1u << (col >> 2) : 0u;
+    if (__builtin_expect(__ballot(lost != 0u) != 0u, 0)) {
+#pragma unroll 1
+        for (uint32_t g = 0; g < GROUPS; ++g) {
+            if (__ballot(lost >> g & 1u) == 0u) continue;
+            const uint32_t at = c0 + g * 4u, first = min(at, max(a.C, 4u) - 4u);               // four columns that exist, or all there are
+            const so_f32x4 e = a.C >= 4u ? exact_outputs(a, row, first, lane & 15u) : exact_outputs<false>(a, row, first, lane & 15u);
 #pragma unroll
-            for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-            if (lane == l) out[k] = sum;
+            for (int k = 0; k < R; ++k) {
+                const uint32_t v = c0 + col + k - first;
+                const float again = v == 0u ? e[0] : v == 1u ? e[1] : v == 2u ? e[2] : e[3];
+                if (col >> 2 == g && live(k) && __builtin_isnan(out[k])) out[k] = again;
+            }
         }
-        if (live) a.Y[(size_t)row * a.C + c0 + col + k] = so_epilogue<ACT>(out[k] + (a.bias ? a.bias[row] : 0.0f));
     }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+        if (live(k)) a.Y[(size_t)row * a.C + c0 + col + k] = so_epilogue<ACT>(out[k] + (a.bias ? a.bias[row] : 0.0f));
 }
 
 // 16-byte groups of a row of X in LDS for C <= 32 columns.

@@ -41,6 +41,7 @@
 // row's own nonzeros (`exact_outputs`): 2048 x 2048 x 64, 80 % sparse, 10.6 us, 18 with one column of NaNs in X, 125 with
 // nothing else (91 and 384 with a lane per output).
 #include "so_internal.h"
+#include "exact_outputs.h"
 #include "lds_sync.h"
 
 #include <algorithm>
@@ -72,37 +73,6 @@ struct QuadArgs {
     const uint32_t *idx, *nnz;
     uint32_t r;
 };
-
-// The outputs of columns col .. col + 3 from the row's own nonzeros, added up by the 16 lanes that share the row (lane
-// `sub` every 16th, eight of them requested at a time), in an order that depends on the row's length alone.
-__device__ __forceinline__ f32x4 exact_outputs(const QuadArgs &a, uint32_t row, uint32_t col, uint32_t sub)
-{
-    constexpr uint32_t AHEAD = 8;
-    const uint32_t cnt = row < a.m ? a.nnz[row] : 0u;
-    const float *w = a.Wd + (size_t)row * a.r;
-    const uint32_t *ix = a.idx + (size_t)row * a.r;
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t k = sub; k < cnt; k += 16u * AHEAD) {
-        float wk[AHEAD];
-        f32x4 x[AHEAD];
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u) {
-            const uint32_t at = min(k + 16u * u, cnt - 1u);
-            wk[u] = w[at];
-            x[u] = *reinterpret_cast<const f32x4u *>(a.X + (size_t)ix[at] * a.C + col);
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u)
-            if (k + 16u * u < cnt)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) sum[v] = __builtin_fmaf(wk[u], x[u][v], sum[v]);
-    }
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) sum[v] += __shfl_xor(sum[v], off, 64);
-    return sum;
-}
 
 // ---- the chunk loop ---------------------------------------------------------------------------------
 //

@@ -71,6 +71,32 @@ def test_values_that_are_not_finite(ctx, oracle, C):
     assert np.abs(Y[fin] - want[fin]).max() <= TOL * np.abs(want[fin]).max()
 
 
+@pytest.mark.parametrize("m,n,C,sp", [(2847, 1952, 8, .6), (1067, 900, 28, .6), (256, 1136, 36, .7), (2000, 1500, 3, .5)])
+def test_time_with_values_that_are_not_finite(ctx, m, n, C, sp):
+    """An infinity in every column: groups of four columns of four rows are computed again at a time, not output by output."""
+    rng = np.random.default_rng(3)
+    E = datagen.encode_dense(sparse_matrix(rng, m, n, sp))
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    dE, dX, dY = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM), ctx.array(X), ctx.empty((m, C))
+
+    def shortest():
+        ms = []
+        for _ in range(5):
+            ctx.timer_begin()
+            for _ in range(10):
+                ctx.matmul(dE, dX, C, None, dY)
+            ms.append(ctx.timer_end())
+        return min(ms)
+    with ctx.tuning(SPARSEOPS_MATMUL_NARROW="1"):
+        shortest()
+        before = shortest()
+        X[rng.integers(0, n, C), np.arange(C)] = np.inf
+        dX.upload(X)
+        assert shortest() <= 6.5 * before
+    for a in (dX, dY, dE):
+        a.free()
+
+
 @pytest.mark.parametrize("C,want", [(65535 * 16, "narrow"), (65535 * 16 + 4, None), (2 ** 20, None)])
 def test_very_wide(ctx, C, want):
     """A grid has at most 65 535 workgroups in y: slabs of 16 columns, all that fit beside more than 1280 rows of X, end at 1 048 560."""
