@@ -71,6 +71,22 @@ def test_values_that_are_not_finite(ctx, oracle, C):
     assert np.abs(Y[fin] - want[fin]).max() <= TOL * np.abs(want[fin]).max()
 
 
+@pytest.mark.parametrize("C,n", [(36, 300), (100, 300), (36, 1300), (100, 1300), (64, 2560)])
+def test_values_that_are_not_finite_in_slabs(ctx, oracle, C, n):
+    """The same with more than 32 columns: slabs of 16 or 32 where n rows of 32 columns fit into LDS, else of 16, the last of them partial;
+    in its last column, in one before it and in another slab."""
+    rng = np.random.default_rng(C)
+    W = sparse_matrix(rng, 203, n, .8)
+    E = datagen.encode_dense(W)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    X[7, C - 1], X[9, C - 3], X[n - 1, C // 2], X[100, 1] = np.inf, -np.inf, np.nan, np.inf
+    b = rng.standard_normal(203).astype(np.float32)
+    Y, want = narrow_matmul(ctx, E, X, b), oracle.matmul(as_oracle(E), X, b)
+    fin = np.isfinite(want)
+    assert np.array_equal(Y[~fin], want[~fin], equal_nan=True) and fin.any() and not fin.all()
+    assert np.abs(Y[fin] - want[fin]).max() <= TOL * np.abs(want[fin]).max()
+
+
 @pytest.mark.parametrize("m,n,C,sp", [(2847, 1952, 8, .6), (1067, 900, 28, .6), (256, 1136, 36, .7), (2000, 1500, 3, .5)])
 def test_time_with_values_that_are_not_finite(ctx, m, n, C, sp):
     """An infinity in every column: groups of four columns of four rows are computed again at a time, not output by output."""
