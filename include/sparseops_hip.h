@@ -135,7 +135,8 @@ so_status so_stage_in(so_ctx *ctx, void *dst, const void *src, size_t bytes, voi
 so_status so_stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes);
 /* The same with a transpose on the way: dDst[cols][stride] from the host's src[rows][cols], zeros in the places from `rows` to
  * `stride` of its rows; the host's dst[cols][rows] from dSrc[rows][stride].  *done = 0, with nothing queued, for arrays that
- * the staging memory does not hold (about 4 MB in, 1 MB out).  No counterpart in the reference. */
+ * the staging memory does not hold (4 MB in, rows counted in whole groups of four; 1 MB out), and on the way in for more than 4096 rows (1024 per
+ * column up to four), where staging and a transpose behind it are as fast.  No counterpart in the reference. */
 so_status so_stage_in_transposed(so_ctx *ctx, float *dDst, uint32_t stride, const float *src, uint32_t rows, uint32_t cols, int *done);
 so_status so_stage_out_transposed(so_ctx *ctx, float *dst, const float *dSrc, uint32_t stride, uint32_t rows, uint32_t cols, int *done);
 so_status so_d2d(so_ctx *ctx, void *dst, const void *src, size_t bytes);

@@ -110,3 +110,21 @@ def test_transposed_there_and_back(ctx, rows, cols, stride):
     assert ctx.lib.so_stage_in_transposed(ctx.h, d.ptr, rows - 1, None, rows, cols, ct.byref(done)) == hipabi.SO_ERR_INVALID
     assert ctx.lib.so_stage_out_transposed(ctx.h, None, d.ptr, stride, cols, rows, ct.byref(done)) == hipabi.SO_ERR_INVALID
     d.free()
+
+
+@pytest.mark.parametrize("rows,cols,taken", [(4000, 64, True), (4096, 252, True), (4096, 253, False), (4097, 64, False), (1024, 1, True), (1025, 1, False),
+                                             (3072, 3, True), (3073, 3, False), (4, 262128, True), (4, 262129, False)])
+def test_transposed_many_rows(ctx, rows, cols, taken):
+    """The rule's edges: 16 bytes per four columns and row, 255 bytes on top, in 4 MB; 1024 rows per column up to 4096."""
+    assert taken == ((cols + 3) // 4 * 16 * rows + 255 <= IN and rows <= 1024 * min(cols, 4))
+    a = np.random.default_rng(rows + cols).integers(0, 1 << 32, (rows, cols), dtype=np.uint32)
+    d, done = ctx.array(np.full(cols * (rows + 4) + 8, 7.0, np.float32)), ct.c_int(-1)
+    ctx._ck(ctx.lib.so_stage_in_transposed(ctx.h, d.ptr, rows + 4, a.ctypes.data_as(ct.c_void_p), rows, cols, ct.byref(done)))
+    got = d.download()
+    assert done.value == int(taken) and (got[cols * (rows + 4):] == 7.0).all()
+    if taken:
+        got = got[:cols * (rows + 4)].view(np.uint32).reshape(cols, rows + 4)
+        assert np.array_equal(got[:, :rows], a.T) and not got[:, rows:].any()
+    else:
+        assert (got == 7.0).all()
+    d.free()
