@@ -314,22 +314,9 @@ void so_stage_in_transposed_kernel(float *dst, uint32_t stride, const float *src
         if (c0 + c < cols && r0 + r < stride) dst[(size_t)(c0 + c) * stride + r0 + r] = tile[c][r];
 }
 
-// The last workgroup to finish tells the host: `turn`, and beside it the word of the bounded waits.  `cols` != 0: dst is the transpose
-// of src, whose rows of `cols` words lie `pitch` apart.
-__global__ __launch_bounds__(256)
-void so_stage_out_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t cols, uint32_t pitch, uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
+// The end of a way out: the last workgroup to finish tells the host: `turn`, and beside it the word of the bounded waits.
+__device__ __forceinline__ void tell_host(uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
 {
-    const uint32_t quads = words / 4u, stride = gridDim.x * 256u;
-    if (cols != 0u) {
-        const uint32_t rows = words / cols;
-        auto word = [&](uint32_t e) { const uint32_t c = e / rows; return src[(size_t)(e - c * rows) * pitch + c]; };
-        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride)
-            reinterpret_cast<uint4 *>(dst)[i] = make_uint4(word(4u * i), word(4u * i + 1u), word(4u * i + 2u), word(4u * i + 3u));
-        if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = word(quads * 4u + threadIdx.x);
-    } else {
-        for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
-        if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = src[quads * 4u + threadIdx.x];
-    }
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x != 0) return;
@@ -340,6 +327,28 @@ void so_stage_out_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uin
     flag[1] = *gave_up;
     __threadfence_system();
     __hip_atomic_store(flag, turn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// (Kernels of their own: one kernel for both, on a branch, cost each ellpack_matvec from host arrays 0.2 to 0.4 us of 18 to 20.)
+__global__ __launch_bounds__(256)
+void so_stage_out_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
+{
+    const uint32_t quads = words / 4u, stride = gridDim.x * 256u;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride) reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = src[quads * 4u + threadIdx.x];
+    tell_host(done, gave_up, flag, turn);
+}
+
+// dst is the transpose of src, whose rows of `cols` words lie `pitch` apart.
+__global__ __launch_bounds__(256)
+void so_stage_out_transposed_kernel(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t cols, uint32_t pitch, uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
+{
+    const uint32_t quads = words / 4u, stride = gridDim.x * 256u, rows = words / cols;
+    auto word = [&](uint32_t e) { const uint32_t c = e / rows; return src[(size_t)(e - c * rows) * pitch + c]; };
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < quads; i += stride)
+        reinterpret_cast<uint4 *>(dst)[i] = make_uint4(word(4u * i), word(4u * i + 1u), word(4u * i + 2u), word(4u * i + 3u));
+    if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = word(quads * 4u + threadIdx.x);
+    tell_host(done, gave_up, flag, turn);
 }
 
 // The staging memory, made on first use.  False where there is none: the callers then copy as so_h2d and so_d2h do.
@@ -403,8 +412,12 @@ static so_status stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes
     volatile uint32_t *const flag = (volatile uint32_t *)(ctx->h_stage + kStageFlag);
     const uint32_t turn = ++ctx->stage_turn;
     const uint32_t blocks = (uint32_t)std::min<size_t>((bytes + 8191) / 8192, 128);
-    so_stage_out_kernel<<<blocks, 256, 0, ctx->stream>>>((uint32_t *)(ctx->h_stage + kStageIn), (const uint32_t *)src, (uint32_t)(bytes / 4), cols, pitch,
-                                                         ctx->d_stage_done, ctx->d_wait_gave_up, (uint32_t *)flag, turn);
+    uint32_t *const to = (uint32_t *)(ctx->h_stage + kStageIn);
+    if (cols == 0)
+        so_stage_out_kernel<<<blocks, 256, 0, ctx->stream>>>(to, (const uint32_t *)src, (uint32_t)(bytes / 4), ctx->d_stage_done, ctx->d_wait_gave_up, (uint32_t *)flag, turn);
+    else
+        so_stage_out_transposed_kernel<<<blocks, 256, 0, ctx->stream>>>(to, (const uint32_t *)src, (uint32_t)(bytes / 4), cols, pitch,
+                                                                        ctx->d_stage_done, ctx->d_wait_gave_up, (uint32_t *)flag, turn);
     SO_LAUNCH_CHECK();
     // The word comes when the stream's work is done; a stream that has ended without it, or failed, ends the wait as well.
     for (uint32_t spin = 1; *flag != turn; ++spin) {
