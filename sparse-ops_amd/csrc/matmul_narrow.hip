@@ -300,9 +300,10 @@ bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C
 }
 
 // Up to 32 columns the narrowest slab that holds them, beyond (whole groups of four only: the others' copies take up to twice as
-// long) slabs of 16 or 32 columns (blockIdx.y), whichever is estimated faster; as few quads per workgroup as give no more workgroups than compute units.  The estimate -- a workgroup's start and its
-// copy of X, the chunks of a wave, the bytes that slabs share -- was fitted to 260 launches of 10..4096 rows, 512..4096 columns, 1..32 dense columns, 50-95 %
-// sparse, one handle again and again: 3 % off on average, 11 % at most.
+// long) slabs of 16 or 32 columns (blockIdx.y), whichever is estimated faster; as few quads per workgroup as give no more workgroups than compute units.  The estimate -- the launch, a workgroup's
+// start and its copy of X, the chunks of a wave, the bytes that slabs share -- was fitted to 696 launches of 10..4096 rows, 512..4096 columns, 1..64 dense
+// columns, 50-95 % sparse on three cards, one handle again and again: 0.7 % too low on average, 5 % off (standard deviation; the same handle differs by
+// as much from one allocation to the next), 20 % at most.
 so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
@@ -314,8 +315,8 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
         uint32_t ql = 0;
         while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
         const double rounds = so_ceil_div((uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs, (uint64_t)ctx->compute_units);
-        const double copy = 1e-4 * E->n * (slabs > 1 ? 4.6 * groups : C) * (C % 4u ? 0.77 : 0.65), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
-        const double us = 2.5 + rounds * (1.0 + (groups == 8u ? 0.3 : 0.0) + copy + chunks * (0.079 + 0.0185 * groups)) + 1.1e-5 * Q.total_chunks;
+        const double copy = 1e-4 * E->n * (slabs > 1 ? 4.6 * groups : C) * (C % 4u ? 0.6 : 0.45), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
+        const double us = 3.0 + rounds * (1.0 + (groups == 8u ? 0.55 : 0.0) + copy + chunks * (0.077 + 0.021 * groups)) + 0.84e-5 * Q.total_chunks;
         if (us < best.us) best = so_narrow_plan{ql, groups, slabs, us};
     }
     return best;
