@@ -4,10 +4,11 @@
 // A float is the exact sum of three bf16 numbers, hi + mid + lo (8 significant bits each, rounded to nearest, the next one
 // holding what the last left).  The matrix is kept as three bf16 planes, zeros included, in the order in which
 // v_mfma_f32_32x32x16_bf16 reads its operand; X is split on its way into LDS.  Of the nine products of planes the six
-// whose size is 2^-16 of the whole or more are added up: the other three are below 2^-26, a quarter of what fp32 rounds
-// away.  hi * hi goes to one set of accumulators and the five small products to another, so that the large sums are
-// rounded once per 16 columns, and every 512 columns they are added to totals in LDS; a bf16 MFMA adds its 16 products
-// with at most the error of a chain of fmaf.
+// whose size may be 2^-17 of the whole or more are added up.  What the other three leave out is at most 2^-24 of the product (where both
+// factors are near 1 + 2^-8 - 2^-17 times a power of two), as much as one fp32 rounding, and 2^-27.5 in the 2-norm over all mantissas.
+// hi * hi goes to one set of accumulators and the five small products (2^-7 of it at most) to another, so that the large sums are
+// rounded once per 16 columns, and every 512 columns they are added to totals in LDS.  So long sums are closer than a chain of fmaf, but an output of a
+// single nonzero may be 1.7 x 2^-24 off instead of 2^-24.
 //
 // Why: an MFMA of 32 x 32 x 16 takes a SIMD 32 clocks, so six of them do 85 fp32 multiply-adds per clock on zeros and
 // nonzeros alike.  The quad-union kernel (matmul_quad.hip) does 32 per clock on the union of four rows, which is 59 % of

@@ -4,9 +4,10 @@ every number of workgroups per tile.
 
 Bound: max|y - ref| <= 1e-5 * max|ref| against the in-order oracle and the fp64 product, as for the layout's other kernels
 (tests/test_gpu_matmul_rbm.py).  Beside it the error in the 2-norm: with x = hi + mid + lo exactly, the products left out
-are below 2^-26 of |w x|, and a sum that is rounded once per 16 terms over at most 32 roundings, five times that often for
-parts 2^-9 as large, once per 512 terms and once per workgroup, each time by at most 2^-24 of a partial sum, is off by less than
-(sqrt(32 + n / 512 + 16) + 1) * 2^-24 of the 2-norm when roundings are independent: 2.5 times that is asked."""
+are 2^-27.5 of |w x| in the 2-norm (2^-24 at most), and a sum that is rounded once per 16 terms over at most 32 roundings, five times that often for
+parts 2^-7 as large, once per 512 terms and once per workgroup, each time by at most 2^-24 of a partial sum, is off by less than
+(sqrt(32 + n / 512 + 16) + 1) * 2^-24 of the 2-norm when roundings are independent: 2.5 times that is asked.  Output by output, and where roundings are not
+independent: test_planes_worst_mantissas and test_planes_one_step_of_the_matrix_cores."""
 
 import numpy as np
 import pytest
@@ -58,6 +59,43 @@ def test_planes_shapes(ctx, oracle, m, n, C, sp, split, act):
     assert rel_err(Y, ref) <= TOL
     assert rel_err(Y, oracle.matmul(as_oracle(E), X, b, act)) <= TOL
     assert np.linalg.norm(Y - ref) <= 2.5 * (np.sqrt(48 + n / 512) + 1) * 2.0 ** -24 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [1, 16, 100, 512, 2048, 4100])
+@pytest.mark.parametrize("split", [1, 3])
+def test_planes_worst_mantissas(ctx, n, split):
+    """Weights and X that the planes split worst: every product loses 0.99 * 2^-24 of itself, all of one sign, and every sum grows.  Output by output,
+    in units of 2^-24 of |w||x|: that, the small products' sums (2^-7 as large, 5 n / 16 additions), 32 additions to the large sums at
+    most, n / 512 to the totals, and one per part and for the small sums; each by 1."""
+    rng = np.random.default_rng(n)
+    m, C, worst = 130, 66, np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    W = np.where(rng.random((m, n)) < .6, worst, 0).astype(np.float32)
+    W[0], W[1, :-1] = worst, 0
+    W[1, -1] = worst
+    X = np.full((n, C), worst, np.float32)
+    X[:, 1::2] *= -1
+    W[2] *= np.ldexp(np.float32(1), rng.integers(-20, 20, n).astype(np.int32))
+    Y, ref = planes_matmul(ctx, datagen.encode_dense(W), X, None, split=split), W.astype(np.float64) @ X.astype(np.float64)
+    bound = 1 + 5 * n / 16 / 128 + min(32, n / 16) + n / 512 + split + 1
+    assert (np.abs(Y - ref) <= bound * 2.0 ** -24 * (np.abs(W).astype(np.float64) @ np.abs(X).astype(np.float64))).all()
+
+
+@pytest.mark.parametrize("spread", [0, 8, 30, 60])
+def test_planes_one_step_of_the_matrix_cores(ctx, spread):
+    """A v_mfma_f32_32x32x16_bf16 adds 16 products with at most the error of a chain of fmaf, 16 * 2^-24 of sum |w x|: factors of eight significant
+    bits, whose other planes are zeros, of very different sizes and both signs, and large ones that cancel."""
+    rng = np.random.default_rng(spread)
+    m, n, C = 256, 16, 128
+
+    def eight_bits(shape, spread):
+        v = rng.integers(128, 256, shape).astype(np.float32) * rng.choice([-1, 1], shape)
+        return np.ldexp(v, rng.integers(-spread, spread + 1, shape) - 7).astype(np.float32)
+    W, X = eight_bits((m, n), min(spread, 30)), eight_bits((n, C), spread)
+    W[:64, 8:] = -W[:64, :8]
+    X[8:, :32] = X[:8, :32] * rng.choice([1, 1, 1, 0, 0.5], (8, 32))
+    assert not (W.view(np.uint32) & 0xffff).any() and not (X.view(np.uint32) & 0xffff).any()
+    Y, ref = planes_matmul(ctx, datagen.encode_dense(W), X, None, split=1), W.astype(np.float64) @ X.astype(np.float64)
+    assert (np.abs(Y - ref) <= 16 * 2.0 ** -24 * (np.abs(W).astype(np.float64) @ np.abs(X).astype(np.float64))).all()
 
 
 @pytest.mark.parametrize("act", ["sigmoid", "tanh"])
