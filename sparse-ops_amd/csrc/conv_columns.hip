@@ -14,8 +14,9 @@
 // two quads of entries ahead of the multiply-adds.  Workgroups shrink to 8 or 4 waves where that spreads the launch
 // over more compute units.
 //
-// What bounds it: a wave's own chain.  An entry takes a wave on a SIMD of its own 28 clocks (add, read and multiply-add
-// each wait for the one before; four at a time, the adds between the multiply-adds), so the chains of 922 of a
+// What bounds it: the latency of a wave's LDS reads.  An entry takes a wave on a SIMD of its own 28 clocks, a step of four 112: each step begins by waiting
+// for the quad that was requested at the end of the step before last, so that a read's round trip has one step's eight vector instructions and four
+// reads, about 50 clocks to issue, to hide in.  (The chain of multiply-adds itself would allow 9 clocks an entry.)  The chains of 922 of a
 // ResNet-18-shaped 7 x 7 x 512 layer at 80 % are 11 of its 16 us; the rest is launch, first loads and the window's copy.
 #include "so_internal.h"
 #include "conv_internal.h"
