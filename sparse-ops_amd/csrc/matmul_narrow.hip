@@ -16,13 +16,13 @@
 // x 8, 50 % dense: 65 MB, 16 us, 4.1 TB/s) and, from 17 columns on, bank conflicts of the 128-byte rows.  Copying X in
 // two rounds of eight loads cost 1 to 2 us more, and 16-byte loads across the ends of rows of no multiple of four columns 1.5.
 //
-// Measured, one handle launched again and again, the quad-union kernel and this one: 2847 x 1952 x 8, 61 % sparse, 14.7 and 7.7 us
-// (17.5 MB of copy); 4096 x 2048 x 16, 50 %, 17.6 and 11.5; 317 x 930 x 11, 74 %, 6.8 and 4.8; 10 x 512 x 4, 80 %, 4.5 (row
-// kernel) and 3.8.  Error against 64 bits: 0.67 of the replaced kernels' on average over 120 launches.
+// Measured, one handle launched again and again, the quad-union kernel and this one: 2847 x 1952 x 8, 61 % sparse, 14.3 and 7.8 us
+// (17.5 MB of copy); 4096 x 2048 x 16, 50 %, 16.0 and 11.3; 317 x 930 x 11, 74 %, 7.0 and 5.0; 10 x 512 x 4, 80 %, 5.0 (row
+// kernel) and 4.3 (on another card 4.5 and 3.8).  Error against 64 bits: 0.67 of the replaced kernels' on average over 120 launches.
 //
 // More columns, in slabs of 16 or 32: pays where a matrix is so small that the quad-union kernel's exchange of partial tiles and its
-// tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 6.8 and 4.6 us; 256 x 1136 x 36, 69 %, 7.5 and 5.4; 45 x 757 x 224, 75 %
-// (shared gather) 5.4 and 4.6.  Every slab reads the copy of the matrix again, so large ones stay there.
+// tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 7.0 and 5.4 us; 256 x 1136 x 36, 69 %, 7.6 and 5.8; 45 x 757 x 224, 75 %
+// (shared gather) 6.1 and 5.4.  Every slab reads the copy of the matrix again, so large ones stay there.
 //
 // Sums, zero weights and values that are not finite: as there.  With an infinity in one column of X / in each, us: 2847 x 1952 x 8 16 / 21 (the quad-union
 // kernel 35 / 52), 1067 x 900 x 28, 60 %, 11 / 27 (12 / 36), 256 x 1136 x 36 8 / 15 (10 / 28), 2000 x 1500 x 3, 50 %, 13 / 13 (row kernel 12); output

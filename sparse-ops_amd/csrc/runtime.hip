@@ -269,8 +269,8 @@ extern "C" so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t byte
 // Bound by latencies in a row: per kernel the launch, the link's 2 to 3 us and 256 KB at about 50 GB/s.  A model's input and output
 // are [batch][features] on the host and [features][batch] in memory, so their kernels transpose (and pad) on the way, in
 // pieces of columns that double from 128 KB on, instead of a transpose and a padding kernel each behind the copies: the same MLP
-// 141 -> 123 us (at batch 2 / 4 / 16 54 / 67 / 69 -> 44 / 45 / 60, its narrow kernel included), 100-300-20 at batch 7 27 -> 20, the ResNet-18-shaped
-// stack on 12 images of 96 x 96 246 -> 222.
+// 139 to 142 -> 129 to 135 us (at batch 2 / 4 / 16 54 / 67 / 69 -> 45 / 45 / 60, its narrow kernel included), 100-300-20 at batch 7 27 -> 20, the
+// ResNet-18-shaped stack on 12 images of 96 x 96 490 -> 470.  One image (or sample) is the same in either order and goes as before.
 constexpr size_t kStageIn = 4u << 20, kStageOut = 1u << 20, kStagePiece = 256u << 10, kStagePieceFirst = 128u << 10, kStagePieceMost = 1u << 20;
 constexpr size_t kStageFlag = kStageIn + kStageOut;      // {turn, waits given up} behind the two areas
 

@@ -32,7 +32,7 @@ const float *stage_operands(so_ctx *ctx, const float *X, std::size_t xbytes, con
 namespace sparseops {
 // Device layouts worth keeping for Y = E * X with C dense columns.  Large, reasonably filled
 // matrices and wide X pay for a second copy: the K-tiled one (LDS-staged kernel, the reference's
-// bits) or, with `fast`, the RBM layout's two (the fastest kernels; sums in another order,
+// bits) or, with `fast`, the RBM layout's copies (the fastest kernels; sums in another order,
 // accurate to fp32 round-off).
 int matmul_layouts(const Ellpack &E, uint32_t C, bool fast)
 {
@@ -44,7 +44,7 @@ int matmul_layouts(const Ellpack &E, uint32_t C, bool fast)
     // (4096 x 784 x 256 at 90 %: 12.0 us against 15.2) and, from the 4 columns it needs, of the row kernel, which
     // fetches a line of X per nonzero however few of its columns there are; up to three columns go to so_matvec's kernel.
     // At any C: the batch may grow after the load.  MLP 784-4096-4096-4096-10 host to host, batch 1 / 2 / 3 / 4 / 16 / 48:
-    // 117 / 117 / 118 / 116 / 118 / 125 us with ROW alone, 39 / 57 / 66 / 67 / 69 / 75 now.
+    // 117 / 117 / 118 / 116 / 118 / 125 us with ROW alone, 37 / 45 / 46 / 45 / 60 / 68 now.
     if (fast) return SO_LAYOUT_ROW | SO_LAYOUT_RBM;
     if (C < 64) return SO_LAYOUT_ROW;
     return C % 4 == 0 ? (SO_LAYOUT_ROW | SO_LAYOUT_TILED) : SO_LAYOUT_ROW;
