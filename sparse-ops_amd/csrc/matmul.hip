@@ -334,7 +334,7 @@ RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t
 constexpr double kPlanesBelow = 0.9;
 
 // The narrow kernel where it is estimated a little below the others.  Of 447 drawn launches where it is this rule that decides, against the row, shared-gather or quad
-// kernel, it takes the narrow one in 356, which was the slower one in three of them, by 1.1 to 2.3 % (with an estimate 9 % lower and a limit of 0.88:
+// kernel, it takes the narrow one in 355, which was the slower one in three of them, by 1.1 to 2.3 % (with an estimate 9 % lower and a limit of 0.88:
 // 338, four, by 1.1 to 9.2 %).  Us, the others and the narrow one, one handle launched again and again: quad 2847 x 1952 x 8 at 61 % sparse 14.7 / 7.8, 4096 x 2048 x 16 at 90 / 50 %
 // 10.9 / 7.8 and 17.6 / 11.5, 1152 x 546 x 18 at 54 % 7.2 / 5.4, 317 x 930 x 11 at 74 % 6.8 / 4.8, 2745 x 1203 x 30 at 56 % 11.7 / 11.0;
 // shared-gather 1145 columns, 21 rows, 5 dense 6.6 / 4.1, 627, 41, 28 4.8 / 5.5; row 1595, 981, 10 7.2 / 5.4, 1067, 3000, 28 5.1 / 6.7.  In place

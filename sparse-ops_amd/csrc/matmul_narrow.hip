@@ -303,7 +303,9 @@ bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C
 // long) slabs of 16 or 32 columns (blockIdx.y), whichever is estimated faster; as few quads per workgroup as give no more workgroups than compute units.  The estimate -- the launch, a workgroup's
 // start and its copy of X, the chunks of a wave, the bytes that slabs share -- was fitted to 696 launches of 10..4096 rows, 512..4096 columns, 1..64 dense
 // columns, 50-95 % sparse on three cards, one handle again and again: 0.7 % too low on average, 5 % off (standard deviation; the same handle differs by
-// as much from one allocation to the next), 20 % at most.
+// as much from one allocation to the next), 20 % at most.  Slabs also to 320 launches of up to 1500 rows and 4800 dense columns, 10 % off: once X is more than an XCD's
+// 4 MB of L2, the 64 bytes of a row that a slab of 16 takes cost a whole line from beyond it (4 x 1792 x 3780, 27 MB, 14.2 us, shared gather
+// 7.6; 12 x 2172 x 1860 17.7, quad-union 8.5); those of 32 columns take whole lines.
 so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
@@ -316,7 +318,8 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
         while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
         const double rounds = so_ceil_div((uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs, (uint64_t)ctx->compute_units);
         const double copy = 1e-4 * E->n * (slabs > 1 ? 4.6 * groups : C) * (C % 4u ? 0.6 : 0.45), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
-        const double us = 3.0 + rounds * (1.0 + (groups == 8u ? 0.55 : 0.0) + copy + chunks * (0.077 + 0.021 * groups)) + 0.84e-5 * Q.total_chunks;
+        const double megabytes = 4.0 * E->n * C / (1u << 20), far = slabs > 1 && groups == 4u && megabytes > 4.0 ? 0.6 * megabytes : 0.0;
+        const double us = 3.0 + rounds * (1.0 + (slabs > 1 ? 0.2 : 0.0) + (groups == 8u ? 0.55 : 0.0) + copy + chunks * (0.077 + 0.021 * groups)) + 0.84e-5 * Q.total_chunks + far;
         if (us < best.us) best = so_narrow_plan{ql, groups, slabs, us};
     }
     return best;

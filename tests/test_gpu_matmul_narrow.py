@@ -151,7 +151,7 @@ def test_rows_in_any_order(ctx, oracle):
 
 @pytest.mark.parametrize("m,n,C,sp,want", [(2000, 1500, 8, .6, True), (2000, 1500, 33, .6, False), (2000, 1500, 64, .6, False), (84, 692, 148, .5, True), (84, 692, 149, .5, False), (2000, 2600, 16, .6, False), (2000, 600, 30, .97, False),
                                            (2000, 1500, 3, .5, True), (300, 1500, 3, .5, False), (2000, 1500, 1, .5, False),
-                                           (2126, 531, 17, .85, False)])
+                                           (2126, 531, 17, .85, False), (4, 1792, 3780, .8, False), (12, 2172, 1860, .7, False)])
 def test_which_calls_take_it(ctx, m, n, C, sp, want):
     """Also while a graph is recorded (no workspace is needed), whose replays give the same bits."""
     rng = np.random.default_rng(m + n)
