@@ -189,7 +189,7 @@ so_status so_ellpack_encode(so_ctx *ctx, const float *dDense, uint32_t m, uint32
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Calls no hipMalloc,
  * hipFree or allocating routine: the caller brings the outputs -- dNnz[m], dWd and dIdx of
  * m * r_cap slots each -- and the counting pass's partial results live in a static device array of
- * the library (524 544 bytes per GPU, held until the process ends), which limits a call to
+ * the library (540 928 bytes per GPU, held until the process ends), which limits a call to
  * 1 048 576 rows (more: SO_ERR_INVALID).  Output: dNnz[i] = nonzeros of row i, and dWd/dIdx packed
  * with row pitch r = the longest row, i.e. the first m * r slots hold exactly the arrays
  * so_ellpack_encode produces.  When r exceeds r_cap nothing is packed (dNnz is still valid).
@@ -220,8 +220,8 @@ so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t 
  * connected layer -- the reference's documented way to get its allocation-free run(), README.md:146).
  * No counterpart in the reference. */
 so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
-/* Which kernel the context's last so_matmul or so_conv2d launched, for tests and tuning: "merged", "quad", "planes", "narrow" and "vector" (on
- * handles with the RBM layout), "tiled", "shared", "row"; "columns", "merged-window", "window", "gather"; "" before the
+/* Which kernel the context's last so_matmul, so_conv2d or encode launched, for tests and tuning: "merged", "quad", "planes", "narrow" and "vector" (on
+ * handles with the RBM layout), "tiled", "shared", "row"; "columns", "merged-window", "window", "gather"; "encode-once", "encode-twice"; "" before the
  * first.  A static string.  No counterpart in the reference. */
 const char *so_last_kernel(const so_ctx *ctx);
 

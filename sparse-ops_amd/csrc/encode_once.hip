@@ -1,0 +1,318 @@
+// The device encoder from one read of W: so_ellpack_encode_noalloc where the caller waits for the counts.
+//
+// ELLPACK's row pitch is the longest row's length, which is known only when every row has been looked at, so the two
+// passes of csrc/runtime.hip read W twice.  Here one workgroup per compute unit takes its rows piece by piece, keeps what
+// it finds -- values, a byte of column each -- in the 160 KB of its compute unit's LDS (40 MB over the chip), tells the
+// others its longest row and its count, waits for theirs and writes its rows out at the pitch they agree on.  Pieces
+// that LDS has no room for are read and packed again.
+//
+// Decomposition.  A piece is up to 2048 columns of a row (less where a workgroup would have fewer pieces than waves); the
+// 16 waves take a workgroup's pieces in turn, each the next one's eight 16-byte loads ahead of the one it packs.  A wave packs into a
+// part of LDS of its own, from the front on: nothing is synchronised until all pieces are counted.  A row's places are
+// then a prefix sum over its pieces.
+//
+// The wait for the other workgroups has every one of them resident (a workgroup per compute unit), unless somebody else's
+// kernel holds some of the chip: it gives up after a bounded number of looks, the host is told, and the two passes do
+// the call again.  The words the workgroups tell each other carry the call's number, so nothing needs clearing.
+//
+// What bounds it: the read of W (8192 x 8192: 47 to 54 us, by workgroup, of which the copy's rate would take 43), then what
+// follows the slowest workgroup: 4 us until all know of all, 8 to 12 us of writing 61 MB at 90 % sparse; launch and the
+// host's wait 15.  The whole call on one matrix again and again, two passes / this one, us: 8192 x 8192 at 98 / 90 / 80 / 50 % sparse 100 / 75, 112 / 85, 135 / 108, 195 / 175
+// (6.7 M nonzeros fill the LDS; at 50 % seven pieces of eight are read again), 4096 x 4096 at 90 % 45 / 36, 2048 x 2048 27 / 24;
+// on changing matrices 8192 x 8192 at 90 % 127.6 / 91.9.
+#include "so_internal.h"
+
+#include <atomic>
+
+namespace {
+
+constexpr uint32_t THREADS = 1024, WAVES = 16, GROUPS = 8;        // groups of 256 columns a piece has at most
+constexpr uint32_t HEAD = 256;                                    // bytes of LDS before the table of counts
+constexpr uint32_t kEntryLimit = 4096;                            // words of the table of counts
+constexpr uint32_t kLooks = 1u << 11;                             // of a bounded wait: about 3 ms, where the workgroups differ by some 10 us
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Where one pass is the faster: the workgroups' wait for one another costs 3 us more than a second launch, which a matrix of
+// 16 MB repays (us, two passes / one: 256 x 8192 20.1 / 24.4, 911 x 1901 23.6 / 25.4, 1289 x 6285 30.7 / 28.4, 2048 x 2048 26.8 / 24.1); rows
+// well below three groups of 256 columns leave lanes idle (16384 x 520 35.5 / 40.2, 40000 x 600 60.2 / 69.4, 6549 x 786 35.3 / 31.3); and few
+// rows divide badly over the workgroups (520 rows, three on some, two on most: 22.5 / 24.2; 512 rows 30.5 / 27.4).
+constexpr uint64_t kLeastElements = 4u << 20;
+constexpr uint32_t kLeastColumns = 768;
+
+struct EncodeArgs {
+    const float *W;
+    uint32_t m, n, r_cap, groups, segs, part, table_bytes, call, looks;
+    unsigned long long *told;        // [2][workgroups]: {call, longest row}, {call, nonzeros}
+    uint32_t *host, *nnz, *idx;
+    float *Wd;
+};
+
+// A packed piece of c entries: the counts after each group but the last (two bytes each), values, column bytes.
+__device__ __forceinline__ uint32_t piece_bytes(uint32_t c) { return 16u + ((c * 5u + 15u) & ~15u); }
+
+__device__ __forceinline__ uint32_t piece_count(const f32x4u (&v)[GROUPS])
+{
+    uint32_t c = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < GROUPS; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c += (uint32_t)__popcll(__ballot(v[u][e] != 0.0f));
+    return c;
+}
+
+// Packs the piece a wave holds (a lane has four consecutive columns of each group) to `to` in ascending column order.
+__device__ __forceinline__ void piece_pack(const f32x4u (&v)[GROUPS], uint32_t c, char *to, uint32_t lane)
+{
+    float *val = reinterpret_cast<float *>(to + 16);
+    uint8_t *col = reinterpret_cast<uint8_t *>(to + 16u + 4u * c);
+    uint32_t at = 0, ends[GROUPS / 2];
+#pragma unroll
+    for (uint32_t u = 0; u < GROUPS; ++u) {
+        uint32_t pos = at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint64_t mask = __ballot(v[u][e] != 0.0f);
+            pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, pos));
+            at += (uint32_t)__popcll(mask);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (v[u][e] != 0.0f) {
+                val[pos] = v[u][e];
+                col[pos] = (uint8_t)(lane * 4u + (uint32_t)e);
+                ++pos;
+            }
+        if (u % 2u == 0u) ends[u / 2u] = at;
+        else ends[u / 2u] |= at << 16;
+    }
+    if (lane == 0) *reinterpret_cast<uint4 *>(to) = make_uint4(ends[0], ends[1], ends[2], ends[3]);
+}
+
+// Writes a packed piece whose first column is c0 to the row's slots from wd, ix on, four entries per lane.
+__device__ __forceinline__ void piece_write(const char *from, uint32_t c, uint32_t c0, float *wd, uint32_t *ix, uint32_t lane)
+{
+    const float *val = reinterpret_cast<const float *>(from + 16);
+    const uint8_t *col = reinterpret_cast<const uint8_t *>(from + 16u + 4u * c);
+    const uint4 e4 = *reinterpret_cast<const uint4 *>(from);
+    uint32_t ends[GROUPS];
+    const uint32_t words[4] = {e4.x, e4.y, e4.z, e4.w};
+#pragma unroll
+    for (uint32_t u = 0; u < GROUPS; ++u) ends[u] = __builtin_amdgcn_readfirstlane(u % 2u == 0u ? words[u / 2u] & 0xffffu : words[u / 2u] >> 16);
+    auto column = [&](uint32_t k, uint32_t byte) {
+        uint32_t g = 0;
+#pragma unroll
+        for (uint32_t u = 0; u + 1u < GROUPS; ++u) g += k >= ends[u] ? 256u : 0u;
+        return c0 + g + byte;
+    };
+    for (uint32_t k = lane * 4u; k < c; k += 256u) {
+        if (k + 4u <= c) {
+            const uint32_t b = *reinterpret_cast<const uint32_t *>(col + k);
+            *reinterpret_cast<f32x4u *>(wd + k) = *reinterpret_cast<const f32x4u *>(val + k);
+            *reinterpret_cast<u32x4u *>(ix + k) = u32x4u{column(k, b & 0xffu), column(k + 1u, (b >> 8) & 0xffu), column(k + 2u, (b >> 16) & 0xffu), column(k + 3u, b >> 24)};
+        } else {
+            for (uint32_t i = k; i < c; ++i) {
+                wd[i] = val[i];
+                ix[i] = column(i, col[i]);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(THREADS)
+void ellpack_encode_once_kernel(EncodeArgs a)
+{
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    uint32_t *smax = reinterpret_cast<uint32_t *>(lds), &gave_up = smax[WAVES];
+    unsigned long long *ssum = reinterpret_cast<unsigned long long *>(lds + 128);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wgs = gridDim.x, wg = blockIdx.x, rows = (a.m - wg + wgs - 1u) / wgs, items = rows * a.segs;     // rows wg, wg + wgs, ...
+    uint32_t *table = reinterpret_cast<uint32_t *>(lds + HEAD);      // [rows][segs + 1]: counts, then the places of the pieces in their row
+    char *part = lds + HEAD + a.table_bytes + wave * a.part;
+    if (tid == 0) gave_up = 0u;
+
+    auto load = [&](uint32_t j, f32x4u (&v)[GROUPS]) {
+        const uint32_t row = j / a.segs, c0 = (j - row * a.segs) * a.groups * 256u, jw = c0 + lane * 4u;
+        const float *wr = a.W + (size_t)(wg + row * wgs) * a.n;
+        if (a.groups == GROUPS && c0 + GROUPS * 256u <= a.n) {
+#pragma unroll
+            for (uint32_t u = 0; u < GROUPS; ++u) v[u] = *reinterpret_cast<const f32x4u *>(wr + jw + u * 256u);
+        } else {
+#pragma unroll
+            for (uint32_t u = 0; u < GROUPS; ++u) {
+                v[u] = f32x4u{0.f, 0.f, 0.f, 0.f};
+                if (u >= a.groups) continue;
+                const uint32_t c = jw + u * 256u;
+                if (c + 4u <= a.n) v[u] = *reinterpret_cast<const f32x4u *>(wr + c);
+                else {
+                    if (c < a.n) v[u][0] = wr[c];
+                    if (c + 1u < a.n) v[u][1] = wr[c + 1u];
+                    if (c + 2u < a.n) v[u][2] = wr[c + 2u];
+                }
+            }
+        }
+    };
+
+    // the pieces, counted, and packed while there is room
+    f32x4u v[GROUPS], next[GROUPS];
+    uint32_t used = 0;
+    if (wave < items) load(wave, v);
+    for (uint32_t j = wave; j < items; j += WAVES) {
+        if (j + WAVES < items) load(j + WAVES, next);
+        const uint32_t c = piece_count(v);
+#pragma unroll
+        for (uint32_t u = 0; u < GROUPS; ++u) asm volatile("" : "+v"(v[u]));     // the 32 ballots are taken again, not kept: they would not fit the scalar registers
+        if (used + piece_bytes(c) <= a.part) {
+            piece_pack(v, c, part + used, lane);
+            used += piece_bytes(c);
+        }
+        if (lane == 0) table[j + j / a.segs] = c;
+        if (j + WAVES < items) {
+#pragma unroll
+            for (uint32_t u = 0; u < GROUPS; ++u) v[u] = next[u];
+        }
+    }
+    __syncthreads();
+
+    // counts -> places; the workgroup's longest row and its count
+    uint32_t vmax = 0;
+    unsigned long long vsum = 0;
+    for (uint32_t row = tid; row < rows; row += THREADS) {
+        uint32_t *t = table + (size_t)row * (a.segs + 1u), at = 0;
+        for (uint32_t s = 0; s < a.segs; ++s) { const uint32_t c = t[s]; t[s] = at; at += c; }
+        t[a.segs] = at;
+        a.nnz[wg + row * wgs] = at;
+        vmax = max(vmax, at);
+        vsum += at;
+    }
+    auto reduce = [&]() {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) { vmax = max(vmax, (uint32_t)__shfl_xor(vmax, off, 64)); vsum += __shfl_xor(vsum, off, 64); }
+        if (lane == 0) { smax[wave] = vmax; ssum[wave] = vsum; }
+        __syncthreads();
+        vmax = smax[0];
+        vsum = ssum[0];
+        for (uint32_t w = 1; w < WAVES; ++w) { vmax = max(vmax, smax[w]); vsum += ssum[w]; }
+    };
+    reduce();
+    if (tid == 0) {
+        __hip_atomic_store(a.told + wg, (unsigned long long)a.call << 32 | vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(a.told + wgs + wg, (unsigned long long)a.call << 32 | (uint32_t)vsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // every workgroup's, a thread each
+    vmax = 0;
+    vsum = 0;
+    bool got = tid >= wgs;
+    for (uint32_t look = 0; look < a.looks && !__all(got); ++look) {
+        if (!got) {
+            const unsigned long long x = __hip_atomic_load(a.told + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long y = __hip_atomic_load(a.told + wgs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if ((uint32_t)(x >> 32) == a.call && (uint32_t)(y >> 32) == a.call) { got = true; vmax = (uint32_t)x; vsum = (uint32_t)y; }
+        }
+        if (!__all(got)) __builtin_amdgcn_s_sleep(4);
+    }
+    if (!__all(got) && lane == 0) gave_up = 1u;
+    __syncthreads();                                              // also: everybody has read smax and ssum
+    if (gave_up) {
+        if (tid == 0) a.host[3] = 1u;
+        return;
+    }
+    reduce();
+    const uint32_t r = __builtin_amdgcn_readfirstlane(vmax);
+    if (wg == 0 && tid == 0) { a.host[0] = r; a.host[1] = (uint32_t)vsum; a.host[2] = (uint32_t)(vsum >> 32); }
+    if (r > a.r_cap) return;
+
+    // out: first the pieces that were kept, then the others, packed again now that LDS has room
+    bool again = false;
+    for (uint32_t pass = 0; pass == 0u || (pass == 1u && again); ++pass) {
+        uint32_t at = 0;
+        for (uint32_t j = wave; j < items; j += WAVES) {
+            const uint32_t row = j / a.segs, s = j - row * a.segs;
+            const uint32_t *t = table + (size_t)row * (a.segs + 1u) + s;
+            const uint32_t first = __builtin_amdgcn_readfirstlane(t[0]), c = __builtin_amdgcn_readfirstlane(t[1]) - first, c0 = s * a.groups * 256u;
+            const size_t slot = (size_t)(wg + row * wgs) * r + first;
+            float *wd = a.Wd + slot;
+            uint32_t *ix = a.idx + slot;
+            const char *from = part + at;
+            const bool kept = at + piece_bytes(c) <= a.part;
+            if (kept) at += piece_bytes(c);
+            else again = true;
+            if (kept != (pass == 0u)) continue;
+            if (pass == 0u) {
+                piece_write(from, c, c0, wd, ix, lane);
+                continue;
+            }
+            if (j + WAVES < items) load(j, next);
+            else {
+#pragma unroll
+                for (uint32_t u = 0; u < GROUPS; ++u) next[u] = v[u];          // the wave's last piece is still here
+            }
+            if (piece_bytes(c) <= a.part) {
+                piece_pack(next, c, part, lane);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                piece_write(part, c, c0, wd, ix, lane);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                continue;
+            }
+            uint32_t k = 0;                                       // more than a wave's part of LDS holds: straight to memory
+#pragma unroll
+            for (uint32_t u = 0; u < GROUPS; ++u) {
+                uint32_t pos = k;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint64_t mask = __ballot(next[u][e] != 0.0f);
+                    pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, pos));
+                    k += (uint32_t)__popcll(mask);
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (next[u][e] != 0.0f) {
+                        wd[pos] = next[u][e];
+                        ix[pos] = c0 + u * 256u + lane * 4u + (uint32_t)e;
+                        ++pos;
+                    }
+            }
+        }
+    }
+    for (uint32_t row = wave; row < rows; row += WAVES) {
+        const size_t slot = (size_t)(wg + row * wgs) * r;
+        for (uint32_t k = table[(size_t)row * (a.segs + 1u) + a.segs] + lane; k < r; k += 64u) { a.Wd[slot + k] = 0.0f; a.idx[slot + k] = 0u; }
+    }
+}
+
+} // namespace
+
+so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, uint32_t r_cap, uint32_t *dNnz, float *dWd, uint32_t *dIdx,
+                         void *told, uint32_t *host_header, bool *done)
+{
+    *done = false;
+    if ((uint64_t)m * n < kLeastElements || n < kLeastColumns) return SO_OK;
+    const uint32_t wgs = std::min({m, (uint32_t)ctx->compute_units, kEncodeTold}), rows = so_ceil_div(m, wgs);
+    if (4ull * m < 3ull * rows * wgs) return SO_OK;
+    // pieces of equal width, one per wave at least
+    const uint32_t n256 = so_ceil_div(n, 256u);
+    uint32_t segs = std::max(so_ceil_div(n256, GROUPS), std::min(n256, so_ceil_div(WAVES, rows)));
+    const uint32_t groups = so_ceil_div(n256, segs);
+    segs = so_ceil_div(n256, groups);
+    const uint64_t entries = (uint64_t)rows * (segs + 1u);
+    if (entries > kEntryLimit) return SO_OK;
+    const size_t lds = (size_t)ctx->max_lds_bytes;
+    if (lds < (64u << 10)) return SO_OK;
+    static std::atomic<uint32_t> calls{0};
+    EncodeArgs a;
+    a.W = dDense; a.m = m; a.n = n; a.r_cap = r_cap; a.groups = groups; a.segs = segs;
+    a.table_bytes = ((uint32_t)entries * 4u + 15u) & ~15u;
+    a.part = (uint32_t)((lds - HEAD - a.table_bytes) / WAVES) & ~15u;
+    do a.call = ++calls; while (a.call == 0u);                    // zero is what the words held first
+    a.looks = ctx->tune.wait_spins >= 0 ? (uint32_t)ctx->tune.wait_spins : kLooks;
+    a.told = (unsigned long long *)told;
+    a.host = host_header; a.nnz = dNnz; a.idx = dIdx; a.Wd = dWd;
+    SO_HIP(so_allow_big_lds(ctx, (const void *)ellpack_encode_once_kernel));
+    host_header[3] = 0u;
+    ellpack_encode_once_kernel<<<wgs, THREADS, lds, ctx->stream>>>(a);
+    SO_LAUNCH_CHECK();
+    ctx->last_kernel = "encode-once";
+    *done = true;
+    return SO_OK;
+}

@@ -11,10 +11,10 @@
 static thread_local std::string g_last_error;
 
 // Scratch memory of so_ellpack_encode_noalloc: the counting pass's header and per-workgroup partial
-// results (layout further down, at the encoder).  Every GPU the library runs on holds its own copy
+// results (layout further down, at the encoder), then the words of so_encode_once.  Every GPU the library runs on holds its own copy
 // at its own address; host code never uses this name as a pointer, only the address that so_init
 // looks up for the context's device.
-constexpr size_t kStaticScratchBytes = 256 + 65536 * 8;
+constexpr size_t kEncodeToldOffset = 256 + 65536 * 8, kStaticScratchBytes = kEncodeToldOffset + kEncodeTold * 16;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 void so_set_error(const char *fmt, ...)
@@ -1082,7 +1082,7 @@ constexpr uint32_t kEncodeMaxBlocks = 65536;      // workgroups whose partials t
 constexpr uint32_t kEncodeHeaderBytes = 256;
 constexpr uint32_t kEncodeMaxCols = (1u << 28) - 1;     // the 16 rows of a workgroup, all dense, still count in 32 bits
 constexpr size_t kEncodeScratchBytes = kEncodeHeaderBytes + (size_t)kEncodeMaxBlocks * sizeof(uint2);
-static_assert(kEncodeScratchBytes <= kStaticScratchBytes, "the static scratch array holds the encoder's partials");
+static_assert(kEncodeScratchBytes <= kEncodeToldOffset, "the static scratch array holds the encoder's partials");
 
 // Rows per counting workgroup: with few rows the four waves of a workgroup share one, so that the chip is covered;
 // never more partials than kEncodeFoldBlocks up to 16 384 rows.
@@ -1284,6 +1284,7 @@ void ellpack_pack_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, ui
 so_status encode_launch(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, void *scratch, uint32_t r_cap,
                         uint32_t *dNnz, float *dWd, uint32_t *dIdx, uint32_t tail_words, bool count, bool pack, uint32_t *host_header)
 {
+    ctx->last_kernel = "encode-twice";
     uint32_t *header = (uint32_t *)scratch;
     uint2 *partial = (uint2 *)((char *)scratch + kEncodeHeaderBytes);
     const uint32_t rpb = encode_rows_per_block(m), nblocks = so_ceil_div(m, rpb);
@@ -1355,6 +1356,17 @@ extern "C" so_status so_ellpack_encode(so_ctx *ctx, const float *dDense, uint32_
     return SO_OK;
 }
 
+// What the kernels left in the pinned header, to the caller.
+static so_status encode_counts(const so_ctx *ctx, uint32_t r_cap, uint32_t *r_out, uint64_t *total_nnz_out)
+{
+    const uint32_t *header = ctx->h_encode_header;
+    if (r_out) *r_out = header[0];
+    if (total_nnz_out) *total_nnz_out = (uint64_t)header[1] | ((uint64_t)header[2] << 32);
+    SO_REQUIRE(header[0] <= r_cap, "so_ellpack_encode_noalloc: the longest row has %u nonzeros, dWd/dIdx hold %u per row (nothing was packed)",
+               header[0], r_cap);
+    return SO_OK;
+}
+
 extern "C" so_status so_ellpack_encode_noalloc(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, uint32_t r_cap,
                                               float *dWd, uint32_t *dIdx, uint32_t *dNnz, uint32_t *r_out,
                                               uint64_t *total_nnz_out)
@@ -1370,18 +1382,21 @@ extern "C" so_status so_ellpack_encode_noalloc(so_ctx *ctx, const float *dDense,
     SO_REQUIRE(ctx->static_scratch != nullptr, "so_ellpack_encode_noalloc: the context has no scratch address");
     const bool counts = r_out || total_nnz_out;
     SO_REQUIRE(!counts || !ctx->capturing, "so_ellpack_encode_noalloc: r_out/total_nnz_out need a wait, which a graph recording forbids");
-    // The kernels leave the counts in pinned host memory themselves: no copy to queue behind them.
+    // The kernels leave the counts in pinned host memory themselves: no copy to queue behind them.  A call that waits for them
+    // can also be done again by the two passes if the single one says so (its workgroups wait for one another, with a bound).
+    if (counts && (uint64_t)m * r_cap != 0) {
+        bool once = false;
+        so_status s = so_encode_once(ctx, dDense, m, n, r_cap, dNnz, dWd, dIdx, (char *)ctx->static_scratch + kEncodeToldOffset, ctx->h_encode_header, &once);
+        if (s == SO_OK && once) s = so_stream_wait(ctx, "so_ellpack_encode_noalloc");
+        if (s != SO_OK) return s;
+        if (once && ctx->h_encode_header[3] == 0) return encode_counts(ctx, r_cap, r_out, total_nnz_out);
+    }
     const so_status s = encode_launch(ctx, dDense, m, n, ctx->static_scratch, r_cap, dNnz, dWd, dIdx, 0, true,
                                       (uint64_t)m * r_cap != 0, counts ? ctx->h_encode_header : nullptr);
     if (s != SO_OK || !counts) return s;
     const so_status waited = so_stream_wait(ctx, "so_ellpack_encode_noalloc");
     if (waited != SO_OK) return waited;
-    const uint32_t *header = ctx->h_encode_header;
-    if (r_out) *r_out = header[0];
-    if (total_nnz_out) *total_nnz_out = (uint64_t)header[1] | ((uint64_t)header[2] << 32);
-    SO_REQUIRE(header[0] <= r_cap, "so_ellpack_encode_noalloc: the longest row has %u nonzeros, dWd/dIdx hold %u per row (nothing was packed)",
-               header[0], r_cap);
-    return SO_OK;
+    return encode_counts(ctx, r_cap, r_out, total_nnz_out);
 }
 
 extern "C" so_status so_ellpack_decode(so_ctx *ctx, const so_ellpack *E, float *dDense)

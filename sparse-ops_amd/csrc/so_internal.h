@@ -243,6 +243,12 @@ so_status so_matmul_planes_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C)
 so_status so_matmul_planes_launch(so_ctx *ctx, const so_ellpack *E, const so_planes_plan &p, const float *dX, uint32_t C,
                                   const float *dBias, float *dY, int act);
 
+// csrc/encode_once.hip: encode from one read of the matrix.  `told` holds 2 * kEncodeTold words of 64 bits that nothing else writes;
+// *done: launched, and after the stream's end host_header has {r, total nnz (low, high), 1 where it has to be done again}.
+constexpr uint32_t kEncodeTold = 1024;
+so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, uint32_t r_cap, uint32_t *dNnz, float *dWd, uint32_t *dIdx,
+                         void *told, uint32_t *host_header, bool *done);
+
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
 // since the last look (their results are invalid).  Every entry point that waits for the stream ends with this.
 so_status so_stream_wait(so_ctx *ctx, const char *who);
