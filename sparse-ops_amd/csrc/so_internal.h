@@ -69,6 +69,7 @@ struct so_ctx {
     uint32_t *d_stage_done = nullptr;      // workgroups of a way out that have finished
     size_t stage_used = 0;
     uint32_t stage_turn = 0;
+    uint32_t told_turn = 0;                // of the word behind the encoder's header in h_wait_gave_up's memory
     // Workspace of so_matmul's kernels that split a tile over workgroups: partial tiles, a zeroed counter per tile
     so_block_ref mm_part, mm_counters;
     std::vector<so_block_ref> recorded;          // what the launches of the recording under way use (so_keep_recorded)

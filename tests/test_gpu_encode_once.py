@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import datagen
+import hipabi
 
 pytestmark = pytest.mark.gpu
 
@@ -72,4 +73,21 @@ def test_row_longer_than_the_capacity(ctx):
         ctx.encode_dense_noalloc(dW, 2048, 2100, cap, dWd, dIdx, dNnz)
     assert (dWd.download() == 7.5).all() and np.array_equal(dNnz.download(), E.nnz)
     for a in (dW, dWd, dIdx, dNnz):
+        a.free()
+
+
+@pytest.mark.parametrize("m,n,kernel", [(2048, 2100, "encode-once"), (40, 300, "encode-twice")])
+def test_reports_waits_that_gave_up(ctx, m, n, kernel):
+    """The encoder's wait for its counts reports, once, a wait on LDS counters that gave up in an earlier launch of the stream."""
+    rng = np.random.default_rng(8)
+    E = datagen.encode_dense(datagen.bernoulli_dense(rng, 256, 1024, .1))
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, hipabi.LAYOUT_ROW | hipabi.LAYOUT_TILED)
+    dX, dY = ctx.array(rng.standard_normal((1024, 64)).astype(np.float32)), ctx.empty((256, 64))
+    W = _matrix(m, n, .2, 9)
+    with ctx.tuning(SPARSEOPS_MATMUL_TILED="1", SPARSEOPS_WAIT_SPINS="0"):
+        ctx.matmul(dE, dX, 64, None, dY)
+    with pytest.raises(hipabi.SoError, match="gave up"):
+        _check(ctx, W, kernel)
+    _check(ctx, W, kernel)
+    for a in (dE, dX, dY):
         a.free()
