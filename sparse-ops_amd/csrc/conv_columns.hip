@@ -11,13 +11,13 @@
 // input channels if 150 KB of LDS hold them, else a chunk at a time -- is copied to LDS with zeros outside the image; a
 // channel's entries {weight, LDS offset of its tap} come 16 at a time in lanes (the same 16 in every row of 16), four
 // such groups ahead, and are handed round by DPP: per entry one address add, one read, one multiply-add.  The reads run
-// two quads of entries ahead of the multiply-adds.  Workgroups shrink to 8 or 4 waves where that spreads the launch
+// three quads of entries ahead of the multiply-adds.  Workgroups shrink to 8 or 4 waves where that spreads the launch
 // over more compute units.
 //
-// What bounds it: the latency of a wave's LDS reads.  An entry takes a wave on a SIMD of its own 28 clocks, a step of four 112: each step begins by waiting
-// for the quad that was requested at the end of the step before last, so that a read's round trip has one step's eight vector instructions and four
-// reads, about 50 clocks to issue, to hide in.  (The chain of multiply-adds itself would allow 9 clocks an entry.)  The chains of 922 of a
-// ResNet-18-shaped 7 x 7 x 512 layer at 80 % are 11 of its 16 us; the rest is launch, first loads and the window's copy.
+// What bounds it: what one wave alone on a SIMD issues, about 5.8 clocks an instruction -- 18 an entry in a loop of nothing else, 23 with the entries'
+// loads, groups and waits (two, three or four quads of reads in flight: the same).  A ResNet-18-shaped 7 x 7 x 512 layer at 80 %, chains of 922:
+// 9.0 us of its 15.9; before them 3.0 us in which 16 waves issue the window's 592 copies, 12 clocks each (beginning in another place in each
+// workgroup: 1.5 us slower), 1 until all is there, 0.6 of arguments and places, and the launch.
 #include "so_internal.h"
 #include "conv_internal.h"
 #include "dpp_steps.h"
@@ -32,6 +32,7 @@ struct ColArgs {
     uint32_t PE;                 // pixels of a window plane in LDS order (rows of IP pixels)
     uint32_t IP, PL;             // row pitch in pixels; floats per plane (PE * B)
     uint32_t cc, nch, G, waves;  // channels per chunk, chunks; computing waves (= channels) and waves of a workgroup
+    uint32_t pitch;              // groups from one (channel, chunk) to the next; 0: first[] says where they begin
     uint32_t sth, stw, sbh, sbw; // window pixels per output pixel, input pixels per window pixel
     uint32_t mB, mIP, mPL, mTW, mTilesX;
 };
@@ -84,10 +85,25 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
     const uint32_t tile_y = window_div(blockIdx.x, a.tiles_x, a.mTilesX);
     const uint32_t th0 = tile_y * a.TH, tw0 = (blockIdx.x - tile_y * a.tiles_x) * a.TW;
 
-    // the wave's entries, groups of 16 (the stream ends with eight padding groups)
-    const uint32_t *__restrict__ first = first_group + (size_t)(computes ? co : 0u) * a.nch;
+    // The wave's entries, groups of 16 (the stream ends with eight padding groups).  At a pitch their place needs no look
+    // into a table, whose round trip to memory -- nothing is cached when a kernel starts -- would come before theirs.
+    const uint32_t run0 = (computes ? co : 0u) * a.nch;
     const int2 *__restrict__ ep = entries + (lane & 15u);
     int2 cur[4], nxt[4];
+    uint32_t g0, g1;
+    auto first_entries = [&](uint32_t t) {
+        if (a.pitch != 0u) {
+            g0 = (run0 + t) * a.pitch;
+            g1 = g0 + __builtin_amdgcn_readfirstlane(first_group[run0 + t]);
+        } else {
+            g0 = __builtin_amdgcn_readfirstlane(first_group[run0 + t]);
+            g1 = __builtin_amdgcn_readfirstlane(first_group[run0 + t + 1u]);
+        }
+        if (!computes) g1 = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) cur[i] = ep[(size_t)(g0 + i) * 16u];
+    };
+    first_entries(0);
 
     // this lane's output column
     const uint32_t pix = window_div(lane, B, a.mB), b = lane - pix * B;
@@ -133,24 +149,24 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
         }
     };
     const uint32_t base = so_lds::lds_address(window) + lane_off;
-    // Quads 2 and 3 of the group before this one still owe their multiply-adds: operands in xA, xB, weights in owed.
-    float xA[4] = {0.f, 0.f, 0.f, 0.f}, xB[4] = {0.f, 0.f, 0.f, 0.f}, xC[4], xD[4], owed = -0.0f;
+    // Quads 1, 2 and 3 of the group before this one still owe their multiply-adds: operands in xB, xC, xD, weights in owed.
+    float xA[4], xB[4] = {0.f, 0.f, 0.f, 0.f}, xC[4] = {0.f, 0.f, 0.f, 0.f}, xD[4] = {0.f, 0.f, 0.f, 0.f}, owed = -0.0f;
     auto group = [&](const int2 &e) {
         float w = __int_as_float(e.x);
         uint32_t off = (uint32_t)e.y;
         asm volatile("s_nop 4" : "+v"(w), "+v"(off), "+v"(owed));      // DPP operands: not within two cycles of a vector write
-        step4<0, 8>(base, off, xC, owed, xA, acc);
-        step4<4, 12>(base, off, xD, owed, xB, acc);
-        step4<8, 0>(base, off, xA, w, xC, acc);
-        step4<12, 4>(base, off, xB, w, xD, acc);
+        step4<0, 4>(base, off, xA, owed, xB, acc);
+        step4<4, 8>(base, off, xB, owed, xC, acc);
+        step4<8, 12>(base, off, xC, owed, xD, acc);
+        step4<12, 0>(base, off, xD, w, xA, acc);
         owed = w;
     };
     for (uint32_t t = 0; t < a.nch; ++t) {
-        if (t) __syncthreads();                                        // every wave has read what it needs of the last chunk
+        if (t) {
+            first_entries(t);
+            __syncthreads();                                           // every wave has read what it needs of the last chunk
+        }
         copy_window(t);
-        const uint32_t g0 = __builtin_amdgcn_readfirstlane(first[t]), g1 = computes ? __builtin_amdgcn_readfirstlane(first[t + 1u]) : 0u;
-#pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) cur[i] = ep[(size_t)(g0 + i) * 16u];
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");             // this thread's part of the window is in LDS
         __syncthreads();
         for (uint32_t gi = g0; gi < g1; gi += 4u) {
@@ -165,8 +181,9 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
         }
     }
     asm volatile("s_nop 4" : "+v"(owed));
-    fma4<8>(owed, xA, acc);
-    fma4<12>(owed, xB, acc);
+    fma4<4>(owed, xB, acc);
+    fma4<8>(owed, xC, acc);
+    fma4<12>(owed, xD, acc);
 
     if (live) {
         const size_t at = (((size_t)co * g.H_out + th0 + ty) * g.W_out + tw0 + tx) * B + b;
@@ -235,31 +252,39 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
     if ((uint64_t)c.tiles_x * c.tiles_x * c.tiles_y >= (1ull << 32) || plane * plane >= (1ull << 32) || plane * 1024 >= (1ull << 32)) return SO_OK;
     if ((uint64_t)c.tiles_x * c.tiles_y >= (1ull << 31) || ((uint64_t)c.cc + 1024) * g.H_in * g.W_in * B >= (1ull << 30)) return SO_OK;
     const uint32_t kHW = g.kH * g.kW;
-    std::vector<uint32_t> first((size_t)E->m * c.nch + 1);
-    std::vector<int2> entries;
-    entries.reserve((size_t)E->total_nnz + (size_t)E->m * c.nch * 8 + 128);
+    const size_t runs = (size_t)E->m * c.nch;
+    std::vector<uint32_t> first(runs + 1);      // entries of every (channel, chunk), then groups, then where they begin
+    for (uint32_t co = 0; co < E->m; ++co)
+        for (uint32_t j = 0; j < nnz[co]; ++j) ++first[(size_t)co * c.nch + idx[(size_t)co * E->r + j] / kHW / c.cc];
+    uint64_t total = 0;
+    for (uint32_t &f : first) { f = (f + 15u) / 16u; total += f; c.pitch = std::max(c.pitch, f); }
+    // at a pitch unless few long runs make that much larger
+    if ((uint64_t)runs * c.pitch > 2 * total + 1024) c.pitch = 0;
+    else total = (uint64_t)runs * c.pitch;
+    if (total > 0xfffffff0ull) return SO_OK;
     uint32_t pad_bits;
     const float neg_zero = -0.0f;
     std::memcpy(&pad_bits, &neg_zero, 4);
-    const int2 pad = make_int2((int)pad_bits, (int)(c.cc * plane * 4));
+    std::vector<int2> entries((size_t)total * 16 + 128, make_int2((int)pad_bits, (int)(c.cc * plane * 4)));
+    size_t next = 0;                            // group
     for (uint32_t co = 0; co < E->m; ++co) {
         uint32_t j = 0;
         for (uint32_t t = 0; t < c.nch; ++t) {
-            first[(size_t)co * c.nch + t] = (uint32_t)(entries.size() / 16);
+            const size_t run = (size_t)co * c.nch + t;
+            if (c.pitch) next = run * c.pitch;
+            int2 *e = entries.data() + next * 16;
             for (; j < nnz[co]; ++j) {
                 const size_t slot = (size_t)co * E->r + j;
                 const uint32_t k = idx[slot], cin = k / kHW, kh = (k / g.kW) % g.kH, kw = k % g.kW;
                 if (cin >= (t + 1) * c.cc) break;
                 uint32_t wb;
                 std::memcpy(&wb, &Wd[slot], 4);
-                entries.push_back(make_int2((int)wb, (int)(((uint64_t)(cin - t * c.cc) * plane + (uint64_t)(kh * g.dil_h * c.IP + kw * g.dil_w) * B) * 4)));
+                *e++ = make_int2((int)wb, (int)(((uint64_t)(cin - t * c.cc) * plane + (uint64_t)(kh * g.dil_h * c.IP + kw * g.dil_w) * B) * 4));
             }
-            while (entries.size() % 16) entries.push_back(pad);
+            if (!c.pitch) { const uint32_t groups = first[run]; first[run] = (uint32_t)next; next += groups; }
         }
     }
-    first.back() = (uint32_t)(entries.size() / 16);
-    if (entries.size() / 16 > 0xfffffff0ull) return SO_OK;
-    entries.resize(entries.size() + 128, pad);
+    if (!c.pitch) first.back() = (uint32_t)next;
     for (const void *k : {(const void *)conv2d_column_kernel<SO_ACT_NONE>, (const void *)conv2d_column_kernel<SO_ACT_RELU>,
                           (const void *)conv2d_column_kernel<SO_ACT_SIGMOID>, (const void *)conv2d_column_kernel<SO_ACT_TANH>})
         SO_HIP(so_allow_big_lds(ctx, k));
@@ -289,7 +314,7 @@ struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 // Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
 // longest chain at 12 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
 // more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 9.0 us, 28x28x128 10.2, 14x14x256
-// 10.4, 7x7x512 16; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
+// 10.4, 7x7x512 15.9; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
 ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
 {
     const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
@@ -340,7 +365,7 @@ so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const fl
     const so_conv_columns &c = plan->col[B - 1];
     const so_conv_geom &g = plan->g;
     ColArgs a;
-    a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch;
+    a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch; a.pitch = c.pitch;
     a.sth = window_step(g.kH, g.stride_h); a.stw = window_step(g.kW, g.stride_w);
     a.sbh = window_subsample(g.kH, g.stride_h); a.sbw = window_subsample(g.kW, g.stride_w);
     a.mB = window_magic(B); a.mIP = window_magic(a.IP); a.mPL = window_magic(a.PL); a.mTW = window_magic(a.TW); a.mTilesX = window_magic(a.tiles_x);

@@ -41,8 +41,9 @@ constexpr uint32_t kColMaxBatch = 4;
 struct so_conv_columns {
     uint32_t batch = 0;              // the batch the tile and the offsets are for; 0: not built, or the kernel does not apply
     uint32_t TH = 0, TW = 0, tiles_x = 0, tiles_y = 0, IP = 0, PE = 0, cc = 0, nch = 0;
+    uint32_t pitch = 0;              // groups from one (channel, chunk) to the next; 0: one right behind the other
     int2 *d_entries = nullptr;       // groups of 16 {weight bits, LDS byte offset}, channel by channel, chunk by chunk
-    uint32_t *d_first = nullptr;     // [Cout * nch + 1]: first group of (channel, chunk)
+    uint32_t *d_first = nullptr;     // [Cout * nch + 1]: groups of (channel, chunk) where there is a pitch, else its first group
 };
 
 struct so_conv_plan {
