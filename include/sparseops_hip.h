@@ -256,7 +256,7 @@ so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan);
 so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t B);
 /* The LDS-windowed kernel's parameters for this plan (no counterpart in the reference:
  * a tuning/inspection aid): out = {tile_h, tile_w, window_h, window_w, channels per
- * chunk, chunks, output channels per wave, 0}; all zero when the geometry does not
+ * chunk, chunks, output channels per wave, pixel groups per wave at batch tile 16}; all zero when the geometry does not
  * suit that kernel and so_conv2d always takes the gather kernel. */
 so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[8]);
 

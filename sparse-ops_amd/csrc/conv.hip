@@ -271,6 +271,12 @@ __device__ __forceinline__ void touch_stream(const int4 *p, uint32_t quads, uint
         : "scc");
 }
 
+// PX pixel groups per wave.  With scalar entries a multiply-add whose weight is a scalar operand takes the vector unit 3.3 clocks, one of
+// three vector registers 2.5: a wave that applies an entry to two pixel groups moves its weight to a vector register once for
+// eight multiply-adds, and the loop around them -- scalar loads, shifts, counters -- turns half as often.  Vector instructions were
+// what bounded the step loop; now LDS reads are (6.8 of the 8.3 us of a chunk of a 56x56x64 layer).  ResNet-18-shaped layers
+// at batch 32, PX 1 with twice the channels per wave / PX 2, us: 56x56x64 52.7-56.2 / 45.8-51.1, 28x28x128 53.0-54.5 / 46.0-46.5, the whole stack 1043 / 988.
+//
 // The four waves that share a SIMD are served oldest first: left alone, the first of them finishes a
 // chunk's steps in half the time of the last (measured with the shader clock on the 56x56x64 layer:
 // 14.1 k, 17.4 k, 22.1 k, 28.7 k clocks by age), and everybody then waits for the last one at the
@@ -288,7 +294,7 @@ __device__ __forceinline__ void rotate_priority(uint32_t turn)
     }
 }
 
-template <int CPW, int LPP, int ACT>
+template <int CPW, int LPP, int ACT, int PX>
 __global__ __launch_bounds__(kWinThreads)
 void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__restrict__ gbase,
                           const uint32_t *__restrict__ quads, WinArgs a, so_conv_geom g,
@@ -308,13 +314,18 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     const bool computes = cgi < a.cg && grp < a.groups;              // the other waves only help copying
     const uint32_t gi = computes ? grp : 0u;
 
-    // this lane's output pixel and its corner inside the window
-    const uint32_t pl = pgi * PPW + lane / LPP, b4 = lane % LPP;
-    const bool pvalid = pl < a.TH * a.TW;
-    const uint32_t pc = window_slot_pixel(a, pl & 63u);          // slots beyond the tile repeat a pixel of their group
-    const uint32_t ty = window_div(pc, a.TW, a.mTW), tx = pc - ty * a.TW;
-    const bool live = computes && pvalid && th0 + ty < g.H_out && tw0 + tx < g.W_out;
-    const uint32_t lanebase = ((ty * a.sth * a.IW + tx * a.stw) << SHIFT) + b4 * 16u;   // bytes
+    // this lane's output pixels and their corners inside the window
+    const uint32_t b4 = lane % LPP;
+    uint32_t ty[PX], tx[PX], lanebase[PX];
+    bool live[PX];
+#pragma unroll
+    for (int x = 0; x < PX; ++x) {
+        const uint32_t pl = (pgi * PX + (uint32_t)x) * PPW + lane / LPP;
+        const uint32_t pc = window_slot_pixel(a, pl & 63u);      // slots beyond the tile repeat a pixel of their group
+        ty[x] = window_div(pc, a.TW, a.mTW); tx[x] = pc - ty[x] * a.TW;
+        live[x] = computes && pl < a.TH * a.TW && th0 + ty[x] < g.H_out && tw0 + tx[x] < g.W_out;
+        lanebase[x] = ((ty[x] * a.sth * a.IW + tx[x] * a.stw) << SHIFT) + b4 * 16u;   // bytes
+    }
     const uint32_t buf_bytes = a.buf_f4 * 16u;
 
     // window elements this thread copies: element e = tid + k*1024 is float4 (cl, ih, iw, b4)
@@ -354,11 +365,12 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
             if (gcl[k] != 0xffffffffu) win_lds[buf * a.buf_f4 + tid + (uint32_t)k * kWinThreads] = xr[k];
     };
 
-    float acc[CPW][4];
+    float acc[CPW][PX][4];
 #pragma unroll
     for (int c = 0; c < CPW; ++c) {
         const float b0 = (bias && computes && co0 + c < g.Cout) ? bias[co0 + c] : 0.0f;
-        acc[c][0] = acc[c][1] = acc[c][2] = acc[c][3] = b0;
+#pragma unroll
+        for (int x = 0; x < PX; ++x) acc[c][x][0] = acc[c][x][1] = acc[c][x][2] = acc[c][x][3] = b0;
     }
 
     // the all-zero plane behind each window buffer (padding entries point into it)
@@ -389,7 +401,7 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     // wins wherever a wave has enough runs per chunk to amortise its scalar loads: measured on the
     // ResNet-18-shaped layers at batch 32, scalar against lanes: 8 channels per wave 55 against 60 us,
     // 4 channels 56.1 against 63.2, 2 channels 58.8 against 56.6; small batches use 1-2 channels.
-    constexpr bool LANE_ENT = CPW < 4;
+    constexpr bool LANE_ENT = PX == 1 && CPW < 4;
     // priorities rotate on the full batch tile only: on the smaller ones (batches below 16) it measured 5 % slower
     constexpr bool ROTATE = LPP == 4;
     // progress counters instead of a barrier per chunk: the same (batch 8: 0.466 -> 0.474 ms, batch 1: 0.365 -> 0.374 with them)
@@ -417,7 +429,9 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
         const bool more = t + 1 < a.nch;
         if (more) fetch_window(t + 1);
         const uint32_t cur_buf = a.nbuf == 2 ? (t & 1u) : 0u;
-        const uint32_t base = lanebase + cur_buf * buf_bytes;
+        uint32_t base[PX];
+#pragma unroll
+        for (int x = 0; x < PX; ++x) base[x] = lanebase[x] + cur_buf * buf_bytes;
         uint32_t nq[CPW];
 #pragma unroll
         for (int c = 0; c < CPW; ++c) nq[c] = computes ? qp[t * CPW + c] : 0u;
@@ -444,12 +458,12 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
                 // (2 channels per wave) 63.5 -> 58.4 us, 7x7x512 (1 per wave) 69.1 -> 66.1 us; with 4
                 // channels per wave the four copies of these bodies made 28x28x128 11 % slower.
                 const uint32_t n = nq[c];
-                const char *xb = lds_bytes + base;
+                const char *xb = lds_bytes + base[0];
                 float4 xA[4], xB[4];
                 if (n >= 4u) {
                     ep += 16;
                     int2 enxt = ep[0];                                    // the stream ends with 16 padding entries
-                    so_dpp::group16<false>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c]);
+                    so_dpp::group16<false>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c][0]);
                     float ewp = __int_as_float(ecur.x);
                     ecur = enxt;
                     uint32_t q = 4u;
@@ -459,22 +473,22 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
                         if constexpr (ROTATE) rotate_priority(turn + (q >> 2));
                         ep += 16;
                         enxt = ep[0];
-                        so_dpp::group16<true>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c]);
+                        so_dpp::group16<true>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c][0]);
                         ewp = __int_as_float(ecur.x);
                         ecur = enxt;
                     }
                     if (q < n) {
                         ep += 4u * (n - q);
                         enxt = ep[0];
-                        so_dpp::group_tail<true>(n - q, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c]);
+                        so_dpp::group_tail<true>(n - q, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c][0]);
                         ecur = enxt;
                     } else {
-                        so_dpp::group_drain(ewp, xB, acc[c]);
+                        so_dpp::group_drain(ewp, xB, acc[c][0]);
                     }
                 } else if (n != 0u) {
                     ep += 4u * n;
                     const int2 enxt = ep[0];
-                    so_dpp::group_tail<false>(n, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c]);
+                    so_dpp::group_tail<false>(n, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c][0]);
                     ecur = enxt;
                 }
                 continue;
@@ -485,7 +499,7 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
                     const uint32_t steps = 4u * min(4u, nq[c] - q);      // this group: 4, 8, 12 or 16 entries
                     ep += steps;
                     const int2 enxt = ep[0];                              // the stream ends with 16 padding entries
-                    so_dpp::tiled_chunk(lds_bytes + base, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, steps, acc[c]);
+                    so_dpp::tiled_chunk(lds_bytes + base[0], __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, steps, acc[c][0]);
                     ecur = enxt;
                 }
                 continue;
@@ -493,20 +507,22 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
             for (uint32_t q = 0; q < nq[c]; ++q) {
                 const i32x4 nxt0 = sp[0], nxt1 = sp[1];
                 sp += 2;
-                const float4 x0 = *reinterpret_cast<const float4 *>(lds_bytes + base + ((uint32_t)cur0.y << SHIFT));
-                const float4 x1 = *reinterpret_cast<const float4 *>(lds_bytes + base + ((uint32_t)cur0.w << SHIFT));
-                const float4 x2 = *reinterpret_cast<const float4 *>(lds_bytes + base + ((uint32_t)cur1.y << SHIFT));
-                const float4 x3 = *reinterpret_cast<const float4 *>(lds_bytes + base + ((uint32_t)cur1.w << SHIFT));
-                const float w0 = __int_as_float(cur0.x), w1 = __int_as_float(cur0.z);
-                const float w2 = __int_as_float(cur1.x), w3 = __int_as_float(cur1.z);
-                acc[c][0] = __builtin_fmaf(w0, x0.x, acc[c][0]); acc[c][1] = __builtin_fmaf(w0, x0.y, acc[c][1]);
-                acc[c][2] = __builtin_fmaf(w0, x0.z, acc[c][2]); acc[c][3] = __builtin_fmaf(w0, x0.w, acc[c][3]);
-                acc[c][0] = __builtin_fmaf(w1, x1.x, acc[c][0]); acc[c][1] = __builtin_fmaf(w1, x1.y, acc[c][1]);
-                acc[c][2] = __builtin_fmaf(w1, x1.z, acc[c][2]); acc[c][3] = __builtin_fmaf(w1, x1.w, acc[c][3]);
-                acc[c][0] = __builtin_fmaf(w2, x2.x, acc[c][0]); acc[c][1] = __builtin_fmaf(w2, x2.y, acc[c][1]);
-                acc[c][2] = __builtin_fmaf(w2, x2.z, acc[c][2]); acc[c][3] = __builtin_fmaf(w2, x2.w, acc[c][3]);
-                acc[c][0] = __builtin_fmaf(w3, x3.x, acc[c][0]); acc[c][1] = __builtin_fmaf(w3, x3.y, acc[c][1]);
-                acc[c][2] = __builtin_fmaf(w3, x3.z, acc[c][2]); acc[c][3] = __builtin_fmaf(w3, x3.w, acc[c][3]);
+                float w[4] = {__int_as_float(cur0.x), __int_as_float(cur0.z), __int_as_float(cur1.x), __int_as_float(cur1.z)};
+                const uint32_t off[4] = {(uint32_t)cur0.y << SHIFT, (uint32_t)cur0.w << SHIFT, (uint32_t)cur1.y << SHIFT, (uint32_t)cur1.w << SHIFT};
+                float4 v[4][PX];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int x = 0; x < PX; ++x) v[e][x] = *reinterpret_cast<const float4 *>(lds_bytes + base[x] + off[e]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (PX > 1) asm("v_mov_b32 %0, %1" : "=v"(w[e]) : "s"(w[e]));
+#pragma unroll
+                    for (int x = 0; x < PX; ++x) {
+                        acc[c][x][0] = __builtin_fmaf(w[e], v[e][x].x, acc[c][x][0]); acc[c][x][1] = __builtin_fmaf(w[e], v[e][x].y, acc[c][x][1]);
+                        acc[c][x][2] = __builtin_fmaf(w[e], v[e][x].z, acc[c][x][2]); acc[c][x][3] = __builtin_fmaf(w[e], v[e][x].w, acc[c][x][3]);
+                    }
+                }
                 cur0 = nxt0;
                 cur1 = nxt1;
             }
@@ -533,32 +549,35 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
         }
     }
 
-    if (live) {
-        const uint32_t ho = th0 + ty, wo = tw0 + tx;
+#pragma unroll
+    for (int x = 0; x < PX; ++x) {
+        if (!live[x]) continue;
+        const uint32_t ho = th0 + ty[x], wo = tw0 + tx[x];
 #pragma unroll
         for (int c = 0; c < CPW; ++c) {
             const uint32_t co = co0 + c;
             if (co < g.Cout) {
                 const size_t at = (((size_t)co * g.H_out + ho) * g.W_out + wo) * B + bz + b4 * 4u;
+                float (&v)[4] = acc[c][x];
                 if (resid) {             // conv + skip, then the activation
                     const float4 rv = *reinterpret_cast<const float4 *>(resid + at);
-                    acc[c][0] += rv.x; acc[c][1] += rv.y; acc[c][2] += rv.z; acc[c][3] += rv.w;
+                    v[0] += rv.x; v[1] += rv.y; v[2] += rv.z; v[3] += rv.w;
                 }
                 float4 out;
-                out.x = so_epilogue<ACT>(acc[c][0]); out.y = so_epilogue<ACT>(acc[c][1]);
-                out.z = so_epilogue<ACT>(acc[c][2]); out.w = so_epilogue<ACT>(acc[c][3]);
+                out.x = so_epilogue<ACT>(v[0]); out.y = so_epilogue<ACT>(v[1]);
+                out.z = so_epilogue<ACT>(v[2]); out.w = so_epilogue<ACT>(v[3]);
                 *reinterpret_cast<float4 *>(Y + at) = out;
             }
         }
     }
 }
 
-template <int CPW, int LPP>
+template <int CPW, int LPP, int PX>
 void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, dim3 grid, size_t lds,
                        const float *dX, uint32_t B, const float *dBias, const float *dResid, float *dY, int act)
 {
 #define SO_WIN_LAUNCH(A)                                                                                   \
-    conv2d_window_kernel<CPW, LPP, A><<<grid, kWinThreads, lds, ctx->stream>>>(                            \
+    conv2d_window_kernel<CPW, LPP, A, PX><<<grid, kWinThreads, lds, ctx->stream>>>(                            \
         reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a,       \
         plan->g, dX, B, dBias, dResid, dY)
     switch (act) {
@@ -572,12 +591,12 @@ void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, 
 
 // The windowed kernels use more than the default 64 KB of dynamic LDS: raise the limit of every
 // instantiation once, at plan creation (never from so_conv2d, which may run under graph capture).
-template <int CPW, int LPP>
+template <int CPW, int LPP, int PX>
 hipError_t window_allow_lds(so_ctx *ctx)
 {
     hipError_t e = hipSuccess;
-    const void *k[4] = {(const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_NONE>, (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_RELU>,
-                        (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_SIGMOID>, (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_TANH>};
+    const void *k[4] = {(const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_NONE, PX>, (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_RELU, PX>,
+                        (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_SIGMOID, PX>, (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_TANH, PX>};
     for (const void *f : k)
         if (e == hipSuccess) e = so_allow_big_lds(ctx, f);
     return e;
@@ -585,12 +604,13 @@ hipError_t window_allow_lds(so_ctx *ctx)
 
 so_status window_configure(so_ctx *ctx)
 {
-    SO_HIP((window_allow_lds<8, 4>(ctx))); SO_HIP((window_allow_lds<4, 4>(ctx)));
-    SO_HIP((window_allow_lds<2, 4>(ctx))); SO_HIP((window_allow_lds<1, 4>(ctx)));
-    SO_HIP((window_allow_lds<8, 2>(ctx))); SO_HIP((window_allow_lds<4, 2>(ctx)));
-    SO_HIP((window_allow_lds<2, 2>(ctx))); SO_HIP((window_allow_lds<1, 2>(ctx)));
-    SO_HIP((window_allow_lds<8, 1>(ctx))); SO_HIP((window_allow_lds<4, 1>(ctx)));
-    SO_HIP((window_allow_lds<2, 1>(ctx))); SO_HIP((window_allow_lds<1, 1>(ctx)));
+    SO_HIP((window_allow_lds<8, 4, 1>(ctx))); SO_HIP((window_allow_lds<4, 4, 1>(ctx)));
+    SO_HIP((window_allow_lds<2, 4, 1>(ctx))); SO_HIP((window_allow_lds<1, 4, 1>(ctx)));
+    SO_HIP((window_allow_lds<8, 2, 1>(ctx))); SO_HIP((window_allow_lds<4, 2, 1>(ctx)));
+    SO_HIP((window_allow_lds<2, 2, 1>(ctx))); SO_HIP((window_allow_lds<1, 2, 1>(ctx)));
+    SO_HIP((window_allow_lds<8, 1, 1>(ctx))); SO_HIP((window_allow_lds<4, 1, 1>(ctx)));
+    SO_HIP((window_allow_lds<2, 1, 1>(ctx))); SO_HIP((window_allow_lds<1, 1, 1>(ctx)));
+    SO_HIP((window_allow_lds<4, 4, 2>(ctx))); SO_HIP((window_allow_lds<2, 4, 2>(ctx)));
     return SO_OK;
 }
 
@@ -613,7 +633,8 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     WinArgs a;
     a.TH = w.TH; a.TW = w.TW; a.IH = w.IH; a.IW = w.IW; a.cc = w.cc; a.nch = w.nch; a.tiles_x = w.tiles_x;
     a.groups = w.groups;
-    a.pg = so_ceil_div(w.TH * w.TW, PPW);
+    const uint32_t px = LPP == 4 ? w.px : 1u;
+    a.pg = so_ceil_div(w.TH * w.TW, PPW * px);
     a.cg = 16 / a.pg;
     // A grid of at most half the CUs (small batches on small images): halve the computing waves of
     // a workgroup -- the others still help copying the window -- while the doubled grid still fits
@@ -643,11 +664,17 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     // 14x14 and 7x7 layers of a ResNet-18-shaped stack at batch 8); below that the gather kernel's finer waves win.
     if (!forced && 8 * wgs < (uint64_t)ctx->compute_units) return SO_OK;
     if (grid.y > 65535u || grid.z > 65535u) return SO_OK;
+    if (px == 2u) {
+        if constexpr (LPP == 4) {
+            if (w.cpw == 4) window_launch_act<4, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
+            else window_launch_act<2, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
+        }
+    } else
     switch (w.cpw) {
-    case 8:  window_launch_act<8, (int)LPP>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
-    case 4:  window_launch_act<4, (int)LPP>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
-    case 2:  window_launch_act<2, (int)LPP>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
-    default: window_launch_act<1, (int)LPP>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 8:  window_launch_act<8, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 4:  window_launch_act<4, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 2:  window_launch_act<2, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    default: window_launch_act<1, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
     }
     ctx->waits_pending = true;
     *done = true;
@@ -766,6 +793,10 @@ so_status build_window(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32
     if (run < 6.0) return SO_OK;
     if ((uint64_t)cc * g.H_in * g.W_in >= (1ull << 24)) return SO_OK;   // int32 offsets up to batch 128
     w.cpw = choose_cpw(ctx, w, g.Cout, run, batch);
+    // Two pixel groups and four or more channels per wave: two waves would walk the same entries, now one does for both.
+    // With two channels per wave not: tiles of 32 pixels and one channel take 69 us where tiles of 14 and two take 53 (14x14x256),
+    // the window's chunks being half as long.
+    if (w.lpp == 4 && w.cpw >= 4 && so_ceil_div(w.TH * w.TW, 16u) == 2) { w.px = 2; w.cpw /= 2; }
     const uint32_t cpw = (uint32_t)w.cpw;
     w.groups = so_ceil_div(E->m, cpw);
 
@@ -932,7 +963,7 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
     if (window && plan->win.cc == 0) window = lpp != plan->tried_lpp;
     else if (window) {
         const double run = (double)E->total_nnz / (double)plan->g.Cout / plan->win.nch;
-        window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw;
+        window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw * (int)plan->win.px;
     }
     const bool columns = B >= 1 && B <= kColMaxBatch && !plan->col_tried[B - 1];
     if (!window && !columns) { plan->tuned_batch = batch; return SO_OK; }
@@ -959,7 +990,7 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
 {
     SO_REQUIRE(plan && out, "so_conv_plan_window: null argument");
     const so_conv_window &w = plan->win;
-    const uint32_t v[8] = {w.TH, w.TW, w.IH, w.IW, w.cc, w.nch, (uint32_t)w.cpw, 0u};
+    const uint32_t v[8] = {w.TH, w.TW, w.IH, w.IW, w.cc, w.nch, (uint32_t)w.cpw, w.px};
     for (int i = 0; i < 8; ++i) out[i] = w.cc ? v[i] : 0u;
     return SO_OK;
 }
@@ -982,7 +1013,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
         const bool alone = B < 4 || plan->win.cc == 0;           // no windowed kernel: else the gather kernel
         bool use = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
         if (!use && !alone && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
-            const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw, B), (uint64_t)ctx->compute_units);
+            const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw * plan->win.px, B), (uint64_t)ctx->compute_units);
             use = so_conv_columns_estimate(ctx, plan, B) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
         }
         if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for

@@ -21,6 +21,7 @@ struct so_conv_window {
     uint32_t TH = 0, TW = 0, IH = 0, IW = 0, cc = 0, nch = 0, tiles_x = 0, tiles_y = 0;
     uint32_t groups = 0;          // ceil(Cout / cpw)
     int cpw = 0;                  // output channels per wave
+    uint32_t px = 1;              // pixel groups per wave where the batch tile is 16: 1 or 2
     uint32_t lpp = 0;             // lanes per pixel (batch tile / 4) the chunk size was chosen for: 4, 2 or 1
     int2 *d_stream = nullptr;     // all groups' streams, followed by one padding quad
     uint32_t *d_gbase = nullptr;  // [groups]: first quad (4 entries) of the group's stream

@@ -312,8 +312,8 @@ class Context:
         """-> dict of the LDS-windowed kernel's parameters, or None when the plan has none."""
         out = (ct.c_uint32 * 8)()
         self._ck(self.lib.so_conv_plan_window(plan, out))
-        keys = ("tile_h", "tile_w", "window_h", "window_w", "chunk_channels", "chunks", "channels_per_wave")
-        return dict(zip(keys, out[:7])) if out[4] else None
+        keys = ("tile_h", "tile_w", "window_h", "window_w", "chunk_channels", "chunks", "channels_per_wave", "pixel_groups")
+        return dict(zip(keys, out)) if out[4] else None
 
     def upload_rbm(self, M, N, Ct_max, block_union, krel, colptr, pair_row, pair_w):
         """The flattened row-block-merged format (see so_rbm_upload) -> handle."""

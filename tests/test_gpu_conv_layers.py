@@ -139,6 +139,41 @@ def test_conv_lds_window_kernel_many_launches(ctx, oracle, Cin, Cout, H, B, sp):
         a.free()
 
 
+@pytest.mark.parametrize("Cin,Cout,H,Wi,B,s,chunks", [
+    (12, 64, 56, 56, 32, 1, 1), (40, 61, 55, 53, 16, 1, 2), (12, 128, 28, 28, 32, 1, 1), (30, 130, 29, 27, 48, 1, 2), (8, 64, 111, 113, 32, 2, 1)])
+def test_conv_window_two_pixel_groups_per_wave(ctx, oracle, Cin, Cout, H, Wi, B, s, chunks):
+    """Layers large enough for four or eight channels per wave: a wave takes both pixel groups of a tile instead, with half
+    the channels.  Channel counts that are no multiple of a workgroup's, tiles cut off at the image's edge, several chunks;
+    the same plan at the batch tiles of 8 and 4, which have one pixel group."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin + Cout + H + B)
+    Wc = sparse_matrix(rng, Cout, Cin * 9, .75)
+    Wc[3] = 0
+    Wc[4] = rng.standard_normal(Cin * 9)
+    E = datagen.encode_dense(Wc)
+    g, og = hipabi.conv_geom(Cin, Cout, 3, 3, H, Wi, (s, s), (1, 1), (1, 1)), ocg(Cin, Cout, 3, 3, H, Wi, (s, s), (1, 1), (1, 1))
+    b = rng.standard_normal(Cout).astype(np.float32)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan = ctx.conv_plan(dE, g)
+    ctx.conv_plan_tune(plan, B)
+    win = ctx.conv_plan_window(plan)
+    assert win["pixel_groups"] == 2 and win["chunks"] >= chunks, win
+    for batch in (B, 8, 4):
+        X = rng.standard_normal((Cin, H, Wi, batch)).astype(np.float32)
+        R = rng.standard_normal((Cout, g.H_out, g.W_out, batch)).astype(np.float32)
+        Yo = oracle.conv2d_pf(as_oracle(E), og, X, batch, b, "none")
+        dX, dB, dR, dY = ctx.array(X), ctx.array(b), ctx.array(R), ctx.empty(R.shape)
+        with ctx.tuning(SPARSEOPS_CONV_WINDOW="1"):
+            ctx.conv2d(plan, dX, batch, dB, dY, "none")
+            assert ctx.last_kernel() == "window" and np.array_equal(dY.download(), Yo)
+            ctx.conv2d(plan, dX, batch, dB, dY, "relu", dR)
+            assert np.array_equal(dY.download(), np.maximum(Yo + R, 0))
+        for a in (dX, dB, dR, dY):
+            a.free()
+    ctx.conv_plan_free(plan)
+    dE.free()
+
+
 @pytest.mark.parametrize("B,window", [(3, False), (4, False), (32, False), (32, True), (16, True), (8, True), (4, True)])
 def test_conv_with_fused_residual_add(ctx, oracle, B, window):
     """so_conv2d_add == conv, then the reference's Add, then the activation: same bits as
