@@ -343,7 +343,7 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
             const uint32_t rest = window_div(px, a.IW, a.mIW), iw = px - rest * a.IW;
             const uint32_t cl = window_div(rest, a.IH, a.mIH), ih = rest - cl * a.IH;
             const int32_t gh = (int32_t)(th0 * g.stride_h + ih * a.sbh) - (int32_t)g.pad_h;
-            const int32_t gw = (int32_t)(tw0 * g.stride_w + iw * a.sbw) - (int32_t)g.pad_w;
+            const int32_t gw = (int32_t)(tw0 * g.stride_w + window_column(a, iw) * a.sbw) - (int32_t)g.pad_w;
             gcl[k] = cl;
             if ((uint32_t)gh < g.H_in && (uint32_t)gw < g.W_in)
                 goff[k] = (int32_t)(((cl * g.H_in + (uint32_t)gh) * g.W_in + (uint32_t)gw) * B + bz + eb * 4u);
@@ -651,7 +651,8 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     a.win_f4 = w.cc * w.IH * w.IW * LPP;
     a.buf_f4 = (w.cc + 1) * w.IH * w.IW * LPP;
     a.nbuf = w.nch > 1 ? 2u : 1u;
-    a.sth = window_step(plan->g.kH, plan->g.stride_h); a.stw = window_step(plan->g.kW, plan->g.stride_w);
+    a.sth = window_step(plan->g.kH, plan->g.stride_h);
+    window_columns(a, w, plan->g);
     a.sbh = window_subsample(plan->g.kH, plan->g.stride_h); a.sbw = window_subsample(plan->g.kW, plan->g.stride_w);
     window_pixel_order(a, LPP);
     a.mIW = window_magic(a.IW); a.mIH = window_magic(a.IH); a.mTW = window_magic(a.TW);
@@ -771,6 +772,12 @@ so_status build_window(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32
     w.TH = bestTH; w.TW = bestTW;
     w.IH = (w.TH - 1) * window_step(g.kH, g.stride_h) + (g.kH - 1) * g.dil_h + 1;
     w.IW = (w.TW - 1) * window_step(g.kW, g.stride_w) + (g.kW - 1) * g.dil_w + 1;
+    w.PW = w.IW;
+    if (window_step(g.kW, g.stride_w) % 2u == 0 && w.IW >= window_step(g.kW, g.stride_w)) {
+        w.planes = window_step(g.kW, g.stride_w);
+        w.PW = so_ceil_div(w.IW, w.planes);
+        w.IW = (w.planes - 1) * w.PW + w.IW / w.planes;
+    }
     w.tiles_y = so_ceil_div(g.H_out, w.TH);
     w.tiles_x = so_ceil_div(g.W_out, w.TW);
     if ((uint64_t)w.IH * w.IW > 4096) return SO_OK;
@@ -841,7 +848,7 @@ so_status build_window(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32
                         const uint32_t cin = k / kHW, kh = (k / g.kW) % g.kH, kw = k % g.kW;
                         uint32_t wb;
                         std::memcpy(&wb, &Wd[slot], 4);
-                        stream[pos + e] = make_int2((int32_t)wb, (int32_t)(((cin - t * cc) * w.IH + kh * g.dil_h) * w.IW + kw * g.dil_w));
+                        stream[pos + e] = make_int2((int32_t)wb, (int32_t)(((cin - t * cc) * w.IH + kh * g.dil_h) * w.IW + window_tap_place(w, kw * g.dil_w)));
                     }
                     pos += (size_t)((n + 3u) / 4u) * 4u;
                 }
@@ -1037,11 +1044,10 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     // 16, 8 or 4 (SPARSEOPS_CONV_WINDOW=1 forces it whenever possible, =0 forbids it: tuning and tests).
     const uint32_t lpp = window_lpp(B);
     if (plan->win.cc != 0 && lpp != 0 && (align & 15) == 0 && (uint64_t)plan->win.cc * g.H_in * g.W_in * B < (1ull << 31)) {
-        // a plan that carries the row-block-merged streams runs that kernel (SPARSEOPS_CONV_RBM=0 forbids it).  It is an
-        // LDS-windowed kernel itself: SPARSEOPS_CONV_WINDOW=0 forbids it too, unless SPARSEOPS_CONV_RBM=1 asks for it.
-        if (plan->rbm.d_sets && ctx->tune.conv_rbm != 0 && (ctx->tune.conv_window != 0 || ctx->tune.conv_rbm == 1)) {
+        // the row-block-merged kernel for those who ask for it, on a plan that carries its streams
+        if (plan->rbm.d_sets && ctx->tune.conv_rbm == 1) {
             bool done = false;
-            const so_status s = so_conv_rbm_launch(ctx, plan, dX, B, dBias, dResid, dY, act, ctx->tune.conv_rbm == 1, &done);
+            const so_status s = so_conv_rbm_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done);
             if (s != SO_OK) return s;
             if (done) {
                 SO_LAUNCH_CHECK();

@@ -18,6 +18,7 @@
 // {-0.0, offset of an all-zero plane kept behind the window}: fma(-0, +0, acc) leaves any
 // accumulator as it is.
 struct so_conv_window {
+    uint32_t planes = 1, PW = 0;  // column planes of a window row (PW columns, the last ones fewer): column iw lies at iw % planes * PW + iw / planes
     uint32_t TH = 0, TW = 0, IH = 0, IW = 0, cc = 0, nch = 0, tiles_x = 0, tiles_y = 0;
     uint32_t groups = 0;          // ceil(Cout / cpw)
     int cpw = 0;                  // output channels per wave
@@ -73,7 +74,7 @@ so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const fl
 void so_conv_rbm_release(so_conv_plan *plan);
 so_status so_conv_rbm_rebuild(so_ctx *ctx, so_conv_plan *plan);
 so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
-                             const float *dResid, float *dY, int act, bool forced, bool *done);
+                             const float *dResid, float *dY, int act, bool *done);
 
 
 constexpr int kWinThreads = 1024;
@@ -86,11 +87,13 @@ inline uint32_t window_lpp(uint32_t B) { return B % 16 == 0 ? 4u : B % 8 == 0 ? 
 
 struct WinArgs {
     uint32_t TH, TW, IH, IW, cc, nch, tiles_x, pg, cg, groups;
+    uint32_t mYZ, mZ;                // window_magic of gy * gz and gz; 0 where the ids are too many for it
     uint32_t wgs, per_xcd, gy, gz;   // workgroups in all and per XCD; channel blocks and batch tiles (window_workgroup)
     uint32_t win_f4;    // float4 elements of one chunk's window
     uint32_t buf_f4;    // window plus the zero plane: stride between the two buffers
     uint32_t nbuf;      // 2: double-buffered windows; 1: a single chunk, nothing to overlap
-    uint32_t sth, stw;  // window pixels between neighbouring output pixels
+    uint32_t sth, stw;  // window pixels between neighbouring output pixels (stw: in a column plane)
+    uint32_t planes, PW, mPW;   // so_conv_window::planes, the columns of one
     uint32_t sbh, sbw;  // input pixels between neighbouring window pixels
     uint32_t order[16]; // slot -> output pixel of the tile (ty * TW + tx), one byte per slot; see window_pixel_order
     uint32_t mIW, mIH, mTW, mTilesX, mPg;   // window_magic of IW, IH, TW, tiles_x and pg: the kernels' index arithmetic divides by them
@@ -120,16 +123,39 @@ inline void window_shares(WinArgs &a, dim3 grid)
     a.wgs = grid.x * grid.y * grid.z;
     a.gy = grid.y; a.gz = grid.z;
     a.per_xcd = so_ceil_div(a.wgs, 8);
+    const uint64_t yz = (uint64_t)a.gy * a.gz;
+    a.mYZ = (uint64_t)a.wgs * yz < (1ull << 32) ? window_magic((uint32_t)yz) : 0u;
+    a.mZ = yz * a.gz < (1ull << 32) ? window_magic(a.gz) : 0u;
 }
 __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 {
     const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3), yz = a.gy * a.gz;
     if (id >= a.wgs) return false;
-    p.tile = id / yz;
+    p.tile = a.mYZ != 0u ? __umulhi(id, a.mYZ) : id / yz;
     const uint32_t rest = id - p.tile * yz;
-    p.y = rest / a.gz;
+    p.y = a.mZ != 0u ? __umulhi(rest, a.mZ) : rest / a.gz;
     p.z = rest - p.y * a.gz;
     return true;
+}
+
+// With an even stride along a row the lanes' reads of one tap would all fall on even (fourth, ...) window columns, half of the LDS's banks
+// or less: the window's columns then lie in planes, those of one remainder by the stride side by side, so that neighbouring output
+// pixels read neighbouring places.  ResNet-18-shaped layers at batch 32, one row / planes, us: stem 7x7/2 90 / 66 (80.5 on the
+// row-block-merged kernel), 3x3/2 to 28x28x128 40.2 / 34.4, to 14x14x256 39.4 / 34.4, to 7x7x512 53 / 48.8; at batch 8 the stem 26.7 (merged) / 24.7.
+//
+// The input column of place `at` of a window row, from the window's first column on.
+__device__ __forceinline__ uint32_t window_column(const WinArgs &a, uint32_t at)
+{
+    if (a.planes == 1u) return at;
+    const uint32_t plane = window_div(at, a.PW, a.mPW);
+    return (at - plane * a.PW) * a.planes + plane;
+}
+// The same for a tap: where column kw of a tap lies, from an output pixel's corner on.
+inline uint32_t window_tap_place(const so_conv_window &w, uint32_t kw) { return kw % w.planes * w.PW + kw / w.planes; }
+inline void window_columns(WinArgs &a, const so_conv_window &w, const so_conv_geom &g)
+{
+    a.planes = w.planes; a.PW = w.PW; a.mPW = window_magic(a.PW);
+    a.stw = window_step(g.kW, g.stride_w) / w.planes;
 }
 
 // Which output pixel of the tile each pixel slot of the workgroup computes (slot = lanes / lanes per

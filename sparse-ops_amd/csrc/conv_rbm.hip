@@ -269,7 +269,7 @@ void conv2d_rbm_kernel(const int4 *__restrict__ sets, const uint32_t *__restrict
             const uint32_t rest = window_div(px, a.IW, a.mIW), iw = px - rest * a.IW;
             const uint32_t cl = window_div(rest, a.IH, a.mIH), ih = rest - cl * a.IH;
             const int32_t gh = (int32_t)(th0 * g.stride_h + ih * a.sbh) - (int32_t)g.pad_h;
-            const int32_t gw = (int32_t)(tw0 * g.stride_w + iw * a.sbw) - (int32_t)g.pad_w;
+            const int32_t gw = (int32_t)(tw0 * g.stride_w + window_column(a, iw) * a.sbw) - (int32_t)g.pad_w;
             gcl[k] = cl;
             if ((uint32_t)gh < g.H_in && (uint32_t)gw < g.W_in)
                 goff[k] = (int32_t)(((cl * g.H_in + (uint32_t)gh) * g.W_in + (uint32_t)gw) * B + bz + eb * 4u);
@@ -389,18 +389,6 @@ void rbm_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, siz
 #undef SO_RBM_LAUNCH
 }
 
-// A wave of this kernel owns a whole block of channels, so a launch has an eighth of the waves the
-// per-row kernel can spread over the chip: it needs a grid that covers about three quarters of the
-// compute units (28x28x128 at batch 32, 112 workgroups: 113 against 66 us).  With such a grid it is
-// level with the per-row kernel on stride-1 layers (ResNet-18 shapes, 3x3: 56x56x64 at batch 32 64.4
-// against 62.9 us, at batch 128 256 against 258; 28x28x128 at batch 128 224 against 219) and ahead
-// on strided ones (7x7 stride-2 stem 87 against 99 us at batch 32, 299 against 339 at batch 128;
-// 3x3 stride-2 56->28 at batch 64 71 against 80; 1x1 stride-2 18 against 19): it runs there.
-bool rbm_pays(const so_ctx *ctx, const so_conv_geom &g, uint64_t workgroups)
-{
-    return 4ull * workgroups >= 3ull * (uint64_t)ctx->compute_units && (g.stride_h > 1 || g.stride_w > 1);
-}
-
 } // namespace
 
 // ------------------------------------------------------------------ streams of a plan
@@ -442,7 +430,7 @@ so_status so_conv_rbm_rebuild(so_ctx *ctx, so_conv_plan *plan)
             for (; u < u_end && R->krel[u] / kHW / w.cc == t; ++u) {
                 const uint32_t k = R->krel[u];
                 const uint32_t cin = k / kHW, kh = (k / g.kW) % g.kH, kw = k % g.kW;
-                const uint32_t off = ((cin - t * w.cc) * w.IH + kh * g.dil_h) * w.IW + kw * g.dil_w;
+                const uint32_t off = ((cin - t * w.cc) * w.IH + kh * g.dil_h) * w.IW + window_tap_place(w, kw * g.dil_w);
                 for (uint32_t p = R->colptr[u]; p < R->colptr[u + 1]; p += kRbmSlots) {
                     RbmRecord rec = padrec;
                     rec.off_next = off;
@@ -534,11 +522,12 @@ extern "C" so_status so_conv_plan_rbm_info(const so_conv_plan *plan, uint64_t ou
     return SO_OK;
 }
 
-// Launches the RBM kernel if the plan carries its streams, the batch suits the windowed layout and
-// (unless `forced`) the launch is one on which it beats the per-row windowed kernel; *done says
-// whether it did.
+// Launches the RBM kernel if the plan carries its streams and the batch suits the windowed layout; *done says whether it did.
+// For those who ask for it (SPARSEOPS_CONV_RBM=1): the per-row windowed kernel is faster everywhere it was measured since its waves take
+// two pixel groups and strided windows lie in column planes.  Us, this one / that one, ResNet-18-shaped layers: 7x7/2 stem at batch 32 and
+// 50 / 80 / 90 % sparse 144 / 115, 84 / 66, 64 / 54, at batch 64 and 60 % 220 / 179, at batch 8 and 80 % 28.2 / 24.7; 56x56x64 at batch 64 and 75 % 144 / 103.
 so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
-                             const float *dResid, float *dY, int act, bool forced, bool *done)
+                             const float *dResid, float *dY, int act, bool *done)
 {
     *done = false;
     const so_conv_window &w = plan->win;
@@ -554,7 +543,8 @@ so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float 
     a.win_f4 = w.cc * w.IH * w.IW * LPP;
     a.buf_f4 = (w.cc + 1) * w.IH * w.IW * LPP;
     a.nbuf = w.nch > 1 ? 2u : 1u;
-    a.sth = window_step(plan->g.kH, plan->g.stride_h); a.stw = window_step(plan->g.kW, plan->g.stride_w);
+    a.sth = window_step(plan->g.kH, plan->g.stride_h);
+    window_columns(a, w, plan->g);
     a.sbh = window_subsample(plan->g.kH, plan->g.stride_h); a.sbw = window_subsample(plan->g.kW, plan->g.stride_w);
     window_pixel_order(a, LPP);
     a.mIW = window_magic(a.IW); a.mIH = window_magic(a.IH); a.mTW = window_magic(a.TW);
@@ -567,7 +557,6 @@ so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float 
     const dim3 grid(w.tiles_x * w.tiles_y, so_ceil_div(a.groups, a.cg), B / (4 * LPP));
     if (grid.y > 65535u || grid.z > 65535u || (uint64_t)grid.x * grid.y * grid.z >= (1ull << 31)) return SO_OK;
     window_shares(a, grid);
-    if (!forced && !rbm_pays(ctx, plan->g, (uint64_t)grid.x * grid.y * grid.z)) return SO_OK;
     switch (LPP) {
     case 4:  rbm_launch_act<4>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
     case 2:  rbm_launch_act<2>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;

@@ -458,7 +458,8 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     std::size_t bias_total = 0;
     // Large fully connected layers run on the RBM layout's kernels (fp32 round-off accuracy, the fastest);
     // SPARSEOPS_MATMUL_RBM=0 at load time keeps every layer on the kernels that give the reference's bits.
-    const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM");
+    const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM"), *conv_rbm_env = std::getenv("SPARSEOPS_CONV_RBM");
+    const bool conv_rbm = conv_rbm_env && conv_rbm_env[0] == '1';
     // So does a model with convolutions that is loaded at a batch below 64, whatever batch it is resized to later: its
     // samples have the same bits in every batch, and its classifier is a few microseconds of the pass.  Loaded at 64 or
     // more it keeps the fast layers at every batch, and a sample's bits then depend on the batch (the kernel is chosen
@@ -473,9 +474,8 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
             check(so_conv_plan_create(ctx, p.plan.dE, &p.plan.cg, &p.plan.conv), "so_conv_plan_create");
             // The reference builds its row-block-merged plan for wide convolutions at load
             // (src/sparse_onnx.cpp:499-502: Cout >= 32 and K >= 64, blocks of 8 channels) and never
-            // runs it; here the plan goes to the device library, whose so_conv2d walks it wherever
-            // that is the faster kernel for the batch at hand.
-            if (p.plan.cg.Cout >= 32 && p.plan.E->n >= 64) {
+            // runs it; here it is built for those who ask so_conv2d to walk it, which the windowed kernel beats.
+            if (conv_rbm && p.plan.cg.Cout >= 32 && p.plan.E->n >= 64) {
                 p.plan.rbm = upload_rbm(build_rbm_from_ellpack(*p.plan.E, nullptr, 8));
                 check(so_conv_plan_set_rbm(ctx, p.plan.conv, p.plan.rbm), "so_conv_plan_set_rbm");
             }

@@ -174,6 +174,36 @@ def test_conv_window_two_pixel_groups_per_wave(ctx, oracle, Cin, Cout, H, Wi, B,
     dE.free()
 
 
+@pytest.mark.parametrize("Cin,Cout,H,Wi,B,k,s,p,d", [
+    (8, 33, 21, 23, 16, (3, 3), (2, 2), (1, 1), (1, 1)), (5, 40, 30, 41, 16, (5, 5), (4, 4), (2, 2), (1, 1)), (6, 32, 19, 33, 8, (3, 3), (2, 2), (2, 2), (2, 3)),
+    (9, 36, 17, 2, 4, (3, 2), (1, 2), (1, 0), (1, 1)), (4, 32, 26, 40, 32, (2, 7), (3, 6), (0, 3), (1, 1)), (7, 64, 15, 29, 16, (3, 4), (2, 2), (1, 2), (1, 2))])
+def test_conv_window_column_planes(ctx, oracle, Cin, Cout, H, Wi, B, k, s, p, d):
+    """Strides of 2, 4 and 6 along a row: the window's columns lie in as many planes.  Window rows that the planes do not
+    divide evenly, rows shorter than a stride, dilated taps; the same window under the row-block-merged kernel."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin * Cout + Wi)
+    E = datagen.encode_dense(sparse_matrix(rng, Cout, Cin * k[0] * k[1], .5))
+    g, og = hipabi.conv_geom(Cin, Cout, k[0], k[1], H, Wi, s, p, d), ocg(Cin, Cout, k[0], k[1], H, Wi, s, p, d)
+    X, b = rng.standard_normal((Cin, H, Wi, B)).astype(np.float32), rng.standard_normal(Cout).astype(np.float32)
+    Yo = oracle.conv2d_pf(as_oracle(E), og, X, B, b, "relu")
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan = ctx.conv_plan(dE, g)
+    ctx.conv_plan_tune(plan, B)
+    R = oracle.rbm_build(as_oracle(E), 8)
+    rbm = ctx.upload_rbm(R.M, R.N, R.Ct_max, R.block_union, R.krel, R.colptr, R.pair_row, R.pair_w)
+    ctx.conv_plan_set_rbm(plan, rbm)
+    dX, dB, dY = ctx.array(X), ctx.array(b), ctx.empty(Yo.shape)
+    for tuning, kernel in (({"SPARSEOPS_CONV_WINDOW": "1"}, "window"), ({"SPARSEOPS_CONV_RBM": "1"}, "merged-window")):
+        with ctx.tuning(**tuning):
+            ctx.conv2d(plan, dX, B, dB, dY, "relu")
+        assert ctx.last_kernel() == kernel and np.array_equal(dY.download(), Yo)
+    ctx.conv_plan_free(plan)
+    ctx.rbm_free(rbm)
+    dE.free()
+    for a in (dX, dB, dY):
+        a.free()
+
+
 @pytest.mark.parametrize("B,window", [(3, False), (4, False), (32, False), (32, True), (16, True), (8, True), (4, True)])
 def test_conv_with_fused_residual_add(ctx, oracle, B, window):
     """so_conv2d_add == conv, then the reference's Add, then the activation: same bits as
