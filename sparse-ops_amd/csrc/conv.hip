@@ -315,6 +315,12 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     const uint32_t bz = place.z * BT;
     const bool computes = cgi < a.cg && grp < a.groups;              // the other waves only help copying
     const uint32_t gi = computes ? grp : 0u;
+    // Asked for first: the stream's place, on which its first entries wait.
+    const uint32_t first_quad = gbase[gi];
+    const uint32_t *__restrict__ qp = quads + (size_t)gi * a.nch * CPW;
+    uint32_t qfirst[CPW];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) qfirst[c] = qp[c];
 
     // this lane's output pixels and their corners inside the window
     const uint32_t b4 = lane % LPP;
@@ -367,22 +373,6 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
             if (gcl[k] != 0xffffffffu) win_lds[buf * a.buf_f4 + tid + (uint32_t)k * kWinThreads] = xr[k];
     };
 
-    float acc[CPW][PX][4];
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-        const float b0 = (bias && computes && co0 + c < g.Cout) ? bias[co0 + c] : 0.0f;
-#pragma unroll
-        for (int x = 0; x < PX; ++x) acc[c][x][0] = acc[c][x][1] = acc[c][x][2] = acc[c][x][3] = b0;
-    }
-
-    // the all-zero plane behind each window buffer (padding entries point into it)
-    for (uint32_t i = tid; i < a.buf_f4 - a.win_f4; i += kWinThreads) {
-        win_lds[a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (a.nbuf == 2) win_lds[a.buf_f4 + a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    // progress counters behind the buffers: [0], [1] windows stored into buffer 0 / 1 (x 16 waves), [2], [3] chunks read out of them
-    const uint32_t sync_base = so_lds::lds_address(win_lds + (size_t)a.nbuf * a.buf_f4);
-    if (a.nbuf == 2 && tid < 4) reinterpret_cast<uint32_t *>(win_lds + (size_t)a.nbuf * a.buf_f4)[tid] = tid == 0 ? 16u : 0u;
     fetch_window(0);                  // stored below, once the entry stream is set up: the two latencies overlap
 
     // The wave's entry stream: one quad = 4 entries = two int4 {w0, o0, w1, o1}, {w2, o2, w3, o3}.
@@ -392,9 +382,8 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     // assembly of touch_stream)
     typedef int i32x4 __attribute__((ext_vector_type(4)));
     typedef const i32x4 __attribute__((address_space(4))) *const_stream;
-    const int4 *__restrict__ sp0 = stream + 2 * (size_t)gbase[gi];
+    const int4 *__restrict__ sp0 = stream + 2 * (size_t)first_quad;
     const_stream sp = (const_stream)(uintptr_t)sp0;
-    const uint32_t *__restrict__ qp = quads + (size_t)gi * a.nch * CPW;
     i32x4 cur0 = {0, 0, 0, 0}, cur1 = cur0;
     // LANE_ENT: the entries sit in lanes instead (lane l of every 16-lane row holds entry l of the
     // next 16), fetched with vector loads one group ahead and broadcast by DPP: vector loads have
@@ -416,13 +405,29 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     } else {
         if (computes) {
 #pragma unroll
-            for (int c = 0; c < CPW; ++c) qtouch += qp[c];
+            for (int c = 0; c < CPW; ++c) qtouch += qfirst[c];
         }
         touch_stream(sp0, qtouch + 1u, pgi, a.pg);
         cur0 = sp[0];
         cur1 = sp[1];
         sp += 2;
     }
+    float acc[CPW][PX][4];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) {
+        const float b0 = (bias && computes && co0 + c < g.Cout) ? bias[co0 + c] : 0.0f;
+#pragma unroll
+        for (int x = 0; x < PX; ++x) acc[c][x][0] = acc[c][x][1] = acc[c][x][2] = acc[c][x][3] = b0;
+    }
+
+    // the all-zero plane behind each window buffer (padding entries point into it)
+    for (uint32_t i = tid; i < a.buf_f4 - a.win_f4; i += kWinThreads) {
+        win_lds[a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (a.nbuf == 2) win_lds[a.buf_f4 + a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    // progress counters behind the buffers: [0], [1] windows stored into buffer 0 / 1 (x 16 waves), [2], [3] chunks read out of them
+    const uint32_t sync_base = so_lds::lds_address(win_lds + (size_t)a.nbuf * a.buf_f4);
+    if (a.nbuf == 2 && tid < 4) reinterpret_cast<uint32_t *>(win_lds + (size_t)a.nbuf * a.buf_f4)[tid] = tid == 0 ? 16u : 0u;
     store_window(0);
     __syncthreads();
 
@@ -773,7 +778,7 @@ so_status build_window(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32
     w.IH = (w.TH - 1) * window_step(g.kH, g.stride_h) + (g.kH - 1) * g.dil_h + 1;
     w.IW = (w.TW - 1) * window_step(g.kW, g.stride_w) + (g.kW - 1) * g.dil_w + 1;
     w.PW = w.IW;
-    if (window_step(g.kW, g.stride_w) % 2u == 0 && w.IW >= window_step(g.kW, g.stride_w)) {
+    if (window_step(g.kW, g.stride_w) % 2u == 0 && w.IW > window_step(g.kW, g.stride_w)) {
         w.planes = window_step(g.kW, g.stride_w);
         w.PW = so_ceil_div(w.IW, w.planes);
         w.IW = (w.planes - 1) * w.PW + w.IW / w.planes;

@@ -87,7 +87,7 @@ inline uint32_t window_lpp(uint32_t B) { return B % 16 == 0 ? 4u : B % 8 == 0 ? 
 
 struct WinArgs {
     uint32_t TH, TW, IH, IW, cc, nch, tiles_x, pg, cg, groups;
-    uint32_t mYZ, mZ;                // window_magic of gy * gz and gz; 0 where the ids are too many for it
+    uint32_t mYZ, mZ;                // window_magic of gy * gz and gz; mYZ is 0 where that is 1 or the ids are too many
     uint32_t wgs, per_xcd, gy, gz;   // workgroups in all and per XCD; channel blocks and batch tiles (window_workgroup)
     uint32_t win_f4;    // float4 elements of one chunk's window
     uint32_t buf_f4;    // window plus the zero plane: stride between the two buffers
@@ -125,16 +125,24 @@ inline void window_shares(WinArgs &a, dim3 grid)
     a.per_xcd = so_ceil_div(a.wgs, 8);
     const uint64_t yz = (uint64_t)a.gy * a.gz;
     a.mYZ = (uint64_t)a.wgs * yz < (1ull << 32) ? window_magic((uint32_t)yz) : 0u;
-    a.mZ = yz * a.gz < (1ull << 32) ? window_magic(a.gz) : 0u;
+    if (yz * a.gz >= (1ull << 32)) a.mYZ = 0u;
+    a.mZ = window_magic(a.gz);
 }
 __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 {
     const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3), yz = a.gy * a.gz;
     if (id >= a.wgs) return false;
-    p.tile = a.mYZ != 0u ? __umulhi(id, a.mYZ) : id / yz;
-    const uint32_t rest = id - p.tile * yz;
-    p.y = a.mZ != 0u ? __umulhi(rest, a.mZ) : rest / a.gz;
-    p.z = rest - p.y * a.gz;
+    if (a.mYZ != 0u) {
+        p.tile = __umulhi(id, a.mYZ);
+        const uint32_t rest = id - p.tile * yz;
+        p.y = a.gz == 1u ? rest : __umulhi(rest, a.mZ);
+        p.z = rest - p.y * a.gz;
+    } else {
+        p.tile = id / yz;
+        const uint32_t rest = id - p.tile * yz;
+        p.y = rest / a.gz;
+        p.z = rest - p.y * a.gz;
+    }
     return true;
 }
 
@@ -146,15 +154,14 @@ __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 // The input column of place `at` of a window row, from the window's first column on.
 __device__ __forceinline__ uint32_t window_column(const WinArgs &a, uint32_t at)
 {
-    if (a.planes == 1u) return at;
-    const uint32_t plane = window_div(at, a.PW, a.mPW);
+    const uint32_t plane = __umulhi(at, a.mPW);                      // mPW is 0 for a single plane
     return (at - plane * a.PW) * a.planes + plane;
 }
 // The same for a tap: where column kw of a tap lies, from an output pixel's corner on.
 inline uint32_t window_tap_place(const so_conv_window &w, uint32_t kw) { return kw % w.planes * w.PW + kw / w.planes; }
 inline void window_columns(WinArgs &a, const so_conv_window &w, const so_conv_geom &g)
 {
-    a.planes = w.planes; a.PW = w.PW; a.mPW = window_magic(a.PW);
+    a.planes = w.planes; a.PW = w.PW; a.mPW = w.planes > 1 ? window_magic(a.PW) : 0u;
     a.stw = window_step(g.kW, g.stride_w) / w.planes;
 }
 
