@@ -147,4 +147,40 @@ __device__ __forceinline__ void group_drain(float ewp, const float4 (&xB)[4], fl
     quad_fma<12>(ewp, xB, acc);
 }
 
+// ---- one column per lane ---------------------------------------------------------------
+//
+// The four multiply-adds of one quad of entries (weights in lanes N1 .. N1 + 3 of w, operands in xf) between the four
+// address adds of another (offsets in lanes N0 .. of off), then that one's LDS reads (to xr): a multiply-add of the
+// chain may follow the one before it after 9 clocks, and the adds fill that time.
+template <int N0, int N1>
+__device__ __forceinline__ void step4(uint32_t base, uint32_t off, float (&xr)[4], float w, const float (&xf)[4], float &acc)
+{
+    uint32_t p0, p1, p2, p3;
+    asm("v_add_u32_dpp %[p0], %[off], %[base] row_newbcast:%[n0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x0] row_newbcast:%[m0] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p1], %[off], %[base] row_newbcast:%[n1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x1] row_newbcast:%[m1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p2], %[off], %[base] row_newbcast:%[n2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x2] row_newbcast:%[m2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_u32_dpp %[p3], %[off], %[base] row_newbcast:%[n3] row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %[acc], %[w], %[x3] row_newbcast:%[m3] row_mask:0xf bank_mask:0xf"
+        : [p0] "=&v"(p0), [p1] "=&v"(p1), [p2] "=&v"(p2), [p3] "=&v"(p3), [acc] "+v"(acc)
+        : [off] "v"(off), [base] "v"(base), [w] "v"(w), [x0] "v"(xf[0]), [x1] "v"(xf[1]), [x2] "v"(xf[2]), [x3] "v"(xf[3]),
+          [n0] "n"(N0), [n1] "n"(N0 + 1), [n2] "n"(N0 + 2), [n3] "n"(N0 + 3), [m0] "n"(N1), [m1] "n"(N1 + 1), [m2] "n"(N1 + 2), [m3] "n"(N1 + 3));
+    typedef const float __attribute__((address_space(3))) *lds_float;
+    xr[0] = *(lds_float)p0;
+    xr[1] = *(lds_float)p1;
+    xr[2] = *(lds_float)p2;
+    xr[3] = *(lds_float)p3;
+    __builtin_amdgcn_sched_barrier(0);
+}
+template <int N1>
+__device__ __forceinline__ void fma4(float w, const float (&x)[4], float &acc)
+{
+    fmac_bcast<N1>(acc, w, x[0]);
+    fmac_bcast<N1 + 1>(acc, w, x[1]);
+    fmac_bcast<N1 + 2>(acc, w, x[2]);
+    fmac_bcast<N1 + 3>(acc, w, x[3]);
+}
+
 } // namespace so_dpp

@@ -283,6 +283,20 @@ so_status launch_shared_gather(so_ctx *ctx, const so_ellpack *E, const float *dX
 
 namespace {
 
+// The kernel with X in LDS (csrc/matmul_columns.hip) in place of the row and shared-gather kernels, whose bits it gives: wherever it applies and
+// the longest row has kColumnsNnz nonzeros.  Us, row or shared-gather kernel / this one, one handle launched again and again: 1000 x 512 dense, 32 columns, in
+// the ResNet-18-shaped stack 17.4 / 8.2, one column 17.5 / 7.6; 1337 x 2085 x 1 with rows of 383 12.4 / 6.2; 489 x 4566 x 4, 2033 39.7 / 23.6; 12 x 5634 x 1,
+// 1164 19.2 / 14.2; 17843 x 7108 x 4, 1561 269 / 73; 315 x 140 x 34, 112 5.0 / 4.2; 4634 x 58 x 4, 15 3.6 / 3.5; shorter rows are as fast there, or faster where
+// there are many: 1357 x 26 x 8, 25 4.2 / 4.6, 2120 x 254 x 3, 42 4.3 / 4.7, but 13730 x 105 x 8, 62 8.8 / 4.5.
+constexpr uint32_t kColumnsNnz = 48;
+
+bool columns_pays(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    if (ctx->tune.matmul_columns >= 0) return ctx->tune.matmul_columns == 1 && so_matmul_columns_applies(ctx, E, C);
+    // (an override that asks for one of the row kernels' forms stands)
+    return ctx->tune.matmul_share < 0 && ctx->tune.matmul_vec == 0 && E->max_nnz >= kColumnsNnz && so_matmul_columns_applies(ctx, E, C);
+}
+
 enum class RbmKernel { None, Merged, Quad, Vector, Planes, Narrow };
 
 // Which of the kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
@@ -315,6 +329,7 @@ RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
     *us = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
+    if (columns_pays(ctx, E, C)) *us = std::min(*us, so_matmul_columns_estimate(ctx, E, C));
     RbmKernel k = RbmKernel::None;
     if (merged) {
         // one workgroup per (128 rows, 64 columns, share of the columns): pays when that grid covers most of the chip
@@ -448,6 +463,14 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
         if (st != SO_OK) return st;
         SO_LAUNCH_CHECK();
         ctx->last_kernel = "tiled";
+        return SO_OK;
+    }
+
+    if (dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0 && columns_pays(ctx, E, C)) {
+        const so_status st = so_matmul_columns_launch(ctx, E, dX, C, dBias, dY, act);
+        if (st != SO_OK) return st;
+        SO_LAUNCH_CHECK();
+        ctx->last_kernel = "columns";
         return SO_OK;
     }
 

@@ -66,6 +66,7 @@ static void read_tuning(so_tuning &t)
     t.matmul_tiled = env_int("SPARSEOPS_MATMUL_TILED", -1);
     t.matmul_vec = env_int("SPARSEOPS_MATMUL_VEC", 0);
     t.matmul_share = env_int("SPARSEOPS_MATMUL_SHARE", -1);
+    t.matmul_columns = env_int("SPARSEOPS_MATMUL_COLUMNS", -1);
     t.matmul_rbm = env_int("SPARSEOPS_MATMUL_RBM", -1);
     t.matmul_rbm_split = env_int("SPARSEOPS_MATMUL_RBM_SPLIT", 0);
     t.matmul_quad = env_int("SPARSEOPS_MATMUL_QUAD", -1);

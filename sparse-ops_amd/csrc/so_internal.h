@@ -17,6 +17,7 @@ struct so_tuning {
     int matmul_tiled = -1;   // SPARSEOPS_MATMUL_TILED: 1 forces the LDS-staged kernel, 0 forbids it
     int matmul_vec = 0;      // SPARSEOPS_MATMUL_VEC: 1 or 2 columns per lane at most
     int matmul_share = -1;   // SPARSEOPS_MATMUL_SHARE: 0 forbids the shared-gather kernel for few-row launches
+    int matmul_columns = -1; // SPARSEOPS_MATMUL_COLUMNS: 0 forbids the kernel with X in LDS for few columns, 1 forces it where it applies
     int matmul_rbm = -1;     // SPARSEOPS_MATMUL_RBM: 0 forbids every kernel that is only for handles with the RBM layout, 1 forces the row-block-merged one
     int matmul_rbm_split = 0;   // SPARSEOPS_MATMUL_RBM_SPLIT: 1, 2 or 4 workgroups per tile for RBM layouts built from now on
     int matmul_quad = -1;    // SPARSEOPS_MATMUL_QUAD: 0 forbids the quad-union kernel on handles with the RBM layout, 1 forces it
@@ -192,6 +193,11 @@ void so_set_error(const char *fmt, ...);
 // csrc/matmul_tiled.hip: launches the LDS-staged kernel on E's TILED copy (the caller has checked that it applies).
 so_status so_matmul_tiled_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C,
                                  const float *dBias, float *dY, int act);
+
+// csrc/matmul_columns.hip: at most 64 dense columns with X in LDS, in the row kernels' order.
+bool so_matmul_columns_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+double so_matmul_columns_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C);      // us
+so_status so_matmul_columns_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
 
 // csrc/matmul_rbm.hip: the row-block-merged layout and its kernel.
 so_status so_rbmm_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint32_t *idx, const uint32_t *nnz);
