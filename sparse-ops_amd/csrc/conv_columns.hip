@@ -9,15 +9,17 @@
 //
 // Decomposition.  A workgroup of G (16, 8 or 4) waves takes G channels on one tile.  The tile's input window -- all
 // input channels if 150 KB of LDS hold them, else a chunk at a time -- is copied to LDS with zeros outside the image; a
-// channel's entries {weight, LDS offset of its tap} come 16 at a time in lanes (the same 16 in every row of 16), four
-// such groups ahead, and are handed round by DPP: per entry one address add, one read, one multiply-add.  The reads run
+// channel's entries {weight, LDS offset of its tap} come 16 at a time in lanes (the same 16 in every row of 16), eight
+// such groups ahead, each group's place asked for again when it is done, and are handed round by DPP: per entry one address add, one read, one multiply-add.  The reads run
 // three quads of entries ahead of the multiply-adds.  Workgroups shrink to 8 or 4 waves where that spreads the launch
 // over more compute units.
 //
-// What bounds it: what one wave alone on a SIMD issues, about 5.8 clocks an instruction -- 18 an entry in a loop of nothing else, 23 with the entries'
-// loads, groups and waits (two, three or four quads of reads in flight: the same).  A ResNet-18-shaped 7 x 7 x 512 layer at 80 %, chains of 922:
-// 9.0 us of its 15.9; before them 3.0 us in which 16 waves issue the window's 592 copies, 12 clocks each (beginning in another place in each
-// workgroup: 1.5 us slower), 1 until all is there, 0.6 of arguments and places, and the launch.
+// What bounds it: what one wave alone on a SIMD issues, about 5.8 clocks an instruction -- 18 clocks an entry in a loop of nothing else.  With
+// four groups of entries ahead, asked for together, the loop's end waited for memory and the entry took 23; with eight, a place
+// at a time, the ResNet-18-shaped stack at batch 1 takes 216.7 us instead of 230.8, a 7 x 7 x 512 layer (chains of 922) 14.4 instead of 16.2, a
+// 14 x 14 x 256 one 9.8 instead of 11.0.  Before the chain come 3.0 us in which 16 waves issue the window's 592 copies, 12 clocks each (beginning in
+// another place in each workgroup: 1.5 us slower; 16 bytes a lane instead of 4, with the pads cleared afterwards: 217.7 us for the stack), 1 until
+// all is there, 0.6 of arguments and places, and the launch.
 #include "so_internal.h"
 #include "conv_internal.h"
 #include "dpp_steps.h"
@@ -40,6 +42,20 @@ struct ColArgs {
 using so_dpp::fma4;
 using so_dpp::step4;
 
+constexpr uint32_t kAhead = 8;   // groups of entries a wave has asked for
+
+// step(0) .. step(left - 1), at most kAhead - 1 of them.
+template <uint32_t I, class F>
+__device__ __forceinline__ void rest(uint32_t left, F &&step)
+{
+    if constexpr (I + 1u < kAhead) {
+        if (left > I) {
+            step(I);
+            rest<I + 1u>(left, step);
+        }
+    }
+}
+
 template <int ACT>
 __global__ __launch_bounds__(1024)
 void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__restrict__ first_group, ColArgs a, so_conv_geom g,
@@ -54,11 +70,11 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
     const uint32_t tile_y = window_div(blockIdx.x, a.tiles_x, a.mTilesX);
     const uint32_t th0 = tile_y * a.TH, tw0 = (blockIdx.x - tile_y * a.tiles_x) * a.TW;
 
-    // The wave's entries, groups of 16 (the stream ends with eight padding groups).  At a pitch their place needs no look
+    // The wave's entries, groups of 16 (the stream ends with kAhead padding groups).  At a pitch their place needs no look
     // into a table, whose round trip to memory -- nothing is cached when a kernel starts -- would come before theirs.
     const uint32_t run0 = (computes ? co : 0u) * a.nch;
-    const int2 *__restrict__ ep = entries + (lane & 15u);
-    int2 cur[4], nxt[4];
+    const uint32_t l16 = lane & 15u;
+    int2 held[kAhead];
     uint32_t g0, g1;
     auto first_entries = [&](uint32_t t) {
         if (a.pitch != 0u) {
@@ -68,9 +84,9 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
             g0 = __builtin_amdgcn_readfirstlane(first_group[run0 + t]);
             g1 = __builtin_amdgcn_readfirstlane(first_group[run0 + t + 1u]);
         }
-        if (!computes) g1 = 0u;
+        if (!computes) g1 = g0;
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) cur[i] = ep[(size_t)(g0 + i) * 16u];
+        for (uint32_t i = 0; i < kAhead; ++i) held[i] = (entries + (size_t)g0 * 16u)[i * 16u + l16];
     };
     first_entries(0);
 
@@ -138,16 +154,17 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
         copy_window(t);
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");             // this thread's part of the window is in LDS
         __syncthreads();
-        for (uint32_t gi = g0; gi < g1; gi += 4u) {
+        // (no way out of the loop's middle: the compiler joins it to the loop's end, and every wait is then for all loads)
+        const int2 *__restrict__ ahead = entries + (size_t)(g0 + kAhead) * 16u;
+        uint32_t left = g1 - g0;
+        for (; left >= kAhead; left -= kAhead, ahead += kAhead * 16u) {
 #pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) nxt[i] = ep[(size_t)(gi + 4u + i) * 16u];
-            group(cur[0]);
-            if (gi + 1u < g1) group(cur[1]);
-            if (gi + 2u < g1) group(cur[2]);
-            if (gi + 3u < g1) group(cur[3]);
-#pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) cur[i] = nxt[i];
+            for (uint32_t i = 0; i < kAhead; ++i) {
+                group(held[i]);
+                held[i] = ahead[i * 16u + l16];
+            }
         }
+        rest<0>(left, [&](uint32_t i) { group(held[i]); });
     }
     asm volatile("s_nop 4" : "+v"(owed));
     fma4<4>(owed, xB, acc);
@@ -234,7 +251,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
     uint32_t pad_bits;
     const float neg_zero = -0.0f;
     std::memcpy(&pad_bits, &neg_zero, 4);
-    std::vector<int2> entries((size_t)total * 16 + 128, make_int2((int)pad_bits, (int)(c.cc * plane * 4)));
+    std::vector<int2> entries(((size_t)total + kAhead) * 16, make_int2((int)pad_bits, (int)(c.cc * plane * 4)));
     size_t next = 0;                            // group
     for (uint32_t co = 0; co < E->m; ++co) {
         uint32_t j = 0;

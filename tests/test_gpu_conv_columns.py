@@ -57,6 +57,33 @@ def test_columns_match_oracle(ctx, oracle, Cin, Cout, H, Wi, k, s, p, d, sp, B):
             a.free()
 
 
+@pytest.mark.parametrize("Cin,H", [(34, 9), (400, 18)])            # one chunk and several
+def test_columns_groups_per_run(ctx, oracle, Cin, H):
+    """Runs of no group of 16 entries up to three blocks of eight, one entry more or fewer: what a block, the rest behind it
+    and the groups asked for ahead come to."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin)
+    lengths = [n for k in (0, 1, 6, 7, 8, 9, 15, 16, 17) for n in (16 * k - 1, 16 * k, 16 * k + 1) if n >= 0]
+    Wc = np.zeros((len(lengths), Cin * 9), np.float32)
+    for row, n in zip(Wc, lengths):
+        row[rng.choice(Cin * 9, n, replace=False)] = rng.standard_normal(n)
+    E = datagen.encode_dense(Wc)
+    args = Cin, len(lengths), 3, 3, H, H, (1, 1), (1, 1), (1, 1)
+    g, og = hipabi.conv_geom(*args), ocg(*args)
+    X = rng.standard_normal((Cin, H, H, 1)).astype(np.float32)
+    with ctx.tuning(SPARSEOPS_CONV_COLUMNS="1"):
+        dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+        plan = ctx.conv_plan(dE, g)
+        ctx.conv_plan_tune(plan, 1)
+        dX, dY = ctx.array(X), ctx.empty((len(lengths), H, H, 1))
+        ctx.conv2d(plan, dX, 1, None, dY, "none")
+        assert ctx.last_kernel() == "columns"
+        assert np.array_equal(dY.download(), oracle.conv2d_pf(as_oracle(E), og, X, 1, None, "none"))
+        ctx.conv_plan_free(plan)
+        for a in (dX, dY, dE):
+            a.free()
+
+
 @pytest.mark.parametrize("ordered", [True, False])
 def test_streams_are_made_once_per_batch_and_kept(ctx, oracle, ordered):
     """Tuning for one small batch after another neither takes away the streams that a recorded graph replays with nor makes
