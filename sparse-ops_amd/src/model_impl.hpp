@@ -67,11 +67,14 @@ struct SparseOnnxModel::Impl {
     sparseops::DeviceBuffer stage_in, stage_out;  // staging for the caller's layouts (batch-major, or unpadded rows)
     sparseops::DeviceBuffer stage_mid;            // [features x batch] between a transpose and the padded arena rows
     so_graph *graph = nullptr;           // recorded layer chain (arena -> arena)
-    bool use_graph = true;
+    int use_graph = -1;                  // 1: always recorded, 0: never, -1: where record_pays says so
 
     ~Impl();
     float *slot_ptr(int s) const { return arena.f32() + slots[s].offset; }
-    void enqueue_layers() const;                             // one launch per layer, arena slot to arena slot
+    // One launch per layer, arena slot to arena slot; the model's input and output in the caller's memory where given.
+    void enqueue_layers(const float *in = nullptr, float *out = nullptr) const;
+    std::size_t output_layer() const;                        // the layer that makes the model's output; layers.size(): none does
+    bool record_pays() const;
     void launch_chain() const;                               // graph replay or eager
     bool padded() const { return pbatch != batch; }
     void rows_in(const float *d_rows) const;                 // [in_features x batch] -> the input slot (rows padded with zeros)

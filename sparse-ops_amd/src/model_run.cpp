@@ -48,7 +48,7 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
         // launch graph cannot be recorded across an allocation)
         else if (L.op == Op::MatMul && L.dE) check(so_matmul_reserve(ctx, L.dE, pbatch), "so_matmul_reserve");
     }
-    if (M.use_graph && !M.layers.empty()) {
+    if (!M.layers.empty() && M.record_pays()) {
         check(so_graph_begin(ctx), "so_graph_begin");
         try {
             M.enqueue_layers();
@@ -62,16 +62,25 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
     }
 }
 
-void SparseOnnxModel::Impl::enqueue_layers() const
+std::size_t SparseOnnxModel::Impl::output_layer() const
+{
+    for (std::size_t i = layers.size(); i > 0; --i)
+        if (layers[i - 1].out == output_slot) return i - 1;
+    return layers.size();
+}
+
+void SparseOnnxModel::Impl::enqueue_layers(const float *in, float *out) const
 {
     so_ctx *ctx = context();
     const uint32_t B = pbatch;
-    // Every layer reads and writes arena slots.  A slot id is shared by all tensors whose lifetimes
-    // do not overlap, so it identifies neither the graph input nor the graph output: callers' buffers
-    // are copied into the input slot before the chain and out of the output slot after it.
-    auto src = [&](int s) -> const float * { return slot_ptr(s); };
-    auto dst = [&](int s) -> float * { return slot_ptr(s); };
-    for (const LayerPlan &L : layers) {
+    // Every layer reads and writes arena slots.  The input's slot holds nothing else.  A slot is shared by all tensors whose lifetimes do
+    // not overlap, so the output's is the output only from the last layer that writes it on.
+    const std::size_t made = output_layer();
+    std::size_t at = 0;
+    auto src = [&](int s) -> const float * { return in && s == input_slot ? in : out && at > made && s == output_slot ? out : slot_ptr(s); };
+    auto dst = [&](int s) -> float * { return out && at == made ? out : slot_ptr(s); };
+    for (; at < layers.size(); ++at) {
+        const LayerPlan &L = layers[at];
         const float *bias = L.has_bias ? bias_pool.f32() + L.bias_offset : nullptr;
         switch (L.op) {
         case Op::MatMul:
@@ -97,6 +106,29 @@ void SparseOnnxModel::Impl::enqueue_layers() const
             break;
         }
     }
+}
+
+// A launch graph spares the host about 4 us a launch, but the GPU waits 4 to 10 us before and behind one and works on the arena's
+// slots only, so that device callers' input and output are copied: it pays where the chain is shorter than the host needs to launch it.
+// The chain's time: 4 us a layer and the longer of a row's chain at 10 ns an entry and the layer's work at 25 TFLOP/s; the line lies at 6.5 us a
+// layer.  ResNet-18-shaped stacks, 23 launches, us with a graph / without, run_device: 64 x 64 of width 16 at batch 1 108 / 114, 4 119 / 140, 16 145 / 153;
+// 96 x 96 of 32 at 8 195 / 195; 128 x 128 of 32 at 32 352 / 330; 224 x 224 of 64 at 1 245 / 226, at 32 966 / 923.  From host arrays: 64 x 64 at batch
+// 4 125 / 126, 96 x 96 at 8 220 / 222, 128 x 128 of 48 at 2 235 / 247; 160 x 160 of 32 at 11 403 / 397, 224 x 224 of 48 at 4 372 / 367, of 64 at 1 258 / 255.
+// A 4-layer MLP: 111 / 102; chains of fewer than eight layers have no graph.
+bool SparseOnnxModel::Impl::record_pays() const
+{
+    if (use_graph >= 0) return use_graph == 1;
+    if (layers.size() < 8) return false;
+    double us = 0.0;
+    for (const LayerPlan &L : layers) {
+        us += 4.0;
+        if (!L.E || L.E->m == 0) continue;
+        double nnz = 0.0;
+        for (uint32_t c : L.E->nnz) nnz += c;
+        const double columns = (L.op == Op::Conv ? double(L.cg.H_out) * L.cg.W_out : 1.0) * pbatch;
+        us += std::max(0.010 * nnz / L.E->m, 2.0 * nnz * columns / 25e6);
+    }
+    return us < 6.5 * double(layers.size());
 }
 
 void SparseOnnxModel::Impl::launch_chain() const
@@ -175,6 +207,14 @@ void SparseOnnxModel::run_device(const float *dInput, uint32_t B, float *dOutput
         return;
     }
     so_ctx *ctx = context();
+    // Without a launch graph, the layers on the caller's memory, without a copy of the input and of the output, where it is aligned as the slots are for any kernel's
+    // choice: the same kernels and bits.  Memory that overlaps is copied.
+    const std::uintptr_t x = reinterpret_cast<std::uintptr_t>(dInput), y = reinterpret_cast<std::uintptr_t>(dOutput);
+    const bool apart = x + M.in_features * B * sizeof(float) <= y || y + M.out_features * B * sizeof(float) <= x;
+    if (((x | y) & 15u) == 0 && apart && !M.graph && M.output_layer() < M.layers.size()) {
+        M.enqueue_layers(dInput, dOutput);
+        return;
+    }
     check(so_d2d(ctx, M.slot_ptr(M.input_slot), dInput, M.in_features * B * sizeof(float)), "so_d2d(input)");
     M.launch_chain();
     check(so_d2d(ctx, dOutput, M.slot_ptr(M.output_slot), M.out_features * B * sizeof(float)), "so_d2d(output)");

@@ -494,11 +494,7 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     }
     for (auto &p : pend) M.layers.push_back(std::move(p.plan));
 
-    // A recorded launch graph saves host time per launch but adds device time per kernel (measured on
-    // a 4-layer MLP: 111 us per replay against 102 us for the same four launches in a row; on a
-    // 23-launch CNN the two are within 1 %): record one only for chains of eight layers or more.
-    // SPARSEOPS_NO_GRAPH=1 never records, =0 always does.
-    M.use_graph = M.layers.size() >= 8;
+    // SPARSEOPS_NO_GRAPH=1 never records a launch graph, =0 always does.
     if (const char *e = std::getenv("SPARSEOPS_NO_GRAPH")) M.use_graph = !(e[0] && e[0] != '0');
     resize_buffers(uint32_t(B0));
 }

@@ -383,6 +383,35 @@ def test_run_device_mlp_wide_hidden_layers(backend, ctx, oracle, tmp_path):
     assert np.array_equal(_run_device(model, ctx, X), Y)
 
 
+@pytest.mark.parametrize("graph", ["always", "never"])
+@pytest.mark.parametrize("layers", [3, 9])
+def test_run_device_in_callers_memory(backend, ctx, tmp_path, graph, layers):
+    """run_device without a launch graph works on the caller's memory: whole, off a 16-byte boundary, with an output that
+    overlaps the input at either end, and called again after the input has changed; with a graph the same bits."""
+    rng = np.random.default_rng(layers)
+    dims, B = [48] + [40 + 8 * i for i in range(layers - 1)] + [24], 12
+    Ws = [datagen.magnitude_prune(rng.standard_normal((o, i)).astype(np.float32), .5) for i, o in zip(dims[:-1], dims[1:])]
+    os.environ["SPARSEOPS_NO_GRAPH"] = "0" if graph == "always" else "1"
+    try:
+        model = backend.SparseOnnxModel(ow.save(str(tmp_path / "mlp.onnx"), ow.mlp_model(Ws, ["Relu"] * (layers - 1) + [None], B)))
+    finally:
+        del os.environ["SPARSEOPS_NO_GRAPH"]
+    n_in, n_out = dims[0] * B, dims[-1] * B
+    mem = ctx.empty((n_in + n_out + 64,))
+    for x_at, y_at in ((0, n_in), (n_out, 0), (1, n_in + 4), (4, n_in + 7), (0, 0), (0, n_in - n_out), (8, n_in - 4), (n_out - 8, 0)):
+        X = rng.standard_normal((B, dims[0])).astype(np.float32)
+        want = model.run(X).T.ravel()
+        held = np.zeros(n_in + n_out + 64, np.float32)
+        held[x_at:x_at + n_in] = X.T.ravel()
+        mem.upload(held)
+        model.run_device(mem.ptr + 4 * x_at, B, mem.ptr + 4 * y_at)
+        got = mem.download()
+        assert np.array_equal(got[y_at:y_at + n_out], want), (x_at, y_at)
+        held[y_at:y_at + n_out] = want
+        assert np.array_equal(got, held), (x_at, y_at)
+    mem.free()
+
+
 @pytest.mark.parametrize("B", [32, 5])
 def test_run_device_cnn(backend, ctx, tmp_path, B):
     """run_device on a ResNet-shaped stack at a batch carried as is (32) and one carried padded (5)."""
