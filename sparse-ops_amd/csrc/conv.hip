@@ -980,25 +980,28 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
         const double run = (double)E->total_nnz / (double)plan->g.Cout / plan->win.nch;
         window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw * (int)plan->win.px;
     }
-    const bool columns = B >= 1 && B <= kColMaxBatch && !plan->col_tried[B - 1];
+    const int slot = so_conv_columns_slot(B);
+    const bool columns = slot >= 0 && !plan->col_tried[slot];
     if (!window && !columns) { plan->tuned_batch = batch; return SO_OK; }
     const size_t slots = (size_t)E->m * E->r;
     std::vector<uint32_t> idx(slots), nnz(E->m);
     std::vector<float> Wd(slots);
     so_status s = so_ellpack_download(ctx, E, SO_LAYOUT_ROW, Wd.data(), idx.data(), nnz.data());
     if (s != SO_OK) return s;
-    if (columns) {
-        s = so_conv_columns_build(ctx, plan, idx, nnz, Wd, B);
+    if (window) {
+        SO_HIP(hipStreamSynchronize(ctx->stream));      // no launch may still be reading the old arrays
+        free_window(plan);
+        s = build_window(ctx, plan, idx, nnz, Wd, batch);
+        if (s == SO_OK) s = so_conv_rbm_rebuild(ctx, plan);          // the record streams follow the window's chunks
         if (s != SO_OK) return s;
-        plan->col_tried[B - 1] = true;
     }
     plan->tuned_batch = batch;
-    if (!window) return SO_OK;
-    SO_HIP(hipStreamSynchronize(ctx->stream));      // no launch may still be reading the old arrays
-    free_window(plan);
-    s = build_window(ctx, plan, idx, nnz, Wd, batch);
-    if (s != SO_OK) return s;
-    return so_conv_rbm_rebuild(ctx, plan);          // the record streams follow the window's chunks
+    if (columns) {                                      // (looks at the window's layout)
+        s = so_conv_columns_build(ctx, plan, idx, nnz, Wd, B);
+        if (s != SO_OK) return s;
+        plan->col_tried[slot] = true;
+    }
+    return SO_OK;
 }
 
 extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[8])
@@ -1008,6 +1011,21 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
     const uint32_t v[8] = {w.TH, w.TW, w.IH, w.IW, w.cc, w.nch, (uint32_t)w.cpw, w.px};
     for (int i = 0; i < 8; ++i) out[i] = w.cc ? v[i] : 0u;
     return SO_OK;
+}
+
+// Whether the column kernel, at four entries or more, is taken before the windowed one: where its shorter chains on more waves win.  The windowed kernel's time
+// is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (batch 4: 7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4);
+// at 8, 16 and 32 entries, looked at where its waves have one channel each, which they have on small images, 3.8 us, 1 a chunk of channels and 16 ns (8
+// entries) or 20.5 per nonzero.  Us windowed / column: 2x2x256 with 921 nonzeros a row at batch 8 / 16 / 32 19.8 / 14.2, 28.3 / 16.3, 28.9 / 18.9; 4x4x128
+// with 461 12.5 / 9.4, 18.0 / 10.2, 18.0 / 12.4; 8x8x64 with 231 8.7 / 6.8, 10.9 / 7.0, 11.2 / 8.0; 3x3x512 with 921 24.3 / 18.6, 36.0 / 25.8, 36.0 / 41.6;
+// 8x8x256 with 690 21.2 / 16.6, 27.6 / 22.4, 31.6 / 51.1; 7x7x512 with 921 29.9 / 34.4, 44.5 / 72, 59 / 160.
+bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us)
+{
+    const so_conv_window &w = plan->win;
+    if (w.cc == 0 || (B > 4 && w.cpw * (int)w.px != 1)) return false;
+    const double rounds = so_ceil_div(window_workgroups(w, plan->g.Cout, (uint32_t)w.cpw * w.px, B), (uint64_t)ctx->compute_units);
+    const double row = (double)plan->E->total_nnz / plan->g.Cout;
+    return columns_us < 0.9 * rounds * (B <= 4 ? 5.5 + 0.0205 * row : 3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row);
 }
 
 static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,
@@ -1021,16 +1039,13 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
     SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
     // The column kernel where the plan has its streams for this batch: below four entries, which the windowed kernel does
-    // not take, where it pays against the gather kernel (so_conv_columns_pays), at four where its shorter chains on more
-    // waves win -- the windowed kernel's time there is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the
-    // chip (7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
+    // not take, where it pays against the gather kernel (so_conv_columns_pays), from four on against the windowed one
+    // (so_conv_columns_before_window).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
     if (so_conv_columns_for(plan, B) && ctx->tune.conv_columns != 0) {
-        const bool alone = B < 4 || plan->win.cc == 0;           // no windowed kernel: else the gather kernel
+        const bool alone = B < 4 || (B == 4 && plan->win.cc == 0);           // no windowed kernel: else the gather kernel
         bool use = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
-        if (!use && !alone && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1) {
-            const double rounds = so_ceil_div(window_workgroups(plan->win, g.Cout, (uint32_t)plan->win.cpw * plan->win.px, B), (uint64_t)ctx->compute_units);
-            use = so_conv_columns_estimate(ctx, plan, B) < 0.9 * rounds * (5.5 + 0.0205 * (double)plan->E->total_nnz / g.Cout);
-        }
+        if (!use && !alone && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1)
+            use = so_conv_columns_before_window(ctx, plan, B, so_conv_columns_estimate(ctx, plan, B));
         if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for
         bool done = false;
         const so_status s = use ? so_conv_columns_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done) : SO_OK;

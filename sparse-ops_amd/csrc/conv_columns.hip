@@ -1,4 +1,4 @@
-// so_conv2d for small batches: a wave owns one output channel and 64 output columns, a column being one
+// so_conv2d for small batches, and for small images at batches of 8, 16 and 32: a wave owns one output channel and 64 output columns, a column being one
 // (pixel, batch entry) pair.
 //
 // The LDS-windowed kernel (csrc/conv.hip) gives a lane four batch entries of a pixel, so a batch of one is carried as
@@ -182,11 +182,34 @@ template <int ACT>
 void launch_columns(so_ctx *ctx, const so_conv_plan *plan, const ColArgs &a, dim3 grid, size_t lds, const float *dX, uint32_t B,
                     const float *dBias, const float *dResid, float *dY)
 {
-    const so_conv_columns &c = plan->col[B - 1];
+    const so_conv_columns &c = *so_conv_columns_for(plan, B);
     conv2d_column_kernel<ACT><<<grid, a.waves * 64u, lds, ctx->stream>>>(c.d_entries, c.d_first, a, plan->g, dX, B, dBias, dResid, dY);
 }
 
 constexpr uint64_t kColLds = 150 * 1024;
+
+struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
+
+// Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
+// longest chain at 10 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
+// more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
+// 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
+ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
+{
+    const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
+    ColShape best{16, 16, 0, 1e30, 1.0};
+    for (uint32_t G = 16; G >= 4; G /= 2) {
+        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0, 0.0};
+        s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
+        const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
+        const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
+        const double resident = std::min(fit, std::ceil(wgs / cus));
+        s.rounds = std::ceil(wgs / (cus * fit));
+        s.us = 3.0 + s.rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        if (s.us < best.us) best = s;
+    }
+    return best;
+}
 
 } // namespace
 
@@ -201,7 +224,8 @@ void so_conv_columns_free(so_conv_plan *plan)
 
 const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B)
 {
-    return B >= 1 && B <= kColMaxBatch && plan->col[B - 1].batch == B ? &plan->col[B - 1] : nullptr;
+    const int slot = so_conv_columns_slot(B);
+    return slot >= 0 && plan->col[slot].batch == B ? &plan->col[slot] : nullptr;
 }
 
 // Sizes the tile for batch B and uploads the entry streams; leaves the plan without them where the kernel does not apply.
@@ -210,7 +234,8 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
 {
     const so_conv_geom &g = plan->g;
     const so_ellpack *E = plan->E;
-    if (B == 0 || B > kColMaxBatch || E->r == 0 || E->total_nnz == 0 || !E->ascending || (size_t)ctx->max_lds_bytes < kColLds) return SO_OK;
+    const int slot = so_conv_columns_slot(B);
+    if (slot < 0 || E->r == 0 || E->total_nnz == 0 || !E->ascending || (size_t)ctx->max_lds_bytes < kColLds) return SO_OK;
     so_conv_columns c;
     const uint32_t px = 64u / B, sth = window_step(g.kH, g.stride_h), stw = window_step(g.kW, g.stride_w);
     uint64_t best_tiles = ~0ull, best_win = ~0ull;
@@ -237,6 +262,9 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
     // window_div: operand * divisor below 2^32
     if ((uint64_t)c.tiles_x * c.tiles_x * c.tiles_y >= (1ull << 32) || plane * plane >= (1ull << 32) || plane * 1024 >= (1ull << 32)) return SO_OK;
     if ((uint64_t)c.tiles_x * c.tiles_y >= (1ull << 31) || ((uint64_t)c.cc + 1024) * g.H_in * g.W_in * B >= (1ull << 30)) return SO_OK;
+    c.batch = B;
+    // at more than four entries no streams for a plan whose windowed layout the kernel would not be taken before
+    if (B > 4 && ctx->tune.conv_columns != 1 && !so_conv_columns_before_window(ctx, plan, B, column_shape(ctx, plan, c).us)) return SO_OK;
     const uint32_t kHW = g.kH * g.kW;
     const size_t runs = (size_t)E->m * c.nch;
     std::vector<uint32_t> first(runs + 1);      // entries of every (channel, chunk), then groups, then where they begin
@@ -288,37 +316,9 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
         if (c.d_first) (void)hipFree(c.d_first);
         return s;
     }
-    c.batch = B;
-    plan->col[B - 1] = c;
+    plan->col[slot] = c;
     return SO_OK;
 }
-
-namespace {
-
-struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
-
-// Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
-// longest chain at 10 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
-// more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
-// 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
-ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
-{
-    const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
-    ColShape best{16, 16, 0, 1e30, 1.0};
-    for (uint32_t G = 16; G >= 4; G /= 2) {
-        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0, 0.0};
-        s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
-        const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
-        const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
-        const double resident = std::min(fit, std::ceil(wgs / cus));
-        s.rounds = std::ceil(wgs / (cus * fit));
-        s.us = 3.0 + s.rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
-        if (s.us < best.us) best = s;
-    }
-    return best;
-}
-
-} // namespace
 
 // Whether the kernel is taken before the gather kernel: both walk a channel's entries for every output, this one after a
 // copy of the window, which entries enough repay -- more of them where the gather kernel has two or four batch entries to
@@ -334,21 +334,21 @@ ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv
 //   the windowed layout): 72 entries 133 / 170, 75 29.5 / 28.0, 118 54.5 / 46.6, 147 79 / 72.
 bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B)
 {
-    const so_conv_columns &c = plan->col[B - 1];
+    const so_conv_columns &c = *so_conv_columns_for(plan, B);
     const double entries = (double)plan->E->total_nnz / plan->g.Cout, window = (double)c.cc * c.nch * c.PE * B;
     if (entries < 8.0 || window > 480.0 * entries) return false;
     const double least = B == 4 ? 100.0 : B == 2 || plan->g.kH * plan->g.kW == 1 ? 64.0 : 20.0;
     return entries >= least || column_shape(ctx, plan, c).rounds <= 1.0;
 }
 
-double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, plan->col[B - 1]).us; }
+double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, *so_conv_columns_for(plan, B)).us; }
 
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done)
 {
     *done = false;
     if (!so_conv_columns_for(plan, B)) return SO_OK;
-    const so_conv_columns &c = plan->col[B - 1];
+    const so_conv_columns &c = *so_conv_columns_for(plan, B);
     const so_conv_geom &g = plan->g;
     ColArgs a;
     a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch; a.pitch = c.pitch;

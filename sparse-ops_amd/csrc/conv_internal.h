@@ -38,8 +38,9 @@ struct so_conv_rbm {
     uint64_t total_sets = 0, real_pairs = 0, slots = 0;
 };
 
-// Entry streams of the column kernel for small batches (conv_columns.hip).
-constexpr uint32_t kColMaxBatch = 4;
+// Entry streams of the column kernel for small batches and small images (conv_columns.hip): batches of 1 to 4, 8, 16 and 32.
+constexpr uint32_t kColSlots = 7;
+inline int so_conv_columns_slot(uint32_t B) { return B >= 1 && B <= 4 ? (int)B - 1 : B == 8 ? 4 : B == 16 ? 5 : B == 32 ? 6 : -1; }
 struct so_conv_columns {
     uint32_t batch = 0;              // the batch the tile and the offsets are for; 0: not built, or the kernel does not apply
     uint32_t TH = 0, TW = 0, tiles_x = 0, tiles_y = 0, IP = 0, PE = 0, cc = 0, nch = 0;
@@ -56,8 +57,8 @@ struct so_conv_plan {
     int2 *d_taps = nullptr;  // per slot: x = (cin*H + dh)*W + dw (elements of B floats), y = dh<<16 | (dw & 0xffff)
     so_conv_window win;      // win.cc == 0: not built
     so_conv_rbm rbm;         // rbm.d_sets == nullptr: no streams
-    so_conv_columns col[kColMaxBatch];   // streams for batch 1 + index, made by the first tuning for it and kept: graphs may replay with them
-    bool col_tried[kColMaxBatch] = {};   // that tuning has happened, whether the kernel applies or not
+    so_conv_columns col[kColSlots];      // streams by so_conv_columns_slot, made by the first tuning for the batch and kept: graphs may replay with them
+    bool col_tried[kColSlots] = {};      // that tuning has happened, whether the kernel applies or not
 };
 
 // conv_columns.hip
@@ -67,6 +68,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
 const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B);  // null: the plan has no streams for the batch
 bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);            // against the gather kernel
 double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);      // us
+bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us);   // conv.hip
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done);
 

@@ -57,6 +57,39 @@ def test_columns_match_oracle(ctx, oracle, Cin, Cout, H, Wi, k, s, p, d, sp, B):
             a.free()
 
 
+@pytest.mark.parametrize("case", [CASES[0], CASES[1], CASES[2], CASES[3], CASES[5], CASES[6], CASES[9]])
+@pytest.mark.parametrize("B", [8, 16, 32])
+def test_columns_wider_batches(ctx, oracle, case, B):
+    """Batches of 8, 16 and 32: tiles of eight, four and two pixels."""
+    test_columns_match_oracle(ctx, oracle, *case, B)
+
+
+# Cin, Cout, H, k, s, sparsity, B, kernel: small images with long rows go to the column kernel, others keep the windowed one
+@pytest.mark.parametrize("Cin,Cout,H,k,s,sp,B,kernel", [
+    (256, 256, 2, 3, 1, .6, 16, "columns"), (256, 256, 2, 3, 1, .6, 32, "columns"), (128, 128, 4, 3, 1, .6, 16, "columns"),
+    (512, 512, 7, 3, 1, .8, 8, "window"), (256, 256, 8, 3, 1, .7, 32, "window"), (128, 256, 4, 1, 2, .6, 16, "window")])
+def test_columns_or_window(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel):
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin + H + B)
+    E = datagen.encode_dense(sparse_matrix(rng, Cout, Cin * k * k, sp))
+    args = Cin, Cout, k, k, H, H, (s, s), (k // 2, k // 2), (1, 1)
+    g, og = hipabi.conv_geom(*args), ocg(*args)
+    X = rng.standard_normal((Cin, H, H, B)).astype(np.float32)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan = ctx.conv_plan(dE, g)
+    want = oracle.conv2d_pf(as_oracle(E), og, X, B, None, "none")
+    dX, dY = ctx.array(X), ctx.empty(want.shape)
+    for batch, expect in ((B, kernel), (4, None), (B, kernel)):         # and after the plan has been tuned for another batch
+        ctx.conv_plan_tune(plan, batch)
+        if expect:
+            ctx.conv2d(plan, dX, B, None, dY, "none")
+            assert ctx.last_kernel() == expect
+            assert np.array_equal(dY.download(), want)
+    ctx.conv_plan_free(plan)
+    for a in (dX, dY, dE):
+        a.free()
+
+
 @pytest.mark.parametrize("Cin,H", [(34, 9), (400, 18)])            # one chunk and several
 def test_columns_groups_per_run(ctx, oracle, Cin, H):
     """Runs of no group of 16 entries up to three blocks of eight, one entry more or fewer: what a block, the rest behind it
