@@ -1025,7 +1025,7 @@ bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, 
     if (w.cc == 0 || (B > 4 && w.cpw * (int)w.px != 1)) return false;
     const double rounds = so_ceil_div(window_workgroups(w, plan->g.Cout, (uint32_t)w.cpw * w.px, B), (uint64_t)ctx->compute_units);
     const double row = (double)plan->E->total_nnz / plan->g.Cout;
-    return columns_us < 0.9 * rounds * (B <= 4 ? 5.5 + 0.0205 * row : 3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row);
+    return columns_us < rounds * (B <= 4 ? 0.9 * (5.5 + 0.0205 * row) : 3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row);
 }
 
 static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,
