@@ -247,8 +247,8 @@ so_status so_conv_plan_create(so_ctx *ctx, const so_ellpack *E, const so_conv_ge
 so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan);
 /* Re-sizes the plan's internal layouts for launches with batch B (how many output channels
  * a wave takes depends on how many workgroups the batch yields).  Optional: results never
- * depend on it; plans are created for batch 32.  For a batch of at most four it also makes the
- * column kernel's streams for exactly that batch, once; they stay until the plan is freed.
+ * depend on it; plans are created for batch 32.  For a batch of one to four, and of 8, 16 or 32
+ * where it is estimated to pay, it also makes the column kernel's streams for exactly that batch, once; they stay until the plan is freed.
  * Not to be called while a launch that uses the plan may be in flight on another stream, nor during
  * graph capture (it allocates).  A graph recorded with the plan before is recorded again afterwards
  * (SparseOnnxModel::resize_buffers does), unless the new batch falls into the same four-entry step.
@@ -332,8 +332,8 @@ so_status so_copy_rows(so_ctx *ctx, const float *dSrc, size_t src_stride, uint32
 
 /* ---- launch graphs -------------------------------------------------------
  * Record every launch made on the context between begin and end into one
- * hipGraph, then replay it with a single submission (SparseOnnxModel::run uses
- * this for layer chains of eight layers or more, src/model_run.cpp:28-127).  No allocation, copy to
+ * hipGraph, then replay it with a single submission (SparseOnnxModel uses
+ * this for short chains of eight layers or more, sparse-ops_amd/src/model_run.cpp).  No allocation, copy to
  * or from the host, or timer call may happen while recording.  A graph keeps so_matmul's workspace of
  * the time of its recording, so later launches may grow the context's; the handles, plans and arrays
  * that were recorded must outlive it. */

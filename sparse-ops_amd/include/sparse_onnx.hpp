@@ -53,7 +53,8 @@ public:
 
     /// Device-pointer variant: dInput [input_features x B] and dOutput
     /// [output_features x B] are HBM pointers of the process-wide context; only
-    /// kernels are enqueued, the call does not wait for them.
+    /// kernels are enqueued, the call does not wait for them (they read dInput and write dOutput until
+    /// the chain is done).
     void run_device(const float *dInput, uint32_t B, float *dOutput) const;
 
     /// (Re)allocate every activation buffer for `batch` samples and re-record the
