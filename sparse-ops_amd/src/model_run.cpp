@@ -20,15 +20,20 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
     std::lock_guard<std::mutex> lock(context_mutex());
     if (M.graph) { so_graph_free(ctx, M.graph); M.graph = nullptr; }
     M.has_conv = false;
-    for (const LayerPlan &L : M.layers) M.has_conv |= L.conv != nullptr;
+    uint64_t pixels = 0;                       // of the largest convolution's output
+    for (const LayerPlan &L : M.layers) {
+        M.has_conv |= L.conv != nullptr;
+        if (L.conv) pixels = std::max(pixels, uint64_t(L.cg.H_out) * L.cg.W_out);
+    }
     // The convolutions work on batch tiles of 16, 8 or 4 entries, and the larger the tile the less a
     // batch entry costs: a batch is carried in rows of 4 (2 to 4 entries), 8 (up to 8) or the next
     // multiple of 16 (the extra columns are zeros on input and are never copied out; batch entries
     // do not interact).  Measured on a ResNet-18-shaped stack: 12 entries as 12 0.86 ms, as 16
-    // 0.76 ms; 24 as 24 1.31 ms, as 32 1.24 ms.  A single entry has a kernel of its own: 0.35 ms as 4, 0.25 as 1
-    // (two entries as 2: 0.34).
+    // 0.76 ms; 24 as 24 1.31 ms, as 32 1.24 ms.  One and two entries have a kernel of their own: one entry 0.35 ms as 4, 0.22
+    // as 1; two as 4 / as 2, us, ResNet-18-shaped stacks: 224 x 224 of width 64 314 / 272, 48 273 / 219, 16 124 / 110, 64 x 64 of 16 102 / 91, but
+    // 384 x 384 of 32 271 / 278, 448 x 448 of 64 632 / 672, 512 x 512 of 16 200 / 197: as 2 up to 128 x 128 outputs (a stride of two on 256 x 256).
     uint32_t pbatch = batch;
-    if (M.has_conv && batch > 1) pbatch = batch <= 4 ? 4u : batch <= 8 ? 8u : (batch + 15u) / 16u * 16u;
+    if (M.has_conv && batch > 1 && !(batch == 2 && pixels <= 128u * 128u)) pbatch = batch <= 4 ? 4u : batch <= 8 ? 8u : (batch + 15u) / 16u * 16u;
     // Slot offsets for this batch, 256-byte aligned.
     std::size_t total = 0;
     std::size_t widest = std::max(M.in_features, M.out_features);

@@ -383,6 +383,17 @@ def test_run_device_mlp_wide_hidden_layers(backend, ctx, oracle, tmp_path):
     assert np.array_equal(_run_device(model, ctx, X), Y)
 
 
+@pytest.mark.parametrize("hw", [64, 272])          # carried as two entries, and as four (136 x 136 outputs)
+def test_model_batch_of_two(backend, ctx, tmp_path, hw):
+    """Two samples have the bits they have in a batch of four, from host arrays and on the device."""
+    payload, _ = datagen.resnet18_onnx(seed=3, batch=4, hw=hw, sparsity=0.8, classes=10, width=16)
+    model = backend.SparseOnnxModel(ow.save(str(tmp_path / "r18.onnx"), payload))
+    X = np.random.default_rng(hw).standard_normal((4, 3, hw, hw)).astype(np.float32)
+    Y = model.run(X)
+    assert np.array_equal(model.run(X[:2]), Y[:2]) and np.array_equal(model.run(X[1:3]), Y[1:3])
+    assert np.array_equal(_run_device(model, ctx, X[2:]), Y[2:])
+
+
 @pytest.mark.parametrize("graph", ["always", "never"])
 @pytest.mark.parametrize("layers", [3, 9])
 def test_run_device_in_callers_memory(backend, ctx, tmp_path, graph, layers):
