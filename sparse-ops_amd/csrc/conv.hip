@@ -1017,7 +1017,7 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
 // is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (batch 4: 7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4);
 // at 8, 16 and 32 entries, looked at where its waves have one channel each, which they have on small images, 3.8 us, 1 a chunk of channels and 16 ns (8
 // entries) or 20.5 per nonzero.  Us windowed / column: 2x2x256 with 921 nonzeros a row at batch 8 / 16 / 32 19.8 / 14.2, 28.3 / 16.3, 28.9 / 18.9; 4x4x128
-// with 461 12.5 / 9.4, 18.0 / 10.2, 18.0 / 12.4; 8x8x64 with 231 8.7 / 6.8, 10.9 / 7.0, 11.2 / 8.0; 3x3x512 with 921 24.3 / 18.6, 36.0 / 25.8, 36.0 / 41.6;
+// with 461 12.5 / 9.4, 18.0 / 10.2, 18.0 / 12.4; 8x8x64 with 231 8.7 / 6.8, 10.9 / 7.0, 11.2 / 8.0; 3x3x512 with 921 24.3 / 18.6, 36.0 / 25.8, 36.0 / 41.6; 8x8x64 with 58 6.0 / 5.1, 7.3 / 5.5, 7.5 / 6.1;
 // 8x8x256 with 690 21.2 / 16.6, 27.6 / 22.4, 31.6 / 51.1; 7x7x512 with 921 29.9 / 34.4, 44.5 / 72, 59 / 160.
 bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us)
 {
@@ -1025,7 +1025,7 @@ bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, 
     if (w.cc == 0 || (B > 4 && w.cpw * (int)w.px != 1)) return false;
     const double rounds = so_ceil_div(window_workgroups(w, plan->g.Cout, (uint32_t)w.cpw * w.px, B), (uint64_t)ctx->compute_units);
     const double row = (double)plan->E->total_nnz / plan->g.Cout;
-    return columns_us < rounds * (B <= 4 ? 0.9 * (5.5 + 0.0205 * row) : 3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row);
+    return columns_us < rounds * (B <= 4 ? 0.9 * (5.5 + 0.0205 * row) : 0.95 * (3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row));
 }
 
 static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,

@@ -192,7 +192,8 @@ struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 
 // Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
 // longest chain at 10 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
-// more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
+// more waves than compute.  From 8 entries on, where windows of few pixels are the rule, a chunk's start-up goes by its LDS: 0.5 us and 17 ns per KB
+// (batch 16, start-up and chunks in front of the chain: 66 KB 1.9 us, 131 KB 2.8, twice 131 KB 4.5).  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
 // 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
 ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
 {
@@ -205,7 +206,8 @@ ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv
         const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
         const double resident = std::min(fit, std::ceil(wgs / cus));
         s.rounds = std::ceil(wgs / (cus * fit));
-        s.us = 3.0 + s.rounds * (2.5 + c.nch * 1.0 + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        const double start = c.batch <= 4 ? 2.5 + c.nch : c.nch * (0.5 + 0.017 * s.lds / 1024.0);
+        s.us = 3.0 + s.rounds * (start + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
         if (s.us < best.us) best = s;
     }
     return best;

@@ -67,7 +67,7 @@ def test_columns_wider_batches(ctx, oracle, case, B):
 # Cin, Cout, H, k, s, sparsity, B, kernel: small images with long rows go to the column kernel, others keep the windowed one
 @pytest.mark.parametrize("Cin,Cout,H,k,s,sp,B,kernel", [
     (256, 256, 2, 3, 1, .6, 16, "columns"), (256, 256, 2, 3, 1, .6, 32, "columns"), (128, 128, 4, 3, 1, .6, 16, "columns"),
-    (512, 512, 7, 3, 1, .8, 8, "window"), (256, 256, 8, 3, 1, .7, 32, "window"), (128, 256, 4, 1, 2, .6, 16, "window")])
+    (512, 512, 7, 3, 1, .8, 8, "window"), (256, 256, 8, 3, 1, .7, 32, "window"), (128, 128, 12, 3, 1, .8, 16, "window"), (128, 256, 4, 1, 2, .6, 16, "columns")])
 def test_columns_or_window(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel):
     from oracle import conv_geom as ocg
     rng = np.random.default_rng(Cin + H + B)
