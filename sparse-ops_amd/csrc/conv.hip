@@ -580,11 +580,11 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
 }
 
 template <int CPW, int LPP, int PX>
-void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, size_t lds,
+void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, dim3 grid, size_t lds,
                        const float *dX, uint32_t B, const float *dBias, const float *dResid, float *dY, int act)
 {
 #define SO_WIN_LAUNCH(A)                                                                                   \
-    conv2d_window_kernel<CPW, LPP, A, PX><<<8u * a.per_xcd, kWinThreads, lds, ctx->stream>>>(                            \
+    conv2d_window_kernel<CPW, LPP, A, PX><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(        \
         reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a,       \
         plan->g, dX, B, dBias, dResid, dY)
     switch (act) {
@@ -671,19 +671,18 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     // Even a grid that covers an eighth of the chip beats the gather kernel on long rows (measured on the
     // 14x14 and 7x7 layers of a ResNet-18-shaped stack at batch 8); below that the gather kernel's finer waves win.
     if (!forced && 8 * wgs < (uint64_t)ctx->compute_units) return SO_OK;
-    if (grid.y > 65535u || grid.z > 65535u || wgs >= (1ull << 31)) return SO_OK;
-    window_shares(a, grid);
+    if (!window_shares(a, grid)) return SO_OK;
     if (px == 2u) {
         if constexpr (LPP == 4) {
-            if (w.cpw == 4) window_launch_act<4, 4, 2>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act);
-            else window_launch_act<2, 4, 2>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act);
+            if (w.cpw == 4) window_launch_act<4, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
+            else window_launch_act<2, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
         }
     } else
     switch (w.cpw) {
-    case 8:  window_launch_act<8, (int)LPP, 1>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
-    case 4:  window_launch_act<4, (int)LPP, 1>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
-    case 2:  window_launch_act<2, (int)LPP, 1>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
-    default: window_launch_act<1, (int)LPP, 1>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
+    case 8:  window_launch_act<8, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 4:  window_launch_act<4, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 2:  window_launch_act<2, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    default: window_launch_act<1, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
     }
     ctx->waits_pending = true;
     *done = true;

@@ -89,8 +89,8 @@ inline uint32_t window_lpp(uint32_t B) { return B % 16 == 0 ? 4u : B % 8 == 0 ? 
 
 struct WinArgs {
     uint32_t TH, TW, IH, IW, cc, nch, tiles_x, pg, cg, groups;
-    uint32_t mYZ, mZ;                // window_magic of gy * gz and gz; mYZ is 0 where that is 1 or the ids are too many
-    uint32_t wgs, per_xcd, gy, gz;   // workgroups in all and per XCD; channel blocks and batch tiles (window_workgroup)
+    uint32_t mYZ = 0, mZ = 0;        // window_magic of gy * gz and gz; mYZ is 0 where that is 1 or the ids are too many
+    uint32_t wgs, per_xcd, gy, gz;   // workgroups in all and per XCD (0: ids as launched); channel blocks and batch tiles (window_workgroup)
     uint32_t win_f4;    // float4 elements of one chunk's window
     uint32_t buf_f4;    // window plus the zero plane: stride between the two buffers
     uint32_t nbuf;      // 2: double-buffered windows; 1: a single chunk, nothing to overlap
@@ -119,19 +119,32 @@ inline uint32_t window_subsample(uint32_t k, uint32_t stride) { return k == 1 ? 
 // holds an eighth of the input, whose halos neighbouring tiles share, and both halves of the 128-byte lines that two batch
 // tiles of 16 read and write.  ResNet-18-shaped stack at batch 32, ids as (x, y, z) / so, us: 56x56x64 layers 45.8-51.1 / 43.7-47.0 (the
 // write of 25.7 MB at the end of a layer 7 / 4), the stem 84.4 / 80.7, the stack 988 / 967.
+//
+// A launch has fewer than 2^32 work items along a dimension, so fewer than 2^22 workgroups of 1024: a grid whose product does not stay below
+// that keeps its ids in (x, y, z), each of which then has to.
 struct WinPlace { uint32_t tile, y, z; };
-inline void window_shares(WinArgs &a, dim3 grid)
+constexpr uint64_t kWinMaxGrid = (1ull << 32) / kWinThreads;
+// Sets the shares for `grid`; the grid to launch is window_grid(a, grid).  False: no launch can have it.
+inline bool window_shares(WinArgs &a, dim3 grid)
 {
-    a.wgs = grid.x * grid.y * grid.z;
+    if (grid.x >= kWinMaxGrid || grid.y > 65535u || grid.z > 65535u) return false;
+    const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z, yz = (uint64_t)grid.y * grid.z;
     a.gy = grid.y; a.gz = grid.z;
-    a.per_xcd = so_ceil_div(a.wgs, 8);
-    const uint64_t yz = (uint64_t)a.gy * a.gz;
-    a.mYZ = (uint64_t)a.wgs * yz < (1ull << 32) ? window_magic((uint32_t)yz) : 0u;
-    if (yz * a.gz >= (1ull << 32)) a.mYZ = 0u;
+    a.wgs = a.per_xcd = 0;
+    if ((wgs + 7) / 8 * 8 >= kWinMaxGrid) return true;
+    a.wgs = (uint32_t)wgs;
+    a.per_xcd = (uint32_t)((wgs + 7) / 8);
+    a.mYZ = wgs * yz < (1ull << 32) && yz * a.gz < (1ull << 32) ? window_magic((uint32_t)yz) : 0u;
     a.mZ = window_magic(a.gz);
+    return true;
 }
+inline dim3 window_grid(const WinArgs &a, dim3 grid) { return a.per_xcd != 0u ? dim3(8u * a.per_xcd) : grid; }
 __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 {
+    if (a.per_xcd == 0u) {
+        p.tile = blockIdx.x; p.y = blockIdx.y; p.z = blockIdx.z;
+        return true;
+    }
     const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3), yz = a.gy * a.gz;
     if (id >= a.wgs) return false;
     if (a.mYZ != 0u) {

@@ -372,12 +372,12 @@ hipError_t rbm_allow_lds(so_ctx *ctx)
 }
 
 template <int LPP>
-void rbm_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, size_t lds,
+void rbm_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, dim3 grid, size_t lds,
                     const float *dX, uint32_t B, const float *dBias, const float *dResid, float *dY, int act)
 {
     const so_conv_rbm &r = plan->rbm;
 #define SO_RBM_LAUNCH(A)                                                                              \
-    conv2d_rbm_kernel<LPP, A><<<8u * a.per_xcd, kWinThreads, lds, ctx->stream>>>(                               \
+    conv2d_rbm_kernel<LPP, A><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(               \
         reinterpret_cast<const int4 *>(r.d_sets), r.d_gbase, r.d_counts, a, plan->g, r.src->Ct_max,   \
         dX, B, dBias, dResid, dY)
     switch (act) {
@@ -555,12 +555,11 @@ so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float 
     if (LPP > w.lpp && (lds > (size_t)ctx->max_lds_bytes || a.win_f4 > (uint32_t)kRbmMaxPerThread * kWinThreads)) return SO_OK;
     if (a.win_f4 > (uint32_t)kRbmMaxPerThread * kWinThreads) return SO_OK;      // this kernel copies at most that many elements per thread
     const dim3 grid(w.tiles_x * w.tiles_y, so_ceil_div(a.groups, a.cg), B / (4 * LPP));
-    if (grid.y > 65535u || grid.z > 65535u || (uint64_t)grid.x * grid.y * grid.z >= (1ull << 31)) return SO_OK;
-    window_shares(a, grid);
+    if (!window_shares(a, grid)) return SO_OK;
     switch (LPP) {
-    case 4:  rbm_launch_act<4>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
-    case 2:  rbm_launch_act<2>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
-    default: rbm_launch_act<1>(ctx, plan, a, lds, dX, B, dBias, dResid, dY, act); break;
+    case 4:  rbm_launch_act<4>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    case 2:  rbm_launch_act<2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
+    default: rbm_launch_act<1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
     }
     *done = true;
     return SO_OK;

@@ -174,6 +174,30 @@ def test_conv_window_two_pixel_groups_per_wave(ctx, oracle, Cin, Cout, H, Wi, B,
     dE.free()
 
 
+def test_conv_window_more_workgroups_than_a_flat_grid_holds(ctx):
+    """65 channel blocks x 65531 batch tiles are 4.26 million workgroups of 1024 threads: more than 2^32 work items along one
+    dimension, which no launch takes, but well within a grid of three.  A 1 x 1 image, of whose 3 x 3 taps only the middle one
+    lies on it: every output is one product."""
+    rng = np.random.default_rng(8)
+    Cout, B = 1040, 4 * 65531
+    W, X = rng.standard_normal((Cout, 9)).astype(np.float32), rng.standard_normal((1, 1, 1, B)).astype(np.float32)
+    E = datagen.encode_dense(W)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    dX, dY = ctx.array(X), ctx.empty((Cout, B))
+    with ctx.tuning(SPARSEOPS_CONV_CPW="1", SPARSEOPS_CONV_WINDOW="1"):
+        plan = ctx.conv_plan(dE, hipabi.conv_geom(1, Cout, 3, 3, 1, 1, (1, 1), (1, 1), (1, 1)))
+        ctx.conv_plan_tune(plan, B)
+        assert ctx.conv_plan_window(plan)["channels_per_wave"] == 1
+        ctx.conv2d(plan, dX, B, None, dY, "none")
+        assert ctx.last_kernel() == "window"
+    Y = dY.download()
+    for co in range(Cout):
+        assert np.array_equal(Y[co], W[co, 4] * X[0, 0, 0]), co
+    ctx.conv_plan_free(plan)
+    for a in (dX, dY, dE):
+        a.free()
+
+
 @pytest.mark.parametrize("Cin,Cout,H,Wi,B,k,s,p,d", [
     (8, 33, 21, 23, 16, (3, 3), (2, 2), (1, 1), (1, 1)), (5, 40, 30, 41, 16, (5, 5), (4, 4), (2, 2), (1, 1)), (6, 32, 19, 33, 8, (3, 3), (2, 2), (2, 2), (2, 3)),
     (9, 36, 17, 2, 4, (3, 2), (1, 2), (1, 0), (1, 1)), (4, 32, 26, 40, 32, (2, 7), (3, 6), (0, 3), (1, 1)), (7, 64, 15, 29, 16, (3, 4), (2, 2), (1, 2), (1, 2))])
