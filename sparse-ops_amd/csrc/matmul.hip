@@ -283,18 +283,32 @@ so_status launch_shared_gather(so_ctx *ctx, const so_ellpack *E, const float *dX
 
 namespace {
 
-// The kernel with X in LDS (csrc/matmul_columns.hip) in place of the row and shared-gather kernels, whose bits it gives: wherever it applies and
-// the longest row has kColumnsNnz nonzeros.  Us, row or shared-gather kernel / this one, one handle launched again and again: 1000 x 512 dense, 32 columns, in
-// the ResNet-18-shaped stack 17.4 / 8.2, one column 17.5 / 7.6; 1337 x 2085 x 1 with rows of 383 12.4 / 6.2; 489 x 4566 x 4, 2033 39.7 / 23.6; 12 x 5634 x 1,
-// 1164 19.2 / 14.2; 17843 x 7108 x 4, 1561 269 / 73; 315 x 140 x 34, 112 5.0 / 4.2; 4634 x 58 x 4, 15 3.6 / 3.5; shorter rows are as fast there, or faster where
-// there are many: 1357 x 26 x 8, 25 4.2 / 4.6, 2120 x 254 x 3, 42 4.3 / 4.7, but 13730 x 105 x 8, 62 8.8 / 4.5.
+// The row kernel, or the shared-gather one, where X is at most as large as LDS.  The longer of two: the longest row's chain, and two thirds of the mean ones
+// that share its SIMD; or the gathers of all nonzeros and the rows' own lines of memory, which long padding spreads; and with many rows the longest one
+// may begin late.  Us; fitted as so_matmul_columns_estimate, and as close.
+double rows_estimate_small_x(const so_ctx *ctx, const so_ellpack *E)
+{
+    const double m = E->m, longest = E->max_nnz, mean = (double)E->total_nnz / m, per_simd = std::min(8.0, m / (4.0 * ctx->compute_units));
+    if (m <= ctx->compute_units && longest >= 128) return 3.0 + 0.0135 * longest;
+    const double chain = longest + 0.63 * mean * std::max(0.0, per_simd - 1.0), lines = m * (1.0 + 0.85 * std::min(1.0, longest / 256.0));
+    return 0.4 + std::max(2.05 + 0.0201 * chain, 1.054e-5 * (double)E->total_nnz + 1.68e-4 * lines) + 0.0153 * longest * std::min(1.0, m / 20000.0);
+}
+
+// The kernel with X in LDS (csrc/matmul_columns.hip) in place of the row and shared-gather kernels, whose bits it gives: where it applies, the longest
+// row has kColumnsNnz nonzeros and it is estimated the faster.  Of 473 launches of up to 400 000 rows, even, skewed or all short but one, the choice
+// was the slower one by more than 5 % in 30, by 13 % on average; the longest row alone chose wrongly in 96, by 22 %.  Us, row or shared-gather kernel / this
+// one, one handle launched again and again: 1000 x 512 dense, 32 columns 11.4 / 8.1, one column 11.7 / 7.5; 1337 x 2085 x 1 with rows of 383 14.5 / 6.8;
+// 489 x 4566 x 4, 2031 41.7 / 24.8; 12 x 5634 x 1, 1147 19.6 / 14.5; 17843 x 7108 x 4, 1500 293 / 79; 315 x 140 x 34, 112 4.7 / 3.9.  Rows of 600, 64
+// columns, of which a workgroup copies 154 KB: 50 000 rows of 8 and one of 64 20.8 / 34.7, 200 000 of 5 and one of 48 55.4 / 138, 50 000 of 60 42.6 / 52.3,
+// 4096 of 150 9.8 / 7.4.  Shorter rows are as fast there, or faster where there are many: 1357 x 26 x 8, 20 3.5 / 3.9, 2120 x 254 x 3, 42 4.2 / 3.9.
 constexpr uint32_t kColumnsNnz = 48;
 
 bool columns_pays(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     if (ctx->tune.matmul_columns >= 0) return ctx->tune.matmul_columns == 1 && so_matmul_columns_applies(ctx, E, C);
     // (an override that asks for one of the row kernels' forms stands)
-    return ctx->tune.matmul_share < 0 && ctx->tune.matmul_vec == 0 && E->max_nnz >= kColumnsNnz && so_matmul_columns_applies(ctx, E, C);
+    return ctx->tune.matmul_share < 0 && ctx->tune.matmul_vec == 0 && E->max_nnz >= kColumnsNnz && so_matmul_columns_applies(ctx, E, C) &&
+           so_matmul_columns_estimate(ctx, E, C) < rows_estimate_small_x(ctx, E);
 }
 
 enum class RbmKernel { None, Merged, Quad, Vector, Planes, Narrow };
@@ -329,7 +343,7 @@ RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t
     const double cus = ctx->compute_units, slabs = so_ceil_div(C, 64), work = (double)E->total_nnz * slabs;
     const bool shared = (double)E->m * slabs <= cus && E->max_nnz >= 128;      // the shared-gather kernel
     *us = 2.5 + std::max(work * 256.0 / 11e6, (shared ? 0.0135 : 0.018) * E->max_nnz + 0.5);
-    if (columns_pays(ctx, E, C)) *us = std::min(*us, so_matmul_columns_estimate(ctx, E, C));
+    if (columns_pays(ctx, E, C)) *us = so_matmul_columns_estimate(ctx, E, C);      // which is then what runs in their place
     RbmKernel k = RbmKernel::None;
     if (merged) {
         // one workgroup per (128 rows, 64 columns, share of the columns): pays when that grid covers most of the chip

@@ -8,12 +8,13 @@
 // the row kernels.
 //
 // What bounds it: about 20 clocks an entry of the longest row on a SIMD of its own (what one wave alone issues), after 3.5 us of launch and the
-// copy of X.
+// copy of X; with many rows the copies, one of all of X per workgroup.
 #include "so_internal.h"
 #include "dpp_steps.h"
 #include "lds_sync.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace {
 
@@ -103,6 +104,16 @@ void ellpack_matmul_columns_kernel(const float *__restrict__ Wd, const uint32_t 
 
 size_t columns_lds(const so_ellpack *E, uint32_t C) { return (((size_t)E->n + 1) * C * 4 + 15) / 16 * 16; }
 
+uint32_t rows_per_wave(uint32_t C) { return C <= 16u ? 4u : C <= 32u ? 2u : 1u; }
+
+// Waves of a workgroup: four while that leaves compute units free, else up to 16 that share one copy of X.
+uint32_t columns_waves(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    uint32_t waves = 4;
+    while (waves < 16 && so_ceil_div(E->m, waves * rows_per_wave(C)) > (uint32_t)ctx->compute_units) waves *= 2;
+    return waves;
+}
+
 template <int RPW>
 so_status launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
@@ -110,9 +121,7 @@ so_status launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, 
     auto k = act == SO_ACT_RELU ? ellpack_matmul_columns_kernel<RPW, SO_ACT_RELU> : act == SO_ACT_SIGMOID ? ellpack_matmul_columns_kernel<RPW, SO_ACT_SIGMOID>
            : act == SO_ACT_TANH ? ellpack_matmul_columns_kernel<RPW, SO_ACT_TANH> : ellpack_matmul_columns_kernel<RPW, SO_ACT_NONE>;
     SO_HIP(so_allow_big_lds(ctx, (const void *)k));
-    // four waves a workgroup while that leaves compute units free, else up to 16 that share one copy of X
-    uint32_t waves = 4;
-    while (waves < 16 && so_ceil_div(E->m, waves * RPW) > (uint32_t)ctx->compute_units) waves *= 2;
+    const uint32_t waves = columns_waves(ctx, E, C);
     k<<<so_ceil_div(E->m, waves * RPW), waves * 64, lds, ctx->stream>>>(E->d_Wd, E->d_idx, E->d_nnz, E->m, E->r, dX, E->n, C, dBias, dY);
     return SO_OK;
 }
@@ -124,13 +133,20 @@ bool so_matmul_columns_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t 
     return C <= 64u && E->total_nnz != 0 && columns_lds(E, C) <= (size_t)ctx->max_lds_bytes;
 }
 
-// 3 us, the longest row at 9.5 ns an entry on a SIMD of its own (8.2 clocks a wave where more than 2.8 share it), 8 ns per KB of X: within 8 % of 55
-// launches of 100 to 1200 entries at up to 4096 rows.
+// 1.9 us, then the longer of two: the longest row at 9.9 ns an entry, and as much for the mean ones that share its SIMD; or, as often as the chip is filled
+// with workgroups, 1.2 us and 10 ns per KB of X that a compute unit's workgroups copy, and a wave's entries -- its longest row's, which is not known here: at
+// most the longest of all, about three or eight times the mean where it takes two or four rows -- at 4.5 ns by wave of a SIMD.  Fitted on 237 launches of 48
+// nonzeros and more in the longest row, up to 400 000 rows even, skewed and all short but one; half of 236 others are within 8 %.
 double so_matmul_columns_estimate(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    const double lds = (double)columns_lds(E, C), cus = ctx->compute_units, rows = C <= 16 ? 4 : C <= 32 ? 2 : 1;
-    const double per_simd = (double)E->m / rows / (4.0 * cus);
-    return std::max(3.6, 3.0 + 0.0095 * E->max_nnz * std::max(1.0, per_simd / 2.8) + 0.008 * lds / 1024.0);
+    const double cus = ctx->compute_units, kb = (double)columns_lds(E, C) / 1024.0, longest = E->max_nnz, mean = (double)E->total_nnz / E->m;
+    const uint32_t rpw = rows_per_wave(C), waves = columns_waves(ctx, E, C);
+    const double wgs = so_ceil_div(E->m, waves * rpw);
+    const double fit = std::max(1.0, std::min(std::floor((double)ctx->max_lds_bytes / (kb * 1024.0)), std::floor(32.0 / waves)));
+    const double filled = std::max(1.0, wgs / (cus * fit)), resident = std::min(fit, wgs / cus);
+    const double entries = std::min(longest, mean * (1.0 + 2.4 * (rpw - 1)) + 8.7) * wgs * waves / (4.0 * cus);
+    const double chain = longest + mean * std::max(0.0, resident * waves / 4.0 / 1.17 - 1.0);
+    return 1.9 + std::max(1.2 + 0.0099 * chain, filled * (1.2 + 0.01 * kb * std::max(1.0, resident)) + 0.0045 * entries);
 }
 
 so_status so_matmul_columns_launch(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)

@@ -74,3 +74,26 @@ def test_chosen(ctx, m, n, C, sp, layouts, kernel):
     rng = np.random.default_rng(9)
     E = datagen.encode_dense(sparse_matrix(rng, m, n, sp))
     assert _run(ctx, E, rng.standard_normal((n, C)).astype(np.float32), None, "none", layouts=layouts)[0] == kernel
+
+
+@pytest.mark.parametrize("m,n,C,mean,longest,layouts,kernel", [
+    (50000, 600, 64, 8, 64, hipabi.LAYOUT_ROW, "row"), (200000, 600, 64, 5, 48, hipabi.LAYOUT_ROW, "row"), (16000, 600, 60, 2, 48, hipabi.LAYOUT_ROW, "row"),
+    (100000, 2000, 16, 6, 64, hipabi.LAYOUT_ROW, "columns"), (4096, 600, 64, 150, 190, hipabi.LAYOUT_ROW, "columns"), (5000, 600, 64, 8, 600, hipabi.LAYOUT_ROW, "columns"),
+    (20000, 600, 64, 60, 64, hipabi.LAYOUT_ROW | hipabi.LAYOUT_RBM, "quad")])
+def test_chosen_by_rows_and_not_by_the_longest_alone(ctx, oracle, m, n, C, mean, longest, layouts, kernel):
+    """Many short rows and a long one: every workgroup copies X for its few rows, which the row kernel's few gathers undercut.
+    With the RBM layout too, whose kernels are compared with the one that would run in their place."""
+    rng = np.random.default_rng(m + C)
+    step = n // longest
+    first = rng.integers(0, step, m).astype(np.uint32)
+    nnz = np.clip(rng.poisson(mean, m), 0, longest).astype(np.uint32)
+    nnz[m // 2] = longest
+    held = np.arange(longest, dtype=np.uint32)[None, :] < nnz[:, None]
+    idx = np.where(held, first[:, None] + np.arange(longest, dtype=np.uint32) * step, 0).astype(np.uint32)
+    Wd = np.where(held, rng.standard_normal((m, longest), dtype=np.float32), np.float32(0))
+    E = datagen.EllpackHost(m, n, longest, Wd, idx, nnz)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    taken, Y = _run(ctx, E, X, None, "none", layouts=layouts)
+    want = oracle.matmul(as_oracle(E), X, None, "none")
+    assert taken == kernel
+    assert np.array_equal(Y, want) if layouts == hipabi.LAYOUT_ROW else rel_err(Y, want) <= 1e-5
