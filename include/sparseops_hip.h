@@ -292,12 +292,15 @@ so_status so_rbm_free(so_ctx *ctx, so_rbm *R);
 so_status so_rbm_dims(const so_rbm *R, uint32_t *M, uint32_t *N, uint32_t *Ct_max, uint32_t *nblocks,
                       uint64_t *total_union, uint64_t *total_pairs);
 /* Attach the format to a convolution plan (ConvAttr::rbm / use_rbm, include/sparse_onnx.hpp:66-98;
- * the reference builds it at load for Cout >= 32 and K >= 64, src/sparse_onnx.cpp:499-502): so_conv2d
- * and so_conv2d_add then run conv2d_rbm_fmajor_implicit's algorithm (src/layers/conv_kernels.cpp:66-147)
- * -- every union column's input operand fetched once and applied to all rows of the block that use
- * it -- whenever the plan has its LDS-windowed layout and B is a multiple of 4, and the per-row
- * kernels otherwise; the results have the same bits either way.  Blocks of at most 8 rows.  R must
- * describe the plan's weights and outlive the plan; NULL detaches.  Not during graph capture. */
+ * the reference builds it at load for Cout >= 32 and K >= 64, src/sparse_onnx.cpp:499-502), which is the
+ * request for its kernel: so_conv2d and so_conv2d_add then run conv2d_rbm_fmajor_implicit's algorithm
+ * (src/layers/conv_kernels.cpp:66-147) -- every union column's input operand fetched once and applied to
+ * all rows of the block that use it -- whenever the plan has its LDS-windowed layout, B is a multiple of 4
+ * and the tensors are 16-byte aligned, and the per-row kernels otherwise; the results have the same bits
+ * either way.  Without the format so_conv2d chooses among the per-row kernels, which are the faster ones
+ * on this chip (7x7 stride-2 stem of a ResNet-18-shaped stack at batch 32 84 us here, 66 there; a 56x56x64
+ * layer at batch 64 144 and 103): attach it to run this algorithm, not for speed.  Blocks of at most 8
+ * rows.  R must describe the plan's weights and outlive the plan; NULL detaches.  Not during graph capture. */
 so_status so_conv_plan_set_rbm(so_ctx *ctx, so_conv_plan *plan, const so_rbm *R);
 /* Inspection aid (no counterpart in the reference): out = {64-byte sets in the plan's streams,
  * real (row, weight) pairs, slots the kernel multiplies through, slots per record}; zeros when

@@ -1037,13 +1037,20 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
     if (g.Cout == 0 || ncols == 0) return SO_OK;
     SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
     SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
+    const uintptr_t align = (uintptr_t)dX | (uintptr_t)dY | (uintptr_t)dResid;
+    // The kernels on an LDS window when the plan carries its layout and the batch splits into tiles of 16, 8 or 4.
+    const uint32_t lpp = window_lpp(B);
+    const bool windowed = plan->win.cc != 0 && lpp != 0 && (align & 15) == 0 && (uint64_t)plan->win.cc * g.H_in * g.W_in * B < (1ull << 31);
+    // The row-block-merged one of them where the plan has been given its format, which is the request for it: SPARSEOPS_CONV_RBM=0 forbids it,
+    // and so does an override for or against the per-row one, unless SPARSEOPS_CONV_RBM=1 asks.
+    const bool merged = windowed && plan->rbm.d_sets && (ctx->tune.conv_rbm == 1 || (ctx->tune.conv_rbm < 0 && ctx->tune.conv_window < 0));
     // The column kernel where the plan has its streams for this batch: below four entries, which the windowed kernel does
     // not take, where it pays against the gather kernel (so_conv_columns_pays), from four on against the windowed one
     // (so_conv_columns_before_window).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
     if (so_conv_columns_for(plan, B) && ctx->tune.conv_columns != 0) {
         const bool alone = B < 4 || (B == 4 && plan->win.cc == 0);           // no windowed kernel: else the gather kernel
         bool use = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
-        if (!use && !alone && ctx->tune.conv_window != 1 && ctx->tune.conv_rbm != 1)
+        if (!use && !alone && !merged && ctx->tune.conv_window != 1)
             use = so_conv_columns_before_window(ctx, plan, B, so_conv_columns_estimate(ctx, plan, B));
         if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for
         bool done = false;
@@ -1056,15 +1063,10 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
         }
     }
     // Batch entries per lane: as many as divide B and keep 16/8-byte alignment.
-    const uintptr_t align = (uintptr_t)dX | (uintptr_t)dY | (uintptr_t)dResid;
     int maxvec = 4;
     if (ctx->tune.conv_vec > 0) maxvec = ctx->tune.conv_vec;
-    // The LDS-windowed kernel when the plan carries its layout and the batch splits into tiles of
-    // 16, 8 or 4 (SPARSEOPS_CONV_WINDOW=1 forces it whenever possible, =0 forbids it: tuning and tests).
-    const uint32_t lpp = window_lpp(B);
-    if (plan->win.cc != 0 && lpp != 0 && (align & 15) == 0 && (uint64_t)plan->win.cc * g.H_in * g.W_in * B < (1ull << 31)) {
-        // the row-block-merged kernel for those who ask for it, on a plan that carries its streams
-        if (plan->rbm.d_sets && ctx->tune.conv_rbm == 1) {
+    if (windowed) {
+        if (merged) {
             bool done = false;
             const so_status s = so_conv_rbm_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done);
             if (s != SO_OK) return s;
@@ -1074,6 +1076,7 @@ static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const fl
                 return SO_OK;
             }
         }
+        // the per-row one: SPARSEOPS_CONV_WINDOW=1 forces it whenever possible, =0 forbids it (tuning and tests)
         const bool forced = ctx->tune.conv_window == 1;
         if (ctx->tune.conv_window != 0) {
             bool done = false;

@@ -523,7 +523,7 @@ extern "C" so_status so_conv_plan_rbm_info(const so_conv_plan *plan, uint64_t ou
 }
 
 // Launches the RBM kernel if the plan carries its streams and the batch suits the windowed layout; *done says whether it did.
-// For those who ask for it (SPARSEOPS_CONV_RBM=1): the per-row windowed kernel is faster everywhere it was measured since its waves take
+// For those who ask for it (so_conv_plan_set_rbm): the per-row windowed kernel is faster everywhere it was measured since its waves take
 // two pixel groups and strided windows lie in column planes.  Us, this one / that one, ResNet-18-shaped layers: 7x7/2 stem at batch 32 and
 // 50 / 80 / 90 % sparse 144 / 115, 84 / 66, 64 / 54, at batch 64 and 60 % 220 / 179, at batch 8 and 80 % 28.2 / 24.7; 56x56x64 at batch 64 and 75 % 144 / 103.
 so_status so_conv_rbm_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,

@@ -35,7 +35,7 @@ struct so_tuning {
     int conv_columns = -1;   // SPARSEOPS_CONV_COLUMNS: 0 forbids the column kernel, 1 forces it on plans tuned for the batch
     int conv_vec = 0;        // SPARSEOPS_CONV_VEC: most batch entries per lane in the gather kernel
     int wait_spins = -1;     // SPARSEOPS_WAIT_SPINS: most polls of a bounded wait on LDS progress counters (0: every wait gives up at once; tests)
-    int conv_rbm = -1;       // SPARSEOPS_CONV_RBM: 1 asks for the row-block-merged kernel on plans that carry its streams
+    int conv_rbm = -1;       // SPARSEOPS_CONV_RBM: 0 forbids the row-block-merged kernel on plans that carry its streams, 1 asks for it against any other override
 };
 
 // Device memory that the library may replace by itself (a workspace that grows, a layout that is rewritten): its kernels

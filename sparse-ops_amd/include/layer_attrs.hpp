@@ -53,7 +53,7 @@ struct ConvAttr {
     std::size_t sentinel_off = 0;
 
     bool fuse_relu = false;
-    RBMPlan rbm{};               // used when use_rbm is set and the plan is non-empty
+    RBMPlan rbm{};               // used when use_rbm is set and the plan is non-empty: its kernel runs then (so_conv_plan_set_rbm)
     bool use_rbm{false};
 
     // Addition: what the conv2d_* entry points keep on the GPU for this layer between calls (the

@@ -75,6 +75,7 @@ struct SparseOnnxModel::Impl {
     void enqueue_layers(const float *in = nullptr, float *out = nullptr) const;
     std::size_t output_layer() const;                        // the layer that makes the model's output; layers.size(): none does
     bool record_pays() const;
+    void set_conv_rbm();                                     // row-block-merged plans for the convolutions, where the environment asks for them
     void launch_chain() const;                               // graph replay or eager
     bool padded() const { return pbatch != batch; }
     void rows_in(const float *d_rows) const;                 // [in_features x batch] -> the input slot (rows padded with zeros)

@@ -6,9 +6,11 @@
 #include "sparse_onnx.hpp"
 
 #include <algorithm>
+#include <cstdlib>
 #include <stdexcept>
 
 #include "model_impl.hpp"
+#include "rbm_conv.hpp"
 
 using namespace sparseops;
 
@@ -53,6 +55,7 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
         // launch graph cannot be recorded across an allocation)
         else if (L.op == Op::MatMul && L.dE) check(so_matmul_reserve(ctx, L.dE, pbatch), "so_matmul_reserve");
     }
+    M.set_conv_rbm();
     if (!M.layers.empty() && M.record_pays()) {
         check(so_graph_begin(ctx), "so_graph_begin");
         try {
@@ -64,6 +67,22 @@ void SparseOnnxModel::resize_buffers(uint32_t batch)
             throw;
         }
         check(so_graph_end(ctx, &M.graph), "so_graph_end");
+    }
+}
+
+// The reference builds its row-block-merged plan for wide convolutions at load (src/sparse_onnx.cpp:499-502: Cout >= 32 and
+// K >= 64, blocks of 8 channels) and never runs it.  Here it is built where SPARSEOPS_CONV_RBM=1 asks for its kernel, which the
+// windowed one beats: looked at by the loader's and every later resize_buffers, as the other overrides are.
+void SparseOnnxModel::Impl::set_conv_rbm()
+{
+    const char *env = std::getenv("SPARSEOPS_CONV_RBM");
+    const bool asked = env && env[0] == '1';
+    so_ctx *ctx = context();
+    for (LayerPlan &L : layers) {
+        if (!L.conv || L.cg.Cout < 32 || L.E->n < 64 || asked == (L.rbm != nullptr)) continue;
+        if (asked) L.rbm = upload_rbm(build_rbm_from_ellpack(*L.E, nullptr, 8));
+        check(so_conv_plan_set_rbm(ctx, L.conv, asked ? L.rbm : nullptr), "so_conv_plan_set_rbm");
+        if (!asked) { so_rbm_free(ctx, L.rbm); L.rbm = nullptr; }
     }
 }
 

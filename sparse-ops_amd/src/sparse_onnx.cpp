@@ -458,8 +458,7 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     std::size_t bias_total = 0;
     // Large fully connected layers run on the RBM layout's kernels (fp32 round-off accuracy, the fastest);
     // SPARSEOPS_MATMUL_RBM=0 at load time keeps every layer on the kernels that give the reference's bits.
-    const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM"), *conv_rbm_env = std::getenv("SPARSEOPS_CONV_RBM");
-    const bool conv_rbm = conv_rbm_env && conv_rbm_env[0] == '1';
+    const char *rbm_env = std::getenv("SPARSEOPS_MATMUL_RBM");
     // So does a model with convolutions that is loaded at a batch below 64, whatever batch it is resized to later: its
     // samples have the same bits in every batch, and its classifier is a few microseconds of the pass.  Loaded at 64 or
     // more it keeps the fast layers at every batch, and a sample's bits then depend on the batch (the kernel is chosen
@@ -470,16 +469,7 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
     for (auto &p : pend) {
         if (p.plan.op != Op::MatMul && p.plan.op != Op::Conv) continue;
         p.plan.dE = mirror(*p.plan.E, p.plan.op == Op::MatMul ? matmul_layouts(*p.plan.E, uint32_t(B0), fast_fc) : SO_LAYOUT_ROW);
-        if (p.plan.op == Op::Conv) {
-            check(so_conv_plan_create(ctx, p.plan.dE, &p.plan.cg, &p.plan.conv), "so_conv_plan_create");
-            // The reference builds its row-block-merged plan for wide convolutions at load
-            // (src/sparse_onnx.cpp:499-502: Cout >= 32 and K >= 64, blocks of 8 channels) and never
-            // runs it; here it is built for those who ask so_conv2d to walk it, which the windowed kernel beats.
-            if (conv_rbm && p.plan.cg.Cout >= 32 && p.plan.E->n >= 64) {
-                p.plan.rbm = upload_rbm(build_rbm_from_ellpack(*p.plan.E, nullptr, 8));
-                check(so_conv_plan_set_rbm(ctx, p.plan.conv, p.plan.rbm), "so_conv_plan_set_rbm");
-            }
-        }
+        if (p.plan.op == Op::Conv) check(so_conv_plan_create(ctx, p.plan.dE, &p.plan.cg, &p.plan.conv), "so_conv_plan_create");
         if (p.plan.has_bias) {
             p.plan.bias_offset = bias_total;
             bias_total += (p.plan.bias.size() + 63) / 64 * 64;
@@ -528,6 +518,7 @@ std::vector<std::string> SparseOnnxModel::describe() const
             s += " " + std::to_string(L.E->m) + "x" + std::to_string(L.E->n) + " r=" + std::to_string(L.E->r) +
                  " nnz=" + std::to_string(nnz) + " act=" + act_name(L.act) + " bias=" + (L.has_bias ? "1" : "0");
             if (L.residual) s += " +residual";
+            if (L.rbm) s += " +rbm";
         } else if (L.op == Op::Act) {
             s += std::string(" act=") + act_name(L.act);
         }

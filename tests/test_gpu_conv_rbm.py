@@ -102,6 +102,42 @@ def test_conv_rbm_reference_vectors(ctx, oracle, golden):
             assert np.array_equal(Y, golden[key % i]) and np.array_equal(Yrow, golden[key % i])
 
 
+@pytest.mark.parametrize("Cin,Cout,H,B", [(64, 40, 14, 16), (64, 64, 4, 8), (16, 33, 12, 4)])
+def test_attaching_the_format_is_the_request_for_its_kernel(ctx, oracle, Cin, Cout, H, B):
+    """Without any override a plan that carries the format runs the row-block-merged kernel (also where the column kernel, which
+    has streams for these batches, would be taken without it); where the override, the batch, the alignment or the missing
+    format rule that out, another kernel."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(Cin + Cout)
+    E = datagen.encode_dense(sparse_matrix(rng, Cout, Cin * 9, .7))
+    g, og = hipabi.conv_geom(Cin, Cout, 3, 3, H, H, (1, 1), (1, 1)), ocg(Cin, Cout, 3, 3, H, H, (1, 1), (1, 1))
+    R = oracle.rbm_build(as_oracle(E), 8)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan, rbm = ctx.conv_plan(dE, g), ctx.upload_rbm(R.M, R.N, R.Ct_max, R.block_union, R.krel, R.colptr, R.pair_row, R.pair_w)
+
+    def run(batch, off=0, **tuning):
+        X = rng.standard_normal((Cin, H, H, batch)).astype(np.float32)
+        mem, dY = ctx.array(np.concatenate([np.zeros(off, np.float32), X.ravel()])), ctx.empty((Cout, H, H, batch))
+        with ctx.tuning(**tuning):
+            ctx.conv2d(plan, mem.offset(off), batch, None, dY, "none")
+        kernel = ctx.last_kernel()
+        assert np.array_equal(dY.download(), oracle.conv2d_pf(as_oracle(E), og, X, batch, None, "none")), (batch, off, tuning)
+        mem.free(), dY.free()
+        return kernel
+
+    ctx.conv_plan_tune(plan, B)
+    without = run(B)
+    ctx.conv_plan_set_rbm(plan, rbm)
+    assert without != "merged-window" and run(B) == "merged-window" and run(B, SPARSEOPS_CONV_WINDOW="0", SPARSEOPS_CONV_RBM="1") == "merged-window"
+    assert run(B, SPARSEOPS_CONV_RBM="0") == without and run(B, SPARSEOPS_CONV_WINDOW="1") == "window"
+    assert run(B, off=1) != "merged-window" and run(B + 1) != "merged-window"
+    ctx.conv_plan_set_rbm(plan, None)
+    assert run(B) == without
+    ctx.conv_plan_free(plan)
+    ctx.rbm_free(rbm)
+    dE.free()
+
+
 def test_conv_rbm_with_fused_residual_add(ctx, oracle):
     from oracle import conv_geom as ocg
     rng = np.random.default_rng(5)

@@ -436,29 +436,36 @@ def test_run_device_cnn(backend, ctx, tmp_path, B):
 
 @pytest.mark.parametrize("B", [32, 16, 6])
 def test_model_runs_the_row_block_merged_plan(backend, oracle, tmp_path, B):
-    """The loader builds the row-block-merged plan for convolutions with Cout >= 32 and K >= 64 (the
-    reference's rule, src/sparse_onnx.cpp:499-502) and hands it to the device library.  With the RBM kernel
-    forced on every launch it fits, forbidden, and left to the library's choice, a ResNet-shaped model gives
-    the same bits, and they are the oracle chain's."""
+    """SPARSEOPS_CONV_RBM=1 makes a model build the row-block-merged plan for convolutions with Cout >= 32 and K >= 64 (the
+    reference's rule, src/sparse_onnx.cpp:499-502) and run its kernel: at load, or from the next resize_buffers on where
+    it is set, or taken back, later.  With it and without, a ResNet-shaped model gives the same bits, and they are
+    the oracle chain's."""
     from graph_oracle import run_graph
     payload, _ = datagen.resnet18_onnx(seed=11, batch=B, hw=64, sparsity=0.8, classes=10, width=32)
+    path = ow.save(str(tmp_path / "r18.onnx"), payload)
     X = np.random.default_rng(4).standard_normal((B, 3, 64, 64)).astype(np.float32)
-    outs = {}
+
+    def plans(model):
+        return sum("+rbm" in line for line in model.describe())
+
+    default = backend.SparseOnnxModel(path)
+    want = default.run(X)
+    assert plans(default) == 0
     try:
-        for mode in ("1", "0", None):
-            if mode is None:
-                os.environ.pop("SPARSEOPS_CONV_RBM", None)
-            else:
-                os.environ["SPARSEOPS_CONV_RBM"] = mode
-            backend.reload_tuning()
-            model = backend.SparseOnnxModel(ow.save(str(tmp_path / "r18.onnx"), payload))
-            outs[mode] = model.run(X)
-            assert np.array_equal(model.run(X), outs[mode])
+        os.environ["SPARSEOPS_CONV_RBM"] = "1"
+        backend.reload_tuning()
+        loaded = backend.SparseOnnxModel(path)
+        default.resize_buffers(B)
+        for model in (loaded, default):
+            assert plans(model) == 19                # all but the projection of 32 channels
+            assert np.array_equal(model.run(X), want) and np.array_equal(model.run(X), want)
     finally:
         os.environ.pop("SPARSEOPS_CONV_RBM", None)
         backend.reload_tuning()
-    assert np.array_equal(outs["1"], outs["0"]) and np.array_equal(outs[None], outs["0"])
-    assert np.array_equal(outs["0"][:2], run_graph(oracle, payload, X[:2]))
+    for model in (loaded, default):
+        model.resize_buffers(B)
+        assert plans(model) == 0 and np.array_equal(model.run(X), want)
+    assert np.array_equal(want[:2], run_graph(oracle, payload, X[:2]))
 
 
 def test_deep_mlp_records_the_row_block_merged_kernel(backend, oracle, tmp_path):
