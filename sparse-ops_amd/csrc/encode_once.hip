@@ -13,7 +13,7 @@
 //
 // The wait for the other workgroups has every one of them resident (a workgroup per compute unit), unless somebody else's
 // kernel holds some of the chip: it gives up after a bounded number of looks, the host is told, and the two passes do
-// the call again.  The words the workgroups tell each other carry the call's number, so nothing needs clearing.
+// the call again, and the context's next ones.  The words the workgroups tell each other carry the call's number, so nothing needs clearing.
 //
 // What bounds it: the read of W (8192 x 8192: 47 to 54 us, by workgroup, of which the copy's rate would take 43), then what
 // follows the slowest workgroup: 4 us until all know of all, 8 to 12 us of writing 61 MB at 90 % sparse; launch and the
@@ -299,6 +299,10 @@ so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t 
     if (entries > kEntryLimit) return SO_OK;
     const size_t lds = (size_t)ctx->max_lds_bytes;
     if (lds < (64u << 10)) return SO_OK;
+    if (ctx->encode_spared != 0) {
+        ctx->encode_spared -= std::min(ctx->encode_spared, (uint64_t)m * n);
+        return SO_OK;
+    }
     static std::atomic<uint32_t> calls{0};
     EncodeArgs a;
     a.W = dDense; a.m = m; a.n = n; a.r_cap = r_cap; a.groups = groups; a.segs = segs;

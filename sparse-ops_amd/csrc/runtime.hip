@@ -92,6 +92,8 @@ extern "C" so_status so_tuning_reload(so_ctx *ctx)
 {
     SO_REQUIRE(ctx != nullptr, "so_tuning_reload: ctx is null");
     read_tuning(ctx->tune);
+    ctx->encode_spared = 0;                    // the bound of the waits may be another
+    ctx->encode_spare_next = kEncodeSpareFirst;
     return SO_OK;
 }
 
@@ -1415,15 +1417,26 @@ extern "C" so_status so_ellpack_encode_noalloc(so_ctx *ctx, const float *dDense,
     SO_REQUIRE(!counts || !ctx->capturing, "so_ellpack_encode_noalloc: r_out/total_nnz_out need a wait, which a graph recording forbids");
     // The kernels leave the counts in pinned host memory themselves: no copy to queue behind them.  A call that waits for them
     // can also be done again by the two passes if the single one says so (its workgroups wait for one another, with a bound).
+    // Somebody else's kernel that made the wait reach its bound, 3 ms, is likely to be there still, or again: calls of 2^30 elements together are then
+    // spared it, of twice as many each further time up to 2^34 (two passes take 0.5 to 2 us more for 2^20 elements: again some 3 ms).
+    const uint64_t spared = ctx->encode_spared;
     if (counts && (uint64_t)m * r_cap != 0) {
         bool once = false;
         so_status s = so_encode_once(ctx, dDense, m, n, r_cap, dNnz, dWd, dIdx, (char *)ctx->static_scratch + kEncodeToldOffset, ctx->h_encode_header, &once);
         if (s == SO_OK && once) s = told_wait(ctx, (uint64_t)m * n, "so_ellpack_encode_noalloc");
         if (s != SO_OK) return s;
-        if (once && ctx->h_encode_header[3] == 0) return encode_counts(ctx, r_cap, r_out, total_nnz_out);
+        if (once && ctx->h_encode_header[3] == 0) {
+            ctx->encode_spare_next = kEncodeSpareFirst;
+            return encode_counts(ctx, r_cap, r_out, total_nnz_out);
+        }
+        if (once) {
+            ctx->encode_spared = ctx->encode_spare_next;
+            ctx->encode_spare_next = std::min(2 * ctx->encode_spare_next, kEncodeSpareMost);
+        }
     }
     const so_status s = encode_launch(ctx, dDense, m, n, ctx->static_scratch, r_cap, dNnz, dWd, dIdx, 0, true,
                                       (uint64_t)m * r_cap != 0, counts ? ctx->h_encode_header : nullptr);
+    if (ctx->encode_spared < spared) ctx->last_kernel = "encode-spared";
     if (s != SO_OK || !counts) return s;
     const so_status waited = told_wait(ctx, (uint64_t)m * n, "so_ellpack_encode_noalloc");
     if (waited != SO_OK) return waited;

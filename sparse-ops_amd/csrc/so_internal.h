@@ -51,6 +51,8 @@ struct so_block {
 };
 using so_block_ref = std::shared_ptr<so_block>;
 
+constexpr uint64_t kEncodeSpareFirst = 1ull << 30, kEncodeSpareMost = 1ull << 34;
+
 struct so_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -65,6 +67,8 @@ struct so_ctx {
     uint32_t *h_wait_gave_up = nullptr;
     bool waits_pending = false;
     uint32_t *h_encode_header = nullptr;   // pinned: {r, total nnz (low, high)} of the last encode that asked for them
+    // After a one-read encode whose workgroups gave up waiting for one another: elements still to be encoded in two passes, and how many the next time
+    uint64_t encode_spared = 0, encode_spare_next = kEncodeSpareFirst;
     // Staging of host arrays (so_stage_in, so_stage_out): pinned memory, the flag of the last way out in it, its bytes in use
     char *h_stage = nullptr;
     uint32_t *d_stage_done = nullptr;      // workgroups of a way out that have finished

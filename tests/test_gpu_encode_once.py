@@ -62,6 +62,25 @@ def test_a_wait_that_gives_up_is_done_again(ctx):
     _check(ctx, W, "encode-once")
 
 
+def test_calls_after_a_wait_that_gave_up_are_spared_it(ctx):
+    """2^30 elements in calls that the kernel would take, then it is tried again and, having given up again, left out for
+    longer; smaller matrices, which it would not take, do not count; a change of the overrides starts anew."""
+    W, small = _matrix(2048, 2100, .2, 5), _matrix(64, 300, .2, 5)
+    dW, dWd, dIdx, dNnz = ctx.array(W), ctx.empty((W.size,)), ctx.empty((W.size,), np.uint32), ctx.empty((2048,), np.uint32)
+    with ctx.tuning(SPARSEOPS_WAIT_SPINS="0"):
+        for spared in (-(-2**30 // W.size), -(-2**31 // W.size)):
+            _check(ctx, W, "encode-twice")
+            _check(ctx, W, "encode-spared")
+            for _ in range(spared - 1):
+                ctx.encode_dense_noalloc(dW, 2048, 2100, 2100, dWd, dIdx, dNnz)
+                assert ctx.last_kernel() == "encode-spared"
+            _check(ctx, small, "encode-twice")
+        _check(ctx, W, "encode-twice")
+    _check(ctx, W, "encode-once")
+    for a in (dW, dWd, dIdx, dNnz):
+        a.free()
+
+
 def test_row_longer_than_the_capacity(ctx):
     W = _matrix(2048, 2100, .2, 6)
     E = datagen.encode_dense(W)
