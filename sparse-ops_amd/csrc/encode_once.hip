@@ -38,6 +38,11 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
 // 16 MB repays (us, two passes / one: 256 x 8192 20.1 / 24.4, 911 x 1901 23.6 / 25.4, 1289 x 6285 30.7 / 28.4, 2048 x 2048 26.8 / 24.1); rows
 // well below three groups of 256 columns leave lanes idle (16384 x 520 35.5 / 40.2, 40000 x 600 60.2 / 69.4, 6549 x 786 35.3 / 31.3); and few
 // rows divide badly over the workgroups (520 rows, three on some, two on most: 22.5 / 24.2; 512 rows 30.5 / 27.4).
+//
+// No upper size: beyond what LDS holds (6.7 M nonzeros) the gain goes, but little is lost.  Us, two passes / one: 16384 x 16384 with 5 / 10 / 50 % kept
+// 418 / 350, 454 / 438, 664 / 675; 32768 x 16384 with 2 / 10 / 50 % 769 / 605, 880 / 910, 1287 / 1336; 32768 x 32768 1518 / 1427, 1811 / 1838, 2489 / 2359;
+// few long rows gain most (256 x 100 000 at 10 % 64 / 42, 4 x 2 000 000 685 / 348).  Not settled: rows whose last group is mostly empty, at few
+// nonzeros, 50 001 x 800 with 5 / 10 / 50 % 74 / 83, 77 / 83, 128 / 109; 500 000 x 800 665 / 706, 747 / 836, 1220 / 1065: how many are kept is not known before.
 constexpr uint64_t kLeastElements = 4u << 20;
 constexpr uint32_t kLeastColumns = 768;
 
