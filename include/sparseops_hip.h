@@ -248,7 +248,8 @@ so_status so_conv_plan_free(so_ctx *ctx, so_conv_plan *plan);
 /* Re-sizes the plan's internal layouts for launches with batch B (how many output channels
  * a wave takes depends on how many workgroups the batch yields).  Optional: results never
  * depend on it; plans are created for batch 32.  For a batch of one to four, and of 8, 16 or 32
- * where it is estimated to pay, it also makes the column kernel's streams for exactly that batch, once; they stay until the plan is freed.
+ * where it is estimated to pay or SPARSEOPS_CONV_COLUMNS=1 asks, it also makes the column kernel's streams for exactly
+ * that batch, once; they stay until the plan is freed.
  * Not to be called while a launch that uses the plan may be in flight on another stream, nor during
  * graph capture (it allocates).  A graph recorded with the plan before is recorded again afterwards
  * (SparseOnnxModel::resize_buffers does), unless the new batch falls into the same four-entry step.

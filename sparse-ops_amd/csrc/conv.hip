@@ -980,8 +980,8 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
         window = lpp != plan->win.lpp || choose_cpw(ctx, plan->win, plan->g.Cout, run, batch) != plan->win.cpw * (int)plan->win.px;
     }
     const int slot = so_conv_columns_slot(B);
-    const bool columns = slot >= 0 && !plan->col_tried[slot];
-    if (!window && !columns) { plan->tuned_batch = batch; return SO_OK; }
+    auto columns = [&] { return slot >= 0 && !plan->col_tried[slot] && so_conv_columns_wanted(ctx, plan, B); };
+    if (!window && !columns()) { plan->tuned_batch = batch; return SO_OK; }
     const size_t slots = (size_t)E->m * E->r;
     std::vector<uint32_t> idx(slots), nnz(E->m);
     std::vector<float> Wd(slots);
@@ -995,7 +995,7 @@ extern "C" so_status so_conv_plan_tune(so_ctx *ctx, so_conv_plan *plan, uint32_t
         if (s != SO_OK) return s;
     }
     plan->tuned_batch = batch;
-    if (columns) {                                      // (looks at the window's layout)
+    if (columns()) {                                    // (looks at the window's layout)
         s = so_conv_columns_build(ctx, plan, idx, nnz, Wd, B);
         if (s != SO_OK) return s;
         plan->col_tried[slot] = true;

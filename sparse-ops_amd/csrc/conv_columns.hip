@@ -230,15 +230,12 @@ const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B)
     return slot >= 0 && plan->col[slot].batch == B ? &plan->col[slot] : nullptr;
 }
 
-// Sizes the tile for batch B and uploads the entry streams; leaves the plan without them where the kernel does not apply.
-so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
-                                const std::vector<float> &Wd, uint32_t B)
+// The tile and the window for batch B, without streams; false where the kernel does not apply.
+static bool columns_geometry(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, so_conv_columns &c)
 {
     const so_conv_geom &g = plan->g;
     const so_ellpack *E = plan->E;
-    const int slot = so_conv_columns_slot(B);
-    if (slot < 0 || E->r == 0 || E->total_nnz == 0 || !E->ascending || (size_t)ctx->max_lds_bytes < kColLds) return SO_OK;
-    so_conv_columns c;
+    if (so_conv_columns_slot(B) < 0 || E->r == 0 || E->total_nnz == 0 || !E->ascending || (size_t)ctx->max_lds_bytes < kColLds) return false;
     const uint32_t px = 64u / B, sth = window_step(g.kH, g.stride_h), stw = window_step(g.kW, g.stride_w);
     uint64_t best_tiles = ~0ull, best_win = ~0ull;
     for (uint32_t th = 1; th <= px && th <= g.H_out; ++th)
@@ -247,7 +244,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
             const uint64_t win = (uint64_t)((th - 1) * sth + (g.kH - 1) * g.dil_h + 1) * ((tw - 1) * stw + (g.kW - 1) * g.dil_w + 1);
             if (tiles < best_tiles || (tiles == best_tiles && win < best_win)) { best_tiles = tiles; best_win = win; c.TH = th; c.TW = tw; }
         }
-    if (c.TH == 0) return SO_OK;
+    if (c.TH == 0) return false;
     c.tiles_x = so_ceil_div(g.W_out, c.TW);
     c.tiles_y = so_ceil_div(g.H_out, c.TH);
     const uint32_t IH = (c.TH - 1) * sth + (g.kH - 1) * g.dil_h + 1, IW = (c.TW - 1) * stw + (g.kW - 1) * g.dil_w + 1;
@@ -257,16 +254,35 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
     c.IP = share ? IW - 1 : IW;
     c.PE = (IH - 1) * c.IP + IW;
     const uint64_t plane = (uint64_t)c.PE * B;
-    if (plane * 4 * 2 > kColLds) return SO_OK;
+    if (plane * 4 * 2 > kColLds) return false;
     c.cc = (uint32_t)std::min<uint64_t>(g.Cin, kColLds / (plane * 4) - 1);
     c.nch = so_ceil_div(g.Cin, c.cc);
     c.cc = so_ceil_div(g.Cin, c.nch);
     // window_div: operand * divisor below 2^32
-    if ((uint64_t)c.tiles_x * c.tiles_x * c.tiles_y >= (1ull << 32) || plane * plane >= (1ull << 32) || plane * 1024 >= (1ull << 32)) return SO_OK;
-    if ((uint64_t)c.tiles_x * c.tiles_y >= (1ull << 31) || ((uint64_t)c.cc + 1024) * g.H_in * g.W_in * B >= (1ull << 30)) return SO_OK;
+    if ((uint64_t)c.tiles_x * c.tiles_x * c.tiles_y >= (1ull << 32) || plane * plane >= (1ull << 32) || plane * 1024 >= (1ull << 32)) return false;
+    if ((uint64_t)c.tiles_x * c.tiles_y >= (1ull << 31) || ((uint64_t)c.cc + 1024) * g.H_in * g.W_in * B >= (1ull << 30)) return false;
     c.batch = B;
-    // at more than four entries no streams for a plan whose windowed layout the kernel would not be taken before
-    if (B > 4 && ctx->tune.conv_columns != 1 && !so_conv_columns_before_window(ctx, plan, B, column_shape(ctx, plan, c).us)) return SO_OK;
+    return true;
+}
+
+// At more than four entries no streams for a plan whose windowed layout the kernel would not be taken before: looked at anew by every tuning,
+// since the layout and the overrides may be others by then.
+bool so_conv_columns_wanted(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B)
+{
+    so_conv_columns c;
+    if (!columns_geometry(ctx, plan, B, c)) return false;
+    return B <= 4 || ctx->tune.conv_columns == 1 || so_conv_columns_before_window(ctx, plan, B, column_shape(ctx, plan, c).us);
+}
+
+// Uploads the entry streams for batch B; leaves the plan without them where the kernel does not apply.
+so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
+                                const std::vector<float> &Wd, uint32_t B)
+{
+    const so_conv_geom &g = plan->g;
+    const so_ellpack *E = plan->E;
+    so_conv_columns c;
+    if (!columns_geometry(ctx, plan, B, c)) return SO_OK;
+    const uint64_t plane = (uint64_t)c.PE * B;
     const uint32_t kHW = g.kH * g.kW;
     const size_t runs = (size_t)E->m * c.nch;
     std::vector<uint32_t> first(runs + 1);      // entries of every (channel, chunk), then groups, then where they begin
@@ -318,7 +334,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
         if (c.d_first) (void)hipFree(c.d_first);
         return s;
     }
-    plan->col[slot] = c;
+    plan->col[so_conv_columns_slot(B)] = c;
     return SO_OK;
 }
 

@@ -57,12 +57,13 @@ struct so_conv_plan {
     int2 *d_taps = nullptr;  // per slot: x = (cin*H + dh)*W + dw (elements of B floats), y = dh<<16 | (dw & 0xffff)
     so_conv_window win;      // win.cc == 0: not built
     so_conv_rbm rbm;         // rbm.d_sets == nullptr: no streams
-    so_conv_columns col[kColSlots];      // streams by so_conv_columns_slot, made by the first tuning for the batch and kept: graphs may replay with them
-    bool col_tried[kColSlots] = {};      // that tuning has happened, whether the kernel applies or not
+    so_conv_columns col[kColSlots];      // streams by so_conv_columns_slot, made by the first tuning for the batch that wants them and kept: graphs may replay with them
+    bool col_tried[kColSlots] = {};      // they have been made, or could not be
 };
 
 // conv_columns.hip
 void so_conv_columns_free(so_conv_plan *plan);
+bool so_conv_columns_wanted(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);          // streams for the batch pay
 so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vector<uint32_t> &idx, const std::vector<uint32_t> &nnz,
                                 const std::vector<float> &Wd, uint32_t B);
 const so_conv_columns *so_conv_columns_for(const so_conv_plan *plan, uint32_t B);  // null: the plan has no streams for the batch

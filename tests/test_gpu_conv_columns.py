@@ -90,6 +90,28 @@ def test_columns_or_window(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel):
         a.free()
 
 
+def test_declined_by_estimate_is_not_for_good(ctx, oracle):
+    """A plan tuned for a batch of 16 without streams, since the windowed kernel is estimated ahead, gets them when it is tuned
+    again under SPARSEOPS_CONV_COLUMNS=1; without the override the estimate decides as before."""
+    from oracle import conv_geom as ocg
+    rng = np.random.default_rng(61)
+    E = datagen.encode_dense(sparse_matrix(rng, 128, 128 * 9, .8))
+    args = 128, 128, 3, 3, 12, 12, (1, 1), (1, 1), (1, 1)
+    g, og = hipabi.conv_geom(*args), ocg(*args)
+    X = rng.standard_normal((128, 12, 12, 16)).astype(np.float32)
+    dE = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r)
+    plan, dX, dY = ctx.conv_plan(dE, g), ctx.array(X), ctx.empty((128, 12, 12, 16))
+    want = oracle.conv2d_pf(as_oracle(E), og, X, 16, None, "none")
+    for asked, kernel in ((None, "window"), ("1", "columns"), (None, "window"), ("1", "columns")):
+        with ctx.tuning(SPARSEOPS_CONV_COLUMNS=asked):
+            ctx.conv_plan_tune(plan, 16)
+            ctx.conv2d(plan, dX, 16, None, dY, "none")
+        assert ctx.last_kernel() == kernel and np.array_equal(dY.download(), want)
+    ctx.conv_plan_free(plan)
+    for a in (dX, dY, dE):
+        a.free()
+
+
 @pytest.mark.parametrize("Cin,H", [(34, 9), (400, 18)])            # one chunk and several
 def test_columns_groups_per_run(ctx, oracle, Cin, H):
     """Runs of no group of 16 entries up to three blocks of eight, one entry more or fewer: what a block, the rest behind it
