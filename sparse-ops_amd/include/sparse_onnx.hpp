@@ -65,6 +65,8 @@ public:
     std::vector<std::size_t> output_shape() const;
     std::vector<std::size_t> input_shape() const;
     uint32_t batch() const;
+    /// Whether the chain of the current batch is replayed from a launch graph (else it is launched layer by layer).
+    bool recorded() const;
     std::size_t input_features() const;
     std::size_t output_features() const;
 

@@ -423,6 +423,21 @@ def test_run_device_in_callers_memory(backend, ctx, tmp_path, graph, layers):
     mem.free()
 
 
+def test_model_crosses_the_line_between_graph_and_launches(backend, ctx, tmp_path):
+    """Left to itself a model replays a short chain from a launch graph and launches a long one layer by layer, on the caller's
+    memory in run_device: one model resized over that line and back, each way called twice, with the same bits."""
+    payload, _ = datagen.resnet18_onnx(seed=6, batch=4, hw=128, sparsity=0.8, classes=10, width=32)
+    model = backend.SparseOnnxModel(ow.save(str(tmp_path / "r18.onnx"), payload))
+    X = np.random.default_rng(6).standard_normal((32, 3, 128, 128)).astype(np.float32)
+    Y = np.concatenate([model.run(X[i:i + 4]) for i in range(0, 32, 4)])
+    for B, recorded in ((1, True), (32, False), (4, True), (32, False), (1, True)):
+        model.resize_buffers(B)
+        assert model.recorded() == recorded, B
+        for at in (0, 32 - B):
+            assert np.array_equal(model.run(X[at:at + B]), Y[at:at + B])
+            assert np.array_equal(_run_device(model, ctx, X[at:at + B]), Y[at:at + B])
+
+
 @pytest.mark.parametrize("B", [32, 5])
 def test_run_device_cnn(backend, ctx, tmp_path, B):
     """run_device on a ResNet-shaped stack at a batch carried as is (32) and one carried padded (5)."""
