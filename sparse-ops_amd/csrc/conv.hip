@@ -274,8 +274,10 @@ __device__ __forceinline__ void touch_stream(const int4 *p, uint32_t quads, uint
 // PX pixel groups per wave.  With scalar entries a multiply-add whose weight is a scalar operand takes the vector unit 3.3 clocks, one of
 // three vector registers 2.5: a wave that applies an entry to two pixel groups moves its weight to a vector register once for
 // eight multiply-adds, and the loop around them -- scalar loads, shifts, counters -- turns half as often.  Vector instructions were
-// what bounded the step loop; now LDS reads are (6.8 of the 8.3 us of a chunk of a 56x56x64 layer).  ResNet-18-shaped layers
-// at batch 32, PX 1 with twice the channels per wave / PX 2, us: 56x56x64 52.7-56.2 / 45.8-51.1, 28x28x128 53.0-54.5 / 46.0-46.5, the whole stack 1043 / 988.
+// what bounded the step loop; now LDS is the busier: it is active in 63 to 69 % of a compute unit's busy clocks on the 56x56x64 and
+// 28x28x128 layers, 4.0 clocks a read without conflicts, and in 66 to 71 % on the 14x14 and 7x7 ones, a sixth of it conflicts.
+// ResNet-18-shaped layers at batch 32, PX 1 with twice the channels per wave / PX 2, us: 56x56x64 52.7-56.2 / 45.8-51.1, 28x28x128
+// 53.0-54.5 / 46.0-46.5, the whole stack 1043 / 988.
 //
 // The four waves that share a SIMD are served oldest first: left alone, the first of them finishes a
 // chunk's steps in half the time of the last (measured with the shader clock on the 56x56x64 layer:
@@ -1012,12 +1014,20 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
     return SO_OK;
 }
 
-// Whether the column kernel, at four entries or more, is taken before the windowed one: where its shorter chains on more waves win.  The windowed kernel's time
-// is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip (batch 4: 7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4);
-// at 8, 16 and 32 entries, looked at where its waves have one channel each, which they have on small images, 3.8 us, 1 a chunk of channels and 16 ns (8
-// entries) or 20.5 per nonzero.  Us windowed / column: 2x2x256 with 921 nonzeros a row at batch 8 / 16 / 32 19.8 / 14.2, 28.3 / 16.3, 28.9 / 18.9; 4x4x128
-// with 461 12.5 / 9.4, 18.0 / 10.2, 18.0 / 12.4; 8x8x64 with 231 8.7 / 6.8, 10.9 / 7.0, 11.2 / 8.0; 3x3x512 with 921 24.3 / 18.6, 36.0 / 25.8, 36.0 / 41.6; 8x8x64 with 58 6.0 / 5.1, 7.3 / 5.5, 7.5 / 6.1;
-// 8x8x256 with 690 21.2 / 16.6, 27.6 / 22.4, 31.6 / 51.1; 7x7x512 with 921 29.9 / 34.4, 44.5 / 72, 59 / 160.
+// Whether the column kernel, at four entries or more, is taken before the windowed one: where its shorter chains on more waves win.
+// At four entries the windowed kernel's time is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip
+// (7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4).
+// At 8, 16 and 32, looked at where its waves have one channel each, which they have on small images, it is 3.8 us, 1 a chunk of
+// channels and 16 ns (8 entries) or 20.5 per nonzero.  Us, windowed / column:
+//
+//   image, nonzeros a row     batch 8        batch 16       batch 32
+//   2x2x256     921           19.8 / 14.2    28.3 / 16.3    28.9 / 18.9
+//   3x3x512     921           24.3 / 18.6    36.0 / 25.8    36.0 / 41.6
+//   4x4x128     461           12.5 /  9.4    18.0 / 10.2    18.0 / 12.4
+//   7x7x512     921           29.9 / 34.4    44.5 / 72      59   / 160
+//   8x8x64      231            8.7 /  6.8    10.9 /  7.0    11.2 /  8.0
+//   8x8x64       58            6.0 /  5.1     7.3 /  5.5     7.5 /  6.1
+//   8x8x256     690           21.2 / 16.6    27.6 / 22.4    31.6 / 51.1
 bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us)
 {
     const so_conv_window &w = plan->win;

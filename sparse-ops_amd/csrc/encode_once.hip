@@ -17,9 +17,12 @@
 //
 // What bounds it: the read of W (8192 x 8192: 47 to 54 us, by workgroup, of which the copy's rate would take 43), then what
 // follows the slowest workgroup: 4 us until all know of all, 8 to 12 us of writing 61 MB at 90 % sparse; launch and the
-// host's wait 13.  The whole call on one matrix again and again, two passes / this one, us: 8192 x 8192 at 98 / 90 / 80 / 50 % sparse 100 / 75, 112 / 85, 135 / 108, 195 / 175
-// (6.7 M nonzeros fill the LDS; at 50 % seven pieces of eight are read again), 4096 x 4096 at 90 % 45 / 36, 2048 x 2048 27 / 24;
-// on changing matrices 8192 x 8192 at 90 % 127.6 / 91.9.
+// host's wait 13.  Memory moves 269 MB in, W once, and 61 out (counters); at 50 % sparse, where LDS keeps one piece of eight, 450 in.
+// The whole call on one matrix again and again, two passes / this one, us:
+//
+//   8192 x 8192 at 98 / 90 / 80 / 50 % sparse    100 / 75, 112 / 85, 135 / 108, 195 / 175
+//   4096 x 4096, 2048 x 2048 at 90 %              45 / 36,  27 / 24
+//   8192 x 8192 at 90 %, changing matrices       127.6 / 91.9
 #include "so_internal.h"
 
 #include <atomic>

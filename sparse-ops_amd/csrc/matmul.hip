@@ -294,13 +294,20 @@ double rows_estimate_small_x(const so_ctx *ctx, const so_ellpack *E)
     return 0.4 + std::max(2.05 + 0.0201 * chain, 1.054e-5 * (double)E->total_nnz + 1.68e-4 * lines) + 0.0153 * longest * std::min(1.0, m / 20000.0);
 }
 
-// The kernel with X in LDS (csrc/matmul_columns.hip) in place of the row and shared-gather kernels, whose bits it gives: where it applies, the longest
-// row has kColumnsNnz nonzeros and it is estimated the faster.  Of 473 launches of up to 400 000 rows, even, skewed or all short but one, the choice
-// was the slower one by more than 5 % in 30, by 13 % on average; the longest row alone chose wrongly in 96, by 22 %.  Us, row or shared-gather kernel / this
-// one, one handle launched again and again: 1000 x 512 dense, 32 columns 11.4 / 8.1, one column 11.7 / 7.5; 1337 x 2085 x 1 with rows of 383 14.5 / 6.8;
-// 489 x 4566 x 4, 2031 41.7 / 24.8; 12 x 5634 x 1, 1147 19.6 / 14.5; 17843 x 7108 x 4, 1500 293 / 79; 315 x 140 x 34, 112 4.7 / 3.9.  Rows of 600, 64
-// columns, of which a workgroup copies 154 KB: 50 000 rows of 8 and one of 64 20.8 / 34.7, 200 000 of 5 and one of 48 55.4 / 138, 50 000 of 60 42.6 / 52.3,
-// 4096 of 150 9.8 / 7.4.  Shorter rows are as fast there, or faster where there are many: 1357 x 26 x 8, 20 3.5 / 3.9, 2120 x 254 x 3, 42 4.2 / 3.9.
+// The kernel with X in LDS (csrc/matmul_columns.hip) in place of the row and shared-gather kernels, whose bits it gives: where it applies,
+// the longest row has kColumnsNnz nonzeros and it is estimated the faster.  Of 473 launches of up to 400 000 rows, even, skewed or all short
+// but one, the choice was the slower one by more than 5 % in 30, by 13 % on average; the longest row alone chose wrongly in 96, by 22 %.
+// Us, row or shared-gather kernel / this one, one handle launched again and again, rows x columns x dense columns:
+//
+//   even rows of    512    1000 x 512 x 32   11.4 /  8.1    1000 x 512 x 1     11.7 /  7.5
+//                   383    1337 x 2085 x 1   14.5 /  6.8
+//                  2031    489 x 4566 x 4    41.7 / 24.8
+//                  1147    12 x 5634 x 1     19.6 / 14.5
+//                  1500    17843 x 7108 x 4   293 / 79
+//                   112    315 x 140 x 34     4.7 /  3.9
+//                   150    4096 x 600 x 64    9.8 /  7.4      60   50 000 x 600 x 64   42.6 / 52.3  (a workgroup copies 154 KB)
+//   short, one long        50 000 x 600 x 64 rows of 8 and one of 64   20.8 / 34.7     200 000, of 5 and one of 48   55.4 / 138
+//   below kColumnsNnz      1357 x 26 x 8, 20  3.5 /  3.9    2120 x 254 x 3, 42  4.2 / 3.9; faster where there are many rows
 constexpr uint32_t kColumnsNnz = 48;
 
 bool columns_pays(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
