@@ -90,8 +90,8 @@ inline uint32_t window_lpp(uint32_t B) { return B % 16 == 0 ? 4u : B % 8 == 0 ? 
 
 struct WinArgs {
     uint32_t TH, TW, IH, IW, cc, nch, tiles_x, pg, cg, groups;
-    uint32_t mYZ = 0, mZ = 0;        // window_magic of gy * gz and gz; mYZ is 0 where that is 1 or the ids are too many
-    uint32_t wgs, per_xcd, gy, gz;   // workgroups in all and per XCD (0: ids as launched); channel blocks and batch tiles (window_workgroup)
+    uint32_t wgs, per_xcd;           // workgroups in all and per XCD (0: ids as launched)
+    uint32_t yz, gz, mYZ = 0, oneYZ = 0, mZ = 0, oneZ = 0;   // (channel block, batch tile) pairs and batch tiles: window_magic, and all ones where that is one
     uint32_t win_f4;    // float4 elements of one chunk's window
     uint32_t buf_f4;    // window plus the zero plane: stride between the two buffers
     uint32_t nbuf;      // 2: double-buffered windows; 1: a single chunk, nothing to overlap
@@ -122,7 +122,7 @@ inline uint32_t window_subsample(uint32_t k, uint32_t stride) { return k == 1 ? 
 // write of 25.7 MB at the end of a layer 7 / 4), the stem 84.4 / 80.7, the stack 988 / 967.
 //
 // A launch has fewer than 2^32 work items along a dimension, so fewer than 2^22 workgroups of 1024: a grid whose product does not stay below
-// that keeps its ids in (x, y, z), each of which then has to.
+// that, or whose ids window_magic cannot divide, keeps them in (x, y, z), each of which then has to.
 struct WinPlace { uint32_t tile, y, z; };
 constexpr uint64_t kWinMaxGrid = (1ull << 32) / kWinThreads;
 // Sets the shares for `grid`; the grid to launch is window_grid(a, grid).  False: no launch can have it.
@@ -130,36 +130,28 @@ inline bool window_shares(WinArgs &a, dim3 grid)
 {
     if (grid.x >= kWinMaxGrid || grid.y > 65535u || grid.z > 65535u) return false;
     const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z, yz = (uint64_t)grid.y * grid.z;
-    a.gy = grid.y; a.gz = grid.z;
+    a.yz = (uint32_t)yz; a.gz = grid.z;
     a.wgs = a.per_xcd = 0;
-    if ((wgs + 7) / 8 * 8 >= kWinMaxGrid) return true;
+    if ((wgs + 7) / 8 * 8 >= kWinMaxGrid || wgs * yz >= (1ull << 32) || yz * a.gz >= (1ull << 32)) return true;
     a.wgs = (uint32_t)wgs;
     a.per_xcd = (uint32_t)((wgs + 7) / 8);
-    a.mYZ = wgs * yz < (1ull << 32) && yz * a.gz < (1ull << 32) ? window_magic((uint32_t)yz) : 0u;
-    a.mZ = window_magic(a.gz);
+    a.mYZ = window_magic((uint32_t)yz); a.oneYZ = yz == 1 ? ~0u : 0u;
+    a.mZ = window_magic(a.gz); a.oneZ = a.gz == 1u ? ~0u : 0u;
     return true;
 }
 inline dim3 window_grid(const WinArgs &a, dim3 grid) { return a.per_xcd != 0u ? dim3(8u * a.per_xcd) : grid; }
 __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 {
-    if (a.per_xcd == 0u) {
+    if (__builtin_expect(a.per_xcd == 0u, 0)) {
         p.tile = blockIdx.x; p.y = blockIdx.y; p.z = blockIdx.z;
         return true;
     }
-    const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3), yz = a.gy * a.gz;
-    if (id >= a.wgs) return false;
-    if (a.mYZ != 0u) {
-        p.tile = __umulhi(id, a.mYZ);
-        const uint32_t rest = id - p.tile * yz;
-        p.y = a.gz == 1u ? rest : __umulhi(rest, a.mZ);
-        p.z = rest - p.y * a.gz;
-    } else {
-        p.tile = id / yz;
-        const uint32_t rest = id - p.tile * yz;
-        p.y = rest / a.gz;
-        p.z = rest - p.y * a.gz;
-    }
-    return true;
+    const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3);
+    p.tile = __umulhi(id, a.mYZ) + (id & a.oneYZ);
+    const uint32_t rest = id - p.tile * a.yz;
+    p.y = __umulhi(rest, a.mZ) + (rest & a.oneZ);
+    p.z = rest - p.y * a.gz;
+    return id < a.wgs;
 }
 
 // With an even stride along a row the lanes' reads of one tap would all fall on even (fourth, ...) window columns, half of the LDS's banks
@@ -171,7 +163,7 @@ __device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
 __device__ __forceinline__ uint32_t window_column(const WinArgs &a, uint32_t at)
 {
     const uint32_t plane = __umulhi(at, a.mPW);                      // mPW is 0 for a single plane
-    return (at - plane * a.PW) * a.planes + plane;
+    return __umul24(at - __umul24(plane, a.PW), a.planes) + plane;
 }
 // The same for a tap: where column kw of a tap lies, from an output pixel's corner on.
 inline uint32_t window_tap_place(const so_conv_window &w, uint32_t kw) { return kw % w.planes * w.PW + kw / w.planes; }
