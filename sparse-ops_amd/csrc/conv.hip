@@ -1033,8 +1033,9 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
 // Whether the column kernel, at four entries or more, is taken before the windowed one: where its shorter chains on more waves win.
 // At four entries the windowed kernel's time is about 5.5 us + 20.5 ns per nonzero of a row while its grid fits the chip
 // (7x7x512 27.6 against 22.8 us, 14x14x256 17.5 against 24.4).
-// At 8, 16 and 32, looked at where its waves have one channel each, which they have on small images, it is 3.8 us, 1 a chunk of
-// channels and 16 ns (8 entries) or 20.5 per nonzero.  Us, windowed / column:
+// At 8, 16 and 32, looked at where its waves have one channel each, it is 1.7 us and, for every round of workgroups, 1.6, 1.2 a chunk of channels
+// and 43 ns (8 entries) or 59 per nonzero where all 16 waves of a workgroup compute, which share its LDS, down to a third where few do.  Of 351
+// layers of up to 128x128 and 512 channels 219 go to the column kernel; 18 take the slower one by more than 5 %, by 11 % on average.  Us, windowed / column:
 //
 //   image, nonzeros a row     batch 8        batch 16       batch 32
 //   2x2x256     921           19.8 / 14.2    28.3 / 16.3    28.9 / 18.9
@@ -1044,13 +1045,22 @@ extern "C" so_status so_conv_plan_window(const so_conv_plan *plan, uint32_t out[
 //   8x8x64      231            8.7 /  6.8    10.9 /  7.0    11.2 /  8.0
 //   8x8x64       58            6.0 /  5.1     7.3 /  5.5     7.5 /  6.1
 //   8x8x256     690           21.2 / 16.6    27.6 / 22.4    31.6 / 51.1
+//   few channels on large images: 120x120x11 to 4, 1x1, 6.5 at batch 32 14.0 / 23.4; 111x111x5 to 4, 20 at 32 15.0 / 23.2; 88x88x26 to 2, 24 at 8 4.8 / 6.9
 bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us)
 {
     const so_conv_window &w = plan->win;
     if (w.cc == 0 || (B > 4 && w.cpw * (int)w.px != 1)) return false;
-    const double rounds = so_ceil_div(window_workgroups(w, plan->g.Cout, (uint32_t)w.cpw * w.px, B), (uint64_t)ctx->compute_units);
-    const double row = (double)plan->E->total_nnz / plan->g.Cout;
-    return columns_us < rounds * (B <= 4 ? 0.9 * (5.5 + 0.0205 * row) : 0.95 * (3.8 + w.nch + (B == 8 ? 0.016 : 0.0205) * row));
+    const double cus = ctx->compute_units, row = (double)plan->E->total_nnz / plan->g.Cout;
+    if (B <= 4) {
+        const double rounds = so_ceil_div(window_workgroups(w, plan->g.Cout, (uint32_t)w.cpw * w.px, B), (uint64_t)ctx->compute_units);
+        return columns_us < 0.9 * rounds * (5.5 + 0.0205 * row);
+    }
+    // the grid as window_launch makes it
+    const uint32_t lpp = window_lpp(B), pg = so_ceil_div(w.TH * w.TW, 64u / lpp), spatial = w.tiles_x * w.tiles_y * (B / (4 * lpp));
+    uint32_t cg = 16u / pg;
+    while (cg > 1 && cg % 2 == 0 && (double)spatial * so_ceil_div(w.groups, cg) <= cus / 2) cg /= 2;
+    const double rounds = std::ceil((double)spatial * so_ceil_div(w.groups, cg) / cus), waves = std::min(cg, w.groups) * pg;
+    return columns_us < 0.95 * (1.7 + rounds * (1.6 + 1.18 * w.nch + (B == 8 ? 0.0435 : 0.059) * row * std::max(0.35, waves / 16.0)));
 }
 
 static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,

@@ -192,9 +192,13 @@ struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 
 // Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
 // longest chain at 10 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
-// more waves than compute.  From 8 entries on, where windows of few pixels are the rule, a chunk's start-up goes by its LDS: 0.5 us and 17 ns per KB
-// (batch 16, start-up and chunks in front of the chain: 66 KB 1.9 us, 131 KB 2.8, twice 131 KB 4.5).  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
+// more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
 // 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
+//
+// From 8 entries on windows of few pixels are the rule, and many workgroups of few channels on large images: 2.75 us; a chunk's start-up by its
+// LDS, 0.44 us and 24 ns per KB, 9 more for every further workgroup on the compute unit; 0.5 us for each of those, 2.2 for every further filling of the
+// chip; chains at 8.3 ns an entry, 5.9 per wave.  Fitted on 500 layers of up to 128x128 and 512 channels at batches of 8, 16 and 32: half are
+// within 7 %.
 ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
 {
     const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
@@ -206,8 +210,13 @@ ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv
         const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
         const double resident = std::min(fit, std::ceil(wgs / cus));
         s.rounds = std::ceil(wgs / (cus * fit));
-        const double start = c.batch <= 4 ? 2.5 + c.nch : c.nch * (0.5 + 0.017 * s.lds / 1024.0);
-        s.us = 3.0 + s.rounds * (start + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        if (c.batch <= 4) {
+            s.us = 3.0 + s.rounds * (2.5 + c.nch + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
+        } else {
+            const double start = c.nch * (0.44 + 0.024 * s.lds / 1024.0 * (1.0 + 0.38 * (resident - 1.0))), waves = std::min(G, plan->g.Cout);
+            s.us = 2.75 + s.rounds * (start + chain * std::max(0.0083, 0.0059 * std::max(1.0, resident * waves / 4.0))) +
+                   2.2 * std::max(0.0, wgs / (cus * fit) - 1.0) + 0.5 * (resident - 1.0);
+        }
         if (s.us < best.us) best = s;
     }
     return best;

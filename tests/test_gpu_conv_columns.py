@@ -90,6 +90,14 @@ def test_columns_or_window(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel):
         a.free()
 
 
+@pytest.mark.parametrize("Cin,Cout,H,k,s,sp,B,kernel", [
+    (11, 4, 120, 1, 1, .5, 32, "window"), (5, 4, 111, 3, 1, .5, 32, "window"), (26, 2, 88, 3, 1, .9, 8, "window"),
+    (10, 1, 44, 5, 2, .7, 32, "columns"), (282, 4, 38, 1, 1, .5, 8, "columns")])
+def test_columns_or_window_with_few_channels(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel):
+    """Layers of few channels have one channel a wave on large images too: many workgroups of short rows keep the windowed kernel."""
+    test_columns_or_window(ctx, oracle, Cin, Cout, H, k, s, sp, B, kernel)
+
+
 def test_declined_by_estimate_is_not_for_good(ctx, oracle):
     """A plan tuned for a batch of 16 without streams, since the windowed kernel is estimated ahead, gets them when it is tuned
     again under SPARSEOPS_CONV_COLUMNS=1; without the override the estimate decides as before."""
