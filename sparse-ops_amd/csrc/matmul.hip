@@ -369,13 +369,12 @@ RbmKernel rbm_kernel_but_planes(const so_ctx *ctx, const so_ellpack *E, uint32_t
 // 15.8 against 19.6; 1024 x 4096 x 200 at 70 % 18.4 against 22.2; 2048 x 2048 x 128 at 70 % 14.8 against 14.1; 4096 x 784 x 256 at 90 % 15.0 against 10.8.
 constexpr double kPlanesBelow = 0.9;
 
-// The narrow kernel where it is estimated a little below the others.  Of 447 drawn launches where it is this rule that decides, against the row, shared-gather or quad
-// kernel, it takes the narrow one in 355, which was the slower one in three of them, by 1.1 to 2.3 % (with an estimate 9 % lower and a limit of 0.88:
-// 338, four, by 1.1 to 9.2 %).  Us, the others and the narrow one, one handle launched again and again: quad 2847 x 1952 x 8 at 61 % sparse 14.7 / 7.8, 4096 x 2048 x 16 at 90 / 50 %
-// 10.9 / 7.8 and 17.6 / 11.5, 1152 x 546 x 18 at 54 % 7.2 / 5.4, 317 x 930 x 11 at 74 % 6.8 / 4.8, 2745 x 1203 x 30 at 56 % 11.7 / 11.0;
-// shared-gather 1145 columns, 21 rows, 5 dense 6.6 / 4.1, 627, 41, 28 4.8 / 5.5; row 1595, 981, 10 7.2 / 5.4, 1067, 3000, 28 5.1 / 6.7.  In place
-// of so_matvec's row kernel at two and three columns from a million nonzeros on: 1.16 million, three columns, 10.6 / 5.5; 2.7 million, two, 11.4 / 9.1;
-// 0.91 million, two, 4.5 / 5.3; with one column not: 1.4 million 6.7 / 7.1.
+// The narrow kernel where it is estimated a little below the others.  Of 241 drawn launches (10..4096 rows, 512..4096 columns, 4..256 dense ones, 14 of up to
+// 40 000 rows) it is then in no case the slower one by more than 1 %; in nine, the others' choice is slower by 3 to 9 %.  Us, the others and the narrow one, one handle launched again
+// and again: column kernel 2847 x 1952 x 8 at 61 % sparse 11.5 / 5.9, 4096 x 2048 x 16 at 50 % 15.2 / 9.3, 20 000 x 600 x 32 at 90 % 9.5 / 14.0; quad 139 x 1436 x 4 at 60 %
+// 7.2 / 3.7, 2048 x 2048 x 64 at 80 % 9.9 / 9.6, 2000 x 1500 x 64 at 60 % 9.9 / 11.6, 20 000 x 600 x 64 at 90 % 17.6 / 25.3; row 107 x 730 x 16 at 94 % 3.6 / 3.9.
+// In place of so_matvec's row kernel at two and three columns from a million nonzeros on: 1.39 million, two columns, 8.8 / 4.0; 1.5 million, three, 9.6 / 4.3; 2.9 million,
+// three, 17.7 / 6.3.  (Below it would gain less, 0.3 to 0.6 of 4.1; with one column it is not looked at.)
 constexpr double kNarrowBelow = 0.955;
 constexpr uint64_t kNarrowVectorNnz = 1000000;
 

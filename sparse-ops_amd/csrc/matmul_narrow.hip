@@ -12,23 +12,29 @@
 // chunks, which are requested four to eight ahead, the first before X.  No partial tiles are exchanged.  (A matrix whose X does
 // not fit stays on the quad-union kernel.)
 //
-// What bounds it: small launches the latencies of launch (2.5 us) and first loads (1.1); large ones the copy's bytes (4096 x 4096
-// x 8, 50 % dense: 65 MB, 16 us, 4.1 TB/s) and, from 17 columns on, bank conflicts of the 128-byte rows.  Copying X in
-// two rounds of eight loads cost 1 to 2 us more, and 16-byte loads across the ends of rows of no multiple of four columns 1.5.
+// What bounds it: small launches the latencies of launch (2.5 us) and first loads (1.1); in larger ones a chunk is 24 to 45 clocks of
+// its compute unit, of which the MFMAs' 8 V R (at four columns a value and SIMD) and the copy's 288 bytes through L1 are about half each:
+// without the MFMAs but one in four, the LDS reads or the requests 2048 x 2048 x 64 takes 8.3, 8.9 and 8.8 us of 9.8, with no loop 4.7.
+// What it must not pay for is scalar instructions, which a SIMD issues at one in four clocks: with the tile of a chunk counted from
+// a table, clamped requests and a select for the last ones there were 22 per chunk, and 97 clocks of the SIMD.  Hence whole row numbers
+// (`rows`), fixed bases with one offset per batch, and a last batch of its own.  The LDS reads of a batch go out together, in front of its
+// MFMAs.  Steps sorted so that a read's rows lie on different banks changed nothing.
 //
-// Measured, one handle launched again and again, the quad-union kernel and this one: 2847 x 1952 x 8, 61 % sparse, 14.3 and 7.8 us
-// (17.5 MB of copy); 4096 x 2048 x 16, 50 %, 16.0 and 11.3; 317 x 930 x 11, 74 %, 7.0 and 5.0; 10 x 512 x 4, 80 %, 5.0 (row
-// kernel) and 4.3 (on another card 4.5 and 3.8).  Error against 64 bits: 0.67 of the replaced kernels' on average over 120 launches.
+// Measured, one handle launched again and again, the quad-union or column kernel, this one with scalar work per chunk and this one: 2847 x 1952 x 8, 61 % sparse,
+// 11.5, 8.0 and 5.9 us (17.5 MB of copy); 4096 x 2048 x 16, 50 %, 15.2, 11.9 and 9.3; 317 x 930 x 11, 74 %, 5.6, 4.7 and 4.3; 139 x 1436 x 4,
+// 60 %, 7.2, 4.7 and 3.7; 2048 x 2048 x 64, 80 %, 9.9, 12.7 and 9.6.  Error against 64 bits: 0.67
+// of the replaced kernels' on average over 120 launches; the sums are the same bits in both forms of this one.
 //
 // More columns, in slabs of 16 or 32: pays where a matrix is so small that the quad-union kernel's exchange of partial tiles and its
 // tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 7.0 and 5.4 us; 256 x 1136 x 36, 69 %, 7.6 and 5.8; 45 x 757 x 224, 75 %
-// (shared gather) 6.1 and 5.4.  Every slab reads the copy of the matrix again, so large ones stay there.
+// (shared gather) 6.1 and 5.4 (with scalar work per chunk 4.7, 5.3 and 4.6 on another card, now 4.3, 5.2 and 4.3).  Every slab reads the copy of the matrix again, so large ones stay there.
 //
 // Sums, zero weights and values that are not finite: as there.  With an infinity in one column of X / in each, us: 2847 x 1952 x 8 16 / 21 (the quad-union
 // kernel 35 / 52), 1067 x 900 x 28, 60 %, 11 / 27 (12 / 36), 256 x 1136 x 36 8 / 15 (10 / 28), 2000 x 1500 x 3, 50 %, 13 / 13 (row kernel 12); output
 // by output, a whole wave for each, it took 24 / 90, 13 / 116, 10 / 80 and 18 / 42.
 #include "so_internal.h"
 #include "exact_outputs.h"
+#include "lds_sync.h"
 
 #include <algorithm>
 #include <cmath>
@@ -36,18 +42,21 @@
 
 namespace {
 
-constexpr uint32_t KT = so_quads::kTileRows, WAVES = 16, LOG_WAVES = 4, THREADS = WAVES * 64, AHEAD = 4;
+constexpr uint32_t WAVES = 16, LOG_WAVES = 4, THREADS = WAVES * 64, AHEAD = 4;
 constexpr uint32_t MOST_GROUPS = 10 * THREADS;   // 16-byte groups of X in LDS: 160 KB
 constexpr uint32_t RED_BYTES = THREADS * 8;       // the waves' sums, in the place of X
 constexpr uint32_t MOST_COLUMNS = 65535u * 16u;   // slabs of 16 are counted by blockIdx.y
+static_assert(2u * AHEAD * WAVES <= so_quads::kSlack && MOST_GROUPS <= so_quads::kMostRows, "what a wave requests is there");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef const u32x2 __attribute__((address_space(4))) *const_info;
 
 struct NarrowArgs {
     const float *w;             // [chunks][64]
-    const uint8_t *off;         // [chunks][16]: the X row inside its tile
+    const uint16_t *rows;       // [chunks][16]: the X row
     const uint2 *info;          // [quads][ntiles] {first chunk, units of four steps}
     uint32_t m, n, C, nquads, ntiles, qw_log2, magic;   // magic: e / C is the high half of e * magic (e < 2^19, 1 < C <= 32)
     const float *X, *bias;
@@ -72,28 +81,39 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     const uint32_t wq = wave & (qw - 1u), wk = wave >> a.qw_log2, quad = (blockIdx.x << a.qw_log2) + wq;
     const uint32_t c0 = blockIdx.y * (4u * GROUPS), cols = min(a.C - c0, 4u * GROUPS);       // the slab's columns
 
-    // the wave's chunks: every kw-th of the quad's.  Lane t holds the first chunk of tile t, so the tile of a chunk is a count of lanes.
-    uint32_t first = 0xffffffffu, begin = 0, end = 0;
+    // the wave's chunks: every kw-th of the quad's
+    const uint32_t quarter = lane >> 2;
+    uint32_t begin = 0, end = 0;
     if (quad < a.nquads) {
-        const uint2 *inf = a.info + (size_t)quad * a.ntiles;
-        if (lane < a.ntiles) first = inf[lane].x;
-        const uint2 last = inf[a.ntiles - 1u];
-        begin = __builtin_amdgcn_readfirstlane(inf[0].x) + wk;
-        end = __builtin_amdgcn_readfirstlane(last.x + ((last.y + 3u) >> 2));
+        const const_info inf = (const_info)(uintptr_t)(a.info + (size_t)quad * a.ntiles);
+        const u32x2 first = inf[0], last = inf[a.ntiles - 1u];
+        begin = first.x + wk;
+        end = last.x + ((last.y + 3u) >> 2);
     }
     const uint32_t count = begin < end ? (end - begin + kw - 1u) >> (LOG_WAVES - a.qw_log2) : 0u;
-    struct Batch { float w[AHEAD]; uint32_t o[AHEAD]; };
-    auto request = [&](Batch &b, uint32_t i) {                       // past the last chunk: the last one again
+    // Chunk i + u of a batch is at a base per u, which stays, and an offset for all of them, which moves: nothing scalar is issued per chunk.
+    // Requests go up to two batches past the wave's last chunk, into other quads' chunks or the slack behind the last one (2 AHEAD WAVES chunks).
+    const char *wb[AHEAD], *rb[AHEAD];
+#pragma unroll
+    for (uint32_t u = 0; u < AHEAD; ++u) {
+        wb[u] = reinterpret_cast<const char *>(a.w) + (size_t)(begin + u * kw) * 256u;
+        rb[u] = reinterpret_cast<const char *>(a.rows) + (size_t)(begin + u * kw) * 32u;
+    }
+    uint32_t wat = lane * 4u, rat = R == 1 ? quarter * 2u : (lane >> 3) * 4u;
+    const uint32_t wstep = AHEAD * kw * 256u, rstep = AHEAD * kw * 32u;
+    struct Batch { float w[AHEAD]; uint32_t row[AHEAD]; };
+    auto request = [&](Batch &b) {
 #pragma unroll
         for (uint32_t u = 0; u < AHEAD; ++u) {
-            const size_t c = begin + min(i + u, count - 1u) * kw;
-            b.w[u] = a.w[c * 64u + lane];
-            if constexpr (R == 1) b.o[u] = a.off[c * 16u + (lane >> 2)];
-            else b.o[u] = reinterpret_cast<const uint16_t *>(a.off)[c * 8u + (lane >> 3)];
+            b.w[u] = *reinterpret_cast<const float *>(wb[u] + wat);
+            if constexpr (R == 1) b.row[u] = *reinterpret_cast<const uint16_t *>(rb[u] + rat);
+            else b.row[u] = *reinterpret_cast<const uint32_t *>(rb[u] + rat);
         }
+        wat += wstep;
+        rat += rstep;
     };
     Batch b0, b1;
-    if (count != 0u) { request(b0, 0u); request(b1, AHEAD); }
+    if (count != 0u) { request(b0); request(b1); }
 
     // X into LDS, four values per thread and load, all loads in flight: as it lies in memory, and from there to the rows'
     // places, a value at a time where rows are no whole groups of four (128-bit loads across the rows' ends took 1.5 us longer).
@@ -151,38 +171,59 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     for (int i = 0; i < SETS; ++i)
 #pragma unroll
         for (int v = 0; v < V; ++v) part[i][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const char *const mine = lds + (lane % (4u * R)) * (V * 4u);
-    auto multiply = [&](const Batch &b, uint32_t i) {
+    const uint32_t mine = so_lds::lds_address(lds) + (lane % (4u * R)) * (V * 4u);
+    typedef const __attribute__((address_space(3))) char *lds_pointer;
+    struct Operands { float x[R][V]; };
+    auto fetch = [&](uint32_t rows, Operands &o) {
 #pragma unroll
-        for (uint32_t u = 0; u < AHEAD; ++u) {
-            const uint32_t c = begin + min(i + u, count - 1u) * kw;
-            const uint32_t tile = (uint32_t)__popcll(__ballot(first <= c)) - 1u;
-            const float w = i + u < count ? b.w[u] : 0.0f;
-#pragma unroll
-            for (int k = 0; k < R; ++k) {
-                const uint32_t row = tile * KT + (R == 1 ? b.o[u] : (b.o[u] >> (8 * k)) & 255u);
-                const float *x = reinterpret_cast<const float *>(mine + row * (GROUPS * 16u));
-                float xv[V];
-                if constexpr (V == 4) { const f32x4 t = *reinterpret_cast<const f32x4 *>(x); xv[0] = t[0]; xv[1] = t[1]; xv[2] = t[2]; xv[3] = t[3]; }
-                else if constexpr (V == 2) { const float2 t = *reinterpret_cast<const float2 *>(x); xv[0] = t.x; xv[1] = t.y; }
-                else xv[0] = x[0];
-#pragma unroll
-                for (int v = 0; v < V; ++v) {
-                    f32x4 *const acc = part[u % SETS];
-                    if constexpr (R == 1) acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, xv[v], acc[v], 0, 0, 0);
-                    else if (k == 0) acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, xv[v], acc[v], 1, 0, 0);
-                    else acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, xv[v], acc[v], 1, 1, 0);
-                }
-            }
+        for (int k = 0; k < R; ++k) {
+            const uint32_t row = R == 1 ? rows : k == 0 ? rows & 0xffffu : rows >> 16;
+            const lds_pointer x = (lds_pointer)(mine + row * (GROUPS * 16u));
+            if constexpr (V == 4) { const f32x4 t = *(const __attribute__((address_space(3))) f32x4 *)x; o.x[k][0] = t[0]; o.x[k][1] = t[1]; o.x[k][2] = t[2]; o.x[k][3] = t[3]; }
+            else if constexpr (V == 2) { const f32x2 t = *(const __attribute__((address_space(3))) f32x2 *)x; o.x[k][0] = t[0]; o.x[k][1] = t[1]; }
+            else o.x[k][0] = *(const __attribute__((address_space(3))) float *)x;
         }
     };
-    for (uint32_t i = 0; i < count; i += 2u * AHEAD) {
-        multiply(b0, i);
-        request(b0, i + 2u * AHEAD);
-        if (i + AHEAD >= count) break;
-        multiply(b1, i + AHEAD);
-        request(b1, i + 3u * AHEAD);
+    auto multiply = [&](float w, const Operands &o, uint32_t u) {
+        f32x4 *const acc = part[u % SETS];
+#pragma unroll
+        for (int k = 0; k < R; ++k)
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                if constexpr (R == 1) acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, o.x[k][v], acc[v], 0, 0, 0);
+                else if (k == 0) acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, o.x[k][v], acc[v], 1, 0, 0);
+                else acc[v] = __builtin_amdgcn_mfma_f32_4x4x1f32(w, o.x[k][v], acc[v], 1, 1, 0);
+            }
+    };
+    // a batch: its LDS reads, then its multiply-adds (a read at a time in front of its own leaves the reads' latency to the other waves)
+    auto batch = [&](const Batch &b) {
+        Operands o[AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) fetch(b.row[u], o[u]);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u) multiply(b.w[u], o[u], u);
+    };
+    auto rest = [&](const Batch &b, uint32_t chunks) {
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; ++u)
+            if (u < chunks) {
+                Operands o;
+                fetch(b.row[u], o);
+                multiply(b.w[u], o, u);
+            }
+    };
+    uint32_t left = count;
+    for (; left >= 2u * AHEAD; left -= 2u * AHEAD) {
+        batch(b0);
+        request(b0);
+        batch(b1);
+        request(b1);
     }
+    if (left >= AHEAD) {
+        batch(b0);
+        rest(b1, left - AHEAD);
+    } else rest(b0, left);
 
     f32x4 acc[V];
 #pragma unroll
@@ -296,16 +337,16 @@ bool fits(const so_ctx *ctx, const so_ellpack *E, uint32_t groups)
 
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
-    return E->quads.d_w != nullptr && E->n != 0 && C >= 1 && C <= MOST_COLUMNS && (C <= 32 || C % 4 == 0) && E->quads.ntiles <= 64 && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
+    return E->quads.d_rows != nullptr && E->n != 0 && C >= 1 && C <= MOST_COLUMNS && (C <= 32 || C % 4 == 0) && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
 }
 
 // Up to 32 columns the narrowest slab that holds them, beyond (whole groups of four only: the others' copies take up to twice as
 // long) slabs of 16 or 32 columns (blockIdx.y), whichever is estimated faster; as few quads per workgroup as give no more workgroups than compute units.  The estimate -- the launch, a workgroup's
-// start and its copy of X, the chunks of a wave, the bytes that slabs share -- was fitted to 696 launches of 10..4096 rows, 512..4096 columns, 1..64 dense
-// columns, 50-95 % sparse on three cards, one handle again and again: 0.7 % too low on average, 5 % off (standard deviation; the same handle differs by
-// as much from one allocation to the next), 20 % at most.  Slabs also to 320 launches of up to 1500 rows and 4800 dense columns, 10 % off: once X is more than an XCD's
-// 4 MB of L2, the 64 bytes of a row that a slab of 16 takes cost a whole line from beyond it (4 x 1792 x 3780, 27 MB, 14.2 us, shared gather
-// 7.6; 12 x 2172 x 1860 17.7, quad-union 8.5); those of 32 columns take whole lines.
+// start and its copy of X (a value at a time where rows are no whole groups of four), the chunks of a wave, the copy's bytes, again for every
+// slab of 32 -- was fitted to 228 launches of 10..4096 rows, 512..4096 columns, 4..256 dense columns, 50-95 % sparse, and 14 of up to
+// 40 000 rows, one handle again and again: 7 % off (standard deviation; the same handle differs by 5 from one allocation to the next),
+// 30 % at most.  Beyond 4 MB of X, an XCD's L2, the 64 bytes of a row that a slab of 16 takes cost a whole line (4 x 1792 x 3780,
+// 27 MB, 14.2 us, shared gather 7.6; 12 x 2172 x 1860 17.7, quad-union 8.5; 320 launches of up to 1500 rows and 4800 dense columns); those of 32 columns take whole lines.
 so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
@@ -317,9 +358,10 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
         uint32_t ql = 0;
         while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
         const double rounds = so_ceil_div((uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs, (uint64_t)ctx->compute_units);
-        const double copy = 1e-4 * E->n * (slabs > 1 ? 4.6 * groups : C) * (C % 4u ? 0.6 : 0.45), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
+        const double copy = 1e-4 * E->n * (slabs > 1 ? 1.92 * groups : C * (C % 4u ? 0.95 : 0.73)), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
         const double megabytes = 4.0 * E->n * C / (1u << 20), far = slabs > 1 && groups == 4u && megabytes > 4.0 ? 0.6 * megabytes : 0.0;
-        const double us = 3.0 + rounds * (1.0 + (slabs > 1 ? 0.2 : 0.0) + (groups == 8u ? 0.55 : 0.0) + copy + chunks * (0.077 + 0.021 * groups)) + 0.84e-5 * Q.total_chunks + far;
+        const double again = groups == 8u ? slabs : 1.0;                  // slabs of 32 columns are few enough for their reads of the copy to count
+        const double us = 1.05 + rounds * (2.0 + (slabs > 1 ? 0.36 : 0.0) + copy + chunks * (0.025 + 0.0244 * groups)) + 0.75e-5 * Q.total_chunks * again + far;
         if (us < best.us) best = so_narrow_plan{ql, groups, slabs, us};
     }
     return best;
@@ -328,7 +370,7 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
 so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const so_narrow_plan &p, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
     const so_quads &Q = E->quads;
-    const NarrowArgs a{Q.d_w, (const uint8_t *)Q.d_off, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, p.qw_log2, (uint32_t)(((1ull << 32) + C - 1u) / C),
+    const NarrowArgs a{Q.d_w, Q.d_rows, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, p.qw_log2, (uint32_t)(((1ull << 32) + C - 1u) / C),
                        dX, dBias, dY, E->d_Wd, E->d_idx, E->d_nnz, E->r};
     const dim3 blocks(so_ceil_div(Q.nquads, 1u << p.qw_log2), p.slabs);
     const size_t lds = lds_bytes(E->n, p.groups);

@@ -53,7 +53,8 @@ namespace {
 
 constexpr uint32_t KT = so_quads::kTileRows, WAVES = 16, LOG_WAVES = 4, TILE_BYTES = KT * 256, LDS_BYTES = 2 * TILE_BYTES + 16;
 constexpr uint32_t DEPTH = 6;                     // ring slots: chunks whose weights and row bytes are requested ahead
-constexpr uint32_t SLACK = (DEPTH + 2) * WAVES;   // chunks a wave may request past its quad's last one
+constexpr uint32_t SLACK = so_quads::kSlack;      // chunks a wave may request past its quad's last one
+static_assert((DEPTH + 2) * WAVES <= SLACK, "requests ahead stay inside the copy");
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -393,6 +394,20 @@ so_status workspace(so_ctx *ctx, const so_ellpack *E, uint32_t C, const so_quad_
 
 struct Entry { uint32_t col, row; float w; };
 
+// rows: the X row of every step, from its tile and its byte there; zeros for the slack.  16 lanes per (quad, tile) run.  (Made here: written and
+// copied by the host with the rest, they took a tenth of an upload's time.)
+__global__ __launch_bounds__(256)
+void quad_rows_kernel(uint16_t *rows, uint64_t chunks, const uint8_t *off, const uint2 *info, uint64_t runs, uint32_t ntiles)
+{
+    const uint32_t sub = threadIdx.x & 15u;
+    for (uint64_t i = blockIdx.x * 16ull + (threadIdx.x >> 4); i <= runs; i += gridDim.x * 16ull) {
+        const uint2 run = info[i < runs ? i : runs - 1u];
+        const uint64_t past = run.x + (uint64_t)((run.y + 3u) >> 2);
+        if (i < runs) for (uint64_t c = run.x; c < past; ++c) rows[c * 16u + sub] = (uint16_t)(i % ntiles * KT + off[c * 16u + sub]);
+        else for (uint64_t c = past; c < chunks; ++c) rows[c * 16u + sub] = 0u;
+    }
+}
+
 // Rows with ascending columns: tile(t, mask, weights) for every tile of quad q, with a bit per union column and, where
 // WEIGHTS, the four weights of each (weights[4 * column ..], zeros elsewhere: tile puts back zeros where it takes them).
 template <bool WEIGHTS, class F>
@@ -511,12 +526,19 @@ so_status so_quads_build(so_ctx *ctx, so_ellpack *E, const float *Wd, const uint
         }
     });
     void *p = nullptr;
-    const so_status s = so_malloc(ctx, blob.size(), &p);
+    const size_t rows_bytes = E->n <= so_quads::kMostRows ? 2 * off_bytes : 0, rows_at = (blob.size() + 15) & ~(size_t)15;
+    so_status s = so_malloc(ctx, rows_at + rows_bytes, &p);
     if (s != SO_OK) { Q = so_quads(); return s; }
     Q.d_w = (float *)p;
     Q.d_off = (uint32_t *)((char *)p + w_bytes);
     Q.d_info = (uint2 *)((char *)p + w_bytes + off_bytes);
-    return so_h2d(ctx, p, blob.data(), blob.size());
+    s = so_h2d(ctx, p, blob.data(), blob.size());
+    if (s != SO_OK || rows_bytes == 0 || info.empty()) return s;
+    Q.d_rows = (uint16_t *)((char *)p + rows_at);
+    const uint64_t runs = (uint64_t)Q.nquads * Q.ntiles;
+    quad_rows_kernel<<<(uint32_t)std::min<uint64_t>((runs + 16) / 16, 65536), 256, 0, ctx->stream>>>(Q.d_rows, off_bytes / 16, (const uint8_t *)Q.d_off, Q.d_info, runs, Q.ntiles);
+    SO_LAUNCH_CHECK();
+    return so_stream_wait(ctx, "so_ellpack_upload");
 }
 
 void so_quads_free(so_ellpack *E)

@@ -140,11 +140,14 @@ struct so_rbmm {
 struct so_quads {
     static constexpr uint32_t kTileRows = 256;    // X rows per LDS tile
     static constexpr uint32_t kMaxSplit = 64;     // most workgroups per output tile
+    static constexpr uint32_t kSlack = 128;       // chunks behind the last one that requests ahead may reach
     uint32_t nquads = 0, ntiles = 0;
     uint64_t total_units = 0, total_chunks = 0;   // units of four steps and chunks over all (quad, tile) runs
     float *d_w = nullptr;                         // [chunks + slack][64]
     uint32_t *d_off = nullptr;                    // [chunks + slack][4] words: X row inside the tile, a byte per step
     uint2 *d_info = nullptr;                      // [nquads][ntiles] {first chunk, units}
+    static constexpr uint32_t kMostRows = 10240;  // X rows that the narrow kernel's LDS holds
+    uint16_t *d_rows = nullptr;                   // [chunks + slack][16]: the X row of every step, for the narrow kernel (null beyond kMostRows columns)
 };
 
 // The matrix, dense, as three bf16 planes for so_matmul on the bf16 matrix cores (csrc/matmul_planes.hip).
