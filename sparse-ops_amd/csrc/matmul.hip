@@ -318,7 +318,7 @@ bool columns_pays(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
            so_matmul_columns_estimate(ctx, E, C) < rows_estimate_small_x(ctx, E);
 }
 
-enum class RbmKernel { None, Merged, Quad, Vector, Planes, Narrow };
+enum class RbmKernel { None, Merged, Quad, Vector, Planes, Narrow, Slabs };
 
 // Which of the kernels for handles with the RBM layout a launch takes, or None for the kernels below, by estimated
 // time.  Both sides of each line were measured, us with one handle launched again and again, in brackets with 48 handles
@@ -378,6 +378,11 @@ constexpr double kPlanesBelow = 0.9;
 constexpr double kNarrowBelow = 0.955;
 constexpr uint64_t kNarrowVectorNnz = 1000000;
 
+// The same with X in LDS a part at a time, where it is estimated 7 % below what would run: of 200 drawn launches it is then taken in 47, all of
+// them faster, by 17 % on average.  Us, the others and this one: quad 12 x 1238 x 173 at 55 % sparse 7.2 / 5.0, 2000 x 2600 x 16 at 60 % 12.9 / 9.0, 30 x 2988 x 56 at 54 % 7.3 / 7.6,
+// 2000 x 1500 x 64 at 60 % 9.9 / 10.5; shared-gather 26 x 745 x 91 at 69 % 5.9 / 4.9, 10 x 1391 x 138 at 82 % 6.0 / 6.2; narrow 17 x 1090 x 28 at 67 % 6.0 / 4.7, 2000 x 1500 x 8 at 60 % 4.6 / 6.8.
+constexpr double kSlabsBelow = 0.93;
+
 RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad_plan *plan, so_planes_plan *planes, so_narrow_plan *narrow)
 {
     if (ctx->tune.matmul_rbm == 1 && so_matmul_rbm_applies(ctx, E, C)) return RbmKernel::Merged;
@@ -385,6 +390,10 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad
     if (ctx->tune.matmul_narrow == 1 && so_matmul_narrow_applies(ctx, E, C)) {
         *narrow = so_matmul_narrow_choose(ctx, E, C);
         return RbmKernel::Narrow;
+    }
+    if (ctx->tune.matmul_slabs > 0 && so_matmul_slabs_applies(ctx, E, C)) {
+        *narrow = so_matmul_slabs_choose(ctx, E, C);
+        return RbmKernel::Slabs;
     }
     const bool have = ctx->tune.matmul_planes != 0 && so_matmul_planes_applies(ctx, E, C);
     const bool vector = C <= 3 && E->max_nnz >= 64u * C;
@@ -399,9 +408,21 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad
         }
     }
     // (an override that forces another kernel, or forbids the quad-union copy's, stands)
-    if (ctx->tune.matmul_narrow == 0 || ctx->tune.matmul_quad >= 0 || ctx->tune.matmul_planes == 1 || !so_matmul_narrow_applies(ctx, E, C)) return k;
-    *narrow = so_matmul_narrow_choose(ctx, E, C);
-    return (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : narrow->us < kNarrowBelow * us) ? RbmKernel::Narrow : k;
+    if (ctx->tune.matmul_quad >= 0 || ctx->tune.matmul_planes == 1) return k;
+    if (ctx->tune.matmul_narrow != 0 && so_matmul_narrow_applies(ctx, E, C)) {
+        *narrow = so_matmul_narrow_choose(ctx, E, C);
+        if (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : narrow->us < kNarrowBelow * us) {
+            k = RbmKernel::Narrow;
+            us = narrow->us;
+        }
+    }
+    if (vector || ctx->tune.matmul_slabs == 0 || !so_matmul_slabs_applies(ctx, E, C)) return k;
+    const so_narrow_plan slabs = so_matmul_slabs_choose(ctx, E, C);
+    if (slabs.us >= kSlabsBelow * us) return k;
+    // What a recording takes does not change with this kernel, which needs no workspace: the copy's kernels with a reservation, the reference's order without.
+    if (ctx->capturing && k != RbmKernel::Narrow && !(so_matmul_quad_applies(ctx, E, C) && so_matmul_quad_ready(ctx, so_matmul_quad_choose(ctx, E, C)))) return k;
+    *narrow = slabs;
+    return RbmKernel::Slabs;
 }
 
 } // namespace
@@ -447,7 +468,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
 
     // The kernels of the RBM layout, on handles uploaded with it (accurate to fp32 round-off, not bit-identical to
     // the row order: the caller asked for them by asking for the layout; SPARSEOPS_MATMUL_RBM=0 forbids all of them, =1
-    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one, SPARSEOPS_MATMUL_PLANES the bf16-planes one, SPARSEOPS_MATMUL_NARROW the narrow one).
+    // forces the row-block-merged one, SPARSEOPS_MATMUL_QUAD=1 / 0 forces / forbids the quad-union one, SPARSEOPS_MATMUL_PLANES the bf16-planes one, SPARSEOPS_MATMUL_NARROW the narrow one, SPARSEOPS_MATMUL_SLABS the one with X a part at a time).
     if ((E->layouts & SO_LAYOUT_RBM) && dX != nullptr && (((uintptr_t)dX | (uintptr_t)dY) & 3) == 0) {
         so_quad_plan plan;
         so_planes_plan pplan;
@@ -455,13 +476,13 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
         const RbmKernel k = rbm_kernel(ctx, E, C, &plan, &pplan, &nplan);
         if (k != RbmKernel::None) {
             const so_status st = k == RbmKernel::Quad ? so_matmul_quad_launch(ctx, E, plan, dX, C, dBias, dY, act)
-                               : k == RbmKernel::Narrow ? so_matmul_narrow_launch(ctx, E, nplan, dX, C, dBias, dY, act)
+                               : k == RbmKernel::Narrow || k == RbmKernel::Slabs ? so_matmul_narrow_launch(ctx, E, nplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Planes ? so_matmul_planes_launch(ctx, E, pplan, dX, C, dBias, dY, act)
                                : k == RbmKernel::Vector ? so_matvec_columns(ctx, E, dX, C, dBias, dY, act)
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
-            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Narrow ? "narrow" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
+            ctx->last_kernel = k == RbmKernel::Quad || k == RbmKernel::Slabs ? "quad" : k == RbmKernel::Narrow ? "narrow" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
             return SO_OK;
         }
     }

@@ -9,8 +9,7 @@
 //
 // Decomposition.  A workgroup of 16 waves owns 1 to 16 quads of rows, as few as give no more workgroups than compute units, and
 // the whole of K: all of X (up to 160 KB) is copied to LDS once, one barrier, and from there on a wave only waits for its own
-// chunks, which are requested four to eight ahead, the first before X.  No partial tiles are exchanged.  (A matrix whose X does
-// not fit stays on the quad-union kernel.)
+// chunks, which are requested four to eight ahead, the first before X.  No partial tiles are exchanged.
 //
 // What bounds it: small launches the latencies of launch (2.5 us) and first loads (1.1); in larger ones a chunk is 24 to 45 clocks of
 // its compute unit, of which the MFMAs' 8 V R (at four columns a value and SIMD) and the copy's 288 bytes through L1 are about half each:
@@ -29,6 +28,14 @@
 // tiles' barriers are most of the launch: 51 x 697 x 208, 58 % sparse, 7.0 and 5.4 us; 256 x 1136 x 36, 69 %, 7.6 and 5.8; 45 x 757 x 224, 75 %
 // (shared gather) 6.1 and 5.4 (with scalar work per chunk 4.7, 5.3 and 4.6 on another card, now 4.3, 5.2 and 4.3).  Every slab reads the copy of the matrix again, so large ones stay there.
 //
+// X a part at a time (PASSES), for any number of columns: what X in one piece is too large for, or too far from whole groups of four.  The quad-union kernel's
+// launches of few rows and a long K are mostly its exchange of partial tiles; here a workgroup still has the whole of K and takes X in
+// parts of 1280 rows (512 with slabs of 32 columns), two in LDS at a time, the first two asked for together.  A part costs 0.8 us beside its
+// loads: the waves of a SIMD end a part at different times, by up to 1000 clocks, and all meet at its end (clock stamps).  Us, the other kernels / this
+// one: quad-union 12 x 1238 x 173, 55 % sparse, 7.2 / 5.0, 125 x 1172 x 57, 54 %, 7.4 / 5.3, 84 x 692 x 149, 50 %, 7.0 / 5.2, 172 x 1992 x 29, 84 %, 7.6 / 6.3, 2000 x 2600 x 16, 60 %,
+// 12.9 / 9.0; shared gather 26 x 745 x 91, 69 %, 5.9 / 4.9; column kernel 4022 x 1285 x 28, 59 %, 11.1 / 9.7; X in one piece 17 x 1090 x 28, 67 %, 6.0 / 4.7.
+// From three parts on it gains little: 40 x 2835 x 83, 78 %, 7.9 / 7.7, 30 x 2988 x 56, 54 %, 7.3 / 7.6.
+//
 // Sums, zero weights and values that are not finite: as there.  With an infinity in one column of X / in each, us: 2847 x 1952 x 8 16 / 21 (the quad-union
 // kernel 35 / 52), 1067 x 900 x 28, 60 %, 11 / 27 (12 / 36), 256 x 1136 x 36 8 / 15 (10 / 28), 2000 x 1500 x 3, 50 %, 13 / 13 (row kernel 12); output
 // by output, a whole wave for each, it took 24 / 90, 13 / 116, 10 / 80 and 18 / 42.
@@ -45,6 +52,10 @@ namespace {
 constexpr uint32_t WAVES = 16, LOG_WAVES = 4, THREADS = WAVES * 64, AHEAD = 4;
 constexpr uint32_t MOST_GROUPS = 10 * THREADS;   // 16-byte groups of X in LDS: 160 KB
 constexpr uint32_t RED_BYTES = THREADS * 8;       // the waves' sums, in the place of X
+// Rows of X per pass, of which LDS holds two: whole tiles of the copy.  A pass's places in X are counted in 32 bits.
+template <uint32_t GROUPS> constexpr uint32_t PASS_ROWS = GROUPS == 4u ? 1280u : 512u;
+template <uint32_t GROUPS> constexpr uint32_t PASS_BYTES = PASS_ROWS<GROUPS> * GROUPS * 16u;
+constexpr uint32_t MOST_PASS_COLUMNS = 65535u;
 constexpr uint32_t MOST_COLUMNS = 65535u * 16u;   // slabs of 16 are counted by blockIdx.y
 static_assert(2u * AHEAD * WAVES <= so_quads::kSlack && MOST_GROUPS <= so_quads::kMostRows, "what a wave requests is there");
 
@@ -68,8 +79,8 @@ struct NarrowArgs {
 
 __device__ __forceinline__ float xor_add(float keep, float send, int mask) { return keep + __shfl_xor(send, mask, 64); }
 
-// V values of a row of X per lane and LDS read, R reads per chunk: 4 V R columns.
-template <int V, int R, int ACT>
+// V values of a row of X per lane and LDS read, R reads per chunk: 4 V R columns.  PASSES: X in LDS a part at a time.
+template <int V, int R, int ACT, bool PASSES>
 __global__ __launch_bounds__(THREADS)
 void ellpack_matmul_narrow_kernel(NarrowArgs a)
 {
@@ -113,7 +124,40 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
         rat += rstep;
     };
     Batch b0, b1;
-    if (count != 0u) { request(b0); request(b1); }
+    // PASSES: the pass whose chunks are requested next, how many of them are not yet, and the wave's chunks of passes 0 .. `asking`.  Lane p holds
+    // the wave's chunks of passes 0 .. p (a scalar load at the end of each pass would be waited for there).
+    uint32_t asking = 0, unasked = 0, asked = 0, upto = 0;
+    const uint32_t passes = (a.n + PASS_ROWS<GROUPS> - 1u) / PASS_ROWS<GROUPS>;      // 20 at most: 10 240 rows of 512
+    if constexpr (PASSES) {
+        const uint32_t t = (lane + 1u) * (PASS_ROWS<GROUPS> / so_quads::kTileRows);
+        const uint32_t start = a.info[(size_t)min(quad, a.nquads - 1u) * a.ntiles + min(t, a.ntiles - 1u)].x, past = t < a.ntiles ? start : end;
+        upto = past > begin && count != 0u ? (past - begin + kw - 1u) >> (LOG_WAVES - a.qw_log2) : 0u;
+    }
+    const auto chunks_up_to = [&](uint32_t pass) { return (uint32_t)__builtin_amdgcn_readlane(upto, pass); };
+    // The next batch of the wave's: what is left of a pass where that is less than a batch, so that a batch never holds chunks of two passes.  The
+    // marks keep its 2 AHEAD loads between them, and csrc/check_narrow_asks.py counts them there in the assembly of every build: `enter_pass` relies on it.
+    auto ask = [&](Batch &b) {
+        while (unasked == 0u && asking + 1u < passes) {
+            const uint32_t all = chunks_up_to(++asking);
+            unasked = all - asked;
+            asked = all;
+        }
+        if (unasked == 0u) return 0u;
+        asm volatile("; ask" : : : "memory");
+        request(b);
+        asm volatile("; asked" : : : "memory");
+        const uint32_t some = min(unasked, AHEAD);
+        unasked -= some;
+        wat -= (AHEAD - some) * (wstep / AHEAD);
+        rat -= (AHEAD - some) * (rstep / AHEAD);
+        return 1u;
+    };
+    if constexpr (PASSES) {
+        unasked = asked = chunks_up_to(0u);
+        if (count != 0u) { (void)ask(b0); (void)ask(b1); }
+    } else {
+        if (count != 0u) { request(b0); request(b1); }
+    }
 
     // X into LDS, four values per thread and load, all loads in flight: as it lies in memory, and from there to the rows'
     // places, a value at a time where rows are no whole groups of four (128-bit loads across the rows' ends took 1.5 us longer).
@@ -153,7 +197,50 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
         for (uint32_t u = 0; u < N; ++u)
             if (tid + u * THREADS < a.n * GROUPS) reinterpret_cast<f32x4 *>(lds)[tid + u * THREADS] = v[u];
     };
-    if (gridDim.y > 1u) {
+    // PASSES: straight from memory into LDS, a pass in LOADS loads of 16 bytes per thread, into the two halves of LDS in turn; the first two passes
+    // are asked for together.  Groups of four columns past the last column repeat the slab's first group and rows past the last row
+    // repeat it (neither is ever used); a group that would end past the end of X (C not a multiple of 4, last row) is read from where
+    // four values are left and shifted once it is in LDS.
+    constexpr uint32_t ROWS = PASS_ROWS<GROUPS>, HALF = PASS_BYTES<GROUPS>, LOADS = (HALF + 16u * THREADS - 1u) / (16u * THREADS);
+    const uint32_t sgrp = tid % GROUPS * 4u, srow = tid / GROUPS, xgrp = c0 + (sgrp < cols ? sgrp : 0u), lds0 = so_lds::lds_address(lds);
+    const auto place = [&](uint32_t pass, uint32_t k) { return min(k * (THREADS / GROUPS) + srow, a.n - 1u - pass * ROWS) * a.C + xgrp; };
+    const auto ends = [&](uint32_t pass) { return (uint32_t)min((uint64_t)(a.n - pass * ROWS) * a.C - 4u, (uint64_t)0x3ffffff0u); };   // the last place four values can be read from
+    auto fetch_pass = [&](uint32_t pass) {
+        const float *p = a.X + (size_t)pass * ROWS * a.C;
+        const uint32_t to = lds0 + (pass & 1u) * HALF + wave * 1024u, e = ends(pass);
+#pragma unroll
+        for (uint32_t k = 0; k < LOADS; ++k)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         : : "v"(min(place(pass, k), e) * 4u), "s"(p), "s"(to + k * (16u * THREADS)) : "memory", "m0");
+    };
+    // This wave's part of a pass is in LDS, then everybody's; the next pass's way in.  Loads return in order: `asks` batches have been asked for
+    // since the pass was, and may still be on their way.
+    auto enter_pass = [&](uint32_t pass, uint32_t asks) {
+        if (pass == 0u && passes > 1u) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(LOADS) : "memory");      // pass 1 is on its way
+        else if (asks >= 2u) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(4u * AHEAD) : "memory");
+        else if (asks == 1u) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(2u * AHEAD) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        if (a.C % 4u != 0u && pass + 1u == passes) {
+            const uint32_t e = ends(pass);
+#pragma unroll
+            for (uint32_t k = 0; k < LOADS; ++k) {
+                const uint32_t at = place(pass, k);
+                if (at > e) {
+                    f32x4 *q = reinterpret_cast<f32x4 *>(lds + (pass & 1u) * HALF + (k * THREADS + tid) * 16u);
+                    const f32x4 u = *q;
+                    const uint32_t shift = at - e;
+                    *q = f32x4{shift == 1u ? u[1] : shift == 2u ? u[2] : u[3], shift == 1u ? u[2] : u[3], u[3], u[3]};
+                }
+            }
+        }
+        __syncthreads();
+        if (pass != 0u && pass + 1u < passes) fetch_pass(pass + 1u);
+    };
+    if constexpr (PASSES) {
+        fetch_pass(0u);
+        if (passes > 1u) fetch_pass(1u);
+        enter_pass(0u, 0u);
+    } else if (gridDim.y > 1u) {
         if constexpr (GROUPS >= 4u) {
             if (a.n * GROUPS <= 4u * THREADS) stage_slab(std::integral_constant<uint32_t, 4>());
             else stage_slab(std::integral_constant<uint32_t, MOST_GROUPS / THREADS>());
@@ -162,7 +249,7 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
         if (tid < total) *reinterpret_cast<float *>(lds + tid / a.C * (GROUPS * 16u) + tid % a.C * 4u) = a.X[tid];
     } else if (groups <= 4u * THREADS) stage(std::integral_constant<uint32_t, 4>());
     else stage(std::integral_constant<uint32_t, MOST_GROUPS / THREADS>());
-    __syncthreads();
+    if constexpr (!PASSES) __syncthreads();
 
     // Four accumulators at least: a chain of multiply-adds takes every SETS-th chunk, which rounds less and waits less.
     constexpr int SETS = 4 / V;
@@ -171,7 +258,7 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     for (int i = 0; i < SETS; ++i)
 #pragma unroll
         for (int v = 0; v < V; ++v) part[i][v] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const uint32_t mine = so_lds::lds_address(lds) + (lane % (4u * R)) * (V * 4u);
+    uint32_t mine = lds0 + (lane % (4u * R)) * (V * 4u);       // of X's row 0, wherever the pass's first one lies
     typedef const __attribute__((address_space(3))) char *lds_pointer;
     struct Operands { float x[R][V]; };
     auto fetch = [&](uint32_t rows, Operands &o) {
@@ -213,17 +300,42 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
                 multiply(b.w[u], o, u);
             }
     };
-    uint32_t left = count;
-    for (; left >= 2u * AHEAD; left -= 2u * AHEAD) {
-        batch(b0);
-        request(b0);
-        batch(b1);
-        request(b1);
+    if constexpr (PASSES) {
+        uint32_t pass = 0, done = chunks_up_to(0u), left = done, asks = 0;
+        // to the next pass that has chunks for the wave; all waves enter every pass.  False: none is left.
+        auto next_pass = [&]() {
+            while (left == 0u) {
+                if (++pass == passes) return false;
+                const uint32_t all = chunks_up_to(pass);
+                left = all - done;
+                done = all;
+                enter_pass(pass, asks);
+                asks = 0u;
+                mine = lds0 + (pass & 1u) * HALF - pass * HALF + (lane % (4u * R)) * (V * 4u);
+            }
+            return true;
+        };
+        auto some = [&](Batch &b) {
+            if (left >= AHEAD) { batch(b); left -= AHEAD; }
+            else { rest(b, left); left = 0u; }
+            asks += ask(b);
+            return left != 0u || next_pass();
+        };
+        if (next_pass())
+            while (some(b0) && some(b1)) {}
+    } else {
+        uint32_t left = count;
+        for (; left >= 2u * AHEAD; left -= 2u * AHEAD) {
+            batch(b0);
+            request(b0);
+            batch(b1);
+            request(b1);
+        }
+        if (left >= AHEAD) {
+            batch(b0);
+            rest(b1, left - AHEAD);
+        } else rest(b0, left);
     }
-    if (left >= AHEAD) {
-        batch(b0);
-        rest(b1, left - AHEAD);
-    } else rest(b0, left);
 
     f32x4 acc[V];
 #pragma unroll
@@ -309,12 +421,12 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
 // 16-byte groups of a row of X in LDS for C <= 32 columns.
 uint32_t groups_for(uint32_t C) { return C <= 4 ? 1u : C <= 8 ? 2u : C <= 16 ? 4u : 8u; }
 
-template <int V, int R>
+template <int V, int R, bool PASSES = false>
 so_status launch(so_ctx *ctx, const NarrowArgs &a, dim3 blocks, size_t lds, int act)
 {
 #define SO_NARROW(A)                                                                              \
-    SO_HIP(so_allow_big_lds(ctx, (const void *)ellpack_matmul_narrow_kernel<V, R, A>));           \
-    ellpack_matmul_narrow_kernel<V, R, A><<<blocks, THREADS, lds, ctx->stream>>>(a);              \
+    SO_HIP(so_allow_big_lds(ctx, (const void *)ellpack_matmul_narrow_kernel<V, R, A, PASSES>));   \
+    ellpack_matmul_narrow_kernel<V, R, A, PASSES><<<blocks, THREADS, lds, ctx->stream>>>(a);      \
     break
     switch (act) {
     case SO_ACT_RELU:    SO_NARROW(SO_ACT_RELU);
@@ -362,7 +474,33 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
         const double megabytes = 4.0 * E->n * C / (1u << 20), far = slabs > 1 && groups == 4u && megabytes > 4.0 ? 0.6 * megabytes : 0.0;
         const double again = groups == 8u ? slabs : 1.0;                  // slabs of 32 columns are few enough for their reads of the copy to count
         const double us = 1.05 + rounds * (2.0 + (slabs > 1 ? 0.36 : 0.0) + copy + chunks * (0.025 + 0.0244 * groups)) + 0.75e-5 * Q.total_chunks * again + far;
-        if (us < best.us) best = so_narrow_plan{ql, groups, slabs, us};
+        if (us < best.us) best = so_narrow_plan{ql, groups, slabs, false, us};
+    }
+    return best;
+}
+
+bool so_matmul_slabs_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    return E->quads.d_rows != nullptr && E->n != 0 && C >= 4 && C <= MOST_PASS_COLUMNS && 2u * PASS_BYTES<4> <= (size_t)ctx->max_lds_bytes;
+}
+
+// Slabs of 16 or of 32 columns, whichever is estimated faster.  Fitted to 400 launches of 10..4096 rows, 512..4096 columns, 4..256 dense columns, 50-95 % sparse:
+// 5.5 % off (standard deviation), 28 % at most (too low, for X of 3 MB and more, which the quad-union kernel's tiles serve better by far).
+so_narrow_plan so_matmul_slabs_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
+{
+    const so_quads &Q = E->quads;
+    so_narrow_plan best{};
+    best.us = 1e30;
+    for (uint32_t groups : {4u, 8u}) {
+        if (ctx->tune.matmul_slabs > 0 && groups != (ctx->tune.matmul_slabs == 8 ? 8u : 4u)) continue;
+        const uint32_t slabs = so_ceil_div(C, 4u * groups);
+        uint32_t ql = 0;
+        while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
+        const double wgs = (double)so_ceil_div(Q.nquads, 1u << ql) * slabs, cus = ctx->compute_units, rounds = std::ceil(wgs / cus);
+        const double passes = so_ceil_div(E->n, groups == 4u ? PASS_ROWS<4> : PASS_ROWS<8>), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
+        const double copy = (groups == 4u ? 0.53e-3 : 0.474e-3) * E->n * std::min(1.0, wgs / cus);
+        const double us = 1.0 + rounds * (3.43 + 0.966 * (passes - 1.0) + copy + chunks * (0.0635 + 0.0142 * groups)) + 0.2e-5 * Q.total_chunks * (groups == 8u ? slabs : 1.0);
+        if (us < best.us) best = so_narrow_plan{ql, groups, slabs, true, us};
     }
     return best;
 }
@@ -373,6 +511,7 @@ so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const so_nar
     const NarrowArgs a{Q.d_w, Q.d_rows, Q.d_info, E->m, E->n, C, Q.nquads, Q.ntiles, p.qw_log2, (uint32_t)(((1ull << 32) + C - 1u) / C),
                        dX, dBias, dY, E->d_Wd, E->d_idx, E->d_nnz, E->r};
     const dim3 blocks(so_ceil_div(Q.nquads, 1u << p.qw_log2), p.slabs);
+    if (p.passes) return p.groups == 4u ? launch<4, 1, true>(ctx, a, blocks, 2u * PASS_BYTES<4>, act) : launch<4, 2, true>(ctx, a, blocks, 2u * PASS_BYTES<8>, act);
     const size_t lds = lds_bytes(E->n, p.groups);
     switch (p.groups) {
     case 1:  return launch<1, 1>(ctx, a, blocks, lds, act);

@@ -73,6 +73,7 @@ static void read_tuning(so_tuning &t)
     t.matmul_quad_rows = env_int("SPARSEOPS_MATMUL_QUAD_ROWS", -1);
     t.matmul_quad_split = env_int("SPARSEOPS_MATMUL_QUAD_SPLIT", 0);
     t.matmul_narrow = env_int("SPARSEOPS_MATMUL_NARROW", -1);
+    t.matmul_slabs = env_int("SPARSEOPS_MATMUL_SLABS", -1);
     t.matmul_planes = env_int("SPARSEOPS_MATMUL_PLANES", -1);
     t.matmul_planes_split = env_int("SPARSEOPS_MATMUL_PLANES_SPLIT", 0);
     const int lanes = env_int("SPARSEOPS_MATVEC_LANES", 0);

@@ -24,6 +24,7 @@ struct so_tuning {
     int matmul_quad_rows = -1;  // SPARSEOPS_MATMUL_QUAD_ROWS: log2 of the quads per workgroup (0..4)
     int matmul_quad_split = 0;  // SPARSEOPS_MATMUL_QUAD_SPLIT: workgroups per output tile
     int matmul_narrow = -1;  // SPARSEOPS_MATMUL_NARROW: 0 forbids the narrow kernel on handles with the RBM layout, 1 forces it where it applies
+    int matmul_slabs = -1;   // SPARSEOPS_MATMUL_SLABS: 0 forbids the quad-union copy's kernel with X in LDS a part at a time, 4 and 8 force it where it applies, with slabs of 16 and 32 columns
     int matmul_planes = -1;  // SPARSEOPS_MATMUL_PLANES: 0 forbids the bf16-planes kernel on handles with the RBM layout, 1 forces it where the handle has the planes
     int matmul_planes_split = 0;   // SPARSEOPS_MATMUL_PLANES_SPLIT: workgroups per output tile
     int matvec_lanes = 0;    // SPARSEOPS_MATVEC_LANES: 8, 16, 32 or 64 lanes per row
@@ -240,9 +241,11 @@ so_status so_matmul_quad_launch(so_ctx *ctx, const so_ellpack *E, const so_quad_
                                 const float *dBias, float *dY, int act);
 
 // csrc/matmul_narrow.hip: few dense columns, or few rows, on the quad-union copy.
-struct so_narrow_plan { uint32_t qw_log2, groups, slabs; double us; };   // log2 of the quads per workgroup, 16-byte groups of a slab's row of X, slabs
+struct so_narrow_plan { uint32_t qw_log2, groups, slabs; bool passes; double us; };   // log2 of the quads per workgroup, 16-byte groups of a slab's row of X, slabs, X in LDS a part at a time
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
+bool so_matmul_slabs_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C);          // with X in LDS a part at a time
+so_narrow_plan so_matmul_slabs_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C);
 so_status so_matmul_narrow_launch(so_ctx *ctx, const so_ellpack *E, const so_narrow_plan &p, const float *dX, uint32_t C, const float *dBias, float *dY, int act);
 
 // csrc/matmul_planes.hip: the bf16 planes and their kernel.
