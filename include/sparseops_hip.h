@@ -234,6 +234,9 @@ const char *so_last_kernel(const so_ctx *ctx);
  * from the SO_LAYOUT_IDX16 copy when the handle has one (same result). */
 so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx,
                     const float *dBias, float *dy, int layout);
+/* The same with the result in host memory: waits, and reports as so_stage_out does.  `dy` holds m floats of device memory, which
+ * the call may use on the way.  Refused while a graph is being recorded. */
+so_status so_matvec_to_host(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, float *y, int layout);
 
 /* Per-layer convolution plan, built once at load time: for every stored nonzero
  * of E (Cout x Cin*kH*kW) the input offset and (dh, dw) of its tap -- the role of

@@ -53,6 +53,28 @@ template <> struct ColGroup<true> {
     }
 };
 
+// A launch whose result goes to pinned host memory (TELL): row i is the pair {y[i], turn}, in one store of 8 bytes, so that what the host
+// polls is the result itself.  The link takes some 10 ns per store instruction's line, whatever it holds: a workgroup's rows are
+// collected in LDS and leave 64 at a time.  (Each row by its own wave: 13 to 40 us more for 1500 to 4096 rows; words of 4 bytes
+// with a flag and a fence for all memory per workgroup 20 to 60.)
+struct Tell {
+    uint2 *rows;
+    uint32_t turn;
+};
+
+// What a workgroup holds for the host: `per` results of each of its passes, those of pass p from place p * stride + first on.
+template <bool TELL>
+__device__ __forceinline__ void tell_host(const Tell &tell, const float *held, uint32_t per, uint32_t stride, uint32_t first, uint32_t count, uint32_t at)
+{
+    if constexpr (TELL) {
+        __syncthreads();
+        const uint32_t pass = threadIdx.x / per, mine = pass * stride + first + threadIdx.x % per;
+        if (mine < count)
+            __hip_atomic_store(reinterpret_cast<unsigned long long *>(tell.rows + at + mine), (unsigned long long)tell.turn << 32 | __float_as_uint(held[threadIdx.x]),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 template <int G>
 __device__ __forceinline__ float group_sum(float v)
 {
@@ -156,12 +178,12 @@ __device__ __forceinline__ float group_row_dot(const float *__restrict__ Wd, con
 // slots, a half, a quarter or an eighth of a wave for shorter ones, so that short rows do not leave lanes idle).
 // MM: so_matmul's products with few columns, one of the row-major X and Y per blockIdx.y (their rows `C` floats apart),
 // with an activation.
-template <bool XLDS, int G, bool I16, bool MM>
+template <bool XLDS, int G, bool I16, bool MM, bool TELL>
 __global__ __launch_bounds__(kBlock)
 void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ idx,
                         const uint32_t *__restrict__ nnz, uint32_t count, uint32_t r,
                         const float *__restrict__ x, uint32_t n,
-                        const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act)
+                        const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act, Tell tell)
 {
     extern __shared__ float lds_x[];
     constexpr uint32_t RPW = 64 / G;                                     // rows per wave
@@ -174,7 +196,7 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
     // row is reduced, and those of the group's first row before x is staged, so that a wave always
     // has a row's worth of loads in flight.  Row lengths are fetched two rows ahead, so that
     // requesting a row never waits for its length.
-    uint32_t row = wave * RPW + grp;
+    uint32_t row = wave * RPW + grp, held = threadIdx.x / G;
     uint64_t beg = (uint64_t)row * r, end = beg + (row < count ? nnz[row] : 0u);
     uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
     RowLoads<I16> cur, nxt;
@@ -204,22 +226,26 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
             float v = (bias ? bias[row] : 0.0f) + s;
             if (MM) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
                        : act == SO_ACT_TANH ? so_epilogue<SO_ACT_TANH>(v) : v;
-            y[MM ? (size_t)row * C + blockIdx.y : row] = v;
+            if constexpr (TELL) {
+                lds_x[(XLDS ? n : 0u) + held] = v;      // behind x: the workgroup's 16 RPW consecutive rows of each pass
+            } else y[MM ? (size_t)row * C + blockIdx.y : row] = v;
         }
         cur = nxt;
         beg = nbeg;
         end = nend;
         len1 = len2;
+        held += kWavesPerBlock * RPW;
     }
+    tell_host<TELL>(tell, lds_x + (XLDS ? n : 0u), kWavesPerBlock * RPW, stride, blockIdx.x * (kWavesPerBlock * RPW), count, 0u);
 }
 
 // Rows of at most G*T nonzeros, G lanes per row.  Such a row is a chain of memory round trips and
 // nothing else, so all of a group's first row is requested before x is staged.
-template <bool XLDS, int G, int T, typename IdxT>
+template <bool XLDS, bool TELL, int G, int T, typename IdxT>
 __device__ __forceinline__ void short_rows(const float *__restrict__ Wd, const IdxT *__restrict__ idx,
                                            const uint2 *__restrict__ rows, uint32_t count, uint32_t block, uint32_t blocks,
                                            uint32_t r, const float *__restrict__ x, uint32_t n, float *lds_x,
-                                           const float *__restrict__ bias, float *__restrict__ y)
+                                           const float *__restrict__ bias, float *__restrict__ y, const Tell &tell, float *held, uint32_t at)
 {
     const uint32_t sub = threadIdx.x % G;
     const uint32_t stride = blocks * (kBlock / G);
@@ -245,14 +271,17 @@ __device__ __forceinline__ void short_rows(const float *__restrict__ Wd, const I
         }
         for (uint32_t j = sub + G * T; j < e.y; j += G) a = __builtin_fmaf(Wd[base + j], xs[idx[base + j]], a);
         a = group_sum<G>(a);
-        if (sub == 0) y[e.x] = (bias ? bias[e.x] : 0.0f) + a;
+        if (sub == 0) (TELL ? held[threadIdx.x / G] : y[e.x]) = (bias ? bias[e.x] : 0.0f) + a;
     }
+    uint32_t place = threadIdx.x / G;
     for (g += stride; g < count; g += stride) {
         const uint2 ec = en;
         if (g + stride < count) en = rows[g + stride];
         const float s = group_row_dot<G>(Wd, idx, (uint64_t)ec.x * r, ec.y, xs, sub);
-        if (sub == 0) y[ec.x] = (bias ? bias[ec.x] : 0.0f) + s;
+        place += kBlock / G;
+        if (sub == 0) (TELL ? held[place] : y[ec.x]) = (bias ? bias[ec.x] : 0.0f) + s;
     }
+    tell_host<TELL>(tell, held, kBlock / G, stride, block * (kBlock / G), count, at);
 }
 
 struct BinArgs {
@@ -263,13 +292,15 @@ struct BinArgs {
 
 constexpr uint32_t kBinnedTailBytes = 64;            // behind x in LDS: the 16 waves' partial sums of a workgroup-wide row
 
-template <bool XLDS, bool I16>
-__global__ __launch_bounds__(kBlock, 8)          // 64 registers: two workgroups per compute unit
+template <bool XLDS, bool I16, bool TELL>
+__global__ __launch_bounds__(kBlock, TELL ? 4 : 8)          // 64 registers: two workgroups per compute unit (TELL would spill)
 void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__ idxv, BinArgs ba, uint32_t r,
                           const float *__restrict__ x, uint32_t n,
-                          const float *__restrict__ bias, float *__restrict__ y)
+                          const float *__restrict__ bias, float *__restrict__ y, Tell tell)
 {
     extern __shared__ float lds_x[];
+    // TELL: the result in the classes' order, the longest first
+    float *const held = lds_x + (XLDS ? ((n + 3u) & ~3u) : 0u) + kBinnedTailBytes / sizeof(float);
     uint32_t b = blockIdx.x;
     if (b < ba.bwg) {
         // Rows of more than 4096 nonzeros: the 16 waves take the row's passes of 1024 slots in turn,
@@ -297,10 +328,11 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
                 float t = part[0];
 #pragma unroll
                 for (int w = 1; w < kWavesPerBlock; ++w) t += part[w];
-                y[e.x] = (bias ? bias[e.x] : 0.0f) + t;
+                (TELL ? held[g / ba.bwg] : y[e.x]) = (bias ? bias[e.x] : 0.0f) + t;
             }
             __syncthreads();                                        // part[] is reused by the next row
         }
+        tell_host<TELL>(tell, held, 1u, ba.bwg, b, ba.nwg, 0u);
         return;
     }
     b -= ba.bwg;
@@ -334,22 +366,25 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
                 }
             }
             const float s = group_sum<64>((a0 + a1) + (a2 + a3));
-            if (lane == 0) y[e.x] = (bias ? bias[e.x] : 0.0f) + s;
+            if (lane == 0) (TELL ? held[threadIdx.x >> 6] : y[e.x]) = (bias ? bias[e.x] : 0.0f) + s;
         }
+        uint32_t place = threadIdx.x >> 6;
         for (g += stride; g < ba.n64; g += stride) {
             const uint2 ec = en;
             if (g + stride < ba.n64) en = ba.rows64[g + stride];
             const uint64_t nbeg = (uint64_t)ec.x * r;
             const float s = wave_row_dot<I16>(Wd4, idx4, nbeg, nbeg + ec.y, xs, lane);
-            if (lane == 0) y[ec.x] = (bias ? bias[ec.x] : 0.0f) + s;
+            place += kWavesPerBlock;
+            if (lane == 0) (TELL ? held[place] : y[ec.x]) = (bias ? bias[ec.x] : 0.0f) + s;
         }
+        tell_host<TELL>(tell, held, kWavesPerBlock, stride, b * kWavesPerBlock, ba.n64, ba.nwg);
     } else if (b < ba.b64 + ba.b16) {
         const typename ColGroup<I16>::E *idx = reinterpret_cast<const typename ColGroup<I16>::E *>(idxv);
-        short_rows<XLDS, 16, 8>(Wd, idx, ba.rows16, ba.n16, b - ba.b64, ba.b16, r, x, n, lds_x, bias, y);
+        short_rows<XLDS, TELL, 16, 8>(Wd, idx, ba.rows16, ba.n16, b - ba.b64, ba.b16, r, x, n, lds_x, bias, y, tell, held, ba.nwg + ba.n64);
     } else {
         const typename ColGroup<I16>::E *idx = reinterpret_cast<const typename ColGroup<I16>::E *>(idxv);
-        short_rows<XLDS, 4, 4>(Wd, idx, ba.rows4, ba.n4, b - ba.b64 - ba.b16, gridDim.x - ba.bwg - ba.b64 - ba.b16, r, x, n,
-                               lds_x, bias, y);
+        short_rows<XLDS, TELL, 4, 4>(Wd, idx, ba.rows4, ba.n4, b - ba.b64 - ba.b16, gridDim.x - ba.bwg - ba.b64 - ba.b16, r, x, n,
+                               lds_x, bias, y, tell, held, ba.nwg + ba.n64 + ba.n16);
     }
 }
 
@@ -387,11 +422,11 @@ bool use_lds(so_ctx *ctx, K kernel, uint32_t n, uint64_t nnz_total, uint32_t blo
 }
 
 // The row kernel on the row-major arrays, on the 16-bit columns when the handle has them.
-template <bool MM>
-void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, const float *dBias, float *dy, int act)
+template <bool MM, bool TELL>
+void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, const float *dBias, float *dy, int act, const Tell &tell)
 {
     const uint32_t cus = (uint32_t)ctx->compute_units;
-    const size_t lds = (size_t)E->n * sizeof(float);
+    const size_t held = TELL ? kBlock * sizeof(float) : 0, lds = (size_t)E->n * sizeof(float) + held;
     const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
     const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
     // Lanes per row by the longest row (one pass of 16 G slots should cover it), but never so
@@ -405,12 +440,12 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
     const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
 #define SO_MV_ROWS(G, I16)                                                                                         \
     do {                                                                                                       \
-        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, MM>, E->n, E->total_nnz, blocks))                        \
-            matvec_rows_kernel<true, G, I16, MM><<<dim3(blocks, C), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
-                                                                                   dx, E->n, dBias, dy, C, act);       \
+        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, MM, TELL>, E->n, E->total_nnz, blocks, held))            \
+            matvec_rows_kernel<true, G, I16, MM, TELL><<<dim3(blocks, C), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
+                                                                                   dx, E->n, dBias, dy, C, act, tell); \
         else                                                                                                   \
-            matvec_rows_kernel<false, G, I16, MM><<<dim3(blocks, C), kBlock, 0, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
-                                                                                  dx, E->n, dBias, dy, C, act);        \
+            matvec_rows_kernel<false, G, I16, MM, TELL><<<dim3(blocks, C), kBlock, held, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
+                                                                                  dx, E->n, dBias, dy, C, act, tell);  \
     } while (0)
 #define SO_MV_ROWS_G(I16)                                                                                          \
     do {                                                                                                       \
@@ -425,12 +460,76 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
 #undef SO_MV_ROWS
 }
 
+// The length classes in one launch; false: nothing to launch.
+template <bool TELL>
+bool launch_bins(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, const Tell &tell)
+{
+    const uint32_t cus = (uint32_t)ctx->compute_units;
+    const size_t held = TELL ? kBlock * sizeof(float) : 0, lds = (size_t)E->n * sizeof(float);
+    const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
+    const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
+    // One launch over the four length classes.  bins[] is ordered 4, 16, 64 lanes, workgroup.
+    BinArgs ba;
+    ba.rowswg = reinterpret_cast<const uint2 *>(E->bins[3].d_rows);  ba.nwg = E->bins[3].count;
+    ba.bwg = std::min(ba.nwg, cus);
+    ba.rows4 = reinterpret_cast<const uint2 *>(E->bins[0].d_rows);   ba.n4 = E->bins[0].count;
+    ba.rows16 = reinterpret_cast<const uint2 *>(E->bins[1].d_rows);  ba.n16 = E->bins[1].count;
+    ba.rows64 = reinterpret_cast<const uint2 *>(E->bins[2].d_rows);  ba.n64 = E->bins[2].count;
+    ba.b64 = std::min(so_ceil_div(ba.n64, kWavesPerBlock), 2u * cus);
+    ba.b16 = std::min(so_ceil_div(ba.n16, kBlock / 16), std::max(1u, cus / 4));
+    const uint32_t b4 = std::min(so_ceil_div(ba.n4, kBlock / 4), std::max(1u, cus / 4));
+    // Staging x pays while a workgroup gathers at least as many elements as it stages (use_lds): rather than
+    // give that up, a launch with few nonzeros per workgroup takes fewer workgroups of the wave-per-row class,
+    // down to one per compute unit (8192 rows of 820 nonzeros: 20.8 us unstaged on 512 workgroups).
+    if (E->n > 0) {
+        const uint64_t pays = E->total_nnz / E->n;                       // workgroups for which staging pays
+        const uint32_t others = ba.bwg + ba.b16 + b4;
+        if ((uint64_t)others + ba.b64 > pays && ba.b64 > cus)
+            ba.b64 = (uint32_t)std::max<uint64_t>(cus, pays > others ? pays - others : 0);
+    }
+    const uint32_t blocks = ba.bwg + ba.b64 + ba.b16 + b4;
+    if (blocks == 0) return false;
+    // TELL: a workgroup holds the results of all its passes, a thread each
+    if (TELL && (ba.nwg > ba.bwg * kBlock || ba.n64 > ba.b64 * kBlock || ba.n16 > ba.b16 * kBlock || ba.n4 > b4 * kBlock)) return false;
+    // x padded to whole 16-byte groups, then the partial sums of a workgroup-wide row
+    const size_t lds_tail = (((size_t)E->n + 3) & ~(size_t)3) * sizeof(float) + kBinnedTailBytes + held;
+#define SO_MV_BINNED(I16) \
+    do { \
+        if (use_lds(ctx, matvec_binned_kernel<true, I16, TELL>, E->n, E->total_nnz, blocks, lds_tail - lds)) \
+            matvec_binned_kernel<true, I16, TELL><<<blocks, kBlock, lds_tail, ctx->stream>>>(E->d_Wd, cols, ba, E->r, \
+                                                                                       dx, E->n, dBias, dy, tell); \
+        else \
+            matvec_binned_kernel<false, I16, TELL><<<blocks, kBlock, kBinnedTailBytes + held, ctx->stream>>>( \
+                E->d_Wd, cols, ba, E->r, dx, E->n, dBias, dy, tell); \
+    } while (0)
+    if (i16) SO_MV_BINNED(true);
+    else SO_MV_BINNED(false);
+#undef SO_MV_BINNED
+    return true;
+}
+
 } // namespace
 
 so_status so_matvec_columns(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
-    launch_rows<true>(ctx, E, dX, C, dBias, dY, act);
+    launch_rows<true, false>(ctx, E, dX, C, dBias, dY, act, Tell());
     return SO_OK;
+}
+
+// The layout of a launch that leaves it to the library.
+static int choose_layout(const so_ctx *ctx, const so_ellpack *E)
+{
+    // Length classes for skewed rows (the widest row far above the mean).  For even rows the row kernel, which
+    // requests a wave's next row while it sums the current one, is the better one except on 16-bit columns
+    // where the length-class launch fills its two workgroups per compute unit with two or three rows per wave
+    // (16384 columns, 820 nonzeros per row; rows / us row kernel / us length classes: 8192 / 9.3 / 10.1,
+    // 16384 / 15.6 / 15.0, 24576 / 21.7 / 21.7, 32768 / 27.5 / 28.3, 49152 / 39.3 / 42.4, 65536 / 51 / 56).
+    const bool skewed = (uint64_t)E->r * E->m > 2 * E->total_nnz + E->m;
+    const uint32_t per_wave_x2 = E->m / (16u * (uint32_t)ctx->compute_units);           // rows per wave of 2 x CUs workgroups, doubled
+    const bool few_rows = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0 && per_wave_x2 >= 4 && per_wave_x2 < 6;
+    if ((E->layouts & SO_LAYOUT_BINS) && (skewed || few_rows)) return SO_LAYOUT_BINS;
+    if ((E->layouts & SO_LAYOUT_SLOT) && E->max_nnz <= 64) return SO_LAYOUT_SLOT;
+    return SO_LAYOUT_ROW;
 }
 
 extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx,
@@ -440,30 +539,15 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
     if (E->m == 0) return SO_OK;
     SO_REQUIRE(dy != nullptr, "so_matvec: y is null");
     SO_REQUIRE(dx != nullptr || E->total_nnz == 0, "so_matvec: x is null");
-    if (layout == 0) {
-        // Length classes for skewed rows (the widest row far above the mean).  For even rows the row kernel, which
-        // requests a wave's next row while it sums the current one, is the better one except on 16-bit columns
-        // where the length-class launch fills its two workgroups per compute unit with two or three rows per wave
-        // (16384 columns, 820 nonzeros per row; rows / us row kernel / us length classes: 8192 / 9.3 / 10.1,
-        // 16384 / 15.6 / 15.0, 24576 / 21.7 / 21.7, 32768 / 27.5 / 28.3, 49152 / 39.3 / 42.4, 65536 / 51 / 56).
-        const bool skewed = (uint64_t)E->r * E->m > 2 * E->total_nnz + E->m;
-        const uint32_t per_wave_x2 = E->m / (16u * (uint32_t)ctx->compute_units);           // rows per wave of 2 x CUs workgroups, doubled
-        const bool few_rows = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0 && per_wave_x2 >= 4 && per_wave_x2 < 6;
-        if ((E->layouts & SO_LAYOUT_BINS) && (skewed || few_rows)) layout = SO_LAYOUT_BINS;
-        else if ((E->layouts & SO_LAYOUT_SLOT) && E->max_nnz <= 64) layout = SO_LAYOUT_SLOT;
-        else layout = SO_LAYOUT_ROW;
-    }
+    if (layout == 0) layout = choose_layout(ctx, E);
     SO_REQUIRE(layout == SO_LAYOUT_ROW || layout == SO_LAYOUT_SLOT || layout == SO_LAYOUT_BINS,
                "so_matvec: unknown layout %d", layout);
     SO_REQUIRE((E->layouts & layout) != 0, "so_matvec: layout %d was not uploaded", layout);
 
     const uint32_t cus = (uint32_t)ctx->compute_units;
     const size_t lds = (size_t)E->n * sizeof(float);
-    // the row-major kernels read the 16-bit copy of the columns when the handle has one
-    const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
-    const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
     if (layout == SO_LAYOUT_ROW) {
-        launch_rows<false>(ctx, E, dx, 1, dBias, dy, SO_ACT_NONE);
+        launch_rows<false, false>(ctx, E, dx, 1, dBias, dy, SO_ACT_NONE, Tell());
     } else if (layout == SO_LAYOUT_SLOT) {
         const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kBlock), 2u * cus));
 #define SO_MV_SLOT(T, COLS)                                                                                        \
@@ -478,43 +562,33 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
         if (E->d_idxT16 && ctx->tune.matvec_idx16 != 0) SO_MV_SLOT(uint16_t, E->d_idxT16);
         else SO_MV_SLOT(uint32_t, E->d_idxT);
 #undef SO_MV_SLOT
-    } else {
-        // One launch over the four length classes.  bins[] is ordered 4, 16, 64 lanes, workgroup.
-        BinArgs ba;
-        ba.rowswg = reinterpret_cast<const uint2 *>(E->bins[3].d_rows);  ba.nwg = E->bins[3].count;
-        ba.bwg = std::min(ba.nwg, cus);
-        ba.rows4 = reinterpret_cast<const uint2 *>(E->bins[0].d_rows);   ba.n4 = E->bins[0].count;
-        ba.rows16 = reinterpret_cast<const uint2 *>(E->bins[1].d_rows);  ba.n16 = E->bins[1].count;
-        ba.rows64 = reinterpret_cast<const uint2 *>(E->bins[2].d_rows);  ba.n64 = E->bins[2].count;
-        ba.b64 = std::min(so_ceil_div(ba.n64, kWavesPerBlock), 2u * cus);
-        ba.b16 = std::min(so_ceil_div(ba.n16, kBlock / 16), std::max(1u, cus / 4));
-        const uint32_t b4 = std::min(so_ceil_div(ba.n4, kBlock / 4), std::max(1u, cus / 4));
-        // Staging x pays while a workgroup gathers at least as many elements as it stages (use_lds): rather than
-        // give that up, a launch with few nonzeros per workgroup takes fewer workgroups of the wave-per-row class,
-        // down to one per compute unit (8192 rows of 820 nonzeros: 20.8 us unstaged on 512 workgroups).
-        if (E->n > 0) {
-            const uint64_t pays = E->total_nnz / E->n;                       // workgroups for which staging pays
-            const uint32_t others = ba.bwg + ba.b16 + b4;
-            if ((uint64_t)others + ba.b64 > pays && ba.b64 > cus)
-                ba.b64 = (uint32_t)std::max<uint64_t>(cus, pays > others ? pays - others : 0);
-        }
-        const uint32_t blocks = ba.bwg + ba.b64 + ba.b16 + b4;
-        if (blocks == 0) return SO_OK;
-        // x padded to whole 16-byte groups, then the partial sums of a workgroup-wide row
-        const size_t lds_tail = (((size_t)E->n + 3) & ~(size_t)3) * sizeof(float) + kBinnedTailBytes;
-#define SO_MV_BINNED(I16)                                                                                          \
-        do {                                                                                                       \
-            if (use_lds(ctx, matvec_binned_kernel<true, I16>, E->n, E->total_nnz, blocks, lds_tail - lds))         \
-                matvec_binned_kernel<true, I16><<<blocks, kBlock, lds_tail, ctx->stream>>>(E->d_Wd, cols, ba, E->r, \
-                                                                                           dx, E->n, dBias, dy);   \
-            else                                                                                                   \
-                matvec_binned_kernel<false, I16><<<blocks, kBlock, kBinnedTailBytes, ctx->stream>>>(               \
-                    E->d_Wd, cols, ba, E->r, dx, E->n, dBias, dy);                                                 \
-        } while (0)
-        if (i16) SO_MV_BINNED(true);
-        else SO_MV_BINNED(false);
-#undef SO_MV_BINNED
-    }
+    } else if (!launch_bins<false>(ctx, E, dx, dBias, dy, Tell())) return SO_OK;
     SO_LAUNCH_CHECK();
     return SO_OK;
+}
+
+// The result straight into the staging memory, one launch fewer in a chain that is nothing but launches and the link.  ellpack_matvec from
+// host arrays, us, a kernel for the way back / this: 1500 x 1000 at 90 % sparse 17.9 / 14.9, 2864 x 3084 at 97 % 19.3 / 16.1, 4096 x 4096 at 80 %
+// 21.6 / 17.6, 8000 x 2000 at 90 % 23.6 / 21.2; Zipf rows 1077 x 3800 19.4 / 15.8, 4096 x 4096 20.2 / 17.4.  Beyond kStagePairsMost rows the host's look at each
+// pair, and in the classes' order its walk over y, take longer than the launch did: 16384 x 2000 29.0 / 32.7, 12000 x 2000 with Zipf rows 24.2 / 26.3.
+extern "C" so_status so_matvec_to_host(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, float *y, int layout)
+{
+    SO_REQUIRE(ctx && E, "so_matvec_to_host: null argument");
+    if (E->m == 0) return SO_OK;
+    SO_REQUIRE(y != nullptr && dy != nullptr, "so_matvec_to_host: y is null");
+    SO_REQUIRE(!ctx->capturing, "so_matvec_to_host: not allowed while a graph is being recorded");
+    const int kernel = layout == 0 ? choose_layout(ctx, E) : layout;
+    const bool rows = kernel == SO_LAYOUT_ROW, bins = kernel == SO_LAYOUT_BINS && (E->layouts & SO_LAYOUT_BINS) && E->bin_order.size() == E->m;
+    Tell tell;
+    if ((rows || bins) && (dx != nullptr || E->total_nnz == 0) && so_stage_result(ctx, E->m, &tell.rows, &tell.turn)) {
+        bool told = false;
+        if (rows) launch_rows<false, true>(ctx, E, dx, 1, dBias, nullptr, SO_ACT_NONE, tell);
+        if (rows || launch_bins<true>(ctx, E, dx, dBias, nullptr, tell)) {
+            SO_LAUNCH_CHECK();
+            const so_status s = so_stage_result_take(ctx, E->m, rows ? nullptr : E->bin_order.data(), y, tell.turn, &told);
+            if (s != SO_OK || told) return s;
+        }
+    }
+    const so_status s = so_matvec(ctx, E, dx, dBias, dy, layout);
+    return s != SO_OK ? s : so_stage_out(ctx, y, dy, (size_t)E->m * sizeof(float));
 }

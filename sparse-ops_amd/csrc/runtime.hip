@@ -277,6 +277,7 @@ extern "C" so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t byte
 // ResNet-18-shaped stack on 12 images of 96 x 96 490 -> 470.  One image (or sample) is the same in either order and goes as before.
 constexpr size_t kStageIn = 4u << 20, kStageOut = 1u << 20, kStagePiece = 256u << 10, kStagePieceFirst = 128u << 10, kStagePieceMost = 1u << 20;
 constexpr size_t kStageFlag = kStageIn + kStageOut;      // {turn, waits given up} behind the two areas
+constexpr size_t kStagePairs = kStageFlag + 64;          // then the results that a launch writes itself: nothing else is ever there, so that an old pair has an old turn
 
 // Words of up to two arrays, 16 bytes per thread and load (ends by the word).
 __global__ __launch_bounds__(256)
@@ -360,7 +361,7 @@ static bool stage_ready(so_ctx *ctx)
 {
     if (ctx->h_stage) return true;
     void *p = nullptr, *d = nullptr;
-    if (hipHostMalloc(&p, kStageFlag + 64, hipHostMallocCoherent) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (hipHostMalloc(&p, kStagePairs + kStagePairsMost * 8, hipHostMallocCoherent) != hipSuccess) { (void)hipGetLastError(); return false; }
     // cleared on the context's stream, which does not wait for the null stream
     if (hipMalloc(&d, 64) != hipSuccess || so_fill_zero(ctx, d, 64) != SO_OK) {
         (void)hipGetLastError();
@@ -368,7 +369,7 @@ static bool stage_ready(so_ctx *ctx)
         (void)hipHostFree(p);
         return false;
     }
-    std::memset((char *)p + kStageFlag, 0, 64);
+    std::memset((char *)p + kStageFlag, 0, 64 + kStagePairsMost * 8);
     ctx->h_stage = (char *)p;
     ctx->d_stage_done = (uint32_t *)d;
     ctx->stage_used = 0;
@@ -424,6 +425,38 @@ static so_status poll_word(so_ctx *ctx, volatile uint32_t *flag, uint32_t turn, 
         __builtin_ia32_pause();
     }
     std::atomic_thread_fence(std::memory_order_acquire);
+    ctx->stage_used = 0;                       // the stream's earlier work, and with it every way in, is done
+    return SO_OK;
+}
+
+bool so_stage_result(so_ctx *ctx, uint32_t floats, uint2 **rows, uint32_t *turn)
+{
+    // (a launch with bounded waits before this one: the general way back looks at their word)
+    if (floats > kStagePairsMost || ctx->waits_pending || !stage_ready(ctx)) return false;
+    *rows = (uint2 *)(ctx->h_stage + kStagePairs);
+    *turn = ++ctx->stage_turn;
+    return true;
+}
+
+so_status so_stage_result_take(so_ctx *ctx, uint32_t floats, const uint32_t *order, float *dst, uint32_t turn, bool *told)
+{
+    volatile const uint64_t *const rows = (volatile const uint64_t *)(ctx->h_stage + kStagePairs);
+    *told = true;
+    uint32_t at = 0;
+    for (uint32_t spin = 1; at < floats; ++spin) {
+        for (uint64_t pair; at < floats && (uint32_t)((pair = rows[at]) >> 32) == turn; ++at) {
+            const uint32_t bits = (uint32_t)pair;
+            std::memcpy(dst + (order ? order[at] : at), &bits, 4);
+        }
+        if (at == floats) break;
+        if (spin % 4096u == 0) {
+            const hipError_t e = hipStreamQuery(ctx->stream);
+            if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+            SO_HIP(e);
+            if ((uint32_t)(rows[at] >> 32) != turn) { *told = false; return SO_OK; }
+        }
+        __builtin_ia32_pause();
+    }
     ctx->stage_used = 0;                       // the stream's earlier work, and with it every way in, is done
     return SO_OK;
 }
@@ -885,6 +918,8 @@ extern "C" so_status so_ellpack_upload(so_ctx *ctx, const float *Wd, const uint3
                 }
                 if (!pairs.empty()) s = upload_array(ctx, pairs.data(), pairs.size(), &E->bins[b].d_rows);
             }
+            if (m <= kStagePairsMost)
+                for (int b = 3; b >= 0; --b) E->bin_order.insert(E->bin_order.end(), rows[b].begin(), rows[b].end());
         }
 
         if (s == SO_OK && (layouts & SO_LAYOUT_TILED) && m > 0) s = build_tiled(ctx, E, Wd, idx, nnz);

@@ -86,6 +86,8 @@ struct so_ctx {
 };
 
 // Rows of one length class for the binned matvec: `group` lanes cooperate on a row.
+constexpr uint32_t kStagePairsMost = 8192;       // floats of a result that a launch writes to the staging memory itself (so_matvec_to_host)
+
 struct so_bin {
     uint32_t group = 0;      // 4, 16 or 64 lanes per row, 1024: a whole workgroup
     uint32_t count = 0;      // rows in this class
@@ -172,6 +174,7 @@ struct so_ellpack {
     uint16_t *d_idx16 = nullptr; // [m*r] the columns of d_idx in 16 bits (SO_LAYOUT_IDX16, n <= 65536)
     uint16_t *d_idxT16 = nullptr;// [r*m] the same for d_idxT (SO_LAYOUT_SLOT with SO_LAYOUT_IDX16)
     so_bin bins[4];              // SO_LAYOUT_BINS
+    std::vector<uint32_t> bin_order;   // their rows, the class of the longest first (kept up to kStagePairsMost rows)
     so_tiled tiled;              // SO_LAYOUT_TILED
     so_rbmm rbmm;                // SO_LAYOUT_RBM
     so_quads quads;              // SO_LAYOUT_RBM, unless the matrix is too sparse for it (d_w is null)
@@ -269,6 +272,11 @@ so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t 
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
 // since the last look (their results are invalid).  Every entry point that waits for the stream ends with this.
 so_status so_stream_wait(so_ctx *ctx, const char *who);
+
+// A result of up to kStagePairsMost floats that a launch itself writes to the staging memory, as a pair {value, turn} for each of them, and the wait for
+// all of them.  False: there is no room, or no staging memory; *told false: the stream ended without them.
+bool so_stage_result(so_ctx *ctx, uint32_t floats, uint2 **rows, uint32_t *turn);
+so_status so_stage_result_take(so_ctx *ctx, uint32_t floats, const uint32_t *order, float *dst, uint32_t turn, bool *told);   // float i goes to dst[order[i]]
 
 // Kernels that ask for more than 48 KB of dynamic LDS must be told so once per device: this does
 // it the first time `kernel` is seen on the context's device (hipSuccess when already done).

@@ -20,7 +20,7 @@ LAYOUT_ROW, LAYOUT_SLOT, LAYOUT_BINS, LAYOUT_TILED, LAYOUT_RBM, LAYOUT_IDX16 = 1
 SYMBOLS = (
     "so_device_count so_init so_destroy so_last_error so_device_info so_tuning_reload so_malloc so_free so_h2d so_d2h "
     "so_stage_in so_stage_out so_stage_in_transposed so_stage_out_transposed so_d2d so_fill_zero so_sync so_timer_begin so_timer_end so_ellpack_upload so_ellpack_free "
-    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
+    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_matvec_to_host so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
     "so_conv2d so_maxpool so_gap so_add so_act so_transpose so_reverse_axes3 so_copy_rows so_graph_begin so_graph_end "
     "so_graph_launch so_graph_free so_rbm_upload so_rbm_free so_rbm_dims so_conv_plan_set_rbm so_conv_plan_rbm_info").split()
 
@@ -87,6 +87,7 @@ def load_library(path=None):
         "so_matmul": [_vp, _vp, _vp, _u32, _vp, _vp, ct.c_int],
         "so_matmul_reserve": [_vp, _vp, _u32],
         "so_matvec": [_vp, _vp, _vp, _vp, _vp, ct.c_int],
+        "so_matvec_to_host": [_vp, _vp, _vp, _vp, _vp, _vp, ct.c_int],
         "so_conv_plan_create": [_vp, _vp, ct.POINTER(ConvGeom), ct.POINTER(_vp)],
         "so_conv_plan_free": [_vp, _vp],
         "so_conv_plan_window": [_vp, ct.POINTER(ct.c_uint32)],

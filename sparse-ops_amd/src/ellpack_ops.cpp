@@ -104,6 +104,5 @@ void ellpack_matvec(const Ellpack &E, const float *x, const float *bias, float *
     st.x.reserve(std::size_t(E.n) * sizeof(float));
     st.y.reserve(std::size_t(E.m) * sizeof(float));
     const float *dBias = stage_operands(ctx, x, std::size_t(E.n) * sizeof(float), bias, E.m);
-    check(so_matvec(ctx, dE, st.x.f32(), dBias, st.y.f32(), 0), "so_matvec");
-    check(so_stage_out(ctx, y, st.y.get(), std::size_t(E.m) * sizeof(float)), "so_stage_out(y)");
+    check(so_matvec_to_host(ctx, dE, st.x.f32(), dBias, st.y.f32(), y, 0), "so_matvec_to_host");
 }
