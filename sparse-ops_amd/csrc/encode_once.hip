@@ -13,25 +13,37 @@
 //
 // The wait for the other workgroups has every one of them resident (a workgroup per compute unit), unless somebody else's
 // kernel holds some of the chip: it gives up after a bounded number of looks, the host is told, and the two passes do
-// the call again, and the context's next ones.  The words the workgroups tell each other carry the call's number, so nothing needs clearing.
+// the call again, and the context's next ones.  The words the workgroups tell each other carry the call's number, so nothing needs clearing.  One
+// wave of each looks, at four workgroups per lane, and everything it adds up is in DPP steps: the places, the wait and the agreement took 1.2, 3.0 and 1.0 us by
+// barriers and shuffles over the workgroup, and 0.6, 1.8 and 0.2 now.
 //
-// What bounds it: the read of W (8192 x 8192: 47 to 54 us, by workgroup, of which the copy's rate would take 43), then what
-// follows the slowest workgroup: 4 us until all know of all, 8 to 12 us of writing 61 MB at 90 % sparse; launch and the
-// host's wait 13.  Memory moves 269 MB in, W once, and 61 out (counters); at 50 % sparse, where LDS keeps one piece of eight, 450 in.
-// The whole call on one matrix again and again, two passes / this one, us:
+// Results of up to kThroughSlots slots are stored past the L2, and the first workgroup tells the host when all are done: the end of the kernel, its
+// writing back of the caches, and a kernel or a wait of the runtime's behind it cost 3 us more.
 //
-//   8192 x 8192 at 98 / 90 / 80 / 50 % sparse    100 / 75, 112 / 85, 135 / 108, 195 / 175
-//   4096 x 4096, 2048 x 2048 at 90 %              45 / 36,  27 / 24
-//   8192 x 8192 at 90 %, changing matrices       127.6 / 91.9
+// What bounds it: the read of W (8192 x 8192: 42 to 57 us, by workgroup and XCD, of which the copy's rate would take 43), then what
+// follows the slowest workgroup: 2 us until all know of all, 15 of writing 61 MB at 90 % sparse; launch and the
+// host's word 9.  Memory moves 269 MB in, W once, and 61 out (counters); at 50 % sparse, where LDS keeps one piece of eight, 450 in.
+// The whole call on one matrix again and again, two passes / this one with the host told behind the kernel / this one, us:
+//
+//   8192 x 8192 at 97 / 50 % sparse                            100 / 78.9 / 74.2, 195 / 174 / 174
+//   4096 x 4096, 2199 x 2165 at 90 %, 5442 x 2598 at 63 %      45 / 33.4 / 30.5,  27 / 22.9 / 20.8,  - / 39.6 / 37.1
+//   8192 x 8192 at 97 / 90 %, 2199 x 2165 at 91 %, changing matrices   - / 85.9 / 80.3, 127.6 / 92.9 / 91.6,  - / 24.7 / 22.8
 #include "so_internal.h"
 
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
 constexpr uint32_t THREADS = 1024, WAVES = 16, GROUPS = 8;        // groups of 256 columns a piece has at most
 constexpr uint32_t HEAD = 256;                                    // bytes of LDS before the table of counts
 constexpr uint32_t kEntryLimit = 4096;                            // words of the table of counts
+constexpr uint32_t MOST_WGS = 256, kGaveUp = 0xffffffffu;
+// Up to this many slots of the result are stored past the L2, and the host is told from the kernel; beyond, the caches' writing together of neighbouring pieces gains
+// more than the end of the kernel and its wait cost.  Changing matrices, slots, us past the L2 / not: 4096 x 4096 at 80 % sparse, 3.5 M, 39.2 / 41.3, 5442 x 2598 at 63 %, 5.3 M,
+// 45.5 / 47.1, 3491 x 4690 at 56 %, 7.5 M, 52.4 / 49.2, 8192 x 8192 at 97 / 90 %, 2.2 and 7.5 M, 80.3 / 84.6, 99 to 109 / 91.6.
+constexpr uint64_t kThroughSlots = 6u << 20;
+static_assert(3 * MOST_WGS <= 2 * kEncodeTold, "the words have room");
 constexpr uint32_t kLooks = 1u << 11;                             // of a bounded wait: about 3 ms, where the workgroups differ by some 10 us
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -52,10 +64,40 @@ constexpr uint32_t kLeastColumns = 768;
 struct EncodeArgs {
     const float *W;
     uint32_t m, n, r_cap, groups, segs, part, table_bytes, call, looks;
-    unsigned long long *told;        // [2][workgroups]: {call, longest row}, {call, nonzeros}
+    unsigned long long *told;        // [3][MOST_WGS]: {call, longest row}, {call, nonzeros}, {call, 0} when done
     uint32_t *host, *nnz, *idx;
     float *Wd;
+    so_tell tell;
 };
+
+// THROUGH: stores past the L2, which other compute units and streams do not share: what has been written is there when the host is told, without the end of
+// the kernel.  (The s_nop: a store of 16 bytes reads its registers late, which the compiler sees to for its own stores only.)
+template <bool THROUGH, typename T>
+__device__ __forceinline__ void store(T *p, T v)
+{
+    if constexpr (THROUGH) so_store_through(p, v);
+    else *p = v;
+}
+template <bool THROUGH, typename T, typename V>
+__device__ __forceinline__ void store4(T *p, V v)
+{
+    if constexpr (THROUGH) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(v) : "memory");
+    else *reinterpret_cast<V *>(p) = v;
+}
+
+// Over the 64 lanes, in DPP steps; in every lane.
+template <bool MAX>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v)
+{
+    const auto step = [&](uint32_t u) { v = MAX ? max(v, u) : v + u; };
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true));      // row_shr:1, 2, 4, 8
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true));
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, true));      // row_bcast:15 into rows 1 and 3, :31 into 2 and 3
+    step(__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, true));
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
 
 // A packed piece of c entries: the counts after each group but the last (two bytes each), values, column bytes.
 __device__ __forceinline__ uint32_t piece_bytes(uint32_t c) { return 16u + ((c * 5u + 15u) & ~15u); }
@@ -99,6 +141,7 @@ __device__ __forceinline__ void piece_pack(const f32x4u (&v)[GROUPS], uint32_t c
 }
 
 // Writes a packed piece whose first column is c0 to the row's slots from wd, ix on, four entries per lane.
+template <bool THROUGH>
 __device__ __forceinline__ void piece_write(const char *from, uint32_t c, uint32_t c0, float *wd, uint32_t *ix, uint32_t lane)
 {
     const float *val = reinterpret_cast<const float *>(from + 16);
@@ -117,12 +160,12 @@ __device__ __forceinline__ void piece_write(const char *from, uint32_t c, uint32
     for (uint32_t k = lane * 4u; k < c; k += 256u) {
         if (k + 4u <= c) {
             const uint32_t b = *reinterpret_cast<const uint32_t *>(col + k);
-            *reinterpret_cast<f32x4u *>(wd + k) = *reinterpret_cast<const f32x4u *>(val + k);
-            *reinterpret_cast<u32x4u *>(ix + k) = u32x4u{column(k, b & 0xffu), column(k + 1u, (b >> 8) & 0xffu), column(k + 2u, (b >> 16) & 0xffu), column(k + 3u, b >> 24)};
+            store4<THROUGH>(wd + k, *reinterpret_cast<const f32x4u *>(val + k));
+            store4<THROUGH>(ix + k, u32x4u{column(k, b & 0xffu), column(k + 1u, (b >> 8) & 0xffu), column(k + 2u, (b >> 16) & 0xffu), column(k + 3u, b >> 24)});
         } else {
             for (uint32_t i = k; i < c; ++i) {
-                wd[i] = val[i];
-                ix[i] = column(i, col[i]);
+                store<THROUGH>(wd + i, val[i]);
+                store<THROUGH>(ix + i, column(i, col[i]));
             }
         }
     }
@@ -132,13 +175,11 @@ __global__ __launch_bounds__(THREADS)
 void ellpack_encode_once_kernel(EncodeArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
-    uint32_t *smax = reinterpret_cast<uint32_t *>(lds), &gave_up = smax[WAVES];
-    unsigned long long *ssum = reinterpret_cast<unsigned long long *>(lds + 128);
+    uint32_t *smax = reinterpret_cast<uint32_t *>(lds), *ssum = smax + WAVES, &agreed = smax[2 * WAVES];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t wgs = gridDim.x, wg = blockIdx.x, rows = (a.m - wg + wgs - 1u) / wgs, items = rows * a.segs;     // rows wg, wg + wgs, ...
     uint32_t *table = reinterpret_cast<uint32_t *>(lds + HEAD);      // [rows][segs + 1]: counts, then the places of the pieces in their row
     char *part = lds + HEAD + a.table_bytes + wave * a.part;
-    if (tid == 0) gave_up = 0u;
 
     auto load = [&](uint32_t j, f32x4u (&v)[GROUPS]) {
         const uint32_t row = j / a.segs, c0 = (j - row * a.segs) * a.groups * 256u, jw = c0 + lane * 4u;
@@ -183,120 +224,155 @@ void ellpack_encode_once_kernel(EncodeArgs a)
     }
     __syncthreads();
 
-    // counts -> places; the workgroup's longest row and its count
-    uint32_t vmax = 0;
-    unsigned long long vsum = 0;
-    for (uint32_t row = tid; row < rows; row += THREADS) {
-        uint32_t *t = table + (size_t)row * (a.segs + 1u), at = 0;
-        for (uint32_t s = 0; s < a.segs; ++s) { const uint32_t c = t[s]; t[s] = at; at += c; }
-        t[a.segs] = at;
-        a.nnz[wg + row * wgs] = at;
-        vmax = max(vmax, at);
-        vsum += at;
-    }
-    auto reduce = [&]() {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) { vmax = max(vmax, (uint32_t)__shfl_xor(vmax, off, 64)); vsum += __shfl_xor(vsum, off, 64); }
-        if (lane == 0) { smax[wave] = vmax; ssum[wave] = vsum; }
-        __syncthreads();
-        vmax = smax[0];
-        vsum = ssum[0];
-        for (uint32_t w = 1; w < WAVES; ++w) { vmax = max(vmax, smax[w]); vsum += ssum[w]; }
-    };
-    reduce();
-    if (tid == 0) {
-        __hip_atomic_store(a.told + wg, (unsigned long long)a.call << 32 | vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(a.told + wgs + wg, (unsigned long long)a.call << 32 | (uint32_t)vsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    // every workgroup's, a thread each
-    vmax = 0;
-    vsum = 0;
-    bool got = tid >= wgs;
-    for (uint32_t look = 0; look < a.looks && !__all(got); ++look) {
-        if (!got) {
-            const unsigned long long x = __hip_atomic_load(a.told + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long y = __hip_atomic_load(a.told + wgs + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((uint32_t)(x >> 32) == a.call && (uint32_t)(y >> 32) == a.call) { got = true; vmax = (uint32_t)x; vsum = (uint32_t)y; }
+    // counts -> places; the workgroup's longest row and its count, by as many waves as 64 rows each take
+    const uint32_t takers = min(WAVES, (rows + 63u) / 64u);
+    if (wave < takers) {
+        uint32_t vmax = 0, vsum = 0;
+        for (uint32_t row = tid; row < rows; row += takers * 64u) {
+            uint32_t *t = table + (size_t)row * (a.segs + 1u), at = 0;
+            for (uint32_t s = 0; s < a.segs; ++s) { const uint32_t c = t[s]; t[s] = at; at += c; }
+            t[a.segs] = at;
+            so_store_through(a.nnz + wg + row * wgs, at);
+            vmax = max(vmax, at);
+            vsum += at;
         }
-        if (!__all(got)) __builtin_amdgcn_s_sleep(4);
+        vmax = wave_reduce<true>(vmax);
+        vsum = wave_reduce<false>(vsum);
+        if (takers > 1u && lane == 0) { smax[wave] = vmax; ssum[wave] = vsum; }
+        if (takers == 1u && lane == 0) { smax[0] = vmax; ssum[0] = vsum; }
     }
-    if (!__all(got) && lane == 0) gave_up = 1u;
-    __syncthreads();                                              // also: everybody has read smax and ssum
-    if (gave_up) {
-        if (tid == 0) a.host[3] = 1u;
+    if (takers > 1u) __syncthreads();
+    // The first wave tells the other workgroups, and looks for their words, four per lane: word(value) for each that has come; true: all have.
+    const auto put = [&](unsigned long long *words, uint32_t value) {
+        __hip_atomic_store(words + wg, (unsigned long long)a.call << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const auto look_for_all = [&](const unsigned long long *words, auto &&start, auto &&word) {
+        bool all = false;
+        for (uint32_t look = 0; look < a.looks && !all; ++look) {
+            unsigned long long x[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) x[i] = __hip_atomic_load(words + min(lane + 64u * i, wgs - 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bool got = true;
+            start();
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                got &= (uint32_t)(x[i] >> 32) == a.call;
+                if (lane + 64u * i < wgs) word((uint32_t)x[i]);
+            }
+            all = __all(got);
+            if (!all) __builtin_amdgcn_s_sleep(1);
+        }
+        return all;
+    };
+    const auto to_host = [&](uint32_t *word, uint32_t value) { __hip_atomic_store(word, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    if (wave == 0) {
+        const uint32_t mine = wave_reduce<true>(lane < takers ? smax[lane] : 0u), sum = wave_reduce<false>(lane < takers ? ssum[lane] : 0u);
+        if (lane == 0) { put(a.told, mine); put(a.told + MOST_WGS, sum); }
+        uint32_t longest = 0;
+        const bool all = look_for_all(a.told, [&]() { longest = 0; }, [&](uint32_t x) { longest = max(longest, x); });
+        longest = wave_reduce<true>(longest);
+        if (lane == 0) agreed = all ? longest : kGaveUp;
+    }
+    __syncthreads();
+    const uint32_t r = __builtin_amdgcn_readfirstlane(agreed);
+    const bool fits = r != kGaveUp && r <= a.r_cap, plain = fits && (uint64_t)a.m * r > kThroughSlots;
+    // By the first workgroup's first wave: the longest row and all counts, or that somebody has given up, and the word that the host polls.
+    const auto tell = [&]() {
+        uint32_t low = 0, high = 0;
+        const bool all = r != kGaveUp && look_for_all(a.told + MOST_WGS, [&]() { low = high = 0; }, [&](uint32_t x) { low += x & 0xffffu; high += x >> 16; });
+        const unsigned long long total = ((unsigned long long)wave_reduce<false>(high) << 16) + wave_reduce<false>(low);
+        if (lane == 0) {
+            if (!all) to_host(a.host + 3, 1u);
+            else { to_host(a.host, r); to_host(a.host + 1, (uint32_t)total); to_host(a.host + 2, (uint32_t)(total >> 32)); }
+            if (plain) to_host(a.tell.flag + 2, 1u);
+        }
+        so_tell_now(a.tell);
+    };
+    if (r == kGaveUp && tid == 0) to_host(a.host + 3, 1u);
+    if (plain && wg == 0 && wave == 0) tell();                    // from here on the host waits for the stream's end
+    auto write_out = [&](auto through) {
+        constexpr bool THROUGH = decltype(through)::value;
+        // out: first the pieces that were kept, then the others, packed again now that LDS has room
+        bool again = false;
+        for (uint32_t pass = 0; pass == 0u || (pass == 1u && again); ++pass) {
+            uint32_t at = 0;
+            for (uint32_t j = wave; j < items; j += WAVES) {
+                const uint32_t row = j / a.segs, s = j - row * a.segs;
+                const uint32_t *t = table + (size_t)row * (a.segs + 1u) + s;
+                const uint32_t first = __builtin_amdgcn_readfirstlane(t[0]), c = __builtin_amdgcn_readfirstlane(t[1]) - first, c0 = s * a.groups * 256u;
+                const size_t slot = (size_t)(wg + row * wgs) * r + first;
+                float *wd = a.Wd + slot;
+                uint32_t *ix = a.idx + slot;
+                const char *from = part + at;
+                const bool kept = at + piece_bytes(c) <= a.part;
+                if (kept) at += piece_bytes(c);
+                else again = true;
+                if (kept != (pass == 0u)) continue;
+                if (pass == 0u) {
+                    piece_write<THROUGH>(from, c, c0, wd, ix, lane);
+                    continue;
+                }
+                if (j + WAVES < items) load(j, next);
+                else {
+#pragma unroll
+                    for (uint32_t u = 0; u < GROUPS; ++u) next[u] = v[u];          // the wave's last piece is still here
+                }
+                if (piece_bytes(c) <= a.part) {
+                    piece_pack(next, c, part, lane);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    piece_write<THROUGH>(part, c, c0, wd, ix, lane);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    continue;
+                }
+                uint32_t k = 0;                                       // more than a wave's part of LDS holds: straight to memory
+#pragma unroll
+                for (uint32_t u = 0; u < GROUPS; ++u) {
+                    uint32_t pos = k;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint64_t mask = __ballot(next[u][e] != 0.0f);
+                        pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, pos));
+                        k += (uint32_t)__popcll(mask);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (next[u][e] != 0.0f) {
+                            store<THROUGH>(wd + pos, (float)next[u][e]);
+                            store<THROUGH>(ix + pos, c0 + u * 256u + lane * 4u + (uint32_t)e);
+                            ++pos;
+                        }
+                }
+            }
+        }
+        for (uint32_t row = wave; row < rows; row += WAVES) {
+            const size_t slot = (size_t)(wg + row * wgs) * r;
+            for (uint32_t k = table[(size_t)row * (a.segs + 1u) + a.segs] + lane; k < r; k += 64u) { store<THROUGH>(a.Wd + slot + k, 0.0f); store<THROUGH>(a.idx + slot + k, 0u); }
+        }
+        };
+    if (plain) {
+        write_out(std::false_type());
         return;
     }
-    reduce();
-    const uint32_t r = __builtin_amdgcn_readfirstlane(vmax);
-    if (wg == 0 && tid == 0) { a.host[0] = r; a.host[1] = (uint32_t)vsum; a.host[2] = (uint32_t)(vsum >> 32); }
-    if (r > a.r_cap) return;
-
-    // out: first the pieces that were kept, then the others, packed again now that LDS has room
-    bool again = false;
-    for (uint32_t pass = 0; pass == 0u || (pass == 1u && again); ++pass) {
-        uint32_t at = 0;
-        for (uint32_t j = wave; j < items; j += WAVES) {
-            const uint32_t row = j / a.segs, s = j - row * a.segs;
-            const uint32_t *t = table + (size_t)row * (a.segs + 1u) + s;
-            const uint32_t first = __builtin_amdgcn_readfirstlane(t[0]), c = __builtin_amdgcn_readfirstlane(t[1]) - first, c0 = s * a.groups * 256u;
-            const size_t slot = (size_t)(wg + row * wgs) * r + first;
-            float *wd = a.Wd + slot;
-            uint32_t *ix = a.idx + slot;
-            const char *from = part + at;
-            const bool kept = at + piece_bytes(c) <= a.part;
-            if (kept) at += piece_bytes(c);
-            else again = true;
-            if (kept != (pass == 0u)) continue;
-            if (pass == 0u) {
-                piece_write(from, c, c0, wd, ix, lane);
-                continue;
-            }
-            if (j + WAVES < items) load(j, next);
-            else {
-#pragma unroll
-                for (uint32_t u = 0; u < GROUPS; ++u) next[u] = v[u];          // the wave's last piece is still here
-            }
-            if (piece_bytes(c) <= a.part) {
-                piece_pack(next, c, part, lane);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                piece_write(part, c, c0, wd, ix, lane);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-                continue;
-            }
-            uint32_t k = 0;                                       // more than a wave's part of LDS holds: straight to memory
-#pragma unroll
-            for (uint32_t u = 0; u < GROUPS; ++u) {
-                uint32_t pos = k;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint64_t mask = __ballot(next[u][e] != 0.0f);
-                    pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, pos));
-                    k += (uint32_t)__popcll(mask);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (next[u][e] != 0.0f) {
-                        wd[pos] = next[u][e];
-                        ix[pos] = c0 + u * 256u + lane * 4u + (uint32_t)e;
-                        ++pos;
-                    }
-            }
-        }
-    }
-    for (uint32_t row = wave; row < rows; row += WAVES) {
-        const size_t slot = (size_t)(wg + row * wgs) * r;
-        for (uint32_t k = table[(size_t)row * (a.segs + 1u) + a.segs] + lane; k < r; k += 64u) { a.Wd[slot + k] = 0.0f; a.idx[slot + k] = 0u; }
-    }
+    if (fits) write_out(std::true_type());
+    // This workgroup is done; the first one tells the host when all are.
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");           // this wave's stores have arrived
+    __syncthreads();
+    if (wave != 0) return;
+    if (lane == 0) put(a.told + 2u * MOST_WGS, 0u);
+    if (wg != 0) return;
+    const bool all = look_for_all(a.told + 2u * MOST_WGS, []() {}, [](uint32_t) {});
+    if (!all && lane == 0) to_host(a.host + 3, 1u);
+    tell();
 }
 
 } // namespace
 
 so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, uint32_t r_cap, uint32_t *dNnz, float *dWd, uint32_t *dIdx,
-                         void *told, uint32_t *host_header, bool *done)
+                         void *told, uint32_t *host_header, bool *done, volatile uint32_t **at_end)
 {
     *done = false;
     if ((uint64_t)m * n < kLeastElements || n < kLeastColumns) return SO_OK;
-    const uint32_t wgs = std::min({m, (uint32_t)ctx->compute_units, kEncodeTold}), rows = so_ceil_div(m, wgs);
+    const uint32_t wgs = std::min({m, (uint32_t)ctx->compute_units, MOST_WGS}), rows = so_ceil_div(m, wgs);
     if (4ull * m < 3ull * rows * wgs) return SO_OK;
     // pieces of equal width, one per wave at least
     const uint32_t n256 = so_ceil_div(n, 256u);
@@ -320,8 +396,10 @@ so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t 
     a.looks = ctx->tune.wait_spins >= 0 ? (uint32_t)ctx->tune.wait_spins : kLooks;
     a.told = (unsigned long long *)told;
     a.host = host_header; a.nnz = dNnz; a.idx = dIdx; a.Wd = dWd;
+    a.tell = so_tell_next(ctx);
+    *at_end = a.tell.flag + 2;
     SO_HIP(so_allow_big_lds(ctx, (const void *)ellpack_encode_once_kernel));
-    host_header[3] = 0u;
+    host_header[3] = a.tell.flag[2] = 0u;
     ellpack_encode_once_kernel<<<wgs, THREADS, lds, ctx->stream>>>(a);
     SO_LAUNCH_CHECK();
     ctx->last_kernel = "encode-once";

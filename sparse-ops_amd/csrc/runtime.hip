@@ -471,12 +471,22 @@ constexpr uint64_t kToldElements = 1u << 25;
 static so_status told_wait(so_ctx *ctx, uint64_t elements, const char *who)
 {
     if (elements > kToldElements) return so_stream_wait(ctx, who);
-    volatile uint32_t *const flag = ctx->h_wait_gave_up + 12;
-    const uint32_t turn = ++ctx->told_turn;
-    so_tell_host_kernel<<<1, 64, 0, ctx->stream>>>(ctx->d_wait_gave_up, (uint32_t *)flag, turn);
+    const so_tell tell = so_tell_next(ctx);
+    so_tell_host_kernel<<<1, 64, 0, ctx->stream>>>(tell.gave_up, tell.flag, tell.turn);
     SO_LAUNCH_CHECK();
+    return so_tell_wait(ctx, who);
+}
+
+so_tell so_tell_next(so_ctx *ctx)
+{
+    return so_tell{ctx->d_wait_gave_up, (uint32_t *)ctx->h_wait_gave_up + 12, ++ctx->told_turn};
+}
+
+so_status so_tell_wait(so_ctx *ctx, const char *who)
+{
+    volatile uint32_t *const flag = ctx->h_wait_gave_up + 12;
     bool told = false;
-    const so_status s = poll_word(ctx, flag, turn, &told);
+    const so_status s = poll_word(ctx, flag, ctx->told_turn, &told);
     if (s != SO_OK) return s;
     if (!told || (ctx->waits_pending && flag[1] != 0)) return so_stream_wait(ctx, who);
     ctx->waits_pending = false;
@@ -1458,8 +1468,10 @@ extern "C" so_status so_ellpack_encode_noalloc(so_ctx *ctx, const float *dDense,
     const uint64_t spared = ctx->encode_spared;
     if (counts && (uint64_t)m * r_cap != 0) {
         bool once = false;
-        so_status s = so_encode_once(ctx, dDense, m, n, r_cap, dNnz, dWd, dIdx, (char *)ctx->static_scratch + kEncodeToldOffset, ctx->h_encode_header, &once);
-        if (s == SO_OK && once) s = told_wait(ctx, (uint64_t)m * n, "so_ellpack_encode_noalloc");
+        volatile uint32_t *at_end = nullptr;
+        so_status s = so_encode_once(ctx, dDense, m, n, r_cap, dNnz, dWd, dIdx, (char *)ctx->static_scratch + kEncodeToldOffset, ctx->h_encode_header, &once, &at_end);
+        if (s == SO_OK && once) s = so_tell_wait(ctx, "so_ellpack_encode_noalloc");
+        if (s == SO_OK && once && *at_end != 0) s = told_wait(ctx, (uint64_t)m * n, "so_ellpack_encode_noalloc");
         if (s != SO_OK) return s;
         if (once && ctx->h_encode_header[3] == 0) {
             ctx->encode_spare_next = kEncodeSpareFirst;

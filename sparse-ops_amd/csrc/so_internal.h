@@ -264,10 +264,32 @@ so_status so_matmul_planes_launch(so_ctx *ctx, const so_ellpack *E, const so_pla
                                   const float *dBias, float *dY, int act);
 
 // csrc/encode_once.hip: encode from one read of the matrix.  `told` holds 2 * kEncodeTold words of 64 bits that nothing else writes;
-// *done: launched, and after the stream's end host_header has {r, total nnz (low, high), 1 where it has to be done again}.
+// *done: launched, and once the host has been told (so_tell_wait) or, where *at_end then says so, the stream has ended host_header has
+// {r, total nnz (low, high), 1 where it has to be done again}.
 constexpr uint32_t kEncodeTold = 1024;
 so_status so_encode_once(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n, uint32_t r_cap, uint32_t *dNnz, float *dWd, uint32_t *dIdx,
-                         void *told, uint32_t *host_header, bool *done);
+                         void *told, uint32_t *host_header, bool *done, volatile uint32_t **at_end);
+
+// A launch that tells the host itself when its results are there: stored past the L2, so that the end of the kernel is not needed for others to see them.
+struct so_tell {
+    const uint32_t *gave_up;      // the context's word of bounded waits, for flag[1]
+    uint32_t *flag;               // pinned: the turn, that word, one for the launch's own use
+    uint32_t turn;
+};
+so_tell so_tell_next(so_ctx *ctx);
+// Waits for such a launch, the context's last so_tell_next's, and reports as so_stream_wait does.
+so_status so_tell_wait(so_ctx *ctx, const char *who);
+
+template <typename T>
+__device__ __forceinline__ void so_store_through(T *p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// By a whole wave whose stores before it, also to the host, are to be there first.
+__device__ __forceinline__ void so_tell_now(const so_tell &tell)
+{
+    if ((threadIdx.x & 63u) == 0) __hip_atomic_store(tell.flag + 1, __hip_atomic_load(tell.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+    if ((threadIdx.x & 63u) == 0) __hip_atomic_store(tell.flag, tell.turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Waits for the context's stream and then reports, as SO_ERR_HIP, bounded waits that gave up in kernels launched
 // since the last look (their results are invalid).  Every entry point that waits for the stream ends with this.
