@@ -1379,9 +1379,12 @@ so_status encode_launch(so_ctx *ctx, const float *dDense, uint32_t m, uint32_t n
         }
     }
     if (pack && m) {
-        // A row of 1024 columns or more is shared by a workgroup's four waves.
+        // A row of more than the 2048 columns that a wave holds at a time is shared by a workgroup's four waves, but where there are rows enough for all
+        // waves and it is no more than twice as long.  Us, shared / a wave per row, 90 % sparse: 4072 x 1030 33.2 / 23.2, 2796 x 1500 28.4 / 21.6,
+        // 2036 x 1030 24.3 / 19.2, 254 x 1030 17.7 / 17.2 (three of the four waves have nothing there); 2036 x 2060 26.1 / 22.7, 1398 x 3000 23.6 / 23.1, 1025 x 4090
+        // 23.6 / 23.5, 509 x 2060 18.9 / 19.3, 254 x 2060 18.2 / 20.3.
         const uint32_t fold = count && !fold_apart ? nblocks : 0u;
-        const bool shared = n >= 1024u;
+        const bool shared = n > 4096u || (n > 2048u && m < 4u * (uint32_t)ctx->compute_units);
         const uint32_t blocks = std::max(1u, std::min(shared ? m : so_ceil_div(m, 4u), 16u * (uint32_t)ctx->compute_units));
         if (shared) ellpack_pack_kernel<4><<<blocks, 256, 0, ctx->stream>>>(dDense, m, n, header, fold, host_header, r_cap, dNnz, dWd, dIdx, tail_words);
         else ellpack_pack_kernel<1><<<blocks, 256, 0, ctx->stream>>>(dDense, m, n, header, fold, host_header, r_cap, dNnz, dWd, dIdx, tail_words);
