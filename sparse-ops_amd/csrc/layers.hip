@@ -5,99 +5,95 @@
 #include "so_internal.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
 constexpr int kBlock = 256;
 
-// applyMaxPool (src/layers/pool.cpp:28-101): -inf start, taps outside the image skipped.
+// applyMaxPool (src/layers/pool.cpp:28-101): -inf start, taps outside the image skipped.  A lane takes VEC batch entries of an output (4: B % 4 == 0,
+// 16-byte aligned tensors) and BH x BW taps at a time, row by row, all requested before the first comparison: a tap outside the image is read at the window's
+// nearest place inside and compared as -inf, which replaces nothing.  Kernels of more than three columns go a row of eight taps at a time.
+//
+// What bounds it: memory on large images, the launch and two round trips on small ones.  One tap at a time, a load each, 3x3/2 on 64 channels of 112x112 took
+// 24.5 us at batch 32 (128 MB in and out) and 6.8 at 8, now 19.2 (6.7 TB/s) and 5.4; 5x5 and 9x9 on 16 of 20x20 5.7 -> 4.5 and 12.6 -> 8.5.
+template <int VEC, int BH, int BW, class Index>
 __global__ __launch_bounds__(kBlock)
-void maxpool_kernel(so_pool_geom p, const float *__restrict__ X, uint32_t B, uint64_t total,
-                    float *__restrict__ Y)
+void maxpool_kernel(so_pool_geom p, const float *__restrict__ X, uint32_t Bv, Index total, float *__restrict__ Y)
 {
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t q = (uint64_t)blockIdx.x * kBlock + threadIdx.x; q < total; q += stride) {
-        const uint32_t b = (uint32_t)(q % B);
-        uint64_t t = q / B;
-        const uint32_t wo = (uint32_t)(t % p.W_out); t /= p.W_out;
-        const uint32_t ho = (uint32_t)(t % p.H_out);
-        const uint32_t c = (uint32_t)(t / p.H_out);
-        const int32_t h0 = (int32_t)ho * p.sH - p.padH0, w0 = (int32_t)wo * p.sW - p.padW0;
-        float v = -INFINITY;
-        for (int32_t kh = 0; kh < p.kH; ++kh) {
-            const int32_t hin = h0 + kh;
-            if ((uint32_t)hin >= p.H) continue;
-            for (int32_t kw = 0; kw < p.kW; ++kw) {
-                const int32_t win = w0 + kw;
-                if ((uint32_t)win >= p.W) continue;
-                const float x = X[(((uint64_t)c * p.H + (uint32_t)hin) * p.W + (uint32_t)win) * B + b];
-                v = x > v ? x : v;
-            }
-        }
-        Y[q] = v;
-    }
-}
-
-// The same with four batch entries per lane (B % 4 == 0, 16-byte aligned tensors): one 16-byte
-// load per tap, 32-bit index arithmetic.  Per component the comparisons run in the same order.
-__global__ __launch_bounds__(kBlock)
-void maxpool4_kernel(so_pool_geom p, const float *__restrict__ X, uint32_t B4, uint32_t total,
-                     float *__restrict__ Y)
-{
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const vec *__restrict__ Xv = reinterpret_cast<const vec *>(X);
     // Workgroups are dealt round-robin to the 8 XCDs; give each XCD one contiguous eighth of the
     // output instead, so that the input rows two neighbouring output rows share meet in one L2.
     const uint32_t per_xcd = gridDim.x / 8u;                     // the grid is a multiple of 8
     const uint32_t vblock = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-    const uint32_t chunk = (total + 8u * per_xcd - 1u) / (8u * per_xcd);        // outputs per workgroup
-    const uint32_t q_end = min(total, (vblock + 1u) * chunk);
-    for (uint32_t q = vblock * chunk + threadIdx.x; q < q_end; q += kBlock) {
-        const uint32_t b = q % B4;
-        uint32_t t = q / B4;
-        const uint32_t wo = t % p.W_out; t /= p.W_out;
-        const uint32_t ho = t % p.H_out;
-        const uint32_t c = t / p.H_out;
+    const Index chunk = (total + 8u * per_xcd - 1u) / (8u * per_xcd);           // outputs per workgroup
+    const Index q_end = min(total, (Index)(vblock + 1u) * chunk);
+    for (Index q = (Index)vblock * chunk + threadIdx.x; q < q_end; q += kBlock) {
+        Index t = q / Bv;
+        const uint32_t b = (uint32_t)(q - t * Bv);
+        const Index row = t / p.W_out;
+        const uint32_t wo = (uint32_t)(t - row * p.W_out);
+        const Index c = row / p.H_out;
+        const uint32_t ho = (uint32_t)(row - c * p.H_out);
         const int32_t h0 = (int32_t)ho * p.sH - p.padH0, w0 = (int32_t)wo * p.sW - p.padW0;
-        float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-        const float4 *__restrict__ Xc = reinterpret_cast<const float4 *>(X) + (size_t)c * p.H * p.W * B4 + b;
-        for (int32_t kh = 0; kh < p.kH; ++kh) {
-            const int32_t hin = h0 + kh;
-            if ((uint32_t)hin >= p.H) continue;
-            for (int32_t kw = 0; kw < p.kW; ++kw) {
-                const int32_t win = w0 + kw;
-                if ((uint32_t)win >= p.W) continue;
-                const float4 x = Xc[((uint32_t)hin * p.W + (uint32_t)win) * B4];
-                v.x = x.x > v.x ? x.x : v.x;
-                v.y = x.y > v.y ? x.y : v.y;
-                v.z = x.z > v.z ? x.z : v.z;
-                v.w = x.w > v.w ? x.w : v.w;
+        const vec *__restrict__ Xc = Xv + (size_t)c * p.H * p.W * Bv + b;
+        vec v = -INFINITY;
+        for (int32_t kh = 0; kh < p.kH; kh += BH)
+            for (int32_t kw = 0; kw < p.kW; kw += BW) {
+                vec x[BH][BW];
+                bool in[BH][BW];
+#pragma unroll
+                for (int i = 0; i < BH; ++i)
+#pragma unroll
+                    for (int j = 0; j < BW; ++j) {
+                        const int32_t h = h0 + kh + i, w = w0 + kw + j;
+                        in[i][j] = ((uint32_t)h < p.H) & ((uint32_t)w < p.W) & (kh + i < p.kH) & (kw + j < p.kW);
+                        const uint32_t hc = min((uint32_t)max(h, 0), p.H - 1u), wc = min((uint32_t)max(w, 0), p.W - 1u);
+                        x[i][j] = Xc[((Index)hc * p.W + wc) * Bv];
+                    }
+#pragma unroll
+                for (int i = 0; i < BH; ++i)
+#pragma unroll
+                    for (int j = 0; j < BW; ++j)
+#pragma unroll
+                        for (int e = 0; e < VEC; ++e) {
+                            const float xe = in[i][j] ? x[i][j][e] : -INFINITY;
+                            v[e] = xe > v[e] ? xe : v[e];
+                        }
             }
-        }
-        reinterpret_cast<float4 *>(Y)[q] = v;
+        reinterpret_cast<vec *>(Y)[q] = v;
     }
 }
 
 // applyGlobalAveragePool (src/layers/pool.cpp:103-154): fp32 running sum over h
-// then w, times 1.0f/float(H*W).  One lane per (c, b).
-__global__ __launch_bounds__(kBlock)
+// then w, times 1.0f/float(H*W).  One lane per (c, b), 32 of its values requested before the first is added: what bounds it is a round trip for each such
+// group and, with few batch entries, a cache line per value and lane.  Waves of their own, so that 512 channels of one image meet
+// eight compute units.  Eight at a time, 512 channels of 7x7 at batch 1 took 4.6 us, now 3.6, which is the launch; 256 of 14x14 at batch 32 6.5 -> 5.8.
+constexpr int kGapBlock = 64;
+__global__ __launch_bounds__(kGapBlock)
 void gap_kernel(uint32_t C, uint32_t HW, const float *__restrict__ X, uint32_t B, float scale,
                 float *__restrict__ Y)
 {
     const uint64_t total = (uint64_t)C * B;
-    const uint64_t stride = (uint64_t)gridDim.x * kBlock;
-    for (uint64_t q = (uint64_t)blockIdx.x * kBlock + threadIdx.x; q < total; q += stride) {
-        const uint32_t b = (uint32_t)(q % B);
-        const uint64_t c = q / B;
-        const float *xp = X + c * HW * B + b;
+    const uint64_t stride = (uint64_t)gridDim.x * kGapBlock;
+    for (uint64_t q = (uint64_t)blockIdx.x * kGapBlock + threadIdx.x; q < total; q += stride) {
+        const uint64_t c = total < (1ull << 32) ? (uint32_t)q / B : q / B;
+        const float *xp = X + c * HW * B + (q - c * B);
         float s = 0.0f;
         uint32_t i = 0;
-        for (; i + 8 <= HW; i += 8) {            // eight loads in flight, the additions still in order
-            float v[8];
+        auto add = [&](auto count) {
+            constexpr uint32_t U = decltype(count)::value;
+            float v[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = xp[(uint64_t)(i + u) * B];
+            for (uint32_t u = 0; u < U; ++u) v[u] = xp[(uint64_t)min(i + u, HW - 1u) * B];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) s = s + v[u];
-        }
-        for (; i < HW; ++i) s = s + xp[(uint64_t)i * B];
+            for (uint32_t u = 0; u < U; ++u) s = s + (i + u < HW ? v[u] : -0.0f);
+        };
+        for (; HW - i > 32u; i += 32u) add(std::integral_constant<uint32_t, 32>());
+        if (HW - i > 16u) add(std::integral_constant<uint32_t, 32>());
+        else if (HW - i > 8u) add(std::integral_constant<uint32_t, 16>());
+        else add(std::integral_constant<uint32_t, 8>());
         Y[q] = s * scale;
     }
 }
@@ -226,11 +222,29 @@ extern "C" so_status so_maxpool(so_ctx *ctx, const so_pool_geom *p, const float 
     SO_REQUIRE((uint64_t)(p->H_out - 1) * p->sH < (uint64_t)p->H + p->padH0 &&
                (uint64_t)(p->W_out - 1) * p->sW < (uint64_t)p->W + p->padW0,
                "so_maxpool: output size does not fit the input");
-    if (B % 4 == 0 && (((uintptr_t)dX | (uintptr_t)dY) & 15) == 0 && total / 4 < (1ull << 31) &&
-        (uint64_t)p->H * p->W * (B / 4) < (1ull << 31))
-        maxpool4_kernel<<<(blocks_for(ctx, total / 4) + 7u) / 8u * 8u, kBlock, 0, ctx->stream>>>(*p, dX, B / 4, (uint32_t)(total / 4), dY);   // a multiple of 8: the kernel deals whole eighths to the XCDs
-    else
-        maxpool_kernel<<<blocks_for(ctx, total), kBlock, 0, ctx->stream>>>(*p, dX, B, total, dY);
+    const bool four = B % 4 == 0 && (((uintptr_t)dX | (uintptr_t)dY) & 15) == 0;
+    const uint32_t Bv = four ? B / 4 : B;
+    const uint64_t outputs = four ? total / 4 : total;
+    const uint32_t blocks = (blocks_for(ctx, outputs) + 7u) / 8u * 8u;       // a multiple of 8: the kernel deals whole eighths to the XCDs
+    so_pool_geom taps = *p;
+    if (p->H == 0 || p->W == 0) taps.kH = 0;                                 // no tap to read
+    const bool small = outputs < (1ull << 31) && (uint64_t)p->H * p->W * Bv < (1ull << 31);
+#define SO_POOL_LAUNCH(VEC, BH, BW)                                                                                                     \
+    do {                                                                                                                                 \
+        if (small) maxpool_kernel<VEC, BH, BW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, (uint32_t)outputs, dY);                   \
+        else maxpool_kernel<VEC, BH, BW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, outputs, dY);                                   \
+    } while (0)
+#define SO_POOL_TAPS(VEC)                                                                                                               \
+    do {                                                                                                                                 \
+        if (p->kH == 1 && p->kW == 1) SO_POOL_LAUNCH(VEC, 1, 1);                                                                         \
+        else if (p->kH <= 2 && p->kW <= 2) SO_POOL_LAUNCH(VEC, 2, 2);                                                                         \
+        else if (p->kW <= 3) SO_POOL_LAUNCH(VEC, 3, 3);                                                                                  \
+        else SO_POOL_LAUNCH(VEC, 1, 8);                                                                                                  \
+    } while (0)
+    if (four) SO_POOL_TAPS(4);
+    else SO_POOL_TAPS(1);
+#undef SO_POOL_TAPS
+#undef SO_POOL_LAUNCH
     SO_LAUNCH_CHECK();
     return SO_OK;
 }
@@ -243,7 +257,8 @@ extern "C" so_status so_gap(so_ctx *ctx, uint32_t C, uint32_t H, uint32_t W, con
     if (total == 0) return SO_OK;
     SO_REQUIRE(dX && dY && H && W, "so_gap: null tensor or empty plane");
     const float scale = 1.0f / (float)(H * W);
-    gap_kernel<<<blocks_for(ctx, total), kBlock, 0, ctx->stream>>>(C, H * W, dX, B, scale, dY);
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>((total + kGapBlock - 1) / kGapBlock, (uint64_t)ctx->compute_units * 32);
+    gap_kernel<<<blocks, kGapBlock, 0, ctx->stream>>>(C, H * W, dX, B, scale, dY);
     SO_LAUNCH_CHECK();
     return SO_OK;
 }
