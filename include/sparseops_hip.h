@@ -278,6 +278,12 @@ so_status so_conv2d(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint
  * and must not alias dY. */
 so_status so_conv2d_add(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,
                         const float *dBias, const float *dResidual, float *dY, int act);
+/* so_conv2d of two plans on the same input, one after the other: a residual block's first convolution and the
+ * projection of its skip connection.  One launch where both would take the column kernel, or the same form of the
+ * windowed one, with SO_ACT_NONE or SO_ACT_RELU; the same bits either way.  The input and the two outputs must not
+ * overlap.  No counterpart in the reference. */
+so_status so_conv2d_pair(so_ctx *ctx, const so_conv_plan *planA, const so_conv_plan *planB, const float *dX, uint32_t B,
+                         const float *dBiasA, float *dYA, int actA, const float *dBiasB, float *dYB, int actB);
 
 /* ---- row-block-merged (RBM) format ---------------------------------------
  * RBMPlan / RBMBlock / RBMColPair (include/rbm_conv.hpp:8-27) as build_rbm_from_ellpack

@@ -300,11 +300,8 @@ __device__ __forceinline__ void rotate_priority(uint32_t turn)
 // All of the kernel's arguments into the scalar cache in one round trip.  Left to the compiler they are asked for where they are first used, and a line that
 // nobody has touched yet is a round trip of its own, some 0.2 us: launches of a few microseconds (3 channels of 60x31 at batch 48, 5 of 13x27 at
 // batch 20, 6 of 80x80 at batch 16) take 4.3 us instead of 4.7, 6.7 instead of 7.2, 6.9 instead of 7.4.
-constexpr size_t kWinKernelArgs = 3 * sizeof(void *) + sizeof(WinArgs) + sizeof(so_conv_geom) + 5 * sizeof(void *);
-static_assert(kWinKernelArgs > 0x140 + 4 && kWinKernelArgs <= 0x180, "lines of 64 bytes that touch_arguments reads");
-__device__ __forceinline__ void touch_arguments()
+__device__ __forceinline__ void touch_arguments(const __attribute__((address_space(4))) char *args)
 {
-    const auto *args = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
     uint32_t sink;
     asm volatile("s_load_dword %0, %1, 0x0\n\ts_load_dword %0, %1, 0x40\n\ts_load_dword %0, %1, 0x80\n\t"
                  "s_load_dword %0, %1, 0xc0\n\ts_load_dword %0, %1, 0x100\n\ts_load_dword %0, %1, 0x140\n\ts_waitcnt lgkmcnt(0)"
@@ -312,20 +309,18 @@ __device__ __forceinline__ void touch_arguments()
 }
 
 template <int CPW, int LPP, int ACT, int PX>
-__global__ __launch_bounds__(kWinThreads)
-void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__restrict__ gbase,
-                          const uint32_t *__restrict__ quads, WinArgs a, so_conv_geom g,
-                          const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
-                          const float *__restrict__ resid, float *__restrict__ Y)
+__device__ __forceinline__ void window_convolution(const int4 *__restrict__ stream, const uint32_t *__restrict__ gbase,
+                                                   const uint32_t *__restrict__ quads, const WinArgs &a, const so_conv_geom &g,
+                                                   const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
+                                                   const float *__restrict__ resid, float *__restrict__ Y, uint32_t wg, bool relu)
 {
     extern __shared__ float4 win_lds[];
-    touch_arguments();
     constexpr uint32_t BT = LPP * 4, PPW = 64 / LPP, SHIFT = (LPP == 8 ? 7 : LPP == 4 ? 6 : LPP == 2 ? 5 : 4);
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t cgi = window_div(wave, a.pg, a.mPg), pgi = wave - cgi * a.pg;
     WinPlace place;
-    if (!window_workgroup(a, place)) return;
+    if (!window_workgroup(a, wg, place)) return;
     const uint32_t tile_y = window_div(place.tile, a.tiles_x, a.mTilesX);
     const uint32_t th0 = tile_y * a.TH, tw0 = (place.tile - tile_y * a.tiles_x) * a.TW;
     const uint32_t grp = place.y * a.cg + cgi;                       // channel group of this wave
@@ -334,8 +329,8 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     const bool computes = cgi < a.cg && grp < a.groups;              // the other waves only help copying
     const uint32_t gi = computes ? grp : 0u;
     // Asked for first: the stream's place, on which its first entries wait.
-    const uint32_t first_quad = gbase[gi];
-    const uint32_t *__restrict__ qp = quads + (size_t)gi * a.nch * CPW;
+    const uint32_t first_quad = ((so_constant<uint32_t>)(uintptr_t)gbase)[gi];
+    const so_constant<uint32_t> qp = (so_constant<uint32_t>)(uintptr_t)quads + (size_t)gi * a.nch * CPW;
     uint32_t qfirst[CPW];
 #pragma unroll
     for (int c = 0; c < CPW; ++c) qfirst[c] = qp[c];
@@ -433,7 +428,7 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
     float acc[CPW][PX][4];
 #pragma unroll
     for (int c = 0; c < CPW; ++c) {
-        const float b0 = (bias && computes && co0 + c < g.Cout) ? bias[co0 + c] : 0.0f;
+        const float b0 = (bias && computes && co0 + c < g.Cout) ? ((so_constant<float>)(uintptr_t)bias)[co0 + c] : 0.0f;
 #pragma unroll
         for (int x = 0; x < PX; ++x) acc[c][x][0] = acc[c][x][1] = acc[c][x][2] = acc[c][x][3] = b0;
     }
@@ -589,22 +584,60 @@ void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__res
                     v[0] += rv.x; v[1] += rv.y; v[2] += rv.z; v[3] += rv.w;
                 }
                 float4 out;
-                out.x = so_epilogue<ACT>(v[0]); out.y = so_epilogue<ACT>(v[1]);
-                out.z = so_epilogue<ACT>(v[2]); out.w = so_epilogue<ACT>(v[3]);
+                out.x = conv_epilogue<ACT>(v[0], relu); out.y = conv_epilogue<ACT>(v[1], relu);
+                out.z = conv_epilogue<ACT>(v[2], relu); out.w = conv_epilogue<ACT>(v[3], relu);
                 *reinterpret_cast<float4 *>(Y + at) = out;
             }
         }
     }
 }
 
+// One convolution's operands.  The kernels read them where they are used, from the arguments: held as values from the start, as the compiler does with
+// a kernel's own, 20 to 31 scalar registers spill when the body is shared (84 to 117 reads back: stems of 96x96 images 12.4 and 22.5 us instead of 11.0 and 20.9).
+struct WinCall {
+    const int4 *stream;
+    const uint32_t *gbase, *quads;
+    WinArgs a;
+    so_conv_geom g;
+    const float *X, *bias, *resid;
+    float *Y;
+    uint32_t B, relu;                // relu: kActNoneOrRelu
+};
+struct WinPair {
+    WinCall call[2];
+    uint32_t wgs0;
+};
+static_assert(sizeof(WinCall) > 0x140 + 4 && sizeof(WinCall) <= 0x180, "lines of 64 bytes that touch_arguments reads");
+template <int CPW, int LPP, int ACT, int PX>
+__global__ __launch_bounds__(kWinThreads)
+void conv2d_window_kernel(WinCall)
+{
+    const auto *args = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    touch_arguments(args);
+    const WinCall &c = *(const WinCall *)args;
+    window_convolution<CPW, LPP, ACT, PX>(c.stream, c.gbase, c.quads, c.a, c.g, c.X, c.B, c.bias, c.resid, c.Y, blockIdx.x, false);
+}
+
+// Two convolutions of one input: the first's workgroups, a multiple of 8 of them, then the second's.
+template <int CPW, int LPP, int PX>
+__global__ __launch_bounds__(kWinThreads)
+void conv2d_window_pair_kernel(WinPair)
+{
+    const auto *args = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
+    const uint32_t wgs0 = *(const uint32_t *)(args + offsetof(WinPair, wgs0));
+    const bool second = blockIdx.x >= wgs0;
+    args += second ? sizeof(WinCall) : 0;
+    touch_arguments(args);
+    const WinCall &c = *(const WinCall *)args;
+    window_convolution<CPW, LPP, kActNoneOrRelu, PX>(c.stream, c.gbase, c.quads, c.a, c.g, c.X, c.B, c.bias, nullptr, c.Y, blockIdx.x - (second ? wgs0 : 0u), c.relu != 0u);
+}
+
 template <int CPW, int LPP, int PX>
 void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, dim3 grid, size_t lds,
                        const float *dX, uint32_t B, const float *dBias, const float *dResid, float *dY, int act)
 {
-#define SO_WIN_LAUNCH(A)                                                                                   \
-    conv2d_window_kernel<CPW, LPP, A, PX><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(        \
-        reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a,       \
-        plan->g, dX, B, dBias, dResid, dY)
+    const WinCall c{reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a, plan->g, dX, dBias, dResid, dY, B, 0};
+#define SO_WIN_LAUNCH(A) conv2d_window_kernel<CPW, LPP, A, PX><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(c)
     switch (act) {
     case SO_ACT_RELU:    SO_WIN_LAUNCH(SO_ACT_RELU); break;
     case SO_ACT_SIGMOID: SO_WIN_LAUNCH(SO_ACT_SIGMOID); break;
@@ -624,7 +657,7 @@ hipError_t window_allow_lds(so_ctx *ctx)
                         (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_SIGMOID, PX>, (const void *)conv2d_window_kernel<CPW, LPP, SO_ACT_TANH, PX>};
     for (const void *f : k)
         if (e == hipSuccess) e = so_allow_big_lds(ctx, f);
-    return e;
+    return e == hipSuccess ? so_allow_big_lds(ctx, (const void *)conv2d_window_pair_kernel<CPW, LPP, PX>) : e;
 }
 
 so_status window_configure(so_ctx *ctx)
@@ -647,15 +680,13 @@ uint64_t window_workgroups(const so_conv_window &w, uint32_t cout, uint32_t cpw,
     return (uint64_t)w.tiles_x * w.tiles_y * so_ceil_div(so_ceil_div(cout, cpw), cg) * std::max(1u, B / (4u * lpp));
 }
 
-// Launches the windowed kernel if the plan has the layout, the batch suits it and the grid
-// covers the chip; *done says whether it did.
+// The windowed kernel's arguments and grid; false: the plan's layout, the batch or a grid that does not cover the chip
+// rules it out (the last unless it is forced).
 template <uint32_t LPP>
-so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
-                        const float *dResid, float *dY, int act, bool forced, bool *done)
+bool window_arguments(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, bool forced, WinArgs &a, dim3 &grid, size_t &lds)
 {
     const so_conv_window &w = plan->win;
     constexpr uint32_t PPW = 64 / LPP;
-    WinArgs a;
     a.TH = w.TH; a.TW = w.TW; a.IH = w.IH; a.IW = w.IW; a.cc = w.cc; a.nch = w.nch; a.tiles_x = w.tiles_x;
     a.groups = w.groups;
     const uint32_t px = LPP == 4 ? w.px : 1u;
@@ -681,16 +712,28 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     a.mIW = window_magic(a.IW); a.mIH = window_magic(a.IH); a.mTW = window_magic(a.TW);
     a.mTilesX = window_magic(a.tiles_x); a.mPg = window_magic(a.pg);
     a.ws = so_lds::wait_status{ctx->tune.wait_spins >= 0 ? (uint32_t)ctx->tune.wait_spins : so_lds::kSyncSpins, ctx->d_wait_gave_up};
-    const size_t lds = (size_t)a.nbuf * a.buf_f4 * 16 + so_lds::kSyncBytes;
+    lds = (size_t)a.nbuf * a.buf_f4 * 16 + so_lds::kSyncBytes;
     // a layout whose chunks were sized for a smaller batch tile than this batch's does not fit
-    if (LPP > w.lpp && (lds > (size_t)ctx->max_lds_bytes || a.win_f4 > (uint32_t)kWinMaxPerThread * kWinThreads)) return SO_OK;
-    const dim3 grid(w.tiles_x * w.tiles_y, so_ceil_div(w.groups, a.cg), B / (4 * LPP));
+    if (LPP > w.lpp && (lds > (size_t)ctx->max_lds_bytes || a.win_f4 > (uint32_t)kWinMaxPerThread * kWinThreads)) return false;
+    grid = dim3(w.tiles_x * w.tiles_y, so_ceil_div(w.groups, a.cg), B / (4 * LPP));
     const uint64_t wgs = (uint64_t)grid.x * grid.y * grid.z;
     // Even a grid that covers an eighth of the chip beats the gather kernel on long rows (measured on the
     // 14x14 and 7x7 layers of a ResNet-18-shaped stack at batch 8); below that the gather kernel's finer waves win.
-    if (!forced && 8 * wgs < (uint64_t)ctx->compute_units) return SO_OK;
-    if (!window_shares(a, grid)) return SO_OK;
-    if (px == 2u) {
+    if (!forced && 8 * wgs < (uint64_t)ctx->compute_units) return false;
+    return window_shares(a, grid);
+}
+
+// Launches the windowed kernel where it applies; *done says whether it did.
+template <uint32_t LPP>
+so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
+                        const float *dResid, float *dY, int act, bool forced, bool *done)
+{
+    const so_conv_window &w = plan->win;
+    WinArgs a;
+    dim3 grid;
+    size_t lds;
+    if (!window_arguments<LPP>(ctx, plan, B, forced, a, grid, lds)) return SO_OK;
+    if (LPP == 4 && w.px == 2u) {
         if constexpr (LPP == 4) {
             if (w.cpw == 4) window_launch_act<4, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
             else window_launch_act<2, 4, 2>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act);
@@ -702,6 +745,51 @@ so_status window_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, 
     case 2:  window_launch_act<2, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
     default: window_launch_act<1, (int)LPP, 1>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY, act); break;
     }
+    ctx->waits_pending = true;
+    *done = true;
+    return SO_OK;
+}
+
+// Both convolutions of one input in one launch, where the same form of the kernel would take each.  A compute unit holds one workgroup of this kernel whatever
+// its window, so the second's fill the units that the first's leave and follow where those end: never later than after a launch of their own.  Us, ResNet-18-shaped
+// stacks, one after the other / together: 224x224 of width 64 at batch 32 34.5 + 12.2 / 42.3, 34.3 + 11.7 / 43.0, 48.5 + 13.0 / 59.0, at 8 15.0 + 6.8 / 20.1;
+// 96x96 of 48 at 32 13.1 + 6.1 / 17.7; 64x64 of 32 at 4 6.9 + 4.3 / 6.8.
+template <uint32_t LPP>
+so_status window_launch_pair(so_ctx *ctx, const so_conv_call (&call)[2], const float *dX, uint32_t B, bool forced, bool *done)
+{
+    WinPair p;
+    dim3 grid[2];
+    size_t lds[2];
+    const uint32_t px = LPP == 4 ? call[0].plan->win.px : 1u;
+    const int cpw = call[0].plan->win.cpw;
+    if (call[1].plan->win.cpw != cpw || (LPP == 4 && call[1].plan->win.px != px)) return SO_OK;
+    for (int i = 0; i < 2; ++i) {
+        const so_conv_window &w = call[i].plan->win;
+        WinCall &c = p.call[i];
+        if (!window_arguments<LPP>(ctx, call[i].plan, B, forced, c.a, grid[i], lds[i]) || c.a.per_xcd == 0u) return SO_OK;
+        c.stream = reinterpret_cast<const int4 *>(w.d_stream); c.gbase = w.d_gbase; c.quads = w.d_quads;
+        c.g = call[i].plan->g;
+        c.X = dX; c.bias = call[i].dBias; c.resid = nullptr; c.Y = call[i].dY; c.B = B;
+        c.relu = call[i].act == SO_ACT_RELU;
+    }
+    p.wgs0 = 8u * p.call[0].a.per_xcd;
+    const uint64_t wgs = (uint64_t)p.wgs0 + 8u * p.call[1].a.per_xcd;
+    if (wgs >= kWinMaxGrid) return SO_OK;
+    const size_t most = std::max(lds[0], lds[1]);
+#define SO_WIN_PAIR(CPW, PX) conv2d_window_pair_kernel<CPW, (int)LPP, PX><<<(uint32_t)wgs, kWinThreads, most, ctx->stream>>>(p)
+    if (px == 2u) {
+        if constexpr (LPP == 4) {
+            if (cpw == 4) SO_WIN_PAIR(4, 2);
+            else SO_WIN_PAIR(2, 2);
+        }
+    } else
+    switch (cpw) {
+    case 8:  SO_WIN_PAIR(8, 1); break;
+    case 4:  SO_WIN_PAIR(4, 1); break;
+    case 2:  SO_WIN_PAIR(2, 1); break;
+    default: SO_WIN_PAIR(1, 1); break;
+    }
+#undef SO_WIN_PAIR
     ctx->waits_pending = true;
     *done = true;
     return SO_OK;
@@ -1063,75 +1151,85 @@ bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, 
     return columns_us < 0.95 * (1.7 + rounds * (1.6 + 1.18 * w.nch + (B == 8 ? 0.0435 : 0.059) * row * std::max(0.35, waves / 16.0)));
 }
 
-static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,
-                                 const float *dBias, const float *dResid, float *dY, int act)
+// The kernels that a launch tries, in this order, before the gather kernel.
+struct ConvWays {
+    bool columns, merged, window, forced;        // forced: the windowed one whatever its grid
+    uint32_t lpp;
+};
+
+static ConvWays conv_ways(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, uintptr_t align)
 {
-    SO_REQUIRE(ctx && plan, "so_conv2d: null argument");
-    SO_REQUIRE(act >= SO_ACT_NONE && act <= SO_ACT_TANH, "so_conv2d: unknown activation %d", act);
     const so_conv_geom &g = plan->g;
-    const uint64_t ncols = (uint64_t)g.H_out * g.W_out * B;
-    if (g.Cout == 0 || ncols == 0) return SO_OK;
-    SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
-    SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
-    const uintptr_t align = (uintptr_t)dX | (uintptr_t)dY | (uintptr_t)dResid;
+    ConvWays way{false, false, false, ctx->tune.conv_window == 1, window_lpp(B)};
     // The kernels on an LDS window when the plan carries its layout and the batch splits into tiles of 16, 8 or 4.
-    const uint32_t lpp = window_lpp(B);
-    const bool windowed = plan->win.cc != 0 && lpp != 0 && (align & 15) == 0 && (uint64_t)plan->win.cc * g.H_in * g.W_in * B < (1ull << 31);
+    const bool windowed = plan->win.cc != 0 && way.lpp != 0 && (align & 15) == 0 && (uint64_t)plan->win.cc * g.H_in * g.W_in * B < (1ull << 31);
     // The row-block-merged one of them where the plan has been given its format, which is the request for it: SPARSEOPS_CONV_RBM=0 forbids it,
     // and so does an override for or against the per-row one, unless SPARSEOPS_CONV_RBM=1 asks.
-    const bool merged = windowed && plan->rbm.d_sets && (ctx->tune.conv_rbm == 1 || (ctx->tune.conv_rbm < 0 && ctx->tune.conv_window < 0));
+    way.merged = windowed && plan->rbm.d_sets && (ctx->tune.conv_rbm == 1 || (ctx->tune.conv_rbm < 0 && ctx->tune.conv_window < 0));
+    // the per-row one: SPARSEOPS_CONV_WINDOW=1 forces it whenever possible, =0 forbids it (tuning and tests)
+    way.window = windowed && ctx->tune.conv_window != 0;
     // The column kernel where the plan has its streams for this batch: below four entries, which the windowed kernel does
     // not take, where it pays against the gather kernel (so_conv_columns_pays), from four on against the windowed one
     // (so_conv_columns_before_window).  SPARSEOPS_CONV_COLUMNS=0 forbids it, =1 forces it.
     if (so_conv_columns_for(plan, B) && ctx->tune.conv_columns != 0) {
         const bool alone = B < 4 || (B == 4 && plan->win.cc == 0);           // no windowed kernel: else the gather kernel
-        bool use = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
-        if (!use && !alone && !merged && ctx->tune.conv_window != 1)
-            use = so_conv_columns_before_window(ctx, plan, B, so_conv_columns_estimate(ctx, plan, B));
-        if (use && ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) use = false;      // another kernel is asked for
-        bool done = false;
-        const so_status s = use ? so_conv_columns_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done) : SO_OK;
-        if (s != SO_OK) return s;
-        if (done) {
-            SO_LAUNCH_CHECK();
-            ctx->last_kernel = "columns";
-            return SO_OK;
-        }
+        way.columns = ctx->tune.conv_columns == 1 || (alone && so_conv_columns_pays(ctx, plan, B));
+        if (!way.columns && !alone && !way.merged && ctx->tune.conv_window != 1)
+            way.columns = so_conv_columns_before_window(ctx, plan, B, so_conv_columns_estimate(ctx, plan, B));
+        if (ctx->tune.conv_window == 1 && ctx->tune.conv_columns != 1) way.columns = false;      // another kernel is asked for
     }
-    // Batch entries per lane: as many as divide B and keep 16/8-byte alignment.
-    int maxvec = 4;
-    if (ctx->tune.conv_vec > 0) maxvec = ctx->tune.conv_vec;
-    if (windowed) {
-        if (merged) {
-            bool done = false;
-            const so_status s = so_conv_rbm_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done);
-            if (s != SO_OK) return s;
-            if (done) {
-                SO_LAUNCH_CHECK();
-                ctx->last_kernel = "merged-window";
-                return SO_OK;
-            }
-        }
-        // the per-row one: SPARSEOPS_CONV_WINDOW=1 forces it whenever possible, =0 forbids it (tuning and tests)
-        const bool forced = ctx->tune.conv_window == 1;
-        if (ctx->tune.conv_window != 0) {
-            bool done = false;
-            const so_status s = lpp == 4 ? window_launch<4>(ctx, plan, dX, B, dBias, dResid, dY, act, forced, &done)
-                              : lpp == 2 ? window_launch<2>(ctx, plan, dX, B, dBias, dResid, dY, act, forced, &done)
-                                         : window_launch<1>(ctx, plan, dX, B, dBias, dResid, dY, act, forced, &done);
-            if (s != SO_OK) return s;
-            if (done) {
-                SO_LAUNCH_CHECK();
-                ctx->last_kernel = "window";
-                return SO_OK;
-            }
-        }
+    return way;
+}
+
+// SO_OK with `empty` set where there is nothing to compute.
+static so_status conv2d_check(const so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dY, int act, bool &empty)
+{
+    SO_REQUIRE(ctx && plan, "so_conv2d: null argument");
+    SO_REQUIRE(act >= SO_ACT_NONE && act <= SO_ACT_TANH, "so_conv2d: unknown activation %d", act);
+    const uint64_t ncols = (uint64_t)plan->g.H_out * plan->g.W_out * B;
+    empty = plan->g.Cout == 0 || ncols == 0;
+    if (empty) return SO_OK;
+    SO_REQUIRE(dX && dY, "so_conv2d: null tensor");
+    SO_REQUIRE((ncols + 63) / 64 < (1ull << 31), "so_conv2d: output plane too large");
+    return SO_OK;
+}
+
+static so_status conv2d_dispatch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B,
+                                 const float *dBias, const float *dResid, float *dY, int act)
+{
+    bool empty;
+    so_status s = conv2d_check(ctx, plan, dX, B, dY, act, empty);
+    if (s != SO_OK || empty) return s;
+    const uint64_t ncols = (uint64_t)plan->g.H_out * plan->g.W_out * B;
+    const uintptr_t align = (uintptr_t)dX | (uintptr_t)dY | (uintptr_t)dResid;
+    const ConvWays way = conv_ways(ctx, plan, B, align);
+    const char *kernel = "gather";
+    bool done = false;
+    if (way.columns) {
+        kernel = "columns";
+        s = so_conv_columns_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done);
     }
-    if (maxvec >= 4 && B % 4 == 0 && (align & 15) == 0) conv_launch<4>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
-    else if (maxvec >= 2 && B % 2 == 0 && (align & 7) == 0) conv_launch<2>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
-    else conv_launch<1>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
+    if (s == SO_OK && !done && way.merged) {
+        kernel = "merged-window";
+        s = so_conv_rbm_launch(ctx, plan, dX, B, dBias, dResid, dY, act, &done);
+    }
+    if (s == SO_OK && !done && way.window) {
+        kernel = "window";
+        s = way.lpp == 4 ? window_launch<4>(ctx, plan, dX, B, dBias, dResid, dY, act, way.forced, &done)
+          : way.lpp == 2 ? window_launch<2>(ctx, plan, dX, B, dBias, dResid, dY, act, way.forced, &done)
+                         : window_launch<1>(ctx, plan, dX, B, dBias, dResid, dY, act, way.forced, &done);
+    }
+    if (s != SO_OK) return s;
+    if (!done) {
+        // Batch entries per lane: as many as divide B and keep 16/8-byte alignment.
+        kernel = "gather";
+        const int maxvec = ctx->tune.conv_vec > 0 ? ctx->tune.conv_vec : 4;
+        if (maxvec >= 4 && B % 4 == 0 && (align & 15) == 0) conv_launch<4>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
+        else if (maxvec >= 2 && B % 2 == 0 && (align & 7) == 0) conv_launch<2>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
+        else conv_launch<1>(ctx, plan, dX, B, ncols, dBias, dResid, dY, act);
+    }
     SO_LAUNCH_CHECK();
-    ctx->last_kernel = "gather";
+    ctx->last_kernel = kernel;
     return SO_OK;
 }
 
@@ -1147,4 +1245,44 @@ extern "C" so_status so_conv2d_add(so_ctx *ctx, const so_conv_plan *plan, const 
     SO_REQUIRE(dResidual, "so_conv2d_add: null residual");
     SO_REQUIRE(dResidual != dY, "so_conv2d_add: the residual must not alias the output");
     return conv2d_dispatch(ctx, plan, dX, B, dBias, dResidual, dY, act);
+}
+
+extern "C" so_status so_conv2d_pair(so_ctx *ctx, const so_conv_plan *planA, const so_conv_plan *planB, const float *dX, uint32_t B,
+                                    const float *dBiasA, float *dYA, int actA, const float *dBiasB, float *dYB, int actB)
+{
+    const so_conv_call call[2] = {{planA, dBiasA, dYA, actA}, {planB, dBiasB, dYB, actB}};
+    bool empty[2];
+    for (int i = 0; i < 2; ++i) {
+        const so_status s = conv2d_check(ctx, call[i].plan, dX, B, call[i].dY, call[i].act, empty[i]);
+        if (s != SO_OK) return s;
+    }
+    const so_conv_geom &ga = planA->g, &gb = planB->g;
+    SO_REQUIRE(ga.Cin == gb.Cin && ga.H_in == gb.H_in && ga.W_in == gb.W_in, "so_conv2d_pair: the plans' inputs differ");
+    if (!empty[0] && !empty[1]) {
+        struct Range { uintptr_t from, to; };
+        const auto range = [](const void *p, uint64_t floats) { return Range{(uintptr_t)p, (uintptr_t)p + floats * 4}; };
+        const Range x = range(dX, (uint64_t)ga.Cin * ga.H_in * ga.W_in * B), ya = range(dYA, (uint64_t)ga.Cout * ga.H_out * ga.W_out * B),
+                    yb = range(dYB, (uint64_t)gb.Cout * gb.H_out * gb.W_out * B);
+        const auto apart = [](Range p, Range q) { return p.to <= q.from || q.to <= p.from; };
+        SO_REQUIRE(apart(x, ya) && apart(x, yb) && apart(ya, yb), "so_conv2d_pair: the input and the outputs must not overlap");
+        const auto none_or_relu = [](int act) { return act == SO_ACT_NONE || act == SO_ACT_RELU; };
+        if (none_or_relu(actA) && none_or_relu(actB)) {
+            const ConvWays a = conv_ways(ctx, planA, B, (uintptr_t)dX | (uintptr_t)dYA), b = conv_ways(ctx, planB, B, (uintptr_t)dX | (uintptr_t)dYB);
+            bool done = false;
+            so_status s = SO_OK;
+            if (a.columns && b.columns) s = so_conv_columns_launch_pair(ctx, call, dX, B, &done);
+            else if (!a.columns && !b.columns && !a.merged && !b.merged && a.window && b.window)
+                s = a.lpp == 4 ? window_launch_pair<4>(ctx, call, dX, B, a.forced, &done)
+                  : a.lpp == 2 ? window_launch_pair<2>(ctx, call, dX, B, a.forced, &done)
+                               : window_launch_pair<1>(ctx, call, dX, B, a.forced, &done);
+            if (s != SO_OK) return s;
+            if (done) {
+                SO_LAUNCH_CHECK();
+                ctx->last_kernel = a.columns ? "columns-pair" : "window-pair";
+                return SO_OK;
+            }
+        }
+    }
+    const so_status s = conv2d_dispatch(ctx, planA, dX, B, dBiasA, nullptr, dYA, actA);
+    return s != SO_OK ? s : conv2d_dispatch(ctx, planB, dX, B, dBiasB, nullptr, dYB, actB);
 }

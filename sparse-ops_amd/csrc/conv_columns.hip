@@ -56,19 +56,29 @@ __device__ __forceinline__ void rest(uint32_t left, F &&step)
     }
 }
 
+// One convolution's operands.
+struct ColCall {
+    const int2 *entries;
+    const uint32_t *first_group;
+    const float *bias;
+    float *Y;
+    ColArgs a;
+    so_conv_geom g;
+    uint32_t relu;               // kActNoneOrRelu
+};
+
 template <int ACT>
-__global__ __launch_bounds__(1024)
-void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__restrict__ first_group, ColArgs a, so_conv_geom g,
-                          const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
-                          const float *__restrict__ resid, float *__restrict__ Y)
+__device__ __forceinline__ void column_convolution(const int2 *__restrict__ entries, const uint32_t *__restrict__ first_group, const ColArgs &a, const so_conv_geom &g,
+                                                   const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
+                                                   const float *__restrict__ resid, float *__restrict__ Y, uint32_t tile, uint32_t block, bool relu)
 {
     extern __shared__ __attribute__((aligned(16))) float window[];     // [cc + 1][PL]: the last plane all zeros (padding entries point there)
     const uint32_t tid = threadIdx.x, lane = tid & 63u, threads = a.waves * 64u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t co = blockIdx.y * a.G + wave;
+    const uint32_t co = block * a.G + wave;
     const bool computes = wave < a.G && co < g.Cout;                   // the other waves only help copying
-    const uint32_t tile_y = window_div(blockIdx.x, a.tiles_x, a.mTilesX);
-    const uint32_t th0 = tile_y * a.TH, tw0 = (blockIdx.x - tile_y * a.tiles_x) * a.TW;
+    const uint32_t tile_y = window_div(tile, a.tiles_x, a.mTilesX);
+    const uint32_t th0 = tile_y * a.TH, tw0 = (tile - tile_y * a.tiles_x) * a.TW;
 
     // The wave's entries, groups of 16 (the stream ends with kAhead padding groups).  At a pitch their place needs no look
     // into a table, whose round trip to memory -- nothing is cached when a kernel starts -- would come before theirs.
@@ -76,13 +86,14 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
     const uint32_t l16 = lane & 15u;
     int2 held[kAhead];
     uint32_t g0, g1;
+    const so_constant<uint32_t> first = (so_constant<uint32_t>)(uintptr_t)first_group;
     auto first_entries = [&](uint32_t t) {
         if (a.pitch != 0u) {
             g0 = (run0 + t) * a.pitch;
-            g1 = g0 + __builtin_amdgcn_readfirstlane(first_group[run0 + t]);
+            g1 = g0 + __builtin_amdgcn_readfirstlane(first[run0 + t]);
         } else {
-            g0 = __builtin_amdgcn_readfirstlane(first_group[run0 + t]);
-            g1 = __builtin_amdgcn_readfirstlane(first_group[run0 + t + 1u]);
+            g0 = __builtin_amdgcn_readfirstlane(first[run0 + t]);
+            g1 = __builtin_amdgcn_readfirstlane(first[run0 + t + 1u]);
         }
         if (!computes) g1 = g0;
 #pragma unroll
@@ -95,7 +106,7 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
     const uint32_t ty = window_div(pix, a.TW, a.mTW), tx = pix - ty * a.TW;
     const bool live = computes && pix < a.TH * a.TW && th0 + ty < g.H_out && tw0 + tx < g.W_out;
     const uint32_t lane_off = live ? ((ty * a.sth * a.IP + tx * a.stw) * B + b) * 4u : 0u;
-    float acc = bias && computes ? bias[co] : 0.0f;
+    float acc = bias && computes ? ((so_constant<float>)(uintptr_t)bias)[co] : 0.0f;
 
     for (uint32_t k = tid; k < a.PL; k += threads) window[a.cc * a.PL + k] = 0.0f;
     // Input channels [t * cc, t * cc + cc) of the window, straight from memory into LDS: consecutive threads take
@@ -174,8 +185,34 @@ void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__re
     if (live) {
         const size_t at = (((size_t)co * g.H_out + th0 + ty) * g.W_out + tw0 + tx) * B + b;
         if (resid) acc += resid[at];
-        Y[at] = so_epilogue<ACT>(acc);
+        Y[at] = conv_epilogue<ACT>(acc, relu);
     }
+}
+
+template <int ACT>
+__global__ __launch_bounds__(1024)
+void conv2d_column_kernel(const int2 *__restrict__ entries, const uint32_t *__restrict__ first_group, ColArgs a, so_conv_geom g,
+                          const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
+                          const float *__restrict__ resid, float *__restrict__ Y)
+{
+    column_convolution<ACT>(entries, first_group, a, g, X, B, bias, resid, Y, blockIdx.x, blockIdx.y, false);
+}
+
+// Two convolutions of one input: the first's workgroups, then the second's.  Both read their operands from the arguments at a place that
+// depends on which it is.
+struct ColPair {
+    ColCall call[2];
+    const float *X;
+    uint32_t B, wgs0, tiles[2], mTiles[2];
+};
+__global__ __launch_bounds__(1024)
+void conv2d_column_pair_kernel(ColPair)
+{
+    const ColPair &p = *(const ColPair *)__builtin_amdgcn_kernarg_segment_ptr();
+    const uint32_t which = blockIdx.x >= p.wgs0 ? 1u : 0u, id = blockIdx.x - (which ? p.wgs0 : 0u);
+    const ColCall &c = p.call[which];
+    const uint32_t tiles = p.tiles[which], block = window_div(id, tiles, p.mTiles[which]);
+    column_convolution<kActNoneOrRelu>(c.entries, c.first_group, c.a, c.g, p.X, p.B, c.bias, nullptr, c.Y, id - block * tiles, block, c.relu != 0u);
 }
 
 template <int ACT>
@@ -199,26 +236,30 @@ struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 // LDS, 0.44 us and 24 ns per KB, 9 more for every further workgroup on the compute unit; 0.5 us for each of those, 2.2 for every further filling of the
 // chip; chains at 8.3 ns an entry, 5.9 per wave.  Fitted on 500 layers of up to 128x128 and 512 channels at batches of 8, 16 and 32: half are
 // within 7 %.
-ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
+ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c, uint32_t G)
 {
     const double cus = ctx->compute_units, chain = (double)plan->E->total_nnz / plan->g.Cout + 8.0, tiles = (double)c.tiles_x * c.tiles_y;
-    ColShape best{16, 16, 0, 1e30, 1.0};
-    for (uint32_t G = 16; G >= 4; G /= 2) {
-        ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0, 0.0};
-        s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
-        const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
-        const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
-        const double resident = std::min(fit, std::ceil(wgs / cus));
-        s.rounds = std::ceil(wgs / (cus * fit));
-        if (c.batch <= 4) {
-            s.us = 3.0 + s.rounds * (2.5 + c.nch + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
-        } else {
-            const double start = c.nch * (0.44 + 0.024 * s.lds / 1024.0 * (1.0 + 0.38 * (resident - 1.0))), waves = std::min(G, plan->g.Cout);
-            s.us = 2.75 + s.rounds * (start + chain * std::max(0.0083, 0.0059 * std::max(1.0, resident * waves / 4.0))) +
-                   2.2 * std::max(0.0, wgs / (cus * fit) - 1.0) + 0.5 * (resident - 1.0);
-        }
-        if (s.us < best.us) best = s;
+    ColShape s{G, 0, (size_t)(c.cc + 1) * c.PE * c.batch * 4, 0.0, 0.0};
+    s.waves = s.lds >= 48 * 1024 ? 16u : std::max(G, 8u);
+    const double wgs = tiles * so_ceil_div(plan->g.Cout, G);
+    const double fit = std::max<double>(1.0, std::min<double>(160 * 1024 / s.lds, 32 / s.waves));
+    const double resident = std::min(fit, std::ceil(wgs / cus));
+    s.rounds = std::ceil(wgs / (cus * fit));
+    if (c.batch <= 4) {
+        s.us = 3.0 + s.rounds * (2.5 + c.nch + chain * std::max(0.010, 0.0075 * std::max(1.0, resident * G / 4.0)));
+    } else {
+        const double start = c.nch * (0.44 + 0.024 * s.lds / 1024.0 * (1.0 + 0.38 * (resident - 1.0))), waves = std::min(G, plan->g.Cout);
+        s.us = 2.75 + s.rounds * (start + chain * std::max(0.0083, 0.0059 * std::max(1.0, resident * waves / 4.0))) +
+               2.2 * std::max(0.0, wgs / (cus * fit) - 1.0) + 0.5 * (resident - 1.0);
     }
+    return s;
+}
+
+ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv_columns &c)
+{
+    ColShape best{16, 16, 0, 1e30, 1.0};
+    for (uint32_t G = 16; G >= 4; G /= 2)
+        if (const ColShape s = column_shape(ctx, plan, c, G); s.us < best.us) best = s;
     return best;
 }
 
@@ -327,7 +368,7 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
     }
     if (!c.pitch) first.back() = (uint32_t)next;
     for (const void *k : {(const void *)conv2d_column_kernel<SO_ACT_NONE>, (const void *)conv2d_column_kernel<SO_ACT_RELU>,
-                          (const void *)conv2d_column_kernel<SO_ACT_SIGMOID>, (const void *)conv2d_column_kernel<SO_ACT_TANH>})
+                          (const void *)conv2d_column_kernel<SO_ACT_SIGMOID>, (const void *)conv2d_column_kernel<SO_ACT_TANH>, (const void *)conv2d_column_pair_kernel})
         SO_HIP(so_allow_big_lds(ctx, k));
     void *p = nullptr;
     so_status s = so_malloc(ctx, entries.size() * sizeof(int2), &p);
@@ -370,31 +411,87 @@ bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t 
 
 double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, *so_conv_columns_for(plan, B)).us; }
 
+// The arguments of a launch; false: the kernel does not take it.
+static bool columns_arguments(const so_conv_plan *plan, const so_conv_columns &c, const ColShape &shape, ColArgs &a, dim3 &grid)
+{
+    const so_conv_geom &g = plan->g;
+    const uint32_t B = c.batch;
+    a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch; a.pitch = c.pitch;
+    a.sth = window_step(g.kH, g.stride_h); a.stw = window_step(g.kW, g.stride_w);
+    a.sbh = window_subsample(g.kH, g.stride_h); a.sbw = window_subsample(g.kW, g.stride_w);
+    a.mB = window_magic(B); a.mIP = window_magic(a.IP); a.mPL = window_magic(a.PL); a.mTW = window_magic(a.TW); a.mTilesX = window_magic(a.tiles_x);
+    a.G = shape.G;
+    a.waves = shape.waves;
+    grid = dim3(c.tiles_x * c.tiles_y, so_ceil_div(g.Cout, a.G));
+    return grid.y <= 65535u;
+}
+
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done)
 {
     *done = false;
     if (!so_conv_columns_for(plan, B)) return SO_OK;
     const so_conv_columns &c = *so_conv_columns_for(plan, B);
-    const so_conv_geom &g = plan->g;
-    ColArgs a;
-    a.TH = c.TH; a.TW = c.TW; a.tiles_x = c.tiles_x; a.PE = c.PE; a.IP = c.IP; a.PL = c.PE * B; a.cc = c.cc; a.nch = c.nch; a.pitch = c.pitch;
-    a.sth = window_step(g.kH, g.stride_h); a.stw = window_step(g.kW, g.stride_w);
-    a.sbh = window_subsample(g.kH, g.stride_h); a.sbw = window_subsample(g.kW, g.stride_w);
-    a.mB = window_magic(B); a.mIP = window_magic(a.IP); a.mPL = window_magic(a.PL); a.mTW = window_magic(a.TW); a.mTilesX = window_magic(a.tiles_x);
-    const uint64_t tiles = (uint64_t)c.tiles_x * c.tiles_y;
     const ColShape shape = column_shape(ctx, plan, c);
-    a.G = shape.G;
-    a.waves = shape.waves;
     const size_t lds = shape.lds;
-    const dim3 grid((uint32_t)tiles, so_ceil_div(g.Cout, a.G));
-    if (grid.y > 65535u) return SO_OK;
+    ColArgs a;
+    dim3 grid;
+    if (!columns_arguments(plan, c, shape, a, grid)) return SO_OK;
+    *done = true;
     switch (act) {
     case SO_ACT_RELU:    launch_columns<SO_ACT_RELU>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
     case SO_ACT_SIGMOID: launch_columns<SO_ACT_SIGMOID>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
     case SO_ACT_TANH:    launch_columns<SO_ACT_TANH>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
     default:             launch_columns<SO_ACT_NONE>(ctx, plan, a, grid, lds, dX, B, dBias, dResid, dY); break;
     }
+    return SO_OK;
+}
+
+// A launch of its own for a residual block's projection is mostly start-up.  Here its workgroups run beside the first convolution's where the sizes that are
+// chosen for both let all be resident at once -- the longer of the two is the time -- and behind them otherwise, where each alone is one filling of the chip at
+// the occupancy that the larger window leaves: then a launch's gap is saved.  Us, ResNet-18-shaped stacks, one after the other / together: 224x224 of width 64
+// at batch 1 8.3 + 4.4 / 9.4, 10.6 + 5.1 / 14.1, 16.2 + 5.5 / 16.6, at 8 (into 7x7) 31.2 + 7.1 / 34.6; 96x96 of 64 at 8 12.3 + 5.1 / 12.8,
+// 13.4 + 5.1 / 14.0, 17.6 + 5.9 / 22.7.
+so_status so_conv_columns_launch_pair(so_ctx *ctx, const so_conv_call (&call)[2], const float *dX, uint32_t B, bool *done)
+{
+    *done = false;
+    const so_conv_columns *const c[2] = {so_conv_columns_for(call[0].plan, B), so_conv_columns_for(call[1].plan, B)};
+    if (!c[0] || !c[1]) return SO_OK;
+    double best = column_shape(ctx, call[0].plan, *c[0]).us + column_shape(ctx, call[1].plan, *c[1]).us;
+    ColPair p;
+    uint32_t wgs = 0, waves = 0;
+    size_t lds = 0;
+    for (uint32_t G0 = 16; G0 >= 4; G0 /= 2)
+        for (uint32_t G1 = 16; G1 >= 4; G1 /= 2) {
+            const ColShape s[2] = {column_shape(ctx, call[0].plan, *c[0], G0), column_shape(ctx, call[1].plan, *c[1], G1)};
+            ColArgs a[2];
+            dim3 grid[2];
+            if (!columns_arguments(call[0].plan, *c[0], s[0], a[0], grid[0]) || !columns_arguments(call[1].plan, *c[1], s[1], a[1], grid[1])) continue;
+            const size_t most = std::max(s[0].lds, s[1].lds);
+            const uint32_t w = std::max(s[0].waves, s[1].waves);
+            const uint64_t one = (uint64_t)grid[0].x * grid[0].y, two = (uint64_t)grid[1].x * grid[1].y, all = one + two;
+            const uint64_t resident = (uint64_t)ctx->compute_units * std::max<uint64_t>(1, std::min<uint64_t>(160 * 1024 / most, 32 / w));
+            if (one > resident || two > resident) continue;
+            const double us = all <= resident ? std::max(s[0].us, s[1].us) : s[0].us + s[1].us - 2.0;
+            if (us >= best) continue;
+            best = us; wgs = (uint32_t)all; waves = w; lds = most;
+            p.wgs0 = grid[0].x * grid[0].y;
+            for (int i = 0; i < 2; ++i) {
+                a[i].waves = w;
+                p.call[i].a = a[i];
+                p.tiles[i] = grid[i].x; p.mTiles[i] = window_magic(grid[i].x);
+            }
+        }
+    if (!wgs) return SO_OK;
+    for (int i = 0; i < 2; ++i) {
+        ColCall &o = p.call[i];
+        o.entries = c[i]->d_entries; o.first_group = c[i]->d_first;
+        o.bias = call[i].dBias; o.Y = call[i].dY;
+        o.g = call[i].plan->g;
+        o.relu = call[i].act == SO_ACT_RELU;
+    }
+    p.X = dX; p.B = B;
+    conv2d_column_pair_kernel<<<wgs, waves * 64u, lds, ctx->stream>>>(p);
     *done = true;
     return SO_OK;
 }

@@ -61,6 +61,26 @@ struct so_conv_plan {
     bool col_tried[kColSlots] = {};      // they have been made, or could not be
 };
 
+// Memory that nothing writes while a kernel runs, read by scalar loads also where the compiler does not see that by itself: behind inline assembly,
+// through pointers that are not themselves the kernel's arguments.
+template <class T> using so_constant = const __attribute__((address_space(4))) T *;
+
+// One of the two convolutions of a so_conv2d_pair launch: what so_conv2d is given.
+struct so_conv_call {
+    const so_conv_plan *plan;
+    const float *dBias;
+    float *dY;
+    int act;
+};
+// The pair kernels choose between the two activations that follow most convolutions when they run.
+constexpr int kActNoneOrRelu = -1;
+template <int ACT>
+__device__ __forceinline__ float conv_epilogue(float v, bool relu)
+{
+    if constexpr (ACT == kActNoneOrRelu) return relu ? so_epilogue<SO_ACT_RELU>(v) : v;
+    else return so_epilogue<ACT>(v);
+}
+
 // conv_columns.hip
 void so_conv_columns_free(so_conv_plan *plan);
 bool so_conv_columns_wanted(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B);          // streams for the batch pay
@@ -72,6 +92,8 @@ double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uin
 bool so_conv_columns_before_window(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B, double columns_us);   // conv.hip
 so_status so_conv_columns_launch(so_ctx *ctx, const so_conv_plan *plan, const float *dX, uint32_t B, const float *dBias,
                                  const float *dResid, float *dY, int act, bool *done);
+// Both of one input in one launch, where one is taken.
+so_status so_conv_columns_launch_pair(so_ctx *ctx, const so_conv_call (&call)[2], const float *dX, uint32_t B, bool *done);
 
 // conv_rbm.hip
 void so_conv_rbm_release(so_conv_plan *plan);
@@ -140,13 +162,13 @@ inline bool window_shares(WinArgs &a, dim3 grid)
     return true;
 }
 inline dim3 window_grid(const WinArgs &a, dim3 grid) { return a.per_xcd != 0u ? dim3(8u * a.per_xcd) : grid; }
-__device__ __forceinline__ bool window_workgroup(const WinArgs &a, WinPlace &p)
+__device__ __forceinline__ bool window_workgroup(const WinArgs &a, uint32_t wg, WinPlace &p)
 {
     if (__builtin_expect(a.per_xcd == 0u, 0)) {
         p.tile = blockIdx.x; p.y = blockIdx.y; p.z = blockIdx.z;
         return true;
     }
-    const uint32_t id = (blockIdx.x & 7u) * a.per_xcd + (blockIdx.x >> 3);
+    const uint32_t id = (wg & 7u) * a.per_xcd + (wg >> 3);
     p.tile = __umulhi(id, a.mYZ) + (id & a.oneYZ);
     const uint32_t rest = id - p.tile * a.yz;
     p.y = __umulhi(rest, a.mZ) + (rest & a.oneZ);

@@ -238,7 +238,7 @@ void conv2d_rbm_kernel(const int4 *__restrict__ sets, const uint32_t *__restrict
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t cgi = window_div(wave, a.pg, a.mPg), pgi = wave - cgi * a.pg;
     WinPlace place;
-    if (!window_workgroup(a, place)) return;
+    if (!window_workgroup(a, blockIdx.x, place)) return;
     const uint32_t tile_y = window_div(place.tile, a.tiles_x, a.mTilesX);
     const uint32_t th0 = tile_y * a.TH, tw0 = (place.tile - tile_y * a.tiles_x) * a.TW;
     const uint32_t grp = place.y * a.cg + cgi;                       // block of output channels of this wave

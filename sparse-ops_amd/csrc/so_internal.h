@@ -340,6 +340,7 @@ static inline uint32_t so_ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((
 template <int ACT>
 __device__ __forceinline__ float so_epilogue(float v)
 {
+    static_assert(ACT >= SO_ACT_NONE && ACT <= SO_ACT_TANH, "an activation");
     if (ACT == SO_ACT_RELU) return v > 0.0f ? v : 0.0f;
     if (ACT == SO_ACT_SIGMOID) return 1.0f / (1.0f + expf(-v));
     if (ACT == SO_ACT_TANH) return tanhf(v);

@@ -20,7 +20,7 @@ LAYOUT_ROW, LAYOUT_SLOT, LAYOUT_BINS, LAYOUT_TILED, LAYOUT_RBM, LAYOUT_IDX16 = 1
 SYMBOLS = (
     "so_device_count so_init so_destroy so_last_error so_device_info so_tuning_reload so_malloc so_free so_h2d so_d2h "
     "so_stage_in so_stage_out so_stage_in_transposed so_stage_out_transposed so_d2d so_fill_zero so_sync so_timer_begin so_timer_end so_ellpack_upload so_ellpack_free "
-    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_matvec_to_host so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add "
+    "so_ellpack_dims so_ellpack_download so_ellpack_decode so_ellpack_encode so_ellpack_encode_noalloc so_matmul so_matmul_reserve so_last_kernel so_matvec so_matvec_to_host so_conv_plan_create so_conv_plan_free so_conv_plan_window so_conv_plan_tune so_conv2d_add so_conv2d_pair "
     "so_conv2d so_maxpool so_gap so_add so_act so_transpose so_reverse_axes3 so_copy_rows so_graph_begin so_graph_end "
     "so_graph_launch so_graph_free so_rbm_upload so_rbm_free so_rbm_dims so_conv_plan_set_rbm so_conv_plan_rbm_info").split()
 
@@ -94,6 +94,7 @@ def load_library(path=None):
         "so_conv_plan_tune": [_vp, _vp, ct.c_uint32],
         "so_conv2d": [_vp, _vp, _vp, _u32, _vp, _vp, ct.c_int],
         "so_conv2d_add": [_vp, _vp, _vp, ct.c_uint32, _vp, _vp, _vp, ct.c_int],
+        "so_conv2d_pair": [_vp, _vp, _vp, _vp, _u32, _vp, _vp, ct.c_int, _vp, _vp, ct.c_int],
         "so_maxpool": [_vp, ct.POINTER(PoolGeom), _vp, _u32, _vp],
         "so_gap": [_vp, _u32, _u32, _u32, _vp, _u32, _vp],
         "so_add": [_vp, _vp, _vp, ct.c_size_t, _vp],
@@ -354,6 +355,10 @@ class Context:
             self._ck(self.lib.so_conv2d(self.h, plan, dX.ptr, B, dBias.ptr if dBias else None, dY.ptr, ACT[act]))
         else:
             self._ck(self.lib.so_conv2d_add(self.h, plan, dX.ptr, B, dBias.ptr if dBias else None, residual.ptr, dY.ptr, ACT[act]))
+
+    def conv2d_pair(self, planA, planB, dX, B, dBiasA, dYA, actA, dBiasB, dYB, actB):
+        self._ck(self.lib.so_conv2d_pair(self.h, planA, planB, dX.ptr, B, dBiasA.ptr if dBiasA else None, dYA.ptr, ACT[actA],
+                                         dBiasB.ptr if dBiasB else None, dYB.ptr, ACT[actB]))
 
     def maxpool(self, C, H, W, k, s, pad, dX, B, dY):
         Ho = (H + 2 * pad[0] - k[0]) // s[0] + 1

@@ -108,6 +108,12 @@ void SparseOnnxModel::Impl::enqueue_layers(const float *in, float *out) const
     std::size_t at = 0;
     auto src = [&](int s) -> const float * { return in && s == input_slot ? in : out && at > made && s == output_slot ? out : slot_ptr(s); };
     auto dst = [&](int s) -> float * { return out && at == made ? out : slot_ptr(s); };
+    // A convolution and the next layer, another one of the same input; neither makes the model's output in the caller's memory unless it is the second.
+    const auto pairs = [&](std::size_t i) {
+        if (i + 1 >= layers.size()) return false;
+        const LayerPlan &L = layers[i], &N = layers[i + 1];
+        return L.conv && N.conv && !L.residual && !N.residual && L.in0 == N.in0 && L.out != N.out && L.out != L.in0 && N.out != L.in0 && !(out && i >= made);
+    };
     for (; at < layers.size(); ++at) {
         const LayerPlan &L = layers[at];
         const float *bias = L.has_bias ? bias_pool.f32() + L.bias_offset : nullptr;
@@ -116,7 +122,11 @@ void SparseOnnxModel::Impl::enqueue_layers(const float *in, float *out) const
             check(so_matmul(ctx, L.dE, src(L.in0), B, bias, dst(L.out), L.act), "so_matmul");
             break;
         case Op::Conv:
-            if (L.residual)
+            if (pairs(at)) {
+                const LayerPlan &N = layers[++at];
+                const float *bias2 = N.has_bias ? bias_pool.f32() + N.bias_offset : nullptr;
+                check(so_conv2d_pair(ctx, L.conv, N.conv, src(L.in0), B, bias, slot_ptr(L.out), L.act, bias2, dst(N.out), N.act), "so_conv2d_pair");
+            } else if (L.residual)
                 check(so_conv2d_add(ctx, L.conv, src(L.in0), B, bias, src(L.in1), dst(L.out), L.act), "so_conv2d_add");
             else
                 check(so_conv2d(ctx, L.conv, src(L.in0), B, bias, dst(L.out), L.act), "so_conv2d");

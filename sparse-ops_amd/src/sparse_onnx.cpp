@@ -407,6 +407,34 @@ SparseOnnxModel::SparseOnnxModel(const std::string &onnx_path) : impl_(new Impl(
         }
     }
 
+    // The projection of a block's skip connection, where the exporter put it behind the main branch and the Add has gone into it, moves up behind
+    // the first convolution of its input, with which it shares a launch (so_conv2d_pair); the Add and its activation go to the main branch's last
+    // convolution instead: the same two numbers added.
+    for (std::size_t j = 2; j < pend.size(); ++j) {
+        if (pend[j].plan.op != Op::Conv || !pend[j].plan.residual) continue;
+        const std::string input = pend[j].inputs[0], main = pend[j].inputs[1];
+        const auto readers = [&](const std::string &t) {
+            std::size_t n = t == M.output_name;
+            for (const auto &p : pend) n += std::size_t(std::count(p.inputs.begin(), p.inputs.end(), t));
+            return n;
+        };
+        std::size_t k = 0, i = 0;
+        while (k < j && pend[k].output != main) ++k;
+        const auto plain = [](const Pending &p) { return p.plan.op == Op::Conv && !p.plan.residual; };
+        while (i < k && !(plain(pend[i]) && pend[i].inputs[0] == input)) ++i;
+        if (k == j || i == k || !plain(pend[k]) || pend[k].plan.act != SO_ACT_NONE || readers(main) != 1) continue;
+        Pending &last = pend[k], &proj = pend[j];
+        last.plan.residual = true;
+        last.plan.act = proj.plan.act;
+        last.output = proj.output;
+        proj.plan.residual = false;
+        proj.plan.act = SO_ACT_NONE;
+        proj.output = main;
+        last.inputs.push_back(proj.output);
+        proj.inputs.pop_back();
+        std::rotate(pend.begin() + long(i) + 1, pend.begin() + long(j), pend.begin() + long(j) + 1);
+    }
+
     // Arena slots: a tensor keeps its slot until its last reader has been
     // enqueued; slots are then recycled, so the arena holds the live set only.
     {
