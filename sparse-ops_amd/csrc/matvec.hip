@@ -75,12 +75,31 @@ __device__ __forceinline__ void tell_host(const Tell &tell, const float *held, u
     }
 }
 
+// The sum over G lanes in all of them: pairs G / 2 apart, then G / 4 and so on, by lane moves inside the vector unit (six exchanges through LDS, one
+// after the other, at the end of a launch: 1000 x 1000 at 70 % sparse 4.00 us, so 3.75).  From 8 lanes on a rotation of the row of 16 is the exchange, since a value then
+// comes again every 2 * distance lanes.
+template <int CONTROL, int BANKS = 0xf>
+__device__ __forceinline__ float lanes_moved(float old, float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CONTROL, 0xf, BANKS, false));
+}
 template <int G>
 __device__ __forceinline__ float group_sum(float v)
 {
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, G);
-    return v;
+    constexpr int kRorBase = 0x120, kShl = 0x100, kShr = 0x110;          // row_ror:n, row_shl:n, row_shr:n
+    if constexpr (G >= 64) {
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    }
+    if constexpr (G >= 32) {
+        const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    }
+    if constexpr (G >= 16) v += lanes_moved<kRorBase + 8>(v, v);
+    if constexpr (G >= 16) v += lanes_moved<kRorBase + 4>(v, v);
+    else if constexpr (G == 8) v += lanes_moved<kShr + 4, 0xa>(lanes_moved<kShl + 4, 0x5>(v, v), v);
+    v += lanes_moved<0x4e>(v, v);                                        // quad_perm: [2, 3, 0, 1]
+    return v + lanes_moved<0xb1>(v, v);                                  // [1, 0, 3, 2]
 }
 
 // Stage x in LDS (XLDS) or read it through the cache hierarchy.  `pitch`: floats from one element of x to the next.
@@ -126,9 +145,9 @@ __device__ __forceinline__ void row_issue(const f32x4 *__restrict__ Wd4, const t
     }
 }
 
-template <int G, bool I16>
-__device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg, uint64_t end, uint64_t q0, const float *xs,
-                                            float &a0, float &a1, float &a2, float &a3, size_t pitch = 1)
+// a[j]: the four partial sums of column j of the W dense ones, which lie side by side in xs, `pitch` floats from one element to the next.
+template <int G, bool I16, int W>
+__device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg, uint64_t end, uint64_t q0, const float *xs, float (&a)[W][4], size_t pitch = W)
 {
     // slot k of group u is live iff its distance from the row's start is in [0, end - beg): one
     // unsigned 32-bit comparison (a slot before the row gives a huge distance)
@@ -137,15 +156,18 @@ __device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int32_t rel = rel0 + 4 * G * u;
-        const bool v0 = (uint32_t)rel < len, v1 = (uint32_t)(rel + 1) < len;
-        const bool v2 = (uint32_t)(rel + 2) < len, v3 = (uint32_t)(rel + 3) < len;
         const u32x4 c = ColGroup<I16>::cols(L.c[u]);
-        const float x0 = xs[(v0 ? c.x : 0u) * pitch], x1 = xs[(v1 ? c.y : 0u) * pitch];
-        const float x2 = xs[(v2 ? c.z : 0u) * pitch], x3 = xs[(v3 ? c.w : 0u) * pitch];
-        a0 = __builtin_fmaf(v0 ? L.w[u].x : 0.0f, v0 ? x0 : 0.0f, a0);
-        a1 = __builtin_fmaf(v1 ? L.w[u].y : 0.0f, v1 ? x1 : 0.0f, a1);
-        a2 = __builtin_fmaf(v2 ? L.w[u].z : 0.0f, v2 ? x2 : 0.0f, a2);
-        a3 = __builtin_fmaf(v3 ? L.w[u].w : 0.0f, v3 ? x3 : 0.0f, a3);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool v = (uint32_t)(rel + k) < len;
+            const float *xk = xs + (v ? c[k] : 0u) * pitch;
+            const float w = v ? L.w[u][k] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < W; ++j) {
+                const float x = xk[j];
+                a[j][k] = __builtin_fmaf(w, v ? x : 0.0f, a[j][k]);
+            }
+        }
     }
 }
 
@@ -154,15 +176,15 @@ template <bool I16>
 __device__ __forceinline__ float wave_row_dot(const f32x4 *__restrict__ Wd4, const typename ColGroup<I16>::T *__restrict__ idx4,
                                               uint64_t beg, uint64_t end, const float *xs, uint32_t lane)
 {
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+    float a[1][4] = {};
     if (end == beg) return 0.0f;
     const uint64_t qlast = (end - 1) >> 2;
     for (uint64_t q0 = (beg >> 2) + lane; q0 <= qlast; q0 += 256) {
         RowLoads<I16> L;
         row_issue<64, I16>(Wd4, idx4, beg, end, q0, L);
-        row_consume<64, I16>(L, beg, end, q0, xs, a0, a1, a2, a3);
+        row_consume<64, I16>(L, beg, end, q0, xs, a);
     }
-    return group_sum<64>((a0 + a1) + (a2 + a3));
+    return group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
 }
 
 template <int G, typename IdxT>
@@ -176,9 +198,8 @@ __device__ __forceinline__ float group_row_dot(const float *__restrict__ Wd, con
 
 // G lanes per row: a wave works on 64/G rows at a time (whole waves for rows longer than 512
 // slots, a half, a quarter or an eighth of a wave for shorter ones, so that short rows do not leave lanes idle).
-// MM: so_matmul's products with few columns, one of the row-major X and Y per blockIdx.y (their rows `C` floats apart),
-// with an activation.
-template <bool XLDS, int G, bool I16, bool MM, bool TELL>
+// MM: so_matmul's products with few columns of row-major X and Y (their rows `C` floats apart), W of them per blockIdx.y, with an activation.
+template <bool XLDS, int G, bool I16, int W, bool MM, bool TELL>
 __global__ __launch_bounds__(kBlock)
 void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ idx,
                         const uint32_t *__restrict__ nnz, uint32_t count, uint32_t r,
@@ -186,6 +207,7 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
                         const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act, Tell tell)
 {
     extern __shared__ float lds_x[];
+    static_assert(W == 1 || (MM && XLDS), "several columns at once are all the columns, and in LDS");
     constexpr uint32_t RPW = 64 / G;                                     // rows per wave
     const uint32_t lane = threadIdx.x & 63u, sub = lane % G, grp = lane / G;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6));
@@ -195,40 +217,46 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
     // Rows are pipelined: the first 16 G slots of the next row are requested before the current
     // row is reduced, and those of the group's first row before x is staged, so that a wave always
     // has a row's worth of loads in flight.  Row lengths are fetched two rows ahead, so that
-    // requesting a row never waits for its length.
+    // requesting a row never waits for its length -- nor does the first, whose slots are requested up to its
+    // pitch (200 x 3000 and 40 x 600: 0.03 to 0.12 us of 3.7).
     uint32_t row = wave * RPW + grp, held = threadIdx.x / G;
-    uint64_t beg = (uint64_t)row * r, end = beg + (row < count ? nnz[row] : 0u);
-    uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
+    const uint64_t first = (uint64_t)row * r;
     RowLoads<I16> cur, nxt;
-    if (row < count) row_issue<G, I16>(Wd4, idx4, beg, end, (beg >> 2) + sub, cur);
-    const uint32_t pitch = MM ? C : 1u;
-    const float *xs = stage_x<XLDS>(MM ? x + blockIdx.y : x, n, lds_x, pitch);
-    const size_t xpitch = MM && !XLDS ? C : 1u;
+    if (row < count) row_issue<G, I16>(Wd4, idx4, first, first + r, (first >> 2) + sub, cur);
+    uint64_t beg = first, end = beg + (row < count ? nnz[row] : 0u);
+    uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
+    const uint32_t pitch = MM && W == 1 ? C : 1u;
+    const float *xs = stage_x<XLDS>(MM && W == 1 ? x + blockIdx.y : x, n * W, lds_x, pitch);
+    const size_t xpitch = XLDS ? W : pitch;
     // all groups of a wave make the same number of trips (the reductions need every lane)
     for (uint32_t base = wave * RPW; base < count; base += stride, row += stride) {
         const uint64_t nrow = (uint64_t)row + stride;
         const uint64_t nbeg = nrow * r, nend = nbeg + len1;
         if (nrow < count) row_issue<G, I16>(Wd4, idx4, nbeg, nend, (nbeg >> 2) + sub, nxt);
         const uint32_t len2 = nrow + stride < count ? nnz[nrow + stride] : 0u;
-        float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+        float a[W][4] = {};
         if (row < count && end > beg) {
             const uint64_t qlast = (end - 1) >> 2;
             uint64_t q0 = (beg >> 2) + sub;
-            row_consume<G, I16>(cur, beg, end, q0, xs, a0, a1, a2, a3, xpitch);
+            row_consume<G, I16>(cur, beg, end, q0, xs, a, xpitch);
             for (q0 += 4 * G; q0 <= qlast; q0 += 4 * G) {        // rows longer than one pass
                 RowLoads<I16> more;
                 row_issue<G, I16>(Wd4, idx4, beg, end, q0, more);
-                row_consume<G, I16>(more, beg, end, q0, xs, a0, a1, a2, a3, xpitch);
+                row_consume<G, I16>(more, beg, end, q0, xs, a, xpitch);
             }
         }
-        const float s = group_sum<G>((a0 + a1) + (a2 + a3));
-        if (sub == 0 && row < count) {
-            float v = (bias ? bias[row] : 0.0f) + s;
-            if (MM) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
-                       : act == SO_ACT_TANH ? so_epilogue<SO_ACT_TANH>(v) : v;
-            if constexpr (TELL) {
-                lds_x[(XLDS ? n : 0u) + held] = v;      // behind x: the workgroup's 16 RPW consecutive rows of each pass
-            } else y[MM ? (size_t)row * C + blockIdx.y : row] = v;
+        const float b = sub == 0 && row < count && bias ? bias[row] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < W; ++j) {
+            const float s = group_sum<G>((a[j][0] + a[j][1]) + (a[j][2] + a[j][3]));
+            if (sub == 0 && row < count) {
+                float v = b + s;
+                if (MM) v = act == SO_ACT_RELU ? so_epilogue<SO_ACT_RELU>(v) : act == SO_ACT_SIGMOID ? so_epilogue<SO_ACT_SIGMOID>(v)
+                          : act == SO_ACT_TANH ? so_epilogue<SO_ACT_TANH>(v) : v;
+                if constexpr (TELL) {
+                    lds_x[(XLDS ? n : 0u) + held] = v;      // behind x: the workgroup's 16 RPW consecutive rows of each pass
+                } else y[!MM ? row : W > 1 ? (size_t)row * W + j : (size_t)row * C + blockIdx.y] = v;
+            }
         }
         cur = nxt;
         beg = nbeg;
@@ -315,13 +343,13 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
             const uint2 e = ba.rowswg[g];
             const uint64_t beg = (uint64_t)e.x * r, end = beg + e.y;
             const uint64_t qlast = (end - 1) >> 2;                  // e.y > 4096
-            float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+            float a[1][4] = {};
             for (uint64_t q = (beg >> 2) + wave * 256u + lane; q <= qlast; q += 256u * kWavesPerBlock) {
                 RowLoads<I16> L;
                 row_issue<64, I16>(Wd4, idx4, beg, end, q, L);
-                row_consume<64, I16>(L, beg, end, q, xs, a0, a1, a2, a3);
+                row_consume<64, I16>(L, beg, end, q, xs, a);
             }
-            const float s = group_sum<64>((a0 + a1) + (a2 + a3));
+            const float s = group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
             if (lane == 0) part[wave] = s;
             __syncthreads();
             if (threadIdx.x == 0) {
@@ -355,17 +383,17 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
         RowLoads<I16> A;
         if (e.y > 0) row_issue<64, I16>(Wd4, idx4, beg, end, q0, A);
         if (g < ba.n64) {
-            float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+            float a[1][4] = {};
             if (e.y > 0) {
-                row_consume<64, I16>(A, beg, end, q0, xs, a0, a1, a2, a3);
+                row_consume<64, I16>(A, beg, end, q0, xs, a);
                 const uint64_t qlast = (end - 1) >> 2;
                 for (uint64_t q = q0 + 256; q <= qlast; q += 256) {
                     RowLoads<I16> L;
                     row_issue<64, I16>(Wd4, idx4, beg, end, q, L);
-                    row_consume<64, I16>(L, beg, end, q, xs, a0, a1, a2, a3);
+                    row_consume<64, I16>(L, beg, end, q, xs, a);
                 }
             }
-            const float s = group_sum<64>((a0 + a1) + (a2 + a3));
+            const float s = group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
             if (lane == 0) (TELL ? held[threadIdx.x >> 6] : y[e.x]) = (bias ? bias[e.x] : 0.0f) + s;
         }
         uint32_t place = threadIdx.x >> 6;
@@ -421,12 +449,17 @@ bool use_lds(so_ctx *ctx, K kernel, uint32_t n, uint64_t nnz_total, uint32_t blo
     return true;
 }
 
-// The row kernel on the row-major arrays, on the 16-bit columns when the handle has them.
-template <bool MM, bool TELL>
-void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, const float *dBias, float *dy, int act, const Tell &tell)
+// The row kernel on the row-major arrays, on the 16-bit columns when the handle has them: the C columns of X in turn (MM), or W = C at once, where that
+// is the better way; false: it is not.
+//
+// At once a workgroup streams its rows once and stages all columns, in turn each column has workgroups of its own: better while those fit the chip, whose
+// compute units would stand idle otherwise.  Us, in turn / at once, two and three columns: 200 x 3000 at 80 % sparse 4.2 / 4.8 and 4.3 / 5.3, 1000 x 1000 at 70 %
+// 4.0 / 4.3 and 4.1 / 4.8, 2000 x 4000 at 90 % 5.0 / 4.9 and 8.6 / 5.4, 4096 x 4096 at 90 % 8.8 / 5.3 and 12.3 / 5.9, 2500 x 12 000 at 90 % 16.4 / 8.9 and 18.4 / 10.1.
+template <int W, bool MM, bool TELL>
+bool launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, const float *dBias, float *dy, int act, const Tell &tell)
 {
     const uint32_t cus = (uint32_t)ctx->compute_units;
-    const size_t held = TELL ? kBlock * sizeof(float) : 0, lds = (size_t)E->n * sizeof(float) + held;
+    const size_t held = TELL ? kBlock * sizeof(float) : 0, more_x = (size_t)(W - 1) * E->n * sizeof(float), lds = (size_t)E->n * sizeof(float) + more_x + held;
     const bool i16 = E->d_idx16 != nullptr && ctx->tune.matvec_idx16 != 0;
     const void *cols = i16 ? (const void *)E->d_idx16 : (const void *)E->d_idx;
     // Lanes per row by the longest row (one pass of 16 G slots should cover it), but never so
@@ -438,13 +471,15 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
     // One resident workgroup per compute unit (the pipelined rows need the registers); each of
     // its 16 waves keeps two passes' loads in flight.
     const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
+    if (W > 1 && blocks * C <= cus) return false;
 #define SO_MV_ROWS(G, I16)                                                                                         \
     do {                                                                                                       \
-        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, MM, TELL>, E->n, E->total_nnz, blocks, held))            \
-            matvec_rows_kernel<true, G, I16, MM, TELL><<<dim3(blocks, C), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
+        if (use_lds(ctx, matvec_rows_kernel<true, G, I16, W, MM, TELL>, E->n, E->total_nnz, blocks, more_x + held)) \
+            matvec_rows_kernel<true, G, I16, W, MM, TELL><<<dim3(blocks, C / W), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
                                                                                    dx, E->n, dBias, dy, C, act, tell); \
+        else if constexpr (W > 1) return false;                                                                \
         else                                                                                                   \
-            matvec_rows_kernel<false, G, I16, MM, TELL><<<dim3(blocks, C), kBlock, held, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
+            matvec_rows_kernel<false, G, I16, W, MM, TELL><<<dim3(blocks, C), kBlock, held, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
                                                                                   dx, E->n, dBias, dy, C, act, tell);  \
     } while (0)
 #define SO_MV_ROWS_G(I16)                                                                                          \
@@ -458,6 +493,7 @@ void launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
     else SO_MV_ROWS_G(false);
 #undef SO_MV_ROWS_G
 #undef SO_MV_ROWS
+    return true;
 }
 
 // The length classes in one launch; false: nothing to launch.
@@ -512,7 +548,9 @@ bool launch_bins(so_ctx *ctx, const so_ellpack *E, const float *dx, const float 
 
 so_status so_matvec_columns(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t C, const float *dBias, float *dY, int act)
 {
-    launch_rows<true, false>(ctx, E, dX, C, dBias, dY, act, Tell());
+    if (C == 2u && launch_rows<2, true, false>(ctx, E, dX, C, dBias, dY, act, Tell())) return SO_OK;
+    if (C == 3u && launch_rows<3, true, false>(ctx, E, dX, C, dBias, dY, act, Tell())) return SO_OK;
+    launch_rows<1, true, false>(ctx, E, dX, C, dBias, dY, act, Tell());
     return SO_OK;
 }
 
@@ -547,7 +585,7 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
     const uint32_t cus = (uint32_t)ctx->compute_units;
     const size_t lds = (size_t)E->n * sizeof(float);
     if (layout == SO_LAYOUT_ROW) {
-        launch_rows<false, false>(ctx, E, dx, 1, dBias, dy, SO_ACT_NONE, Tell());
+        launch_rows<1, false, false>(ctx, E, dx, 1, dBias, dy, SO_ACT_NONE, Tell());
     } else if (layout == SO_LAYOUT_SLOT) {
         const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kBlock), 2u * cus));
 #define SO_MV_SLOT(T, COLS)                                                                                        \
@@ -582,7 +620,7 @@ extern "C" so_status so_matvec_to_host(so_ctx *ctx, const so_ellpack *E, const f
     Tell tell;
     if ((rows || bins) && (dx != nullptr || E->total_nnz == 0) && so_stage_result(ctx, E->m, &tell.rows, &tell.turn)) {
         bool told = false;
-        if (rows) launch_rows<false, true>(ctx, E, dx, 1, dBias, nullptr, SO_ACT_NONE, tell);
+        if (rows) launch_rows<1, false, true>(ctx, E, dx, 1, dBias, nullptr, SO_ACT_NONE, tell);
         if (rows || launch_bins<true>(ctx, E, dx, dBias, nullptr, tell)) {
             SO_LAUNCH_CHECK();
             const so_status s = so_stage_result_take(ctx, E->m, rows ? nullptr : E->bin_order.data(), y, tell.turn, &told);
