@@ -267,8 +267,8 @@ extern "C" so_status so_d2h(so_ctx *ctx, void *dst, const void *src, size_t byte
 // hipMemcpyAsync from and to pageable memory takes 15 us in and 21 us out for 4 KB, each with a wait of its own, and
 // 34 and 42 us for 800 KB.  Here the host copies to pinned memory (4 KB 0.2 us, 800 KB 9 us) in pieces, and a kernel per
 // piece reads that over the link while the next piece is copied; the way out is a kernel that writes pinned memory and
-// then a word that the host polls.  Host to host, before and now: a 1500 x 1000 ellpack_matvec with bias 49 and 19 us,
-// the MLP 784-4096-4096-4096-10 at batch 256 150 and 141, one image through the ResNet-18-shaped stack 312 and 284.
+// then a word that the host polls.  Host to host, before and now: the MLP 784-4096-4096-4096-10 at batch 256 150 and 141 us, one image through the
+// ResNet-18-shaped stack 312 and 284.
 //
 // Bound by latencies in a row: per kernel the launch, the link's 2 to 3 us and 256 KB at about 50 GB/s.  A model's input and output
 // are [batch][features] on the host and [features][batch] in memory, so their kernels transpose (and pad) on the way, in
@@ -319,7 +319,8 @@ void so_stage_in_transposed_kernel(float *dst, uint32_t stride, const float *src
         if (c0 + c < cols && r0 + r < stride) dst[(size_t)(c0 + c) * stride + r0 + r] = tile[c][r];
 }
 
-// The end of a way out: the last workgroup to finish tells the host: `turn`, and beside it the word of the bounded waits.
+// The end of a way out: the last workgroup to finish tells the host: `turn`, and with it in one store the word of the bounded waits.  (A store
+// for each and a fence between them: 0.6 us more of the encoder's 16 to 18 on small matrices, 0.7 of a model's 24.)
 __device__ __forceinline__ void tell_host(uint32_t *done, const uint32_t *gave_up, uint32_t *flag, uint32_t turn)
 {
     __threadfence_system();
@@ -329,9 +330,7 @@ __device__ __forceinline__ void tell_host(uint32_t *done, const uint32_t *gave_u
         if (__hip_atomic_fetch_add(done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1u) return;
         __hip_atomic_store(done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    flag[1] = *gave_up;
-    __threadfence_system();
-    __hip_atomic_store(flag, turn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(flag), (unsigned long long)*gave_up << 32 | turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // (Kernels of their own: one kernel for both, on a branch, cost each ellpack_matvec from host arrays 0.2 to 0.4 us of 18 to 20.)
@@ -354,6 +353,24 @@ void so_stage_out_transposed_kernel(uint32_t *dst, const uint32_t *src, uint32_t
         reinterpret_cast<uint4 *>(dst)[i] = make_uint4(word(4u * i), word(4u * i + 1u), word(4u * i + 2u), word(4u * i + 3u));
     if (blockIdx.x == 0 && threadIdx.x < words % 4u) dst[quads * 4u + threadIdx.x] = word(quads * 4u + threadIdx.x);
     tell_host(done, gave_up, flag, turn);
+}
+
+// A result of fewer than kStagePairsMost words as pairs {value, turn}, behind them the word of the bounded waits: what the host polls is the result itself, without
+// a fence over the link and a word behind it.  cols != 0: a transpose, as above.  Models host to host, us, with the fence and the word / so: 85-351-177 at batch 5
+// 20.5 / 18.5, 100-300-20 at 1 18.4 / 16.6, 100-300-1000 at 8 (8000 words) 22.8 / 20.9, 100-300-64 at 100 25.0 / 22.9.
+__global__ __launch_bounds__(256)
+void so_stage_pairs_kernel(uint2 *pairs, const uint32_t *src, uint32_t words, uint32_t cols, uint32_t pitch, const uint32_t *gave_up, uint32_t turn)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, rows = cols ? words / cols : 0u;
+    if (i > words) return;
+    uint32_t v;
+    if (i == words) v = *gave_up;
+    else if (cols == 0u) v = src[i];
+    else {
+        const uint32_t c = i / rows;
+        v = src[(size_t)(i - c * rows) * pitch + c];
+    }
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(pairs + i), (unsigned long long)turn << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The staging memory, made on first use.  False where there is none: the callers then copy as so_h2d and so_d2h do.
@@ -438,15 +455,16 @@ bool so_stage_result(so_ctx *ctx, uint32_t floats, uint2 **rows, uint32_t *turn)
     return true;
 }
 
-so_status so_stage_result_take(so_ctx *ctx, uint32_t floats, const uint32_t *order, float *dst, uint32_t turn, bool *told)
+// The pairs from place `from` on, as their turn comes.
+static so_status take_pairs(so_ctx *ctx, uint32_t from, uint32_t floats, const uint32_t *order, void *dst, uint32_t turn, bool *told)
 {
-    volatile const uint64_t *const rows = (volatile const uint64_t *)(ctx->h_stage + kStagePairs);
+    volatile const uint64_t *const rows = (volatile const uint64_t *)(ctx->h_stage + kStagePairs) + from;
     *told = true;
     uint32_t at = 0;
     for (uint32_t spin = 1; at < floats; ++spin) {
         for (uint64_t pair; at < floats && (uint32_t)((pair = rows[at]) >> 32) == turn; ++at) {
             const uint32_t bits = (uint32_t)pair;
-            std::memcpy(dst + (order ? order[at] : at), &bits, 4);
+            std::memcpy((char *)dst + 4 * (size_t)(order ? order[at] : at), &bits, 4);
         }
         if (at == floats) break;
         if (spin % 4096u == 0) {
@@ -459,6 +477,11 @@ so_status so_stage_result_take(so_ctx *ctx, uint32_t floats, const uint32_t *ord
     }
     ctx->stage_used = 0;                       // the stream's earlier work, and with it every way in, is done
     return SO_OK;
+}
+
+so_status so_stage_result_take(so_ctx *ctx, uint32_t floats, const uint32_t *order, float *dst, uint32_t turn, bool *told)
+{
+    return take_pairs(ctx, 0u, floats, order, dst, turn, told);
 }
 
 __global__ void so_tell_host_kernel(const uint32_t *gave_up, uint32_t *flag, uint32_t turn) { tell_host(nullptr, gave_up, flag, turn); }
@@ -499,6 +522,17 @@ static so_status stage_out(so_ctx *ctx, void *dst, const void *src, size_t bytes
 {
     volatile uint32_t *const flag = (volatile uint32_t *)(ctx->h_stage + kStageFlag);
     const uint32_t turn = ++ctx->stage_turn;
+    if (bytes / 4 < kStagePairsMost) {
+        const uint32_t words = (uint32_t)(bytes / 4);
+        so_stage_pairs_kernel<<<words / 256u + 1u, 256, 0, ctx->stream>>>((uint2 *)(ctx->h_stage + kStagePairs), (const uint32_t *)src, words, cols, pitch, ctx->d_wait_gave_up, turn);
+        SO_LAUNCH_CHECK();
+        uint32_t gave_up = 0;
+        so_status s = ctx->waits_pending ? take_pairs(ctx, words, 1u, nullptr, &gave_up, turn, told) : SO_OK;
+        if (s == SO_OK && gave_up != 0) return so_stream_wait(ctx, who);
+        if (s == SO_OK && (!ctx->waits_pending || *told)) s = take_pairs(ctx, 0u, words, nullptr, dst, turn, told);
+        if (s == SO_OK && *told) ctx->waits_pending = false;
+        return s;
+    }
     const uint32_t blocks = (uint32_t)std::min<size_t>((bytes + 8191) / 8192, 128);
     uint32_t *const to = (uint32_t *)(ctx->h_stage + kStageIn);
     if (cols == 0)

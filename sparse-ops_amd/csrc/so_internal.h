@@ -86,7 +86,7 @@ struct so_ctx {
 };
 
 // Rows of one length class for the binned matvec: `group` lanes cooperate on a row.
-constexpr uint32_t kStagePairsMost = 8192;       // floats of a result that a launch writes to the staging memory itself (so_matvec_to_host)
+constexpr uint32_t kStagePairsMost = 8192;       // floats of a result that goes to the staging memory as pairs {value, turn}
 
 struct so_bin {
     uint32_t group = 0;      // 4, 16 or 64 lanes per row, 1024: a whole workgroup
