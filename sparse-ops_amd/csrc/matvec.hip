@@ -146,7 +146,10 @@ __device__ __forceinline__ void row_issue(const f32x4 *__restrict__ Wd4, const t
 }
 
 // a[j]: the four partial sums of column j of the W dense ones, which lie side by side in xs, `pitch` floats from one element to the next.
-template <int G, bool I16, int W>
+// FOURS: the four slots of a group together, which the compiler turns into branches around the last of them: the better code for the row kernel's one column
+// (8000 x 8000 at 85 % sparse 12.65 against 13.35 us, 12 000 x 2000 at 95 % 5.98 and 5.88), not for the length classes' waves (Zipf rows, 12 000 x 12 000, 8.57 and 8.43) nor
+// for three columns, which spill.
+template <int G, bool I16, bool FOURS, int W>
 __device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg, uint64_t end, uint64_t q0, const float *xs, float (&a)[W][4], size_t pitch = W)
 {
     // slot k of group u is live iff its distance from the row's start is in [0, end - beg): one
@@ -157,6 +160,18 @@ __device__ __forceinline__ void row_consume(const RowLoads<I16> &L, uint64_t beg
     for (int u = 0; u < 4; ++u) {
         const int32_t rel = rel0 + 4 * G * u;
         const u32x4 c = ColGroup<I16>::cols(L.c[u]);
+        if constexpr (FOURS) {
+            static_assert(W == 1, "one column");
+            const bool v0 = (uint32_t)rel < len, v1 = (uint32_t)(rel + 1) < len;
+            const bool v2 = (uint32_t)(rel + 2) < len, v3 = (uint32_t)(rel + 3) < len;
+            const float x0 = xs[(v0 ? c.x : 0u) * pitch], x1 = xs[(v1 ? c.y : 0u) * pitch];
+            const float x2 = xs[(v2 ? c.z : 0u) * pitch], x3 = xs[(v3 ? c.w : 0u) * pitch];
+            a[0][0] = __builtin_fmaf(v0 ? L.w[u].x : 0.0f, v0 ? x0 : 0.0f, a[0][0]);
+            a[0][1] = __builtin_fmaf(v1 ? L.w[u].y : 0.0f, v1 ? x1 : 0.0f, a[0][1]);
+            a[0][2] = __builtin_fmaf(v2 ? L.w[u].z : 0.0f, v2 ? x2 : 0.0f, a[0][2]);
+            a[0][3] = __builtin_fmaf(v3 ? L.w[u].w : 0.0f, v3 ? x3 : 0.0f, a[0][3]);
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const bool v = (uint32_t)(rel + k) < len;
@@ -182,7 +197,7 @@ __device__ __forceinline__ float wave_row_dot(const f32x4 *__restrict__ Wd4, con
     for (uint64_t q0 = (beg >> 2) + lane; q0 <= qlast; q0 += 256) {
         RowLoads<I16> L;
         row_issue<64, I16>(Wd4, idx4, beg, end, q0, L);
-        row_consume<64, I16>(L, beg, end, q0, xs, a);
+        row_consume<64, I16, false>(L, beg, end, q0, xs, a);
     }
     return group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
 }
@@ -222,9 +237,10 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
     uint32_t row = wave * RPW + grp, held = threadIdx.x / G;
     const uint64_t first = (uint64_t)row * r;
     RowLoads<I16> cur, nxt;
-    if (row < count) row_issue<G, I16>(Wd4, idx4, first, first + r, (first >> 2) + sub, cur);
-    uint64_t beg = first, end = beg + (row < count ? nnz[row] : 0u);
+    const uint32_t len0 = row < count ? nnz[row] : 0u;
     uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
+    if (row < count) row_issue<G, I16>(Wd4, idx4, first, first + r, (first >> 2) + sub, cur);
+    uint64_t beg = first, end = beg + len0;
     const uint32_t pitch = MM && W == 1 ? C : 1u;
     const float *xs = stage_x<XLDS>(MM && W == 1 ? x + blockIdx.y : x, n * W, lds_x, pitch);
     const size_t xpitch = XLDS ? W : pitch;
@@ -238,11 +254,11 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
         if (row < count && end > beg) {
             const uint64_t qlast = (end - 1) >> 2;
             uint64_t q0 = (beg >> 2) + sub;
-            row_consume<G, I16>(cur, beg, end, q0, xs, a, xpitch);
+            row_consume<G, I16, W == 1>(cur, beg, end, q0, xs, a, xpitch);
             for (q0 += 4 * G; q0 <= qlast; q0 += 4 * G) {        // rows longer than one pass
                 RowLoads<I16> more;
                 row_issue<G, I16>(Wd4, idx4, beg, end, q0, more);
-                row_consume<G, I16>(more, beg, end, q0, xs, a, xpitch);
+                row_consume<G, I16, W == 1>(more, beg, end, q0, xs, a, xpitch);
             }
         }
         const float b = sub == 0 && row < count && bias ? bias[row] : 0.0f;
@@ -347,7 +363,7 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
             for (uint64_t q = (beg >> 2) + wave * 256u + lane; q <= qlast; q += 256u * kWavesPerBlock) {
                 RowLoads<I16> L;
                 row_issue<64, I16>(Wd4, idx4, beg, end, q, L);
-                row_consume<64, I16>(L, beg, end, q, xs, a);
+                row_consume<64, I16, false>(L, beg, end, q, xs, a);
             }
             const float s = group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
             if (lane == 0) part[wave] = s;
@@ -385,12 +401,12 @@ void matvec_binned_kernel(const float *__restrict__ Wd, const void *__restrict__
         if (g < ba.n64) {
             float a[1][4] = {};
             if (e.y > 0) {
-                row_consume<64, I16>(A, beg, end, q0, xs, a);
+                row_consume<64, I16, false>(A, beg, end, q0, xs, a);
                 const uint64_t qlast = (end - 1) >> 2;
                 for (uint64_t q = q0 + 256; q <= qlast; q += 256) {
                     RowLoads<I16> L;
                     row_issue<64, I16>(Wd4, idx4, beg, end, q, L);
-                    row_consume<64, I16>(L, beg, end, q, xs, a);
+                    row_consume<64, I16, false>(L, beg, end, q, xs, a);
                 }
             }
             const float s = group_sum<64>((a[0][0] + a[0][1]) + (a[0][2] + a[0][3]));
