@@ -40,6 +40,7 @@
 // kernel 35 / 52), 1067 x 900 x 28, 60 %, 11 / 27 (12 / 36), 256 x 1136 x 36 8 / 15 (10 / 28), 2000 x 1500 x 3, 50 %, 13 / 13 (row kernel 12); output
 // by output, a whole wave for each, it took 24 / 90, 13 / 116, 10 / 80 and 18 / 42.
 #include "so_internal.h"
+#include "lane_moves.h"
 #include "exact_outputs.h"
 #include "lds_sync.h"
 
@@ -77,7 +78,9 @@ struct NarrowArgs {
     uint32_t r;
 };
 
-__device__ __forceinline__ float xor_add(float keep, float send, int mask) { return keep + __shfl_xor(send, mask, 64); }
+// (By lane moves; through LDS a launch of 4.4 to 6 us takes 0.09 to 0.14 more.)
+template <int D>
+__device__ __forceinline__ float xor_add(float keep, float send) { return keep + so_lanes::across<D>(send); }
 
 // V values of a row of X per lane and LDS read, R reads per chunk: 4 V R columns.  PASSES: X in LDS a part at a time.
 template <int V, int R, int ACT, bool PASSES>
@@ -354,20 +357,20 @@ void ellpack_matmul_narrow_kernel(NarrowArgs a)
     float out[R];
     uint32_t col;
     if constexpr (R == 2) {
-        out[0] = xor_add(hi8 ? s[2] : s[0], hi8 ? s[0] : s[2], 8);
-        out[1] = xor_add(hi8 ? s[3] : s[1], hi8 ? s[1] : s[3], 8);
+        out[0] = xor_add<8>(hi8 ? s[2] : s[0], hi8 ? s[0] : s[2]);
+        out[1] = xor_add<8>(hi8 ? s[3] : s[1], hi8 ? s[1] : s[3]);
         col = (lane & 7u) * 4u + (hi8 ? 2u : 0u);
     } else if constexpr (V == 4) {
-        const float t0 = xor_add(hi8 ? s[2] : s[0], hi8 ? s[0] : s[2], 8), t1 = xor_add(hi8 ? s[3] : s[1], hi8 ? s[1] : s[3], 8);
-        out[0] = xor_add(hi4 ? t1 : t0, hi4 ? t0 : t1, 4);
+        const float t0 = xor_add<8>(hi8 ? s[2] : s[0], hi8 ? s[0] : s[2]), t1 = xor_add<8>(hi8 ? s[3] : s[1], hi8 ? s[1] : s[3]);
+        out[0] = xor_add<4>(hi4 ? t1 : t0, hi4 ? t0 : t1);
         col = (lane & 3u) * 4u + (hi8 ? 2u : 0u) + (hi4 ? 1u : 0u);
     } else if constexpr (V == 2) {
-        const float t = xor_add(hi8 ? s[1] : s[0], hi8 ? s[0] : s[1], 8);
-        out[0] = xor_add(t, t, 4);
+        const float t = xor_add<8>(hi8 ? s[1] : s[0], hi8 ? s[0] : s[1]);
+        out[0] = xor_add<4>(t, t);
         col = hi4 ? 0xffffu : (lane & 3u) * 2u + (hi8 ? 1u : 0u);    // (lanes with bit 2 hold the same again)
     } else {
-        const float t = xor_add(s[0], s[0], 8);
-        out[0] = xor_add(t, t, 4);
+        const float t = xor_add<8>(s[0], s[0]);
+        out[0] = xor_add<4>(t, t);
         col = hi4 || hi8 ? 0xffffu : lane & 3u;
     }
     // Sum over the waves of a quad, through LDS.

@@ -22,6 +22,7 @@
 // 16 interleaved partials and a tree (:72-96); the orders here differ, so results
 // agree to fp32 round-off, not bit for bit.
 #include "so_internal.h"
+#include "lane_moves.h"
 
 #include <algorithm>
 
@@ -75,32 +76,10 @@ __device__ __forceinline__ void tell_host(const Tell &tell, const float *held, u
     }
 }
 
-// The sum over G lanes in all of them: pairs G / 2 apart, then G / 4 and so on, by lane moves inside the vector unit (six exchanges through LDS, one
-// after the other, at the end of a launch: 1000 x 1000 at 70 % sparse 4.00 us, so 3.75).  From 8 lanes on a rotation of the row of 16 is the exchange, since a value then
-// comes again every 2 * distance lanes.
-template <int CONTROL, int BANKS = 0xf>
-__device__ __forceinline__ float lanes_moved(float old, float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CONTROL, 0xf, BANKS, false));
-}
+// The sum over G lanes in all of them, by lane moves (by six exchanges through LDS, one after the other, at the end of a launch: 1000 x 1000 at 70 % sparse
+// 4.00 us, so 3.75).
 template <int G>
-__device__ __forceinline__ float group_sum(float v)
-{
-    constexpr int kRorBase = 0x120, kShl = 0x100, kShr = 0x110;          // row_ror:n, row_shl:n, row_shr:n
-    if constexpr (G >= 64) {
-        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    }
-    if constexpr (G >= 32) {
-        const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    }
-    if constexpr (G >= 16) v += lanes_moved<kRorBase + 8>(v, v);
-    if constexpr (G >= 16) v += lanes_moved<kRorBase + 4>(v, v);
-    else if constexpr (G == 8) v += lanes_moved<kShr + 4, 0xa>(lanes_moved<kShl + 4, 0x5>(v, v), v);
-    v += lanes_moved<0x4e>(v, v);                                        // quad_perm: [2, 3, 0, 1]
-    return v + lanes_moved<0xb1>(v, v);                                  // [1, 0, 3, 2]
-}
+__device__ __forceinline__ float group_sum(float v) { return so_lanes::reduce<G>(v, so_lanes::Sum()); }
 
 // Stage x in LDS (XLDS) or read it through the cache hierarchy.  `pitch`: floats from one element of x to the next.
 template <bool XLDS>

@@ -1,5 +1,6 @@
 // Context, memory, timing, launch graphs and the device-resident ELLPACK layouts.
 #include "so_internal.h"
+#include "lane_moves.h"
 
 #include <algorithm>
 #include <atomic>
@@ -1246,8 +1247,7 @@ void ellpack_count_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, u
 #pragma unroll
             for (int e = 0; e < 4; ++e) c += v[e] != 0.0f ? 1u : 0u;
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+        c = so_lanes::reduce<64>(c, so_lanes::Sum());
         if (sharers == 1u && lane == 0) nnz[row] = c;
         vmax = max(vmax, c);
         vsum += c;
@@ -1275,11 +1275,8 @@ void ellpack_count_fold_kernel(const uint2 *__restrict__ partial, uint32_t nbloc
         vmax = max(vmax, p.x);
         vsum += p.y;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        vmax = max(vmax, (uint32_t)__shfl_xor(vmax, off, 64));
-        vsum += __shfl_xor(vsum, off, 64);
-    }
+    vmax = so_lanes::reduce<64>(vmax, so_lanes::Max());
+    vsum = so_lanes::reduce<64>(vsum, so_lanes::Sum());
     if ((threadIdx.x & 63u) == 0) { smax[threadIdx.x >> 6] = vmax; ssum[threadIdx.x >> 6] = vsum; }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -1318,8 +1315,8 @@ void ellpack_pack_kernel(const float *__restrict__ W, uint32_t m, uint32_t n, ui
         const uint2 *partial = reinterpret_cast<const uint2 *>(reinterpret_cast<const char *>(header) + kEncodeHeaderBytes);
         unsigned long long sum = 0;
         for (uint32_t i = tid; i < fold; i += 256u) { const uint2 p = partial[i]; r = max(r, p.x); sum += p.y; }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) { r = max(r, (uint32_t)__shfl_xor(r, off, 64)); sum += __shfl_xor(sum, off, 64); }
+        r = so_lanes::reduce<64>(r, so_lanes::Max());
+        sum = so_lanes::reduce<64>(sum, so_lanes::Sum());
         if (lane == 0) { smax[wave] = r; ssum[wave] = sum; }
         __syncthreads();
         r = max(max(smax[0], smax[1]), max(smax[2], smax[3]));
