@@ -230,7 +230,10 @@ struct ColShape { uint32_t G, waves; size_t lds; double us, rounds; };
 // Channels per workgroup by estimated time: rounds of workgroups over the chip, each with a start-up of 2.5 us and its
 // longest chain at 10 ns per entry on a SIMD of its own, 7.5 ns per wave that shares it.  A large window is copied by
 // more waves than compute.  Measured at batch 1 on a ResNet-18-shaped stack: 56x56x64 8.9 us, 28x28x128 8.1, 14x14x256
-// 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.
+// 9.8, 7x7x512 14.4; the windowed kernel with the batch carried as four: 12.3, 14.1, 17.5, 27.6.  Of two sizes that the estimate holds equal the smaller where
+// the larger fills the chip more than once: its start-ups run beside others' chains.  Of 242 layers of 20x20 to 260x260 at batch 1 to 3 that changes 54, none to
+// the worse by more than the runs differ, by up to 1.6: 3 -> 64 at 224x224, 7x7/2, batch 1 15.3 -> 10.6 us, 6 -> 128 at 194x194, 5x5, 64.5 -> 42.6.  (Where the larger is
+// resident at once the smaller copies more windows: 64 -> 64 at 56x56 8.0 -> 9.5.)
 //
 // From 8 entries on windows of few pixels are the rule, and many workgroups of few channels on large images: 2.75 us; a chunk's start-up by its
 // LDS, 0.44 us and 24 ns per KB, 9 more for every further workgroup on the compute unit; 0.5 us for each of those, 2.2 for every further filling of the
@@ -259,7 +262,7 @@ ColShape column_shape(const so_ctx *ctx, const so_conv_plan *plan, const so_conv
 {
     ColShape best{16, 16, 0, 1e30, 1.0};
     for (uint32_t G = 16; G >= 4; G /= 2)
-        if (const ColShape s = column_shape(ctx, plan, c, G); s.us < best.us) best = s;
+        if (const ColShape s = column_shape(ctx, plan, c, G); s.us < best.us || (s.us == best.us && best.rounds > 1.0)) best = s;
     return best;
 }
 
@@ -395,8 +398,10 @@ so_status so_conv_columns_build(so_ctx *ctx, so_conv_plan *plan, const std::vect
 //   6.7 / 3.7 and 6.8 / 4.1; 5 -> 47 at 14 x 10, 3x3/2, 9 entries 4.1 / 3.4 and 4.1 / 3.5; 4 -> 314 at 34 x 38, 1x1/2, 4 entries
 //   3.3 / 3.5 and 3.4 / 4.8; a large window for few entries: 587 -> 359 at 19 x 17, 1x1/2, 30 entries 6.8 / 8.8 and 5.5 / 13.4,
 //   106 -> 41 at 123 x 150, 3x3/2, 48 entries 13.1 / 14.9 and 17.8 / 42;
-//   more rounds, 3x3 to 7x7: 3 -> 16 at 512 x 512, 13 entries 39.7 / 45.7 and 42 / 86; 3 -> 32 at 1000 x 1000, 19 entries 243 / 325 and
-//   309 / 638; 7 -> 220 at 450 x 451, /2, 32 entries 185 / 158 and 197 / 285; 17 -> 5 at 651 x 456, /2, 75 entries 24.6 / 17.6 and 25.1 / 26.2;
+//   more rounds, 3x3 to 7x7: 3 -> 16 at 512 x 512, 12 entries 37.5 / 29.0 and 40.6 / 55.0; 3 -> 32 at 1000 x 1000, 16 entries 215 / 210;
+//   7 -> 220 at 450 x 450, /2, 32 entries 163 / 110 and 173 / 184; 17 -> 5 at 600 x 600, /2, 75 entries 28.1 / 13.7 and 26.9 / 21.2; 3 -> 64 at 224 x 224, 15 entries
+//   28.7 / 22.7 and 31.6 / 40.5; 3 -> 48 at 160 x 160, 7x7/2, 45 entries, batch 2 13.1 / 8.1; 5 -> 173 at 219 x 219, 5x5, 44 entries, batch 2 166 / 120; with many channels in
+//   the window 64 -> 64 at 300 x 300, 17 entries 64 / 123 and 99 / 229;
 //   34 -> 116 at 160 x 207, 168 entries 224 / 91 and 327 / 228; 1x1: 33 -> 197 at 509 x 526, /2, 10 entries 97 / 695 and 131 / 1121; 63 -> 74
 //   at 92 x 74, 63 entries 13.4 / 14.8 and 20 / 27; 214 -> 12 at 77 x 77, 214 entries 21.8 / 10.2 and 29.6 / 9.4.  At batch 4 (plans without
 //   the windowed layout): 72 entries 133 / 170, 75 29.5 / 28.0, 118 54.5 / 46.6, 147 79 / 72.
@@ -405,8 +410,10 @@ bool so_conv_columns_pays(const so_ctx *ctx, const so_conv_plan *plan, uint32_t 
     const so_conv_columns &c = *so_conv_columns_for(plan, B);
     const double entries = (double)plan->E->total_nnz / plan->g.Cout, window = (double)c.cc * c.nch * c.PE * B;
     if (entries < 8.0 || window > 480.0 * entries) return false;
-    const double least = B == 4 ? 100.0 : B == 2 || plan->g.kH * plan->g.kW == 1 ? 64.0 : 20.0;
-    return entries >= least || column_shape(ctx, plan, c).rounds <= 1.0;
+    const bool taps = plan->g.kH * plan->g.kW > 1;
+    const double least = B == 4 ? 100.0 : B == 2 || !taps ? 64.0 : 20.0;
+    if (entries >= least || column_shape(ctx, plan, c).rounds <= 1.0) return true;
+    return taps && B < 4 && entries >= (B == 2 ? 40.0 : 14.0) && window <= 100.0 * entries;
 }
 
 double so_conv_columns_estimate(const so_ctx *ctx, const so_conv_plan *plan, uint32_t B) { return column_shape(ctx, plan, *so_conv_columns_for(plan, B)).us; }
