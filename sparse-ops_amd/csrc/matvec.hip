@@ -198,7 +198,7 @@ __global__ __launch_bounds__(kBlock)
 void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ idx,
                         const uint32_t *__restrict__ nnz, uint32_t count, uint32_t r,
                         const float *__restrict__ x, uint32_t n,
-                        const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act, Tell tell)
+                        const float *__restrict__ bias, float *__restrict__ y, uint32_t C, int act, uint32_t whole, Tell tell)
 {
     extern __shared__ float lds_x[];
     static_assert(W == 1 || (MM && XLDS), "several columns at once are all the columns, and in LDS");
@@ -211,14 +211,18 @@ void matvec_rows_kernel(const float *__restrict__ Wd, const void *__restrict__ i
     // Rows are pipelined: the first 16 G slots of the next row are requested before the current
     // row is reduced, and those of the group's first row before x is staged, so that a wave always
     // has a row's worth of loads in flight.  Row lengths are fetched two rows ahead, so that
-    // requesting a row never waits for its length -- nor does the first, whose slots are requested up to its
-    // pitch (200 x 3000 and 40 x 600: 0.03 to 0.12 us of 3.7).
+    // requesting a row never waits for its length -- nor does the first of a small launch, whose slots are requested up to its pitch (`whole`).
     uint32_t row = wave * RPW + grp, held = threadIdx.x / G;
     const uint64_t first = (uint64_t)row * r;
     RowLoads<I16> cur, nxt;
     const uint32_t len0 = row < count ? nnz[row] : 0u;
     uint32_t len1 = (uint64_t)row + stride < count ? nnz[row + stride] : 0u;          // length of the next row
-    if (row < count) row_issue<G, I16>(Wd4, idx4, first, first + r, (first >> 2) + sub, cur);
+    uint32_t ask = r;
+    if (whole == 0u) {
+        ask = len0;
+        asm volatile("" : "+v"(ask));                                    // (a branch: a choice of values would wait for the length)
+    }
+    if (row < count) row_issue<G, I16>(Wd4, idx4, first, first + ask, (first >> 2) + sub, cur);
     uint64_t beg = first, end = beg + len0;
     const uint32_t pitch = MM && W == 1 ? C : 1u;
     const float *xs = stage_x<XLDS>(MM && W == 1 ? x + blockIdx.y : x, n * W, lds_x, pitch);
@@ -467,15 +471,18 @@ bool launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
     // its 16 waves keeps two passes' loads in flight.
     const uint32_t blocks = std::max(1u, std::min(so_ceil_div(E->m, kWavesPerBlock * (64u / G)), cus));
     if (W > 1 && blocks * C <= cus) return false;
+    // The first rows up to their pitch: 0.03 to 0.13 us of 3.7 (40 x 600, 200 x 3000), but up to a quarter more bytes where a wave has one row (8559 x 9895 at 97 %
+    // sparse 13.35 -> 13.66 us): up to half a million slots.
+    const uint32_t whole = (uint64_t)E->m * E->r <= (1u << 19) ? 1u : 0u;
 #define SO_MV_ROWS(G, I16)                                                                                         \
     do {                                                                                                       \
         if (use_lds(ctx, matvec_rows_kernel<true, G, I16, W, MM, TELL>, E->n, E->total_nnz, blocks, more_x + held)) \
             matvec_rows_kernel<true, G, I16, W, MM, TELL><<<dim3(blocks, C / W), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
-                                                                                   dx, E->n, dBias, dy, C, act, tell); \
+                                                                                   dx, E->n, dBias, dy, C, act, whole, tell); \
         else if constexpr (W > 1) return false;                                                                \
         else                                                                                                   \
             matvec_rows_kernel<false, G, I16, W, MM, TELL><<<dim3(blocks, C), kBlock, held, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
-                                                                                  dx, E->n, dBias, dy, C, act, tell);  \
+                                                                                  dx, E->n, dBias, dy, C, act, whole, tell);  \
     } while (0)
 #define SO_MV_ROWS_G(I16)                                                                                          \
     do {                                                                                                       \
