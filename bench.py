@@ -43,8 +43,8 @@ LDS_OPERAND_PEAK_TF = 78.6   # 256 CUs x 256 B/clk of ds_read_b128 (measured 255
 TRAFFIC_TABLE = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 HEADLINE_KERNEL = "ellpack_matmul_rbm_kernel<0>"
 TILED_KERNEL = "ellpack_matmul_tiled_kernel<0>"
-MATVEC_KERNELS = {"ellpack_matvec 16384x16384, 95% Bernoulli": ("matvec_binned_kernel<true,true>", "matvec 16384^2 uniform"),
-                  "ellpack_matvec 16384x16384, Zipf(1.2) rows capped at 2048": ("matvec_binned_kernel<true,true>", "matvec 16384^2 zipf")}
+MATVEC_KERNELS = {"ellpack_matvec 16384x16384, 95% Bernoulli": ("matvec_binned_kernel<true,true,false>", "matvec 16384^2 uniform"),
+                  "ellpack_matvec 16384x16384, Zipf(1.2) rows capped at 2048": ("matvec_binned_kernel<true,true,false>", "matvec 16384^2 zipf")}
 
 
 def measured_traffic(kernel, workload=None):
