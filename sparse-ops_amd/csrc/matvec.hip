@@ -449,7 +449,8 @@ bool use_lds(so_ctx *ctx, K kernel, uint32_t n, uint64_t nnz_total, uint32_t blo
 }
 
 // The row kernel on the row-major arrays, on the 16-bit columns when the handle has them: the C columns of X in turn (MM), or W = C at once, where that
-// is the better way; false: it is not.
+// is the better way; false: it is not.  TELL: also where the results held for the host take the place that x would have in LDS, as launch_bins does (40 874 columns,
+// 5236 rows at 94 % sparse from host arrays 81.8 us with x outside LDS, 42.8 with a kernel for the way back).
 //
 // At once a workgroup streams its rows once and stages all columns, in turn each column has workgroups of its own: better while those fit the chip, whose
 // compute units would stand idle otherwise.  Us, in turn / at once, two and three columns: 200 x 3000 at 80 % sparse 4.2 / 4.8 and 4.3 / 5.3, 1000 x 1000 at 70 %
@@ -480,9 +481,11 @@ bool launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
             matvec_rows_kernel<true, G, I16, W, MM, TELL><<<dim3(blocks, C / W), kBlock, lds, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r, \
                                                                                    dx, E->n, dBias, dy, C, act, whole, tell); \
         else if constexpr (W > 1) return false;                                                                \
-        else                                                                                                   \
+        else {                                                                                                 \
+            if (TELL && use_lds(ctx, matvec_rows_kernel<true, G, I16, W, MM, TELL>, E->n, E->total_nnz, blocks)) return false; \
             matvec_rows_kernel<false, G, I16, W, MM, TELL><<<dim3(blocks, C), kBlock, held, ctx->stream>>>(E->d_Wd, cols, E->d_nnz, E->m, E->r,  \
                                                                                   dx, E->n, dBias, dy, C, act, whole, tell);  \
+        }                                                                                                      \
     } while (0)
 #define SO_MV_ROWS_G(I16)                                                                                          \
     do {                                                                                                       \
@@ -498,7 +501,7 @@ bool launch_rows(so_ctx *ctx, const so_ellpack *E, const float *dx, uint32_t C, 
     return true;
 }
 
-// The length classes in one launch; false: nothing to launch.
+// The length classes in one launch; false: nothing to launch, or TELL has no room for both x and the results in LDS.
 template <bool TELL>
 bool launch_bins(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, const Tell &tell)
 {
@@ -536,9 +539,11 @@ bool launch_bins(so_ctx *ctx, const so_ellpack *E, const float *dx, const float 
         if (use_lds(ctx, matvec_binned_kernel<true, I16, TELL>, E->n, E->total_nnz, blocks, lds_tail - lds)) \
             matvec_binned_kernel<true, I16, TELL><<<blocks, kBlock, lds_tail, ctx->stream>>>(E->d_Wd, cols, ba, E->r, \
                                                                                        dx, E->n, dBias, dy, tell); \
-        else \
+        else { \
+            if (TELL && use_lds(ctx, matvec_binned_kernel<true, I16, TELL>, E->n, E->total_nnz, blocks, lds_tail - lds - held)) return false; \
             matvec_binned_kernel<false, I16, TELL><<<blocks, kBlock, kBinnedTailBytes + held, ctx->stream>>>( \
                 E->d_Wd, cols, ba, E->r, dx, E->n, dBias, dy, tell); \
+        } \
     } while (0)
     if (i16) SO_MV_BINNED(true);
     else SO_MV_BINNED(false);
@@ -622,8 +627,7 @@ extern "C" so_status so_matvec_to_host(so_ctx *ctx, const so_ellpack *E, const f
     Tell tell;
     if ((rows || bins) && (dx != nullptr || E->total_nnz == 0) && so_stage_result(ctx, E->m, &tell.rows, &tell.turn)) {
         bool told = false;
-        if (rows) launch_rows<1, false, true>(ctx, E, dx, 1, dBias, nullptr, SO_ACT_NONE, tell);
-        if (rows || launch_bins<true>(ctx, E, dx, dBias, nullptr, tell)) {
+        if (rows ? launch_rows<1, false, true>(ctx, E, dx, 1, dBias, nullptr, SO_ACT_NONE, tell) : launch_bins<true>(ctx, E, dx, dBias, nullptr, tell)) {
             SO_LAUNCH_CHECK();
             const so_status s = so_stage_result_take(ctx, E->m, rows ? nullptr : E->bin_order.data(), y, tell.turn, &told);
             if (s != SO_OK || told) return s;

@@ -1,6 +1,7 @@
 """so_matvec_to_host: so_matvec's bits in host memory, on every layout; one to 8193 rows (more than 8192 go the general way), rows for every length
 class, workgroups of one and of several passes, no columns, and many calls in a row, whose results lie in the same places of the staging memory."""
 import ctypes as ct
+import time
 
 import numpy as np
 import pytest
@@ -47,6 +48,37 @@ def test_bits_of_so_matvec(ctx, m, n, kind, idx16):
             assert np.array_equal(to_host(ctx, dE, dx, dB, dscratch, m, layout), dy.download())
         dx.free()
     for a in (dy, dscratch, dE):
+        a.free()
+
+
+@pytest.mark.parametrize("n", [39936, 39937, 40960, 40961])
+@pytest.mark.parametrize("layout", [hipabi.LAYOUT_ROW, hipabi.LAYOUT_BINS])
+def test_x_keeps_its_place_in_lds(ctx, n, layout):
+    """160 KB of LDS hold 40 960 elements of x, 39 936 (less the length classes' 64 bytes) with a workgroup's results beside them: the call is no slower in between than
+    the product and so_stage_out on their own (which took half its time there when x gave way)."""
+    rng = np.random.default_rng(n)
+    m, r = 2048, 6000
+    idx = np.sort(rng.integers(0, n - r, (m, r)), axis=1).astype(np.uint32) + np.arange(r, dtype=np.uint32)
+    dE = ctx.upload_ellpack(rng.standard_normal((m, r)).astype(np.float32), idx, np.full(m, r, np.uint32), m, n, r, layout | hipabi.LAYOUT_ROW | hipabi.LAYOUT_IDX16)
+    dx, dy, dscratch, y = ctx.array(rng.standard_normal(n).astype(np.float32)), ctx.empty((m,)), ctx.empty((m,)), np.empty(m, np.float32)
+
+    def apart():
+        ctx.matvec(dE, dx, None, dy, layout)
+        ctx._ck(ctx.lib.so_stage_out(ctx.h, y.ctypes.data_as(ct.c_void_p), dy.ptr, 4 * m))
+
+    def us(call):
+        best = 1e9
+        for _ in range(8):
+            t = time.perf_counter()
+            for _ in range(20):
+                call()
+            best = min(best, (time.perf_counter() - t) / 20)
+        return best * 1e6
+
+    apart()
+    assert np.array_equal(to_host(ctx, dE, dx, None, dscratch, m, layout), y)
+    assert us(lambda: to_host(ctx, dE, dx, None, dscratch, m, layout)) < 1.3 * us(apart)
+    for a in (dE, dx, dy, dscratch):
         a.free()
 
 
