@@ -220,9 +220,11 @@ so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX, uint32_t 
  * connected layer -- the reference's documented way to get its allocation-free run(), README.md:146).
  * No counterpart in the reference. */
 so_status so_matmul_reserve(so_ctx *ctx, const so_ellpack *E, uint32_t C);
-/* Which kernel the context's last so_matmul, so_conv2d or encode launched, for tests and tuning: "merged", "quad", "planes", "narrow" and "vector" (on
- * handles with the RBM layout), "tiled", "columns", "shared", "row"; "columns", "merged-window", "window", "gather"; "encode-once", "encode-twice", "encode-spared" (twice, since
- * an earlier one-read encode gave up waiting); "" before the first.  A static string.  No counterpart in the reference. */
+/* Which kernel the context's last so_matmul, so_conv2d, so_conv2d_pair or encode launched, for tests and tuning.  so_matmul: "merged", "quad", "planes", "narrow",
+ * "slabs" (the quad-union copy with X in LDS a part at a time) and "vector" (on handles with the RBM layout), "tiled", "columns", "shared", "row"; so_conv2d: "columns",
+ * "merged-window", "window", "gather"; so_conv2d_pair: "columns-pair", "window-pair", or so_conv2d's for its second convolution where it makes two launches; encode:
+ * "encode-once", "encode-twice", "encode-spared" (twice, since an earlier one-read encode gave up waiting); "" before the first.  A static string.  No counterpart in
+ * the reference. */
 const char *so_last_kernel(const so_ctx *ctx);
 
 /* y[m] = E * x[n] + bias: ellpack_matvec (src/ellpack_matvec.cpp:20-147).

@@ -482,7 +482,7 @@ extern "C" so_status so_matmul(so_ctx *ctx, const so_ellpack *E, const float *dX
                                                         : so_matmul_rbm_launch(ctx, E, dX, C, dBias, dY, act);
             if (st != SO_OK) return st;
             SO_LAUNCH_CHECK();
-            ctx->last_kernel = k == RbmKernel::Quad || k == RbmKernel::Slabs ? "quad" : k == RbmKernel::Narrow ? "narrow" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
+            ctx->last_kernel = k == RbmKernel::Quad ? "quad" : k == RbmKernel::Narrow ? "narrow" : k == RbmKernel::Slabs ? "slabs" : k == RbmKernel::Planes ? "planes" : k == RbmKernel::Vector ? "vector" : "merged";
             return SO_OK;
         }
     }

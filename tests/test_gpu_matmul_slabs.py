@@ -25,7 +25,7 @@ def slabs_matmul(ctx, E, X, bias, slab, act="none", at=0):
     with ctx.tuning(SPARSEOPS_MATMUL_SLABS=slab):
         for _ in range(2):
             ctx.matmul(dE, flat.offset(at), C, dB, out.offset(at), act)
-            assert ctx.last_kernel() == "quad"
+            assert ctx.last_kernel() == "slabs"
     Y = out.download()
     assert (Y[:at] == 7.0).all() and (Y[at + m * C:] == 7.0).all()
     for a in (flat, out, dB, dE):
@@ -89,7 +89,7 @@ def test_rows_in_any_order(ctx):
 @pytest.mark.parametrize("m,n,C,sp,want", [(84, 692, 149, .5, True), (12, 1238, 173, .55, True), (2000, 2600, 16, .6, True), (17, 1090, 28, .67, True),
                                            (300, 300, 300, .9, False), (2000, 1500, 8, .6, False), (40, 4000, 83, .78, False), (200, 1500, 3, .5, False)])
 def test_which_calls_take_it(ctx, m, n, C, sp, want):
-    """Seen by the bits, which forbidding it changes; recorded after a reservation, whose replays give the same bits."""
+    """By name; forbidding it changes the bits.  Recorded after a reservation, whose replays give the same bits."""
     rng = np.random.default_rng(m + n)
     W = sparse_matrix(rng, m, n, sp)
     E = datagen.encode_dense(W)
@@ -100,6 +100,7 @@ def test_which_calls_take_it(ctx, m, n, C, sp, want):
     for slabs in (None, "0", "4", "8"):
         with ctx.tuning(SPARSEOPS_MATMUL_SLABS=slabs):
             ctx.matmul(dE, dX, C, None, dY)
+            assert (ctx.last_kernel() == "slabs") == (want if slabs is None else slabs != "0" and C >= 4)
             bits[slabs] = dY.download()
             assert rel_err(bits[slabs], W.astype(np.float64) @ X) <= TOL
     assert (not np.array_equal(bits[None], bits["0"])) == want
