@@ -450,6 +450,17 @@ bool fits(const so_ctx *ctx, const so_ellpack *E, uint32_t groups)
 
 } // namespace
 
+// Beyond 4 MB of X, an XCD's L2, what a launch of slabs waits for X from further away, by the workgroups that take a slab each: they lie on different XCDs, and each of the first
+// three fetches the slab for itself.  A slab of 16 columns uses 64 bytes of every line.  Us per MB of X, measured less estimated without it, 260 launches of 4..2000 rows, 257..8000
+// dense columns: slabs of 16 0.27, 0.58 and 0.7 for one, two, and three workgroups and more, of 32 0.12, 0.34 and 0.5.  (Without it X in parts was taken for 4 x 1187 x 3347 at 82 %
+// sparse, 15 MB, 9.6 us, shared gather 5.8, and 5 x 2003 x 1119 at 84 %, 8.5 MB, 11.6, quad-union 7.5; whole X in slabs of 32 for 9 x 956 x 2264 at 67 %, 8.3 MB, 10.4, quad-union 7.0.)
+static double narrow_far(uint32_t n, uint32_t C, uint32_t groups, uint32_t workgroups)
+{
+    const double megabytes = 4.0 * n * C / (1u << 20);
+    static constexpr double us[2][3] = {{0.3, 0.6, 0.7}, {0.15, 0.35, 0.5}};
+    return megabytes > 4.0 ? megabytes * us[groups == 8u][std::min(workgroups, 3u) - 1u] : 0.0;
+}
+
 bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     return E->quads.d_rows != nullptr && E->n != 0 && C >= 1 && C <= MOST_COLUMNS && (C <= 32 || C % 4 == 0) && fits(ctx, E, C <= 32 ? groups_for(C) : 4u);
@@ -460,8 +471,8 @@ bool so_matmul_narrow_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C
 // start and its copy of X (a value at a time where rows are no whole groups of four), the chunks of a wave, the copy's bytes, again for every
 // slab of 32 -- was fitted to 228 launches of 10..4096 rows, 512..4096 columns, 4..256 dense columns, 50-95 % sparse, and 14 of up to
 // 40 000 rows, one handle again and again: 7 % off (standard deviation; the same handle differs by 5 from one allocation to the next),
-// 30 % at most.  Beyond 4 MB of X, an XCD's L2, the 64 bytes of a row that a slab of 16 takes cost a whole line (4 x 1792 x 3780,
-// 27 MB, 14.2 us, shared gather 7.6; 12 x 2172 x 1860 17.7, quad-union 8.5; 320 launches of up to 1500 rows and 4800 dense columns); those of 32 columns take whole lines.
+// 30 % at most; beyond 4 MB of X narrow_far is added.
+// (Slabs of 16 are charged as for two workgroups, whatever there are.)
 so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
@@ -474,7 +485,7 @@ so_narrow_plan so_matmul_narrow_choose(const so_ctx *ctx, const so_ellpack *E, u
         while (ql < LOG_WAVES && (uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs > (uint64_t)ctx->compute_units) ++ql;
         const double rounds = so_ceil_div((uint64_t)so_ceil_div(Q.nquads, 1u << ql) * slabs, (uint64_t)ctx->compute_units);
         const double copy = 1e-4 * E->n * (slabs > 1 ? 1.92 * groups : C * (C % 4u ? 0.95 : 0.73)), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
-        const double megabytes = 4.0 * E->n * C / (1u << 20), far = slabs > 1 && groups == 4u && megabytes > 4.0 ? 0.6 * megabytes : 0.0;
+        const double far = slabs == 1 ? 0.0 : narrow_far(E->n, C, groups, groups == 4u ? 2u : so_ceil_div(Q.nquads, 1u << ql));
         const double again = groups == 8u ? slabs : 1.0;                  // slabs of 32 columns are few enough for their reads of the copy to count
         const double us = 1.05 + rounds * (2.0 + (slabs > 1 ? 0.36 : 0.0) + copy + chunks * (0.025 + 0.0244 * groups)) + 0.75e-5 * Q.total_chunks * again + far;
         if (us < best.us) best = so_narrow_plan{ql, groups, slabs, false, us};
@@ -488,7 +499,7 @@ bool so_matmul_slabs_applies(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 }
 
 // Slabs of 16 or of 32 columns, whichever is estimated faster.  Fitted to 400 launches of 10..4096 rows, 512..4096 columns, 4..256 dense columns, 50-95 % sparse:
-// 5.5 % off (standard deviation), 28 % at most (too low, for X of 3 MB and more, which the quad-union kernel's tiles serve better by far).
+// 5.5 % off (standard deviation), 28 % at most; beyond 4 MB of X narrow_far is added.
 so_narrow_plan so_matmul_slabs_choose(const so_ctx *ctx, const so_ellpack *E, uint32_t C)
 {
     const so_quads &Q = E->quads;
@@ -502,8 +513,9 @@ so_narrow_plan so_matmul_slabs_choose(const so_ctx *ctx, const so_ellpack *E, ui
         const double wgs = (double)so_ceil_div(Q.nquads, 1u << ql) * slabs, cus = ctx->compute_units, rounds = std::ceil(wgs / cus);
         const double passes = so_ceil_div(E->n, groups == 4u ? PASS_ROWS<4> : PASS_ROWS<8>), chunks = (double)Q.total_chunks / Q.nquads * (1u << ql) / WAVES;
         const double copy = (groups == 4u ? 0.53e-3 : 0.474e-3) * E->n * std::min(1.0, wgs / cus);
+        const double far = narrow_far(E->n, C, groups, so_ceil_div(Q.nquads, 1u << ql));
         const double us = 1.0 + rounds * (3.43 + 0.966 * (passes - 1.0) + copy + chunks * (0.0635 + 0.0142 * groups)) + 0.2e-5 * Q.total_chunks * (groups == 8u ? slabs : 1.0);
-        if (us < best.us) best = so_narrow_plan{ql, groups, slabs, true, us};
+        if (us + far < best.us) best = so_narrow_plan{ql, groups, slabs, true, us + far};
     }
     return best;
 }

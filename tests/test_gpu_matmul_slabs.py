@@ -117,3 +117,19 @@ def test_which_calls_take_it(ctx, m, n, C, sp, want):
     ctx.graph_free(g)
     for a in (dX, dY, dE):
         a.free()
+
+
+@pytest.mark.parametrize("m,n,C,sp", [(4, 1187, 3347, .82), (5, 2003, 1119, .84), (4, 1280, 4095, .6), (9, 956, 2264, .67), (35, 944, 1329, .62)])
+def test_slabs_of_a_large_x(ctx, m, n, C, sp):
+    """X beyond an XCD's L2 (4.7 to 20 MB): slabs, in parts or whole, were up to 1.7 times as slow as what runs without them."""
+    rng = np.random.default_rng(m + C)
+    W = sparse_matrix(rng, m, n, sp)
+    E = datagen.encode_dense(W)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    dE, dX, dY = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM), ctx.array(X), ctx.empty((m, C))
+    ctx.matmul_reserve(dE, C)
+    ctx.matmul(dE, dX, C, None, dY)
+    assert ctx.last_kernel() not in ("slabs", "narrow")
+    assert rel_err(dY.download(), W.astype(np.float64) @ X) <= TOL
+    for a in (dX, dY, dE):
+        a.free()
