@@ -11,13 +11,26 @@ namespace {
 
 constexpr int kBlock = 256;
 
+// f with the compile-time number that n, 0 .. MOST, is (none for 0).
+template <int MOST, class F>
+__device__ __forceinline__ void exactly(int32_t n, F &&f)
+{
+    if constexpr (MOST > 0) {
+        if (n == MOST) f(std::integral_constant<int, MOST>());
+        else exactly<MOST - 1>(n, f);
+    }
+}
+
 // applyMaxPool (src/layers/pool.cpp:28-101): -inf start, taps outside the image skipped.  A lane takes VEC batch entries of an output (4: B % 4 == 0,
-// 16-byte aligned tensors) and BH x BW taps at a time, row by row, all requested before the first comparison: a tap outside the image is read at the window's
-// nearest place inside and compared as -inf, which replaces nothing.  Kernels of more than three columns go a row of eight taps at a time.
+// 16-byte aligned tensors) and a block of taps at a time, all requested before the first comparison: a tap outside the image is read at the window's
+// nearest place inside and compared as -inf, which replaces nothing.  Kernels of up to 3x3 are one block (KH, KW); others of one, two or three columns (KH = 0) go eight, four or
+// three rows at a time, wider ones (KW = 0) a row of eight taps, and what is left is a block of that size: no tap is read that the kernel does not have.
 //
 // What bounds it: memory on large images, the launch and two round trips on small ones.  One tap at a time, a load each, 3x3/2 on 64 channels of 112x112 took
-// 24.5 us at batch 32 (128 MB in and out) and 6.8 at 8, now 19.2 (6.7 TB/s) and 5.4; 5x5 and 9x9 on 16 of 20x20 5.7 -> 4.5 and 12.6 -> 8.5.
-template <int VEC, int BH, int BW, class Index>
+// 24.5 us at batch 32 (128 MB in and out) and 6.8 at 8, now 18.7 (6.9 TB/s) and 5.4; 5x5 and 9x9 on 16 of 20x20 5.8 -> 4.1 and 13.2 -> 7.7.  One tap at a time / blocks of 3x3 and
+// 1x8 for all kernels but the smallest / now, at 112x112 and batch 32: 4x1/2 14.5 / 25.9 / 12.5, 1x2/2 12.3 / 19.5 / 11.9, 1x3/2 12.9 / 19.0 / 12.1, 4x4 90 / 111 / 66, 3x9 155 / 163 / 107.  (Taps
+// that are not there left out by a branch each: 4x4 126, 3x9 195.)
+template <int VEC, int KH, int KW, class Index>
 __global__ __launch_bounds__(kBlock)
 void maxpool_kernel(so_pool_geom p, const float *__restrict__ X, uint32_t Bv, Index total, float *__restrict__ Y)
 {
@@ -39,29 +52,49 @@ void maxpool_kernel(so_pool_geom p, const float *__restrict__ X, uint32_t Bv, In
         const int32_t h0 = (int32_t)ho * p.sH - p.padH0, w0 = (int32_t)wo * p.sW - p.padW0;
         const vec *__restrict__ Xc = Xv + (size_t)c * p.H * p.W * Bv + b;
         vec v = -INFINITY;
-        for (int32_t kh = 0; kh < p.kH; kh += BH)
-            for (int32_t kw = 0; kw < p.kW; kw += BW) {
-                vec x[BH][BW];
-                bool in[BH][BW];
+        auto taps = [&](int32_t kh, int32_t kw, auto rows, auto columns) {
+            constexpr int BH = decltype(rows)::value, BW = decltype(columns)::value;
+            vec x[BH][BW];
+            bool in[BH][BW];
 #pragma unroll
-                for (int i = 0; i < BH; ++i)
+            for (int i = 0; i < BH; ++i)
 #pragma unroll
-                    for (int j = 0; j < BW; ++j) {
-                        const int32_t h = h0 + kh + i, w = w0 + kw + j;
-                        in[i][j] = ((uint32_t)h < p.H) & ((uint32_t)w < p.W) & (kh + i < p.kH) & (kw + j < p.kW);
-                        const uint32_t hc = min((uint32_t)max(h, 0), p.H - 1u), wc = min((uint32_t)max(w, 0), p.W - 1u);
-                        x[i][j] = Xc[((Index)hc * p.W + wc) * Bv];
+                for (int j = 0; j < BW; ++j) {
+                    const int32_t h = h0 + kh + i, w = w0 + kw + j;
+                    in[i][j] = ((uint32_t)h < p.H) & ((uint32_t)w < p.W);
+                    const uint32_t hc = min((uint32_t)max(h, 0), p.H - 1u), wc = min((uint32_t)max(w, 0), p.W - 1u);
+                    x[i][j] = Xc[((Index)hc * p.W + wc) * Bv];
+                }
+#pragma unroll
+            for (int i = 0; i < BH; ++i)
+#pragma unroll
+                for (int j = 0; j < BW; ++j)
+#pragma unroll
+                    for (int e = 0; e < VEC; ++e) {
+                        const float xe = in[i][j] ? x[i][j][e] : -INFINITY;
+                        v[e] = xe > v[e] ? xe : v[e];
                     }
-#pragma unroll
-                for (int i = 0; i < BH; ++i)
-#pragma unroll
-                    for (int j = 0; j < BW; ++j)
-#pragma unroll
-                        for (int e = 0; e < VEC; ++e) {
-                            const float xe = in[i][j] ? x[i][j][e] : -INFINITY;
-                            v[e] = xe > v[e] ? xe : v[e];
-                        }
+        };
+        if (KH == 2 && KW == 2 && p.sH >= 2) {
+            // no row is read twice: one after the other, 2x2/2 at 112x112 and batch 32 19.2 -> 18.9 us (one tap at a time 18.8); 2x2/1 would take 44.7 instead of 41.5
+#pragma unroll 1
+            for (int32_t kh = 0; kh < 2; ++kh) taps(kh, 0, std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+        } else if constexpr (KH != 0) {
+            taps(0, 0, std::integral_constant<int, KH>(), std::integral_constant<int, KW>());
+        } else if constexpr (KW != 0) {
+            constexpr int R = KW == 1 ? 8 : KW == 2 ? 4 : 3;
+            const std::integral_constant<int, KW> columns;
+            int32_t kh = 0;
+            for (; kh + R <= p.kH; kh += R) taps(kh, 0, std::integral_constant<int, R>(), columns);
+            exactly<R - 1>(p.kH - kh, [&](auto rows) { taps(kh, 0, rows, columns); });
+        } else {
+            const std::integral_constant<int, 1> one;
+            for (int32_t kh = 0; kh < p.kH; ++kh) {
+                int32_t kw = 0;
+                for (; kw + 8 <= p.kW; kw += 8) taps(kh, kw, one, std::integral_constant<int, 8>());
+                exactly<7>(p.kW - kw, [&](auto columns) { taps(kh, kw, one, columns); });
             }
+        }
         reinterpret_cast<vec *>(Y)[q] = v;
     }
 }
@@ -229,20 +262,28 @@ extern "C" so_status so_maxpool(so_ctx *ctx, const so_pool_geom *p, const float 
     so_pool_geom taps = *p;
     if (p->H == 0 || p->W == 0) taps.kH = 0;                                 // no tap to read
     const bool small = outputs < (1ull << 31) && (uint64_t)p->H * p->W * Bv < (1ull << 31);
-#define SO_POOL_LAUNCH(VEC, BH, BW)                                                                                                     \
+#define SO_POOL_LAUNCH(VEC, KH, KW)                                                                                                     \
     do {                                                                                                                                 \
-        if (small) maxpool_kernel<VEC, BH, BW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, (uint32_t)outputs, dY);                   \
-        else maxpool_kernel<VEC, BH, BW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, outputs, dY);                                   \
+        if (small) maxpool_kernel<VEC, KH, KW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, (uint32_t)outputs, dY);                   \
+        else maxpool_kernel<VEC, KH, KW><<<blocks, kBlock, 0, ctx->stream>>>(taps, dX, Bv, outputs, dY);                                   \
+    } while (0)
+#define SO_POOL_ROWS(VEC, KW)                                                                                                           \
+    do {                                                                                                                                 \
+        if (taps.kH == 1) SO_POOL_LAUNCH(VEC, 1, KW);                                                                                    \
+        else if (taps.kH == 2) SO_POOL_LAUNCH(VEC, 2, KW);                                                                               \
+        else if (taps.kH == 3) SO_POOL_LAUNCH(VEC, 3, KW);                                                                               \
+        else SO_POOL_LAUNCH(VEC, 0, KW);                                                                                                 \
     } while (0)
 #define SO_POOL_TAPS(VEC)                                                                                                               \
     do {                                                                                                                                 \
-        if (p->kH == 1 && p->kW == 1) SO_POOL_LAUNCH(VEC, 1, 1);                                                                         \
-        else if (p->kH <= 2 && p->kW <= 2) SO_POOL_LAUNCH(VEC, 2, 2);                                                                         \
-        else if (p->kW <= 3) SO_POOL_LAUNCH(VEC, 3, 3);                                                                                  \
-        else SO_POOL_LAUNCH(VEC, 1, 8);                                                                                                  \
+        if (taps.kW == 1) SO_POOL_ROWS(VEC, 1);                                                                                          \
+        else if (taps.kW == 2) SO_POOL_ROWS(VEC, 2);                                                                                     \
+        else if (taps.kW == 3) SO_POOL_ROWS(VEC, 3);                                                                                     \
+        else SO_POOL_LAUNCH(VEC, 0, 0);                                                                                                  \
     } while (0)
     if (four) SO_POOL_TAPS(4);
     else SO_POOL_TAPS(1);
+#undef SO_POOL_ROWS
 #undef SO_POOL_TAPS
 #undef SO_POOL_LAUNCH
     SO_LAUNCH_CHECK();
