@@ -1,4 +1,4 @@
-"""The one-read encoder tells the host from its kernel: what it wrote is there for another context's stream at once, on both sides of the line (12 Mi slots
+"""The one-read encoder tells the host from its kernel: what it wrote is there for another context's stream at once, on both sides of the line (6 Mi slots
 of the result) beyond which the host waits for the stream's end instead, for one and many rows per workgroup, and call after call."""
 import numpy as np
 import pytest
@@ -32,3 +32,9 @@ def test_seen_from_another_stream(ctx, m, n, keep):
     for a in (dWd, dIdx, dNnz):
         a.free()
     other.close()
+
+
+@pytest.mark.parametrize("m,n", [(2048, 3072), (2049, 3072), (5000, 1023), (512, 10241)])
+def test_the_line_and_pieces_packed_again(ctx, m, n):
+    """No zeros: exactly 6 Mi slots and a row more; and, below the line, pieces that LDS does not keep, which are packed again or go straight to memory."""
+    test_seen_from_another_stream(ctx, m, n, 2.0)
