@@ -20,9 +20,9 @@
 // Results of up to kThroughSlots slots are stored past the L2, and the first workgroup tells the host when all are done: the end of the kernel, its
 // writing back of the caches, and a kernel or a wait of the runtime's behind it cost 3 us more.
 //
-// What bounds it: the read of W (8192 x 8192: 42 to 57 us, by workgroup and XCD, of which the copy's rate would take 43), then what
-// follows the slowest workgroup: 2 us until all know of all, 15 of writing 61 MB at 90 % sparse; launch and the
-// host's word 9.  Memory moves 269 MB in, W once, and 61 out (counters); at 50 % sparse, where LDS keeps one piece of eight, 450 in.
+// What bounds it: the read of W (8192 x 8192: 42 to 63 us, by workgroup and XCD, half of them at 50; the copy's rate would take 43), then what
+// follows the slowest workgroup: 1.5 us until all know of all, 12 to 14 of writing 61 MB at 90 % sparse; launch and the host's
+// wait 14, its word 10 (clock stamps).  Memory moves 269 MB in, W once, and 61 out (counters); at 50 % sparse, where LDS keeps one piece of eight, 450 in.
 // The whole call on one matrix again and again, two passes / this one with the host told behind the kernel / this one, us:
 //
 //   8192 x 8192 at 97 / 50 % sparse                            100 / 78.9 / 74.2, 195 / 174 / 174
@@ -44,7 +44,9 @@ constexpr uint32_t MOST_WGS = 256, kGaveUp = 0xffffffffu;
 // 45.5 / 47.1, 3491 x 4690 at 56 %, 7.5 M, 52.4 / 49.2, 8192 x 8192 at 97 / 90 %, 2.2 and 7.5 M, 80.3 / 84.6, 99 to 109 / 91.6.
 constexpr uint64_t kThroughSlots = 6u << 20;
 static_assert(3 * MOST_WGS <= 2 * kEncodeTold, "the words have room");
-constexpr uint32_t kLooks = 1u << 11;                             // of a bounded wait: about 3 ms, where the workgroups differ by some 10 us
+// Of a bounded wait, 0.19 us each: 3 ms.  The workgroups end the read of 8192 x 8192 some 16 to 21 us apart, of 32768 x 32768 115; those of a result that is stored past the L2 are
+// done 2 to 4 us apart.  The rest is for whoever holds part of the chip for a while: giving up costs this call the two passes and the next ones too.
+constexpr uint32_t kLooks = 1u << 14;
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -238,8 +240,7 @@ void ellpack_encode_once_kernel(EncodeArgs a)
         }
         vmax = wave_reduce<true>(vmax);
         vsum = wave_reduce<false>(vsum);
-        if (takers > 1u && lane == 0) { smax[wave] = vmax; ssum[wave] = vsum; }
-        if (takers == 1u && lane == 0) { smax[0] = vmax; ssum[0] = vsum; }
+        if (lane == 0) { smax[wave] = vmax; ssum[wave] = vsum; }
     }
     if (takers > 1u) __syncthreads();
     // The first wave tells the other workgroups, and looks for their words, four per lane: word(value) for each that has come; true: all have.
