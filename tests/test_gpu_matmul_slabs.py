@@ -1,5 +1,5 @@
 """The quad-union copy's kernel with X in LDS a part at a time (csrc/matmul_narrow.hip), forced, with slabs of 16 and 32 columns: at the edges of its
-parts (1024 and 512 rows of X), its slabs, its chunks of 16 steps and batches of 4 chunks, its quads per workgroup; with C of no multiple of four, whose
+parts (1280 and 512 rows of X), its slabs, its chunks of 16 steps and batches of 4 chunks, its quads per workgroup; with C of no multiple of four, whose
 last groups overhang X; and which calls it takes by itself.
 
 Bound: max|y - ref| <= 1e-5 * max|ref|, as for the layout's other kernels (tests/test_gpu_matmul_quad.py)."""
@@ -133,3 +133,18 @@ def test_slabs_of_a_large_x(ctx, m, n, C, sp):
     assert rel_err(dY.download(), W.astype(np.float64) @ X) <= TOL
     for a in (dX, dY, dE):
         a.free()
+
+
+@pytest.mark.parametrize("n,C", [(1279, 5), (1281, 5), (1281, 18), (1281, 39), (2559, 17), (2561, 6), (2561, 35), (3841, 4), (3841, 23), (3839, 50)])
+@pytest.mark.parametrize("slab", ["4", "8"])
+@pytest.mark.parametrize("m", [3, 90])
+def test_last_parts_of_one_row(ctx, m, n, C, slab):
+    """One row more or less than parts of 1280 rows: every row of the last part is its first one, and a group that overhangs X is read from four values before its end."""
+    rng = np.random.default_rng(m + n + C)
+    W = sparse_matrix(rng, m, n, .6)
+    W[:, n - 1] = 1 + np.arange(m)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    b = rng.standard_normal(m).astype(np.float32)
+    ref = W.astype(np.float64) @ X + b[:, None]
+    for at in (0, 1, 2, 3):
+        assert rel_err(slabs_matmul(ctx, datagen.encode_dense(W), X, b, slab, "none", at), ref) <= TOL
