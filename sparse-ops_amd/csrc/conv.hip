@@ -314,292 +314,32 @@ __device__ __forceinline__ void window_convolution(const int4 *__restrict__ stre
                                                    const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
                                                    const float *__restrict__ resid, float *__restrict__ Y, uint32_t wg, bool relu)
 {
-    extern __shared__ float4 win_lds[];
-    constexpr uint32_t BT = LPP * 4, PPW = 64 / LPP, SHIFT = (LPP == 8 ? 7 : LPP == 4 ? 6 : LPP == 2 ? 5 : 4);
-    const uint32_t tid = threadIdx.x, lane = tid & 63u;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t cgi = window_div(wave, a.pg, a.mPg), pgi = wave - cgi * a.pg;
-    WinPlace place;
-    if (!window_workgroup(a, wg, place)) return;
-    const uint32_t tile_y = window_div(place.tile, a.tiles_x, a.mTilesX);
-    const uint32_t th0 = tile_y * a.TH, tw0 = (place.tile - tile_y * a.tiles_x) * a.TW;
-    const uint32_t grp = place.y * a.cg + cgi;                       // channel group of this wave
-    const uint32_t co0 = grp * CPW;
-    const uint32_t bz = place.z * BT;
-    const bool computes = cgi < a.cg && grp < a.groups;              // the other waves only help copying
-    const uint32_t gi = computes ? grp : 0u;
-    // Asked for first: the stream's place, on which its first entries wait.
-    const uint32_t first_quad = ((so_constant<uint32_t>)(uintptr_t)gbase)[gi];
-    const so_constant<uint32_t> qp = (so_constant<uint32_t>)(uintptr_t)quads + (size_t)gi * a.nch * CPW;
-    uint32_t qfirst[CPW];
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) qfirst[c] = qp[c];
-
-    // this lane's output pixels and their corners inside the window
-    const uint32_t b4 = lane % LPP;
-    uint32_t ty[PX], tx[PX], lanebase[PX];
-    bool live[PX];
-#pragma unroll
-    for (int x = 0; x < PX; ++x) {
-        const uint32_t pl = (pgi * PX + (uint32_t)x) * PPW + lane / LPP;
-        const uint32_t pc = window_slot_pixel(a, pl & 63u);      // slots beyond the tile repeat a pixel of their group
-        ty[x] = window_div(pc, a.TW, a.mTW); tx[x] = pc - ty[x] * a.TW;
-        live[x] = computes && pl < a.TH * a.TW && th0 + ty[x] < g.H_out && tw0 + tx[x] < g.W_out;
-        lanebase[x] = ((ty[x] * a.sth * a.IW + tx[x] * a.stw) << SHIFT) + b4 * 16u;   // bytes
-    }
-    const uint32_t buf_bytes = a.buf_f4 * 16u;
-
-    // window elements this thread copies: element e = tid + k*1024 is float4 (cl, ih, iw, b4)
-    int32_t goff[kWinMaxPerThread];      // float offset from the chunk's first channel; -1: outside the image
-    uint32_t gcl[kWinMaxPerThread];      // channel inside the chunk; 0xffffffff: no such element
-#pragma unroll
-    for (int k = 0; k < kWinMaxPerThread; ++k) {
-        const uint32_t e = tid + (uint32_t)k * kWinThreads;
-        goff[k] = -1;
-        gcl[k] = 0xffffffffu;
-        if (e < a.win_f4) {
-            const uint32_t eb = e % LPP, px = e / LPP;
-            const uint32_t rest = window_div(px, a.IW, a.mIW), iw = px - rest * a.IW;
-            const uint32_t cl = window_div(rest, a.IH, a.mIH), ih = rest - cl * a.IH;
-            const int32_t gh = (int32_t)(th0 * g.stride_h + ih * a.sbh) - (int32_t)g.pad_h;
-            const int32_t gw = (int32_t)(tw0 * g.stride_w + window_column(a, iw) * a.sbw) - (int32_t)g.pad_w;
-            gcl[k] = cl;
-            if ((uint32_t)gh < g.H_in && (uint32_t)gw < g.W_in)
-                goff[k] = (int32_t)(((cl * g.H_in + (uint32_t)gh) * g.W_in + (uint32_t)gw) * B + bz + eb * 4u);
-        }
-    }
-    const size_t chunk_floats = (size_t)a.cc * g.H_in * g.W_in * B;
-
-    float4 xr[kWinMaxPerThread];
-    auto fetch_window = [&](uint32_t t) {
-        const float *__restrict__ Xc = X + (size_t)t * chunk_floats;
-        const uint32_t cleft = g.Cin - t * a.cc;                       // channels left from this chunk on
-#pragma unroll
-        for (int k = 0; k < kWinMaxPerThread; ++k) {
-            xr[k] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (goff[k] >= 0 && gcl[k] < cleft) xr[k] = *reinterpret_cast<const float4 *>(Xc + goff[k]);
-        }
-    };
-    auto store_window = [&](uint32_t buf) {
-#pragma unroll
-        for (int k = 0; k < kWinMaxPerThread; ++k)
-            if (gcl[k] != 0xffffffffu) win_lds[buf * a.buf_f4 + tid + (uint32_t)k * kWinThreads] = xr[k];
-    };
-
-    fetch_window(0);                  // stored below, once the entry stream is set up: the two latencies overlap
-
-    // The wave's entry stream: one quad = 4 entries = two int4 {w0, o0, w1, o1}, {w2, o2, w3, o3}.
-    // `cur` is the quad about to be used, the next one is requested before cur is consumed; the
-    // stream ends with a padding quad, so the request after the last quad is harmless.
-    // (read through the constant address space: that keeps them scalar loads next to the inline
-    // assembly of touch_stream)
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    typedef const i32x4 __attribute__((address_space(4))) *const_stream;
-    const int4 *__restrict__ sp0 = stream + 2 * (size_t)first_quad;
-    const_stream sp = (const_stream)(uintptr_t)sp0;
-    i32x4 cur0 = {0, 0, 0, 0}, cur1 = cur0;
-    // LANE_ENT: the entries sit in lanes instead (lane l of every 16-lane row holds entry l of the
-    // next 16), fetched with vector loads one group ahead and broadcast by DPP: vector loads have
-    // their own counter, so waiting for LDS data never waits for entries.  A DPP multiply-add keeps
-    // the vector unit busy a third longer than one with a scalar weight, though, so the scalar form
-    // wins wherever a wave has enough runs per chunk to amortise its scalar loads: measured on the
-    // ResNet-18-shaped layers at batch 32, scalar against lanes: 8 channels per wave 55 against 60 us,
-    // 4 channels 56.1 against 63.2, 2 channels 58.8 against 56.6; small batches use 1-2 channels.
-    constexpr bool LANE_ENT = PX == 1 && CPW < 4;
-    // priorities rotate on the full batch tile only: on the smaller ones (batches below 16) it measured 5 % slower
-    constexpr bool ROTATE = LPP == 4;
-    // progress counters instead of a barrier per chunk: the same (batch 8: 0.466 -> 0.474 ms, batch 1: 0.365 -> 0.374 with them)
-    constexpr bool DRIFT = LPP == 4;
-    const int2 *__restrict__ ep = reinterpret_cast<const int2 *>(sp0) + (lane & 15u);
-    int2 ecur = make_int2(0, 0);
-    uint32_t qtouch = 0;                                             // quads of the chunk about to start
-    if constexpr (LANE_ENT) {
-        ecur = ep[0];
-    } else {
-        if (computes) {
-#pragma unroll
-            for (int c = 0; c < CPW; ++c) qtouch += qfirst[c];
-        }
-        touch_stream(sp0, qtouch + 1u, pgi, a.pg);
-        cur0 = sp[0];
-        cur1 = sp[1];
-        sp += 2;
-    }
-    float acc[CPW][PX][4];
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-        const float b0 = (bias && computes && co0 + c < g.Cout) ? ((so_constant<float>)(uintptr_t)bias)[co0 + c] : 0.0f;
-#pragma unroll
-        for (int x = 0; x < PX; ++x) acc[c][x][0] = acc[c][x][1] = acc[c][x][2] = acc[c][x][3] = b0;
-    }
-
-    // the all-zero plane behind each window buffer (padding entries point into it)
-    for (uint32_t i = tid; i < a.buf_f4 - a.win_f4; i += kWinThreads) {
-        win_lds[a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (a.nbuf == 2) win_lds[a.buf_f4 + a.win_f4 + i] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    // progress counters behind the buffers: [0], [1] windows stored into buffer 0 / 1 (x 16 waves), [2], [3] chunks read out of them
-    const uint32_t sync_base = so_lds::lds_address(win_lds + (size_t)a.nbuf * a.buf_f4);
-    if (a.nbuf == 2 && tid < 4) reinterpret_cast<uint32_t *>(win_lds + (size_t)a.nbuf * a.buf_f4)[tid] = tid == 0 ? 16u : 0u;
-    store_window(0);
-    __syncthreads();
-
-    const char *lds_bytes = reinterpret_cast<const char *>(win_lds);
-    for (uint32_t t = 0; t < a.nch; ++t) {
-        const bool more = t + 1 < a.nch;
-        if (more) fetch_window(t + 1);
-        const uint32_t cur_buf = a.nbuf == 2 ? (t & 1u) : 0u;
-        uint32_t base[PX];
-#pragma unroll
-        for (int x = 0; x < PX; ++x) base[x] = lanebase[x] + cur_buf * buf_bytes;
-        uint32_t nq[CPW];
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) nq[c] = computes ? qp[t * CPW + c] : 0u;
-        // Half-way through the chunk the wave stores its part of the next window, as soon as every wave
-        // has finished the chunk before this one (which read the buffer it goes to).  A wave that is
-        // done with its steps then only needs every wave to be past that half-way point, not to be
-        // done as well: the waves of a SIMD finish a chunk up to a third of its length apart.
-        bool stored = !(DRIFT && more && a.nbuf == 2);
-        auto store_next = [&]() {
-            if (stored) return;
-            stored = true;
-            so_lds::wait(sync_base + 8u + ((t + 1u) & 1u) * 4u, 16u * ((t + 1u) / 2u), a.ws);
-            store_window((t + 1u) & 1u);
-            so_lds::signal(sync_base + ((t + 1u) & 1u) * 4u, lane);
-        };
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-            if (CPW >= 2 && c == CPW / 2) store_next();
-            const uint32_t turn = (wave >> 2) + (uint32_t)c + t;      // a new priority per run; per group of 16 entries where the entries sit in lanes
-            if constexpr (ROTATE) rotate_priority(turn);
-            if constexpr (LANE_ENT && CPW <= 2) {
-                // Pipelined: a quad's LDS reads overlap the previous quad's multiply-adds all through
-                // the run (so_dpp::group16).  Measured on ResNet-18 shapes at batch 32: 14x14x256
-                // (2 channels per wave) 63.5 -> 58.4 us, 7x7x512 (1 per wave) 69.1 -> 66.1 us; with 4
-                // channels per wave the four copies of these bodies made 28x28x128 11 % slower.
-                const uint32_t n = nq[c];
-                const char *xb = lds_bytes + base[0];
-                float4 xA[4], xB[4];
-                if (n >= 4u) {
-                    ep += 16;
-                    int2 enxt = ep[0];                                    // the stream ends with 16 padding entries
-                    so_dpp::group16<false>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c][0]);
-                    float ewp = __int_as_float(ecur.x);
-                    ecur = enxt;
-                    uint32_t q = 4u;
-                    const uint32_t q_mid = CPW == 1 ? n / 8u * 4u : 0xffffffffu;
-                    for (; q + 4u <= n; q += 4u) {
-                        if (CPW == 1 && q == q_mid) store_next();
-                        if constexpr (ROTATE) rotate_priority(turn + (q >> 2));
-                        ep += 16;
-                        enxt = ep[0];
-                        so_dpp::group16<true>(xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c][0]);
-                        ewp = __int_as_float(ecur.x);
-                        ecur = enxt;
-                    }
-                    if (q < n) {
-                        ep += 4u * (n - q);
-                        enxt = ep[0];
-                        so_dpp::group_tail<true>(n - q, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, ewp, xA, xB, acc[c][0]);
-                        ecur = enxt;
-                    } else {
-                        so_dpp::group_drain(ewp, xB, acc[c][0]);
-                    }
-                } else if (n != 0u) {
-                    ep += 4u * n;
-                    const int2 enxt = ep[0];
-                    so_dpp::group_tail<false>(n, xb, __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, 0.0f, xA, xB, acc[c][0]);
-                    ecur = enxt;
-                }
-                continue;
-            }
-            if constexpr (LANE_ENT) {
-                for (uint32_t q = 0; q < nq[c]; q += 4u) {
-                    if (ROTATE && q) rotate_priority(turn + (q >> 2));
-                    const uint32_t steps = 4u * min(4u, nq[c] - q);      // this group: 4, 8, 12 or 16 entries
-                    ep += steps;
-                    const int2 enxt = ep[0];                              // the stream ends with 16 padding entries
-                    so_dpp::tiled_chunk(lds_bytes + base[0], __int_as_float(ecur.x), (uint32_t)ecur.y << SHIFT, steps, acc[c][0]);
-                    ecur = enxt;
-                }
-                continue;
-            }
-            for (uint32_t q = 0; q < nq[c]; ++q) {
-                const i32x4 nxt0 = sp[0], nxt1 = sp[1];
-                sp += 2;
-                float w[4] = {__int_as_float(cur0.x), __int_as_float(cur0.z), __int_as_float(cur1.x), __int_as_float(cur1.z)};
-                const uint32_t off[4] = {(uint32_t)cur0.y << SHIFT, (uint32_t)cur0.w << SHIFT, (uint32_t)cur1.y << SHIFT, (uint32_t)cur1.w << SHIFT};
-                float4 v[4][PX];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int x = 0; x < PX; ++x) v[e][x] = *reinterpret_cast<const float4 *>(lds_bytes + base[x] + off[e]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if constexpr (PX > 1) asm("v_mov_b32 %0, %1" : "=v"(w[e]) : "s"(w[e]));
-#pragma unroll
-                    for (int x = 0; x < PX; ++x) {
-                        acc[c][x][0] = __builtin_fmaf(w[e], v[e][x].x, acc[c][x][0]); acc[c][x][1] = __builtin_fmaf(w[e], v[e][x].y, acc[c][x][1]);
-                        acc[c][x][2] = __builtin_fmaf(w[e], v[e][x].z, acc[c][x][2]); acc[c][x][3] = __builtin_fmaf(w[e], v[e][x].w, acc[c][x][3]);
-                    }
-                }
-                cur0 = nxt0;
-                cur1 = nxt1;
-            }
-        }
-        if constexpr (!LANE_ENT) {
-            if (more && computes) {                // the next chunk's entries, while the slower waves finish this one
-                uint32_t qn = 0;
-#pragma unroll
-                for (int c = 0; c < CPW; ++c) qn += qp[(t + 1) * CPW + c];
-                if (qn) touch_stream((const int4 *)(uintptr_t)sp, qn, pgi, a.pg);
-            }
-        }
-        if (DRIFT && a.nbuf == 2) {
-            store_next();
-            so_lds::signal(sync_base + 8u + cur_buf * 4u, lane);                    // done reading this chunk's buffer
-            if (more) so_lds::wait(sync_base + (cur_buf ^ 1u) * 4u, 16u * ((t + 1u) / 2u + 1u), a.ws);   // the next window is complete
-        } else if (a.nbuf == 2) {
-            if (more) store_window(cur_buf ^ 1u);
-            __syncthreads();
-        } else {
-            __syncthreads();                       // every wave has finished reading the only buffer
-            if (more) store_window(0);
-            __syncthreads();
-        }
-    }
-
-#pragma unroll
-    for (int x = 0; x < PX; ++x) {
-        if (!live[x]) continue;
-        const uint32_t ho = th0 + ty[x], wo = tw0 + tx[x];
-#pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-            const uint32_t co = co0 + c;
-            if (co < g.Cout) {
-                const size_t at = (((size_t)co * g.H_out + ho) * g.W_out + wo) * B + bz + b4 * 4u;
-                float (&v)[4] = acc[c][x];
-                if (resid) {             // conv + skip, then the activation
-                    const float4 rv = *reinterpret_cast<const float4 *>(resid + at);
-                    v[0] += rv.x; v[1] += rv.y; v[2] += rv.z; v[3] += rv.w;
-                }
-                float4 out;
-                out.x = conv_epilogue<ACT>(v[0], relu); out.y = conv_epilogue<ACT>(v[1], relu);
-                out.z = conv_epilogue<ACT>(v[2], relu); out.w = conv_epilogue<ACT>(v[3], relu);
-                *reinterpret_cast<float4 *>(Y + at) = out;
-            }
-        }
-    }
+#include "conv_window_body.inc"
 }
 
-// One convolution's operands.  The kernels read them where they are used, from the arguments: held as values from the start, as the compiler does with
-// a kernel's own, 20 to 31 scalar registers spill when the body is shared (84 to 117 reads back: stems of 96x96 images 12.4 and 22.5 us instead of 11.0 and 20.9).
+constexpr size_t kWinKernelArgs = 3 * sizeof(void *) + sizeof(WinArgs) + sizeof(so_conv_geom) + 5 * sizeof(void *);
+static_assert(kWinKernelArgs > 0x140 + 4 && kWinKernelArgs <= 0x180, "lines of 64 bytes that touch_arguments reads");
+template <int CPW, int LPP, int ACT, int PX>
+__global__ __launch_bounds__(kWinThreads)
+void conv2d_window_kernel(const int4 *__restrict__ stream, const uint32_t *__restrict__ gbase,
+                          const uint32_t *__restrict__ quads, WinArgs a, so_conv_geom g,
+                          const float *__restrict__ X, uint32_t B, const float *__restrict__ bias,
+                          const float *__restrict__ resid, float *__restrict__ Y)
+{
+    touch_arguments((const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr());
+    const uint32_t wg = blockIdx.x;
+    const bool relu = false;
+#include "conv_window_body.inc"
+}
+
+// One convolution's operands.  The pair kernel reads them where they are used, from the arguments: held as values from the start, as the compiler does with
+// a kernel's own, 20 to 31 scalar registers spill (84 to 117 reads back: stems of 96x96 images 12.4 and 22.5 us instead of 11.0 and 20.9).
 struct WinCall {
     const int4 *stream;
     const uint32_t *gbase, *quads;
     WinArgs a;
     so_conv_geom g;
-    const float *X, *bias, *resid;
+    const float *X, *bias;
     float *Y;
     uint32_t B, relu;                // relu: kActNoneOrRelu
 };
@@ -608,15 +348,6 @@ struct WinPair {
     uint32_t wgs0;
 };
 static_assert(sizeof(WinCall) > 0x140 + 4 && sizeof(WinCall) <= 0x180, "lines of 64 bytes that touch_arguments reads");
-template <int CPW, int LPP, int ACT, int PX>
-__global__ __launch_bounds__(kWinThreads)
-void conv2d_window_kernel(WinCall)
-{
-    const auto *args = (const __attribute__((address_space(4))) char *)__builtin_amdgcn_kernarg_segment_ptr();
-    touch_arguments(args);
-    const WinCall &c = *(const WinCall *)args;
-    window_convolution<CPW, LPP, ACT, PX>(c.stream, c.gbase, c.quads, c.a, c.g, c.X, c.B, c.bias, c.resid, c.Y, blockIdx.x, false);
-}
 
 // Two convolutions of one input: the first's workgroups, a multiple of 8 of them, then the second's.
 template <int CPW, int LPP, int PX>
@@ -636,8 +367,10 @@ template <int CPW, int LPP, int PX>
 void window_launch_act(so_ctx *ctx, const so_conv_plan *plan, const WinArgs &a, dim3 grid, size_t lds,
                        const float *dX, uint32_t B, const float *dBias, const float *dResid, float *dY, int act)
 {
-    const WinCall c{reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a, plan->g, dX, dBias, dResid, dY, B, 0};
-#define SO_WIN_LAUNCH(A) conv2d_window_kernel<CPW, LPP, A, PX><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(c)
+#define SO_WIN_LAUNCH(A)                                                                                   \
+    conv2d_window_kernel<CPW, LPP, A, PX><<<window_grid(a, grid), kWinThreads, lds, ctx->stream>>>(        \
+        reinterpret_cast<const int4 *>(plan->win.d_stream), plan->win.d_gbase, plan->win.d_quads, a,       \
+        plan->g, dX, B, dBias, dResid, dY)
     switch (act) {
     case SO_ACT_RELU:    SO_WIN_LAUNCH(SO_ACT_RELU); break;
     case SO_ACT_SIGMOID: SO_WIN_LAUNCH(SO_ACT_SIGMOID); break;
@@ -769,7 +502,7 @@ so_status window_launch_pair(so_ctx *ctx, const so_conv_call (&call)[2], const f
         if (!window_arguments<LPP>(ctx, call[i].plan, B, forced, c.a, grid[i], lds[i]) || c.a.per_xcd == 0u) return SO_OK;
         c.stream = reinterpret_cast<const int4 *>(w.d_stream); c.gbase = w.d_gbase; c.quads = w.d_quads;
         c.g = call[i].plan->g;
-        c.X = dX; c.bias = call[i].dBias; c.resid = nullptr; c.Y = call[i].dY; c.B = B;
+        c.X = dX; c.bias = call[i].dBias; c.Y = call[i].dY; c.B = B;
         c.relu = call[i].act == SO_ACT_RELU;
     }
     p.wgs0 = 8u * p.call[0].a.per_xcd;
