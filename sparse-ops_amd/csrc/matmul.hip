@@ -375,7 +375,11 @@ constexpr double kPlanesBelow = 0.9;
 // 7.2 / 3.7, 2048 x 2048 x 64 at 80 % 9.9 / 9.6, 2000 x 1500 x 64 at 60 % 9.9 / 11.6, 20 000 x 600 x 64 at 90 % 17.6 / 25.3; row 107 x 730 x 16 at 94 % 3.6 / 3.9.
 // In place of so_matvec's row kernel at two and three columns from a million nonzeros on: 1.39 million, two columns, 8.8 / 4.0; 1.5 million, three, 9.6 / 4.3; 2.9 million,
 // three, 17.7 / 6.3.  (Below it would gain less, 0.3 to 0.6 of 4.1; with one column it is not looked at.)
-constexpr double kNarrowBelow = 0.955;
+//
+// At 17 to 32 columns (one slab of 32) its launches of less than 6 us take 0.3 to 0.8 more than estimated, of X with fewer rows than what that was fitted on most; the others'
+// less.  Us, columns or row kernel / narrow: 979 x 223 x 19 at 57 % sparse 3.6 / 4.3, 7064 x 109 x 31 at 70 % 4.6 / 5.4, 123 x 168 x 23 at 54 % 3.4 / 3.9; beyond, 8815 x 295 x 29 at 48 % 10.0 / 7.6.  Of
+// 543 drawn launches of 16..4000 columns that it took without this term it was 0.4 % the slower one on average, in 203 by more than 4 %; with it, 2.6 % the faster one, in 8 slower by that.
+constexpr double kNarrowBelow = 0.955, kNarrowWide = 0.7, kNarrowWideBelow = 6.0;
 constexpr uint64_t kNarrowVectorNnz = 1000000;
 
 // The same with X in LDS a part at a time, where it is estimated 7 % below what would run: of 200 drawn launches it is then taken in 47, all of
@@ -411,10 +415,9 @@ RbmKernel rbm_kernel(const so_ctx *ctx, const so_ellpack *E, uint32_t C, so_quad
     if (ctx->tune.matmul_quad >= 0 || ctx->tune.matmul_planes == 1) return k;
     if (ctx->tune.matmul_narrow != 0 && so_matmul_narrow_applies(ctx, E, C)) {
         *narrow = so_matmul_narrow_choose(ctx, E, C);
-        if (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : narrow->us < kNarrowBelow * us) {
-            k = RbmKernel::Narrow;
-            us = narrow->us;
-        }
+        const double below = kNarrowBelow * us, wide = narrow->groups == 8u && narrow->slabs == 1u && narrow->us < kNarrowWideBelow ? kNarrowWide : 0.0;
+        if (narrow->us < below) us = narrow->us;                          // (what X in parts is compared with)
+        if (vector ? C >= 2 && E->total_nnz >= kNarrowVectorNnz : narrow->us + wide < below) k = RbmKernel::Narrow;
     }
     if (vector || ctx->tune.matmul_slabs == 0 || !so_matmul_slabs_applies(ctx, E, C)) return k;
     const so_narrow_plan slabs = so_matmul_slabs_choose(ctx, E, C);

@@ -180,3 +180,20 @@ def test_which_calls_take_it(ctx, m, n, C, sp, want):
             assert ctx.last_kernel() != "narrow"
     for a in (dX, dY, dE):
         a.free()
+
+
+@pytest.mark.parametrize("m,n,C,sp,want", [(979, 223, 19, .57, False), (7064, 109, 31, .7, False), (123, 168, 23, .54, False), (3280, 171, 19, .89, False), (8815, 295, 29, .48, True),
+                                           (2818, 728, 32, .42, True), (979, 223, 8, .57, True)])
+def test_wide_slabs_of_small_launches(ctx, m, n, C, sp, want):
+    """17 to 32 columns: launches of 3.4 to 4.6 us on the columns or row kernel took up to a fifth longer here; those of 7.6 and more stay."""
+    rng = np.random.default_rng(m + n)
+    W = sparse_matrix(rng, m, n, sp)
+    E = datagen.encode_dense(W)
+    X = rng.standard_normal((n, C)).astype(np.float32)
+    dE, dX, dY = ctx.upload_ellpack(E.Wd, E.idx, E.nnz, E.m, E.n, E.r, RBM), ctx.array(X), ctx.empty((m, C))
+    ctx.matmul_reserve(dE, C)
+    ctx.matmul(dE, dX, C, None, dY)
+    assert (ctx.last_kernel() == "narrow") == want
+    assert rel_err(dY.download(), W.astype(np.float64) @ X) <= TOL
+    for a in (dX, dY, dE):
+        a.free()
