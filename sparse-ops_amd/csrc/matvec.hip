@@ -613,7 +613,7 @@ extern "C" so_status so_matvec(so_ctx *ctx, const so_ellpack *E, const float *dx
 }
 
 // The result straight into the staging memory, one launch fewer in a chain that is nothing but launches and the link.  ellpack_matvec from
-// host arrays, us, a kernel for the way back / this: 1500 x 1000 at 90 % sparse 17.9 / 14.9, 2864 x 3084 at 97 % 19.3 / 16.1, 4096 x 4096 at 80 %
+// host arrays, us, a kernel for the way back / this: 1500 x 1000 at 90 % sparse 17.9 / 15.1, 2864 x 3084 at 97 % 19.3 / 16.1, 4096 x 4096 at 80 %
 // 21.6 / 17.6, 8000 x 2000 at 90 % 23.6 / 21.2; Zipf rows 1077 x 3800 19.4 / 15.8, 4096 x 4096 20.2 / 17.4.  Beyond kStagePairsMost rows the host's look at each
 // pair, and in the classes' order its walk over y, take longer than the launch did: 16384 x 2000 29.0 / 32.7, 12000 x 2000 with Zipf rows 24.2 / 26.3.
 extern "C" so_status so_matvec_to_host(so_ctx *ctx, const so_ellpack *E, const float *dx, const float *dBias, float *dy, float *y, int layout)

@@ -150,9 +150,10 @@ void SparseOnnxModel::Impl::enqueue_layers(const float *in, float *out) const
 // A launch graph spares the host about 4 us a launch, but the GPU waits 4 to 10 us before and behind one and works on the arena's
 // slots only, so that device callers' input and output are copied: it pays where the chain is shorter than the host needs to launch it.
 // The chain's time: 4 us a layer and the longer of a row's chain at 10 ns an entry and the layer's work at 25 TFLOP/s; the line lies at 6.5 us a
-// layer.  ResNet-18-shaped stacks, 23 launches, us with a graph / without, run_device: 64 x 64 of width 16 at batch 1 108 / 114, 4 119 / 140, 16 145 / 153;
-// 96 x 96 of 32 at 8 195 / 195; 128 x 128 of 32 at 32 352 / 330; 224 x 224 of 64 at 1 245 / 226, at 32 966 / 923.  From host arrays: 64 x 64 at batch
-// 4 125 / 126, 96 x 96 at 8 220 / 222, 128 x 128 of 48 at 2 235 / 247; 160 x 160 of 32 at 11 403 / 397, 224 x 224 of 48 at 4 372 / 367, of 64 at 1 258 / 255.
+// layer.  ResNet-18-shaped stacks, 23 layers in 20 launches (three projections share one), us with a graph / without, run_device: 64 x 64 of width 16 at batch 1 110 / 122, 4 121 / 132,
+// 16 125 / 125; 96 x 96 of 32 at 8 158 / 159; 160 x 160 of 48 at 2 189 / 177, which the line still records; 128 x 128 of 32 at 32 268 / 257; 224 x 224 of 64 at 1 222 / 209, at 32
+// 924 / 907.  From host arrays: 64 x 64 at batch 4 127 / 124, 96 x 96 at 8 188 / 192, 128 x 128 of 48 at 2 176 / 176; 160 x 160 of 32 at 11 369 / 365, 224 x 224 of 48 at 4 361 / 356, of 64 at 1
+// 237 / 236.
 // A 4-layer MLP: 111 / 102; chains of fewer than eight layers have no graph.
 bool SparseOnnxModel::Impl::record_pays() const
 {
